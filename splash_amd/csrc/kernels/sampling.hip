@@ -393,8 +393,10 @@ struct Mass {
 __device__ __forceinline__ Mass merge(Mass a, Mass b, float inverse_temperature) {
   const float m = fmaxf(a.maximum, b.maximum);
   if (m == -INFINITY) return {m, 0.f};
-  const float sa = a.maximum == -INFINITY ? 0.f : a.sum * expf((a.maximum - m) * inverse_temperature);
-  const float sb = b.maximum == -INFINITY ? 0.f : b.sum * expf((b.maximum - m) * inverse_temperature);
+  // the side that holds the maximum weighs exp(0) = 1: one exponential, of the other side
+  const bool first = a.maximum == m;
+  const float other = (first ? b.maximum : a.maximum), weight = other == -INFINITY ? 0.f : expf((other - m) * inverse_temperature);
+  const float sa = first ? a.sum : a.sum * weight, sb = first ? b.sum * weight : b.sum;
   return {m, sa + sb};
 }
 __device__ __forceinline__ uint32_t lane_of_row(const TargetSamplingParams &p, uint32_t row) {
@@ -435,11 +437,13 @@ __global__ __launch_bounds__(256) void decode_sample_mass_sharded(const float *_
 }
 SP_REGISTER_KERNEL("decode_sample_mass_sharded", &decode_sample_mass_sharded);
 
-// The row's (max, total) from its shards, in shard order.
+// The row's (max, total) from its shards, in shard order. Called by whole wavefronts: a lane fetches a shard's.
 __device__ __forceinline__ Mass row_mass(const float *masses, uint32_t row, float inverse) {
-  Mass all{masses[2 * row * SAMPLING_SHARDS], masses[2 * row * SAMPLING_SHARDS + 1]};
-  for (uint32_t s = 1; s < SAMPLING_SHARDS; ++s)
-    all = merge(all, Mass{masses[2 * (row * SAMPLING_SHARDS + s)], masses[2 * (row * SAMPLING_SHARDS + s) + 1]}, inverse);
+  const uint32_t shard = (threadIdx.x & 63u) % SAMPLING_SHARDS;
+  const float2 mine = reinterpret_cast<const float2 *>(masses)[row * SAMPLING_SHARDS + shard];
+  Mass all{__shfl(mine.x, 0, 64), __shfl(mine.y, 0, 64)};
+#pragma unroll
+  for (int s = 1; s < int(SAMPLING_SHARDS); ++s) all = merge(all, Mass{__shfl(mine.x, s, 64), __shfl(mine.y, s, 64)}, inverse);
   return all;
 }
 // The child of `row` in its lane's block: the first later row whose parent it is; none: SAMPLING_NO_TOKEN.
@@ -497,16 +501,17 @@ __device__ __forceinline__ float residual_of(float logit, uint32_t token, float 
   return rejected ? fmaxf(w / kept.mass.sum - q, 0.f) : w;
 }
 // ---------------------------------------------------------------------------------------------
-// decode_sample_distribution_end: grid (rows), 256 threads. Writes the row's end words of the
+// decode_sample_distribution_end: grid (rows), 1024 threads. Writes the row's end words of the
 // decisions buffer; rows of lanes that keep every token are left alone.
 // ---------------------------------------------------------------------------------------------
 struct Measure {
   uint32_t count;
   float mass;
 };
+constexpr uint32_t kEndThreads = 1024;
 struct EndScratch {
-  float mass[16][SAMPLING_THREADS];
-  uint32_t count[16][SAMPLING_THREADS];
+  float mass[16][kEndThreads];
+  uint32_t count[16][kEndThreads];
   float binMass[16];
   uint32_t binCount[16];
 };
@@ -520,7 +525,7 @@ __device__ __forceinline__ void end_histogram(const float *x, uint32_t vocabular
     scratch.mass[b][tid] = 0.f;
     scratch.count[b][tid] = 0u;
   }
-  for (uint32_t token = tid; token < vocabulary; token += SAMPLING_THREADS) {
+  for (uint32_t token = tid; token < vocabulary; token += kEndThreads) {
     const float value = x[token];
     if (unselectable(value)) continue;
     const uint32_t key = logit_key(value);
@@ -531,22 +536,23 @@ __device__ __forceinline__ void end_histogram(const float *x, uint32_t vocabular
     scratch.count[b][tid] += 1u;
   }
   __syncthreads();
-  // Wavefront w sums bins 4 w .. 4 w + 3: a lane its four threads in order, the lanes in a fixed butterfly.
-  const uint32_t lane = tid & 63u, wave = tid >> 6;
+  // Wavefront w sums bin w: a lane its sixteen threads in order, the lanes in a fixed butterfly.
+  const uint32_t lane = tid & 63u, b = tid >> 6;
+  float m = 0.f;
+  uint32_t c = 0;
 #pragma unroll
-  for (uint32_t i = 0; i < 4; ++i) {
-    const uint32_t b = 4u * wave + i;
-    float m = ((scratch.mass[b][lane] + scratch.mass[b][lane + 64u]) + scratch.mass[b][lane + 128u]) + scratch.mass[b][lane + 192u];
-    uint32_t c = scratch.count[b][lane] + scratch.count[b][lane + 64u] + scratch.count[b][lane + 128u] + scratch.count[b][lane + 192u];
+  for (uint32_t i = 0; i < kEndThreads / 64u; ++i) {
+    m += scratch.mass[b][lane + 64u * i];
+    c += scratch.count[b][lane + 64u * i];
+  }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      m += __shfl_xor(m, o, 64);
-      c += uint32_t(__shfl_xor(int(c), o, 64));
-    }
-    if (lane == 0) {
-      scratch.binMass[b] = m;
-      scratch.binCount[b] = c;
-    }
+  for (int o = 32; o > 0; o >>= 1) {
+    m += __shfl_xor(m, o, 64);
+    c += uint32_t(__shfl_xor(int(c), o, 64));
+  }
+  if (lane == 0) {
+    scratch.binMass[b] = m;
+    scratch.binCount[b] = c;
   }
   __syncthreads();
 }
@@ -629,27 +635,226 @@ __device__ OrderEnd select_last(const float *x, uint32_t vocabulary, Mass mass, 
   return last;
 }
 
-__global__ __launch_bounds__(SAMPLING_THREADS) void decode_sample_distribution_end(const float *__restrict__ logits,
-                                                                                  const float *__restrict__ masses,
-                                                                                  uint32_t *__restrict__ decisions, TargetSamplingParams p) {
-  __shared__ EndScratch scratch;
-  const uint32_t row = blockIdx.x, tid = threadIdx.x, laneIndex = lane_of_row(p, row);
+// A row whose end lies among its heaviest kEndCandidates tokens, which is nearly every row of a policy in use, is
+// decided from them alone. The row is read twice: once to count its tokens in bins of (maximum - logit) / temperature, a
+// sixteenth of an e-fold each, and once to gather those of the bins that are sure to hold the end. They are sorted by
+// (logit, id) in LDS; the count and the running mass in that order are what top_k and top_p cut. Any other row (a
+// nucleus of many thousand tokens) takes the descent above, a scan of the row a digit. What bounds the pass is one
+// compute unit's reading of the row: 24 rows of 151936 logits under min_p 0.02, top_k 64 and top_p 0.95 took 1244 us by
+// the descent of 256 threads, and 42 us this way.
+constexpr uint32_t kEndCandidates = 8192, kEndBins = 512;
+constexpr float kEndBinsPerFold = 16.f;
+struct EndSelection {
+  uint64_t order[kEndCandidates];  // (key, ~id), descending once sorted
+  uint32_t bins[kEndBins];
+  float waveMass[kEndThreads / 64u];
+  float total;
+  uint32_t selectable, gathered, cut, candidates, keep;
+};
+union EndShared {
+  EndScratch descent;
+  EndSelection selection;
+};
+// Calls take(value, token) of every token of the row, four a load whatever the row's alignment.
+template <class Take> __device__ __forceinline__ void end_scan(const float *x, uint32_t vocabulary, uint32_t tid, Take take) {
+  typedef __attribute__((ext_vector_type(4), aligned(4))) float f32x4_unaligned;
+  const f32x4_unaligned *v = reinterpret_cast<const f32x4_unaligned *>(x);
+  const uint32_t vectors = vocabulary / 4u;
+  constexpr uint32_t kAhead = 8;
+  for (uint32_t base = tid; base < vectors; base += kAhead * kEndThreads) {
+    f32x4_unaligned held[kAhead];
+#pragma unroll
+    for (uint32_t i = 0; i < kAhead; ++i) {
+      const uint32_t at = base + i * kEndThreads;
+      held[i] = at < vectors ? v[at] : f32x4_unaligned{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < kAhead; ++i)
+#pragma unroll
+      for (uint32_t e = 0; e < 4; ++e) take(held[i][e], 4u * (base + i * kEndThreads) + e);
+  }
+  if (tid < vocabulary % 4u) take(x[4u * vectors + tid], 4u * vectors + tid);
+}
+__device__ __forceinline__ uint32_t end_bin(float value, float maximum, float inverse) {
+  return uint32_t(min(int((maximum - value) * inverse * kEndBinsPerFold), int(kEndBins) - 1));  // rises as the logit falls
+}
+
+__global__ __launch_bounds__(kEndThreads) void decode_sample_distribution_end(const float *__restrict__ logits,
+                                                                              const float *__restrict__ masses,
+                                                                              uint32_t *__restrict__ decisions, TargetSamplingParams p) {
+  __shared__ EndShared shared;
+  EndSelection &s = shared.selection;
+  const uint32_t row = blockIdx.x, tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, laneIndex = lane_of_row(p, row);
   if (!((p.truncating_mask >> laneIndex) & 1u)) return;
   const float temperature = p.temperature[laneIndex], inverse = 1.0f / temperature;
-  const Mass mass = row_mass(masses, row, inverse);
   const float *x = logits + size_t(row) * p.logits_stride;
   const float minP = p.min_p[laneIndex], topP = p.top_p[laneIndex];
   const uint32_t topK = p.top_k[laneIndex];
-  OrderEnd end{0u, 0u};
-  // Everything, and what min_p keeps: the tokens at or above the logit that weighs min_p of the heaviest.
-  const uint32_t lowest = minP > 0.f ? logit_key(fminf(mass.maximum + temperature * logf(minP), mass.maximum)) : kLowestKey;
-  end_histogram(x, p.vocabulary, mass, inverse, end, [&](uint32_t, uint32_t key) { return key >= lowest ? 1u : 0u; }, scratch, tid);
-  Measure kept{scratch.binCount[1], scratch.binMass[1]};
-  const uint32_t admitted = scratch.binCount[0] + scratch.binCount[1];
+  const float maximum = wave_max(masses[2u * (row * SAMPLING_SHARDS + lane % SAMPLING_SHARDS)]);
+  // what min_p keeps: the tokens at or above the logit that weighs min_p of the heaviest
+  const uint32_t lowest = minP > 0.f ? logit_key(fminf(maximum + temperature * logf(minP), maximum)) : kLowestKey;
+  for (uint32_t b = tid; b < kEndBins; b += kEndThreads) s.bins[b] = 0;
+  if (wave == 0) {
+    const float total = row_mass(masses, row, inverse).sum;
+    if (lane == 0) {
+      s.total = total;
+      s.selectable = s.gathered = s.candidates = 0;
+      s.cut = kEndBins - 1u;
+    }
+  }
   __syncthreads();
-  if (minP > 0.f && kept.count < admitted) end = {lowest, 0xFFFFFFFFu};
-  if (topK && topK < kept.count) end = select_last<false>(x, p.vocabulary, mass, inverse, end, topK - 1u, 0.f, kept, scratch, tid);
-  if (topP < 1.0f) end = select_last<true>(x, p.vocabulary, mass, inverse, end, 0u, topP * kept.mass, kept, scratch, tid);
+  uint32_t selectable = 0;
+  end_scan(x, p.vocabulary, tid, [&](float value, uint32_t) {
+    if (unselectable(value)) return;
+    ++selectable;
+    if (logit_key(value) >= lowest) atomicAdd(&s.bins[end_bin(value, maximum, inverse)], 1u);
+  });
+  selectable = wave_sum(selectable);
+  if (lane == 0) atomicAdd(&s.selectable, selectable);
+  __syncthreads();
+  // The first bin that ends past top_k tokens, or past a mass that exceeds top_p of the row's, a token of bin b weighing
+  // at least exp(-(b + 1) / 16); a nucleus of what min_p leaves needs the mass of all of it.
+  if (wave == 0) {
+    uint32_t count[kEndBins / 64u], sum = 0;
+    float mass[kEndBins / 64u], massSum = 0.f;
+#pragma unroll
+    for (uint32_t i = 0; i < kEndBins / 64u; ++i) {
+      const uint32_t b = lane * (kEndBins / 64u) + i, c = s.bins[b];
+      sum += c;
+      massSum += b + 1u < kEndBins ? float(c) * expf(-float(b + 1u) / kEndBinsPerFold) * 0.999f : 0.f;
+      count[i] = sum;
+      mass[i] = massSum;
+    }
+    uint32_t before = sum;
+    float massBefore = massSum;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t c = uint32_t(__shfl_up(int(before), o, 64));
+      const float m = __shfl_up(massBefore, o, 64);
+      if (int(lane) >= o) {
+        before += c;
+        massBefore += m;
+      }
+    }
+    const uint32_t all = uint32_t(__shfl(int(before), 63, 64));
+    before -= sum;
+    massBefore -= massSum;
+    const bool byCount = topK && topK < all, byMass = !byCount && minP <= 0.f && topP < 1.0f;
+    uint32_t cut = kEndBins - 1u;
+#pragma unroll
+    for (int i = int(kEndBins / 64u) - 1; i >= 0; --i) {
+      const bool past = byCount ? before + count[i] >= topK : byMass && massBefore + mass[i] > 1.001f * topP * s.total;
+      if (past) cut = lane * (kEndBins / 64u) + uint32_t(i);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) cut = min(cut, uint32_t(__shfl_xor(int(cut), o, 64)));
+    if (lane == cut / (kEndBins / 64u)) {
+      uint32_t upTo = 0;
+#pragma unroll
+      for (uint32_t i = 0; i < kEndBins / 64u; ++i) upTo = i == cut % (kEndBins / 64u) ? before + count[i] : upTo;
+      s.cut = cut;
+      s.candidates = upTo;
+    }
+    if (lane == 0) s.keep = all;
+  }
+  __syncthreads();
+  const uint32_t all = s.keep, admitted = s.selectable, candidates = s.candidates, cut = s.cut;
+  const float rowTotal = s.total;
+  const bool minCuts = minP > 0.f && all < admitted;
+  OrderEnd end{0u, 0u};
+  Measure kept{all, 0.f};
+  if (candidates <= kEndCandidates) {
+    const uint32_t slots = candidates <= 1u ? 1u : 1u << (32u - uint32_t(__builtin_clz(candidates - 1u)));
+    for (uint32_t i = candidates + tid; i < slots; i += kEndThreads) s.order[i] = 0;
+    end_scan(x, p.vocabulary, tid, [&](float value, uint32_t token) {
+      if (unselectable(value)) return;
+      const uint32_t key = logit_key(value);
+      if (key < lowest || end_bin(value, maximum, inverse) > cut) return;
+      s.order[atomicAdd(&s.gathered, 1u)] = uint64_t(key) << 32 | uint64_t(~token);
+    });
+    __syncthreads();
+    // bitonic, descending (the order they were gathered in leaves no trace: no two are equal)
+    for (uint32_t size = 2; size <= slots; size <<= 1)
+      for (uint32_t stride = size / 2; stride; stride >>= 1) {
+        for (uint32_t i = tid; i < slots / 2; i += kEndThreads) {
+          const uint32_t low = 2u * i - (i & (stride - 1u)), high = low + stride;
+          const uint64_t a = s.order[low], b = s.order[high];
+          if ((a < b) == ((low & size) == 0u)) {
+            s.order[low] = b;
+            s.order[high] = a;
+          }
+        }
+        __syncthreads();
+      }
+    const bool countCuts = topK && topK < all;
+    kept.count = countCuts ? topK : all;
+    // The running mass, a thread eight tokens in order; of the kept tokens past the candidates (a nucleus of the whole
+    // row) the row's total says what they weigh.
+    constexpr uint32_t kEach = kEndCandidates / kEndThreads;
+    const uint32_t listed = min(kept.count, candidates);
+    float mine[kEach], sum = 0.f;
+#pragma unroll
+    for (uint32_t i = 0; i < kEach; ++i) {
+      const uint32_t at = tid * kEach + i;
+      sum += at < listed ? expf((key_logit(uint32_t(s.order[at] >> 32)) - maximum) * inverse) : 0.f;
+      mine[i] = sum;
+    }
+    float before = sum;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const float m = __shfl_up(before, o, 64);
+      if (int(lane) >= o) before += m;
+    }
+    if (lane == 63u) s.waveMass[wave] = before;
+    if (tid == 0) s.keep = 0xFFFFFFFFu;
+    __syncthreads();
+    before -= sum;
+    float base = 0.f, total = 0.f;
+    for (uint32_t w = 0; w < kEndThreads / 64u; ++w) {
+      if (w == wave) base = total;
+      total += s.waveMass[w];
+    }
+    kept.mass = candidates < kept.count ? rowTotal : total;
+    const float nucleus = topP * kept.mass;
+    if (topP < 1.0f) {
+#pragma unroll
+      for (int i = int(kEach) - 1; i >= 0; --i) {
+        const uint32_t at = tid * kEach + uint32_t(i);
+        // (a running mass that rounding turned back does not end the nucleus twice: the first token past it does)
+        if (at < listed && base + (before + mine[i]) > nucleus) atomicMin(&s.keep, at + 1u);
+      }
+    }
+    __syncthreads();
+    const uint32_t nucleusEnd = s.keep;
+    const bool massCuts = nucleusEnd != 0xFFFFFFFFu;
+    if (massCuts) kept.count = nucleusEnd;
+    if (minCuts) end = {lowest, 0xFFFFFFFFu};
+    if (countCuts || massCuts) {
+      const uint64_t last = s.order[kept.count - 1u];
+      const uint32_t key = uint32_t(last >> 32);
+      // every token of the last one's key is among the candidates
+      const bool tied = kept.count < candidates && uint32_t(s.order[kept.count] >> 32) == key;
+      end = {key, tied ? ~uint32_t(last) : 0xFFFFFFFFu};
+    }
+    if (massCuts && tid == (nucleusEnd - 1u) / kEach) {
+      float at = 0.f;
+#pragma unroll
+      for (uint32_t i = 0; i < kEach; ++i) at = i == (nucleusEnd - 1u) % kEach ? mine[i] : at;
+      s.total = base + (before + at);
+    }
+    __syncthreads();
+    if (massCuts) kept.mass = s.total;
+  } else {
+    EndScratch &scratch = shared.descent;
+    __syncthreads();
+    const Mass mass{maximum, rowTotal};
+    end_histogram(x, p.vocabulary, mass, inverse, end, [&](uint32_t, uint32_t key) { return key >= lowest ? 1u : 0u; }, scratch, tid);
+    kept = {scratch.binCount[1], scratch.binMass[1]};
+    __syncthreads();
+    if (minCuts) end = {lowest, 0xFFFFFFFFu};
+    if (topK && topK < kept.count) end = select_last<false>(x, p.vocabulary, mass, inverse, end, topK - 1u, 0.f, kept, scratch, tid);
+    if (topP < 1.0f) end = select_last<true>(x, p.vocabulary, mass, inverse, end, 0u, topP * kept.mass, kept, scratch, tid);
+  }
   if (tid == 0) {
     uint32_t *words = decisions + size_t(row) * SAMPLING_DECISION_WORDS;
     words[SAMPLING_END_KEY] = end.key;
@@ -732,8 +937,14 @@ __global__ __launch_bounds__(64) void decode_sample_draw(const float *__restrict
   const Kept kept = row_kept(masses, decisions, row, inverse, (p.truncating_mask >> laneIndex) & 1u);
   const float *x = logits + size_t(row) * p.logits_stride, *q = draft + size_t(row) * p.logits_stride;
   const float *r = ranges + row * SAMPLING_RANGES;
+  // the ranges in LDS: the sums walk them in order without a trip to memory each
+  __shared__ float weights[SAMPLING_RANGES];
+#pragma unroll
+  for (uint32_t i = 0; i < SAMPLING_RANGES / 64u; ++i) weights[lane + 64u * i] = r[lane + 64u * i];
+  __syncthreads();
   float total = 0.f;
-  for (uint32_t j = 0; j < SAMPLING_RANGES; ++j) total += r[j];
+#pragma unroll 32
+  for (uint32_t j = 0; j < SAMPLING_RANGES; ++j) total += weights[j];
   if (!(total > 0.f)) {
     if (lane == 0) tokens[row] = SAMPLING_NO_TOKEN;
     return;
@@ -744,10 +955,12 @@ __global__ __launch_bounds__(64) void decode_sample_draw(const float *__restrict
   float before = 0.f, lastBefore = 0.f;
   {
     float cumulative = 0.f;
-    for (uint32_t j = 0; j < SAMPLING_RANGES && hit == SAMPLING_RANGES; ++j) {
-      if (r[j] > 0.f) { lastWeighted = j; lastBefore = cumulative; }
-      if (point < cumulative + r[j]) { hit = j; before = cumulative; }
-      cumulative += r[j];
+#pragma unroll 32
+    for (uint32_t j = 0; j < SAMPLING_RANGES; ++j) {
+      const float w = weights[j];
+      if (w > 0.f) { lastWeighted = j; lastBefore = cumulative; }
+      if (hit == SAMPLING_RANGES && point < cumulative + w) { hit = j; before = cumulative; }
+      cumulative += w;
     }
   }
   if (hit == SAMPLING_RANGES) { hit = lastWeighted; before = lastBefore; }
@@ -762,6 +975,7 @@ __global__ __launch_bounds__(64) void decode_sample_draw(const float *__restrict
   }
   uint32_t chunk = 64, lastChunk = 0;
   float chunkBefore = 0.f, lastChunkBefore = 0.f, cumulative = 0.f;
+#pragma unroll
   for (int l = 0; l < 64; ++l) {
     const float c = __shfl(sum, l, 64);
     if (c > 0.f) { lastChunk = uint32_t(l); lastChunkBefore = cumulative; }
@@ -770,19 +984,22 @@ __global__ __launch_bounds__(64) void decode_sample_draw(const float *__restrict
   }
   if (chunk == 64) { chunk = lastChunk; chunkBefore = lastChunkBefore; }
   target -= chunkBefore;
-  if (lane == 0) {
-    uint32_t selected = SAMPLING_NO_TOKEN, lastToken = SAMPLING_NO_TOKEN;
-    float walked = 0.f;
-    for (uint32_t i = 0; i < per; ++i) {
-      const uint32_t token = begin + chunk * per + i;
-      if (token >= end) break;
-      const float w = residual_of(x[token], token, rejected ? q[token] : 0.f, kept, inverse, rejected);
+  // The chunk's tokens, weighed a lane each and walked in id order.
+  uint32_t selected = SAMPLING_NO_TOKEN, lastToken = SAMPLING_NO_TOKEN;
+  float walked = 0.f;
+  for (uint32_t i0 = 0; i0 < per; i0 += 64u) {
+    const uint32_t own = begin + chunk * per + i0 + lane;
+    const bool live = i0 + lane < per && own < end;
+    const float weight = live ? residual_of(x[own], own, rejected ? q[own] : 0.f, kept, inverse, rejected) : 0.f;
+    for (uint32_t i = 0; i < 64u && i0 + i < per; ++i) {
+      const float w = __shfl(weight, int(i), 64);
+      const uint32_t token = begin + chunk * per + i0 + i;
       if (w > 0.f) lastToken = token;
       walked += w;
       if (selected == SAMPLING_NO_TOKEN && w > 0.f && target < walked) selected = token;
     }
-    tokens[row] = selected != SAMPLING_NO_TOKEN ? selected : lastToken;
   }
+  if (lane == 0) tokens[row] = selected != SAMPLING_NO_TOKEN ? selected : lastToken;
 }
 SP_REGISTER_KERNEL("decode_sample_draw", &decode_sample_draw);
 

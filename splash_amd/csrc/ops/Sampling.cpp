@@ -99,7 +99,7 @@ void Sampling::addVerify(hip::CommandGraph &graph, const SamplingBuffers &b, uin
   }
   graph.add("decode_sample_mass_sharded", {b.logits, b.masses}, params, {rows * SAMPLING_SHARDS, 1, 1}, {SAMPLING_THREADS, 1, 1});
   if (params.truncating_mask)
-    graph.add("decode_sample_distribution_end", {b.logits, b.masses, b.decisions}, params, {rows, 1, 1}, {SAMPLING_THREADS, 1, 1});
+    graph.add("decode_sample_distribution_end", {b.logits, b.masses, b.decisions}, params, {rows, 1, 1}, {1024, 1, 1});
   // with candidate children no full-vocabulary draft distribution is read: the logits stand in for its binding
   graph.add("decode_sample_residual_ranges",
             {b.logits, children ? b.logits : b.draftProbabilities, b.masses, b.uniforms, b.treeRows, b.inputTokens, b.ranges, b.decisions},

@@ -339,6 +339,41 @@ def test_truncated_distributions_match_oracle(backend, ties):
     assert checked >= 12
 
 
+@pytest.mark.parametrize("V", [5, 1023, 8193, 40001])
+def test_distribution_ends_at_the_candidate_limit(backend, V):
+    """decode_sample_distribution_end sorts up to 8192 candidates in LDS and descends digit by digit past them: ends on
+    either side of that limit, at the smallest and at odd vocabularies, flat rows whose nucleus is most of the row, and
+    runs of equal logits across the end."""
+    print(f"case distribution ends V={V}", flush=True)
+    rng = np.random.default_rng(V)
+    # (temperature, min_p, top_k, top_p); a lane of two rows each
+    policies = [(0.7, 0.0, 8192, 1.0), (0.7, 0.0, 8193, 0.999), (3.0, 0.0, 0, 0.95), (0.8, 0.02, 64, 0.95), (2.0, 1e-6, 0, 1.0), (0.7, 0.0, 2, 1.0)]
+    lanes = [(2 * i, 2) for i in range(len(policies))]
+    rows = 2 * len(policies)
+    logits = (rng.standard_normal((rows, V)) * 1.5).astype(np.float32)
+    logits[1::2] = np.round(logits[1::2] * 4) / 4
+    logits[::3, rng.random(V) < 0.05] = -np.inf
+    logits[:, 0] = 1.0
+    draft = np.full((rows, V), 1.0 / V, np.float32)
+    tokens, tree = np.zeros(rows, np.uint32), ops.chain_tree_rows([n for _, n in lanes])
+    b = sampling_buffers(backend, rows, V, logits, draft, rng.random((rows, 2)).astype(np.float32), tokens, tree)
+    g = splash_amd.CommandGraph()
+    ops.Sampling.add_verify(g, b, V, V, lanes, policies)
+    backend.run(g)
+    words = b["decisions"].download(np.uint32).reshape(rows, 8)
+    checked = 0
+    for (first, n), (T, min_p, top_k, top_p) in zip(lanes, policies):
+        if not (min_p > 0 or (top_k and top_k < V) or top_p < 1):
+            continue
+        for r in range(first, first + n):
+            key, last, mass, count, close_end = orc.distribution_end(logits[r], T, min_p, top_k, top_p)
+            if close_end > 1e-5:
+                assert (words[r, 2], words[r, 3], words[r, 5]) == (key, last, count), (r, top_k, top_p)
+                assert abs(words[r, 4:5].view(np.float32)[0] - mass) <= 1e-5 * mass
+                checked += 1
+    assert checked >= 6
+
+
 def test_constraint_masks_and_stop_exclusion(backend):
     """TargetRow::admits (sampling.metal:42-46): a constrained lane's rows select only tokens of their mask rows, a lane
     that ignores end-of-sequence never a stop token, greedy or sampled; the other lanes' rows are untouched. The
