@@ -190,6 +190,64 @@ struct GgufPrefillParams {
   uint32_t reserved[3];
 };
 
+// THE WIDE TABLE of a chunk's rows: the fp16 operands of the wide projection (gguf_wide_*), `tiles` row tiles (whole
+// GGUF_WIDE_TILES of them) of K / 256 super-blocks each: per super-block nine 1024-byte operands, the eight groups'
+// values fp16 [64 lanes][8] in the order of the activation table, then the row sums' [64 lanes][8]: lane (r, kq) holds in
+// element g the part kq of the sum of row r's group g divided by 32 (three fp16 parts that add up to the fp32 sum; part 3
+// is zero). A row's values are its bf16 values times a power of two, 2^e, that brings its largest finite magnitude into
+// [2^14, 2^15), rounded to fp16: exact but for values more than 2^28 times smaller than that, which keep an absolute
+// error of 2^-40 of it. After the operands fp32 [16 tiles]: a row's 2^-e.
+#define GGUF_WIDE_TILES 8u             // row tiles a workgroup of the wide projection takes at most
+#define GGUF_WIDE_COLUMNS 128u         // and its columns (a gate/up pair: 64 of each)
+#define GGUF_WIDE_OPERANDS 9u          // 1024-byte operands a super-block of a row tile
+#define GGUF_WIDE_MAXIMUM_SPLITS 8u
+#if defined(__HIPCC__) || defined(__cplusplus)
+GGUF_INLINE uint32_t gguf_wide_tiles(uint32_t rows) {
+  return (gguf_row_tiles(rows) + GGUF_WIDE_TILES - 1u) / GGUF_WIDE_TILES * GGUF_WIDE_TILES;
+}
+GGUF_INLINE uint64_t gguf_wide_tile_bytes(uint32_t k) { return uint64_t(k / GGUF_BLOCK) * GGUF_WIDE_OPERANDS * 1024u; }
+GGUF_INLINE uint64_t gguf_wide_scales_offset(uint32_t k, uint32_t tiles) { return tiles * gguf_wide_tile_bytes(k); }
+GGUF_INLINE uint64_t gguf_wide_table_bytes(uint32_t k, uint32_t rows) {
+  const uint32_t tiles = gguf_wide_tiles(rows);
+  return gguf_wide_scales_offset(k, tiles) + tiles * GGUF_ROW_TILE * 4u;
+}
+#endif
+// gguf_wide_table: bf16 rows of up to 8192 inputs -> the wide table (_long: up to 32768); gguf_wide_table_norm: the rows'
+// RMS norm (weights bf16 [K]) on the way, bf16((x * inverse) * weight) as norm_rms writes it. Grid (64 * ceil(16 tiles /
+// 64)), 256 threads: a workgroup a row.
+struct GgufWideTableParams {
+  uint32_t input_size;
+  uint32_t rows;
+  uint32_t tiles;  // gguf_wide_tiles(rows)
+  uint32_t reserved;
+};
+// gguf_wide_<fmt>_{a,r,g,p} (and gguf_wide_staged_*, weights rounded once to half): a chunk of rows, a workgroup up to 128
+// of them x 128 columns. Binds up to three segments of one format (a gate/up pair: gate, up), the wide table, out and the
+// residual rows (any buffer when unused). _p writes fp32 partials of its part of K to out, [part][rows][out_stride], which
+// gguf_wide_reduce adds in part order. Grid: 8 * ceil(items / 8) workgroups of 256 threads, items = row_groups * splits *
+// column groups; workgroup b stands for item (b % 8) * (grid / 8) + b / 8, so that each of the eight dies takes
+// neighbouring items, which share weights (the row groups of a column group) and rows in its L2.
+struct GgufWideParams {
+  uint32_t input_size;
+  uint32_t rows;
+  uint32_t tiles;       // of the table
+  uint32_t row_groups;  // workgroups the row tiles are dealt over, evenly
+  uint32_t splits;      // parts of K (1 unless _p)
+  uint32_t out_stride;
+  uint32_t groups;      // column groups of GGUF_WIDE_COLUMNS over the segments
+  uint32_t cols[3];     // columns per segment: multiples of GGUF_WIDE_COLUMNS (gate/up: of half of it)
+  uint32_t offset[3];   // first destination column per segment
+  uint32_t reserved[3];
+};
+// gguf_wide_reduce_{a,r}: out = bf16(sum of the parts in order [+ residual]). Four columns a thread, grid
+// (ceil(rows * columns / 1024)), 256 threads.
+struct GgufWideReduceParams {
+  uint32_t rows;
+  uint32_t columns;
+  uint32_t splits;
+  uint32_t reserved;
+};
+
 // gguf_column_<fmt>_{a,a_f32,r,g}: one or two rows under the reference's column rule (its GgufColumnParams,
 // metal/abi/Gguf.h:45-55; GGUF_COLUMN_SPLITS parts of K there and here). Binds the tensor's image, a one-pass gate/up's
 // up image (the first is the gate's; the tensor's again otherwise), the rows (bf16 [rows][input_size]), out and the
@@ -309,6 +367,7 @@ struct GgufEmbedParams {
 static_assert(sizeof(GgufPrepareParams) == 16, "prepare parameters are 16 bytes on both sides");
 static_assert(sizeof(GgufDecodeParams) == 64, "decode parameters are 64 bytes on both sides");
 static_assert(sizeof(GgufChainLink) == 96 && sizeof(GgufChainParams) == 400, "chain parameters are 400 bytes on both sides");
+static_assert(sizeof(GgufWideParams) == 64, "wide parameters are 64 bytes on both sides");
 static_assert(sizeof(GgufDequantParams) == 8, "dequant parameters are 8 bytes on both sides");
 static_assert(sizeof(GgufEmbedParams) == 12, "embedding parameters are 12 bytes on both sides");
 #endif

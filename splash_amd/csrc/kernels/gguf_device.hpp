@@ -34,8 +34,8 @@ __device__ __forceinline__ uint32_t and_or(uint32_t a, uint32_t mask, uint32_t b
   asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(mask), "v"(base));
   return r;
 }
-template <bool High> __device__ __forceinline__ uint4 q4_operands(uint32_t wa, uint32_t wb) {
-  constexpr uint32_t kMask = 0x000F000Fu, kBase = 0x43004300u;  // bf16 0x4300 = 128, ulp 1
+template <bool High, uint32_t Base = 0x43004300u> __device__ __forceinline__ uint4 q4_operands(uint32_t wa, uint32_t wb) {
+  constexpr uint32_t kMask = 0x000F000Fu, kBase = Base;  // bf16 0x4300 = 128, ulp 1 (fp16 0x6400 = 1024, ulp 1)
   constexpr uint32_t s = High ? 4u : 0u;
   uint4 r;
   r.x = and_or(s ? wa >> s : wa, kMask, kBase);
@@ -46,9 +46,10 @@ template <bool High> __device__ __forceinline__ uint4 q4_operands(uint32_t wa, u
 }
 // The same for Q6_K: the low nibbles as Q4_K's, then the 2-bit high fields of pair v0..v0+3 of
 // the high-bits word (abi/Gguf.h) at bits 4..5 of each half.
-template <bool High, uint32_t V0> __device__ __forceinline__ uint4 q6_operands(uint32_t wa, uint32_t wb, uint32_t hw) {
+template <bool High, uint32_t V0, uint32_t Base = 0x43004300u>
+__device__ __forceinline__ uint4 q6_operands(uint32_t wa, uint32_t wb, uint32_t hw) {
   constexpr uint32_t kHigh = 0x00300030u;
-  uint4 r = q4_operands<High>(wa, wb);
+  uint4 r = q4_operands<High, Base>(wa, wb);
   auto with = [&](uint32_t v, uint32_t low) -> uint32_t {
     return and_or(2u * v > 4u ? hw >> (2u * v - 4u) : 2u * v < 4u ? hw << (4u - 2u * v) : hw, kHigh, low);
   };
@@ -61,9 +62,10 @@ template <bool High, uint32_t V0> __device__ __forceinline__ uint4 q6_operands(u
 
 // The same for Q5_K: the low nibbles as Q4_K's, then the fifth bits of registers R0 .. R0 + 3 of the record
 // half's fifth-bits word (abi/Gguf.h: bit r the low half's, bit 16 + r the high half's) at bit 4 of each half.
-template <bool High, uint32_t R0> __device__ __forceinline__ uint4 q5_operands(uint32_t wa, uint32_t wb, uint32_t hw) {
+template <bool High, uint32_t R0, uint32_t Base = 0x43004300u>
+__device__ __forceinline__ uint4 q5_operands(uint32_t wa, uint32_t wb, uint32_t hw) {
   constexpr uint32_t kFifth = 0x00100010u;
-  uint4 r = q4_operands<High>(wa, wb);
+  uint4 r = q4_operands<High, Base>(wa, wb);
   auto with = [&](uint32_t reg, uint32_t low) -> uint32_t {
     return and_or(reg > 4u ? hw >> (reg - 4u) : reg < 4u ? hw << (4u - reg) : hw, kFifth, low);
   };

@@ -1,0 +1,579 @@
+// The projections of a prompt chunk: many rows against a K-quant weight image (abi/Gguf.h), bound by the matrix cores.
+//
+// A 4-, 5- or 6-bit weight is d * (sc * code) - dmin * mn with an integer sc * code, which the decode kernels cannot use
+// (their bf16 operands hold eight bits) and so multiply every group's sum by its scale on the vector ALU: an fp32
+// multiply-add for every 32 products of an output, as long as the matrix cores take for them. fp16 holds eleven bits:
+// sc * code is at most 63 * 31 and exact, so a whole super-block of 256 inputs accumulates in the matrix cores and costs
+// an output one multiply-add by d, and the constant term one more MFMA against the rows' group sums and one by dmin. A
+// Q6_K product needs twelve bits: it is the rounded fp16 product plus the exact fp16 remainder, two MFMAs. The rows
+// enter as fp16 too, scaled by a power of two a row (the wide table), which keeps all eight bits of a bf16 value.
+//
+// Split: a wave owns 32 columns (a record of two column tiles each super-block, dequantized once in its registers) of
+// all of the workgroup's 128 rows, whose operands pass through LDS two groups at a time, double-buffered, one barrier
+// each. Two waves a SIMD (256 registers) overlap the conversion of one with the MFMAs of the other. At 2048 rows of the
+// 5120 x 2 x 25600 Q4_K gate/up pair a launch takes 1.35 ms (800 TFLOP/s of the projection's own operations; the 64-row
+// windows of the decode kernels took 2.38 ms), at 25600 x 5120 Q6_K 0.99 ms (2.2 ms): the matrix cores are busy 46 % and
+// 59 % of the cycles of a clock that the card's power limit holds at 2.1 and 1.8 GHz.
+#include "abi/Gguf.h"
+#include "backend/KernelRegistry.hpp"
+#include "kernels/gguf_records.hpp"
+
+namespace splash::kernels {
+
+typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
+typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
+__device__ __forceinline__ f16x2 as_f16x2(uint32_t v) { return __builtin_bit_cast(f16x2, v); }
+__device__ __forceinline__ uint32_t as_word(f16x2 v) { return __builtin_bit_cast(uint32_t, v); }
+__device__ __forceinline__ f16x8 as_f16x8(uint4 v) { return __builtin_bit_cast(f16x8, v); }
+__device__ __forceinline__ f16x2 both(float v) { return f16x2{_Float16(v), _Float16(v)}; }
+
+// ---------------------------------------------------------------------------------------------
+// The wide table.
+// ---------------------------------------------------------------------------------------------
+// A workgroup a row, whose values stay in registers from their one load to their stores: thread t holds the eight inputs of
+// quarter t % 4 of groups t / 4, 64 + t / 4, ... in `Held` pieces. The eight rows that share the table's 128-byte lines are
+// neighbours on one die (workgroup b runs on die b % 8), so that its L2 writes whole lines.
+template <bool Norm, uint32_t Held>
+__global__ __launch_bounds__(256) void gguf_wide_table(const uint16_t *__restrict__ input, const uint16_t *__restrict__ weight,
+                                                       uint8_t *__restrict__ table, GgufWideTableParams p) {
+  __shared__ float scratch[8];
+  const uint32_t die = blockIdx.x % 8u, slot = blockIdx.x / 8u, row = (slot / 8u * 8u + die) * 8u + slot % 8u;
+  if (row >= 16u * p.tiles) return;
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, tile = row / 16u, r = row % 16u;
+  const uint32_t kq = tid & 3u, groups = p.input_size / 32u, held = (groups + 63u) / 64u;
+  const bool live = row < p.rows;
+  uint4 *values = reinterpret_cast<uint4 *>(table + tile * gguf_wide_tile_bytes(p.input_size));
+  // piece i: inputs 4 kq .. + 3, then 16 + 4 kq .. + 3 of group 64 i + t / 4
+  auto groupOf = [&](uint32_t i) { return 64u * i + (tid >> 2); };
+  auto load = [&](const uint16_t *from, uint32_t i) {
+    const uint32_t g = groupOf(i);
+    if (!live || g >= groups) return make_uint4(0u, 0u, 0u, 0u);
+    const uint2 a = *reinterpret_cast<const uint2 *>(from + 32u * g + 4u * kq), b = *reinterpret_cast<const uint2 *>(from + 32u * g + 16u + 4u * kq);
+    return make_uint4(a.x, a.y, b.x, b.y);
+  };
+  uint4 v[Held];
+#pragma unroll
+  for (uint32_t i = 0; i < Held; ++i)
+    if (i < held) v[i] = load(input + size_t(live ? row : 0u) * p.input_size, i);
+  if constexpr (Norm) {
+    uint4 w[Held];
+#pragma unroll
+    for (uint32_t i = 0; i < Held; ++i)
+      if (i < held) w[i] = load(weight, i);
+    float sum = 0.f;
+#pragma unroll
+    for (uint32_t i = 0; i < Held; ++i)
+      if (i < held) {
+        const uint32_t words[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float low = bf16_bits_to_float(words[e] & 0xFFFFu), high = bf16_bits_to_float(words[e] >> 16);
+          sum += low * low;
+          sum += high * high;
+        }
+      }
+    sum = wave_sum(sum);
+    if (lane == 0) scratch[wave] = sum;
+    __syncthreads();
+    const float inverse = 1.0f / sqrtf((((scratch[0] + scratch[1]) + scratch[2]) + scratch[3]) / float(p.input_size) + 1e-6f);
+#pragma unroll
+    for (uint32_t i = 0; i < Held; ++i)
+      if (i < held) {
+        const uint32_t words[4] = {v[i].x, v[i].y, v[i].z, v[i].w}, weights[4] = {w[i].x, w[i].y, w[i].z, w[i].w};
+        uint32_t out[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t low = float_to_bf16_bits((bf16_bits_to_float(words[e] & 0xFFFFu) * inverse) * bf16_bits_to_float(weights[e] & 0xFFFFu));
+          const uint32_t high = float_to_bf16_bits((bf16_bits_to_float(words[e] >> 16) * inverse) * bf16_bits_to_float(weights[e] >> 16));
+          out[e] = low | (high << 16);
+        }
+        v[i] = make_uint4(out[0], out[1], out[2], out[3]);
+      }
+  }
+  uint32_t largest = 0;
+#pragma unroll
+  for (uint32_t i = 0; i < Held; ++i)
+    if (i < held) {
+      const uint32_t words[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t low = words[e] & 0x7FFFu, high = (words[e] >> 16) & 0x7FFFu;
+        if (low < 0x7F80u) largest = max(largest, low);   // (an infinity or NaN stays what it is)
+        if (high < 0x7F80u) largest = max(largest, high);
+      }
+    }
+  largest = wave_max(largest);
+  if (lane == 0) scratch[4u + wave] = __uint_as_float(largest);
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 4; ++w) largest = max(largest, __float_as_uint(scratch[4 + w]));
+  // 2^e, e = 14 - the exponent of the largest magnitude (a row of zeros or of subnormals: the largest 2^e there is)
+  const uint32_t exponent = max(largest >> 7, 15u);
+  const float scale = __uint_as_float((141u + 127u - exponent) << 23), inverseScale = __uint_as_float((exponent - 14u) << 23);
+#pragma unroll
+  for (uint32_t i = 0; i < Held; ++i)
+    if (i < held) {
+      const uint32_t g = groupOf(i);
+      const uint32_t words[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+      float f[8];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        f[2 * e] = bf16_bits_to_float(words[e] & 0xFFFFu) * scale;
+        f[2 * e + 1] = bf16_bits_to_float(words[e] >> 16) * scale;
+      }
+      // inputs 4 kq + {0, 2, 1, 3} of each half group
+      auto pair = [](float a, float b) { return f16x2{_Float16(a), _Float16(b)}; };
+      const f16x2 operand[4] = {pair(f[0], f[2]), pair(f[1], f[3]), pair(f[4], f[6]), pair(f[5], f[7])};
+      if (g < groups)
+        values[(size_t(g >> 3) * GGUF_WIDE_OPERANDS + (g & 7u)) * 64u + kq * 16u + r] =
+            make_uint4(as_word(operand[0]), as_word(operand[1]), as_word(operand[2]), as_word(operand[3]));
+      // the group's sum of what the operands hold, in three fp16 parts
+      float s = 0.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s += float(operand[e].x) + float(operand[e].y);
+      s += __shfl_xor(s, 1, 64);
+      s += __shfl_xor(s, 2, 64);
+      s *= 0.03125f;
+      const float first = float(_Float16(s)), second = float(_Float16(s - first)), third = float(_Float16((s - first) - second));
+      const float mine = kq == 0u ? first : kq == 1u ? second : kq == 2u ? third : 0.f;
+      // element g % 8 of the super-block's operand: the halves of eight threads into one 16-byte store
+      const uint32_t part = as_word(f16x2{_Float16(mine), _Float16(0.f)}) & 0xFFFFu;
+      const uint32_t two = part | (uint32_t(__shfl_down(int(part), 4, 64)) << 16);
+      const uint32_t b = uint32_t(__shfl_down(int(two), 8, 64)), c = uint32_t(__shfl_down(int(two), 16, 64)), d = uint32_t(__shfl_down(int(two), 24, 64));
+      if ((g & 7u) == 0 && g < groups) values[(size_t(g >> 3) * GGUF_WIDE_OPERANDS + 8u) * 64u + kq * 16u + r] = make_uint4(two, b, c, d);
+    }
+  if (tid == 0) reinterpret_cast<float *>(table + gguf_wide_scales_offset(p.input_size, p.tiles))[row] = inverseScale;
+}
+SP_REGISTER_KERNEL("gguf_wide_table", (&gguf_wide_table<false, 4>));
+SP_REGISTER_KERNEL("gguf_wide_table_long", (&gguf_wide_table<false, 16>));
+SP_REGISTER_KERNEL("gguf_wide_table_norm", (&gguf_wide_table<true, 4>));
+
+// ---------------------------------------------------------------------------------------------
+// The wide projection.
+// ---------------------------------------------------------------------------------------------
+#define GGUF_WIDE_PLAIN 0u
+#define GGUF_WIDE_RESIDUAL 1u
+#define GGUF_WIDE_GATE_UP 2u
+#define GGUF_WIDE_PARTIAL 3u
+
+// A record as it passes through a wave: half of its nibbles at a time, what they share with the other half kept.
+template <uint32_t FMT> struct WideRecord {
+  uint4 codes[2];     // the nibbles of stages 0 and 1, of stages 2 and 3
+  uint4 meta;         // Q4_K, Q5_K: d, dmin and the packed scales; Q6_K: the scales
+  uint4 high;         // Q6_K: the high bits
+  uint2 fifth;        // Q5_K: the fifth bits
+  uint32_t d;         // Q6_K
+};
+// What a record's first two stages need, and (`late`) the bits its last stage reads too.
+template <uint32_t FMT> __device__ __forceinline__ void load_first(WideRecord<FMT> &rec, Resource r, uint32_t mine, uint32_t lane) {
+  const uint32_t record = mine - 16u * lane, c = lane & 15u;
+  rec.codes[0] = load128<kStreamOnce>(r, mine);
+  rec.meta = load128<kStreamOnce>(r, record + Cursor<FMT>::kColumnPart + 16u * c);
+  if constexpr (FMT == GGUF_FMT_Q6K) rec.d = __builtin_amdgcn_raw_buffer_load_b16(r, int(record + GGUF_Q6K_D + 2u * c), 0, kStreamOnce);
+}
+template <uint32_t FMT> __device__ __forceinline__ void load_late(WideRecord<FMT> &rec, Resource r, uint32_t mine, uint32_t lane) {
+  if constexpr (FMT == GGUF_FMT_Q6K) rec.high = load128<kStreamOnce>(r, mine + GGUF_Q6K_HIGH);
+  if constexpr (FMT == GGUF_FMT_Q5K) {
+    const u32x2 fifth = __builtin_amdgcn_raw_buffer_load_b64(r, int(mine - 8u * lane + GGUF_Q5K_HIGH), 0, kStreamOnce);
+    rec.fifth = make_uint2(fifth.x, fifth.y);
+  }
+}
+// What its operands need of `meta` once a super-block.
+template <uint32_t FMT> struct WideScales {
+  float d, dmin;
+  uint32_t sc_lo, sc_hi, mn_lo, mn_hi;   // Q6_K: the sixteen signed scales
+};
+__device__ __forceinline__ uint32_t byte_pair(uint32_t word, uint32_t first, uint32_t second) {   // fp16 1024 + byte, of two bytes
+  return __builtin_amdgcn_perm(0x64646464u, word, 0x04000400u | first | (second << 16));
+}
+template <uint32_t FMT> __device__ __forceinline__ WideScales<FMT> wide_scales(const WideRecord<FMT> &rec) {
+  if constexpr (FMT == GGUF_FMT_Q6K) {
+    // signed bytes: byte ^ 0x80 is scale + 128
+    return {half_bits_to_float(rec.d), 0.f, rec.meta.x ^ 0x80808080u, rec.meta.y ^ 0x80808080u, rec.meta.z ^ 0x80808080u, rec.meta.w ^ 0x80808080u};
+  } else {
+    const Q4KScales q = q4k_scales(rec.meta);
+    return {q.d, -32.f * q.dmin, q.sc_lo, q.sc_hi, q.mn_lo, q.mn_hi};   // (the sums are stored divided by 32)
+  }
+}
+// The mins of the eight groups as fp16: the constant term's operand.
+template <uint32_t FMT> __device__ __forceinline__ uint4 wide_mins(const WideScales<FMT> &s) {
+  const f16x2 k = both(1024.f);
+  return make_uint4(as_word(as_f16x2(byte_pair(s.mn_lo, 0, 1)) - k), as_word(as_f16x2(byte_pair(s.mn_lo, 2, 3)) - k),
+                    as_word(as_f16x2(byte_pair(s.mn_hi, 0, 1)) - k), as_word(as_f16x2(byte_pair(s.mn_hi, 2, 3)) - k));
+}
+// Groups 2 S and 2 S + 1 of a record: sc * code as fp16 (Q6_K: rounded, and what the rounding left).
+template <uint32_t FMT> struct WideOperands {
+  uint4 high[2];
+  uint4 low[FMT == GGUF_FMT_Q6K ? 2 : 1];
+};
+template <uint32_t FMT, uint32_t S>
+__device__ __forceinline__ WideOperands<FMT> wide_operands(const WideRecord<FMT> &rec, const WideScales<FMT> &sc) {
+  WideOperands<FMT> out;
+  const uint4 n = rec.codes[S >> 1];
+  const uint32_t wa = S & 1u ? n.z : n.x, wb = S & 1u ? n.w : n.y;
+  if constexpr (FMT == GGUF_FMT_Q4K) {
+    // a nibble at bits 0..3 is 1024 + code under fp16's 2^10, one at bits 4..7 is 64 + code under 2^6
+    const uint32_t words[4] = {wa, wa >> 8, wb, wb >> 8};
+    const uint32_t word = S < 2 ? sc.sc_lo : sc.sc_hi;
+    const f16x2 first = as_f16x2(byte_pair(word, (2u * S) & 3u, (2u * S) & 3u)) - both(1024.f);
+    const f16x2 second = as_f16x2(byte_pair(word, (2u * S + 1u) & 3u, (2u * S + 1u) & 3u)) - both(1024.f);
+    const f16x2 firstOff = first * both(-1024.f), secondOff = second * both(-64.f);
+    uint32_t a[4], b[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      a[i] = as_word(__builtin_elementwise_fma(as_f16x2(and_or(words[i], 0x000F000Fu, 0x64006400u)), first, firstOff));
+      b[i] = as_word(__builtin_elementwise_fma(as_f16x2(and_or(words[i], 0x00F000F0u, 0x54005400u)), second, secondOff));
+    }
+    out.high[0] = make_uint4(a[0], a[1], a[2], a[3]);
+    out.high[1] = make_uint4(b[0], b[1], b[2], b[3]);
+  } else if constexpr (FMT == GGUF_FMT_Q5K) {
+    const uint32_t fifth = S < 2 ? rec.fifth.x : rec.fifth.y;
+    const uint4 code[2] = {q5_operands<false, 8u * (S & 1u), 0x64006400u>(wa, wb, fifth), q5_operands<true, 8u * (S & 1u) + 4u, 0x64006400u>(wa, wb, fifth)};
+    const uint32_t word = S < 2 ? sc.sc_lo : sc.sc_hi;
+#pragma unroll
+    for (uint32_t i = 0; i < 2; ++i) {
+      const f16x2 scale = as_f16x2(byte_pair(word, (2u * S + i) & 3u, (2u * S + i) & 3u)) - both(1024.f), off = scale * both(-1024.f);
+      const uint32_t words[4] = {code[i].x, code[i].y, code[i].z, code[i].w};
+      uint32_t a[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) a[e] = as_word(__builtin_elementwise_fma(as_f16x2(words[e]), scale, off));
+      out.high[i] = make_uint4(a[0], a[1], a[2], a[3]);
+    }
+  } else {
+    const uint32_t hw = S == 0 ? rec.high.x : S == 1 ? rec.high.y : S == 2 ? rec.high.z : rec.high.w;
+    const uint4 code[2] = {q6_operands<false, 0, 0x64006400u>(wa, wb, hw), q6_operands<true, 4, 0x64006400u>(wa, wb, hw)};
+    const uint32_t word = S == 0 ? sc.sc_lo : S == 1 ? sc.sc_hi : S == 2 ? sc.mn_lo : sc.mn_hi;   // of the four 16-input blocks
+#pragma unroll
+    for (uint32_t i = 0; i < 2; ++i) {
+      const uint32_t words[4] = {code[i].x, code[i].y, code[i].z, code[i].w};
+      uint32_t a[4], b[4];
+#pragma unroll
+      for (uint32_t e = 0; e < 4; ++e) {
+        const uint32_t block = 2u * i + (e >> 1);
+        const f16x2 scale = as_f16x2(byte_pair(word, block, block)) - both(1152.f);
+        const f16x2 value = as_f16x2(words[e]) - both(1056.f);   // code - 32
+        const f16x2 product = value * scale;
+        a[e] = as_word(product);
+        b[e] = as_word(__builtin_elementwise_fma(value, scale, -product));   // exact: an integer below the product's last bit
+      }
+      out.high[i] = make_uint4(a[0], a[1], a[2], a[3]);
+      out.low[i] = make_uint4(b[0], b[1], b[2], b[3]);
+    }
+  }
+  return out;
+}
+
+// The same groups' weights rounded once to half: the staged rule (gguf_linear.hip), whole values that need no scale after.
+template <uint32_t FMT, uint32_t S>
+__device__ __forceinline__ WideOperands<FMT> wide_staged_operands(const WideRecord<FMT> &rec, const WideScales<FMT> &sc) {
+  WideOperands<FMT> out{};
+  const uint4 n = rec.codes[S >> 1];
+  const uint32_t wa = S & 1u ? n.z : n.x, wb = S & 1u ? n.w : n.y;
+  uint4 code[2];
+  if constexpr (FMT == GGUF_FMT_Q4K) {
+    code[0] = q4_operands<false, 0x64006400u>(wa, wb);
+    code[1] = q4_operands<true, 0x64006400u>(wa, wb);
+  } else if constexpr (FMT == GGUF_FMT_Q5K) {
+    const uint32_t fifth = S < 2 ? rec.fifth.x : rec.fifth.y;
+    code[0] = q5_operands<false, 8u * (S & 1u), 0x64006400u>(wa, wb, fifth);
+    code[1] = q5_operands<true, 8u * (S & 1u) + 4u, 0x64006400u>(wa, wb, fifth);
+  } else {
+    const uint32_t hw = S == 0 ? rec.high.x : S == 1 ? rec.high.y : S == 2 ? rec.high.z : rec.high.w;
+    code[0] = q6_operands<false, 0, 0x64006400u>(wa, wb, hw);
+    code[1] = q6_operands<true, 4, 0x64006400u>(wa, wb, hw);
+  }
+#pragma unroll
+  for (uint32_t i = 0; i < 2; ++i) {
+    const uint32_t words[4] = {code[i].x, code[i].y, code[i].z, code[i].w};
+    uint32_t a[4];
+#pragma unroll
+    for (uint32_t e = 0; e < 4; ++e) {
+      f16x2 half;
+      if constexpr (FMT == GGUF_FMT_Q6K) {
+        const uint32_t word = S == 0 ? sc.sc_lo : S == 1 ? sc.sc_hi : S == 2 ? sc.mn_lo : sc.mn_hi;
+        const f16x2 value = as_f16x2(words[e]) - both(1056.f);
+        const float s = sc.d * (byte_of(word, 2u * i + (e >> 1)) - 128.f);
+        half = f16x2{_Float16(s * float(value.x)), _Float16(s * float(value.y))};
+      } else {
+        const uint32_t g = 2u * S + i;
+        const f16x2 value = as_f16x2(words[e]) - both(1024.f);
+        const float s = sc.d * byte_of(g < 4 ? sc.sc_lo : sc.sc_hi, g & 3u), m = 0.03125f * sc.dmin * byte_of(g < 4 ? sc.mn_lo : sc.mn_hi, g & 3u);
+        half = f16x2{_Float16(__fmaf_rn(s, float(value.x), m)), _Float16(__fmaf_rn(s, float(value.y), m))};
+      }
+      a[e] = as_word(half);
+    }
+    out.high[i] = make_uint4(a[0], a[1], a[2], a[3]);
+  }
+  return out;
+}
+
+template <uint32_t T> struct WideShared {
+  uint4 rows[2][(T + 1) / 2 * 2][2][64];   // [buffer][row tile][group][lane]
+  uint4 sums[(T + 3) / 4 * 4][64];
+};
+
+// T: the row tiles a workgroup computes, at least those it takes (a tile past them multiplies zeros).
+template <uint32_t FMT, uint32_t EP, uint32_t T, bool Staged = false>
+__global__ __launch_bounds__(256, 2) void gguf_wide(const uint8_t *__restrict__ seg0, const uint8_t *__restrict__ seg1, const uint8_t *__restrict__ seg2,
+                                                    const uint8_t *__restrict__ table, void *__restrict__ out, const uint16_t *__restrict__ residual,
+                                                    GgufWideParams p) {
+  constexpr uint32_t kRecord = gguf_record_bytes(FMT);
+  constexpr bool kSums = FMT != GGUF_FMT_Q6K && !Staged, kTwice = FMT == GGUF_FMT_Q6K && !Staged, kGateUp = EP == GGUF_WIDE_GATE_UP;
+  __shared__ WideShared<T> shared;
+  const uint32_t perDie = gridDim.x / 8u, item = (blockIdx.x % 8u) * perDie + blockIdx.x / 8u;
+  if (item >= p.row_groups * p.splits * p.groups) return;
+  const uint32_t rowGroup = item % p.row_groups, rest = item / p.row_groups, split = rest % p.splits, columnGroup = rest / p.splits;
+  const uint32_t lane = threadIdx.x & 63u, wave = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6))), c = lane & 15u, kq = lane >> 4;
+  const uint32_t blocks = p.input_size / GGUF_BLOCK, liveTiles = (p.rows + 15u) / 16u;
+  const uint32_t tile0 = liveTiles * rowGroup / p.row_groups, tilesHere = liveTiles * (rowGroup + 1u) / p.row_groups - tile0;
+  const uint32_t b0 = blocks * split / p.splits, b1 = blocks * (split + 1u) / p.splits, count = b1 - b0;
+
+  // This wave's two column tiles: neighbours, or of a gate/up pair the same columns of both tensors.
+  const uint8_t *image[2];
+  uint32_t column[2];
+  if constexpr (kGateUp) {
+    const uint32_t tile = columnGroup * 4u + wave;
+    image[0] = seg0 + size_t(tile) * blocks * kRecord;
+    image[1] = seg1 + size_t(tile) * blocks * kRecord;
+    column[0] = column[1] = p.offset[0] + tile * 16u;
+  } else {
+    uint32_t group = columnGroup;
+    const uint8_t *seg = seg0;
+    uint32_t offset = p.offset[0];
+    const uint32_t first = p.cols[0] / GGUF_WIDE_COLUMNS, second = p.cols[1] / GGUF_WIDE_COLUMNS;
+    if (group >= first) {
+      group -= first;
+      seg = seg1;
+      offset = p.offset[1];
+      if (group >= second) {
+        group -= second;
+        seg = seg2;
+        offset = p.offset[2];
+      }
+    }
+#pragma unroll
+    for (uint32_t r = 0; r < 2; ++r) {
+      const uint32_t tile = group * 8u + wave * 2u + r;
+      image[r] = seg + size_t(tile) * blocks * kRecord;
+      column[r] = offset + tile * 16u;
+    }
+  }
+  Resource weights[2];
+#pragma unroll
+  for (uint32_t r = 0; r < 2; ++r) weights[r] = make_resource(image[r] + size_t(b0) * kRecord, count * kRecord);
+  const uint32_t tileBytes = uint32_t(gguf_wide_tile_bytes(p.input_size));
+  // (row tiles past the workgroup's, and super-blocks past its range, read as zeros or are not used)
+  const Resource rowValues = make_resource(table + size_t(tile0) * tileBytes, tilesHere * tileBytes);
+
+  f32x4 acc[2][T], dot[2][T];
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (uint32_t r = 0; r < 2; ++r)
+#pragma unroll
+    for (uint32_t t = 0; t < T; ++t) acc[r][t] = dot[r][t] = zero;
+
+  // Stage n holds groups 2 (n % 4), 2 (n % 4) + 1 of super-block n / 4 (and with a super-block's last, its sums): this
+  // thread's vectors of it, four (six) of 16 bytes.
+  constexpr uint32_t kShare = (T + 1) / 2, kSumShare = (T + 3) / 4;
+  uint4 held[kShare], heldSums[kSumShare];
+  const uint32_t mineAt = (threadIdx.x >> 7) * tileBytes + (threadIdx.x & 127u) * 16u;
+  const uint32_t sumsAt = (threadIdx.x >> 6) * tileBytes + lane * 16u;
+  auto fetch = [&](uint32_t block, uint32_t stage) {   // block counts from b0
+    const uint32_t at = (b0 + block) * (GGUF_WIDE_OPERANDS * 1024u) + stage * 2048u;
+#pragma unroll
+    for (uint32_t i = 0; i < kShare; ++i) {
+      const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rowValues, int(mineAt + (at + 2u * i * tileBytes)), 0, 0);
+      held[i] = make_uint4(v.x, v.y, v.z, v.w);
+    }
+    if (kSums && stage == 3u) {
+#pragma unroll
+      for (uint32_t i = 0; i < kSumShare; ++i) {
+        const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rowValues, int(sumsAt + (at + 2048u + 4u * i * tileBytes)), 0, 0);
+        heldSums[i] = make_uint4(v.x, v.y, v.z, v.w);
+      }
+    }
+  };
+  auto store = [&](uint32_t buffer, uint32_t stage) {
+#pragma unroll
+    for (uint32_t i = 0; i < kShare; ++i) (&shared.rows[buffer][0][0][0])[threadIdx.x + 256u * i] = held[i];
+    if (kSums && stage == 3u) {
+#pragma unroll
+      for (uint32_t i = 0; i < kSumShare; ++i) (&shared.sums[0][0])[threadIdx.x + 256u * i] = heldSums[i];
+    }
+  };
+  // A record's first half (and what both share) is fetched two stages ahead of its use, and so is its second.
+  WideRecord<FMT> rec[2];
+  uint32_t mine = 16u * lane;   // of the next super-block to fetch
+  auto fetchFirst = [&] {
+#pragma unroll
+    for (uint32_t r = 0; r < 2; ++r) load_first<FMT>(rec[r], weights[r], mine, lane);
+  };
+  auto fetchLate = [&] {
+#pragma unroll
+    for (uint32_t r = 0; r < 2; ++r) load_late<FMT>(rec[r], weights[r], mine, lane);
+  };
+  auto fetchSecond = [&] {
+#pragma unroll
+    for (uint32_t r = 0; r < 2; ++r) rec[r].codes[1] = load128<kStreamOnce>(weights[r], mine + 1024u);
+    mine += kRecord;
+  };
+  fetchFirst();
+  fetchLate();
+  fetch(0, 0);
+  store(0, 0);
+  fetch(0, 1);
+  __syncthreads();
+  for (uint32_t block = 0; block < count; ++block) {
+    WideScales<FMT> scales[2];
+#pragma unroll
+    for (uint32_t r = 0; r < 2; ++r) scales[r] = wide_scales(rec[r]);
+    auto run = [&](auto stageConstant) {
+      constexpr uint32_t S = decltype(stageConstant)::value;
+      store((S + 1u) & 1u, (S + 1u) & 3u);
+      fetch(block + (S >= 2u ? 1u : 0u), (S + 2u) & 3u);
+      if constexpr (S == 0) fetchSecond();
+      if constexpr (S == 2u) fetchFirst();
+      WideOperands<FMT> operands[2];
+#pragma unroll
+      for (uint32_t r = 0; r < 2; ++r) {
+        if constexpr (Staged) operands[r] = wide_staged_operands<FMT, S>(rec[r], scales[r]);
+        else operands[r] = wide_operands<FMT, S>(rec[r], scales[r]);
+      }
+      uint4 mins[2];
+      if constexpr (S == 3u && kSums) {
+#pragma unroll
+        for (uint32_t r = 0; r < 2; ++r) mins[r] = wide_mins(scales[r]);
+      }
+      if constexpr (S == 3u) fetchLate();
+      // A row tile's operands leave LDS while the tile before it is multiplied.
+      constexpr uint32_t kReads = S == 3u && kSums ? 3u : 2u;
+      f16x8 a[2][3];
+      auto read = [&](uint32_t t) {
+#pragma unroll
+        for (uint32_t g = 0; g < 2; ++g) a[t & 1u][g] = as_f16x8(shared.rows[S & 1u][t][g][lane]);
+        if constexpr (kReads == 3u) a[t & 1u][2] = as_f16x8(shared.sums[t][lane]);
+      };
+      read(0);
+#pragma unroll
+      for (uint32_t t = 0; t < T; ++t) {
+        if (t + 1 < T) read(t + 1);
+#pragma unroll
+        for (uint32_t g = 0; g < 2; ++g) {
+#pragma unroll
+          for (uint32_t r = 0; r < 2; ++r)
+            dot[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[t & 1u][g], as_f16x8(operands[r].high[g]), !Staged && S == 0 && g == 0 ? zero : dot[r][t], 0, 0, 0);
+          if constexpr (kTwice) {
+#pragma unroll
+            for (uint32_t r = 0; r < 2; ++r) dot[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[t & 1u][g], as_f16x8(operands[r].low[g]), dot[r][t], 0, 0, 0);
+          }
+        }
+        if constexpr (S == 3u && !Staged) {
+          f32x4 least[2];
+          if constexpr (kSums) {
+#pragma unroll
+            for (uint32_t r = 0; r < 2; ++r) least[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[t & 1u][2], as_f16x8(mins[r]), zero, 0, 0, 0);
+          }
+#pragma unroll
+          for (uint32_t r = 0; r < 2; ++r)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+              acc[r][t][v] = __fmaf_rn(dot[r][t][v], scales[r].d, acc[r][t][v]);
+              if constexpr (kSums) acc[r][t][v] = __fmaf_rn(least[r][v], scales[r].dmin, acc[r][t][v]);
+            }
+        }
+      }
+      constexpr uint32_t kProducts = (kTwice ? 8u : 4u) + (S == 3u && kSums ? 2u : 0u);
+      __builtin_amdgcn_sched_group_barrier(0x100, kReads, 0);
+#pragma unroll
+      for (uint32_t t = 0; t < T; ++t) {
+        if (t + 1 < T) __builtin_amdgcn_sched_group_barrier(0x100, kReads, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, kProducts, 0);
+      }
+      __syncthreads();
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    run(std::integral_constant<uint32_t, 0>{});
+    run(std::integral_constant<uint32_t, 1>{});
+    run(std::integral_constant<uint32_t, 2>{});
+    run(std::integral_constant<uint32_t, 3>{});
+  }
+  if constexpr (Staged) {
+#pragma unroll
+    for (uint32_t r = 0; r < 2; ++r)
+#pragma unroll
+      for (uint32_t t = 0; t < T; ++t) acc[r][t] = dot[r][t];
+  }
+  // Element (t, v) of this lane is row 16 (tile0 + t) + 4 kq + v, column column[r] + c.
+  const float *inverse = reinterpret_cast<const float *>(table + gguf_wide_scales_offset(p.input_size, p.tiles));
+#pragma unroll
+  for (uint32_t t = 0; t < T; ++t) {
+    if (t >= tilesHere) break;
+#pragma unroll
+    for (uint32_t v = 0; v < 4; ++v) {
+      const uint32_t row = 16u * (tile0 + t) + 4u * kq + v;
+      if (row >= p.rows) continue;
+      const float scale = inverse[row];
+      if constexpr (kGateUp) {
+        const float gate = round_bf16(acc[0][t][v] * scale), up = round_bf16(acc[1][t][v] * scale);
+        static_cast<uint16_t *>(out)[size_t(row) * p.out_stride + column[0] + c] = uint16_t(float_to_bf16_bits(up * silu(gate)));
+      } else {
+#pragma unroll
+        for (uint32_t r = 0; r < 2; ++r) {
+          const float value = acc[r][t][v] * scale;
+          const size_t at = size_t(row) * p.out_stride + column[r] + c;
+          if constexpr (EP == GGUF_WIDE_PARTIAL) static_cast<float *>(out)[size_t(split) * p.rows * p.out_stride + at] = value;
+          else if constexpr (EP == GGUF_WIDE_RESIDUAL)
+            static_cast<uint16_t *>(out)[at] = uint16_t(float_to_bf16_bits(value + bf16_bits_to_float(residual[at])));
+          else static_cast<uint16_t *>(out)[at] = uint16_t(float_to_bf16_bits(value));
+        }
+      }
+    }
+  }
+}
+#define SP_GGUF_WIDE_T(fmt, FMT, T)                                                          \
+  SP_REGISTER_KERNEL("gguf_wide_" fmt "_t" #T "_a", (&gguf_wide<FMT, GGUF_WIDE_PLAIN, T>));        \
+  SP_REGISTER_KERNEL("gguf_wide_" fmt "_t" #T "_r", (&gguf_wide<FMT, GGUF_WIDE_RESIDUAL, T>));     \
+  SP_REGISTER_KERNEL("gguf_wide_" fmt "_t" #T "_g", (&gguf_wide<FMT, GGUF_WIDE_GATE_UP, T>));      \
+  SP_REGISTER_KERNEL("gguf_wide_" fmt "_t" #T "_p", (&gguf_wide<FMT, GGUF_WIDE_PARTIAL, T>))
+#define SP_GGUF_WIDE(fmt, FMT)  \
+  SP_GGUF_WIDE_T(fmt, FMT, 4);  \
+  SP_GGUF_WIDE_T(fmt, FMT, 6);  \
+  SP_GGUF_WIDE_T(fmt, FMT, 7);  \
+  SP_GGUF_WIDE_T(fmt, FMT, 8)
+// (the staged rule's chunks are long ones: the tallest tile alone)
+#define SP_GGUF_WIDE_STAGED(fmt, FMT)                                                                          \
+  SP_REGISTER_KERNEL("gguf_wide_staged_" fmt "_t8_a", (&gguf_wide<FMT, GGUF_WIDE_PLAIN, 8, true>));      \
+  SP_REGISTER_KERNEL("gguf_wide_staged_" fmt "_t8_r", (&gguf_wide<FMT, GGUF_WIDE_RESIDUAL, 8, true>));   \
+  SP_REGISTER_KERNEL("gguf_wide_staged_" fmt "_t8_g", (&gguf_wide<FMT, GGUF_WIDE_GATE_UP, 8, true>));    \
+  SP_REGISTER_KERNEL("gguf_wide_staged_" fmt "_t8_p", (&gguf_wide<FMT, GGUF_WIDE_PARTIAL, 8, true>))
+SP_GGUF_WIDE_STAGED("q4k", GGUF_FMT_Q4K);
+SP_GGUF_WIDE_STAGED("q5k", GGUF_FMT_Q5K);
+SP_GGUF_WIDE_STAGED("q6k", GGUF_FMT_Q6K);
+SP_GGUF_WIDE("q4k", GGUF_FMT_Q4K);
+SP_GGUF_WIDE("q5k", GGUF_FMT_Q5K);
+SP_GGUF_WIDE("q6k", GGUF_FMT_Q6K);
+
+template <bool Residual>
+__global__ __launch_bounds__(256) void gguf_wide_reduce(const float4 *__restrict__ partials, uint2 *__restrict__ out,
+                                                        const uint2 *__restrict__ residual, GgufWideReduceParams p) {
+  const uint64_t at = uint64_t(blockIdx.x) * 256u + threadIdx.x, all = uint64_t(p.rows) * (p.columns / 4u);
+  if (at >= all) return;
+  float4 part[GGUF_WIDE_MAXIMUM_SPLITS];
+#pragma unroll
+  for (uint32_t s = 0; s < GGUF_WIDE_MAXIMUM_SPLITS; ++s)
+    if (s < p.splits) part[s] = partials[s * all + at];
+  float4 sum = part[0];
+#pragma unroll
+  for (uint32_t s = 1; s < GGUF_WIDE_MAXIMUM_SPLITS; ++s)
+    if (s < p.splits) sum = make_float4(sum.x + part[s].x, sum.y + part[s].y, sum.z + part[s].z, sum.w + part[s].w);
+  if constexpr (Residual) {
+    const uint2 r = residual[at];
+    sum = make_float4(sum.x + bf16_bits_to_float(r.x & 0xFFFFu), sum.y + bf16_bits_to_float(r.x >> 16), sum.z + bf16_bits_to_float(r.y & 0xFFFFu),
+                      sum.w + bf16_bits_to_float(r.y >> 16));
+  }
+  out[at] = make_uint2(float_to_bf16_bits(sum.x) | (float_to_bf16_bits(sum.y) << 16), float_to_bf16_bits(sum.z) | (float_to_bf16_bits(sum.w) << 16));
+}
+SP_REGISTER_KERNEL("gguf_wide_reduce_a", &gguf_wide_reduce<false>);
+SP_REGISTER_KERNEL("gguf_wide_reduce_r", &gguf_wide_reduce<true>);
+
+} // namespace splash::kernels

@@ -91,6 +91,15 @@ DenseVerify::DenseVerify(hip::Backend &backend, DenseDimensions d, uint32_t maxL
   nextTable_ = device(gguf_tables_bytes(std::max(d.attentionWidth(), d.ffn), gguf_row_tiles(windowRows)), "linear table 2");
   if (rowCapacity_ > maxRows_)
     chunkAttentionTable_ = device(gguf_tables_bytes(d.attentionWidth(), gguf_row_tiles(rowCapacity_)), "chunk attention table");
+  if (wideChunks()) {
+    const uint32_t widest = std::max({d.hidden, d.attentionWidth(), d.ffn});
+    wideTable_ = device(ops::Linear::wideTableBytes(widest, rowCapacity_), "wide table");
+    wideRows_ = device(C * d.ffn * 2, "chunk SwiGLU rows");
+    uint64_t partials = 0;
+    for (ops::LinearMatrix m : {ops::LinearMatrix{d.qkvWidth(), d.hidden}, ops::LinearMatrix{d.hidden, d.attentionWidth()}, ops::LinearMatrix{d.hidden, d.ffn}})
+      partials = std::max(partials, linear_.widePartialBytes(m, rowCapacity_));
+    widePartials_ = device(partials, "wide partials");
+  }
   // Chained projections each keep a table, partials and counters of their own.
   chainTables_[0] = device(gguf_table_bytes(d.hidden, gguf_row_tiles(maxRows_)), "gate/up table");
   chainTables_[1] = device(gguf_table_bytes(d.ffn, gguf_row_tiles(maxRows_)), "down table");
@@ -336,16 +345,53 @@ void DenseVerify::encodeHead(hip::CommandGraph &graph, uint32_t rows, bool input
 }
 
 void DenseVerify::setStagedPrefill(bool staged) {
-  if (staged && !prefillTable_) {
-    if (rowCapacity_ <= maxRows_) throw std::invalid_argument("the driver was created without room for a long prompt chunk");
-    const uint32_t widest = std::max({dims_.hidden, dims_.attentionWidth(), dims_.ffn});
-    prefillTable_ = backend_.allocateBuffer(ops::Linear::prefillTableBytes(widest, rowCapacity_), BufferStorage::Private, "prefill tables");
-    const uint64_t ffnBytes = uint64_t{rowCapacity_} * dims_.ffn * 2;
-    gateRows_ = backend_.allocateBuffer(ffnBytes, BufferStorage::Private, "prefill gate rows");
-    upRows_ = backend_.allocateBuffer(ffnBytes, BufferStorage::Private, "prefill up rows");
-    swigluRows_ = backend_.allocateBuffer(ffnBytes, BufferStorage::Private, "prefill SwiGLU rows");
-  }
+  if (staged && rowCapacity_ <= maxRows_) throw std::invalid_argument("the driver was created without room for a long prompt chunk");
   stagedPrefill_ = staged;
+}
+
+// The rows of the prefill tile's projections, where the wide kernels do not take the model's.
+void DenseVerify::needPrefillRows() {
+  if (prefillTable_) return;
+  const uint32_t widest = std::max({dims_.hidden, dims_.attentionWidth(), dims_.ffn});
+  prefillTable_ = backend_.allocateBuffer(ops::Linear::prefillTableBytes(widest, rowCapacity_), BufferStorage::Private, "prefill tables");
+  const uint64_t ffnBytes = uint64_t{rowCapacity_} * dims_.ffn * 2;
+  gateRows_ = backend_.allocateBuffer(ffnBytes, BufferStorage::Private, "prefill gate rows");
+  upRows_ = backend_.allocateBuffer(ffnBytes, BufferStorage::Private, "prefill up rows");
+  swigluRows_ = backend_.allocateBuffer(ffnBytes, BufferStorage::Private, "prefill SwiGLU rows");
+}
+
+// Whether chunks may take the wide kernels: from this width on the projections are most of a chunk's time. Narrower
+// models' chunks run the step's kernels in windows, whose rows are those of the sixteen-row steps bit for bit.
+bool DenseVerify::wideChunks() const noexcept {
+  return rowCapacity_ > maxRows_ && dims_.hidden >= kWideHidden && dims_.hidden <= ops::Linear::kMaximumWideNormWidth;
+}
+bool DenseVerify::takesWide(uint32_t tokens) const {
+  if (!wideChunks() || tokens < kWideRows) return false;
+  for (const DenseLayer &l : weights_.layers) {
+    for (const ops::Projection *p : {&l.qkv, &l.output, &l.gate, &l.up, &l.down})
+      if (!ops::Linear::takesWide(*p)) return false;
+    if (l.gate.blocks().segments.size() != 1 || l.up.blocks().segments.size() != 1 ||
+        l.gate.blocks().segments.front().formatId != l.up.blocks().segments.front().formatId)
+      return false;
+  }
+  return true;
+}
+
+// A layer of a long chunk through the wide kernels: every projection one pass over all the rows.
+void DenseVerify::encodeWideChunkLayer(hip::CommandGraph &graph, uint32_t layer, const ops::AttentionChunkPlan &plan, uint32_t tokens) {
+  const DenseLayer &w = weights_.layers.at(layer);
+  const hip::Buffer &residual = hidden_[0], &next = hidden_[1];
+  ops::Linear::addWideNormTable(graph, residual, w.inputNorm, wideTable_, dims_.hidden, tokens);
+  linear_.addWide(graph, w.qkv, wideTable_, qkv_, {}, widePartials_, tokens, stagedPrefill_);
+  const ops::KvPages pages{pageTable_, kvPools_.at(layer), pageBytes_};
+  ops::PagedAttention::addChunkProjection(graph, plan, {qkv_, w.queryNorm, w.keyNorm, ropeCos_, ropeSin_}, attentionWorkspace_, pages);
+  ops::PagedAttention::addChunkAttention(graph, plan, attentionWorkspace_, treeRows_, pages, attention_);
+  ops::Linear::addWideTable(graph, attention_, wideTable_, dims_.attentionWidth(), tokens);
+  linear_.addWide(graph, w.output, wideTable_, next, residual, widePartials_, tokens, stagedPrefill_);
+  ops::Linear::addWideNormTable(graph, next, w.postNorm, wideTable_, dims_.hidden, tokens);
+  linear_.addWideGateUp(graph, w.gate, w.up, wideTable_, wideRows_, tokens, stagedPrefill_);
+  ops::Linear::addWideTable(graph, wideRows_, wideTable_, dims_.ffn, tokens);
+  linear_.addWide(graph, w.down, wideTable_, residual, next, widePartials_, tokens, stagedPrefill_);
 }
 
 // A layer of a long chunk under the staged rule: each projection one pass of the prefill tile over all the rows.
@@ -452,8 +498,11 @@ void DenseVerify::encodePrefill(hip::CommandGraph &graph, uint32_t tableFirst, u
     encodeEmbedding(graph, tokens);
     // every window is a step's worth of rows at most, so what holds for one holds for all
     const bool feeds = layersFeedNext(std::min(tokens, kWindowRows));
+    const bool wide = takesWide(tokens);
+    if (stagedPrefill_ && !wide) needPrefillRows();
     for (uint32_t layer = 0; layer < dims_.layers; ++layer) {
-      if (stagedPrefill_) encodeStagedChunkLayer(graph, layer, plan, tokens);
+      if (wide) encodeWideChunkLayer(graph, layer, plan, tokens);
+      else if (stagedPrefill_) encodeStagedChunkLayer(graph, layer, plan, tokens);
       else encodeChunkLayer(graph, layer, plan, tokens, feeds && layer > 0, feeds && layer + 1 < dims_.layers);
       encodeCapture(graph, layer, tokens);
     }

@@ -180,8 +180,15 @@ private:
   void encodeCapture(hip::CommandGraph &graph, uint32_t layer, uint32_t rows) const;
   ops::SamplingBuffers children_;   // the four candidate-children buffers, bound into a step's sampling buffers when it tests them
   bool stagedPrefill_ = false;
-  hip::Buffer prefillTable_, gateRows_, upRows_, swigluRows_;  // the staged prompt chunk's tables and SwiGLU rows
+  hip::Buffer prefillTable_, gateRows_, upRows_, swigluRows_;  // the prefill tile's tables and SwiGLU rows
+  hip::Buffer wideTable_, wideRows_, widePartials_;             // the wide kernels' table, SwiGLU rows and parts' sums
   void encodeStagedChunkLayer(hip::CommandGraph &graph, uint32_t layer, const ops::AttentionChunkPlan &plan, uint32_t tokens);
+  // Chunks of at least kWideRows rows of a model at least kWideHidden wide take the wide kernels.
+  static constexpr uint32_t kWideHidden = 2048, kWideRows = 65;
+  [[nodiscard]] bool wideChunks() const noexcept;
+  [[nodiscard]] bool takesWide(uint32_t tokens) const;
+  void encodeWideChunkLayer(hip::CommandGraph &graph, uint32_t layer, const ops::AttentionChunkPlan &plan, uint32_t tokens);
+  void needPrefillRows();
   hip::Buffer chunkAttentionTable_;  // a long chunk's attention rows as the output projection's tables, every window's
   void encodeChunkLayer(hip::CommandGraph &graph, uint32_t layer, const ops::AttentionChunkPlan &plan, uint32_t tokens, bool first,
                         bool feedsNext);

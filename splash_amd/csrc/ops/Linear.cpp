@@ -482,6 +482,139 @@ void Linear::addPrefill(hip::CommandGraph &graph, const hip::Buffer &input, cons
   }
 }
 
+bool Linear::takesWide(const Projection &p) noexcept {
+  if (p.destination != FloatOutput::BFloat16 || p.inputSize > kMaximumWideWidth) return false;
+  const std::vector<QuantizedSegment> &segments = p.blocks().segments;
+  if (segments.empty() || segments.size() > GGUF_MAXIMUM_SEGMENTS) return false;
+  const uint32_t format = segments.front().formatId;
+  if (format != GGUF_FMT_Q4K && format != GGUF_FMT_Q5K && format != GGUF_FMT_Q6K) return false;
+  for (const QuantizedSegment &s : segments)
+    if (s.formatId != format || s.outputSize % GGUF_WIDE_COLUMNS || s.columnOffset % GGUF_TILE_COLUMNS) return false;
+  return true;
+}
+
+uint64_t Linear::wideTableBytes(uint32_t inputSize, uint32_t rows) noexcept { return gguf_wide_table_bytes(inputSize, rows); }
+
+// How a chunk's workgroups share the work: the row tiles dealt evenly over as few workgroups as hold them, and K in as
+// many parts as fill the device's rounds best. A compute unit holds two workgroups, so `items` workgroups take
+// ceil(items / (2 units)) rounds of 1 / splits of K each; a part more costs its partials' trip to memory and back.
+Linear::WideSplit Linear::wideSplit(uint32_t columnGroups, uint32_t blocks, uint32_t rows, bool splittable) const noexcept {
+  const uint32_t liveTiles = gguf_row_tiles(rows), rowGroups = (liveTiles + GGUF_WIDE_TILES - 1) / GGUF_WIDE_TILES;
+  const uint32_t most = (liveTiles + rowGroups - 1) / rowGroups, tiles = most <= 4 ? 4 : most <= 6 ? 6 : most;
+  const uint32_t slots = 2 * calibration_.computeUnits, items = rowGroups * columnGroups;
+  uint32_t splits = 1;
+  double best = 0;
+  for (uint32_t s = 1; splittable && s <= GGUF_WIDE_MAXIMUM_SPLITS && s * 4 <= blocks; ++s) {
+    const double cost = double((uint64_t{items} * s + slots - 1) / slots) / s + (s > 1 ? 0.05 + 0.02 * s : 0.0);
+    if (s == 1 || cost < best) { best = cost; splits = s; }
+  }
+  return {rowGroups, tiles, splits};
+}
+
+uint64_t Linear::widePartialBytes(LinearMatrix matrix, uint32_t rows) const noexcept {
+  uint64_t bytes = 0;
+  for (uint32_t r = 1; r <= rows; r = r == rows ? rows + 1 : std::min(rows, r + GGUF_ROW_TILE)) {
+    const WideSplit split = wideSplit(matrix.outputSize / GGUF_WIDE_COLUMNS, matrix.inputSize / GGUF_BLOCK, r, true);
+    // (a split of r rows may be that of any row count of the same tiles)
+    if (split.splits > 1) bytes = std::max(bytes, uint64_t{split.splits} * gguf_row_tiles(r) * GGUF_ROW_TILE * matrix.outputSize * 4);
+  }
+  return bytes;
+}
+
+void Linear::addWideTable(hip::CommandGraph &graph, const hip::Buffer &input, const hip::Buffer &table, uint32_t width, uint32_t rows) {
+  if (!rows || rows > kMaximumPrefillRows) throw std::invalid_argument("a prompt chunk takes 1 to 16384 rows");
+  if (!width || width % GGUF_BLOCK || width > kMaximumWideWidth)
+    throw std::invalid_argument("a wide table takes whole super-blocks of up to 32768 inputs");
+  requireBytes(input, uint64_t{rows} * width * 2, "projection input");
+  requireBytes(table, gguf_wide_table_bytes(width, rows), "wide table");
+  const uint32_t tiles = gguf_wide_tiles(rows);
+  graph.add(width <= kMaximumWideNormWidth ? "gguf_wide_table" : "gguf_wide_table_long", {input, input, table},
+            GgufWideTableParams{width, rows, tiles, 0}, {64 * ((16 * tiles + 63) / 64), 1, 1}, {256, 1, 1});
+}
+
+void Linear::addWideNormTable(hip::CommandGraph &graph, const hip::Buffer &input, const hip::Buffer &weight, const hip::Buffer &table,
+                              uint32_t width, uint32_t rows) {
+  if (!rows || rows > kMaximumPrefillRows) throw std::invalid_argument("a prompt chunk takes 1 to 16384 rows");
+  if (!width || width % GGUF_BLOCK || width > kMaximumWideNormWidth)
+    throw std::invalid_argument("a normed wide table takes whole super-blocks of up to 8192 inputs");
+  requireBytes(input, uint64_t{rows} * width * 2, "projection input");
+  requireBytes(weight, uint64_t{width} * 2, "norm weight");
+  requireBytes(table, gguf_wide_table_bytes(width, rows), "wide table");
+  const uint32_t tiles = gguf_wide_tiles(rows);
+  graph.add("gguf_wide_table_norm", {input, weight, table}, GgufWideTableParams{width, rows, tiles, 0},
+            {64 * ((16 * tiles + 63) / 64), 1, 1}, {256, 1, 1});
+}
+
+namespace {
+GgufWideParams wideParams(uint32_t k, uint32_t rows, uint32_t outStride, uint32_t groups, uint32_t rowGroups, uint32_t splits) {
+  GgufWideParams params{};
+  params.input_size = k;
+  params.rows = rows;
+  params.tiles = gguf_wide_tiles(rows);
+  params.row_groups = rowGroups;
+  params.splits = splits;
+  params.out_stride = outStride;
+  params.groups = groups;
+  return params;
+}
+uint32_t wideGrid(const GgufWideParams &p) { return 8 * ((p.row_groups * p.splits * p.groups + 7) / 8); }
+std::string wideName(const char *format, bool staged, uint32_t tiles, const char *suffix) {
+  return std::string(staged ? "gguf_wide_staged_" : "gguf_wide_") + format + "_t" + std::to_string(staged ? GGUF_WIDE_TILES : tiles) + suffix;
+}
+} // namespace
+
+void Linear::addWide(hip::CommandGraph &graph, const Projection &p, const hip::Buffer &table, const hip::Buffer &output,
+                     const hip::Buffer &residual, const hip::Buffer &partials, uint32_t rows, bool staged) const {
+  const uint32_t n = p.outputSize, k = p.inputSize;
+  if (!rows || rows > kMaximumPrefillRows) throw std::invalid_argument("a prompt chunk takes 1 to 16384 rows");
+  requireSegments(p, {n, k});
+  if (!takesWide(p)) throw std::invalid_argument("the wide kernels take tensors of one K-quant format, whole 128-column workgroups, bf16 results");
+  requireBytes(table, gguf_wide_table_bytes(k, rows), "wide table");
+  requireBytes(output, uint64_t{rows} * n * 2, "projection output");
+  if (residual) requireBytes(residual, uint64_t{rows} * n * 2, "projection residual");
+  const std::vector<QuantizedSegment> &segments = p.blocks().segments;
+  const uint32_t groups = n / GGUF_WIDE_COLUMNS;
+  const WideSplit split = wideSplit(groups, k / GGUF_BLOCK, rows, bool(partials));
+  if (split.splits > 1) requireBytes(partials, uint64_t{split.splits} * rows * n * 4, "projection partials");
+  GgufWideParams params = wideParams(k, rows, n, groups, split.rowGroups, split.splits);
+  hip::Buffer images[3];
+  for (size_t s = 0; s < 3; ++s) {
+    const QuantizedSegment &segment = segments[std::min(s, segments.size() - 1)];
+    images[s] = segment.image;
+    if (s < segments.size()) {
+      params.cols[s] = segment.outputSize;
+      params.offset[s] = segment.columnOffset;
+    }
+  }
+  const char *suffix = split.splits > 1 ? "_p" : residual ? "_r" : "_a";
+  graph.add(wideName(segments.front().name(), staged, split.tiles, suffix),
+            {images[0], images[1], images[2], table, split.splits > 1 ? partials : output, residual && split.splits == 1 ? residual : table}, params,
+            {wideGrid(params), 1, 1}, {256, 1, 1});
+  if (split.splits > 1)
+    graph.add(residual ? "gguf_wide_reduce_r" : "gguf_wide_reduce_a", {partials, output, residual ? residual : output},
+              GgufWideReduceParams{rows, n, split.splits, 0}, {uint32_t((uint64_t{rows} * n / 4 + 255) / 256), 1, 1}, {256, 1, 1});
+}
+
+void Linear::addWideGateUp(hip::CommandGraph &graph, const Projection &gate, const Projection &up, const hip::Buffer &table,
+                           const hip::Buffer &output, uint32_t rows, bool staged) const {
+  const uint32_t n = up.outputSize, k = up.inputSize;
+  if (!rows || rows > kMaximumPrefillRows) throw std::invalid_argument("a prompt chunk takes 1 to 16384 rows");
+  requireSegments(gate, {n, k});
+  requireSegments(up, {n, k});
+  if (!takesWide(gate) || !takesWide(up) || gate.blocks().segments.size() != 1 || up.blocks().segments.size() != 1 ||
+      gate.blocks().segments.front().formatId != up.blocks().segments.front().formatId)
+    throw std::invalid_argument("a one-pass block gate/up takes single tensors of one format");
+  requireBytes(table, gguf_wide_table_bytes(k, rows), "wide table");
+  requireBytes(output, uint64_t{rows} * n * 2, "projection output");
+  const uint32_t groups = n / (GGUF_WIDE_COLUMNS / 2);
+  const WideSplit split = wideSplit(groups, k / GGUF_BLOCK, rows, false);
+  GgufWideParams params = wideParams(k, rows, n, groups, split.rowGroups, 1);
+  params.cols[0] = n;
+  const hip::Buffer &first = gate.blocks().segments.front().image, &second = up.blocks().segments.front().image;
+  graph.add(wideName(up.blocks().segments.front().name(), staged, split.tiles, "_g"), {first, second, second, table, output, table}, params,
+            {wideGrid(params), 1, 1}, {256, 1, 1});
+}
+
 void Linear::addProjection(hip::CommandGraph &graph, hip::Buffer input, const Projection &projection, hip::Buffer output,
                            uint32_t rows, LinearScratch scratch) const {
   LinearBuffers buffers;

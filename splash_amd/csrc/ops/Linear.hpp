@@ -233,6 +233,23 @@ public:
   [[nodiscard]] static uint64_t prefillTableBytes(uint32_t inputSize, uint32_t rows) noexcept;
   static void addPrefill(hip::CommandGraph &graph, const hip::Buffer &input, const Projection &projection, const hip::Buffer &output,
                          const hip::Buffer &residual, const hip::Buffer &table, uint32_t rows);
+  // The projections of a prompt chunk of many rows through the matrix cores' fp16 (kernels gguf_wide_*): the register
+  // rule's exact weights, or (staged) each rounded once to half. takesWide: whether the kernels take the projection (one
+  // format of Q4_K, Q5_K, Q6_K; tensors of whole 128-column workgroups; bf16 results). The rows enter as a wide table,
+  // which addWideTable makes of bf16 rows and addWideNormTable of their RMS norm (rows of up to 8192 values).
+  static constexpr uint32_t kMaximumWideNormWidth = 8192, kMaximumWideWidth = 32768;
+  [[nodiscard]] static bool takesWide(const Projection &projection) noexcept;
+  [[nodiscard]] static uint64_t wideTableBytes(uint32_t inputSize, uint32_t rows) noexcept;
+  // fp32 partials of every plan of up to `rows` rows of a matrix.
+  [[nodiscard]] uint64_t widePartialBytes(LinearMatrix matrix, uint32_t rows) const noexcept;
+  static void addWideTable(hip::CommandGraph &graph, const hip::Buffer &input, const hip::Buffer &table, uint32_t width, uint32_t rows);
+  static void addWideNormTable(hip::CommandGraph &graph, const hip::Buffer &input, const hip::Buffer &weight, const hip::Buffer &table,
+                               uint32_t width, uint32_t rows);
+  void addWide(hip::CommandGraph &graph, const Projection &projection, const hip::Buffer &table, const hip::Buffer &output,
+               const hip::Buffer &residual, const hip::Buffer &partials, uint32_t rows, bool staged = false) const;
+  // output = bf16(bf16(up) * silu(bf16(gate))).
+  void addWideGateUp(hip::CommandGraph &graph, const Projection &gate, const Projection &up, const hip::Buffer &table, const hip::Buffer &output,
+                     uint32_t rows, bool staged = false) const;
   void addProjection(hip::CommandGraph &graph, hip::Buffer input, const Projection &projection, hip::Buffer output,
                      uint32_t rows, LinearScratch scratch) const;
   void addResidualProjection(hip::CommandGraph &graph, hip::Buffer input, const Projection &projection,
@@ -245,6 +262,8 @@ public:
 
 private:
   struct Resolved;
+  struct WideSplit { uint32_t rowGroups, tiles, splits; };
+  [[nodiscard]] WideSplit wideSplit(uint32_t columnGroups, uint32_t blocks, uint32_t rows, bool splittable) const noexcept;
   PreparedInput addColumn(hip::CommandGraph &graph, LinearBuffers buffers, const Projection &projection, const LinearPlan &plan,
                           const Projection *gate) const;
   [[nodiscard]] Resolved resolve(LinearBuffers buffers, const Projection &projection, const LinearPlan &plan,

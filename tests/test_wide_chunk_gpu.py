@@ -1,0 +1,63 @@
+"""GPU tests of a prompt chunk through the wide kernels (gguf_wide_*; model::DenseVerify::encodeWideChunkLayer): models of
+2048 columns and more, chunks of more than 64 rows."""
+import numpy as np
+import pytest
+
+from splash_amd import verify
+from tests import oracle as orc
+from tests.dense_reference import DenseModel
+
+pytestmark = pytest.mark.gpu
+
+
+def relative(a, b):
+    a, b = orc.bf16_to_f32(a).astype(np.float64), orc.bf16_to_f32(b).astype(np.float64)
+    return float(np.sqrt(((a - b) ** 2).sum() / (b ** 2).sum()))
+
+
+@pytest.mark.parametrize("down_format", [orc.FMT_Q4K, orc.FMT_Q5K, orc.FMT_Q6K])
+@pytest.mark.parametrize("tokens", [65, 100, 129, 300])
+def test_a_wide_chunk_is_its_blocks_to_rounding(backend, tokens, down_format):
+    """Row counts that fill no, one and several 128-row workgroups and end inside a 16-row tile, an FFN width of nine
+    super-blocks (half a piece of the table's pass), every format the kernels take: the hidden rows and the packed q|k|v
+    rows of the last layer are those of the same blocks run sixteen rows a step, to the rounding of bf16 rows; under the
+    staged rule to that of its half weights. A re-run repeats the bits."""
+    print(f"case wide chunk tokens={tokens} down={down_format}", flush=True)
+    H, layers = 2048, 1
+    model = DenseModel(seed=31, hidden=H, q_heads=16, kv_heads=4, head_dim=128, ffn=2304, vocabulary=512, layers=layers,
+                       down_format=orc.FMT_Q6K if down_format == orc.FMT_Q6K else orc.FMT_Q4K)
+    if down_format == orc.FMT_Q5K:      # (the oracle quantizes to Q4_K and Q6_K)
+        model.down_format, model.layers[0]["down"] = down_format, orc.make_native(down_format, H, 2304, 5)
+    rng = np.random.default_rng(tokens)
+    gpu = model.build_gpu(backend, max_lanes=1, context_tokens=[tokens + 300], prefill_rows=tokens)
+    model.seed_context(gpu, None, rng)
+    first, committed = model.table_first[0], 250
+    prompt = rng.integers(0, 512, tokens).astype(np.uint32)
+    pools = lambda: np.concatenate([gpu.buffer(verify.KV_POOL, layer).download(np.uint8) for layer in range(layers)])
+    start = pools()
+    rows_of = lambda which, rows, width: gpu.buffer(which, 0).download(np.uint16, rows * width).copy()
+    hidden, qkv = [], []
+    for at in range(0, tokens, 16):
+        rows = min(16, tokens - at)
+        lane = verify.Lane(rows, committed + at, table_first=first)
+        gpu.set_block([lane], prompt[at:at + rows])
+        backend.run(gpu.encode([lane], commit=False))
+        hidden.append(rows_of(verify.HIDDEN, rows, H))
+        qkv.append(rows_of(verify.QKV_ROWS, rows, 24 * 128))
+    want_hidden, want_qkv = np.concatenate(hidden), np.concatenate(qkv)
+    for staged in (False, True):
+        gpu.set_staged_prefill(staged)
+        seen = []
+        for _ in range(2):
+            for layer in range(layers):
+                gpu.buffer(verify.KV_POOL, layer).upload(start.reshape(layers, -1)[layer])
+            graph = gpu.encode_prefill(first, committed, tokens)
+            assert any(name.startswith("gguf_wide_staged" if staged else "gguf_wide_q") for name in graph.kernels())
+            gpu.set_prefill_block(prompt)
+            backend.run(graph)
+            seen.append((rows_of(verify.HIDDEN, tokens, H), rows_of(verify.QKV_ROWS, tokens, 24 * 128), pools()))
+        assert all(np.array_equal(a, b) for a, b in zip(*seen))
+        far = relative(seen[0][0], want_hidden), relative(seen[0][1], want_qkv)
+        print(f"  staged={staged}: hidden {far[0]:.5f}, q|k|v {far[1]:.5f}", flush=True)
+        # the q|k|v rows come of the same bf16 rows either way; the hidden rows of several bf16 roundings after them
+        assert far[0] <= 9e-3 and far[1] <= (2.5e-3 if staged else 1e-3)
