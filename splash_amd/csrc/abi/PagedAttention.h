@@ -86,10 +86,21 @@ struct AttentionParams {
   uint32_t gated;            // 1: the output rows are multiplied by the sigmoid of their heads' gates (attention_gate.h:19-44)
   uint32_t int8_queries;     // 1: queries are staged as INT8 codes with one scale a (row, head) and scored by an
                              // INT8 x INT8 product (the reference's q8q kernels, paged_attention_tile.h:294-322)
-  uint32_t reserved;
+  // Nonzero: a prompt chunk of so many rows of one sequence, sequence[0] its first row, the tokens before it, its page
+  // table and the steps of a split; block z of a dispatch is the chunk's z-th sixteen rows (attention_sequence).
+  uint32_t chunk_rows;
   uint64_t page_bytes;       // bytes between physical pages of the layer's pool
   struct AttentionSequence sequence[ATTENTION_MAXIMUM_SEQUENCES];
 };
+#if defined(__HIPCC__)
+__device__ inline AttentionSequence attention_sequence(const AttentionParams &p, uint32_t z) {
+  if (!p.chunk_rows) return p.sequence[z];
+  const AttentionSequence &chunk = p.sequence[0];
+  const uint32_t at = z * ATTENTION_MAXIMUM_ROWS;
+  return {chunk.first_row + at, chunk.committed + at, chunk.table_first,
+          uint16_t(p.chunk_rows - at < ATTENTION_MAXIMUM_ROWS ? p.chunk_rows - at : ATTENTION_MAXIMUM_ROWS), chunk.steps_per_split};
+}
+#endif
 
 // attention_q8_commit: moves the retained path's K/V slots to their depths
 // (the reference's SplashKvPathCommitParams, kv_path_commit.metal:21-48).

@@ -85,7 +85,7 @@ __global__ __launch_bounds__(D) void attention_q8_qkv(const uint16_t *__restrict
   __shared__ float scratch[4];
   __shared__ float normalized[D];
   const uint32_t tid = threadIdx.x, head = blockIdx.x, row = blockIdx.y, z = blockIdx.z;
-  const AttentionSequence seq = p.sequence[z];
+  const AttentionSequence seq = attention_sequence(p, z);
   const bool query = head < p.q_heads;
   const uint32_t group = p.q_heads / p.kv_heads;
   if (row >= seq.rows) {
@@ -176,12 +176,14 @@ SP_REGISTER_KERNEL("attention_q8_qkv_d64", &attention_q8_qkv<64>);
 // v_mfma_i32_16x16x64_i8 per 64 dimensions on the keys' stored bytes, which pass through LDS as they are (no widening,
 // no offset to remove), and a row's scale multiplies its scores after the product.
 typedef __attribute__((ext_vector_type(4))) int i32x4;
-template <int D, int G, bool I8>
-__global__ __launch_bounds__(256, 2) void attention_q8_split(const _Float16 *__restrict__ queries, const float *__restrict__ qsums,
-                                                          const AttentionTreeRow *__restrict__ tree,
-                                                          const uint64_t *__restrict__ page_table, uint8_t *__restrict__ pool,
-                                                          _Float16 *__restrict__ partialO, float *__restrict__ partialML,
-                                                          AttentionParams p) {
+// Whole: the workgroup's split is the block's whole history, and its rows leave finished (to `out`, gated by `packed`'s
+// gates where the layer has them) instead of as partials.
+template <int D, int G, bool I8, bool Whole>
+__device__ __forceinline__ void attention_split(const _Float16 *__restrict__ queries, const float *__restrict__ qsums,
+                                                const AttentionTreeRow *__restrict__ tree, const uint64_t *__restrict__ page_table,
+                                                uint8_t *__restrict__ pool, _Float16 *__restrict__ partialO, float *__restrict__ partialML,
+                                                uint16_t *__restrict__ out, const uint16_t *__restrict__ packed, const AttentionParams &p,
+                                                const uint32_t h, const uint32_t split, const uint32_t z) {
   constexpr int kStep = 64, JD = D / 32, DT = D / 16;
   constexpr int kTiles = (G + 3) / 4;  // fused-row tiles (one query head's 16 rows each) per wave
   constexpr int kKeyVectors = kStep * D / 16 / 256, kValueVectors = kKeyVectors;
@@ -193,8 +195,7 @@ __global__ __launch_bounds__(256, 2) void attention_q8_split(const _Float16 *__r
   __shared__ __align__(16) float ldsKS[2][kStep], ldsVS[2][kStep];
 
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, row = lane & 15u, kq = lane >> 4;
-  const uint32_t h = blockIdx.x, split = blockIdx.y, z = blockIdx.z;
-  const AttentionSequence seq = p.sequence[z];
+  const AttentionSequence seq = attention_sequence(p, z);
   const uint32_t total = seq.committed + seq.rows;
   // The sequence's own splits: ceil(steps / steps_per_split) of them; later grid rows are empty.
   static_assert(kStep == int(ATTENTION_STEP_TOKENS) && ATTENTION_PAGE_TOKENS % ATTENTION_STEP_TOKENS == 0, "a page holds whole steps");
@@ -454,6 +455,29 @@ __global__ __launch_bounds__(256, 2) void attention_q8_split(const _Float16 *__r
     const size_t fused = ((size_t(z) * p.kv_heads + h) * p.splits + split) * (16u * G) + 16u * g + row;
     const float rowSum = o[k][DT][0] * kCodeOffset;
     const float norm = sum > 0.f ? 1.0f / (sum * kPScale) : 0.f;
+    if constexpr (Whole) {
+      // dimensions 16 dt + 4 kq .. + 3 of query head h G + g, four to a store
+      if (row >= seq.rows) continue;
+      const uint32_t head = h * uint32_t(G) + g;
+      const size_t packedRow = size_t(seq.first_row) + row;
+      uint2 *mine = reinterpret_cast<uint2 *>(out + packedRow * (p.q_heads * D) + head * D);
+      const uint2 *gates = reinterpret_cast<const uint2 *>(packed + packedRow * p.qkv_stride + head * 2u * D + D);
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        uint32_t bits[4];
+        const uint2 gate = p.gated ? gates[4 * dt + kq] : make_uint2(0u, 0u);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          bits[i] = float_to_bf16_bits((o[k][dt][i] - rowSum) * norm);
+          if (p.gated) {
+            const float x = bf16_bits_to_float(((i < 2 ? gate.x : gate.y) >> (16 * (i & 1))) & 0xFFFFu);
+            bits[i] = float_to_bf16_bits(bf16_bits_to_float(bits[i]) * (1.0f / (1.0f + __builtin_amdgcn_exp2f(-kLog2e * x))));
+          }
+        }
+        mine[4 * dt + kq] = make_uint2(bits[0] | (bits[1] << 16), bits[2] | (bits[3] << 16));
+      }
+      continue;
+    }
     uint4 *mine = reinterpret_cast<uint4 *>(partialO + fused * D + 4u * DT * kq);
 #pragma unroll
     for (int dt = 0; dt < DT; dt += 2) {
@@ -471,6 +495,32 @@ __global__ __launch_bounds__(256, 2) void attention_q8_split(const _Float16 *__r
     }
   }
 }
+template <int D, int G, bool I8>
+__global__ __launch_bounds__(256, 2) void attention_q8_split(const _Float16 *__restrict__ queries, const float *__restrict__ qsums,
+                                                          const AttentionTreeRow *__restrict__ tree,
+                                                          const uint64_t *__restrict__ page_table, uint8_t *__restrict__ pool,
+                                                          _Float16 *__restrict__ partialO, float *__restrict__ partialML,
+                                                          AttentionParams p) {
+  attention_split<D, G, I8, false>(queries, qsums, tree, page_table, pool, partialO, partialML, nullptr, nullptr, p, blockIdx.x, blockIdx.y,
+                                   blockIdx.z);
+}
+// attention_q8_whole: grid (kv_heads * blocks), 256 threads. A prompt chunk's blocks of sixteen rows, each over its whole
+// history in one workgroup: no partials, no merge, and the fixed cost of a split (its queries, the first step's latency,
+// the partials, about 18 us) once a block. Neighbouring workgroups take the KV heads in turn, so that with eight heads a
+// die (workgroup b runs on die b % 8) keeps one head's keys and values in its L2; the longest blocks start first.
+template <int D, int G>
+__global__ __launch_bounds__(256, 2) void attention_q8_whole(const _Float16 *__restrict__ queries, const float *__restrict__ qsums,
+                                                             const AttentionTreeRow *__restrict__ tree,
+                                                             const uint64_t *__restrict__ page_table, uint8_t *__restrict__ pool,
+                                                             uint16_t *__restrict__ out, const uint16_t *__restrict__ packed,
+                                                             AttentionParams p) {
+  const uint32_t blocks = gridDim.x / p.kv_heads;
+  attention_split<D, G, false, true>(queries, qsums, tree, page_table, pool, nullptr, nullptr, out, packed, p, blockIdx.x % p.kv_heads, 0u,
+                                     blocks - 1u - blockIdx.x / p.kv_heads);
+}
+SP_REGISTER_KERNEL("attention_q8_whole_d128_g8", (&attention_q8_whole<128, 8>));
+SP_REGISTER_KERNEL("attention_q8_whole_d128_g4", (&attention_q8_whole<128, 4>));
+SP_REGISTER_KERNEL("attention_q8_whole_d64_g2", (&attention_q8_whole<64, 2>));
 SP_REGISTER_KERNEL("attention_q8_split_d128_g8", &attention_q8_split<128, 8, false>);
 SP_REGISTER_KERNEL("attention_q8_split_d128_g4", &attention_q8_split<128, 4, false>);
 SP_REGISTER_KERNEL("attention_q8_split_d64_g2", &attention_q8_split<64, 2, false>);
@@ -499,7 +549,7 @@ __global__ __launch_bounds__(256) void attention_reduce(const _Float16 *__restri
   __shared__ __align__(16) float4 sums[kParts][kQuads];
   __shared__ uint16_t staged[D];
   const uint32_t tid = threadIdx.x, head = blockIdx.x, row = blockIdx.y, z = blockIdx.z;
-  const AttentionSequence seq = p.sequence[z];
+  const AttentionSequence seq = attention_sequence(p, z);
   if (row >= seq.rows) return;
   const uint32_t group = p.q_heads / p.kv_heads, h = head / group, g = head % group, fusedRows = 16u * group;
   const size_t base = (size_t(z) * p.kv_heads + h) * p.splits;

@@ -378,14 +378,14 @@ bool DenseVerify::takesWide(uint32_t tokens) const {
 }
 
 // A layer of a long chunk through the wide kernels: every projection one pass over all the rows.
-void DenseVerify::encodeWideChunkLayer(hip::CommandGraph &graph, uint32_t layer, const ops::AttentionChunkPlan &plan, uint32_t tokens) {
+void DenseVerify::encodeWideChunkLayer(hip::CommandGraph &graph, uint32_t layer, const ops::AttentionPromptPlan &plan, uint32_t tokens) {
   const DenseLayer &w = weights_.layers.at(layer);
   const hip::Buffer &residual = hidden_[0], &next = hidden_[1];
   ops::Linear::addWideNormTable(graph, residual, w.inputNorm, wideTable_, dims_.hidden, tokens);
   linear_.addWide(graph, w.qkv, wideTable_, qkv_, {}, widePartials_, tokens, stagedPrefill_);
   const ops::KvPages pages{pageTable_, kvPools_.at(layer), pageBytes_};
-  ops::PagedAttention::addChunkProjection(graph, plan, {qkv_, w.queryNorm, w.keyNorm, ropeCos_, ropeSin_}, attentionWorkspace_, pages);
-  ops::PagedAttention::addChunkAttention(graph, plan, attentionWorkspace_, treeRows_, pages, attention_);
+  ops::PagedAttention::addPromptProjection(graph, plan, {qkv_, w.queryNorm, w.keyNorm, ropeCos_, ropeSin_}, attentionWorkspace_, pages);
+  ops::PagedAttention::addPromptAttention(graph, plan, attentionWorkspace_, treeRows_, pages, attention_);
   ops::Linear::addWideTable(graph, attention_, wideTable_, dims_.attentionWidth(), tokens);
   linear_.addWide(graph, w.output, wideTable_, next, residual, widePartials_, tokens, stagedPrefill_);
   ops::Linear::addWideNormTable(graph, next, w.postNorm, wideTable_, dims_.hidden, tokens);
@@ -481,7 +481,11 @@ void DenseVerify::encodePrefill(hip::CommandGraph &graph, uint32_t tableFirst, u
   if (!tokens || tokens > rowCapacity_) throw std::invalid_argument("a prompt chunk takes 1 to the driver's most prefill rows");
   if (tokens > maxRows_) {
     const ops::AttentionGeometry geometry{dims_.qHeads, dims_.kvHeads, dims_.headDimension, dims_.rotaryPairs, dims_.normalizeHeads};
-    const ops::AttentionChunkPlan plan = ops::PagedAttention::planChunks(geometry, {{0, tokens, committed, tableFirst}});
+    const bool wide = takesWide(tokens);
+    ops::AttentionChunkPlan plan;
+    ops::AttentionPromptPlan widePlan;
+    if (wide) widePlan = ops::PagedAttention::planPrompt(geometry, {0, tokens, committed, tableFirst}, linear_.calibration().computeUnits);
+    else plan = ops::PagedAttention::planChunks(geometry, {{0, tokens, committed, tableFirst}});
     if (dims_.rotaryPairs) {
       // the RoPE tables eight blocks a dispatch, each dispatch over its own rows of the depths and tables
       const uint32_t span = ATTENTION_MAXIMUM_SEQUENCES * ATTENTION_MAXIMUM_ROWS;
@@ -498,10 +502,9 @@ void DenseVerify::encodePrefill(hip::CommandGraph &graph, uint32_t tableFirst, u
     encodeEmbedding(graph, tokens);
     // every window is a step's worth of rows at most, so what holds for one holds for all
     const bool feeds = layersFeedNext(std::min(tokens, kWindowRows));
-    const bool wide = takesWide(tokens);
     if (stagedPrefill_ && !wide) needPrefillRows();
     for (uint32_t layer = 0; layer < dims_.layers; ++layer) {
-      if (wide) encodeWideChunkLayer(graph, layer, plan, tokens);
+      if (wide) encodeWideChunkLayer(graph, layer, widePlan, tokens);
       else if (stagedPrefill_) encodeStagedChunkLayer(graph, layer, plan, tokens);
       else encodeChunkLayer(graph, layer, plan, tokens, feeds && layer > 0, feeds && layer + 1 < dims_.layers);
       encodeCapture(graph, layer, tokens);

@@ -240,6 +240,120 @@ void PagedAttention::addChunkAttention(hip::CommandGraph &graph, const Attention
     addAttention(graph, plan.dispatches()[d], workspaceOf(plan, workspace, d), treeRows, pages, output, outputTable, packed, plan.rows());
 }
 
+AttentionWorkspaceSize AttentionPromptPlan::workspace() const noexcept {
+  const uint64_t fused = uint64_t{blocks()} * geometry_.kvHeads * geometry_.group() * ATTENTION_MAXIMUM_ROWS;
+  AttentionWorkspaceSize size;
+  size.queries = fused * geometry_.headDimension * 2;
+  size.querySums = fused * 4;
+  if (splits_ > 1) {
+    size.partials = fused * splits_ * geometry_.headDimension * 2;
+    size.partialSums = fused * splits_ * 8;
+  }
+  return size;
+}
+
+AttentionParams AttentionPromptPlan::params(uint64_t pageBytes) const noexcept {
+  AttentionParams p{};
+  p.q_heads = geometry_.qHeads;
+  p.kv_heads = geometry_.kvHeads;
+  p.head_dim = geometry_.headDimension;
+  p.rotary_pairs = geometry_.rotaryPairs;
+  p.normalize = geometry_.normalize;
+  p.qkv_stride = geometry_.packedWidth();
+  p.gated = geometry_.gated;
+  p.splits = splits_;
+  p.sequences = blocks();
+  p.chunk_rows = chunk_.tokens;
+  p.page_bytes = pageBytes;
+  p.sequence[0] = {chunk_.firstRow, chunk_.committed, chunk_.tableFirst, uint16_t(ATTENTION_MAXIMUM_ROWS), uint16_t(stepsPerSplit_)};
+  return p;
+}
+
+AttentionPromptPlan PagedAttention::planPrompt(const AttentionGeometry &geometry, const AttentionChunk &chunk, uint32_t computeUnits) {
+  if (!geometry.kvHeads || geometry.qHeads % geometry.kvHeads || !compiled(geometry) || geometry.int8Queries)
+    throw std::invalid_argument("no attention kernel for this head geometry");
+  if (2 * geometry.rotaryPairs > geometry.headDimension) throw std::invalid_argument("the rotated pairs are dimensions of the head");
+  if (!chunk.tokens || chunk.tokens > kMaximumChunkRows) throw std::invalid_argument("a prompt chunk holds 1 to 2048 rows");
+  AttentionPromptPlan plan;
+  plan.geometry_ = geometry;
+  plan.chunk_ = chunk;
+  // A compute unit holds two workgroups. A chunk whose blocks alone give three quarters of the device's places work takes
+  // whole histories; a shorter one splits them into about as many parts as fill the places, at least four steps each.
+  const uint64_t steps = (uint64_t{chunk.committed} + chunk.tokens + ATTENTION_STEP_TOKENS - 1) / ATTENTION_STEP_TOKENS;
+  const uint32_t items = plan.blocks() * geometry.kvHeads, places = 2 * computeUnits;
+  uint64_t splits = 1;
+  if (items * 4 < places * 3) splits = std::min<uint64_t>({(places + items - 1) / items, std::max<uint64_t>(1, steps / 4), ATTENTION_MAXIMUM_SPLITS});
+  const uint64_t perSplit = (steps + splits - 1) / splits;
+  if (perSplit > 0xFFFF) throw std::invalid_argument("the sequence is longer than the attention kernels split");
+  plan.stepsPerSplit_ = uint32_t(perSplit);
+  plan.splits_ = uint32_t((steps + perSplit - 1) / perSplit);
+  return plan;
+}
+
+namespace {
+void requirePromptPages(const AttentionPromptPlan &plan, const AttentionParams &params, const KvPages &pages) {
+  const uint64_t need = plan.geometry().layout().bytesPerLayerPage();
+  if (pages.pageBytes < need || pages.pageBytes % 16) throw std::invalid_argument("KV page stride is smaller than a page or unaligned");
+  if (!pages.pool || pages.pool.sizeBytes() < pages.pageBytes) throw std::invalid_argument("KV pool buffer is too small");
+  const AttentionSequence &s = params.sequence[0];
+  requireBytes(pages.pageTable, (uint64_t{s.table_first} + kv::Layout::pagesFor(uint64_t{s.committed} + plan.rows())) * 8, "KV page table");
+}
+} // namespace
+
+void PagedAttention::addPromptProjection(hip::CommandGraph &graph, const AttentionPromptPlan &plan, const AttentionProjectionBuffers &b,
+                                         const AttentionWorkspace &w, const KvPages &pages) {
+  const AttentionGeometry &g = plan.geometry();
+  const AttentionParams params = plan.params(pages.pageBytes);
+  const uint64_t rows = uint64_t{params.sequence[0].first_row} + plan.rows();
+  requireBytes(b.qkv, rows * g.packedWidth() * 2, "attention qkv");
+  if (g.normalize) {
+    requireBytes(b.queryNorm, g.headDimension * 2, "query norm weight");
+    requireBytes(b.keyNorm, g.headDimension * 2, "key norm weight");
+  }
+  if (g.rotaryPairs) {
+    requireBytes(b.ropeCos, rows * g.rotaryPairs * 4, "RoPE cosine table");
+    requireBytes(b.ropeSin, rows * g.rotaryPairs * 4, "RoPE sine table");
+  }
+  const AttentionWorkspaceSize need = plan.workspace();
+  requireBytes(w.queries, need.queries, "staged queries");
+  requireBytes(w.querySums, need.querySums, "staged query sums");
+  requirePromptPages(plan, params, pages);
+  const hip::Buffer &spare = b.qkv;
+  graph.add("attention_q8_qkv" + kernelSuffix(g),
+            {b.qkv, g.normalize ? b.queryNorm : spare, g.normalize ? b.keyNorm : spare, g.rotaryPairs ? b.ropeCos : spare,
+             g.rotaryPairs ? b.ropeSin : spare, w.queries, w.querySums, pages.pageTable, pages.pool},
+            params, {g.qHeads + g.kvHeads, ATTENTION_MAXIMUM_ROWS, plan.blocks()}, {g.headDimension, 1, 1});
+}
+
+void PagedAttention::addPromptAttention(hip::CommandGraph &graph, const AttentionPromptPlan &plan, const AttentionWorkspace &w,
+                                        const hip::Buffer &treeRows, const KvPages &pages, const hip::Buffer &output, const hip::Buffer &packed) {
+  const AttentionGeometry &g = plan.geometry();
+  const AttentionParams params = plan.params(pages.pageBytes);
+  const uint64_t rows = uint64_t{params.sequence[0].first_row} + plan.rows();
+  const AttentionWorkspaceSize need = plan.workspace();
+  requireBytes(w.queries, need.queries, "staged queries");
+  requireBytes(w.querySums, need.querySums, "staged query sums");
+  if (plan.splits() > 1) {
+    requireBytes(w.partials, need.partials, "attention partials");
+    requireBytes(w.partialSums, need.partialSums, "attention partial sums");
+  }
+  requireBytes(treeRows, rows * sizeof(AttentionTreeRow), "verify tree rows");
+  requireBytes(output, rows * g.qHeads * g.headDimension * 2, "attention output");
+  if (g.gated) requireBytes(packed, rows * g.packedWidth() * 2, "attention qkv (the gates)");
+  requirePromptPages(plan, params, pages);
+  const std::string suffix = kernelSuffix(g) + "_g" + std::to_string(g.group());
+  const hip::Buffer &gates = g.gated ? packed : output;
+  if (plan.splits() == 1) {
+    graph.add("attention_q8_whole" + suffix, {w.queries, w.querySums, treeRows, pages.pageTable, pages.pool, output, gates}, params,
+              {g.kvHeads * plan.blocks(), 1, 1}, {256, 1, 1});
+    return;
+  }
+  graph.add("attention_q8_split" + suffix, {w.queries, w.querySums, treeRows, pages.pageTable, pages.pool, w.partials, w.partialSums}, params,
+            {g.kvHeads, plan.splits(), plan.blocks()}, {256, 1, 1});
+  graph.add("attention_reduce" + kernelSuffix(g), {w.partials, w.partialSums, output, output, gates}, params,
+            {g.qHeads, ATTENTION_MAXIMUM_ROWS, plan.blocks()}, {256, 1, 1});
+}
+
 void PagedAttention::addPathCommit(hip::CommandGraph &graph, const AttentionPlan &plan, const hip::Buffer &retained,
                                    const KvPages &pages, uint32_t layers, uint64_t layerBytes) {
   const AttentionGeometry &g = plan.geometry();

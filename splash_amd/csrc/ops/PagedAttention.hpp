@@ -114,6 +114,25 @@ private:
   uint32_t tiles_ = 0, rows_ = 0;
 };
 
+// A prompt chunk in as few dispatches as it takes: one prepare, one attention over all of its blocks of sixteen rows
+// and, of a chunk too short to fill the device with whole histories, one merge. Its rows are planChunks' to the rounding
+// of where a history is split, not bit for bit.
+class AttentionPromptPlan final {
+public:
+  [[nodiscard]] const AttentionGeometry &geometry() const noexcept { return geometry_; }
+  [[nodiscard]] uint32_t rows() const noexcept { return chunk_.tokens; }
+  [[nodiscard]] uint32_t blocks() const noexcept { return (chunk_.tokens + ATTENTION_MAXIMUM_ROWS - 1) / ATTENTION_MAXIMUM_ROWS; }
+  [[nodiscard]] uint32_t splits() const noexcept { return splits_; }
+  [[nodiscard]] AttentionWorkspaceSize workspace() const noexcept;
+
+private:
+  friend class PagedAttention;
+  [[nodiscard]] AttentionParams params(uint64_t pageBytes) const noexcept;
+  AttentionGeometry geometry_;
+  AttentionChunk chunk_;
+  uint32_t splits_ = 1, stepsPerSplit_ = 1;
+};
+
 struct AttentionProjectionBuffers final {
   hip::Buffer qkv;             // bf16 [packed rows][(q + 2 kv) heads * D]
   hip::Buffer queryNorm, keyNorm;  // bf16 [D]; used when geometry.normalize
@@ -158,6 +177,11 @@ public:
   static void addChunkAttention(hip::CommandGraph &graph, const AttentionChunkPlan &plan, const AttentionWorkspace &workspace,
                                 const hip::Buffer &treeRows, const KvPages &pages, const hip::Buffer &output,
                                 const hip::Buffer &outputTable = {}, const hip::Buffer &packed = {});
+  [[nodiscard]] static AttentionPromptPlan planPrompt(const AttentionGeometry &geometry, const AttentionChunk &chunk, uint32_t computeUnits);
+  static void addPromptProjection(hip::CommandGraph &graph, const AttentionPromptPlan &plan, const AttentionProjectionBuffers &buffers,
+                                  const AttentionWorkspace &workspace, const KvPages &pages);
+  static void addPromptAttention(hip::CommandGraph &graph, const AttentionPromptPlan &plan, const AttentionWorkspace &workspace,
+                                 const hip::Buffer &treeRows, const KvPages &pages, const hip::Buffer &output, const hip::Buffer &packed = {});
   // Moves the retained path's slots to their depths (PagedAttention.cpp:647-667); retained is a
   // uint32 mask per sequence.
   // `layers` pools lie layerBytes apart from pages.pool (one dispatch commits them all, as the
