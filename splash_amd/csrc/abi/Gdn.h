@@ -104,7 +104,7 @@ struct GdnFoldParams {
 // rows that all enter the state (the reference's GDNPrefillParams, runtime/ops/GDN.cpp:176-222): the run reads
 // the layer's convolution carry and recurrent state of `current_cell` and writes those after its rows to
 // `next_cell`, another cell. No tape: a prompt's rows are never rolled back.
-#define GDN_SCAN_STATE_ROWS 8u    // state rows of one scan workgroup (the reference's SPLASH_GDN_SCAN_STATE_ROWS is 16)
+#define GDN_SCAN_STATE_ROWS 16u   // state rows of one scan workgroup (the reference's SPLASH_GDN_SCAN_STATE_ROWS)
 #define GDN_SCAN_BLOCK 16u        // tokens a scan workgroup stages at a time
 struct GdnPrefillParams {
   struct GdnShapeParams shape;
