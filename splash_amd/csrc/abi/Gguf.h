@@ -235,11 +235,19 @@ struct GgufWideParams {
   uint32_t splits;      // parts of K (1 unless _p)
   uint32_t out_stride;
   uint32_t groups;      // column groups of GGUF_WIDE_COLUMNS over the segments
-  uint32_t cols[3];     // columns per segment: multiples of GGUF_WIDE_COLUMNS (gate/up: of half of it)
+  uint32_t cols[3];     // columns per segment: multiples of 16; each segment starts a column group of its own
   uint32_t offset[3];   // first destination column per segment
   uint32_t reserved[3];
 };
-// gguf_wide_reduce_{a,r}: out = bf16(sum of the parts in order [+ residual]). Four columns a thread, grid
+// gguf_wide_moe_<fmt>_t<T>_{a,g}: the routed experts of a chunk (abi/Moe.h, MoeChunkTask): wide.rows, .row_groups and
+// .splits are unused. Binds the experts' images (gate and up, or down twice), the slots' wide table, the slots' output rows,
+// the tasks and their totals. Grid (8 * ceil(most tasks * groups / 8)).
+struct GgufWideMoeParams {
+  struct GgufWideParams wide;
+  uint64_t expert_bytes;  // between experts' images of a tensor
+  uint64_t reserved;
+};
+// gguf_wide_reduce_{a,r,f32}: out = bf16 (or fp32) (sum of the parts in order [+ residual]). Four columns a thread, grid
 // (ceil(rows * columns / 1024)), 256 threads.
 struct GgufWideReduceParams {
   uint32_t rows;
@@ -367,6 +375,7 @@ struct GgufEmbedParams {
 static_assert(sizeof(GgufPrepareParams) == 16, "prepare parameters are 16 bytes on both sides");
 static_assert(sizeof(GgufDecodeParams) == 64, "decode parameters are 64 bytes on both sides");
 static_assert(sizeof(GgufChainLink) == 96 && sizeof(GgufChainParams) == 400, "chain parameters are 400 bytes on both sides");
+static_assert(sizeof(GgufWideMoeParams) == 80, "wide expert parameters are 80 bytes on both sides");
 static_assert(sizeof(GgufWideParams) == 64, "wide parameters are 64 bytes on both sides");
 static_assert(sizeof(GgufDequantParams) == 8, "dequant parameters are 8 bytes on both sides");
 static_assert(sizeof(GgufEmbedParams) == 12, "embedding parameters are 12 bytes on both sides");

@@ -47,6 +47,19 @@ struct MoeGroupParams {
   uint32_t experts, top_k;
   uint32_t maximum_tiles;
 };
+// The routes of a prompt chunk, grouped by expert in windows of MOE_CHUNK_ROUTES routes that run side by side:
+// moe_chunk_count (grid (windows), 1024 threads) counts each window's routes of each expert; moe_chunk_place (the same
+// grid) places them: an expert's slots are whole tiles of 16, its routes in route order, whatever the windows. Window 0
+// also writes tasks of up to `task_tiles` of an expert's tiles, as even as they divide, and totals {tiles, tasks}.
+#define MOE_CHUNK_ROUTES 2048u
+struct MoeChunkTask {
+  uint32_t expert, first_tile, tiles, reserved;
+};
+struct MoeChunkParams {
+  uint32_t routes;      // rows * top_k
+  uint32_t experts, top_k;
+  uint32_t task_tiles;
+};
 // moe_gather_table: grid (hidden / 32, maximum tiles), 64 threads: a tile's rows as its activation table.
 struct MoeGatherParams {
   uint32_t hidden;

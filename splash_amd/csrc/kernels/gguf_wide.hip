@@ -15,6 +15,7 @@
 // windows of the decode kernels took 2.38 ms), at 25600 x 5120 Q6_K 0.99 ms (2.2 ms): the matrix cores are busy 46 % and
 // 59 % of the cycles of a clock that the card's power limit holds at 2.1 and 1.8 GHz.
 #include "abi/Gguf.h"
+#include "abi/Moe.h"
 #include "backend/KernelRegistry.hpp"
 #include "kernels/gguf_records.hpp"
 
@@ -34,14 +35,12 @@ __device__ __forceinline__ f16x2 both(float v) { return f16x2{_Float16(v), _Floa
 // quarter t % 4 of groups t / 4, 64 + t / 4, ... in `Held` pieces. The eight rows that share the table's 128-byte lines are
 // neighbours on one die (workgroup b runs on die b % 8), so that its L2 writes whole lines.
 template <bool Norm, uint32_t Held>
-__global__ __launch_bounds__(256) void gguf_wide_table(const uint16_t *__restrict__ input, const uint16_t *__restrict__ weight,
-                                                       uint8_t *__restrict__ table, GgufWideTableParams p) {
+__device__ __forceinline__ void wide_table_row(const uint16_t *__restrict__ input, const uint16_t *__restrict__ weight, uint8_t *__restrict__ table,
+                                               const GgufWideTableParams &p, const uint32_t row, const uint32_t source) {
   __shared__ float scratch[8];
-  const uint32_t die = blockIdx.x % 8u, slot = blockIdx.x / 8u, row = (slot / 8u * 8u + die) * 8u + slot % 8u;
-  if (row >= 16u * p.tiles) return;
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, tile = row / 16u, r = row % 16u;
   const uint32_t kq = tid & 3u, groups = p.input_size / 32u, held = (groups + 63u) / 64u;
-  const bool live = row < p.rows;
+  const bool live = source < p.rows;
   uint4 *values = reinterpret_cast<uint4 *>(table + tile * gguf_wide_tile_bytes(p.input_size));
   // piece i: inputs 4 kq .. + 3, then 16 + 4 kq .. + 3 of group 64 i + t / 4
   auto groupOf = [&](uint32_t i) { return 64u * i + (tid >> 2); };
@@ -54,7 +53,7 @@ __global__ __launch_bounds__(256) void gguf_wide_table(const uint16_t *__restric
   uint4 v[Held];
 #pragma unroll
   for (uint32_t i = 0; i < Held; ++i)
-    if (i < held) v[i] = load(input + size_t(live ? row : 0u) * p.input_size, i);
+    if (i < held) v[i] = load(input + size_t(live ? source : 0u) * p.input_size, i);
   if constexpr (Norm) {
     uint4 w[Held];
 #pragma unroll
@@ -144,6 +143,29 @@ __global__ __launch_bounds__(256) void gguf_wide_table(const uint16_t *__restric
     }
   if (tid == 0) reinterpret_cast<float *>(table + gguf_wide_scales_offset(p.input_size, p.tiles))[row] = inverseScale;
 }
+__device__ __forceinline__ uint32_t wide_table_row_of(uint32_t block) {
+  const uint32_t die = block % 8u, slot = block / 8u;
+  return (slot / 8u * 8u + die) * 8u + slot % 8u;
+}
+template <bool Norm, uint32_t Held>
+__global__ __launch_bounds__(256) void gguf_wide_table(const uint16_t *__restrict__ input, const uint16_t *__restrict__ weight,
+                                                       uint8_t *__restrict__ table, GgufWideTableParams p) {
+  const uint32_t row = wide_table_row_of(blockIdx.x);
+  if (row < 16u * p.tiles) wide_table_row<Norm, Held>(input, weight, table, p, row, row);
+}
+// The table of the rows that a mixture's slots gather (or, Gathers false, of the slots' own rows): row s is row slot_row[s]
+// of the input, zeros where the slot is empty, for the slots of the tiles there are.
+template <bool Gathers>
+__global__ __launch_bounds__(256) void gguf_wide_moe_table(const uint16_t *__restrict__ input, const uint32_t *__restrict__ slot_row,
+                                                           const uint32_t *__restrict__ tile_total, uint8_t *__restrict__ table,
+                                                           GgufWideTableParams p) {
+  const uint32_t row = wide_table_row_of(blockIdx.x);
+  if (row >= 16u * min(p.tiles, tile_total[0])) return;
+  const uint32_t source = slot_row[row];
+  wide_table_row<false, 4>(input, nullptr, table, p, row, Gathers || source == MOE_NO_ROW ? source : row);
+}
+SP_REGISTER_KERNEL("gguf_wide_moe_gather", &gguf_wide_moe_table<true>);
+SP_REGISTER_KERNEL("gguf_wide_moe_rows", &gguf_wide_moe_table<false>);
 SP_REGISTER_KERNEL("gguf_wide_table", (&gguf_wide_table<false, 4>));
 SP_REGISTER_KERNEL("gguf_wide_table_long", (&gguf_wide_table<false, 16>));
 SP_REGISTER_KERNEL("gguf_wide_table_norm", (&gguf_wide_table<true, 4>));
@@ -312,55 +334,63 @@ template <uint32_t T> struct WideShared {
   uint4 sums[(T + 3) / 4 * 4][64];
 };
 
-// T: the row tiles a workgroup computes, at least those it takes (a tile past them multiplies zeros).
-template <uint32_t FMT, uint32_t EP, uint32_t T, bool Staged = false>
-__global__ __launch_bounds__(256, 2) void gguf_wide(const uint8_t *__restrict__ seg0, const uint8_t *__restrict__ seg1, const uint8_t *__restrict__ seg2,
-                                                    const uint8_t *__restrict__ table, void *__restrict__ out, const uint16_t *__restrict__ residual,
-                                                    GgufWideParams p) {
-  constexpr uint32_t kRecord = gguf_record_bytes(FMT);
-  constexpr bool kSums = FMT != GGUF_FMT_Q6K && !Staged, kTwice = FMT == GGUF_FMT_Q6K && !Staged, kGateUp = EP == GGUF_WIDE_GATE_UP;
-  __shared__ WideShared<T> shared;
-  const uint32_t perDie = gridDim.x / 8u, item = (blockIdx.x % 8u) * perDie + blockIdx.x / 8u;
-  if (item >= p.row_groups * p.splits * p.groups) return;
-  const uint32_t rowGroup = item % p.row_groups, rest = item / p.row_groups, split = rest % p.splits, columnGroup = rest / p.splits;
-  const uint32_t lane = threadIdx.x & 63u, wave = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6))), c = lane & 15u, kq = lane >> 4;
-  const uint32_t blocks = p.input_size / GGUF_BLOCK, liveTiles = (p.rows + 15u) / 16u;
-  const uint32_t tile0 = liveTiles * rowGroup / p.row_groups, tilesHere = liveTiles * (rowGroup + 1u) / p.row_groups - tile0;
-  const uint32_t b0 = blocks * split / p.splits, b1 = blocks * (split + 1u) / p.splits, count = b1 - b0;
-
-  // This wave's two column tiles: neighbours, or of a gate/up pair the same columns of both tensors.
+// What a workgroup computes: its wave's two column tiles (image null: a tile past the last), its row tiles, its part of K.
+struct WideTile {
   const uint8_t *image[2];
   uint32_t column[2];
-  if constexpr (kGateUp) {
-    const uint32_t tile = columnGroup * 4u + wave;
-    image[0] = seg0 + size_t(tile) * blocks * kRecord;
-    image[1] = seg1 + size_t(tile) * blocks * kRecord;
-    column[0] = column[1] = p.offset[0] + tile * 16u;
+  uint32_t tile0, tilesHere, rows;   // rows: those of the output
+  uint32_t b0, count, split;
+};
+// The two column tiles of wave `wave` of column group `group`: neighbours, or of a gate/up pair the same columns of both.
+template <uint32_t FMT, bool GateUp>
+__device__ __forceinline__ void wide_columns(WideTile &w, const uint8_t *seg0, const uint8_t *seg1, const uint8_t *seg2, const GgufWideParams &p,
+                                             uint32_t group, uint32_t wave) {
+  const uint64_t tileBytes = uint64_t(p.input_size / GGUF_BLOCK) * gguf_record_bytes(FMT);
+  if constexpr (GateUp) {
+    const uint32_t tile = group * 4u + wave;
+    const bool live = tile * 16u < p.cols[0];
+    w.image[0] = live ? seg0 + tile * tileBytes : nullptr;
+    w.image[1] = live ? seg1 + tile * tileBytes : nullptr;
+    w.column[0] = w.column[1] = p.offset[0] + tile * 16u;
   } else {
-    uint32_t group = columnGroup;
     const uint8_t *seg = seg0;
-    uint32_t offset = p.offset[0];
-    const uint32_t first = p.cols[0] / GGUF_WIDE_COLUMNS, second = p.cols[1] / GGUF_WIDE_COLUMNS;
+    uint32_t offset = p.offset[0], columns = p.cols[0];
+    const uint32_t first = (p.cols[0] + GGUF_WIDE_COLUMNS - 1u) / GGUF_WIDE_COLUMNS, second = (p.cols[1] + GGUF_WIDE_COLUMNS - 1u) / GGUF_WIDE_COLUMNS;
     if (group >= first) {
       group -= first;
       seg = seg1;
       offset = p.offset[1];
+      columns = p.cols[1];
       if (group >= second) {
         group -= second;
         seg = seg2;
         offset = p.offset[2];
+        columns = p.cols[2];
       }
     }
 #pragma unroll
     for (uint32_t r = 0; r < 2; ++r) {
       const uint32_t tile = group * 8u + wave * 2u + r;
-      image[r] = seg + size_t(tile) * blocks * kRecord;
-      column[r] = offset + tile * 16u;
+      w.image[r] = tile * 16u < columns ? seg + tile * tileBytes : nullptr;
+      w.column[r] = offset + tile * 16u;
     }
   }
+}
+
+// T: the row tiles a workgroup computes, at least those it takes (a tile past them multiplies zeros).
+template <uint32_t FMT, uint32_t EP, uint32_t T, bool Staged>
+__device__ __forceinline__ void wide_workgroup(const WideTile &w, const uint8_t *__restrict__ table, void *__restrict__ out,
+                                               const uint16_t *__restrict__ residual, const GgufWideParams &p) {
+  constexpr uint32_t kRecord = gguf_record_bytes(FMT);
+  constexpr bool kSums = FMT != GGUF_FMT_Q6K && !Staged, kTwice = FMT == GGUF_FMT_Q6K && !Staged, kGateUp = EP == GGUF_WIDE_GATE_UP;
+  __shared__ WideShared<T> shared;
+  const uint32_t lane = threadIdx.x & 63u, c = lane & 15u, kq = lane >> 4;
+  const uint32_t tile0 = w.tile0, tilesHere = w.tilesHere, b0 = w.b0, count = w.count, split = w.split;
+  const uint32_t column[2] = {w.column[0], w.column[1]};
   Resource weights[2];
 #pragma unroll
-  for (uint32_t r = 0; r < 2; ++r) weights[r] = make_resource(image[r] + size_t(b0) * kRecord, count * kRecord);
+  for (uint32_t r = 0; r < 2; ++r)
+    weights[r] = make_resource(w.image[r] ? w.image[r] + size_t(b0) * kRecord : table, w.image[r] ? count * kRecord : 0u);
   const uint32_t tileBytes = uint32_t(gguf_wide_tile_bytes(p.input_size));
   // (row tiles past the workgroup's, and super-blocks past its range, read as zeros or are not used)
   const Resource rowValues = make_resource(table + size_t(tile0) * tileBytes, tilesHere * tileBytes);
@@ -511,17 +541,19 @@ __global__ __launch_bounds__(256, 2) void gguf_wide(const uint8_t *__restrict__ 
 #pragma unroll
     for (uint32_t v = 0; v < 4; ++v) {
       const uint32_t row = 16u * (tile0 + t) + 4u * kq + v;
-      if (row >= p.rows) continue;
+      if (row >= w.rows) continue;
       const float scale = inverse[row];
       if constexpr (kGateUp) {
+        if (!w.image[0]) continue;
         const float gate = round_bf16(acc[0][t][v] * scale), up = round_bf16(acc[1][t][v] * scale);
         static_cast<uint16_t *>(out)[size_t(row) * p.out_stride + column[0] + c] = uint16_t(float_to_bf16_bits(up * silu(gate)));
       } else {
 #pragma unroll
         for (uint32_t r = 0; r < 2; ++r) {
+          if (!w.image[r]) continue;
           const float value = acc[r][t][v] * scale;
           const size_t at = size_t(row) * p.out_stride + column[r] + c;
-          if constexpr (EP == GGUF_WIDE_PARTIAL) static_cast<float *>(out)[size_t(split) * p.rows * p.out_stride + at] = value;
+          if constexpr (EP == GGUF_WIDE_PARTIAL) static_cast<float *>(out)[size_t(split) * w.rows * p.out_stride + at] = value;
           else if constexpr (EP == GGUF_WIDE_RESIDUAL)
             static_cast<uint16_t *>(out)[at] = uint16_t(float_to_bf16_bits(value + bf16_bits_to_float(residual[at])));
           else static_cast<uint16_t *>(out)[at] = uint16_t(float_to_bf16_bits(value));
@@ -529,6 +561,47 @@ __global__ __launch_bounds__(256, 2) void gguf_wide(const uint8_t *__restrict__ 
       }
     }
   }
+}
+template <uint32_t FMT, uint32_t EP, uint32_t T, bool Staged = false>
+__global__ __launch_bounds__(256, 2) void gguf_wide(const uint8_t *__restrict__ seg0, const uint8_t *__restrict__ seg1, const uint8_t *__restrict__ seg2,
+                                                    const uint8_t *__restrict__ table, void *__restrict__ out, const uint16_t *__restrict__ residual,
+                                                    GgufWideParams p) {
+  const uint32_t perDie = gridDim.x / 8u, item = (blockIdx.x % 8u) * perDie + blockIdx.x / 8u;
+  if (item >= p.row_groups * p.splits * p.groups) return;
+  const uint32_t rowGroup = item % p.row_groups, rest = item / p.row_groups;
+  const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)));
+  const uint32_t blocks = p.input_size / GGUF_BLOCK, liveTiles = (p.rows + 15u) / 16u;
+  WideTile w;
+  w.split = rest % p.splits;
+  w.tile0 = liveTiles * rowGroup / p.row_groups;
+  w.tilesHere = liveTiles * (rowGroup + 1u) / p.row_groups - w.tile0;
+  w.rows = p.rows;
+  w.b0 = blocks * w.split / p.splits;
+  w.count = blocks * (w.split + 1u) / p.splits - w.b0;
+  wide_columns<FMT, EP == GGUF_WIDE_GATE_UP>(w, seg0, seg1, seg2, p, rest / p.splits, wave);
+  wide_workgroup<FMT, EP, T, Staged>(w, table, out, residual, p);
+}
+// The routed experts of a prompt chunk: a task is up to T of an expert's row tiles (moe_chunk_place lists them), an item a
+// task's column group, the groups of a task side by side. Output rows are the slots'.
+template <uint32_t FMT, uint32_t EP, uint32_t T>
+__global__ __launch_bounds__(256, 2) void gguf_wide_moe(const uint8_t *__restrict__ seg0, const uint8_t *__restrict__ seg1, const uint8_t *__restrict__ table,
+                                                        void *__restrict__ out, const MoeChunkTask *__restrict__ tasks,
+                                                        const uint32_t *__restrict__ totals, GgufWideMoeParams m) {
+  const GgufWideParams &p = m.wide;
+  const uint32_t items = totals[1] * p.groups, perDie = (items + 7u) / 8u, item = (blockIdx.x % 8u) * perDie + blockIdx.x / 8u;
+  if (blockIdx.x / 8u >= perDie || item >= items) return;
+  const MoeChunkTask task = tasks[item / p.groups];
+  const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)));
+  WideTile w;
+  w.split = 0;
+  w.tile0 = uint32_t(__builtin_amdgcn_readfirstlane(int(task.first_tile)));
+  w.tilesHere = uint32_t(__builtin_amdgcn_readfirstlane(int(task.tiles)));
+  w.rows = (w.tile0 + w.tilesHere) * 16u;
+  w.b0 = 0;
+  w.count = p.input_size / GGUF_BLOCK;
+  const uint64_t expertAt = task.expert * m.expert_bytes;
+  wide_columns<FMT, EP == GGUF_WIDE_GATE_UP>(w, seg0 + expertAt, seg1 + expertAt, seg0 + expertAt, p, item % p.groups, wave);
+  wide_workgroup<FMT, EP, T, false>(w, table, out, nullptr, p);
 }
 #define SP_GGUF_WIDE_T(fmt, FMT, T)                                                          \
   SP_REGISTER_KERNEL("gguf_wide_" fmt "_t" #T "_a", (&gguf_wide<FMT, GGUF_WIDE_PLAIN, T>));        \
@@ -553,8 +626,21 @@ SP_GGUF_WIDE("q4k", GGUF_FMT_Q4K);
 SP_GGUF_WIDE("q5k", GGUF_FMT_Q5K);
 SP_GGUF_WIDE("q6k", GGUF_FMT_Q6K);
 
-template <bool Residual>
-__global__ __launch_bounds__(256) void gguf_wide_reduce(const float4 *__restrict__ partials, uint2 *__restrict__ out,
+#define SP_GGUF_WIDE_MOE(fmt, FMT, T)                                                             \
+  SP_REGISTER_KERNEL("gguf_wide_moe_" fmt "_t" #T "_g", (&gguf_wide_moe<FMT, GGUF_WIDE_GATE_UP, T>)); \
+  SP_REGISTER_KERNEL("gguf_wide_moe_" fmt "_t" #T "_a", (&gguf_wide_moe<FMT, GGUF_WIDE_PLAIN, T>))
+SP_GGUF_WIDE_MOE("q4k", GGUF_FMT_Q4K, 2);
+SP_GGUF_WIDE_MOE("q4k", GGUF_FMT_Q4K, 4);
+SP_GGUF_WIDE_MOE("q4k", GGUF_FMT_Q4K, 5);
+SP_GGUF_WIDE_MOE("q5k", GGUF_FMT_Q5K, 2);
+SP_GGUF_WIDE_MOE("q5k", GGUF_FMT_Q5K, 4);
+SP_GGUF_WIDE_MOE("q5k", GGUF_FMT_Q5K, 5);
+SP_GGUF_WIDE_MOE("q6k", GGUF_FMT_Q6K, 2);
+SP_GGUF_WIDE_MOE("q6k", GGUF_FMT_Q6K, 4);
+SP_GGUF_WIDE_MOE("q6k", GGUF_FMT_Q6K, 5);
+
+template <bool Residual, bool Float = false>
+__global__ __launch_bounds__(256) void gguf_wide_reduce(const float4 *__restrict__ partials, void *__restrict__ out,
                                                         const uint2 *__restrict__ residual, GgufWideReduceParams p) {
   const uint64_t at = uint64_t(blockIdx.x) * 256u + threadIdx.x, all = uint64_t(p.rows) * (p.columns / 4u);
   if (at >= all) return;
@@ -571,9 +657,11 @@ __global__ __launch_bounds__(256) void gguf_wide_reduce(const float4 *__restrict
     sum = make_float4(sum.x + bf16_bits_to_float(r.x & 0xFFFFu), sum.y + bf16_bits_to_float(r.x >> 16), sum.z + bf16_bits_to_float(r.y & 0xFFFFu),
                       sum.w + bf16_bits_to_float(r.y >> 16));
   }
-  out[at] = make_uint2(float_to_bf16_bits(sum.x) | (float_to_bf16_bits(sum.y) << 16), float_to_bf16_bits(sum.z) | (float_to_bf16_bits(sum.w) << 16));
+  if constexpr (Float) static_cast<float4 *>(out)[at] = sum;
+  else static_cast<uint2 *>(out)[at] = make_uint2(float_to_bf16_bits(sum.x) | (float_to_bf16_bits(sum.y) << 16), float_to_bf16_bits(sum.z) | (float_to_bf16_bits(sum.w) << 16));
 }
 SP_REGISTER_KERNEL("gguf_wide_reduce_a", &gguf_wide_reduce<false>);
+SP_REGISTER_KERNEL("gguf_wide_reduce_f32", (&gguf_wide_reduce<false, true>));
 SP_REGISTER_KERNEL("gguf_wide_reduce_r", &gguf_wide_reduce<true>);
 
 } // namespace splash::kernels

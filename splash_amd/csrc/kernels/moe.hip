@@ -147,6 +147,101 @@ __global__ __launch_bounds__(1024) void moe_group_routes(const uint32_t *__restr
 }
 SP_REGISTER_KERNEL("moe_group_routes", &moe_group_routes);
 
+// The chunk's grouping (abi/Moe.h). Counting is an LDS histogram; placing repeats moe_group_routes' bit matrix for a
+// window's routes, offset by the expert's first slot and the windows before: both follow from the counts of every window,
+// which each workgroup sums for itself.
+__global__ __launch_bounds__(1024) void moe_chunk_count(const uint32_t *__restrict__ selected, uint32_t *__restrict__ counts, MoeChunkParams p) {
+  __shared__ uint32_t bins[MOE_MAXIMUM_EXPERTS];
+  const uint32_t tid = threadIdx.x, first = blockIdx.x * MOE_CHUNK_ROUTES, last = min(p.routes, first + MOE_CHUNK_ROUTES);
+  if (tid < MOE_MAXIMUM_EXPERTS) bins[tid] = 0u;
+  __syncthreads();
+  for (uint32_t route = first + tid; route < last; route += 1024u) atomicAdd(&bins[selected[route]], 1u);
+  __syncthreads();
+  if (tid < p.experts) counts[blockIdx.x * p.experts + tid] = bins[tid];
+}
+SP_REGISTER_KERNEL("moe_chunk_count", &moe_chunk_count);
+
+__global__ __launch_bounds__(1024) void moe_chunk_place(const uint32_t *__restrict__ selected, const uint32_t *__restrict__ counts,
+                                                        uint32_t *__restrict__ route_slot, uint32_t *__restrict__ slot_row,
+                                                        MoeChunkTask *__restrict__ tasks, uint32_t *__restrict__ totals, MoeChunkParams p) {
+  constexpr uint32_t kWords = MOE_CHUNK_ROUTES / 32u, kMine = MOE_CHUNK_ROUTES / 1024u;
+  __shared__ uint32_t masks[MOE_MAXIMUM_EXPERTS * kWords];
+  __shared__ uint16_t before[MOE_MAXIMUM_EXPERTS * kWords];
+  __shared__ uint32_t firstSlot[MOE_MAXIMUM_EXPERTS], waveTiles[MOE_MAXIMUM_EXPERTS / 64u], waveTasks[MOE_MAXIMUM_EXPERTS / 64u];
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, window = blockIdx.x, windows = gridDim.x;
+  const uint32_t firstRoute = window * MOE_CHUNK_ROUTES, mineCount = min(p.routes - firstRoute, MOE_CHUNK_ROUTES);
+  for (uint32_t i = tid; i < p.experts * kWords; i += 1024u) masks[i] = 0u;
+  uint32_t mine[kMine];
+#pragma unroll
+  for (uint32_t i = 0; i < kMine; ++i) mine[i] = tid + 1024u * i < mineCount ? selected[firstRoute + tid + 1024u * i] : 0u;
+  // thread e: expert e's routes in all and in the windows before
+  uint32_t total = 0, earlier = 0;
+  if (tid < p.experts)
+    for (uint32_t w = 0; w < windows; ++w) {
+      const uint32_t c = counts[w * p.experts + tid];
+      total += c;
+      if (w < window) earlier += c;
+    }
+  const uint32_t tiles = (total + MOE_TILE_ROWS - 1u) / MOE_TILE_ROWS, parts = (tiles + p.task_tiles - 1u) / p.task_tiles;
+  uint32_t runningTiles = tiles, runningTasks = parts;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t a = uint32_t(__shfl_up(int(runningTiles), o, 64)), b = uint32_t(__shfl_up(int(runningTasks), o, 64));
+    if (lane >= uint32_t(o)) {
+      runningTiles += a;
+      runningTasks += b;
+    }
+  }
+  if (lane == 63u && tid < MOE_MAXIMUM_EXPERTS) {
+    waveTiles[wave] = runningTiles;
+    waveTasks[wave] = runningTasks;
+  }
+  __syncthreads();
+  if (tid < MOE_MAXIMUM_EXPERTS) {
+    uint32_t tile = runningTiles - tiles, task = runningTasks - parts;
+    for (uint32_t w = 0; w < wave; ++w) {
+      tile += waveTiles[w];
+      task += waveTasks[w];
+    }
+    firstSlot[tid] = tile * MOE_TILE_ROWS + earlier;
+    if (window == 0) {
+      for (uint32_t i = 0; i < parts; ++i) {
+        const uint32_t from = tiles * i / parts, to = tiles * (i + 1u) / parts;
+        tasks[task + i] = MoeChunkTask{tid, tile + from, to - from, 0u};
+      }
+      for (uint32_t slot = total; slot < tiles * MOE_TILE_ROWS; ++slot) slot_row[tile * MOE_TILE_ROWS + slot] = MOE_NO_ROW;
+      if (tid == MOE_MAXIMUM_EXPERTS - 1u) {
+        totals[0] = tile + tiles;
+        totals[1] = task + parts;
+      }
+    }
+  }
+#pragma unroll
+  for (uint32_t i = 0; i < kMine; ++i) {
+    const uint32_t route = tid + 1024u * i;
+    if (route < mineCount) atomicOr(&masks[mine[i] * kWords + route / 32u], 1u << (route % 32u));
+  }
+  __syncthreads();
+  if (tid < p.experts) {
+    uint32_t run = 0;
+    for (uint32_t w = 0; w < kWords; ++w) {
+      before[tid * kWords + w] = uint16_t(run);
+      run += uint32_t(__builtin_popcount(masks[tid * kWords + w]));
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t i = 0; i < kMine; ++i) {
+    const uint32_t route = tid + 1024u * i;
+    if (route >= mineCount) continue;
+    const uint32_t at = mine[i] * kWords + route / 32u;
+    const uint32_t slot = firstSlot[mine[i]] + before[at] + uint32_t(__builtin_popcount(masks[at] & ((1u << (route % 32u)) - 1u)));
+    route_slot[firstRoute + route] = slot;
+    slot_row[slot] = (firstRoute + route) / p.top_k;
+  }
+}
+SP_REGISTER_KERNEL("moe_chunk_place", &moe_chunk_place);
+
 // moe_gather_table: the activation table (abi/Gguf.h) of each tile's gathered rows, as
 // gguf_prepare_table writes a block's; empty slots are zero rows.
 __global__ __launch_bounds__(64) void moe_gather_table(const uint16_t *__restrict__ input, const uint32_t *__restrict__ slot_row,

@@ -116,6 +116,26 @@ HybridVerify::HybridVerify(hip::Backend &backend, HybridDimensions d, uint32_t m
   sampling_.uniforms = uniforms_;
   sampling_.inputTokens = inputTokens_;
   sampling_.treeRows = treeRows_;
+  if (wideChunks()) {
+    const uint32_t widest = std::max({d.hidden, d.attentionWidth(), d.gdnWidth(), d.dense() ? d.denseFfn : 0u});
+    wideTable_ = device(ops::Linear::wideTableBytes(widest, rowCapacity_), "wide table");
+    uint64_t partials = 0;
+    for (ops::LinearMatrix m : {ops::LinearMatrix{d.qkvWidth(), d.hidden}, ops::LinearMatrix{d.gdnPackedWidth, d.hidden}, ops::LinearMatrix{d.hidden, d.attentionWidth()},
+                                ops::LinearMatrix{d.hidden, d.gdnWidth()},
+                                d.dense() ? ops::LinearMatrix{d.hidden, d.denseFfn} : ops::LinearMatrix{d.experts, d.hidden}})
+      partials = std::max(partials, linear_.widePartialBytes(m, rowCapacity_));
+    widePartials_ = device(partials, "wide partials");
+    if (d.dense()) {
+      wideRows_ = device(C * d.denseFfn * 2, "chunk SwiGLU rows");
+    } else {
+      wideScores_ = device(C * d.experts * 4, "chunk router scores");
+      const ops::MoeChunkWorkspaceSize chunk = ops::MoE::chunkWorkspace(d.moeShape(), rowCapacity_);
+      moeChunk_ = {device(chunk.selected, "moe chunk selected"), device(chunk.weights, "moe chunk weights"), device(chunk.routeSlot, "moe chunk route slots"),
+                   device(chunk.slotRow, "moe chunk slot rows"), device(chunk.counts, "moe chunk counts"), device(chunk.tasks, "moe chunk tasks"),
+                   device(chunk.totals, "moe chunk totals"), device(chunk.table, "moe chunk tables"), device(chunk.intermediate, "moe chunk SwiGLU rows"),
+                   device(chunk.expertOutput, "moe chunk expert outputs")};
+    }
+  }
   // The rows a Gated DeltaNet layer's prefill passes hand each other, for the longest chunk.
   const uint64_t keyWidth = uint64_t{d.gdnKeyHeads} * GDN_HEAD_DIMENSION;
   gdnPrefill_.queries = device(C * keyWidth * 2, "GDN prefill queries");
@@ -124,6 +144,25 @@ HybridVerify::HybridVerify(hip::Backend &backend, HybridDimensions d, uint32_t m
   gdnPrefill_.decay = device(C * d.gdnValueHeads * 4, "GDN prefill decay");
   gdnPrefill_.beta = device(C * d.gdnValueHeads * 2, "GDN prefill beta");
   gdnPrefill_.recurrentRows = device(C * d.gdnWidth() * 2, "GDN prefill rows");
+}
+
+// Whether chunks may take the wide kernels (DenseVerify::wideChunks has the reason for the line).
+bool HybridVerify::wideChunks() const noexcept {
+  return rowCapacity_ >= kWideRows && dims_.hidden >= kWideHidden && dims_.hidden <= ops::Linear::kMaximumWideNormWidth;
+}
+bool HybridVerify::takesWide(uint32_t tokens) const {
+  if (!wideChunks() || tokens < kWideRows) return false;
+  for (const HybridLayer &l : weights_.layers) {
+    if (!ops::Linear::takesWide(l.mixerInput) || !ops::Linear::takesWide(l.mixerOutput) || l.gateRows) return false;
+    if (dims_.dense()) {
+      for (const ops::Projection *p : {&l.ffnGate, &l.ffnUp, &l.ffnDown})
+        if (!ops::Linear::takesWide(*p) || p->blocks().segments.size() != 1) return false;
+      if (l.ffnGate.blocks().segments.front().formatId != l.ffnUp.blocks().segments.front().formatId) return false;
+    } else if (l.routerRows || !ops::Linear::takesWide(l.router) || !ops::MoE::takesWide(dims_.moeShape(), l.experts)) {
+      return false;
+    }
+  }
+  return true;
 }
 
 const hip::Buffer &HybridVerify::draftProbabilities() {
@@ -370,6 +409,54 @@ void HybridVerify::encode(hip::CommandGraph &graph, const std::vector<HybridLane
                                        layerBytes_);
 }
 
+// A layer of a prompt chunk through the wide kernels: every projection, and the experts, one pass over all the rows.
+void HybridVerify::encodeWidePrefillLayer(hip::CommandGraph &graph, uint32_t layer, const ops::AttentionPromptPlan &plan, uint32_t tokens,
+                                          uint64_t currentCell, uint64_t nextCell) {
+  const HybridLayer &w = weights_.layers.at(layer);
+  const bool attends = dims_.attends(layer);
+  const uint32_t index = dims_.mixerIndex(layer);
+  const hip::Buffer &residual = hidden_[0], &next = hidden_[1];
+  const uint32_t inputWidth = w.mixerInput.outputSize, mixedWidth = w.mixerOutput.inputSize;
+  if (inputWidth != (attends ? dims_.qkvWidth() : dims_.gdnPackedWidth) || mixedWidth != (attends ? dims_.attentionWidth() : dims_.gdnWidth()))
+    throw std::invalid_argument("the layer's projections do not fit the model");
+  ops::Linear::addWideNormTable(graph, residual, w.inputNorm, wideTable_, dims_.hidden, tokens);
+  linear_.addWide(graph, w.mixerInput, wideTable_, packed_, {}, widePartials_, tokens);
+  if (attends) {
+    const ops::KvPages pages{pageTable_, kvPools_.at(index), pageBytes_};
+    ops::PagedAttention::addPromptProjection(graph, plan, {packed_, w.queryNorm, w.keyNorm, ropeCos_, ropeSin_}, attentionWorkspace_, pages);
+    ops::PagedAttention::addPromptAttention(graph, plan, attentionWorkspace_, treeRows_, pages, mixed_, packed_);
+  } else {
+    addGdnPrefill(graph, w, index, tokens, currentCell, nextCell);
+  }
+  ops::Linear::addWideTable(graph, mixed_, wideTable_, mixedWidth, tokens);
+  linear_.addWide(graph, w.mixerOutput, wideTable_, next, residual, widePartials_, tokens);
+  ops::Linear::addWideNormTable(graph, next, w.postNorm, wideTable_, dims_.hidden, tokens);
+  if (dims_.dense()) {
+    linear_.addWideGateUp(graph, w.ffnGate, w.ffnUp, wideTable_, wideRows_, tokens);
+    ops::Linear::addWideTable(graph, wideRows_, wideTable_, dims_.denseFfn, tokens);
+    linear_.addWide(graph, w.ffnDown, wideTable_, residual, next, widePartials_, tokens);
+    return;
+  }
+  linear_.addWide(graph, w.router, wideTable_, wideScores_, {}, widePartials_, tokens);
+  ops::Normalization::addRms(graph, next, w.postNorm, normalized_, dims_.hidden, tokens);
+  ops::MoE::addChunk(graph, wideScores_, dims_.experts, normalized_, next, residual, w.experts, moeChunk_, dims_.moeShape(), tokens, w.sharedScalarGate);
+}
+
+void HybridVerify::addGdnPrefill(hip::CommandGraph &graph, const HybridLayer &w, uint32_t index, uint32_t tokens, uint64_t currentCell, uint64_t nextCell) {
+  ops::GdnPrefillBuffers buffers = gdnPrefill_;
+  buffers.packed = packed_;
+  buffers.convolutionWeights = w.convolutionWeights;
+  buffers.states = states_;
+  buffers.decayWeights = w.decay;
+  buffers.timeBias = w.timeBias;
+  buffers.mixerNorm = w.mixerNorm;
+  buffers.floatNorm = w.mixerNormFloat;
+  buffers.hidden = mixed_;
+  buffers.currentCell = currentCell;
+  buffers.nextCell = nextCell;
+  ops::GDN::addPrefill(graph, buffers, dims_.gdnShape(), index, tokens, strides_, tiledGdnHeads_ ? ops::GdnHeadOrder::Tiled : ops::GdnHeadOrder::Grouped);
+}
+
 // A layer of a prompt chunk: every window's mixer input rows, the mixer over all the chunk's rows, then every window's
 // output projection and FFN. No projection defers its norm here: a window starts with a norm pass.
 void HybridVerify::encodePrefillLayer(hip::CommandGraph &graph, uint32_t layer, const ops::AttentionChunkPlan &plan, uint32_t tokens,
@@ -402,19 +489,7 @@ void HybridVerify::encodePrefillLayer(hip::CommandGraph &graph, uint32_t layer, 
     ops::PagedAttention::addChunkProjection(graph, plan, {packed_, w.queryNorm, w.keyNorm, ropeCos_, ropeSin_}, attentionWorkspace_, pages);
     ops::PagedAttention::addChunkAttention(graph, plan, attentionWorkspace_, treeRows_, pages, mixed_, {}, packed_);
   } else {
-    ops::GdnPrefillBuffers buffers = gdnPrefill_;
-    buffers.packed = packed_;
-    buffers.convolutionWeights = w.convolutionWeights;
-    buffers.states = states_;
-    buffers.decayWeights = w.decay;
-    buffers.timeBias = w.timeBias;
-    buffers.mixerNorm = w.mixerNorm;
-    buffers.floatNorm = w.mixerNormFloat;
-    buffers.hidden = mixed_;
-    buffers.currentCell = currentCell;
-    buffers.nextCell = nextCell;
-    ops::GDN::addPrefill(graph, buffers, dims_.gdnShape(), index, tokens, strides_,
-                         tiledGdnHeads_ ? ops::GdnHeadOrder::Tiled : ops::GdnHeadOrder::Grouped);
+    addGdnPrefill(graph, w, index, tokens, currentCell, nextCell);
   }
   const ops::MoeShape moe = dims_.moeShape();
   forRowPieces(tokens, [&](uint32_t first, uint32_t count) {
@@ -452,9 +527,12 @@ void HybridVerify::encodePrefill(hip::CommandGraph &graph, uint32_t lane, uint32
   if (!tokens || tokens > rowCapacity_) throw std::invalid_argument("a prompt chunk takes 1 to the driver's most prefill rows");
   if (lane >= maxLanes_) throw std::invalid_argument("no such lane");
   if (firstLayer >= dims_.layers || layerCount > dims_.layers - firstLayer) throw std::invalid_argument("no such layers");
-  const ops::AttentionChunkPlan plan = ops::PagedAttention::planChunks(
-      {dims_.qHeads, dims_.kvHeads, dims_.headDimension, dims_.rotaryPairs, dims_.normalizeHeads, dims_.gatedAttention},
-      {{0, tokens, committed, tableFirst}});
+  const ops::AttentionGeometry geometry{dims_.qHeads, dims_.kvHeads, dims_.headDimension, dims_.rotaryPairs, dims_.normalizeHeads, dims_.gatedAttention};
+  const bool wide = takesWide(tokens);
+  ops::AttentionChunkPlan plan;
+  ops::AttentionPromptPlan widePlan;
+  if (wide) widePlan = ops::PagedAttention::planPrompt(geometry, {0, tokens, committed, tableFirst}, linear_.calibration().computeUnits);
+  else plan = ops::PagedAttention::planChunks(geometry, {{0, tokens, committed, tableFirst}});
   if (firstLayer == 0) {
     if (dims_.rotaryPairs) {
       // the RoPE tables eight blocks a dispatch, each dispatch over its own rows of the depths and tables
@@ -473,7 +551,8 @@ void HybridVerify::encodePrefill(hip::CommandGraph &graph, uint32_t lane, uint32
   }
   const uint32_t end = layerCount ? firstLayer + layerCount : dims_.layers;
   for (uint32_t layer = firstLayer; layer < end; ++layer) {
-    encodePrefillLayer(graph, layer, plan, tokens, cellOffset(lane, parity), cellOffset(lane, parity ^ 1u));
+    if (wide) encodeWidePrefillLayer(graph, layer, widePlan, tokens, cellOffset(lane, parity), cellOffset(lane, parity ^ 1u));
+    else encodePrefillLayer(graph, layer, plan, tokens, cellOffset(lane, parity), cellOffset(lane, parity ^ 1u));
     encodeCapture(graph, layer, tokens);
   }
 }

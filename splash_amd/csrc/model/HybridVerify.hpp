@@ -189,6 +189,16 @@ public:
 private:
   void encodePrefillLayer(hip::CommandGraph &graph, uint32_t layer, const ops::AttentionChunkPlan &plan, uint32_t tokens, uint64_t currentCell,
                           uint64_t nextCell);
+  // Chunks of at least kWideRows rows of a model at least kWideHidden wide take the wide kernels: chunks of more than
+  // one window of the step's kernels, which read every expert's weights once a window.
+  static constexpr uint32_t kWideHidden = 2048, kWideRows = 257;
+  [[nodiscard]] bool wideChunks() const noexcept;
+  [[nodiscard]] bool takesWide(uint32_t tokens) const;
+  void encodeWidePrefillLayer(hip::CommandGraph &graph, uint32_t layer, const ops::AttentionPromptPlan &plan, uint32_t tokens, uint64_t currentCell,
+                              uint64_t nextCell);
+  void addGdnPrefill(hip::CommandGraph &graph, const HybridLayer &layer, uint32_t index, uint32_t tokens, uint64_t currentCell, uint64_t nextCell);
+  hip::Buffer wideTable_, wideRows_, widePartials_, wideScores_;
+  ops::MoeChunkWorkspace moeChunk_;
   [[nodiscard]] ops::AttentionPlan planOf(const std::vector<HybridLane> &lanes) const;
   [[nodiscard]] hip::Buffer rowsOf(const hip::Buffer &buffer, uint32_t first, uint32_t count, uint64_t rowBytes) const {
     return backend_.view(buffer, first * rowBytes, count * rowBytes);

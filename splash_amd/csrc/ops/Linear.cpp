@@ -483,41 +483,50 @@ void Linear::addPrefill(hip::CommandGraph &graph, const hip::Buffer &input, cons
 }
 
 bool Linear::takesWide(const Projection &p) noexcept {
-  if (p.destination != FloatOutput::BFloat16 || p.inputSize > kMaximumWideWidth) return false;
+  if (p.inputSize > kMaximumWideWidth) return false;
   const std::vector<QuantizedSegment> &segments = p.blocks().segments;
   if (segments.empty() || segments.size() > GGUF_MAXIMUM_SEGMENTS) return false;
   const uint32_t format = segments.front().formatId;
   if (format != GGUF_FMT_Q4K && format != GGUF_FMT_Q5K && format != GGUF_FMT_Q6K) return false;
   for (const QuantizedSegment &s : segments)
-    if (s.formatId != format || s.outputSize % GGUF_WIDE_COLUMNS || s.columnOffset % GGUF_TILE_COLUMNS) return false;
+    if (s.formatId != format) return false;
   return true;
 }
 
 uint64_t Linear::wideTableBytes(uint32_t inputSize, uint32_t rows) noexcept { return gguf_wide_table_bytes(inputSize, rows); }
 
-// How a chunk's workgroups share the work: the row tiles dealt evenly over as few workgroups as hold them, and K in as
-// many parts as fill the device's rounds best. A compute unit holds two workgroups, so `items` workgroups take
-// ceil(items / (2 units)) rounds of 1 / splits of K each; a part more costs its partials' trip to memory and back.
+// How a chunk's workgroups share the work: the height of a workgroup (row tiles, dealt evenly) and the parts of K that
+// fill the device's rounds best, in microseconds. A compute unit holds two workgroups, so `items` workgroups take
+// ceil(items / (2 units)) rounds of 1 / splits of K each; a super-block of a round takes 0.55 for each row tile and for the
+// conversion of its weights as much as 2.2 of them (5.6 measured at eight tiles); parts cost a launch and their partials'
+// trip to memory and back.
 Linear::WideSplit Linear::wideSplit(uint32_t columnGroups, uint32_t blocks, uint32_t rows, bool splittable) const noexcept {
-  const uint32_t liveTiles = gguf_row_tiles(rows), rowGroups = (liveTiles + GGUF_WIDE_TILES - 1) / GGUF_WIDE_TILES;
-  const uint32_t most = (liveTiles + rowGroups - 1) / rowGroups, tiles = most <= 4 ? 4 : most <= 6 ? 6 : most;
-  const uint32_t slots = 2 * calibration_.computeUnits, items = rowGroups * columnGroups;
-  uint32_t splits = 1;
+  const uint32_t liveTiles = gguf_row_tiles(rows), slots = 2 * calibration_.computeUnits;
+  WideSplit chosen{1, GGUF_WIDE_TILES, 1};
   double best = 0;
-  for (uint32_t s = 1; splittable && s <= GGUF_WIDE_MAXIMUM_SPLITS && s * 4 <= blocks; ++s) {
-    const double cost = double((uint64_t{items} * s + slots - 1) / slots) / s + (s > 1 ? 0.05 + 0.02 * s : 0.0);
-    if (s == 1 || cost < best) { best = cost; splits = s; }
+  for (uint32_t tallest : {8u, 7u, 6u, 4u}) {
+    const uint32_t rowGroups = (liveTiles + tallest - 1) / tallest, items = rowGroups * columnGroups;
+    for (uint32_t s = 1; s == 1 || (splittable && s <= GGUF_WIDE_MAXIMUM_SPLITS && s * 2 <= blocks); ++s) {
+      const double cost = double((uint64_t{items} * s + slots - 1) / slots) / s * (2.2 + tallest) * blocks * 0.55 +
+                          (s > 1 ? 5.0 + double(s) * rows * columnGroups * GGUF_WIDE_COLUMNS * 8 / 4.5e6 : 0.0);
+      if (!best || cost < best) {
+        best = cost;
+        chosen = {rowGroups, tallest, s};
+      }
+    }
   }
-  return {rowGroups, tiles, splits};
+  return chosen;
 }
 
 uint64_t Linear::widePartialBytes(LinearMatrix matrix, uint32_t rows) const noexcept {
   uint64_t bytes = 0;
-  for (uint32_t r = 1; r <= rows; r = r == rows ? rows + 1 : std::min(rows, r + GGUF_ROW_TILE)) {
-    const WideSplit split = wideSplit(matrix.outputSize / GGUF_WIDE_COLUMNS, matrix.inputSize / GGUF_BLOCK, r, true);
-    // (a split of r rows may be that of any row count of the same tiles)
-    if (split.splits > 1) bytes = std::max(bytes, uint64_t{split.splits} * gguf_row_tiles(r) * GGUF_ROW_TILE * matrix.outputSize * 4);
-  }
+  // (every row tile count, and a column group more for each segment that ends inside one)
+  for (uint32_t tiles = 1; tiles <= gguf_row_tiles(rows); ++tiles)
+    for (uint32_t more = 0; more < GGUF_MAXIMUM_SEGMENTS; ++more) {
+      const uint32_t groups = (matrix.outputSize + GGUF_WIDE_COLUMNS - 1) / GGUF_WIDE_COLUMNS + more;
+      const WideSplit split = wideSplit(groups, matrix.inputSize / GGUF_BLOCK, tiles * GGUF_ROW_TILE, true);
+      if (split.splits > 1) bytes = std::max(bytes, uint64_t{split.splits} * tiles * GGUF_ROW_TILE * matrix.outputSize * 4);
+    }
   return bytes;
 }
 
@@ -568,13 +577,17 @@ void Linear::addWide(hip::CommandGraph &graph, const Projection &p, const hip::B
   const uint32_t n = p.outputSize, k = p.inputSize;
   if (!rows || rows > kMaximumPrefillRows) throw std::invalid_argument("a prompt chunk takes 1 to 16384 rows");
   requireSegments(p, {n, k});
-  if (!takesWide(p)) throw std::invalid_argument("the wide kernels take tensors of one K-quant format, whole 128-column workgroups, bf16 results");
+  if (!takesWide(p)) throw std::invalid_argument("the wide kernels take tensors of one K-quant format");
   requireBytes(table, gguf_wide_table_bytes(k, rows), "wide table");
-  requireBytes(output, uint64_t{rows} * n * 2, "projection output");
+  const bool float32 = p.destination == FloatOutput::Float32;
+  if (float32 && residual) throw std::invalid_argument("only a plain projection writes fp32");
+  requireBytes(output, uint64_t{rows} * n * (float32 ? 4 : 2), "projection output");
   if (residual) requireBytes(residual, uint64_t{rows} * n * 2, "projection residual");
   const std::vector<QuantizedSegment> &segments = p.blocks().segments;
-  const uint32_t groups = n / GGUF_WIDE_COLUMNS;
-  const WideSplit split = wideSplit(groups, k / GGUF_BLOCK, rows, bool(partials));
+  uint32_t groups = 0;
+  for (const QuantizedSegment &s : segments) groups += (s.outputSize + GGUF_WIDE_COLUMNS - 1) / GGUF_WIDE_COLUMNS;
+  // (unsplit fp32 rows are the partials of one part)
+  const WideSplit split = wideSplit(groups, k / GGUF_BLOCK, rows, bool(partials) && n % 4 == 0);
   if (split.splits > 1) requireBytes(partials, uint64_t{split.splits} * rows * n * 4, "projection partials");
   GgufWideParams params = wideParams(k, rows, n, groups, split.rowGroups, split.splits);
   hip::Buffer images[3];
@@ -586,12 +599,12 @@ void Linear::addWide(hip::CommandGraph &graph, const Projection &p, const hip::B
       params.offset[s] = segment.columnOffset;
     }
   }
-  const char *suffix = split.splits > 1 ? "_p" : residual ? "_r" : "_a";
+  const char *suffix = split.splits > 1 || float32 ? "_p" : residual ? "_r" : "_a";
   graph.add(wideName(segments.front().name(), staged, split.tiles, suffix),
             {images[0], images[1], images[2], table, split.splits > 1 ? partials : output, residual && split.splits == 1 ? residual : table}, params,
             {wideGrid(params), 1, 1}, {256, 1, 1});
   if (split.splits > 1)
-    graph.add(residual ? "gguf_wide_reduce_r" : "gguf_wide_reduce_a", {partials, output, residual ? residual : output},
+    graph.add(float32 ? "gguf_wide_reduce_f32" : residual ? "gguf_wide_reduce_r" : "gguf_wide_reduce_a", {partials, output, residual ? residual : output},
               GgufWideReduceParams{rows, n, split.splits, 0}, {uint32_t((uint64_t{rows} * n / 4 + 255) / 256), 1, 1}, {256, 1, 1});
 }
 
@@ -601,12 +614,12 @@ void Linear::addWideGateUp(hip::CommandGraph &graph, const Projection &gate, con
   if (!rows || rows > kMaximumPrefillRows) throw std::invalid_argument("a prompt chunk takes 1 to 16384 rows");
   requireSegments(gate, {n, k});
   requireSegments(up, {n, k});
-  if (!takesWide(gate) || !takesWide(up) || gate.blocks().segments.size() != 1 || up.blocks().segments.size() != 1 ||
+  if (!takesWide(gate) || !takesWide(up) || up.destination != FloatOutput::BFloat16 || gate.blocks().segments.size() != 1 || up.blocks().segments.size() != 1 ||
       gate.blocks().segments.front().formatId != up.blocks().segments.front().formatId)
     throw std::invalid_argument("a one-pass block gate/up takes single tensors of one format");
   requireBytes(table, gguf_wide_table_bytes(k, rows), "wide table");
   requireBytes(output, uint64_t{rows} * n * 2, "projection output");
-  const uint32_t groups = n / (GGUF_WIDE_COLUMNS / 2);
+  const uint32_t groups = (n + GGUF_WIDE_COLUMNS / 2 - 1) / (GGUF_WIDE_COLUMNS / 2);
   const WideSplit split = wideSplit(groups, k / GGUF_BLOCK, rows, false);
   GgufWideParams params = wideParams(k, rows, n, groups, split.rowGroups, 1);
   params.cols[0] = n;

@@ -234,8 +234,8 @@ public:
   static void addPrefill(hip::CommandGraph &graph, const hip::Buffer &input, const Projection &projection, const hip::Buffer &output,
                          const hip::Buffer &residual, const hip::Buffer &table, uint32_t rows);
   // The projections of a prompt chunk of many rows through the matrix cores' fp16 (kernels gguf_wide_*): the register
-  // rule's exact weights, or (staged) each rounded once to half. takesWide: whether the kernels take the projection (one
-  // format of Q4_K, Q5_K, Q6_K; tensors of whole 128-column workgroups; bf16 results). The rows enter as a wide table,
+  // rule's exact weights, or (staged) each rounded once to half. takesWide: whether the kernels take the projection (tensors
+  // of one format, Q4_K, Q5_K or Q6_K, up to 32768 inputs). The rows enter as a wide table,
   // which addWideTable makes of bf16 rows and addWideNormTable of their RMS norm (rows of up to 8192 values).
   static constexpr uint32_t kMaximumWideNormWidth = 8192, kMaximumWideWidth = 32768;
   [[nodiscard]] static bool takesWide(const Projection &projection) noexcept;

@@ -1,6 +1,7 @@
 #include "ops/Moe.hpp"
 #include "ops/Linear.hpp"  // requireBytes
 
+#include <algorithm>
 #include <stdexcept>
 #include <string>
 
@@ -131,6 +132,96 @@ void MoE::addRouted(hip::CommandGraph &graph, const hip::Buffer &normalized, con
              writesTable ? following.table : output},
             MoeCombineParams{rows, shape.hidden, shape.routesPerRow(), writesTable ? gguf_row_tiles(rows) : 0u},
             {rows, (shape.hidden + 255) / 256, 1}, {256, 1, 1});
+}
+
+namespace {
+bool wideFormat(uint32_t format) { return format == GGUF_FMT_Q4K || format == GGUF_FMT_Q5K || format == GGUF_FMT_Q6K; }
+// The row tiles of a task: what an expert's share of the routes comes to, and a tile more, in as few tasks as hold it.
+// (The kernels compute all of a task's tiles, live or not.)
+uint32_t taskTiles(uint32_t routes, uint32_t experts) {
+  const uint32_t expected = (routes + experts * MOE_TILE_ROWS - 1) / (experts * MOE_TILE_ROWS) + 1;
+  if (expected <= 2) return 2;
+  const uint32_t parts = (expected + 4) / 5;
+  return (expected + parts - 1) / parts <= 4 ? 4 : 5;
+}
+} // namespace
+
+bool MoE::takesWide(const MoeShape &shape, const MoeExperts &experts) noexcept {
+  return shape.valid() && wideFormat(experts.format) && wideFormat(experts.downFormat) && shape.hidden <= Linear::kMaximumWideNormWidth &&
+         shape.ffn <= Linear::kMaximumWideNormWidth;
+}
+
+MoeChunkWorkspaceSize MoE::chunkWorkspace(const MoeShape &shape, uint32_t rows) {
+  if (!shape.valid()) throw std::invalid_argument("invalid MoE shape");
+  if (!rows || rows > kMaximumChunkRows) throw std::invalid_argument("a prompt chunk holds 1 to 2048 rows");
+  const uint64_t routes = uint64_t{rows} * shape.routesPerRow(), tiles = moe_maximum_tiles(uint32_t(routes), shape.allExperts()),
+                 slots = tiles * MOE_TILE_ROWS, windows = (routes + MOE_CHUNK_ROUTES - 1) / MOE_CHUNK_ROUTES;
+  MoeChunkWorkspaceSize s;
+  s.selected = s.weights = s.routeSlot = routes * 4;
+  s.slotRow = slots * 4;
+  s.counts = windows * shape.allExperts() * 4;
+  s.tasks = (tiles / 2 + shape.allExperts()) * sizeof(MoeChunkTask);
+  s.totals = 16;
+  s.table = gguf_wide_table_bytes(std::max(shape.hidden, shape.ffn), uint32_t(slots));
+  s.intermediate = slots * shape.ffn * 2;
+  s.expertOutput = slots * shape.hidden * 2;
+  return s;
+}
+
+void MoE::addChunk(hip::CommandGraph &graph, const hip::Buffer &scores, uint32_t scoreStride, const hip::Buffer &normalized,
+                   const hip::Buffer &residual, const hip::Buffer &output, const MoeExperts &experts, const MoeChunkWorkspace &w,
+                   const MoeShape &shape, uint32_t rows, const hip::Buffer &sharedScalarGate) {
+  const MoeChunkWorkspaceSize need = chunkWorkspace(shape, rows);
+  if (!takesWide(shape, experts)) throw std::invalid_argument("the wide kernels take experts of K-quants, up to 8192 inputs");
+  if (scoreStride < shape.experts) throw std::invalid_argument("a row of scores holds every expert's");
+  if (shape.sharedGate) requireBytes(sharedScalarGate, uint64_t{shape.hidden} * 4, "shared expert gate");
+  const uint64_t pairBytes = gguf_image_bytes(experts.format, shape.ffn, shape.hidden), downBytes = gguf_image_bytes(experts.downFormat, shape.hidden, shape.ffn);
+  requireBytes(scores, (uint64_t{rows - 1} * scoreStride + shape.experts) * 4, "router scores");
+  requireBytes(normalized, uint64_t{rows} * shape.hidden * 2, "normalized rows");
+  requireBytes(residual, uint64_t{rows} * shape.hidden * 2, "residual rows");
+  requireBytes(output, uint64_t{rows} * shape.hidden * 2, "MoE output");
+  requireBytes(experts.gate, pairBytes * shape.allExperts(), "expert gate images");
+  requireBytes(experts.up, pairBytes * shape.allExperts(), "expert up images");
+  requireBytes(experts.down, downBytes * shape.allExperts(), "expert down images");
+  requireBytes(w.selected, need.selected, "selected experts");
+  requireBytes(w.weights, need.weights, "routing weights");
+  requireBytes(w.routeSlot, need.routeSlot, "route slots");
+  requireBytes(w.slotRow, need.slotRow, "slot rows");
+  requireBytes(w.counts, need.counts, "route counts");
+  requireBytes(w.tasks, need.tasks, "expert tasks");
+  requireBytes(w.totals, need.totals, "tile and task counts");
+  requireBytes(w.table, need.table, "slot tables");
+  requireBytes(w.intermediate, need.intermediate, "slot SwiGLU rows");
+  requireBytes(w.expertOutput, need.expertOutput, "expert outputs");
+
+  const uint32_t routes = rows * shape.routesPerRow(), all = shape.allExperts(), windows = (routes + MOE_CHUNK_ROUTES - 1) / MOE_CHUNK_ROUTES;
+  const uint32_t tiles = moe_maximum_tiles(routes, all), T = taskTiles(routes, all), mostTasks = tiles / T + all;
+  graph.add("moe_route_select", {scores, shape.sharedGate ? normalized : scores, shape.sharedGate ? sharedScalarGate : scores, w.selected, w.weights},
+            MoeRouteParams{rows, shape.experts, shape.topK, scoreStride, shape.sharedSlices, shape.sharedGate, shape.hidden, shape.sigmoidRouter},
+            {rows, 1, 1}, {64, 1, 1});
+  const MoeChunkParams grouping{routes, all, shape.routesPerRow(), T};
+  graph.add("moe_chunk_count", {w.selected, w.counts}, grouping, {windows, 1, 1}, {1024, 1, 1});
+  graph.add("moe_chunk_place", {w.selected, w.counts, w.routeSlot, w.slotRow, w.tasks, w.totals}, grouping, {windows, 1, 1}, {1024, 1, 1});
+  auto project = [&](const char *table, const hip::Buffer &input, uint32_t inputRows, uint32_t k, uint32_t n, uint32_t format, uint64_t expertBytes,
+                     const hip::Buffer &first, const hip::Buffer &second, const hip::Buffer &out, bool gateUp) {
+    graph.add(table, {input, w.slotRow, w.totals, w.table}, GgufWideTableParams{k, inputRows, tiles, 0}, {64 * ((16 * tiles + 63) / 64), 1, 1},
+              {256, 1, 1});
+    GgufWideMoeParams params{};
+    params.wide.input_size = k;
+    params.wide.tiles = tiles;
+    params.wide.out_stride = n;
+    const uint32_t span = gateUp ? GGUF_WIDE_COLUMNS / 2 : GGUF_WIDE_COLUMNS;
+    params.wide.groups = (n + span - 1) / span;
+    params.wide.cols[0] = n;
+    params.expert_bytes = expertBytes;
+    graph.add(std::string("gguf_wide_moe_") + gguf_format_name(format) + "_t" + std::to_string(T) + (gateUp ? "_g" : "_a"),
+              {first, second, w.table, out, w.tasks, w.totals}, params, {8 * ((mostTasks * params.wide.groups + 7) / 8), 1, 1}, {256, 1, 1});
+  };
+  project("gguf_wide_moe_gather", normalized, rows, shape.hidden, shape.ffn, experts.format, pairBytes, experts.gate, experts.up, w.intermediate, true);
+  project("gguf_wide_moe_rows", w.intermediate, 16 * tiles, shape.ffn, shape.hidden, experts.downFormat, downBytes, experts.down, experts.down,
+          w.expertOutput, false);
+  graph.add("moe_combine", {w.expertOutput, w.routeSlot, w.weights, residual, output, output, output},
+            MoeCombineParams{rows, shape.hidden, shape.routesPerRow(), 0u}, {rows, (shape.hidden + 255) / 256, 1}, {256, 1, 1});
 }
 
 } // namespace splash::ops

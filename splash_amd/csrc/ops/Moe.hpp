@@ -54,8 +54,27 @@ struct MoeFollowingNorm final {
   hip::Buffer table;   // gguf_tables_bytes(hidden, row tiles)
 };
 
+// A prompt chunk's experts through the wide kernels: the grouping of every row's routes at once, so that an expert's
+// weights are read for all of its rows, and the slots' rows as wide tables.
+struct MoeChunkWorkspaceSize final {
+  uint64_t selected = 0, weights = 0, routeSlot = 0, slotRow = 0, counts = 0, tasks = 0, totals = 0, table = 0, intermediate = 0, expertOutput = 0;
+};
+struct MoeChunkWorkspace final {
+  hip::Buffer selected, weights, routeSlot, slotRow, counts, tasks, totals;
+  hip::Buffer table;         // the wide table of the gathered rows, then of the SwiGLU rows
+  hip::Buffer intermediate;  // bf16 [slot][ffn]
+  hip::Buffer expertOutput;  // bf16 [slot][hidden]
+};
+
 class MoE final {
 public:
+  [[nodiscard]] static bool takesWide(const MoeShape &shape, const MoeExperts &experts) noexcept;
+  [[nodiscard]] static MoeChunkWorkspaceSize chunkWorkspace(const MoeShape &shape, uint32_t rows);
+  // What addRouting and addRouted do, for up to kMaximumChunkRows rows.
+  static constexpr uint32_t kMaximumChunkRows = 2048;
+  static void addChunk(hip::CommandGraph &graph, const hip::Buffer &scores, uint32_t scoreStride, const hip::Buffer &normalized,
+                       const hip::Buffer &residual, const hip::Buffer &output, const MoeExperts &experts, const MoeChunkWorkspace &workspace,
+                       const MoeShape &shape, uint32_t rows, const hip::Buffer &sharedScalarGate = {});
   [[nodiscard]] static MoeWorkspaceSize workspace(const MoeShape &shape, uint32_t rows);
   // Selects and weighs each row's experts from its fp32 router scores ([rows][scoreStride]), appends the shape's shared
   // slices to every row's routes and groups the routes. `input` (the normalized rows, bf16 [rows][hidden]) and

@@ -61,3 +61,57 @@ def test_a_wide_chunk_is_its_blocks_to_rounding(backend, tokens, down_format):
         print(f"  staged={staged}: hidden {far[0]:.5f}, q|k|v {far[1]:.5f}", flush=True)
         # the q|k|v rows come of the same bf16 rows either way; the hidden rows of several bf16 roundings after them
         assert far[0] <= 9e-3 and far[1] <= (2.5e-3 if staged else 1e-3)
+
+
+@pytest.mark.parametrize("tokens,experts,dense_ffn", [(257, 16, 0), (300, 80, 0), (300, 0, 512)])
+def test_a_wide_hybrid_chunk_is_its_short_chunks_to_rounding(backend, tokens, experts, dense_ffn):
+    """HybridVerify::encodeWidePrefillLayer: the experts' tasks (few and many rows an expert, a shared expert that every row
+    visits, experts with no row), a packed width that ends inside a column group, an attention layer with gates, a dense
+    FFN: the hidden rows and the recurrent state are those of the same prompt in chunks of 64 rows, which take the step's
+    kernels, but for rows whose near-equal router scores rank the other way."""
+    from tests.hybrid_reference import HybridModel
+    print(f"case wide hybrid chunk tokens={tokens} experts={experts}", flush=True)
+    H, V = 2048, 512
+    model = HybridModel(seed=53, hidden=H, vocabulary=V, layers=4, q_heads=8, kv_heads=2, head_dim=128, gdn_key_heads=2, gdn_value_heads=4,
+                        experts=experts, top_k=2 if experts else 0, expert_ffn=256 if experts else 0, shared_slices=1 if experts else 0,
+                        shared_gate=bool(experts), gated_attention=True, dense_ffn=dense_ffn)
+    gpu = model.build_gpu(backend, max_lanes=1, pages_per_lane=3, prefill_rows=tokens)
+    rng = np.random.default_rng(tokens)
+    model.seed_context(rng)
+    model.seed_states(rng, lanes=1)
+    committed = 200
+    prompt = rng.integers(0, V, tokens).astype(np.uint32)
+    start_pool, start_cells = gpu.buffer(verify.KV_POOL, 0).download(np.uint8), gpu.buffer(verify.GDN_STATES).download(np.uint8)
+
+    def restore():
+        gpu.buffer(verify.KV_POOL, 0).upload(start_pool)
+        gpu.buffer(verify.GDN_STATES).upload(start_cells)
+
+    def state(parity):
+        cell = gpu.buffer(verify.GDN_STATES).download(np.uint8, gpu.cell_bytes, gpu.cell_offset(0, parity))
+        return cell[gpu.strides.convolution_state_bytes:].view(np.float32).astype(np.float64)
+    hidden, parity = [], 0
+    restore()
+    for at in range(0, tokens, 64):
+        rows = min(64, tokens - at)
+        gpu.set_prefill_block(prompt[at:at + rows])
+        graph = gpu.encode_prefill(0, 0, committed + at, rows, parity=parity)
+        assert not any("wide" in name for name in graph.kernels())
+        backend.run(graph)
+        hidden.append(gpu.buffer(verify.HIDDEN, 0).download(np.uint16, rows * H).copy())
+        parity ^= 1
+    want, want_state = orc.bf16_to_f32(np.concatenate(hidden)).reshape(tokens, H).astype(np.float64), state(parity)
+    seen = []
+    for _ in range(2):
+        restore()
+        gpu.set_prefill_block(prompt)
+        graph = gpu.encode_prefill(0, 0, committed, tokens, parity=0)
+        assert any("wide" in name for name in graph.kernels())
+        backend.run(graph)
+        seen.append((gpu.buffer(verify.HIDDEN, 0).download(np.uint16, tokens * H).copy(), state(1)))
+    assert np.array_equal(seen[0][0], seen[1][0]) and np.array_equal(seen[0][1], seen[1][1])
+    got = orc.bf16_to_f32(seen[0][0]).reshape(tokens, H).astype(np.float64)
+    far = np.sqrt(((got - want) ** 2).sum(axis=1) / (want ** 2).sum(axis=1))
+    far_state = np.sqrt(((seen[0][1] - want_state) ** 2).sum() / (want_state ** 2).sum())
+    print(f"  rows: median {np.median(far):.5f}, 95th {np.percentile(far, 95):.5f}, worst {far.max():.5f}; state {far_state:.5f}", flush=True)
+    assert np.median(far) <= 1e-2 and np.percentile(far, 90) <= 2e-2 and far_state <= 2e-2
