@@ -52,4 +52,37 @@ template <class T> __device__ __forceinline__ T wave_max(T v) {
   return v;
 }
 
+// Maxima that move data between lanes with DPP row permutations and broadcasts, a few cycles each, and never through the
+// LDS crossbar: for reductions that follow one another, each waiting for the last. A lane no shift reaches keeps its own
+// value, which a maximum does not mind.
+template <int Control> __device__ __forceinline__ uint32_t dpp_move(uint32_t v) {
+  return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(v), static_cast<int>(v), Control, 0xF, 0xF, false));
+}
+constexpr int kRowShiftRight = 0x110, kRowBroadcast15 = 0x142, kRowBroadcast31 = 0x143;
+constexpr int kQuadSwap1 = 0xB1, kQuadSwap2 = 0x4E, kRowMirror = 0x140, kRowHalfMirror = 0x141;
+template <int Control> __device__ __forceinline__ uint32_t dpp_max(uint32_t v) { return max(v, dpp_move<Control>(v)); }
+template <int Control> __device__ __forceinline__ uint64_t dpp_max(uint64_t key) {
+  const uint64_t other = (uint64_t{dpp_move<Control>(static_cast<uint32_t>(key >> 32))} << 32) | dpp_move<Control>(static_cast<uint32_t>(key));
+  return other > key ? other : key;
+}
+// The largest of a wavefront, in every lane: after the shifts by 1, 2, 4 and 8 a row's last lane holds the row's largest,
+// after the two broadcasts lane 63 the wavefront's.
+template <class T> __device__ __forceinline__ T wave_max_dpp(T v) {
+  v = dpp_max<kRowShiftRight + 1>(v);
+  v = dpp_max<kRowShiftRight + 2>(v);
+  v = dpp_max<kRowShiftRight + 4>(v);
+  v = dpp_max<kRowShiftRight + 8>(v);
+  v = dpp_max<kRowBroadcast15>(v);
+  v = dpp_max<kRowBroadcast31>(v);
+  const uint32_t low = __builtin_amdgcn_readlane(static_cast<int>(static_cast<uint32_t>(v)), 63);
+  if constexpr (sizeof(T) == 4) return low;
+  else return (uint64_t{uint32_t(__builtin_amdgcn_readlane(static_cast<int>(static_cast<uint32_t>(v >> 32)), 63))} << 32) | low;
+}
+// The largest of each row of sixteen lanes, in every lane of the row.
+__device__ __forceinline__ uint32_t row_max_dpp(uint32_t v) {
+  return dpp_max<kRowMirror>(dpp_max<kRowHalfMirror>(dpp_max<kQuadSwap2>(dpp_max<kQuadSwap1>(v))));
+}
+// A wavefront's LDS writes before its later reads (its LDS operations are carried out in order).
+__device__ __forceinline__ void wave_lds_fence() { __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront"); }
+
 } // namespace splash::kernels

@@ -2,13 +2,15 @@
 // runtime/metal/abi/Sampling.h:209-241): over the candidates and edge scores draft_select_edges left, each lane grows a
 // tree of up to 16 rows best first by the estimate that the target accepts the path to a row.
 //
-// One wavefront a lane, and no heap: the tree's open steps ("entries": from a row to a token one deeper) sit in LDS, at
-// most five a row, and taking the best is one 64-bit maximum reduction over (estimate bits, complement of the entry's
-// number), which is exactly "the largest estimate, the earlier entry among equal ones". A row's expansion runs on sixteen
-// lanes, one a candidate: the tempered weights, the Gumbel keys of a sampled lane's draws (a hash of the row's key and the
-// candidate's token a lane), each draw a 16-lane maximum reduction. Sums whose order decides a float's bits (a
-// distribution's mass) are taken in candidate order, as a sequential statement takes them, so the values agree with it to
-// the rounding of exp and log alone.
+// One workgroup a lane. What does not depend on the tree (the distributions after every candidate, the lane's tempered ones
+// and the estimates) is computed first, for all 97 of them side by side; then one wavefront grows the tree, a serial chain
+// of up to 15 steps that is nothing but latency, so it holds the rows and the tree's open steps ("entries": from a row to a
+// token one deeper, at most five a row) in its lanes' registers and reads them by lane number: no heap, no barrier, and no
+// LDS write to wait for. The best entry is one 64-bit maximum over (estimate bits, complement of the entry's number),
+// exactly "the largest estimate, the earlier entry among equal ones"; a draw is a 16-lane maximum over the Gumbel keys (a
+// hash of the row's key and the candidate's token a lane). Sums whose order decides a float's bits (a distribution's mass)
+// are taken in candidate order, as a sequential statement takes them, so the values agree with it to the rounding of exp
+// and log alone. Eight lanes' trees of 16 rows: 61 -> 36 us (all of it in one wavefront, with LDS between the steps, before).
 #include "abi/PagedAttention.h"
 #include "abi/Sampling.h"
 #include "backend/KernelRegistry.hpp"
@@ -36,256 +38,267 @@ __device__ __forceinline__ uint32_t order_bits(float value) {
   const uint32_t bits = __float_as_uint(value);
   return (bits & 0x80000000u) ? ~bits : (bits | 0x80000000u);
 }
-// The largest key of each group of `Width` neighbouring lanes, in every lane of the group.
-template <int Width> __device__ __forceinline__ uint64_t group_max(uint64_t key) {
+// Lane `from`'s value (`from` the same in every lane).
+__device__ __forceinline__ uint32_t lane_value(uint32_t v, uint32_t from) {
+  return uint32_t(__builtin_amdgcn_readlane(int(v), int(__builtin_amdgcn_readfirstlane(int(from)))));
+}
+__device__ __forceinline__ float lane_value(float v, uint32_t from) { return __uint_as_float(lane_value(__float_as_uint(v), from)); }
+// A row's sixteen values in candidate order, summed in that order.
+__device__ __forceinline__ float ordered_sum(const float *values) {
+  float sum = 0.f;
 #pragma unroll
-  for (int step = 1; step < Width; step <<= 1) {
-    const uint32_t lo = uint32_t(__shfl_xor(int(uint32_t(key)), step, 64)), hi = uint32_t(__shfl_xor(int(uint32_t(key >> 32)), step, 64));
-    const uint64_t other = uint64_t(hi) << 32 | lo;
-    key = other > key ? other : key;
-  }
-  return key;
+  for (uint32_t c = 0; c < kCandidates; ++c) sum += values[c];
+  return sum;
 }
 
+// By position, predecessor and candidate: the draft's probability, the lane's tempered one, and its estimate.
 struct TreeState {
   float probability[kPositions][kCandidates][kCandidates];
+  float drafted[kPositions][kCandidates][kCandidates];
+  float estimate[kPositions][kCandidates][kCandidates];
+  uint32_t order[kPositions][kCandidates][kCandidates];
   uint8_t likeliest[kPositions][kCandidates][kChildren];
   uint32_t ids[kPositions][kCandidates];
-  // rows
-  uint32_t token[kRows], ancestors[kRows], parent[kRows], depth[kRows], onChain[kRows];
-  float q[kRows], estimate[kRows], cap[kRows];
-  uint64_t key[kRows];
-  uint8_t draw[kRows][kChildren];
-  float left[kRows][kChildren], next[kRows][kCandidates];
-  // entries: the steps the tree may still take, in the order made
-  float entryScore[kEntries];
-  uint32_t entryInfo[kEntries];  // kChainEntry | parent row << 16 | proposal position << 8 | candidate index; kDead once taken
 };
 
 } // namespace
 
-__global__ __launch_bounds__(64) void draft_select_tree(const uint32_t *__restrict__ candidates, const float *__restrict__ unary,
-                                                        const float *__restrict__ edges, const uint32_t *__restrict__ chain_tokens,
-                                                        const float *__restrict__ chain_rates, uint32_t *__restrict__ tokens,
-                                                        AttentionTreeRow *__restrict__ tree, float *__restrict__ scores,
-                                                        uint32_t *__restrict__ sizes, uint8_t *__restrict__ draws,
-                                                        float *__restrict__ next, float *__restrict__ caps, DraftTreeParams p) {
+__global__ __launch_bounds__(256) void draft_select_tree(const uint32_t *__restrict__ candidates, const float *__restrict__ unary,
+                                                         const float *__restrict__ edges, const uint32_t *__restrict__ chain_tokens,
+                                                         const float *__restrict__ chain_rates, uint32_t *__restrict__ tokens,
+                                                         AttentionTreeRow *__restrict__ tree, float *__restrict__ scores,
+                                                         uint32_t *__restrict__ sizes, uint8_t *__restrict__ draws,
+                                                         float *__restrict__ next, float *__restrict__ caps, DraftTreeParams p) {
   __shared__ TreeState s;
   const uint32_t lane = blockIdx.x, tid = threadIdx.x, i = tid & 15u;
   const size_t origin = size_t(lane) * kPositions * kCandidates;
+  const float temperature = p.temperature[lane], slope = p.slope[lane];
+  const uint32_t chain = tid < DRAFT_CHAIN_TOKENS ? chain_tokens[size_t(lane) * DRAFT_CHAIN_TOKENS + tid] : 0u;
+  constexpr uint32_t kRates = DRAFT_CHAIN_TOKENS * DRAFT_CHAIN_AGREEMENTS;
+  const float rates = tid < kRates ? chain_rates[size_t(lane) * kRates + tid] : 0.f;
 
-  // ---- The lattice: a thread a (position, predecessor candidate); position 0 follows the anchor alone.
-  for (uint32_t at = tid; at < kPositions * kCandidates; at += 64u) {
-    const uint32_t position = at / kCandidates, predecessor = at % kCandidates;
-    s.ids[position][predecessor] = candidates[origin + at];
-    if (position == 0 && predecessor != 0) continue;
-    const float *edge = edges + (origin + at) * kCandidates;
-    float score[kCandidates];
+  // ---- The lattice: sixteen threads, a candidate each, a predecessor (position 0 follows the anchor alone, predecessor 0;
+  // what the others compute there is not read), all positions side by side. Sixteen threads share a wavefront, whose LDS
+  // operations are in order, so nothing here waits for the workgroup.
+  {
+    const uint32_t predecessor = tid / kCandidates;
+    float score[kPositions], weight[kPositions];
 #pragma unroll
-    for (uint32_t c = 0; c < kCandidates; ++c) score[c] = unary[origin + position * kCandidates + c] + edge[c];
-    float best = score[0];
-#pragma unroll
-    for (uint32_t c = 1; c < kCandidates; ++c) best = fmaxf(best, score[c]);
-    float weight[kCandidates], mass = 0.f;
-#pragma unroll
-    for (uint32_t c = 0; c < kCandidates; ++c) {
-      weight[c] = expf(score[c] - best);
-      mass += weight[c];
+    for (uint32_t position = 0; position < kPositions; ++position) {
+      const size_t at = origin + position * kCandidates;
+      if (tid < kCandidates) s.ids[position][i] = candidates[at + i];
+      score[position] = unary[at + i] + edges[(at + predecessor) * kCandidates + i];
     }
+    auto largest = [](float v) {   // of sixteen, as fmaxf has it
+      v = fmaxf(v, __uint_as_float(dpp_move<kQuadSwap1>(__float_as_uint(v))));
+      v = fmaxf(v, __uint_as_float(dpp_move<kQuadSwap2>(__float_as_uint(v))));
+      v = fmaxf(v, __uint_as_float(dpp_move<kRowHalfMirror>(__float_as_uint(v))));
+      return fmaxf(v, __uint_as_float(dpp_move<kRowMirror>(__float_as_uint(v))));
+    };
 #pragma unroll
-    for (uint32_t c = 0; c < kCandidates; ++c) s.probability[position][predecessor][c] = weight[c] / mass;
-    // its four likeliest, the lower index first among equal scores: four passes over a key of (score, complement of index)
-    uint64_t last = ~uint64_t{0};
-    for (uint32_t child = 0; child < kChildren; ++child) {
-      uint64_t pick = 0;
+    for (uint32_t position = 0; position < kPositions; ++position) {
+      weight[position] = expf(score[position] - largest(score[position]));
+      s.probability[position][predecessor][i] = weight[position];
+      s.order[position][predecessor][i] = order_bits(score[position] + 0.0f);
+    }
+    wave_lds_fence();
+#pragma unroll
+    for (uint32_t position = 0; position < kPositions; ++position) {
+      // the four likeliest, the lower index first among equal scores
+      uint32_t rank = 0;
+      const uint32_t mine = order_bits(score[position] + 0.0f);
 #pragma unroll
       for (uint32_t c = 0; c < kCandidates; ++c) {
-        const uint64_t key = uint64_t(order_bits(score[c] + 0.0f)) << 32 | (kCandidates - c);
-        pick = key < last && key > pick ? key : pick;
+        const uint32_t other = s.order[position][predecessor][c];
+        rank += other > mine || (other == mine && c < i) ? 1u : 0u;
       }
-      last = pick;
-      s.likeliest[position][predecessor][child] = uint8_t(kCandidates - uint32_t(pick));
+      if (rank < kChildren) s.likeliest[position][predecessor][rank] = uint8_t(i);
+      weight[position] /= ordered_sum(s.probability[position][predecessor]);
+    }
+    wave_lds_fence();
+#pragma unroll
+    for (uint32_t position = 0; position < kPositions; ++position) {
+      const float q = weight[position], top = largest(q);
+      s.probability[position][predecessor][i] = q;
+      weight[position] = temperature == 0.0f || !(q > 0.0f) ? q : expf((logf(q) - logf(top)) / temperature);
+      s.drafted[position][predecessor][i] = weight[position];
+    }
+    wave_lds_fence();
+#pragma unroll
+    for (uint32_t position = 0; position < kPositions; ++position) weight[position] /= ordered_sum(s.drafted[position][predecessor]);
+    wave_lds_fence();
+#pragma unroll
+    for (uint32_t position = 0; position < kPositions; ++position) {
+      s.drafted[position][predecessor][i] = weight[position];
+      const float q = fminf(fmaxf(weight[position], 1.0e-6f), 1.0f - 1.0e-6f);
+      const float z = slope * logf(q / (1.0f - q)) + p.intercept[lane][position];
+      s.estimate[position][predecessor][i] = 1.0f / (1.0f + expf(-z));
     }
   }
   __syncthreads();
+  if (tid >= 64u) return;
 
-  const uint32_t *chain = chain_tokens + size_t(lane) * DRAFT_CHAIN_TOKENS;
-  const float *rates = chain_rates + size_t(lane) * DRAFT_CHAIN_TOKENS * DRAFT_CHAIN_AGREEMENTS;
+  // ---- The growth, by the first wavefront. Thread r holds row r, thread e open entry e (and 64 + e).
   const uint32_t children = min(p.children[lane], kChildren), deepest = p.depth[lane], chained = min(p.chain[lane], uint32_t(DRAFT_CHAIN_TOKENS));
-  const float temperature = p.temperature[lane], slope = p.slope[lane];
-  uint32_t made = 1, entryCount = 0;
+  static_assert(kRates <= 64 && kRows <= 64 && kEntries <= 128 && kChildren == 4, "a thread a rate, a row, two entries; four draws a word");
+  uint32_t made = 1, entryCount = 0, expanded = 0;
+  uint32_t rowToken = p.anchor[lane], rowAncestors = 1u, rowParent = SAMPLING_TREE_ROOT, rowDepth = 0, rowOnChain = 1u, rowPredecessor = 0;
+  uint32_t rowDraws = SAMPLING_NO_DRAW * 0x01010101u;
+  uint32_t rowKeyLow = p.noise[lane][0], rowKeyHigh = p.noise[lane][1];
+  float rowQ = 1.0f, rowEstimate = 1.0f, rowCap = 1.0f, rowLeft[kChildren] = {};
+  uint64_t entryKey[2] = {0, 0};   // 0: taken, or none
+  uint32_t entryInfo[2] = {0, 0};
+  float entryScore[2] = {0.f, 0.f};
 
   // A host chain token's rate at depth d, by its agreement with the draft there: its likeliest candidate, another of its
   // candidates, none of them, or past its positions.
-  auto chainRate = [&](uint32_t d) {
-    const uint32_t token = chain[d];
+  auto chainRate = [&](uint32_t d) __attribute__((always_inline)) {
+    const uint32_t token = lane_value(chain, d);
     uint32_t agreement = 3;
     if (d < kPositions) {
-      const bool mine = tid < kCandidates && s.ids[d][tid] == token;
+      const bool mine = tid < kCandidates && s.ids[d][i] == token;
       const uint64_t among = __builtin_amdgcn_ballot_w64(mine);
       agreement = among & 1u ? 0u : among ? 1u : 2u;
     }
-    return rates[d * DRAFT_CHAIN_AGREEMENTS + agreement];
+    return lane_value(rates, d * DRAFT_CHAIN_AGREEMENTS + agreement);
   };
-  auto estimateOf = [&](float q, uint32_t position) {
-    q = fminf(fmaxf(q, 1.0e-6f), 1.0f - 1.0e-6f);
-    const float z = slope * logf(q / (1.0f - q)) + p.intercept[lane][position];
-    return 1.0f / (1.0f + expf(-z));
-  };
-  auto push = [&](float score, uint32_t info) {
-    if (entryCount < kEntries) {
-      if (tid == 0) {
-        s.entryScore[entryCount] = score;
-        s.entryInfo[entryCount] = info;
+  auto push = [&](float score, uint32_t info) __attribute__((always_inline)) {
+    if (entryCount >= kEntries) return;
+    const uint64_t key = uint64_t(order_bits(score + 0.0f)) << 32 | (kDead - entryCount);
+#pragma unroll
+    for (uint32_t half = 0; half < 2; ++half)
+      if (tid + 64u * half == entryCount) {
+        entryKey[half] = key;
+        entryInfo[half] = info;
+        entryScore[half] = score;
       }
-      ++entryCount;
-    }
+    ++entryCount;
   };
-  auto capOf = [&](uint32_t parent, uint32_t index) {
+  auto capOf = [&](uint32_t parent, uint32_t index) __attribute__((always_inline)) {
+    const uint32_t drawn = lane_value(rowDraws, parent);
     float cap = 1.0f;
-    bool found = false;
-    for (uint32_t child = 0; child < kChildren; ++child)
-      if (!found && s.draw[parent][child] == index) {
-        cap = s.left[parent][child];
-        found = true;
-      }
+#pragma unroll
+    for (uint32_t child = kChildren; child-- > 0;)
+      if ((drawn >> (8u * child) & 0xFFu) == index) cap = lane_value(rowLeft[child], parent);
     return cap;
   };
-  auto clearRow = [&](uint32_t row) {
-    if (tid < kChildren) s.draw[row][tid] = uint8_t(SAMPLING_NO_DRAW);
-    if (tid < kCandidates) s.next[row][tid] = 0.f;
-  };
   // A draft row's children at `position`, after its candidate `predecessor`: its drawn candidates, each an entry.
-  auto expand = [&](uint32_t row, uint32_t position, uint32_t predecessor, float score, bool hasChain, uint32_t chainToken, float chainRateHere) {
-    const float q = s.probability[position][predecessor][i];
-    float top = q;
-#pragma unroll
-    for (int step = 1; step < 16; step <<= 1) top = fmaxf(top, __shfl_xor(top, step, 64));
-    const float weight = temperature == 0.0f || !(q > 0.0f) ? q : expf((logf(q) - logf(top)) / temperature);
-    if (tid < kCandidates) s.next[row][i] = weight;
-    __syncthreads();
-    float mass = 0.f;
-#pragma unroll
-    for (uint32_t c = 0; c < kCandidates; ++c) mass += s.next[row][c];
-    __syncthreads();
-    const float mine = weight / mass;
-    if (tid < kCandidates) s.next[row][i] = mine;
-    __syncthreads();
-    const float key = temperature > 0.0f && mine > 0.0f ? logf(mine) + gumbel_of(s.key[row], s.ids[position][i]) : -INFINITY;
+  auto expand = [&](uint32_t row, uint32_t position, uint32_t predecessor, float score, bool hasChain, uint32_t chainToken,
+                    float chainRateHere) __attribute__((always_inline)) {
+    const float q = s.probability[position][predecessor][i], mine = s.drafted[position][predecessor][i];
+    const float estimate = s.estimate[position][predecessor][i];
+    const uint32_t id = s.ids[position][i], likeliest = *reinterpret_cast<const uint32_t *>(s.likeliest[position][predecessor]);
+    if (tid < kCandidates) next[(size_t(lane) * kRows + row) * kCandidates + i] = mine;
+    expanded |= 1u << row;
+    if (tid == row) rowPredecessor = predecessor;
+    float key = -INFINITY;
+    if (temperature > 0.0f) {
+      const uint64_t rowKey = uint64_t(lane_value(rowKeyHigh, row)) << 32 | lane_value(rowKeyLow, row);
+      if (mine > 0.0f) key = logf(mine) + gumbel_of(rowKey, id);
+    }
     uint32_t taken = 0;
     float bound = score, left = 1.0f - chainRateHere, reserved = chainRateHere;
-    for (uint32_t child = 0; child < children; ++child) {
+#pragma unroll
+    for (uint32_t child = 0; child < kChildren; ++child) {
+      if (child >= children) break;
       uint32_t drawn = kCandidates;
       if (temperature == 0.0f) {
-        const uint32_t likely = s.likeliest[position][predecessor][child];
-        drawn = s.probability[position][predecessor][likely] > 0.0f ? likely : kCandidates;
+        const uint32_t likely = uint32_t(__builtin_amdgcn_readfirstlane(int(likeliest))) >> (8u * child) & 0xFFu;
+        drawn = lane_value(q, likely) > 0.0f ? likely : kCandidates;
       } else {
-        const bool open = !(taken >> i & 1u) && key > -INFINITY;
-        const uint64_t best = group_max<16>(open ? uint64_t(order_bits(key)) << 32 | (kCandidates - i) : 0);
-        drawn = best ? kCandidates - uint32_t(best) : kCandidates;
-        drawn = uint32_t(__builtin_amdgcn_readfirstlane(int(drawn)));
+        const uint32_t open = !(taken >> i & 1u) && key > -INFINITY ? order_bits(key) : 0u;
+        const uint32_t best = row_max_dpp(open);
+        const uint64_t at = __builtin_amdgcn_ballot_w64(open && open == best);
+        drawn = at ? uint32_t(__builtin_ctzll(at)) : kCandidates;   // (the sixteen lanes four times over)
       }
       if (drawn == kCandidates) break;
       taken |= 1u << drawn;
-      const bool joins = hasChain && s.ids[position][drawn] == chainToken;
+      const bool joins = hasChain && lane_value(id, drawn) == chainToken;
       const float cap = joins ? left + reserved : left;
-      const float own = fminf(estimateOf(s.next[row][drawn], position), cap);
+      const float own = fminf(lane_value(estimate, drawn), cap);
       left = joins ? cap - fmaxf(own, reserved) : left - own;
       reserved = joins ? 0.0f : reserved;
       bound = fminf(bound, score * own);
-      if (tid == 0) {
-        s.draw[row][child] = uint8_t(drawn);
-        s.left[row][child] = cap;
+      if (tid == row) {
+        rowDraws = (rowDraws & ~(0xFFu << (8u * child))) | drawn << (8u * child);
+        rowLeft[child] = cap;
       }
       push(bound, row << 16 | position << 8 | drawn);
     }
-    __syncthreads();
   };
 
-  if (tid == 0) {
-    s.token[0] = p.anchor[lane];
-    s.ancestors[0] = 1u;
-    s.parent[0] = SAMPLING_TREE_ROOT;
-    s.depth[0] = 0;
-    s.onChain[0] = 1u;
-    s.q[0] = s.estimate[0] = s.cap[0] = 1.0f;
-    s.key[0] = uint64_t(p.noise[lane][1]) << 32 | p.noise[lane][0];
-  }
-  clearRow(0);
-  __syncthreads();
   if (deepest > 0) {
     const float rate = chained ? chainRate(0) : 0.0f;
-    expand(0, 0, 0, 1.0f, chained != 0, chained ? chain[0] : 0u, rate);
+    expand(0, 0, 0, 1.0f, chained != 0, chained ? lane_value(chain, 0) : 0u, rate);
     if (chained) push(rate, kChainEntry);
   }
-  __syncthreads();
   const uint32_t most = min(kRows, deepest + 1u);
   while (made < most) {
     // the best open entry: the largest estimate, the earliest made among equal ones
-    uint64_t best = 0;
-    for (uint32_t e = tid; e < entryCount; e += 64u)
-      if (s.entryInfo[e] != kDead) {
-        const uint64_t key = uint64_t(order_bits(s.entryScore[e] + 0.0f)) << 32 | (kDead - e);
-        best = key > best ? key : best;
-      }
-    best = group_max<64>(best);
+    const uint64_t best = wave_max_dpp(entryKey[0] > entryKey[1] ? entryKey[0] : entryKey[1]);
     if (!best) break;
     const uint32_t entry = kDead - uint32_t(best);
-    const float score = s.entryScore[entry];
-    const uint32_t info = s.entryInfo[entry];
-    __syncthreads();
-    if (tid == 0) s.entryInfo[entry] = kDead;
+    const float score = lane_value(entry < 64u ? entryScore[0] : entryScore[1], entry & 63u);
+    const uint32_t info = lane_value(entry < 64u ? entryInfo[0] : entryInfo[1], entry & 63u);
+#pragma unroll
+    for (uint32_t half = 0; half < 2; ++half)
+      if (tid + 64u * half == entry) entryKey[half] = 0;
     const bool fromChain = (info & kChainEntry) != 0;
     const uint32_t parent = info >> 16 & 0x7FFFu, position = info >> 8 & 0xFFu, index = info & 0xFFu;
-    const uint32_t token = fromChain ? chain[position] : s.ids[position][index];
+    const uint32_t drafted = min(position, kPositions - 1u);   // (a chain step's position may lie past the draft's)
+    const uint32_t id = uint32_t(__builtin_amdgcn_readfirstlane(int(s.ids[drafted][index & 15u]))), token = fromChain ? lane_value(chain, position) : id;
+    // (a draft step's own probability: in the distribution its parent's children were drawn from)
+    const float q = fromChain ? -1.0f : s.drafted[drafted][lane_value(rowPredecessor, parent)][index & 15u];
     // a token path the tree holds already gains no row
-    const uint64_t same = __builtin_amdgcn_ballot_w64(tid >= 1u && tid < made && s.parent[tid] == parent && s.token[tid] == token);
+    const uint64_t same = __builtin_amdgcn_ballot_w64(tid >= 1u && tid < made && rowParent == parent && rowToken == token);
     uint32_t row = same ? uint32_t(__builtin_ctzll(same)) : 0u;
     if (!row) {
       row = made++;
       const float cap = fromChain ? 1.0f : capOf(parent, index);
-      if (tid == 0) {
-        s.token[row] = token;
-        s.ancestors[row] = s.ancestors[parent] | 1u << row;
-        s.parent[row] = parent;
-        s.depth[row] = position + 1u;
-        s.onChain[row] = s.onChain[parent] && position < chained && token == chain[position];
-        s.q[row] = fromChain ? -1.0f : s.next[parent][index];   // a row a host chain token made is no draft step
-        s.estimate[row] = score;
-        s.cap[row] = cap;
-        s.key[row] = mix64(s.key[parent] + 0x9e3779b97f4a7c15ull * (uint64_t(token) + 1u));
+      const uint32_t ancestors = lane_value(rowAncestors, parent);
+      const bool onChain = lane_value(rowOnChain, parent) && position < chained && token == lane_value(chain, position);
+      const uint64_t parentKey = uint64_t(lane_value(rowKeyHigh, parent)) << 32 | lane_value(rowKeyLow, parent);
+      const uint64_t key = mix64(parentKey + 0x9e3779b97f4a7c15ull * (uint64_t(token) + 1u));
+      if (tid == row) {
+        rowToken = token;
+        rowAncestors = ancestors | 1u << row;
+        rowParent = parent;
+        rowDepth = position + 1u;
+        rowOnChain = onChain;
+        rowQ = q;   // (a row a host chain token made is no draft step)
+        rowEstimate = score;
+        rowCap = cap;
+        rowKeyLow = uint32_t(key);
+        rowKeyHigh = uint32_t(key >> 32);
       }
-      clearRow(row);
-    } else if (!fromChain && s.q[row] < 0.0f) {
+    } else if (!fromChain && lane_value(rowQ, row) < 0.0f) {
       // a draft step that joins a host chain's row gives it its draft probability and cap
       const float cap = capOf(parent, index);
-      __syncthreads();
-      if (tid == 0) {
-        s.q[row] = s.next[parent][index];
-        s.cap[row] = cap;
+      if (tid == row) {
+        rowQ = q;
+        rowCap = cap;
       }
     }
-    __syncthreads();
     if (position + 1u >= deepest) continue;   // the row's children would lie too deep
-    const bool chainChild = s.onChain[row] && position + 1u < chained;
+    const bool chainChild = lane_value(rowOnChain, row) && position + 1u < chained;
     if (!fromChain && position + 1u < kPositions)
-      expand(row, position + 1u, index, score, chainChild, chainChild ? chain[position + 1u] : 0u, chainChild ? chainRate(position + 1u) : 0.0f);
+      expand(row, position + 1u, index, score, chainChild, chainChild ? lane_value(chain, position + 1u) : 0u, chainChild ? chainRate(position + 1u) : 0.0f);
     else if (fromChain && position + 1u < chained)
       push(score * chainRate(position + 1u), kChainEntry | row << 16 | (position + 1u) << 8);
-    __syncthreads();
   }
-  __syncthreads();
   if (tid == 0) sizes[lane] = made;
   if (tid < made) {
     const size_t at = size_t(lane) * kRows + tid;
-    tokens[at] = s.token[tid];
-    tree[at] = AttentionTreeRow{s.ancestors[tid], uint16_t(s.parent[tid]), uint16_t(s.depth[tid])};
-    scores[2 * at] = s.q[tid];
-    scores[2 * at + 1] = s.estimate[tid];
-    caps[at] = s.cap[tid];
-    for (uint32_t child = 0; child < kChildren; ++child) draws[at * kChildren + child] = s.draw[tid][child];
-    for (uint32_t c = 0; c < kCandidates; ++c) next[at * kCandidates + c] = s.next[tid][c];
+    tokens[at] = rowToken;
+    tree[at] = AttentionTreeRow{rowAncestors, uint16_t(rowParent), uint16_t(rowDepth)};
+    scores[2 * at] = rowQ;
+    scores[2 * at + 1] = rowEstimate;
+    caps[at] = rowCap;
+#pragma unroll
+    for (uint32_t child = 0; child < kChildren; ++child) draws[at * kChildren + child] = uint8_t(rowDraws >> (8u * child));
   }
+  for (uint32_t k = tid; k < made * kCandidates; k += 64u)   // (a row that was expanded has its probabilities already)
+    if (!(expanded >> (k / kCandidates) & 1u)) next[size_t(lane) * kRows * kCandidates + k] = 0.f;
 }
 SP_REGISTER_KERNEL("draft_select_tree", &draft_select_tree);
 

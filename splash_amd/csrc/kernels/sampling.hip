@@ -213,7 +213,12 @@ __global__ __launch_bounds__(128) void draft_verify_rows(const uint32_t *__restr
   const uint32_t t = threadIdx.x, lane = t / kRows, row = t % kRows, lanes = min(p.lanes, kLanes);
   const uint32_t size = lane < lanes ? min(sizes[lane], kRows) : 0u;
   const bool candidate = row >= 1 && row < size;
-  const float estimate = candidate ? scores[t].y : 0.f;
+  // (all that is read of a row is on its way at once: the kernel is one workgroup's chain of waits)
+  const bool held = lane < lanes;
+  const float scored = held ? scores[t].y : 0.f;
+  const AttentionTreeRow read = held ? trees[t] : AttentionTreeRow{0u, 0u, 0u};
+  const uint32_t token = held ? tree_tokens[t] : 0u;
+  const float estimate = candidate ? scored : 0.f;
   estimateOf[t] = candidate ? estimate : -INFINITY;
   rankedOwner[t] = kLanes;
   rankedEstimate[t] = -INFINITY;
@@ -221,9 +226,10 @@ __global__ __launch_bounds__(128) void draft_verify_rows(const uint32_t *__restr
   __syncthreads();
   if (candidate) {
     uint32_t rank = 0;
-    for (uint32_t other = 0; other < kAll; ++other) {
+#pragma unroll 16
+    for (uint32_t other = 0; other < kAll; ++other) {   // (no candidate: -infinity)
       const float e = estimateOf[other];
-      rank += (e > estimate || (e == estimate && other < t)) && (other % kRows) >= 1 && e != -INFINITY ? 1u : 0u;
+      rank += (e > estimate || (e == estimate && other < t)) && e != -INFINITY ? 1u : 0u;
     }
     rankedOwner[rank] = lane;
     rankedEstimate[rank] = estimate;
@@ -232,12 +238,18 @@ __global__ __launch_bounds__(128) void draft_verify_rows(const uint32_t *__restr
   // Thread t now stands for place t of the order.
   const uint32_t owner = rankedOwner[t];
   uint32_t before = 0;   // candidates of the same lane at earlier places
-  for (uint32_t place = 0; place < t; ++place) before += rankedOwner[place] == owner ? 1u : 0u;
+  const uint64_t earlierLanes = (uint64_t{1} << (t & 63u)) - 1u;
+  const uint32_t firstOwner = rankedOwner[t & 63u];   // (the first wave's places, for the second)
+#pragma unroll
+  for (uint32_t l = 0; l < kLanes; ++l) {
+    const uint64_t here = __builtin_amdgcn_ballot_w64(owner == l), ahead = __builtin_amdgcn_ballot_w64(t >= 64u && firstOwner == l);
+    if (owner == l) before = uint32_t(__builtin_popcountll(here & earlierLanes) + __builtin_popcountll(ahead));
+  }
   const bool eligible = owner < kLanes && !(rankedEstimate[t] < p.floor) && before + 1u < p.lane_cap;
   const uint64_t ballot = __builtin_amdgcn_ballot_w64(eligible);
   if ((t & 63u) == 0) eligibleBefore[t >> 6] = uint32_t(__builtin_popcountll(ballot));
   __syncthreads();
-  const uint32_t earlier = uint32_t(__builtin_popcountll(ballot & ((uint64_t{1} << (t & 63u)) - 1u))) + (t >= 64 ? eligibleBefore[0] : 0u);
+  const uint32_t earlier = uint32_t(__builtin_popcountll(ballot & earlierLanes)) + (t >= 64 ? eligibleBefore[0] : 0u);
   const uint32_t budget = p.rows > lanes ? p.rows - lanes : 0u;
   if (eligible && earlier < budget) atomicAdd(&takenOf[owner], 1u);
   __syncthreads();
@@ -250,7 +262,7 @@ __global__ __launch_bounds__(128) void draft_verify_rows(const uint32_t *__restr
   }
   if (p.slots) first = lane * p.lane_cap;
   const bool placed = row < mine;
-  const AttentionTreeRow node = placed ? trees[t] : AttentionTreeRow{0u, 0u, 0u};
+  const AttentionTreeRow node = placed ? read : AttentionTreeRow{0u, 0u, 0u};
   pathOf[t] = placed ? node.ancestors : 0u;
   __syncthreads();
   uint32_t place = 0;
@@ -271,7 +283,7 @@ __global__ __launch_bounds__(128) void draft_verify_rows(const uint32_t *__restr
     for (uint32_t walk = node.ancestors; walk; walk &= walk - 1u) ancestors |= 1u << placeOf[lane * kRows + uint32_t(__builtin_ctz(walk))];
     const uint32_t depth = uint32_t(__builtin_popcount(node.ancestors)) - 1u;
     const uint32_t up = row ? placeOf[lane * kRows + node.parent] : SAMPLING_TREE_ROOT;
-    tokens[first + place] = tree_tokens[t];
+    tokens[first + place] = token;
     tree[first + place] = AttentionTreeRow{ancestors, uint16_t(up), uint16_t(depth)};
     sources[first + place] = row;
   }

@@ -684,6 +684,29 @@ def test_draft_candidates_and_edges(backend):
                                          backend.from_array(before), backend.from_array(after), 600000, 600000, 600000, [0])
 
 
+@pytest.mark.parametrize("equal", [1, 15, 16, 17, 255, 256, 257, 4000])
+def test_draft_candidates_among_equal_logits(backend, equal):
+    """`equal` columns of a row's first shard hold its one largest value: up to 256 keys that reach the shard's threshold are
+    ranked, more take the rounds. The candidates are the oracle's, the lower column first among equal logits."""
+    print("case draft candidates equal", equal, flush=True)
+    rng = np.random.default_rng(equal)
+    columns = 4096 + 300
+    logits = rng.standard_normal((8, columns)).astype(np.float32)
+    for row in logits:
+        row[rng.choice(4096, equal, replace=False)] = 9.0
+    logits[3, ::7] = np.nan
+    out = [backend.allocate_buffer(7 * 16 * 4), backend.allocate_buffer(7 * 16 * 4), backend.allocate_buffer(7 * 256 * 4)]
+    scratch = backend.allocate_buffer(ops.DraftSelector.candidate_scratch_bytes(1, columns))
+    zeros = backend.from_array(np.zeros((columns, 256), np.uint16))
+    graph = splash_amd.CommandGraph()
+    ops.DraftSelector.add_candidates(graph, backend.from_array(logits), backend.from_array(np.zeros((8, 256), np.uint16)), scratch, *out,
+                                     zeros, zeros, columns, columns, columns, [0])
+    backend.run(graph)
+    want = orc.draft_candidates(logits, 1, columns, columns)
+    assert np.array_equal(out[0].download(np.uint32).reshape(7, 16), want[0])
+    assert np.array_equal(out[1].download(np.uint32).reshape(7, 16), want[1].view(np.uint32).reshape(7, 16))
+
+
 def _padded(codebook, vocabulary):
     """A codebook of `vocabulary` rows whose rows past the given ones repeat them."""
     rows = codebook.shape[0]
