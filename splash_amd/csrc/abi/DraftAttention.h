@@ -56,6 +56,14 @@ struct DraftConvParams {
   uint32_t finish;
   uint32_t hidden;
 };
+// draft_conv_table, draft_conv_norm_table: `rows` rows of the lanes' eight each, the row tiles of the table, and the widest
+// row that they take.
+struct DraftConvTableParams {
+  uint32_t hidden;
+  uint32_t rows;
+  uint32_t tiles;
+};
+#define DRAFT_CONVOLUTION_TABLE_WIDTH 8192u
 
 // draft_attention_qkv: grid (40, lanes) of 512 threads: a wave a (row, head) task of the 8 x (32 + 8) a lane, every
 // thread a share of the value rows' transpose. draft_attention_merge: grid (8 KV heads, lanes), 1024 threads.

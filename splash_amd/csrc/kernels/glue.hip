@@ -2,6 +2,7 @@
 // RoPE tables per packed row, token embedding from native K-quant rows (the reference's
 // kernels/shared/normalization.metal, rope.metal, embedding.metal).
 #include "abi/Glue.h"
+#include "abi/DraftAttention.h"
 #include "abi/Gguf.h"
 #include "backend/KernelRegistry.hpp"
 #include "kernels/device_common.hpp"
@@ -32,10 +33,15 @@ __device__ __forceinline__ void stage_row(const uint16_t *__restrict__ source, u
 // order; a wavefront sums its lanes by butterfly, the four wavefronts' sums are added in order
 // (normalization.metal:59-99 and common/rms_inverse.h:15-33, on 64-lane wavefronts).
 __device__ __forceinline__ float rms_inverse(const uint16_t *row, uint32_t width, float *scratch) {
+  // (ten reads at a time: a column past the row adds a zero)
+  constexpr uint32_t kAhead = 10;
   float sum = 0.f;
-  for (uint32_t c = threadIdx.x; c < width; c += 256) {
-    const float v = bf16_bits_to_float(row[c]);
-    sum += v * v;
+  for (uint32_t first = threadIdx.x; first < width; first += 256u * kAhead) {
+    float v[kAhead];
+#pragma unroll
+    for (uint32_t j = 0; j < kAhead; ++j) v[j] = bf16_bits_to_float(row[min(first + 256u * j, width - 1u)]);
+#pragma unroll
+    for (uint32_t j = 0; j < kAhead; ++j) sum += first + 256u * j < width ? v[j] * v[j] : 0.f;
   }
   sum = wave_sum(sum);
   if ((threadIdx.x & 63u) == 0) scratch[threadIdx.x >> 6] = sum;
@@ -63,62 +69,164 @@ __global__ __launch_bounds__(256) void norm_rms(const uint16_t *__restrict__ inp
 }
 SP_REGISTER_KERNEL("norm_rms", &norm_rms);
 
+// A row's part of an activation table, and (Normed) the normalized row it describes: 256 threads, each the runs of four
+// inputs q = t, t + 256, ... (4 kq .. 4 kq + 3 of a group's half, one 8-byte piece of a table entry), kRuns of them in
+// flight together. A row past the live ones is zeros. The width is a multiple of 256, so a wavefront's runs are all inside
+// the row or all past it.
+template <bool Normed>
+__device__ __forceinline__ void write_table_row(const uint16_t *x, const uint16_t *w, float inverse, bool live, uint32_t row,
+                                                uint16_t *__restrict__ output, uint8_t *__restrict__ table, uint32_t width, uint32_t allTiles) {
+  constexpr uint32_t kRuns = 5;
+  const uint32_t r = row % 16u, G = width / 32u, runs = width / 4u;
+  // Row tile row / 16 is tile `tile` of its piece's table, which holds `tiles` row tiles.
+  const uint32_t piece = row / 16u / GGUF_PIECE_TILES, tile = row / 16u % GGUF_PIECE_TILES;
+  const uint32_t tiles = min(uint32_t(GGUF_PIECE_TILES), allTiles - piece * GGUF_PIECE_TILES);
+  table += piece * gguf_table_bytes(width, GGUF_PIECE_TILES);
+  uint2 *values = reinterpret_cast<uint2 *>(table);
+  float *sums32 = reinterpret_cast<float *>(table + gguf_table_sums32_offset(width, tiles));
+  float *sums16 = reinterpret_cast<float *>(table + gguf_table_sums16_offset(width, tiles));
+  for (uint32_t first = 0; first < runs; first += 256u * kRuns) {
+    uint32_t bits[kRuns][4];
+    float sum[kRuns];
+#pragma unroll
+    for (uint32_t j = 0; j < kRuns; ++j) {
+      const uint32_t q = min(first + 256u * j + threadIdx.x, runs - 1u);
+      uint2 xs = make_uint2(0u, 0u), ws = xs;
+      if (live) {
+        xs = *reinterpret_cast<const uint2 *>(x + 4u * q);
+        if constexpr (Normed) ws = *reinterpret_cast<const uint2 *>(w + 4u * q);
+      }
+      const uint32_t xb[4] = {xs.x & 0xFFFFu, xs.x >> 16, xs.y & 0xFFFFu, xs.y >> 16};
+      const uint32_t wb[4] = {ws.x & 0xFFFFu, ws.x >> 16, ws.y & 0xFFFFu, ws.y >> 16};
+      float v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        bits[j][i] = xb[i];
+        if constexpr (Normed) bits[j][i] = live ? float_to_bf16_bits((bf16_bits_to_float(xb[i]) * inverse) * bf16_bits_to_float(wb[i])) : 0u;
+        v[i] = bf16_bits_to_float(bits[j][i]);
+      }
+      sum[j] = (v[0] + v[1]) + (v[2] + v[3]);
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < kRuns; ++j) {
+      const uint32_t q = first + 256u * j + threadIdx.x;
+      // run q: group g = q / 8, half = (q / 4) % 2, kq = q % 4; the four runs of a half sit in four consecutive lanes
+      const float s1 = __shfl_down(sum[j], 1, 64), s2 = __shfl_down(sum[j], 2, 64), s3 = __shfl_down(sum[j], 3, 64);
+      const float s = ((sum[j] + s1) + s2) + s3;   // of 16 inputs, in input order
+      const float other = __shfl_down(s, 4, 64);
+      if (q >= runs) continue;
+      if constexpr (Normed)
+        if (live)
+          *reinterpret_cast<uint2 *>(output + size_t(row) * width + 4u * q) =
+              make_uint2(bits[j][0] | (bits[j][1] << 16), bits[j][2] | (bits[j][3] << 16));
+      const uint32_t g = q / 8u, half = (q / 4u) % 2u, kq = q % 4u;
+      // operand elements 4 half + {0,1,2,3} are inputs 4 kq + {0,2,1,3} of the half
+      values[((size_t(tile) * G + g) * 64u + kq * 16u + r) * 2u + half] =
+          make_uint2(bits[j][0] | (bits[j][2] << 16), bits[j][1] | (bits[j][3] << 16));
+      if (kq == 0) {
+        sums16[(size_t(tile) * 2u * G + 2u * g + half) * 16u + r] = s;
+        if (half == 0) sums32[(size_t(tile) * G + g) * 16u + r] = s + other;
+      }
+    }
+  }
+}
+
 // The same, and the activation table of the normalized rows: grid (tiles * 16) so that the rows
-// past the live ones are written as zeros. Each thread normalizes runs of four inputs
-// (4 kq .. 4 kq + 3 of a group's half), which are one 8-byte piece of a table entry.
+// past the live ones are written as zeros. A handful of workgroups that only wait: every loop keeps several reads in
+// flight (8.7 us at 8 rows of 5120 either way).
 __global__ __launch_bounds__(256) void norm_rms_table16(const uint16_t *__restrict__ input, const uint16_t *__restrict__ weight,
                                                         uint16_t *__restrict__ output, uint8_t *__restrict__ table, NormParams p) {
   __shared__ float scratch[4];
   __shared__ __align__(16) uint16_t rowX[kStagedWidth], rowW[kStagedWidth];
-  const uint32_t row = blockIdx.x, r = row % 16u, G = p.width / 32u;
-  // Row tile row / 16 is tile `tile` of its piece's table, which holds `tiles` row tiles.
-  const uint32_t piece = row / 16u / GGUF_PIECE_TILES, tile = row / 16u % GGUF_PIECE_TILES;
-  const uint32_t tiles = min(uint32_t(GGUF_PIECE_TILES), p.tiles - piece * GGUF_PIECE_TILES);
-  table += piece * gguf_table_bytes(p.width, GGUF_PIECE_TILES);
+  const uint32_t row = blockIdx.x;
   const bool live = row < p.rows;
-  const uint16_t *x = input + size_t(live ? row : 0) * p.width, *w = weight;
-  if (live && p.width <= kStagedWidth) {  // the width is a multiple of 256
-    stage_row(x, p.width, rowX);
-    stage_row(w, p.width, rowW);
-    __syncthreads();
-    x = rowX;
-    w = rowW;
-  }
-  const float inverse = live ? rms_inverse(x, p.width, scratch) : 0.f;
-  uint2 *values = reinterpret_cast<uint2 *>(table);
-  float *sums32 = reinterpret_cast<float *>(table + gguf_table_sums32_offset(p.width, tiles));
-  float *sums16 = reinterpret_cast<float *>(table + gguf_table_sums16_offset(p.width, tiles));
-  // run q covers inputs 4 q .. 4 q + 3: group g = q / 8, half = (q / 4) % 2, kq = q % 4
-  for (uint32_t q = threadIdx.x; q < p.width / 4u; q += 256) {
-    uint32_t bits[4] = {0, 0, 0, 0};
-    float v[4] = {0.f, 0.f, 0.f, 0.f};
+  const uint16_t *x = input + size_t(live ? row : 0) * p.width;
+  if (p.width <= kStagedWidth) {  // the width is a multiple of 256
     if (live) {
-      const uint2 xs = *reinterpret_cast<const uint2 *>(x + 4u * q), ws = *reinterpret_cast<const uint2 *>(w + 4u * q);
-      const uint32_t xb[4] = {xs.x & 0xFFFFu, xs.x >> 16, xs.y & 0xFFFFu, xs.y >> 16};
-      const uint32_t wb[4] = {ws.x & 0xFFFFu, ws.x >> 16, ws.y & 0xFFFFu, ws.y >> 16};
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        bits[i] = float_to_bf16_bits((bf16_bits_to_float(xb[i]) * inverse) * bf16_bits_to_float(wb[i]));
-        v[i] = bf16_bits_to_float(bits[i]);
-      }
-      *reinterpret_cast<uint2 *>(output + size_t(row) * p.width + 4u * q) = make_uint2(bits[0] | (bits[1] << 16), bits[2] | (bits[3] << 16));
+      stage_row(x, p.width, rowX);
+      stage_row(weight, p.width, rowW);
     }
-    const uint32_t g = q / 8u, half = (q / 4u) % 2u, kq = q % 4u;
-    // operand elements 4 half + {0,1,2,3} are inputs 4 kq + {0,2,1,3} of the half
-    const uint2 piece = make_uint2(bits[0] | (bits[2] << 16), bits[1] | (bits[3] << 16));
-    values[((size_t(tile) * G + g) * 64u + kq * 16u + r) * 2u + half] = piece;
-    // sums of 16 inputs in input order: the four runs of a half sit in four consecutive lanes
-    float s = (v[0] + v[1]) + (v[2] + v[3]);
-    const float s1 = __shfl_down(s, 1, 64), s2 = __shfl_down(s, 2, 64), s3 = __shfl_down(s, 3, 64);
-    s = ((s + s1) + s2) + s3;
-    const float other = __shfl_down(s, 4, 64);
-    if (kq == 0) {
-      sums16[(size_t(tile) * 2u * G + 2u * g + half) * 16u + r] = s;
-      if (half == 0) sums32[(size_t(tile) * G + g) * 16u + r] = s + other;
-    }
+    __syncthreads();
+    const float inverse = live ? rms_inverse(rowX, p.width, scratch) : 0.f;
+    write_table_row<true>(rowX, rowW, inverse, live, row, output, table, p.width, p.tiles);
+  } else {
+    const float inverse = live ? rms_inverse(x, p.width, scratch) : 0.f;
+    write_table_row<true>(x, weight, inverse, live, row, output, table, p.width, p.tiles);
   }
 }
 SP_REGISTER_KERNEL("norm_rms_table16", &norm_rms_table16);
+
+// draft_conv (draft_attention.hip) and the pass that reads its rows, one workgroup a row: a Prepare stage's rows and their
+// activation table; a Residual stage's rows, their RMS norm (of `norm_weight`, into `normalized`) and its table. Each
+// convolution was a launch of its own before a launch of as few workgroups. Values and their order are the two kernels'.
+// The rows' 16-byte accesses are the host's rule (DraftAttention::addConvolutionTable). 8 rows of 5120: 5.3 us
+// for 3.1 + 3.0, 8.8 us for 3.1 + 8.7, and a launch less each: the draft model's pass of one lane 920 -> 868 us.
+template <bool Residual>
+__global__ __launch_bounds__(256) void draft_conv_table(const uint16_t *__restrict__ input, const uint16_t *__restrict__ dynamic,
+                                                        const uint16_t *__restrict__ base, const uint16_t *__restrict__ residual,
+                                                        const uint16_t *__restrict__ norm_weight, uint16_t *__restrict__ output,
+                                                        uint16_t *__restrict__ normalized, uint8_t *__restrict__ table, DraftConvTableParams p) {
+  constexpr uint32_t kHeld = kStagedWidth / 8u / 256u;
+  static_assert(DRAFT_CONVOLUTION_TABLE_WIDTH <= kStagedWidth && DRAFT_CONVOLUTION_GROUP % 8u == 0, "eight channels share their dynamic weights");
+  __shared__ float scratch[4];
+  __shared__ __align__(16) uint16_t rowX[kStagedWidth], rowW[Residual ? kStagedWidth : 8];
+  const uint32_t row = blockIdx.x, width = p.hidden, vectors = width / 8u, groups = width / DRAFT_CONVOLUTION_GROUP;
+  const bool live = row < p.rows;
+  if (live) {
+    const bool follows = row % DRAFT_ATTENTION_QUERY_ROWS > 0;   // a lane's first row has none before it
+    const size_t before = row - (follows ? 1u : 0u);
+    const uint16_t *mine = dynamic + size_t(row) * draft_dynamic_width(width) + (Residual ? DRAFT_CONVOLUTION_TAPS : 0u) * groups;
+    const uint16_t *taps = base + (Residual ? DRAFT_CONVOLUTION_TAPS : 0u) * size_t(width);
+    auto vector = [](const uint16_t *from, uint32_t v) { return reinterpret_cast<const uint4 *>(from)[v]; };
+    uint4 now[kHeld], last[kHeld], tap0[kHeld], tap1[kHeld], added[kHeld];
+    uint32_t dynamic0[kHeld], dynamic1[kHeld];
+#pragma unroll
+    for (uint32_t i = 0; i < kHeld; ++i) {
+      const uint32_t v = threadIdx.x + 256u * i;
+      if (v >= vectors) continue;
+      now[i] = vector(input + size_t(row) * width, v);
+      last[i] = vector(input + before * width, v);
+      tap0[i] = vector(taps, v);
+      tap1[i] = vector(taps + width, v);
+      if constexpr (Residual) added[i] = vector(residual + size_t(row) * width, v);
+      dynamic0[i] = mine[v / (DRAFT_CONVOLUTION_GROUP / 8u)];
+      dynamic1[i] = mine[groups + v / (DRAFT_CONVOLUTION_GROUP / 8u)];
+    }
+    if constexpr (Residual) stage_row(norm_weight, width, rowW);
+#pragma unroll
+    for (uint32_t i = 0; i < kHeld; ++i) {
+      const uint32_t v = threadIdx.x + 256u * i;
+      if (v >= vectors) continue;
+      const float d0 = bf16_bits_to_float(dynamic0[i]), d1 = bf16_bits_to_float(dynamic1[i]);
+      auto channel = [&](uint32_t x, uint32_t y, uint32_t t0, uint32_t t1, uint32_t a) {
+        float value = bf16_bits_to_float(x) * (bf16_bits_to_float(t0) + d0);
+        if (follows) value += bf16_bits_to_float(y) * (bf16_bits_to_float(t1) + d1);
+        if constexpr (Residual) value += bf16_bits_to_float(a);
+        return float_to_bf16_bits(value);
+      };
+      const uint32_t x[4] = {now[i].x, now[i].y, now[i].z, now[i].w}, y[4] = {last[i].x, last[i].y, last[i].z, last[i].w};
+      const uint32_t t0[4] = {tap0[i].x, tap0[i].y, tap0[i].z, tap0[i].w}, t1[4] = {tap1[i].x, tap1[i].y, tap1[i].z, tap1[i].w};
+      uint32_t a[4] = {}, out[4];
+      if constexpr (Residual) a[0] = added[i].x, a[1] = added[i].y, a[2] = added[i].z, a[3] = added[i].w;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        out[e] = channel(x[e] & 0xFFFFu, y[e] & 0xFFFFu, t0[e] & 0xFFFFu, t1[e] & 0xFFFFu, a[e] & 0xFFFFu) |
+                 (channel(x[e] >> 16, y[e] >> 16, t0[e] >> 16, t1[e] >> 16, a[e] >> 16) << 16);
+      const uint4 packed = make_uint4(out[0], out[1], out[2], out[3]);
+      reinterpret_cast<uint4 *>(output + size_t(row) * width)[v] = packed;
+      reinterpret_cast<uint4 *>(rowX)[v] = packed;
+    }
+  }
+  __syncthreads();
+  if constexpr (Residual) {
+    const float inverse = live ? rms_inverse(rowX, width, scratch) : 0.f;
+    write_table_row<true>(rowX, rowW, inverse, live, row, normalized, table, width, p.tiles);
+  } else {
+    write_table_row<false>(rowX, rowW, 0.f, live, row, normalized, table, width, p.tiles);
+  }
+}
+SP_REGISTER_KERNEL("draft_conv_table", &draft_conv_table<false>);
+SP_REGISTER_KERNEL("draft_conv_norm_table", &draft_conv_table<true>);
 
 // copy_rows_bf16: grid (ceil(rows * width / 256)), 256 threads.
 __global__ __launch_bounds__(256) void copy_rows_bf16(const uint16_t *__restrict__ source, uint16_t *__restrict__ destination, RowCopyParams p) {

@@ -87,51 +87,56 @@ void DFlashDraft::addDecode(hip::CommandGraph &graph, const DFlashDecodeBuffers 
   const ops::DraftAttentionPlan plan = ops::DraftAttention::plan(layout.attentionShape(), count);
   std::array<uint64_t, 8> keys{}, values{};
 
+  auto project = [&](const hip::Buffer &input, const ops::Projection &projection, const hip::Buffer &output, ops::PreparedInput prepared) {
+    ops::LinearBuffers buffers;
+    buffers.input = input;
+    buffers.output = output;
+    buffers.scratch = b.scratch;
+    buffers.prepared = std::move(prepared);
+    linear_.add(graph, buffers, projection, linear_.plan(projection, rows));
+  };
+  // (every norm but the first rides in the convolution before it)
+  ops::PreparedInput normalized =
+      ops::Normalization::addRmsTable(graph, b.hidden[0], weights_.layers[0].inputNorm, b.normalized, b.scratch, hidden, rows);
   for (uint32_t index = 0; index < layout.layers; ++index) {
     const DFlashDraftLayerWeights &w = weights_.layers[index];
     const hip::Buffer &current = b.hidden[index & 1], &next = b.hidden[(index & 1) ^ 1];
+    const bool last = index + 1 == layout.layers;
     // attention: norm -> dynamic weights -> convolution -> q|k|v -> attention -> output -> convolution with the residual
-    ops::PreparedInput normalized = ops::Normalization::addRmsTable(graph, current, w.inputNorm, b.normalized, b.scratch, hidden, rows);
-    ops::LinearBuffers dynamic;
-    dynamic.input = b.normalized;
-    dynamic.output = b.dynamic;
-    dynamic.scratch = b.scratch;
-    dynamic.prepared = normalized;
-    linear_.add(graph, dynamic, w.attentionDynamic, linear_.plan(w.attentionDynamic, rows));
-    ops::DraftAttention::addConvolution(graph, {b.normalized, b.dynamic, w.attentionConvolution, current, b.convolved}, plan,
-                                        ops::DraftConvolutionStage::Prepare);
-    linear_.addProjection(graph, b.convolved, w.qkvProjection, b.proposalQkv, rows, b.scratch);
+    project(b.normalized, w.attentionDynamic, b.dynamic, normalized);
+    ops::PreparedInput convolved = ops::DraftAttention::addConvolutionTable(
+        graph, {b.normalized, b.dynamic, w.attentionConvolution, current, b.convolved}, plan, ops::DraftConvolutionStage::Prepare, {}, {}, b.scratch);
+    project(b.convolved, w.qkvProjection, b.proposalQkv, convolved);
     ops::DraftAttention::addPrepare(graph, {b.proposalQkv, b.attention, w.queryNorm, w.keyNorm, b.ropeCos, b.ropeSin, b.queryKeys, b.queryValues},
                                     plan);
     ops::DraftAttention::addDecode(graph, {b.attention, ringsOf(b.rings, lanes, index, keys, values), b.queryKeys, b.queryValues}, cacheLengths,
                                    plan);
     linear_.addProjection(graph, b.attention, w.outputProjection, b.projected, rows, b.scratch);
-    ops::DraftAttention::addConvolution(graph, {b.projected, b.dynamic, w.attentionConvolution, current, b.residual}, plan,
-                                        ops::DraftConvolutionStage::Residual);
+    normalized = ops::DraftAttention::addConvolutionTable(graph, {b.projected, b.dynamic, w.attentionConvolution, current, b.residual}, plan,
+                                                          ops::DraftConvolutionStage::Residual, w.postAttentionNorm, b.normalized, b.scratch);
     // MLP: norm -> dynamic weights -> convolution -> SwiGLU -> down -> convolution with the residual
-    normalized = ops::Normalization::addRmsTable(graph, b.residual, w.postAttentionNorm, b.normalized, b.scratch, hidden, rows);
-    dynamic.prepared = normalized;
-    linear_.add(graph, dynamic, w.mlpDynamic, linear_.plan(w.mlpDynamic, rows));
-    ops::DraftAttention::addConvolution(graph, {b.normalized, b.dynamic, w.mlpConvolution, b.residual, b.convolved}, plan,
-                                        ops::DraftConvolutionStage::Prepare);
+    project(b.normalized, w.mlpDynamic, b.dynamic, normalized);
+    convolved = ops::DraftAttention::addConvolutionTable(graph, {b.normalized, b.dynamic, w.mlpConvolution, b.residual, b.convolved}, plan,
+                                                         ops::DraftConvolutionStage::Prepare, {}, {}, b.scratch);
     ops::LinearBuffers pair;
     pair.input = b.convolved;
     pair.output = b.intermediate;
     pair.scratch = b.scratch;
+    pair.prepared = convolved;
     linear_.add(graph, pair, w.upProjection, linear_.plan(w.upProjection, rows, ops::LinearEpilogue::GateUp), &w.gateProjection);
     linear_.addProjection(graph, b.intermediate, w.downProjection, b.projected, rows, b.scratch);
-    ops::DraftAttention::addConvolution(graph, {b.projected, b.dynamic, w.mlpConvolution, b.residual, next}, plan,
-                                        ops::DraftConvolutionStage::Residual);
+    // (the last layer's rows take the final norm, into the head's input)
+    normalized = ops::DraftAttention::addConvolutionTable(
+        graph, {b.projected, b.dynamic, w.mlpConvolution, b.residual, next}, plan, ops::DraftConvolutionStage::Residual,
+        last ? weights_.finalNorm : weights_.layers[index + 1].inputNorm, last ? b.finalHidden : b.normalized, b.scratch);
   }
   // The final norm feeds the shared vocabulary head and then the selector's projection, which reads the table the
   // head's plan left.
-  ops::PreparedInput finalHidden =
-      ops::Normalization::addRmsTable(graph, b.hidden[layout.layers & 1], weights_.finalNorm, b.finalHidden, b.scratch, hidden, rows);
   ops::LinearBuffers head;
   head.input = b.finalHidden;
   head.output = b.logits;
   head.scratch = b.scratch;
-  head.prepared = finalHidden;
+  head.prepared = normalized;
   const ops::PreparedInput afterHead = linear_.add(graph, head, head_, linear_.plan(head_, rows));
   ops::LinearBuffers selector;
   selector.input = b.finalHidden;

@@ -1,5 +1,7 @@
 #include "ops/DraftAttention.hpp"
 
+#include "abi/Gguf.h"
+#include "ops/Glue.hpp"
 #include "ops/Linear.hpp"  // requireBytes
 
 #include <algorithm>
@@ -80,6 +82,41 @@ void DraftAttention::addConvolution(hip::CommandGraph &graph, const DraftConvolu
   const uint64_t groups = (uint64_t{kRows} * shape.hiddenSize + 255) / 256;
   graph.add("draft_conv", {buffers.input, buffers.dynamic, buffers.weights, finish ? buffers.residual : buffers.input, buffers.output},
             DraftConvParams{finish ? 1u : 0u, shape.hiddenSize}, {groups, lanes, 1});
+}
+
+PreparedInput DraftAttention::addConvolutionTable(hip::CommandGraph &graph, const DraftConvolutionBuffers &buffers, const DraftAttentionPlan &plan,
+                                                  DraftConvolutionStage stage, const hip::Buffer &normWeight, const hip::Buffer &normalized,
+                                                  const LinearScratch &scratch) {
+  const DraftAttentionShape shape = plan.shape();
+  const DraftAttentionWorkspace workspace = plan.workspace();
+  const uint32_t lanes = plan.lanes(), width = shape.hiddenSize, rows = lanes * kRows, tiles = gguf_row_tiles(rows);
+  const bool finish = stage == DraftConvolutionStage::Residual;
+  if (width % GGUF_BLOCK) throw std::invalid_argument("the activation table takes whole 256-input super-blocks");
+  requireBytes(buffers.input, workspace.convolutionBytes, "draft convolution input");
+  requireBytes(buffers.output, workspace.convolutionBytes, "draft convolution output");
+  if (finish) {
+    requireBytes(buffers.residual, workspace.convolutionBytes, "draft convolution residual");
+    requireBytes(normWeight, uint64_t{width} * 2, "norm weight");
+    requireBytes(normalized, workspace.convolutionBytes, "norm output");
+  }
+  requireBytes(buffers.dynamic, uint64_t{lanes} * kRows * shape.dynamicSize * 2, "draft dynamic convolution");
+  requireBytes(buffers.weights, uint64_t{DRAFT_CONVOLUTION_STAGES} * DRAFT_CONVOLUTION_TAPS * width * 2, "draft convolution weight");
+  requireBytes(scratch.input, gguf_tables_bytes(width, tiles), "projection table");
+  auto vectors = [](const hip::Buffer &buffer) { return buffer.gpuAddress() % 16 == 0; };
+  const bool whole = width <= DRAFT_CONVOLUTION_TABLE_WIDTH && vectors(buffers.input) && vectors(buffers.output) && vectors(buffers.weights) &&
+                     (!finish || (vectors(buffers.residual) && vectors(normWeight) && vectors(normalized)));
+  if (!whole) {
+    addConvolution(graph, buffers, plan, stage);
+    if (finish) return Normalization::addRmsTable(graph, buffers.output, normWeight, normalized, scratch, width, rows);
+    Linear::addPrepare(graph, buffers.output, scratch, width, rows);
+    return {buffers.output, LinearInput::Table16};
+  }
+  const hip::Buffer &residual = finish ? buffers.residual : buffers.input, &norm = finish ? normWeight : buffers.weights,
+                    &after = finish ? normalized : buffers.output;
+  graph.add(finish ? "draft_conv_norm_table" : "draft_conv_table",
+            {buffers.input, buffers.dynamic, buffers.weights, residual, norm, buffers.output, after, scratch.input},
+            DraftConvTableParams{width, rows, tiles}, {tiles * GGUF_ROW_TILE, 1, 1}, {256, 1, 1});
+  return {after, LinearInput::Table16};
 }
 
 void DraftAttention::addPrepare(hip::CommandGraph &graph, const DraftPrepareBuffers &buffers, const DraftAttentionPlan &plan) {

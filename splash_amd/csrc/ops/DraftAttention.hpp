@@ -8,6 +8,7 @@
 #include "abi/DraftAttention.h"
 #include "hip/Backend.hpp"
 #include "ops/DraftSelector.hpp"  // StepRows
+#include "ops/Linear.hpp"         // PreparedInput
 
 #include <cstdint>
 #include <span>
@@ -95,6 +96,12 @@ public:
 
   static void addConvolution(hip::CommandGraph &graph, const DraftConvolutionBuffers &buffers, const DraftAttentionPlan &plan,
                              DraftConvolutionStage stage);
+  // The same rows, and what the projection after them reads: a Prepare stage's table of the rows; a Residual stage's RMS
+  // norm of them (`normWeight`, written to `normalized`) and that one's table. One dispatch where the rows are whole
+  // 16-byte vectors of a width the kernel holds, the operators one after the other elsewhere.
+  static PreparedInput addConvolutionTable(hip::CommandGraph &graph, const DraftConvolutionBuffers &buffers, const DraftAttentionPlan &plan,
+                                           DraftConvolutionStage stage, const hip::Buffer &normWeight, const hip::Buffer &normalized,
+                                           const LinearScratch &scratch);
   static void addPrepare(hip::CommandGraph &graph, const DraftPrepareBuffers &buffers, const DraftAttentionPlan &plan);
   static void addDecode(hip::CommandGraph &graph, const DraftDecodeAttentionBuffers &buffers, std::span<const uint32_t> cacheLengths,
                         const DraftAttentionPlan &plan);

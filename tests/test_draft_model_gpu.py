@@ -136,6 +136,46 @@ def test_a_steps_rows_through_the_draft(backend, draft):
     assert np.array_equal(got_logits.argmax(axis=1)[clear], exact["exact"].argmax(axis=1)[clear]) and clear.sum() >= lanes * ROWS // 2
 
 
+def test_a_convolution_with_its_table_equals_the_two_passes(backend, draft):
+    """A draft whose convolution weights lie two bytes off a vector's start runs each convolution and the norm or table after
+    it as two dispatches, one whose weights are aligned as one: the same rows bit for bit, for one lane, an odd number and
+    two (a row tile half empty, one over, and full)."""
+    print("case draft convolution tables", flush=True)
+    model, gpu = draft
+
+    class Shifted:
+        """A backend that puts the convolution weights two bytes into their buffers."""
+
+        def __getattr__(self, name):
+            return getattr(backend, name)
+
+        def from_array(self, array, *args, **kwargs):
+            if not any(array is w[name] for w in model.layers for name in ("attention_convolution", "mlp_convolution")):
+                return backend.from_array(array, *args, **kwargs)
+            view = backend.allocate_buffer(array.nbytes + 16).view(2, array.nbytes)
+            view.upload(np.ascontiguousarray(array))
+            return view
+
+    apart = model.build_gpu(Shifted(), max_lanes=3, context_rows=64)
+    rng = np.random.default_rng(31)
+    for lanes in (1, 2, 3):
+        hidden = bits(rng.standard_normal((lanes * ROWS, model.hidden)))
+        tables = [rope_tables(np.arange(16)) for _ in range(lanes)]
+        got = []
+        for target in (gpu, apart):
+            target.buffer(verify.DFLASH_HIDDEN, 0).upload(hidden)
+            target.buffer(verify.DFLASH_ROPE_COS).upload(np.stack([t[0] for t in tables]))
+            target.buffer(verify.DFLASH_ROPE_SIN).upload(np.stack([t[1] for t in tables]))
+            graph = target.encode_decode([0] * lanes)
+            backend.run(graph)
+            rows = lanes * ROWS
+            got.append((len(graph.kernels()), target.buffer(verify.DFLASH_HIDDEN, model.layer_count & 1).download(np.uint16)[:rows * model.hidden],
+                        target.buffer(verify.DFLASH_FINAL_HIDDEN).download(np.uint16)[:rows * model.hidden],
+                        target.buffer(verify.DFLASH_LOGITS).download(np.uint32)[:rows * model.vocabulary]))
+        assert got[1][0] - got[0][0] == 4 * model.layer_count
+        assert all(np.array_equal(a, b) for a, b in zip(got[0][1:], got[1][1:]))
+
+
 def test_the_selector_reads_the_drafts_rows_in_place(backend, draft):
     """The candidates of every proposal position from the logits and selector rows the draft left, against the oracle's
     selection over the same downloaded logits."""
