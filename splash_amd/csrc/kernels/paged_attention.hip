@@ -65,10 +65,31 @@ template <int N> __device__ __forceinline__ float block_max(float v, float *scra
   return v;
 }
 
+// Block z of a dispatch. A prompt chunk's kernels (Chunk) work it out from the chunk's one sequence; a step's read its
+// sequence at once: the test of chunk_rows was one more wait in each of the layer's three short kernels, 1 % of a step.
+template <bool Chunk> __device__ __forceinline__ AttentionSequence block_sequence(const AttentionParams &p, uint32_t z) {
+  if constexpr (Chunk) return attention_sequence(p, z);
+  else return p.sequence[z];
+}
+
 // The page of logical page `index` of a sequence.
 __device__ __forceinline__ uint8_t *page_of(uint8_t *pool, const uint64_t *page_table, const AttentionSequence &seq,
                                             uint64_t page_bytes, uint32_t index) {
   return pool + page_table[seq.table_first + index] * page_bytes;
+}
+
+// attention_store.h:52-85: scale = max / 127, code = clamp(rint(v 127 / max)); the scale is stored fp16.
+__device__ __forceinline__ int8_t cache_code(float v, float maximum) {
+  if (maximum == 0.0f) return 0;
+  const int q = int(rintf(v * 127.0f / maximum));
+  return int8_t(q < -127 ? -127 : q > 127 ? 127 : q);
+}
+__device__ __forceinline__ void store_cache_scales(uint8_t *page, uint32_t kv_heads, uint32_t D, uint32_t head, uint32_t token, float keyMax,
+                                                   float valueMax) {
+  uint16_t *ks = reinterpret_cast<uint16_t *>(page + attention_page_key_scales_offset(kv_heads, D));
+  uint16_t *vs = reinterpret_cast<uint16_t *>(page + attention_page_value_scales_offset(kv_heads, D));
+  ks[attention_scale_index(head, token)] = uint16_t(float_to_half_bits(keyMax == 0.0f ? 0.0f : keyMax / 127.0f));
+  vs[attention_scale_index(head, token)] = uint16_t(float_to_half_bits(valueMax == 0.0f ? 0.0f : valueMax / 127.0f));
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -76,7 +97,7 @@ __device__ __forceinline__ uint8_t *page_of(uint8_t *pool, const uint64_t *page_
 // Staged queries: fp16 [sequence][kv head][group head][16 rows][D] (rows past the block zero) and
 // their fp32 sums [sequence][kv head][group head][16].
 // ---------------------------------------------------------------------------------------------
-template <int D>
+template <int D, bool Chunk>
 __global__ __launch_bounds__(D) void attention_q8_qkv(const uint16_t *__restrict__ qkv, const uint16_t *__restrict__ q_norm,
                                                       const uint16_t *__restrict__ k_norm, const float *__restrict__ rope_cos,
                                                       const float *__restrict__ rope_sin, _Float16 *__restrict__ queries,
@@ -85,7 +106,7 @@ __global__ __launch_bounds__(D) void attention_q8_qkv(const uint16_t *__restrict
   __shared__ float scratch[4];
   __shared__ float normalized[D];
   const uint32_t tid = threadIdx.x, head = blockIdx.x, row = blockIdx.y, z = blockIdx.z;
-  const AttentionSequence seq = attention_sequence(p, z);
+  const AttentionSequence seq = block_sequence<Chunk>(p, z);
   const bool query = head < p.q_heads;
   const uint32_t group = p.q_heads / p.kv_heads;
   if (row >= seq.rows) {
@@ -144,28 +165,164 @@ __global__ __launch_bounds__(D) void attention_q8_qkv(const uint16_t *__restrict
     if (tid == 0) qsums[at] = sum;
     return;
   }
-  // attention_store.h:52-85: scale = max / 127, code = clamp(rint(v 127 / max)); the scale is stored fp16.
   const float value = bf16_bits_to_float(source[p.kv_heads * D + tid]);
   const float keyMax = block_max<D>(fabsf(result), scratch, tid), valueMax = block_max<D>(fabsf(value), scratch, tid);
   const uint32_t slot = seq.committed + row, token = slot % ATTENTION_PAGE_TOKENS;
   uint8_t *page = page_of(pool, page_table, seq, p.page_bytes, slot / ATTENTION_PAGE_TOKENS);
-  auto code = [](float v, float maximum) -> int8_t {
-    if (maximum == 0.0f) return 0;
-    const int q = int(rintf(v * 127.0f / maximum));
-    return int8_t(q < -127 ? -127 : q > 127 ? 127 : q);
-  };
-  reinterpret_cast<int8_t *>(page)[attention_key_index(index, token, tid, D)] = code(result, keyMax);
+  reinterpret_cast<int8_t *>(page)[attention_key_index(index, token, tid, D)] = cache_code(result, keyMax);
   reinterpret_cast<int8_t *>(page + attention_page_values_offset(p.kv_heads, D))[attention_value_index(index, token, tid, D)] =
-      code(value, valueMax);
-  if (tid == 0) {
-    uint16_t *ks = reinterpret_cast<uint16_t *>(page + attention_page_key_scales_offset(p.kv_heads, D));
-    uint16_t *vs = reinterpret_cast<uint16_t *>(page + attention_page_value_scales_offset(p.kv_heads, D));
-    ks[attention_scale_index(index, token)] = uint16_t(float_to_half_bits(keyMax == 0.0f ? 0.0f : keyMax / 127.0f));
-    vs[attention_scale_index(index, token)] = uint16_t(float_to_half_bits(valueMax == 0.0f ? 0.0f : valueMax / 127.0f));
+      cache_code(value, valueMax);
+  if (tid == 0) store_cache_scales(page, p.kv_heads, D, index, token, keyMax, valueMax);
+}
+SP_REGISTER_KERNEL("attention_q8_qkv_d128", (&attention_q8_qkv<128, false>));
+SP_REGISTER_KERNEL("attention_q8_qkv_d64", (&attention_q8_qkv<64, false>));
+SP_REGISTER_KERNEL("attention_q8_qkv_chunk_d128", (&attention_q8_qkv<128, true>));
+SP_REGISTER_KERNEL("attention_q8_qkv_chunk_d64", (&attention_q8_qkv<64, true>));
+
+// The same for a prompt chunk's many blocks: grid (q_heads + kv_heads, sequences), a workgroup a head's whole block, each
+// wavefront four of its rows with their loads in flight together and lane l elements l and l + 64 of each. No barrier, and
+// sums and maxima in attention_q8_qkv's order (each 64 elements by a wavefront, then the halves), so every byte is the same.
+// A workgroup a row is bound by how fast workgroups start (147456 of them for 2048 rows of 64 / 8 heads): 114 us there, 45 at
+// 777 rows, against 80 and 34 here. Four rows one after the other take 14.5 us however few the blocks are, 5 us a row each.
+template <int D>
+__global__ __launch_bounds__(256) void attention_q8_qkv_rows(const uint16_t *__restrict__ qkv, const uint16_t *__restrict__ q_norm,
+                                                            const uint16_t *__restrict__ k_norm, const float *__restrict__ rope_cos,
+                                                            const float *__restrict__ rope_sin, _Float16 *__restrict__ queries,
+                                                            float *__restrict__ qsums, const uint64_t *__restrict__ page_table,
+                                                            uint8_t *__restrict__ pool, AttentionParams p) {
+  constexpr uint32_t E = D / 64, kRows = 4;
+  __shared__ float normalized[4][D];
+  const uint32_t l = threadIdx.x & 63u, wave = threadIdx.x >> 6, head = blockIdx.x, z = blockIdx.y;
+  const AttentionSequence seq = block_sequence<true>(p, z);
+  const bool query = head < p.q_heads;
+  const uint32_t group = p.q_heads / p.kv_heads, index = query ? head : head - p.q_heads, pairs = p.rotary_pairs;
+  const uint32_t queryStride = p.gated ? 2u * D : uint32_t(D);
+  const uint32_t offset = query ? index * queryStride : p.q_heads * queryStride + index * D;
+  auto sumOf = [](const float (&v)[E]) __attribute__((always_inline)) {
+    float total = wave_sum(v[0]);
+    if constexpr (E > 1) {
+      total = 0.f + total;
+#pragma unroll
+      for (uint32_t e = 1; e < E; ++e) total += wave_sum(v[e]);
+    }
+    return total;
+  };
+  auto maximumOf = [](const float (&v)[E]) __attribute__((always_inline)) {
+    if constexpr (E == 1) return wave_max(v[0]);
+    auto first = [](float m) { return __uint_as_float(uint32_t(__builtin_amdgcn_readfirstlane(int(__float_as_uint(m))))); };
+    float most = first(wave_max(v[0]));
+#pragma unroll
+    for (uint32_t e = 1; e < E; ++e) most = fmaxf(most, first(wave_max(v[e])));
+    return most;
+  };
+
+  float element[kRows][E], value[kRows][E], cosine[kRows][E], sine[kRows][E], weight[E];
+#pragma unroll
+  for (uint32_t j = 0; j < kRows; ++j) {
+    const uint32_t row = 4u * wave + j;
+    const bool live = row < seq.rows;
+    const size_t packed = size_t(seq.first_row) + row;
+    const uint16_t *source = qkv + packed * p.qkv_stride + offset;
+#pragma unroll
+    for (uint32_t e = 0; e < E; ++e) {
+      const uint32_t d = l + 64u * e;
+      const bool turns = live && d < 2u * pairs;
+      element[j][e] = live ? bf16_bits_to_float(source[d]) : 0.f;
+      value[j][e] = live && !query ? bf16_bits_to_float(source[p.kv_heads * D + d]) : 0.f;
+      const uint32_t pair = d < pairs ? d : d - pairs;
+      cosine[j][e] = turns ? rope_cos[packed * pairs + pair] : 0.f;
+      sine[j][e] = turns ? rope_sin[packed * pairs + pair] : 0.f;
+    }
+  }
+#pragma unroll
+  for (uint32_t e = 0; e < E; ++e) weight[e] = p.normalize ? bf16_bits_to_float((query ? q_norm : k_norm)[l + 64u * e]) : 1.f;
+
+#pragma unroll
+  for (uint32_t j = 0; j < kRows; ++j) {
+    const uint32_t row = 4u * wave + j;
+    const size_t at = ((size_t(z) * p.kv_heads + index / group) * group + index % group) * 16u + row;   // (a query head's)
+    if (row >= seq.rows) {
+      if (query) {
+#pragma unroll
+        for (uint32_t e = 0; e < E; ++e) {
+          if (p.int8_queries) reinterpret_cast<int8_t *>(queries)[at * D + l + 64u * e] = 0;
+          else queries[at * D + l + 64u * e] = _Float16(0.f);
+        }
+        if (l == 0) qsums[at] = 0.f;
+      }
+      continue;
+    }
+    float result[E];
+#pragma unroll
+    for (uint32_t e = 0; e < E; ++e) result[e] = element[j][e];
+    if (p.normalize) {
+      float squares[E];
+#pragma unroll
+      for (uint32_t e = 0; e < E; ++e) squares[e] = element[j][e] * element[j][e];
+      const float inverse = 1.0f / sqrtf(sumOf(squares) / float(D) + 1e-6f);
+#pragma unroll
+      for (uint32_t e = 0; e < E; ++e) result[e] = round_bf16(element[j][e] * inverse * weight[e]);
+    }
+    if (pairs) {
+      wave_lds_fence();
+#pragma unroll
+      for (uint32_t e = 0; e < E; ++e) normalized[wave][l + 64u * e] = result[e];
+      wave_lds_fence();
+#pragma unroll
+      for (uint32_t e = 0; e < E; ++e) {
+        const uint32_t d = l + 64u * e;
+        if (d < 2u * pairs) {
+          const float first = normalized[wave][d < pairs ? d : d - pairs], second = normalized[wave][d < pairs ? d + pairs : d];
+          result[e] = d < pairs ? round_bf16(first * cosine[j][e] - second * sine[j][e]) : round_bf16(second * cosine[j][e] + first * sine[j][e]);
+        }
+      }
+    }
+    float magnitude[E];
+#pragma unroll
+    for (uint32_t e = 0; e < E; ++e) magnitude[e] = fabsf(result[e]);
+    if (query && p.int8_queries) {
+      float wild[E];
+#pragma unroll
+      for (uint32_t e = 0; e < E; ++e) wild[e] = (__float_as_uint(result[e]) & 0x7F800000u) == 0x7F800000u ? 1.f : 0.f;
+      const float notFinite = maximumOf(wild), largest = maximumOf(magnitude);
+      const bool coded = largest > 0x1p-100f;
+      const float inverse = coded ? 127.0f / largest : 0.0f;
+#pragma unroll
+      for (uint32_t e = 0; e < E; ++e) {
+        const float code = fminf(fmaxf(rintf(result[e] * inverse), -127.0f), 127.0f);
+        reinterpret_cast<int8_t *>(queries)[at * D + l + 64u * e] = notFinite != 0.f ? int8_t(0) : int8_t(code);
+      }
+      if (l == 0) qsums[at] = notFinite != 0.f ? __builtin_bit_cast(float, 0x7FC00000u) : coded ? largest / 127.0f : 0.0f;
+    } else if (query) {
+      float staged[E];
+#pragma unroll
+      for (uint32_t e = 0; e < E; ++e) {
+        const _Float16 half = _Float16(result[e]);
+        queries[at * D + l + 64u * e] = half;
+        staged[e] = float(half);
+      }
+      const float sum = sumOf(staged);
+      if (l == 0) qsums[at] = sum;
+    } else {
+      float valueMagnitude[E];
+#pragma unroll
+      for (uint32_t e = 0; e < E; ++e) valueMagnitude[e] = fabsf(value[j][e]);
+      const float keyMax = maximumOf(magnitude), valueMax = maximumOf(valueMagnitude);
+      const uint32_t slot = seq.committed + row, token = slot % ATTENTION_PAGE_TOKENS;
+      uint8_t *page = page_of(pool, page_table, seq, p.page_bytes, slot / ATTENTION_PAGE_TOKENS);
+#pragma unroll
+      for (uint32_t e = 0; e < E; ++e) {
+        const uint32_t d = l + 64u * e;
+        reinterpret_cast<int8_t *>(page)[attention_key_index(index, token, d, D)] = cache_code(result[e], keyMax);
+        reinterpret_cast<int8_t *>(page + attention_page_values_offset(p.kv_heads, D))[attention_value_index(index, token, d, D)] =
+            cache_code(value[j][e], valueMax);
+      }
+      if (l == 0) store_cache_scales(page, p.kv_heads, D, index, token, keyMax, valueMax);
+    }
   }
 }
-SP_REGISTER_KERNEL("attention_q8_qkv_d128", &attention_q8_qkv<128>);
-SP_REGISTER_KERNEL("attention_q8_qkv_d64", &attention_q8_qkv<64>);
+SP_REGISTER_KERNEL("attention_q8_qkv_rows_d128", &attention_q8_qkv_rows<128>);
+SP_REGISTER_KERNEL("attention_q8_qkv_rows_d64", &attention_q8_qkv_rows<64>);
 
 // ---------------------------------------------------------------------------------------------
 // attention_q8_split: grid (kv_heads, splits, sequences), 256 threads.
@@ -178,7 +335,7 @@ SP_REGISTER_KERNEL("attention_q8_qkv_d64", &attention_q8_qkv<64>);
 typedef __attribute__((ext_vector_type(4))) int i32x4;
 // Whole: the workgroup's split is the block's whole history, and its rows leave finished (to `out`, gated by `packed`'s
 // gates where the layer has them) instead of as partials.
-template <int D, int G, bool I8, bool Whole>
+template <int D, int G, bool I8, bool Whole, bool Chunk>
 __device__ __forceinline__ void attention_split(const _Float16 *__restrict__ queries, const float *__restrict__ qsums,
                                                 const AttentionTreeRow *__restrict__ tree, const uint64_t *__restrict__ page_table,
                                                 uint8_t *__restrict__ pool, _Float16 *__restrict__ partialO, float *__restrict__ partialML,
@@ -195,7 +352,7 @@ __device__ __forceinline__ void attention_split(const _Float16 *__restrict__ que
   __shared__ __align__(16) float ldsKS[2][kStep], ldsVS[2][kStep];
 
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, row = lane & 15u, kq = lane >> 4;
-  const AttentionSequence seq = attention_sequence(p, z);
+  const AttentionSequence seq = block_sequence<Chunk>(p, z);
   const uint32_t total = seq.committed + seq.rows;
   // The sequence's own splits: ceil(steps / steps_per_split) of them; later grid rows are empty.
   static_assert(kStep == int(ATTENTION_STEP_TOKENS) && ATTENTION_PAGE_TOKENS % ATTENTION_STEP_TOKENS == 0, "a page holds whole steps");
@@ -495,13 +652,13 @@ __device__ __forceinline__ void attention_split(const _Float16 *__restrict__ que
     }
   }
 }
-template <int D, int G, bool I8>
+template <int D, int G, bool I8, bool Chunk = false>
 __global__ __launch_bounds__(256, 2) void attention_q8_split(const _Float16 *__restrict__ queries, const float *__restrict__ qsums,
                                                           const AttentionTreeRow *__restrict__ tree,
                                                           const uint64_t *__restrict__ page_table, uint8_t *__restrict__ pool,
                                                           _Float16 *__restrict__ partialO, float *__restrict__ partialML,
                                                           AttentionParams p) {
-  attention_split<D, G, I8, false>(queries, qsums, tree, page_table, pool, partialO, partialML, nullptr, nullptr, p, blockIdx.x, blockIdx.y,
+  attention_split<D, G, I8, false, Chunk>(queries, qsums, tree, page_table, pool, partialO, partialML, nullptr, nullptr, p, blockIdx.x, blockIdx.y,
                                    blockIdx.z);
 }
 // attention_q8_whole: grid (kv_heads * blocks), 256 threads. A prompt chunk's blocks of sixteen rows, each over its whole
@@ -515,7 +672,7 @@ __global__ __launch_bounds__(256, 2) void attention_q8_whole(const _Float16 *__r
                                                              uint16_t *__restrict__ out, const uint16_t *__restrict__ packed,
                                                              AttentionParams p) {
   const uint32_t blocks = gridDim.x / p.kv_heads;
-  attention_split<D, G, false, true>(queries, qsums, tree, page_table, pool, nullptr, nullptr, out, packed, p, blockIdx.x % p.kv_heads, 0u,
+  attention_split<D, G, false, true, true>(queries, qsums, tree, page_table, pool, nullptr, nullptr, out, packed, p, blockIdx.x % p.kv_heads, 0u,
                                      blocks - 1u - blockIdx.x / p.kv_heads);
 }
 SP_REGISTER_KERNEL("attention_q8_whole_d128_g8", (&attention_q8_whole<128, 8>));
@@ -524,6 +681,9 @@ SP_REGISTER_KERNEL("attention_q8_whole_d64_g2", (&attention_q8_whole<64, 2>));
 SP_REGISTER_KERNEL("attention_q8_split_d128_g8", &attention_q8_split<128, 8, false>);
 SP_REGISTER_KERNEL("attention_q8_split_d128_g4", &attention_q8_split<128, 4, false>);
 SP_REGISTER_KERNEL("attention_q8_split_d64_g2", &attention_q8_split<64, 2, false>);
+SP_REGISTER_KERNEL("attention_q8_split_chunk_d128_g8", (&attention_q8_split<128, 8, false, true>));
+SP_REGISTER_KERNEL("attention_q8_split_chunk_d128_g4", (&attention_q8_split<128, 4, false, true>));
+SP_REGISTER_KERNEL("attention_q8_split_chunk_d64_g2", (&attention_q8_split<64, 2, false, true>));
 SP_REGISTER_KERNEL("attention_q8q_split_d128_g8", &attention_q8_split<128, 8, true>);
 SP_REGISTER_KERNEL("attention_q8q_split_d128_g4", &attention_q8_split<128, 4, true>);
 SP_REGISTER_KERNEL("attention_q8q_split_d64_g2", &attention_q8_split<64, 2, true>);
@@ -539,7 +699,7 @@ SP_REGISTER_KERNEL("attention_q8q_split_d64_g2", &attention_q8_split<64, 2, true
 // The _t variant also writes the rows as the activation table (abi/Gguf.h) of the projection that
 // follows, as gguf_prepare_table would from `out`; p.table_tiles is the table's row tiles. Rows of
 // a tile past the packed rows keep what the table held.
-template <int D, bool Table>
+template <int D, bool Table, bool Chunk = false>
 __global__ __launch_bounds__(256) void attention_reduce(const _Float16 *__restrict__ partialO, const float *__restrict__ partialML,
                                                         uint16_t *__restrict__ out, uint8_t *__restrict__ table,
                                                         const uint16_t *__restrict__ qkv, AttentionParams p) {
@@ -549,7 +709,7 @@ __global__ __launch_bounds__(256) void attention_reduce(const _Float16 *__restri
   __shared__ __align__(16) float4 sums[kParts][kQuads];
   __shared__ uint16_t staged[D];
   const uint32_t tid = threadIdx.x, head = blockIdx.x, row = blockIdx.y, z = blockIdx.z;
-  const AttentionSequence seq = attention_sequence(p, z);
+  const AttentionSequence seq = block_sequence<Chunk>(p, z);
   if (row >= seq.rows) return;
   const uint32_t group = p.q_heads / p.kv_heads, h = head / group, g = head % group, fusedRows = 16u * group;
   const size_t base = (size_t(z) * p.kv_heads + h) * p.splits;
@@ -636,6 +796,8 @@ __global__ __launch_bounds__(256) void attention_reduce(const _Float16 *__restri
 }
 SP_REGISTER_KERNEL("attention_reduce_d128", &attention_reduce<128, false>);
 SP_REGISTER_KERNEL("attention_reduce_d64", &attention_reduce<64, false>);
+SP_REGISTER_KERNEL("attention_reduce_chunk_d128", (&attention_reduce<128, false, true>));
+SP_REGISTER_KERNEL("attention_reduce_chunk_d64", (&attention_reduce<64, false, true>));
 SP_REGISTER_KERNEL("attention_reduce_d128_t", &attention_reduce<128, true>);
 SP_REGISTER_KERNEL("attention_reduce_d64_t", &attention_reduce<64, true>);
 

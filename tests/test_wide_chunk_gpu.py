@@ -115,3 +115,12 @@ def test_a_wide_hybrid_chunk_is_its_short_chunks_to_rounding(backend, tokens, ex
     far_state = np.sqrt(((seen[0][1] - want_state) ** 2).sum() / (want_state ** 2).sum())
     print(f"  rows: median {np.median(far):.5f}, 95th {np.percentile(far, 95):.5f}, worst {far.max():.5f}; state {far_state:.5f}", flush=True)
     assert np.median(far) <= 1e-2 and np.percentile(far, 90) <= 2e-2 and far_state <= 2e-2
+
+
+@pytest.mark.parametrize("tokens", [511, 512, 525])
+def test_chunks_of_many_blocks_prepare_a_block_a_workgroup(backend, tokens):
+    """From 32 blocks on a chunk's head norms, RoPE and cache store take a workgroup a block (attention_q8_qkv_rows), a ragged
+    last block among them, for plain heads and for gated ones with partial RoPE: held to the same bounds against the
+    sixteen-row steps and the short chunks, whose workgroups take a row."""
+    test_a_wide_chunk_is_its_blocks_to_rounding(backend, tokens, orc.FMT_Q4K)
+    test_a_wide_hybrid_chunk_is_its_short_chunks_to_rounding(backend, tokens, 0, 512)
