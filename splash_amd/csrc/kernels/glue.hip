@@ -161,7 +161,7 @@ SP_REGISTER_KERNEL("norm_rms_table16", &norm_rms_table16);
 // convolution was a launch of its own before a launch of as few workgroups. Values and their order are the two kernels'.
 // The rows' 16-byte accesses are the host's rule (DraftAttention::addConvolutionTable). 8 rows of 5120: 5.3 us
 // for 3.1 + 3.0, 8.8 us for 3.1 + 8.7, and a launch less each: the draft model's pass of one lane 930 -> 888 us
-// on most runs, 908 -> 904 on another.
+// in three runs, 908 -> 904 in another.
 template <bool Residual>
 __global__ __launch_bounds__(256) void draft_conv_table(const uint16_t *__restrict__ input, const uint16_t *__restrict__ dynamic,
                                                         const uint16_t *__restrict__ base, const uint16_t *__restrict__ residual,
