@@ -686,9 +686,14 @@ sp_status spo_dense_verify_set_head(spo_dense_verify *verify, uint32_t embedding
                                     sp_buffer *final_norm, const spo_projection *head);
 /* DenseVerify::setStagedPrefill: a prompt chunk of more rows than a step's runs its projections through the prefill tile
  * (spo_linear_add_prefill: the staged rule, as the reference's prompt chunks do, LinearTile::GgufPrefill), its norms and
- * SwiGLU as passes of their own; off by default (the chunk then equals its blocks run as steps bit for bit). Needs a
- * driver created with prefill_rows and tensors of whole 128-column workgroups. */
+ * SwiGLU as passes of their own; a chunk that takes the wide kernels (spo_dense_verify_encode_prefill) takes their staged
+ * ones. Off by default. Needs a driver created with prefill_rows and tensors of whole 128-column workgroups. */
 sp_status spo_dense_verify_set_staged_prefill(spo_dense_verify *verify, int on);
+/* DenseVerify::setExactPrefill: the prompt chunks encoded from now on take no wide kernel (spo_dense_verify_encode_prefill
+ * says which chunks would), for a caller that reuses or replays pages: each leaves the pages and hidden rows of its blocks
+ * run as steps, bit for bit, however the prompt is cut (with the staged prefill on, those of the prefill tile). Off by
+ * default. */
+sp_status spo_dense_verify_set_exact_prefill(spo_dense_verify *verify, int on);
 /* The hidden rows a draft's context is computed from (QwenTarget's addCapture over RowCopy, runtime/ops/RowCopy.hpp:17-28):
  * after layer layers[i] (ascending) every row's output goes to columns [i * hidden, (i + 1) * hidden) of its row of
  * destination, bf16 [rows][count * hidden], in a step and in a prompt chunk alike; what spo_dflash_draft's context calls
@@ -775,8 +780,11 @@ sp_status spo_dense_verify_chain_status(spo_dense_verify *verify, uint32_t *stat
  * chunks (Runtime.cpp's chunked prefill over QwenTarget.cpp:457-496): the tokens go in SPO_VERIFY_INPUT_TOKENS, a chain
  * of tree rows a block of sixteen in SPO_VERIFY_TREE_ROWS, each row's depth in its block in SPO_VERIFY_DEPTHS, as a
  * step's. Every layer runs, the head and the acceptance do not: the tokens' keys and values are in the pages and the
- * hidden rows where a step leaves them, bit for bit those of the blocks run one step after the other; the caller
- * advances the sequence's committed tokens. */
+ * hidden rows where a step leaves them; the caller advances the sequence's committed tokens. What a chunk leaves is, bit
+ * for bit, what its blocks leave run one step after the other, but for a chunk that takes the wide kernels: one of more
+ * than a step's rows and at least 65, of a model of 2048 to 8192 columns whose projections are each of one format, Q4_K,
+ * Q5_K or Q6_K, gate and up of the same one. That one equals the blocks to the rounding of bf16 rows, and a prompt cut
+ * into other chunks leaves other bits; spo_dense_verify_set_exact_prefill keeps every chunk off those kernels. */
 sp_status spo_dense_verify_encode_prefill(spo_dense_verify *verify, spo_graph *graph, uint32_t table_first, uint32_t committed,
                                           uint32_t tokens);
 sp_status spo_dense_verify_set_chained(spo_dense_verify *verify, int chained);
@@ -844,10 +852,16 @@ sp_status spo_hybrid_verify_set_thinking_cutoff(spo_hybrid_verify *verify, uint3
  * layer_count) (layer_count 0: to the last; the embedding with first_layer 0), no head: the reference's chunked prefill over
  * its hybrid target (QwenTarget.cpp:206-347 with GDN::addPrefill, GDN.cpp:132-222; PagedAttention.cpp:351-389). Attention
  * layers store the chunk's keys and values and attend causally; Gated DeltaNet layers take every row into the state, from
- * the lane's cell of `parity` to its other cell: the lane's next step has the other parity and no pending path. */
+ * the lane's cell of `parity` to its other cell: the lane's next step has the other parity and no pending path. A prompt
+ * cut into other chunks leaves the same bits, but for chunks that take the wide kernels: of at least 257 rows, of a model
+ * of 2048 to 8192 columns whose projections, router and gate columns among them, are each of one format, Q4_K, Q5_K or
+ * Q6_K, its experts too (a model loaded from a GGUF, whose router and gates are rows of floats, is not one). Those equal
+ * the others to the rounding of bf16 rows. */
 sp_status spo_hybrid_verify_encode_prefill(spo_hybrid_verify *verify, spo_graph *graph, uint32_t lane, uint32_t table_first,
                                            uint32_t committed, uint32_t tokens, uint32_t parity, uint32_t first_layer,
                                            uint32_t layer_count);
+/* As spo_dense_verify_set_exact_prefill: the chunks encoded from now on take no wide kernel. Off by default. */
+sp_status spo_hybrid_verify_set_exact_prefill(spo_hybrid_verify *verify, int on);
 /* As spo_dense_verify_results. */
 sp_status spo_hybrid_verify_results(spo_hybrid_verify *verify, const spo_hybrid_lane *lanes, uint32_t count, uint32_t *tokens,
                                     uint32_t *retained, uint32_t *accepted, uint32_t *retained_rows);

@@ -80,6 +80,13 @@ sp_status spo_hybrid_verify_set_capture(spo_hybrid_verify *verify, const uint32_
   });
 }
 
+sp_status spo_hybrid_verify_set_exact_prefill(spo_hybrid_verify *verify, int on) {
+  return capi::guard([&] {
+    capi::require(verify, "verify");
+    verify->verify->setExactPrefill(on != 0);
+  });
+}
+
 sp_status spo_hybrid_verify_set_penalties(spo_hybrid_verify *verify, uint32_t lane, float repetition, float presence, float frequency) {
   return capi::guard([&] {
     capi::require(verify, "verify");

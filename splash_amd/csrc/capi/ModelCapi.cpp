@@ -270,6 +270,12 @@ sp_status spo_dense_verify_set_staged_prefill(spo_dense_verify *verify, int on) 
     verify->verify->setStagedPrefill(on != 0);
   });
 }
+sp_status spo_dense_verify_set_exact_prefill(spo_dense_verify *verify, int on) {
+  return capi::guard([&] {
+    capi::require(verify, "verify");
+    verify->verify->setExactPrefill(on != 0);
+  });
+}
 
 sp_status spo_dense_verify_set_capture(spo_dense_verify *verify, const uint32_t *layers, uint32_t count, sp_buffer *destination) {
   return capi::guard([&] {

@@ -366,7 +366,7 @@ bool DenseVerify::wideChunks() const noexcept {
   return rowCapacity_ > maxRows_ && dims_.hidden >= kWideHidden && dims_.hidden <= ops::Linear::kMaximumWideNormWidth;
 }
 bool DenseVerify::takesWide(uint32_t tokens) const {
-  if (!wideChunks() || tokens < kWideRows) return false;
+  if (exactPrefill_ || !wideChunks() || tokens < kWideRows) return false;
   for (const DenseLayer &l : weights_.layers) {
     for (const ops::Projection *p : {&l.qkv, &l.output, &l.gate, &l.up, &l.down})
       if (!ops::Linear::takesWide(*p)) return false;

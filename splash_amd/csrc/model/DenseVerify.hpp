@@ -126,10 +126,16 @@ public:
   // depths where a step's are) in one pass over the layers: the chunk runs as blocks of sixteen rows of one sequence,
   // block i's history ending where block i - 1's rows end, through every layer and no head, so the tokens' keys and
   // values are in the pages and the hidden rows where a step leaves them. The counterpart of the reference's chunked
-  // prefill (Runtime.cpp's prefill chunks over QwenTarget's layers) with the verify step's own kernels: the pools and
-  // the hidden rows are those of the blocks run one step after the other, bit for bit. A chunk of more rows than a
-  // step's runs layer by layer: the projections in windows of ops::kMaximumDispatchRows rows around one chunked
-  // attention (ops::PagedAttention::planChunks) over all of them.
+  // prefill (Runtime.cpp's prefill chunks over QwenTarget's layers). A chunk of up to a step's rows is one pass of the
+  // verify step's own kernels: the pools and the hidden rows are those of the blocks run one step after the other, bit
+  // for bit. A chunk of more rows than a step's runs layer by layer, in one of two ways:
+  //  - through the wide kernels (ops::Linear::addWide, ops::PagedAttention::planPrompt), where the chunk has at least
+  //    kWideRows rows, the model at least kWideHidden columns and every layer's projections are tensors the kernels take
+  //    (each projection of one format, Q4_K, Q5_K or Q6_K; gate and up of the same one). The weights and the rows are the
+  //    step's, the sums in another order and a norm's rounding in another place: what it leaves equals the blocks run as
+  //    steps to the rounding of bf16 rows, and a prompt cut into other chunks leaves other bits;
+  //  - otherwise, and always under setExactPrefill, the projections in windows of ops::kMaximumDispatchRows rows around one
+  //    chunked attention (ops::PagedAttention::planChunks) over all of them: the bits of the blocks run as steps.
   void encodePrefill(hip::CommandGraph &graph, uint32_t tableFirst, uint32_t committed, uint32_t tokens);
   // A layer's q|k|v projection also prepares its attention block (ops::PagedAttention::addFusedProjection) where the
   // kernels take the pair: off by default (the projection and the prepare kernel run one after the other). The results
@@ -140,11 +146,16 @@ public:
   // A long prompt chunk (more rows than a step's) runs its projections through the prefill tile (ops::Linear::addPrefill:
   // 128 rows x 128 columns a workgroup under the staged rule, every weight rounded once to half), as the reference's
   // prompt chunks do (LinearTile::GgufPrefill, gguf_linear.metal:79-118): the norms and the SwiGLU are passes of their
-  // own, the attention the same chunked plan. Off by default: a chunk then equals its blocks run as steps bit for bit;
-  // on, it equals them to the staged rule's rounding and runs at the matrix cores' rate, not the step kernels'.
+  // own, the attention the same chunked plan; a chunk that takes the wide kernels (encodePrefill) takes their staged ones.
+  // Off by default; on, a chunk equals its blocks run as steps to the staged rule's rounding.
   // Every tensor's columns must be whole 128-column workgroups.
   void setStagedPrefill(bool staged);
   [[nodiscard]] bool stagedPrefill() const noexcept { return stagedPrefill_; }
+  // Whether the prompt chunks encoded after keep to kernels whose rows do not depend on how a prompt is cut, for a caller
+  // that reuses or replays pages: no chunk takes the wide kernels. Every chunk then leaves the pools and hidden rows of its
+  // blocks run as steps, bit for bit (with setStagedPrefill, those of the prefill tile over any other cut). Off by default.
+  void setExactPrefill(bool exact) noexcept { exactPrefill_ = exact; }
+  [[nodiscard]] bool exactPrefill() const noexcept { return exactPrefill_; }
   // The hidden rows a draft's context is computed from (the reference's QwenTarget addCapture over RowCopy,
   // RowCopy.hpp:17-28): after layer layers[i] (ascending), every row's output goes to columns [i hidden, (i + 1) hidden)
   // of its row of `destination`, bf16 [rows][layers.size() x hidden]; a step's rows and a prompt chunk's alike. A
@@ -179,7 +190,7 @@ private:
   hip::Buffer captured_;
   void encodeCapture(hip::CommandGraph &graph, uint32_t layer, uint32_t rows) const;
   ops::SamplingBuffers children_;   // the four candidate-children buffers, bound into a step's sampling buffers when it tests them
-  bool stagedPrefill_ = false;
+  bool stagedPrefill_ = false, exactPrefill_ = false;
   hip::Buffer prefillTable_, gateRows_, upRows_, swigluRows_;  // the prefill tile's tables and SwiGLU rows
   hip::Buffer wideTable_, wideRows_, widePartials_;             // the wide kernels' table, SwiGLU rows and parts' sums
   void encodeStagedChunkLayer(hip::CommandGraph &graph, uint32_t layer, const ops::AttentionChunkPlan &plan, uint32_t tokens);

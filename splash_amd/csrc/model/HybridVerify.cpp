@@ -151,7 +151,7 @@ bool HybridVerify::wideChunks() const noexcept {
   return rowCapacity_ >= kWideRows && dims_.hidden >= kWideHidden && dims_.hidden <= ops::Linear::kMaximumWideNormWidth;
 }
 bool HybridVerify::takesWide(uint32_t tokens) const {
-  if (!wideChunks() || tokens < kWideRows) return false;
+  if (exactPrefill_ || !wideChunks() || tokens < kWideRows) return false;
   for (const HybridLayer &l : weights_.layers) {
     if (!ops::Linear::takesWide(l.mixerInput) || !ops::Linear::takesWide(l.mixerOutput) || l.gateRows) return false;
     if (dims_.dense()) {

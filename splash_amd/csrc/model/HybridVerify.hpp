@@ -182,9 +182,17 @@ public:
   // values and attend causally (ops::PagedAttention::planChunks); Gated DeltaNet layers take every row into the state
   // (ops::GDN::addPrefill), from the lane's cell of `parity` to its other cell, so the lane's next step has the other
   // parity and no pending path. The embedding runs with firstLayer 0. Projections and experts run in windows of
-  // ops::kMaximumDispatchRows rows.
+  // ops::kMaximumDispatchRows rows, and a prompt cut into other chunks leaves the same bits; or, for a chunk of at least
+  // kWideRows rows of a model of at least kWideHidden columns whose every layer the wide kernels take (projections of one
+  // format each, Q4_K, Q5_K or Q6_K, the router and the gate columns among them; expert images of those formats), in one
+  // pass of the wide kernels over all the rows, equal to the windows to the rounding of bf16 rows. A model loaded from a
+  // GGUF keeps its router and its GDN gates as rows of floats, so its chunks run in windows.
   void encodePrefill(hip::CommandGraph &graph, uint32_t lane, uint32_t tableFirst, uint32_t committed, uint32_t tokens, uint32_t parity,
                      uint32_t firstLayer = 0, uint32_t layerCount = 0);
+  // As DenseVerify::setExactPrefill: the chunks encoded after run in windows, whose rows do not depend on how the prompt is
+  // cut. Off by default.
+  void setExactPrefill(bool exact) noexcept { exactPrefill_ = exact; }
+  [[nodiscard]] bool exactPrefill() const noexcept { return exactPrefill_; }
 
 private:
   void encodePrefillLayer(hip::CommandGraph &graph, uint32_t layer, const ops::AttentionChunkPlan &plan, uint32_t tokens, uint64_t currentCell,
@@ -210,7 +218,7 @@ private:
   ops::Linear linear_;
   uint32_t maxRows_ = 0, maxLanes_ = 0, rowCapacity_ = 0;
   LanePolicies lanePolicies_;
-  bool tiledGdnHeads_ = false;
+  bool tiledGdnHeads_ = false, exactPrefill_ = false;
   std::vector<uint32_t> captureLayers_;
   hip::Buffer captured_;
   void encodeCapture(hip::CommandGraph &graph, uint32_t layer, uint32_t rows) const;

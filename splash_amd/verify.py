@@ -76,6 +76,11 @@ class DenseVerify:
         """Long prompt chunks through the prefill tile (the staged rule) instead of the step's kernels; off by default."""
         check(lib.spo_dense_verify_set_staged_prefill(self.handle, int(on)))
 
+    def set_exact_prefill(self, on):
+        """Whether the prompt chunks encoded from now on keep off the wide kernels, so that each leaves the bits of its blocks
+        run as steps however the prompt is cut; off by default."""
+        check(lib.spo_dense_verify_set_exact_prefill(self.handle, int(bool(on))))
+
     def set_penalties(self, lane, repetition=1.0, presence=0.0, frequency=0.0):
         """The sampling penalties of dispatch lane `lane` for the steps encoded after; its row of the PENALTY_WORDS buffer
         (uint32 [lanes][vocabulary]; ops.Sampling.rebuild_penalty_words makes a row) holds what they read."""
@@ -347,6 +352,10 @@ class HybridVerify:
                                                    layer_count))
         graph._keep.append(self)
         return graph
+
+    def set_exact_prefill(self, on):
+        """As DenseVerify.set_exact_prefill."""
+        check(lib.spo_hybrid_verify_set_exact_prefill(self.handle, int(bool(on))))
 
     set_block = DenseVerify.set_block
     set_prefill_block = DenseVerify.set_prefill_block

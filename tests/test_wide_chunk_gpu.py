@@ -124,3 +124,81 @@ def test_chunks_of_many_blocks_prepare_a_block_a_workgroup(backend, tokens):
     sixteen-row steps and the short chunks, whose workgroups take a row."""
     test_a_wide_chunk_is_its_blocks_to_rounding(backend, tokens, orc.FMT_Q4K)
     test_a_wide_hybrid_chunk_is_its_short_chunks_to_rounding(backend, tokens, 0, 512)
+
+
+@pytest.mark.parametrize("tokens", [65, 300])
+def test_an_exact_wide_model_chunk_equals_its_blocks(backend, tokens):
+    """DenseVerify::setExactPrefill: a chunk that would take the wide kernels leaves the pages and the hidden rows of its
+    blocks run as steps, bit for bit, whole or cut in two; the switch off, the wide kernels run again."""
+    print(f"case exact chunk tokens={tokens}", flush=True)
+    H, layers = 2048, 2
+    model = DenseModel(seed=37, hidden=H, q_heads=16, kv_heads=4, head_dim=128, ffn=2304, vocabulary=512, layers=layers)
+    rng = np.random.default_rng(tokens)
+    gpu = model.build_gpu(backend, max_lanes=1, context_tokens=[tokens + 300], prefill_rows=tokens)
+    model.seed_context(gpu, None, rng)
+    first, committed = model.table_first[0], 250
+    prompt = rng.integers(0, 512, tokens).astype(np.uint32)
+    pools = lambda: np.concatenate([gpu.buffer(verify.KV_POOL, layer).download(np.uint8) for layer in range(layers)])
+    rows_of = lambda rows: gpu.buffer(verify.HIDDEN, 0).download(np.uint16, rows * H).copy()
+    start = pools()
+
+    def restore():
+        for layer in range(layers):
+            gpu.buffer(verify.KV_POOL, layer).upload(start.reshape(layers, -1)[layer])
+    hidden = []
+    for at in range(0, tokens, 16):
+        rows = min(16, tokens - at)
+        lane = verify.Lane(rows, committed + at, table_first=first)
+        gpu.set_block([lane], prompt[at:at + rows])
+        backend.run(gpu.encode([lane], commit=False))
+        hidden.append(rows_of(rows))
+    want_hidden, want_pools = np.concatenate(hidden), pools()
+    gpu.set_exact_prefill(True)
+    for cuts in ([0, tokens], [0, 23, tokens]):
+        restore()
+        got = []
+        for a, b in zip(cuts, cuts[1:]):
+            gpu.set_prefill_block(prompt[a:b])
+            graph = gpu.encode_prefill(first, committed + a, b - a)
+            assert not any("wide" in name for name in graph.kernels())
+            backend.run(graph)
+            got.append(rows_of(b - a))
+        assert np.array_equal(np.concatenate(got), want_hidden) and np.array_equal(pools(), want_pools)
+    gpu.set_exact_prefill(False)
+    assert any("wide" in name for name in gpu.encode_prefill(first, committed, tokens).kernels())
+
+
+def test_an_exact_wide_hybrid_chunk_is_the_same_however_it_is_cut(backend):
+    """HybridVerify::setExactPrefill: the chunk whole leaves the hidden rows, pages and recurrent state of the same prompt in
+    chunks of 64 rows, bit for bit."""
+    from tests.hybrid_reference import HybridModel
+    print("case exact hybrid chunk", flush=True)
+    H, V, tokens, committed = 2048, 512, 300, 200
+    model = HybridModel(seed=59, hidden=H, vocabulary=V, layers=4, q_heads=8, kv_heads=2, head_dim=128, gdn_key_heads=2, gdn_value_heads=4,
+                        experts=16, top_k=2, expert_ffn=256, shared_slices=1, shared_gate=True, gated_attention=True)
+    gpu = model.build_gpu(backend, max_lanes=1, pages_per_lane=3, prefill_rows=tokens)
+    rng = np.random.default_rng(tokens)
+    model.seed_context(rng)
+    model.seed_states(rng, lanes=1)
+    prompt = rng.integers(0, V, tokens).astype(np.uint32)
+    start_pool, start_cells = gpu.buffer(verify.KV_POOL, 0).download(np.uint8), gpu.buffer(verify.GDN_STATES).download(np.uint8)
+    seen = []
+    for size in (64, tokens):
+        gpu.buffer(verify.KV_POOL, 0).upload(start_pool)
+        gpu.buffer(verify.GDN_STATES).upload(start_cells)
+        gpu.set_exact_prefill(size == tokens)
+        hidden, parity = [], 0
+        for at in range(0, tokens, size):
+            rows = min(size, tokens - at)
+            gpu.set_prefill_block(prompt[at:at + rows])
+            graph = gpu.encode_prefill(0, 0, committed + at, rows, parity=parity)
+            assert not any("wide" in name for name in graph.kernels())
+            backend.run(graph)
+            hidden.append(gpu.buffer(verify.HIDDEN, 0).download(np.uint16, rows * H).copy())
+            parity ^= 1
+        cell = gpu.buffer(verify.GDN_STATES).download(np.uint8, gpu.cell_bytes, gpu.cell_offset(0, parity))
+        seen.append((np.concatenate(hidden), gpu.buffer(verify.KV_POOL, 0).download(np.uint8), cell))
+    for got, want in zip(seen[1], seen[0]):
+        assert np.array_equal(got, want)
+    gpu.set_exact_prefill(False)
+    assert any("wide" in name for name in gpu.encode_prefill(0, 0, committed, tokens).kernels())
