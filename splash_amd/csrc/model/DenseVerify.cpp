@@ -345,19 +345,17 @@ void DenseVerify::encodeHead(hip::CommandGraph &graph, uint32_t rows, bool input
 }
 
 void DenseVerify::setStagedPrefill(bool staged) {
-  if (staged && rowCapacity_ <= maxRows_) throw std::invalid_argument("the driver was created without room for a long prompt chunk");
+  if (staged && !swigluRows_) {
+    if (rowCapacity_ <= maxRows_) throw std::invalid_argument("the driver was created without room for a long prompt chunk");
+    // (also where the wide kernels take the model's long chunks: shorter ones, and exact ones, take the prefill tile)
+    const uint32_t widest = std::max({dims_.hidden, dims_.attentionWidth(), dims_.ffn});
+    prefillTable_ = backend_.allocateBuffer(ops::Linear::prefillTableBytes(widest, rowCapacity_), BufferStorage::Private, "prefill tables");
+    const uint64_t ffnBytes = uint64_t{rowCapacity_} * dims_.ffn * 2;
+    gateRows_ = backend_.allocateBuffer(ffnBytes, BufferStorage::Private, "prefill gate rows");
+    upRows_ = backend_.allocateBuffer(ffnBytes, BufferStorage::Private, "prefill up rows");
+    swigluRows_ = backend_.allocateBuffer(ffnBytes, BufferStorage::Private, "prefill SwiGLU rows");
+  }
   stagedPrefill_ = staged;
-}
-
-// The rows of the prefill tile's projections, where the wide kernels do not take the model's.
-void DenseVerify::needPrefillRows() {
-  if (prefillTable_) return;
-  const uint32_t widest = std::max({dims_.hidden, dims_.attentionWidth(), dims_.ffn});
-  prefillTable_ = backend_.allocateBuffer(ops::Linear::prefillTableBytes(widest, rowCapacity_), BufferStorage::Private, "prefill tables");
-  const uint64_t ffnBytes = uint64_t{rowCapacity_} * dims_.ffn * 2;
-  gateRows_ = backend_.allocateBuffer(ffnBytes, BufferStorage::Private, "prefill gate rows");
-  upRows_ = backend_.allocateBuffer(ffnBytes, BufferStorage::Private, "prefill up rows");
-  swigluRows_ = backend_.allocateBuffer(ffnBytes, BufferStorage::Private, "prefill SwiGLU rows");
 }
 
 // Whether chunks may take the wide kernels: from this width on the projections are most of a chunk's time. Narrower
@@ -502,7 +500,6 @@ void DenseVerify::encodePrefill(hip::CommandGraph &graph, uint32_t tableFirst, u
     encodeEmbedding(graph, tokens);
     // every window is a step's worth of rows at most, so what holds for one holds for all
     const bool feeds = layersFeedNext(std::min(tokens, kWindowRows));
-    if (stagedPrefill_ && !wide) needPrefillRows();
     for (uint32_t layer = 0; layer < dims_.layers; ++layer) {
       if (wide) encodeWideChunkLayer(graph, layer, widePlan, tokens);
       else if (stagedPrefill_) encodeStagedChunkLayer(graph, layer, plan, tokens);

@@ -148,7 +148,7 @@ public:
   // prompt chunks do (LinearTile::GgufPrefill, gguf_linear.metal:79-118): the norms and the SwiGLU are passes of their
   // own, the attention the same chunked plan; a chunk that takes the wide kernels (encodePrefill) takes their staged ones.
   // Off by default; on, a chunk equals its blocks run as steps to the staged rule's rounding.
-  // Every tensor's columns must be whole 128-column workgroups.
+  // Every tensor's columns must be whole 128-column workgroups. Turning it on allocates the tile's rows, once.
   void setStagedPrefill(bool staged);
   [[nodiscard]] bool stagedPrefill() const noexcept { return stagedPrefill_; }
   // Whether the prompt chunks encoded after keep to kernels whose rows do not depend on how a prompt is cut, for a caller
@@ -199,7 +199,6 @@ private:
   [[nodiscard]] bool wideChunks() const noexcept;
   [[nodiscard]] bool takesWide(uint32_t tokens) const;
   void encodeWideChunkLayer(hip::CommandGraph &graph, uint32_t layer, const ops::AttentionPromptPlan &plan, uint32_t tokens);
-  void needPrefillRows();
   hip::Buffer chunkAttentionTable_;  // a long chunk's attention rows as the output projection's tables, every window's
   void encodeChunkLayer(hip::CommandGraph &graph, uint32_t layer, const ops::AttentionChunkPlan &plan, uint32_t tokens, bool first,
                         bool feedsNext);

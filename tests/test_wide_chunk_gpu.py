@@ -202,3 +202,19 @@ def test_an_exact_wide_hybrid_chunk_is_the_same_however_it_is_cut(backend):
         assert np.array_equal(got, want)
     gpu.set_exact_prefill(False)
     assert any("wide" in name for name in gpu.encode_prefill(0, 0, committed, tokens).kernels())
+
+
+@pytest.mark.parametrize("hidden,tokens", [(1024, 100), (2048, 40)])
+def test_a_staged_chunk_allocates_nothing(backend, hidden, tokens):
+    """The rows of the prefill tile are there once setStagedPrefill returns, also those of a model whose longer chunks take
+    the wide kernels: encoding a chunk takes no memory, and cannot run out of it after dispatches were added to the graph."""
+    print(f"case staged chunk memory hidden={hidden}", flush=True)
+    model = DenseModel(seed=41, hidden=hidden, q_heads=16, kv_heads=4, head_dim=128, ffn=1024, vocabulary=512, layers=1)
+    gpu = model.build_gpu(backend, max_lanes=1, context_tokens=[256], prefill_rows=128)
+    before = backend.memory_stats().allocated_bytes
+    gpu.set_staged_prefill(True)
+    held = backend.memory_stats().allocated_bytes
+    assert held - before >= 3 * 128 * 1024 * 2
+    graph = gpu.encode_prefill(0, 0, tokens)
+    assert any(name.startswith("gguf_prefill") for name in graph.kernels())
+    assert backend.memory_stats().allocated_bytes == held
