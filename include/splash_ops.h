@@ -784,7 +784,9 @@ sp_status spo_dense_verify_chain_status(spo_dense_verify *verify, uint32_t *stat
  * for bit, what its blocks leave run one step after the other, but for a chunk that takes the wide kernels: one of more
  * than a step's rows and at least 65, of a model of 2048 to 8192 columns whose projections are each of one format, Q4_K,
  * Q5_K or Q6_K, gate and up of the same one. That one equals the blocks to the rounding of bf16 rows, and a prompt cut
- * into other chunks leaves other bits; spo_dense_verify_set_exact_prefill keeps every chunk off those kernels. */
+ * into other chunks leaves other bits; spo_dense_verify_set_exact_prefill keeps every chunk off those kernels. A driver
+ * whose weights they take holds their buffers (420 MB at the 27B shape and 2048 rows) from the last layer's weights on,
+ * unless its chunks were exact before. */
 sp_status spo_dense_verify_encode_prefill(spo_dense_verify *verify, spo_graph *graph, uint32_t table_first, uint32_t committed,
                                           uint32_t tokens);
 sp_status spo_dense_verify_set_chained(spo_dense_verify *verify, int chained);

@@ -178,6 +178,7 @@ sp_status spo_hybrid_verify_set_layer(spo_hybrid_verify *verify, uint32_t layer,
     }
     if (l->shared_scalar_gate) out.sharedScalarGate = B(l->shared_scalar_gate);
     w.layers[layer] = std::move(out);
+    verify->verify->prepareChunks();
   });
 }
 sp_status spo_hybrid_verify_set_head(spo_hybrid_verify *verify, uint32_t embedding_format, sp_buffer *embedding_rows, sp_buffer *final_norm,

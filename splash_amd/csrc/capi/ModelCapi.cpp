@@ -325,6 +325,7 @@ sp_status spo_dense_verify_set_layer(spo_dense_verify *verify, uint32_t layer, c
     if (layer >= w.layers.size()) throw std::invalid_argument("no such layer");
     w.layers[layer] = {capi::projectionOf(qkv), capi::projectionOf(output), capi::projectionOf(gate), capi::projectionOf(up),
                        capi::projectionOf(down), B(input_norm), B(post_norm), B(query_norm), B(key_norm)};
+    verify->verify->prepareChunks();
   });
 }
 sp_status spo_dense_verify_set_head(spo_dense_verify *verify, uint32_t embedding_format, sp_buffer *embedding_rows,

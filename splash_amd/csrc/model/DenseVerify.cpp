@@ -91,15 +91,6 @@ DenseVerify::DenseVerify(hip::Backend &backend, DenseDimensions d, uint32_t maxL
   nextTable_ = device(gguf_tables_bytes(std::max(d.attentionWidth(), d.ffn), gguf_row_tiles(windowRows)), "linear table 2");
   if (rowCapacity_ > maxRows_)
     chunkAttentionTable_ = device(gguf_tables_bytes(d.attentionWidth(), gguf_row_tiles(rowCapacity_)), "chunk attention table");
-  if (wideChunks()) {
-    const uint32_t widest = std::max({d.hidden, d.attentionWidth(), d.ffn});
-    wideTable_ = device(ops::Linear::wideTableBytes(widest, rowCapacity_), "wide table");
-    wideRows_ = device(C * d.ffn * 2, "chunk SwiGLU rows");
-    uint64_t partials = 0;
-    for (ops::LinearMatrix m : {ops::LinearMatrix{d.qkvWidth(), d.hidden}, ops::LinearMatrix{d.hidden, d.attentionWidth()}, ops::LinearMatrix{d.hidden, d.ffn}})
-      partials = std::max(partials, linear_.widePartialBytes(m, rowCapacity_));
-    widePartials_ = device(partials, "wide partials");
-  }
   // Chained projections each keep a table, partials and counters of their own.
   chainTables_[0] = device(gguf_table_bytes(d.hidden, gguf_row_tiles(maxRows_)), "gate/up table");
   chainTables_[1] = device(gguf_table_bytes(d.ffn, gguf_row_tiles(maxRows_)), "down table");
@@ -364,7 +355,10 @@ bool DenseVerify::wideChunks() const noexcept {
   return rowCapacity_ > maxRows_ && dims_.hidden >= kWideHidden && dims_.hidden <= ops::Linear::kMaximumWideNormWidth;
 }
 bool DenseVerify::takesWide(uint32_t tokens) const {
-  if (exactPrefill_ || !wideChunks() || tokens < kWideRows) return false;
+  return tokens > maxRows_ && tokens >= kWideRows && modelTakesWide();
+}
+bool DenseVerify::modelTakesWide() const {
+  if (exactPrefill_ || !wideChunks()) return false;
   for (const DenseLayer &l : weights_.layers) {
     for (const ops::Projection *p : {&l.qkv, &l.output, &l.gate, &l.up, &l.down})
       if (!ops::Linear::takesWide(*p)) return false;
@@ -373,6 +367,19 @@ bool DenseVerify::takesWide(uint32_t tokens) const {
       return false;
   }
   return true;
+}
+
+void DenseVerify::prepareChunks() {
+  if (widePartials_ || !modelTakesWide()) return;
+  const DenseDimensions &d = dims_;
+  auto device = [&](uint64_t bytes, const char *label) { return backend_.allocateBuffer(std::max<uint64_t>(bytes, 16), BufferStorage::Private, label); };
+  const uint32_t widest = std::max({d.hidden, d.attentionWidth(), d.ffn});
+  uint64_t partials = 0;
+  for (ops::LinearMatrix m : {ops::LinearMatrix{d.qkvWidth(), d.hidden}, ops::LinearMatrix{d.hidden, d.attentionWidth()}, ops::LinearMatrix{d.hidden, d.ffn}})
+    partials = std::max(partials, linear_.widePartialBytes(m, rowCapacity_));
+  wideTable_ = device(ops::Linear::wideTableBytes(widest, rowCapacity_), "wide table");
+  wideRows_ = device(uint64_t{rowCapacity_} * d.ffn * 2, "chunk SwiGLU rows");
+  widePartials_ = device(partials, "wide partials");
 }
 
 // A layer of a long chunk through the wide kernels: every projection one pass over all the rows.
@@ -480,6 +487,7 @@ void DenseVerify::encodePrefill(hip::CommandGraph &graph, uint32_t tableFirst, u
   if (tokens > maxRows_) {
     const ops::AttentionGeometry geometry{dims_.qHeads, dims_.kvHeads, dims_.headDimension, dims_.rotaryPairs, dims_.normalizeHeads};
     const bool wide = takesWide(tokens);
+    if (wide) prepareChunks();
     ops::AttentionChunkPlan plan;
     ops::AttentionPromptPlan widePlan;
     if (wide) widePlan = ops::PagedAttention::planPrompt(geometry, {0, tokens, committed, tableFirst}, linear_.calibration().computeUnits);

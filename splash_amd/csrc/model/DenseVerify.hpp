@@ -60,6 +60,12 @@ public:
 
   [[nodiscard]] const DenseDimensions &dimensions() const noexcept { return dims_; }
   DenseWeights &weights() noexcept { return weights_; }
+  // Allocates what the model's long prompt chunks hold beyond a step's rows, where they take the wide kernels
+  // (encodePrefill): a table, SwiGLU rows and partial sums, 420 MB at the 27B shape and 2048 rows. For whoever set the
+  // weights to call then (the GGUF loader and the C entry points do); without it the first such chunk allocates, before it
+  // adds a dispatch. A driver whose chunks are exact (setExactPrefill, before the weights are set) or whose weights the wide
+  // kernels do not take holds none of it.
+  void prepareChunks();
   // Host-visible step inputs and results (Shared storage).
   [[nodiscard]] const hip::Buffer &inputTokens() const noexcept { return inputTokens_; }
   [[nodiscard]] const hip::Buffer &treeRows() const noexcept { return treeRows_; }
@@ -154,7 +160,10 @@ public:
   // Whether the prompt chunks encoded after keep to kernels whose rows do not depend on how a prompt is cut, for a caller
   // that reuses or replays pages: no chunk takes the wide kernels. Every chunk then leaves the pools and hidden rows of its
   // blocks run as steps, bit for bit (with setStagedPrefill, those of the prefill tile over any other cut). Off by default.
-  void setExactPrefill(bool exact) noexcept { exactPrefill_ = exact; }
+  void setExactPrefill(bool exact) {
+    exactPrefill_ = exact;
+    prepareChunks();
+  }
   [[nodiscard]] bool exactPrefill() const noexcept { return exactPrefill_; }
   // The hidden rows a draft's context is computed from (the reference's QwenTarget addCapture over RowCopy,
   // RowCopy.hpp:17-28): after layer layers[i] (ascending), every row's output goes to columns [i hidden, (i + 1) hidden)
@@ -197,6 +206,7 @@ private:
   // Chunks of at least kWideRows rows of a model at least kWideHidden wide take the wide kernels.
   static constexpr uint32_t kWideHidden = 2048, kWideRows = 65;
   [[nodiscard]] bool wideChunks() const noexcept;
+  [[nodiscard]] bool modelTakesWide() const;   // by its weights and exactPrefill_
   [[nodiscard]] bool takesWide(uint32_t tokens) const;
   void encodeWideChunkLayer(hip::CommandGraph &graph, uint32_t layer, const ops::AttentionPromptPlan &plan, uint32_t tokens);
   hip::Buffer chunkAttentionTable_;  // a long chunk's attention rows as the output projection's tables, every window's

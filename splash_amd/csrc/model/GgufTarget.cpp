@@ -163,6 +163,7 @@ void loadGgufDenseWeights(hip::Backend &backend, const GgufFile &file, DenseVeri
   for (const GgufTensor &t : file.tensors())
     if (!load.read.count(t.name)) problems.add(t.name + " is not read by the dense driver");
   if (!problems.text.empty()) throw GgufError("GGUF tensors this build cannot load: " + problems.text);
+  verify.prepareChunks();
 }
 
 namespace {
@@ -437,6 +438,7 @@ void loadGgufHybridWeights(hip::Backend &backend, const GgufFile &file, HybridVe
     if (!load.read.count(t.name) && !inLaterBlocks(t.name, d.layers)) problems.add(t.name + " is not read by the hybrid driver");
   if (!problems.text.empty()) throw GgufError("GGUF tensors this build cannot load: " + problems.text);
   verify.setTiledGdnHeads(true);
+  verify.prepareChunks();
 }
 
 } // namespace splash::model

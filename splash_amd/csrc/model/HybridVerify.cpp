@@ -116,26 +116,6 @@ HybridVerify::HybridVerify(hip::Backend &backend, HybridDimensions d, uint32_t m
   sampling_.uniforms = uniforms_;
   sampling_.inputTokens = inputTokens_;
   sampling_.treeRows = treeRows_;
-  if (wideChunks()) {
-    const uint32_t widest = std::max({d.hidden, d.attentionWidth(), d.gdnWidth(), d.dense() ? d.denseFfn : 0u});
-    wideTable_ = device(ops::Linear::wideTableBytes(widest, rowCapacity_), "wide table");
-    uint64_t partials = 0;
-    for (ops::LinearMatrix m : {ops::LinearMatrix{d.qkvWidth(), d.hidden}, ops::LinearMatrix{d.gdnPackedWidth, d.hidden}, ops::LinearMatrix{d.hidden, d.attentionWidth()},
-                                ops::LinearMatrix{d.hidden, d.gdnWidth()},
-                                d.dense() ? ops::LinearMatrix{d.hidden, d.denseFfn} : ops::LinearMatrix{d.experts, d.hidden}})
-      partials = std::max(partials, linear_.widePartialBytes(m, rowCapacity_));
-    widePartials_ = device(partials, "wide partials");
-    if (d.dense()) {
-      wideRows_ = device(C * d.denseFfn * 2, "chunk SwiGLU rows");
-    } else {
-      wideScores_ = device(C * d.experts * 4, "chunk router scores");
-      const ops::MoeChunkWorkspaceSize chunk = ops::MoE::chunkWorkspace(d.moeShape(), rowCapacity_);
-      moeChunk_ = {device(chunk.selected, "moe chunk selected"), device(chunk.weights, "moe chunk weights"), device(chunk.routeSlot, "moe chunk route slots"),
-                   device(chunk.slotRow, "moe chunk slot rows"), device(chunk.counts, "moe chunk counts"), device(chunk.tasks, "moe chunk tasks"),
-                   device(chunk.totals, "moe chunk totals"), device(chunk.table, "moe chunk tables"), device(chunk.intermediate, "moe chunk SwiGLU rows"),
-                   device(chunk.expertOutput, "moe chunk expert outputs")};
-    }
-  }
   // The rows a Gated DeltaNet layer's prefill passes hand each other, for the longest chunk.
   const uint64_t keyWidth = uint64_t{d.gdnKeyHeads} * GDN_HEAD_DIMENSION;
   gdnPrefill_.queries = device(C * keyWidth * 2, "GDN prefill queries");
@@ -150,8 +130,9 @@ HybridVerify::HybridVerify(hip::Backend &backend, HybridDimensions d, uint32_t m
 bool HybridVerify::wideChunks() const noexcept {
   return rowCapacity_ >= kWideRows && dims_.hidden >= kWideHidden && dims_.hidden <= ops::Linear::kMaximumWideNormWidth;
 }
-bool HybridVerify::takesWide(uint32_t tokens) const {
-  if (exactPrefill_ || !wideChunks() || tokens < kWideRows) return false;
+bool HybridVerify::takesWide(uint32_t tokens) const { return tokens >= kWideRows && modelTakesWide(); }
+bool HybridVerify::modelTakesWide() const {
+  if (exactPrefill_ || !wideChunks()) return false;
   for (const HybridLayer &l : weights_.layers) {
     if (!ops::Linear::takesWide(l.mixerInput) || !ops::Linear::takesWide(l.mixerOutput) || l.gateRows) return false;
     if (dims_.dense()) {
@@ -163,6 +144,32 @@ bool HybridVerify::takesWide(uint32_t tokens) const {
     }
   }
   return true;
+}
+
+void HybridVerify::prepareChunks() {
+  if (wideTable_ || !modelTakesWide()) return;
+  const HybridDimensions &d = dims_;
+  auto device = [&](uint64_t bytes, const char *label) { return backend_.allocateBuffer(std::max<uint64_t>(bytes, 16), BufferStorage::Private, label); };
+  const uint64_t C = rowCapacity_;
+  uint64_t partials = 0;
+  for (ops::LinearMatrix m : {ops::LinearMatrix{d.qkvWidth(), d.hidden}, ops::LinearMatrix{d.gdnPackedWidth, d.hidden}, ops::LinearMatrix{d.hidden, d.attentionWidth()},
+                              ops::LinearMatrix{d.hidden, d.gdnWidth()},
+                              d.dense() ? ops::LinearMatrix{d.hidden, d.denseFfn} : ops::LinearMatrix{d.experts, d.hidden}})
+    partials = std::max(partials, linear_.widePartialBytes(m, rowCapacity_));
+  widePartials_ = device(partials, "wide partials");
+  if (d.dense()) {
+    wideRows_ = device(C * d.denseFfn * 2, "chunk SwiGLU rows");
+  } else {
+    wideScores_ = device(C * d.experts * 4, "chunk router scores");
+    const ops::MoeChunkWorkspaceSize chunk = ops::MoE::chunkWorkspace(d.moeShape(), rowCapacity_);
+    moeChunk_ = {device(chunk.selected, "moe chunk selected"), device(chunk.weights, "moe chunk weights"), device(chunk.routeSlot, "moe chunk route slots"),
+                 device(chunk.slotRow, "moe chunk slot rows"), device(chunk.counts, "moe chunk counts"), device(chunk.tasks, "moe chunk tasks"),
+                 device(chunk.totals, "moe chunk totals"), device(chunk.table, "moe chunk tables"), device(chunk.intermediate, "moe chunk SwiGLU rows"),
+                 device(chunk.expertOutput, "moe chunk expert outputs")};
+  }
+  // last: what says that the others are there
+  const uint32_t widest = std::max({d.hidden, d.attentionWidth(), d.gdnWidth(), d.dense() ? d.denseFfn : 0u});
+  wideTable_ = device(ops::Linear::wideTableBytes(widest, rowCapacity_), "wide table");
 }
 
 const hip::Buffer &HybridVerify::draftProbabilities() {
@@ -529,6 +536,7 @@ void HybridVerify::encodePrefill(hip::CommandGraph &graph, uint32_t lane, uint32
   if (firstLayer >= dims_.layers || layerCount > dims_.layers - firstLayer) throw std::invalid_argument("no such layers");
   const ops::AttentionGeometry geometry{dims_.qHeads, dims_.kvHeads, dims_.headDimension, dims_.rotaryPairs, dims_.normalizeHeads, dims_.gatedAttention};
   const bool wide = takesWide(tokens);
+  if (wide) prepareChunks();
   ops::AttentionChunkPlan plan;
   ops::AttentionPromptPlan widePlan;
   if (wide) widePlan = ops::PagedAttention::planPrompt(geometry, {0, tokens, committed, tableFirst}, linear_.calibration().computeUnits);

@@ -112,6 +112,8 @@ public:
 
   [[nodiscard]] const HybridDimensions &dimensions() const noexcept { return dims_; }
   HybridWeights &weights() noexcept { return weights_; }
+  // As DenseVerify::prepareChunks: a table, router scores, the experts' slot rows and partial sums.
+  void prepareChunks();
   [[nodiscard]] const hip::Buffer &inputTokens() const noexcept { return inputTokens_; }
   [[nodiscard]] const hip::Buffer &treeRows() const noexcept { return treeRows_; }
   [[nodiscard]] const hip::Buffer &depths() const noexcept { return depths_; }
@@ -191,7 +193,10 @@ public:
                      uint32_t firstLayer = 0, uint32_t layerCount = 0);
   // As DenseVerify::setExactPrefill: the chunks encoded after run in windows, whose rows do not depend on how the prompt is
   // cut. Off by default.
-  void setExactPrefill(bool exact) noexcept { exactPrefill_ = exact; }
+  void setExactPrefill(bool exact) {
+    exactPrefill_ = exact;
+    prepareChunks();
+  }
   [[nodiscard]] bool exactPrefill() const noexcept { return exactPrefill_; }
 
 private:
@@ -201,6 +206,7 @@ private:
   // one window of the step's kernels, which read every expert's weights once a window.
   static constexpr uint32_t kWideHidden = 2048, kWideRows = 257;
   [[nodiscard]] bool wideChunks() const noexcept;
+  [[nodiscard]] bool modelTakesWide() const;
   [[nodiscard]] bool takesWide(uint32_t tokens) const;
   void encodeWidePrefillLayer(hip::CommandGraph &graph, uint32_t layer, const ops::AttentionPromptPlan &plan, uint32_t tokens, uint64_t currentCell,
                               uint64_t nextCell);

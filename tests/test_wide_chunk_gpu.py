@@ -3,7 +3,7 @@
 import numpy as np
 import pytest
 
-from splash_amd import verify
+from splash_amd import ops, verify
 from tests import oracle as orc
 from tests.dense_reference import DenseModel
 
@@ -218,3 +218,33 @@ def test_a_staged_chunk_allocates_nothing(backend, hidden, tokens):
     graph = gpu.encode_prefill(0, 0, tokens)
     assert any(name.startswith("gguf_prefill") for name in graph.kernels())
     assert backend.memory_stats().allocated_bytes == held
+
+
+@pytest.mark.parametrize("values,exact", [(orc.FMT_Q4K, False), (orc.FMT_Q4K, True), (orc.FMT_Q6K, False)])
+def test_only_a_driver_that_takes_the_wide_kernels_holds_their_buffers(backend, values, exact):
+    """The wide kernels' table, SwiGLU rows and partials come with the last layer's weights, if all are tensors those kernels
+    take (not with values of another format than the queries and keys) and chunks are not exact; encoding allocates nothing."""
+    print(f"case wide memory values={values} exact={exact}", flush=True)
+    H, F, rows = 2048, 2304, 300
+    native = lambda n, k, fmt=orc.FMT_Q4K: (fmt, n, orc.make_native(fmt, n, k, n + k))
+    project = lambda segments, k: ops.Projection.from_native(backend, segments, k)
+    norm = lambda n: backend.from_array(orc.f32_to_bf16(np.ones(n, np.float32)))
+    layer = (project([native(2048, H), native(512, H), native(512, H, values)], H), project([native(H, 2048)], 2048), project([native(F, H)], H),
+             project([native(F, H)], H), project([native(H, F)], F), norm(H), norm(H), norm(128), norm(128))
+    embedding, head = backend.from_array(native(512, H)[2]), ops.Projection.from_native(backend, [native(512, H)], H, float32=True)
+    gpu = verify.DenseVerify(backend, H, 16, 4, 128, F, 512, 2, physical_pages=3, page_table_entries=2, prefill_rows=rows)
+    gpu.set_exact_prefill(exact)
+    held = lambda: backend.memory_stats().allocated_bytes
+    created = held()
+    gpu.set_layer(0, *layer)
+    assert held() == created
+    gpu.set_layer(1, *layer)
+    gpu.set_head(orc.FMT_Q4K, embedding, norm(H), head)
+    complete, wide = held(), values == orc.FMT_Q4K and not exact
+    assert complete - created > rows * F * 2 if wide else complete - created < 1 << 16
+    assert any("wide" in name for name in gpu.encode_prefill(0, 0, rows).kernels()) == wide
+    assert held() == complete
+    if exact:
+        gpu.set_exact_prefill(False)
+        switched = held()
+        assert switched > complete and any("wide" in name for name in gpu.encode_prefill(0, 0, rows).kernels()) and held() == switched
