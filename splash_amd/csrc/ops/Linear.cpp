@@ -442,6 +442,11 @@ uint64_t Linear::prefillTableBytes(uint32_t inputSize, uint32_t rows) noexcept {
 }
 
 namespace {
+// The staged rule's chunks are refused alike, whichever kernels take them.
+void requirePrefillSegments(const Projection &p) {
+  for (const QuantizedSegment &s : p.blocks().segments)
+    if (s.outputSize % 128 || s.columnOffset % 16) throw std::invalid_argument("a prefill projection's tensors hold whole 128-column workgroups");
+}
 hip::Buffer viewOf(const hip::Buffer &base, uint64_t offset, uint64_t length) {
   sp_buffer *raw = nullptr;
   hip::throwStatus(sp_buffer_view(base.handle(), offset, length, &raw));
@@ -454,8 +459,7 @@ void Linear::addPrefill(hip::CommandGraph &graph, const hip::Buffer &input, cons
   const uint32_t n = p.outputSize, k = p.inputSize;
   if (!rows || rows > kMaximumPrefillRows) throw std::invalid_argument("a prefill chunk takes 1 to 16384 rows");
   requireSegments(p, {n, k});
-  for (const QuantizedSegment &s : p.blocks().segments)
-    if (s.outputSize % 128 || s.columnOffset % 16) throw std::invalid_argument("a prefill projection's tensors hold whole 128-column workgroups");
+  requirePrefillSegments(p);
   const bool float32 = p.destination == FloatOutput::Float32;
   if (float32 && residual) throw std::invalid_argument("only a plain prefill projection writes fp32");
   requireBytes(input, uint64_t{rows} * k * 2, "projection input");
@@ -579,6 +583,7 @@ void Linear::addWide(hip::CommandGraph &graph, const Projection &p, const hip::B
   requireSegments(p, {n, k});
   if (!takesWide(p)) throw std::invalid_argument("the wide kernels take tensors of one K-quant format");
   requireBytes(table, gguf_wide_table_bytes(k, rows), "wide table");
+  if (staged) requirePrefillSegments(p);
   const bool float32 = p.destination == FloatOutput::Float32;
   if (float32 && residual) throw std::invalid_argument("only a plain projection writes fp32");
   requireBytes(output, uint64_t{rows} * n * (float32 ? 4 : 2), "projection output");
@@ -617,6 +622,10 @@ void Linear::addWideGateUp(hip::CommandGraph &graph, const Projection &gate, con
   if (!takesWide(gate) || !takesWide(up) || up.destination != FloatOutput::BFloat16 || gate.blocks().segments.size() != 1 || up.blocks().segments.size() != 1 ||
       gate.blocks().segments.front().formatId != up.blocks().segments.front().formatId)
     throw std::invalid_argument("a one-pass block gate/up takes single tensors of one format");
+  if (staged) {
+    requirePrefillSegments(gate);
+    requirePrefillSegments(up);
+  }
   requireBytes(table, gguf_wide_table_bytes(k, rows), "wide table");
   requireBytes(output, uint64_t{rows} * n * 2, "projection output");
   const uint32_t groups = (n + GGUF_WIDE_COLUMNS / 2 - 1) / (GGUF_WIDE_COLUMNS / 2);

@@ -248,3 +248,22 @@ def test_only_a_driver_that_takes_the_wide_kernels_holds_their_buffers(backend, 
         gpu.set_exact_prefill(False)
         switched = held()
         assert switched > complete and any("wide" in name for name in gpu.encode_prefill(0, 0, rows).kernels()) and held() == switched
+
+
+@pytest.mark.parametrize("tokens", [40, 100])
+def test_a_staged_chunk_refuses_ragged_tensors_whichever_kernels_take_it(backend, tokens):
+    """Tensors that end inside a 128-column workgroup: the prefill tile refuses them, and so does a chunk of the same driver
+    that is long enough for the wide kernels; without the staged rule both run."""
+    print(f"case staged ragged tokens={tokens}", flush=True)
+    H, F = 2048, 2304
+    native = lambda n, k: (orc.FMT_Q4K, n, orc.make_native(orc.FMT_Q4K, n, k, n + k))
+    project = lambda segments, k: ops.Projection.from_native(backend, segments, k)
+    norm = lambda n: backend.from_array(orc.f32_to_bf16(np.ones(n, np.float32)))
+    gpu = verify.DenseVerify(backend, H, 16, 4, 128, F, 512, 1, physical_pages=3, page_table_entries=2, prefill_rows=128)
+    gpu.set_layer(0, project([native(1040, H), native(1008, H), native(1024, H)], H), project([native(H, 2048)], 2048), project([native(F, H)], H),
+                  project([native(F, H)], H), project([native(H, F)], F), norm(H), norm(H), norm(128), norm(128))
+    gpu.set_head(orc.FMT_Q4K, backend.from_array(native(512, H)[2]), norm(H), ops.Projection.from_native(backend, [native(512, H)], H, float32=True))
+    assert len(gpu.encode_prefill(0, 0, tokens)) > 0
+    gpu.set_staged_prefill(True)
+    with pytest.raises(ValueError, match="128-column"):
+        gpu.encode_prefill(0, 0, tokens)
