@@ -354,8 +354,8 @@ void DenseVerify::setStagedPrefill(bool staged) {
 bool DenseVerify::wideChunks() const noexcept {
   return rowCapacity_ > maxRows_ && dims_.hidden >= kWideHidden && dims_.hidden <= ops::Linear::kMaximumWideNormWidth;
 }
-bool DenseVerify::takesWide(uint32_t tokens) const {
-  return tokens > maxRows_ && tokens >= kWideRows && modelTakesWide();
+bool DenseVerify::takesWide(uint32_t committed, uint32_t tokens) const {
+  return tokens > maxRows_ && tokens >= kWideRows && uint64_t{committed} + tokens <= ops::PagedAttention::kMaximumPromptTokens && modelTakesWide();
 }
 bool DenseVerify::modelTakesWide() const {
   if (exactPrefill_ || !wideChunks()) return false;
@@ -486,7 +486,7 @@ void DenseVerify::encodePrefill(hip::CommandGraph &graph, uint32_t tableFirst, u
   if (!tokens || tokens > rowCapacity_) throw std::invalid_argument("a prompt chunk takes 1 to the driver's most prefill rows");
   if (tokens > maxRows_) {
     const ops::AttentionGeometry geometry{dims_.qHeads, dims_.kvHeads, dims_.headDimension, dims_.rotaryPairs, dims_.normalizeHeads};
-    const bool wide = takesWide(tokens);
+    const bool wide = takesWide(committed, tokens);
     if (wide) prepareChunks();
     ops::AttentionChunkPlan plan;
     ops::AttentionPromptPlan widePlan;

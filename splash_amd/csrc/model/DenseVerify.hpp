@@ -207,7 +207,7 @@ private:
   static constexpr uint32_t kWideHidden = 2048, kWideRows = 65;
   [[nodiscard]] bool wideChunks() const noexcept;
   [[nodiscard]] bool modelTakesWide() const;   // by its weights and exactPrefill_
-  [[nodiscard]] bool takesWide(uint32_t tokens) const;
+  [[nodiscard]] bool takesWide(uint32_t committed, uint32_t tokens) const;
   void encodeWideChunkLayer(hip::CommandGraph &graph, uint32_t layer, const ops::AttentionPromptPlan &plan, uint32_t tokens);
   hip::Buffer chunkAttentionTable_;  // a long chunk's attention rows as the output projection's tables, every window's
   void encodeChunkLayer(hip::CommandGraph &graph, uint32_t layer, const ops::AttentionChunkPlan &plan, uint32_t tokens, bool first,

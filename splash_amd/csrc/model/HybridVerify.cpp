@@ -130,7 +130,9 @@ HybridVerify::HybridVerify(hip::Backend &backend, HybridDimensions d, uint32_t m
 bool HybridVerify::wideChunks() const noexcept {
   return rowCapacity_ >= kWideRows && dims_.hidden >= kWideHidden && dims_.hidden <= ops::Linear::kMaximumWideNormWidth;
 }
-bool HybridVerify::takesWide(uint32_t tokens) const { return tokens >= kWideRows && modelTakesWide(); }
+bool HybridVerify::takesWide(uint32_t committed, uint32_t tokens) const {
+  return tokens >= kWideRows && uint64_t{committed} + tokens <= ops::PagedAttention::kMaximumPromptTokens && modelTakesWide();
+}
 bool HybridVerify::modelTakesWide() const {
   if (exactPrefill_ || !wideChunks()) return false;
   for (const HybridLayer &l : weights_.layers) {
@@ -535,7 +537,7 @@ void HybridVerify::encodePrefill(hip::CommandGraph &graph, uint32_t lane, uint32
   if (lane >= maxLanes_) throw std::invalid_argument("no such lane");
   if (firstLayer >= dims_.layers || layerCount > dims_.layers - firstLayer) throw std::invalid_argument("no such layers");
   const ops::AttentionGeometry geometry{dims_.qHeads, dims_.kvHeads, dims_.headDimension, dims_.rotaryPairs, dims_.normalizeHeads, dims_.gatedAttention};
-  const bool wide = takesWide(tokens);
+  const bool wide = takesWide(committed, tokens);
   if (wide) prepareChunks();
   ops::AttentionChunkPlan plan;
   ops::AttentionPromptPlan widePlan;

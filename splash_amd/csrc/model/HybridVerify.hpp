@@ -207,7 +207,7 @@ private:
   static constexpr uint32_t kWideHidden = 2048, kWideRows = 257;
   [[nodiscard]] bool wideChunks() const noexcept;
   [[nodiscard]] bool modelTakesWide() const;
-  [[nodiscard]] bool takesWide(uint32_t tokens) const;
+  [[nodiscard]] bool takesWide(uint32_t committed, uint32_t tokens) const;
   void encodeWidePrefillLayer(hip::CommandGraph &graph, uint32_t layer, const ops::AttentionPromptPlan &plan, uint32_t tokens, uint64_t currentCell,
                               uint64_t nextCell);
   void addGdnPrefill(hip::CommandGraph &graph, const HybridLayer &layer, uint32_t index, uint32_t tokens, uint64_t currentCell, uint64_t nextCell);

@@ -177,6 +177,8 @@ public:
   static void addChunkAttention(hip::CommandGraph &graph, const AttentionChunkPlan &plan, const AttentionWorkspace &workspace,
                                 const hip::Buffer &treeRows, const KvPages &pages, const hip::Buffer &output,
                                 const hip::Buffer &outputTable = {}, const hip::Buffer &packed = {});
+  // The most tokens of a sequence whose blocks can attend whole histories (the steps of a split are 16 bits).
+  static constexpr uint64_t kMaximumPromptTokens = uint64_t{0xFFFF} * ATTENTION_STEP_TOKENS;
   [[nodiscard]] static AttentionPromptPlan planPrompt(const AttentionGeometry &geometry, const AttentionChunk &chunk, uint32_t computeUnits);
   static void addPromptProjection(hip::CommandGraph &graph, const AttentionPromptPlan &plan, const AttentionProjectionBuffers &buffers,
                                   const AttentionWorkspace &workspace, const KvPages &pages);

@@ -267,3 +267,19 @@ def test_a_staged_chunk_refuses_ragged_tensors_whichever_kernels_take_it(backend
     gpu.set_staged_prefill(True)
     with pytest.raises(ValueError, match="128-column"):
         gpu.encode_prefill(0, 0, tokens)
+
+
+def test_a_chunk_behind_millions_of_tokens_runs_in_windows(backend):
+    """A history of more steps than a split counts: the whole-history attention cannot take it, the chunked one does. (The
+    chunk is encoded, not run: its pages are named, not there.)"""
+    print("case long history", flush=True)
+    H, F, rows, limit = 2048, 256, 2048, 0xFFFF * 64
+    native = lambda n, k: (orc.FMT_Q4K, n, orc.make_native(orc.FMT_Q4K, n, k, n + k))
+    project = lambda segments, k: ops.Projection.from_native(backend, segments, k)
+    norm = lambda n: backend.from_array(orc.f32_to_bf16(np.ones(n, np.float32)))
+    gpu = verify.DenseVerify(backend, H, 16, 4, 128, F, 512, 1, physical_pages=2, page_table_entries=(limit >> 8) + 9, prefill_rows=rows)
+    gpu.set_layer(0, project([native(2048, H), native(512, H), native(512, H)], H), project([native(H, 2048)], 2048), project([native(F, H)], H),
+                  project([native(F, H)], H), project([native(H, F)], F), norm(H), norm(H), norm(128), norm(128))
+    gpu.set_head(orc.FMT_Q4K, backend.from_array(native(512, H)[2]), norm(H), ops.Projection.from_native(backend, [native(512, H)], H, float32=True))
+    for committed, wide in ((limit - rows, True), (limit - rows + 1, False)):
+        assert any("wide" in name for name in gpu.encode_prefill(0, committed, rows).kernels()) == wide
