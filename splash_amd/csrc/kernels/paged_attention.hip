@@ -113,7 +113,7 @@ __global__ __launch_bounds__(D) void attention_q8_qkv(const uint16_t *__restrict
     if (query) {
       const uint32_t kv = head / group, g = head % group;
       const size_t at = ((size_t(z) * p.kv_heads + kv) * group + g) * 16u + row;
-      if (p.int8_queries) reinterpret_cast<int8_t *>(queries)[at * D + tid] = 0;
+      if (!Chunk && p.int8_queries) reinterpret_cast<int8_t *>(queries)[at * D + tid] = 0;
       else queries[at * D + tid] = _Float16(0.f);
       if (tid == 0) qsums[at] = 0.f;
     }
@@ -145,7 +145,7 @@ __global__ __launch_bounds__(D) void attention_q8_qkv(const uint16_t *__restrict
   if (query) {
     const uint32_t kv = index / group, g = index % group;
     const size_t at = ((size_t(z) * p.kv_heads + kv) * group + g) * 16u + row;
-    if (p.int8_queries) {
+    if (!Chunk && p.int8_queries) {   // (a prompt chunk's queries are fp16: planPrompt refuses others)
       // common/int8_activations.h:22-28: code = clamp(rint(x (127 / m))), the quotient rounded first; scale = m / 127; a
       // head at or below 2^-100 codes as zeros with scale 0; one that is not finite takes a NaN scale. The codes lie
       // where the fp16 queries would, one byte a dimension, and the scale in the sums' slot.
@@ -244,10 +244,7 @@ __global__ __launch_bounds__(256) void attention_q8_qkv_rows(const uint16_t *__r
     if (row >= seq.rows) {
       if (query) {
 #pragma unroll
-        for (uint32_t e = 0; e < E; ++e) {
-          if (p.int8_queries) reinterpret_cast<int8_t *>(queries)[at * D + l + 64u * e] = 0;
-          else queries[at * D + l + 64u * e] = _Float16(0.f);
-        }
+        for (uint32_t e = 0; e < E; ++e) queries[at * D + l + 64u * e] = _Float16(0.f);
         if (l == 0) qsums[at] = 0.f;
       }
       continue;
@@ -277,23 +274,7 @@ __global__ __launch_bounds__(256) void attention_q8_qkv_rows(const uint16_t *__r
         }
       }
     }
-    float magnitude[E];
-#pragma unroll
-    for (uint32_t e = 0; e < E; ++e) magnitude[e] = fabsf(result[e]);
-    if (query && p.int8_queries) {
-      float wild[E];
-#pragma unroll
-      for (uint32_t e = 0; e < E; ++e) wild[e] = (__float_as_uint(result[e]) & 0x7F800000u) == 0x7F800000u ? 1.f : 0.f;
-      const float notFinite = maximumOf(wild), largest = maximumOf(magnitude);
-      const bool coded = largest > 0x1p-100f;
-      const float inverse = coded ? 127.0f / largest : 0.0f;
-#pragma unroll
-      for (uint32_t e = 0; e < E; ++e) {
-        const float code = fminf(fmaxf(rintf(result[e] * inverse), -127.0f), 127.0f);
-        reinterpret_cast<int8_t *>(queries)[at * D + l + 64u * e] = notFinite != 0.f ? int8_t(0) : int8_t(code);
-      }
-      if (l == 0) qsums[at] = notFinite != 0.f ? __builtin_bit_cast(float, 0x7FC00000u) : coded ? largest / 127.0f : 0.0f;
-    } else if (query) {
+    if (query) {
       float staged[E];
 #pragma unroll
       for (uint32_t e = 0; e < E; ++e) {
@@ -304,10 +285,13 @@ __global__ __launch_bounds__(256) void attention_q8_qkv_rows(const uint16_t *__r
       const float sum = sumOf(staged);
       if (l == 0) qsums[at] = sum;
     } else {
-      float valueMagnitude[E];
+      float keyMagnitude[E], valueMagnitude[E];
 #pragma unroll
-      for (uint32_t e = 0; e < E; ++e) valueMagnitude[e] = fabsf(value[j][e]);
-      const float keyMax = maximumOf(magnitude), valueMax = maximumOf(valueMagnitude);
+      for (uint32_t e = 0; e < E; ++e) {
+        keyMagnitude[e] = fabsf(result[e]);
+        valueMagnitude[e] = fabsf(value[j][e]);
+      }
+      const float keyMax = maximumOf(keyMagnitude), valueMax = maximumOf(valueMagnitude);
       const uint32_t slot = seq.committed + row, token = slot % ATTENTION_PAGE_TOKENS;
       uint8_t *page = page_of(pool, page_table, seq, p.page_bytes, slot / ATTENTION_PAGE_TOKENS);
 #pragma unroll
