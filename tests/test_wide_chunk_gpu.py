@@ -3,7 +3,7 @@
 import numpy as np
 import pytest
 
-from splash_amd import ops, verify
+from splash_amd import ops, synthetic, verify
 from tests import oracle as orc
 from tests.dense_reference import DenseModel
 
@@ -283,3 +283,125 @@ def test_a_chunk_behind_millions_of_tokens_runs_in_windows(backend):
     gpu.set_head(orc.FMT_Q4K, backend.from_array(native(512, H)[2]), norm(H), ops.Projection.from_native(backend, [native(512, H)], H, float32=True))
     for committed, wide in ((limit - rows, True), (limit - rows + 1, False)):
         assert any("wide" in name for name in gpu.encode_prefill(0, committed, rows).kernels()) == wide
+
+
+_stage_model = {}
+
+
+def stage_model(down):
+    """The model of the stage tests with its down projection in a format."""
+    H, F = 2048, 8448
+    if not _stage_model:
+        _stage_model["model"] = DenseModel(seed=61, hidden=H, q_heads=16, kv_heads=4, head_dim=128, ffn=F, vocabulary=512, layers=1, down_format=orc.FMT_Q6K)
+        _stage_model[orc.FMT_Q6K] = _stage_model["model"].layers[0]["down"]
+        _stage_model[orc.FMT_Q4K] = orc.quantize_rows(orc.FMT_Q4K, (np.random.default_rng(62).standard_normal((H, F), dtype=np.float32) * np.float32(0.02)))
+        # Q5_K blocks of model-like scales: Q4_K's, the fifth bits drawn and the minimum's scale doubled
+        drawn = np.random.default_rng(63)
+        four = synthetic.q4k_native(drawn, H, F).reshape(-1, 144)
+        four[:, 2:4] = (2 * four[:, 0:2].copy().view(np.float16)).view(np.uint8)
+        fifth = drawn.integers(0, 256, (four.shape[0], 32), dtype=np.uint8)
+        _stage_model[orc.FMT_Q5K] = np.ascontiguousarray(np.concatenate([four[:, :16], fifth, four[:, 16:]], axis=1)).ravel()
+    model = _stage_model["model"]
+    model.down_format, model.layers[0]["down"] = down, _stage_model[down]
+    return model
+
+
+@pytest.mark.parametrize("tokens,down,heights", [(100, orc.FMT_Q5K, ("_t4_g", "_t4_p")), (513, orc.FMT_Q6K, ("q4k_t6_g", "q6k_t7_p")),
+                                                 (1300, orc.FMT_Q4K, ("q4k_t8_g", "q4k_t6_p")), (1543, orc.FMT_Q5K, ("q4k_t6_a", "q4k_t7_g", "q5k_t7_p"))])
+def test_a_wide_chunks_stages_are_as_close_to_64_bits_as_the_steps(backend, tokens, down, heights):
+    """Chunks whose plans take every tile height, K whole and in parts, an FFN wider than a table pass holds in one sweep, and
+    (1543 rows) whole-history attention: each stage of the layer against 64-bit arithmetic on its own input rows, a row of
+    every tile and all of the last ones, no further from it than the exact chunk's, on the whole and at the worst row."""
+    print(f"case wide stages tokens={tokens} down={down}", flush=True)
+    model = stage_model(down)
+    d, w = model.dims, model.layers[0]
+    H, F, W = d["hidden"], d["ffn"], 24 * 128
+    rng = np.random.default_rng(tokens)
+    gpu = model.build_gpu(backend, max_lanes=1, context_tokens=[tokens + 300], prefill_rows=tokens)
+    model.seed_context(gpu, None, rng)
+    prompt = rng.integers(0, 512, tokens).astype(np.uint32)
+    picked = np.unique(np.concatenate([np.minimum(16 * np.arange((tokens + 15) // 16) + 7 * np.arange((tokens + 15) // 16) % 16, tokens - 1),
+                                       np.arange(max(0, tokens - 20), tokens)]))
+    wide64 = lambda bits: orc.bf16_to_f32(bits).astype(np.float64)
+    weights = {name: orc.dequant_rows(down if name == "down" else orc.FMT_Q4K, w[name], n, k).astype(np.float64)
+               for name, n, k in (("q", 2048, H), ("k", 512, H), ("v", 512, H), ("o", H, 2048), ("gate", F, H), ("up", F, H), ("down", H, F))}
+    norm64 = lambda x, weight: x / np.sqrt((x * x).mean(axis=1, keepdims=True) + 1e-6) * wide64(weight)
+    embedded = wide64(model.oracle_embedding(prompt))[picked]
+    distance = {}
+    for exact in (True, False):
+        gpu.set_exact_prefill(exact)
+        graph = gpu.encode_prefill(model.table_first[0], 250, tokens)
+        names = graph.kernels()
+        assert exact or all(any(name.startswith("gguf_wide_q") and height in name for name in names) for height in heights), names
+        assert exact or tokens < 1543 or any("attention_q8_whole" in name for name in names)
+        gpu.set_prefill_block(prompt)
+        backend.run(graph)
+        rows = lambda which, index, width: wide64(gpu.buffer(which, index).download(np.uint16, tokens * width).reshape(tokens, width)[picked])
+        qkv, attention, middle, out = rows(verify.QKV_ROWS, 0, W), rows(verify.ATTENTION_ROWS, 0, 2048), rows(verify.HIDDEN, 1, H), rows(verify.HIDDEN, 0, H)
+        n = norm64(embedded, w["input_norm"])
+        m = norm64(middle, w["post_norm"])
+        gate = m @ weights["gate"].T
+        want = {"q|k|v": (qkv, np.concatenate([n @ weights[part].T for part in "qkv"], axis=1)),
+                "output": (middle, embedded + attention @ weights["o"].T),
+                "FFN": (out, middle + (gate / (1 + np.exp(-gate)) * (m @ weights["up"].T)) @ weights["down"].T)}
+        for stage, (got, reference) in want.items():
+            far = ((got - reference) ** 2).mean(axis=1) / (reference ** 2).mean(axis=1)
+            distance[stage, exact] = np.sqrt(far.mean()), np.sqrt(far.max())
+    for stage in ("q|k|v", "output", "FFN"):
+        (a, worst_a), (b, worst_b) = distance[stage, True], distance[stage, False]
+        print(f"  {stage}: exact {a:.3e} (worst row {worst_a:.3e}), wide {b:.3e} ({worst_b:.3e})", flush=True)
+        # (an exact chunk rounds a norm's rows before their scale, a wide one after it: one rounding each, whose errors over
+        # these rows differ by the draw, 0.3 % on the whole in exact arithmetic and 10 % at the worst row)
+        assert b <= 1.03 * a and worst_b <= 1.5 * worst_a, stage
+
+
+@pytest.mark.parametrize("tokens,experts,q_heads,kv_heads", [(300, 80, 8, 2), (784, 0, 32, 8)])
+def test_a_wide_hybrid_chunk_layer_by_layer(backend, tokens, experts, q_heads, kv_heads):
+    """HybridVerify::encodeWidePrefillLayer against the oracle from the GPU's own layer input, every row: a mixture whose
+    routes take two windows, with a shared expert; gated attention over whole histories (784 rows of eight KV heads)."""
+    from tests.hybrid_reference import HybridModel
+    from tests.test_hybrid_step_gpu import close_bf16, sure_routes, ulps
+    print(f"case wide hybrid layers tokens={tokens} experts={experts}", flush=True)
+    H, V, committed = 2048, 512, 200
+    model = HybridModel(seed=67, hidden=H, vocabulary=V, layers=4, q_heads=q_heads, kv_heads=kv_heads, head_dim=128, gdn_key_heads=2, gdn_value_heads=4,
+                        experts=experts, top_k=8 if experts else 0, expert_ffn=256 if experts else 0, shared_slices=1 if experts else 0,
+                        shared_gate=bool(experts), gated_attention=True, dense_ffn=0 if experts else 512)
+    gpu = model.build_gpu(backend, max_lanes=1, pages_per_lane=4, prefill_rows=tokens)
+    rng = np.random.default_rng(tokens)
+    model.seed_context(rng)
+    model.seed_states(rng, lanes=1)
+    prompt = rng.integers(0, V, tokens).astype(np.uint32)
+    gpu.set_prefill_block(prompt)
+    hidden_of = lambda i=0: gpu.buffer(verify.HIDDEN, i).download(np.uint16, tokens * H).reshape(tokens, H)
+    before = model.oracle_embedding(prompt)
+    for layer in range(4):
+        g = gpu.mixer_index(layer)
+        if layer:
+            before = hidden_of()
+        if not model.attends(layer):
+            conv_in, state_in = model.read_cell(0, 0, g)
+        graph = gpu.encode_prefill(0, 0, committed, tokens, parity=0, first_layer=layer, layer_count=1)
+        names = graph.kernels()
+        assert any("gguf_wide_moe" in name for name in names) == bool(experts) and any("gguf_wide_q" in name for name in names)
+        assert any("attention_q8_whole" in name for name in names) == (model.attends(layer) and tokens == 784)
+        backend.run(graph)
+        packed = model.oracle_mixer_input(before, layer)
+        if model.attends(layer):
+            mixed = model.oracle_attention_chunk(packed, layer, 0, committed)
+        else:
+            w = model.layers[layer]
+            want = orc.gdn_prefill(model.gdn_shape, packed, w["conv_w"], w["a_scale"], w["dt_bias"], w["mixer_norm"], conv_in, state_in)
+            mixed = want["hidden"]
+            conv, state = model.read_cell(0, 1, g)
+            ok, detail = close_bf16(conv, want["conv_out"])
+            assert ok and (ulps(conv, want["conv_out"]) > 0).mean() < 0.01, (layer, detail)
+            assert np.abs(state - want["state_out"]).max() <= 2e-3 * np.abs(want["state_out"]).max(), layer
+        ok, detail = close_bf16(hidden_of(1), model.oracle_mixer_output(mixed, before, layer))
+        print(f"  layer {layer} mixer {detail}", flush=True)
+        assert ok, ("mixer", layer, detail)
+        scores, want = model.oracle_ffn(hidden_of(1), layer)
+        sure = sure_routes(scores, 8) if experts else np.ones(tokens, bool)
+        assert sure.mean() >= 0.9
+        ok, detail = close_bf16(hidden_of()[sure], want[sure])
+        print(f"  layer {layer} ffn {detail}, sure {sure.mean():.3f}", flush=True)
+        assert ok, ("ffn", layer, detail)
