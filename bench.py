@@ -729,8 +729,8 @@ def main():
                     help="instead of the verify step: a chunk of this many prompt tokens (up to 2048) of one sequence "
                          "through every layer, no head (DenseVerify.encode_prefill)")
     ap.add_argument("--staged-prefill", action="store_true",
-                    help="with --prompt-chunk above a step's rows: the chunk's projections through the prefill tile (the staged "
-                         "rule, as the reference's prompt chunks run) instead of windows of the step's kernels")
+                    help="with --prompt-chunk above a step's rows: the chunk's projections under the staged rule (as the "
+                         "reference's prompt chunks run), through the wide kernels or the prefill tile")
     ap.add_argument("--calibrate-traffic", action="store_true",
                     help="after the steps, run plain read and copy kernels of known size: the scale of the FETCH_SIZE / "
                          "WRITE_SIZE counters of a rocprofv3 --pmc run of this command")
@@ -783,7 +783,9 @@ def main():
         if args.staged_prefill:
             gpu.set_staged_prefill(True)
         gpu.set_prefill_block(rng.integers(0, w["vocabulary"], tokens).astype(np.uint32))
-        command = backend.record(gpu.encode_prefill(0, w["context"] - tokens, tokens))
+        chunk = gpu.encode_prefill(0, w["context"] - tokens, tokens)
+        wide = any(name.startswith("gguf_wide") for name in chunk.kernels())
+        command = backend.record(chunk)
         for _ in range(args.warmup):
             command.submit().wait()
         seconds = sum(command.submit().wait()[0] for _ in range(args.steps)) / args.steps
@@ -791,7 +793,8 @@ def main():
         print(json.dumps({"metric": "prompt chunk ms (every layer of the 27B shape, no head)", "value": round(seconds * 1e3, 4),
                           "unit": "ms", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup, "tokens": tokens,
                           "tokens_per_s": round(tokens / seconds, 1), "higher_is_better": False, "data": "synthetic",
-                          "projections": "prefill tile, staged rule" if args.staged_prefill else "the step's kernels, register rule",
+                          "projections": ("wide kernels" if wide else "prefill tile" if args.staged_prefill else "the step's kernels") +
+                                         (", staged rule" if args.staged_prefill else ", register rule"),
                           "config": {"workload": w["name"] if "name" in w else args.workload, "context_tokens": w["context"]}}), flush=True)
         return
     if args.penalties:

@@ -6,14 +6,15 @@
 // sc * code is at most 63 * 31 and exact, so a whole super-block of 256 inputs accumulates in the matrix cores and costs
 // an output one multiply-add by d, and the constant term one more MFMA against the rows' group sums and one by dmin. A
 // Q6_K product needs twelve bits: it is the rounded fp16 product plus the exact fp16 remainder, two MFMAs. The rows
-// enter as fp16 too, scaled by a power of two a row (the wide table), which keeps all eight bits of a bf16 value.
+// enter as fp16 too, scaled by a power of two a row (the wide table), which keeps all eight bits of a bf16 value down to
+// 2^-28 of its row's largest. The fp32 sums of 768 inputs lie 4 to 12 times closer to 64-bit ones than the decode kernels'.
 //
 // Split: a wave owns 32 columns (a record of two column tiles each super-block, dequantized once in its registers) of
 // all of the workgroup's 128 rows, whose operands pass through LDS two groups at a time, double-buffered, one barrier
 // each. Two waves a SIMD (256 registers) overlap the conversion of one with the MFMAs of the other. At 2048 rows of the
-// 5120 x 2 x 25600 Q4_K gate/up pair a launch takes 1.35 ms (800 TFLOP/s of the projection's own operations; the 64-row
-// windows of the decode kernels took 2.38 ms), at 25600 x 5120 Q6_K 0.99 ms (2.2 ms): the matrix cores are busy 46 % and
-// 59 % of the cycles of a clock that the card's power limit holds at 2.1 and 1.8 GHz.
+// 5120 x 2 x 25600 Q4_K gate/up pair a launch takes 1.25 ms (860 TFLOP/s of the projection's own operations; the 64-row
+// windows of the decode kernels took 2.38 ms), at 25600 x 5120 Q6_K 0.96 ms (2.2 ms): the matrix cores are busy 47 % and
+// 56 % of the cycles of a clock that the card's power limit holds at 2.0 and 1.9 GHz.
 #include "abi/Gguf.h"
 #include "abi/Moe.h"
 #include "backend/KernelRegistry.hpp"

@@ -160,8 +160,8 @@ SP_REGISTER_KERNEL("norm_rms_table16", &norm_rms_table16);
 // activation table; a Residual stage's rows, their RMS norm (of `norm_weight`, into `normalized`) and its table. Each
 // convolution was a launch of its own before a launch of as few workgroups. Values and their order are the two kernels'.
 // The rows' 16-byte accesses are the host's rule (DraftAttention::addConvolutionTable). 8 rows of 5120: 5.3 us
-// for 3.1 + 3.0, 8.8 us for 3.1 + 8.7, and a launch less each: the draft model's pass of one lane 930 -> 888 us
-// in three runs, 908 -> 904 in another.
+// for 3.1 + 3.0, 8.9 us for 3.1 + 8.7, and a launch less each: the draft model's pass of one lane 928, 923 and 938 us
+// before, 869, 888 and 889 after, in three runs of both sides in turn whose repeats differ by 1 to 2 %.
 template <bool Residual>
 __global__ __launch_bounds__(256) void draft_conv_table(const uint16_t *__restrict__ input, const uint16_t *__restrict__ dynamic,
                                                         const uint16_t *__restrict__ base, const uint16_t *__restrict__ residual,

@@ -66,7 +66,7 @@ template <int N> __device__ __forceinline__ float block_max(float v, float *scra
 }
 
 // Block z of a dispatch. A prompt chunk's kernels (Chunk) work it out from the chunk's one sequence; a step's read its
-// sequence at once: the test of chunk_rows was one more wait in each of the layer's three short kernels, 1 % of a step.
+// sequence at once, without a test of chunk_rows before it.
 template <bool Chunk> __device__ __forceinline__ AttentionSequence block_sequence(const AttentionParams &p, uint32_t z) {
   if constexpr (Chunk) return attention_sequence(p, z);
   else return p.sequence[z];
@@ -183,7 +183,7 @@ SP_REGISTER_KERNEL("attention_q8_qkv_chunk_d64", (&attention_q8_qkv<64, true>));
 // wavefront four of its rows with their loads in flight together and lane l elements l and l + 64 of each. No barrier, and
 // sums and maxima in attention_q8_qkv's order (each 64 elements by a wavefront, then the halves), so every byte is the same.
 // A workgroup a row is bound by how fast workgroups start (147456 of them for 2048 rows of 64 / 8 heads): 114 us there, 45 at
-// 777 rows, against 80 and 34 here. Four rows one after the other take 14.5 us however few the blocks are, 5 us a row each.
+// 777 rows, against 76 and 36 here. Four rows one after the other take 14.5 us however few the blocks are.
 template <int D>
 __global__ __launch_bounds__(256) void attention_q8_qkv_rows(const uint16_t *__restrict__ qkv, const uint16_t *__restrict__ q_norm,
                                                             const uint16_t *__restrict__ k_norm, const float *__restrict__ rope_cos,

@@ -203,7 +203,9 @@ private:
   hip::Buffer prefillTable_, gateRows_, upRows_, swigluRows_;  // the prefill tile's tables and SwiGLU rows
   hip::Buffer wideTable_, wideRows_, widePartials_;             // the wide kernels' table, SwiGLU rows and parts' sums
   void encodeStagedChunkLayer(hip::CommandGraph &graph, uint32_t layer, const ops::AttentionChunkPlan &plan, uint32_t tokens);
-  // Chunks of at least kWideRows rows of a model at least kWideHidden wide take the wide kernels.
+  // Chunks of at least kWideRows rows of a model at least kWideHidden wide take the wide kernels: more rows than one pass
+  // of the step's widest tile. A layer of the 27B shape behind 8192 tokens, windows against wide: 48 rows 246 / 261 us, 64
+  // 267 / 267, 65 396 / 318, 128 460 / 352, 256 859 / 570, 512 1735 / 1003; behind none 64 rows 232 / 242, 65 353 / 272.
   static constexpr uint32_t kWideHidden = 2048, kWideRows = 65;
   [[nodiscard]] bool wideChunks() const noexcept;
   [[nodiscard]] bool modelTakesWide() const;   // by its weights and exactPrefill_

@@ -278,7 +278,10 @@ AttentionPromptPlan PagedAttention::planPrompt(const AttentionGeometry &geometry
   plan.geometry_ = geometry;
   plan.chunk_ = chunk;
   // A compute unit holds two workgroups. A chunk whose blocks alone give three quarters of the device's places work takes
-  // whole histories; a shorter one splits them into about as many parts as fill the places, at least four steps each.
+  // whole histories; a shorter one splits them into about as many parts as fill the places, at least four steps each. Of
+  // 64 / 8 heads behind 8192 tokens, whole against split: 8 blocks 253 / 83 us, 16 253 / 126, 32 260 / 226, 40 322 / 353,
+  // 48 328 / 367, 64 358 / 434. (The line is late from 36 blocks on, and for short histories: 40 blocks of none take 40
+  // whole and 87 in two parts.)
   const uint64_t steps = (uint64_t{chunk.committed} + chunk.tokens + ATTENTION_STEP_TOKENS - 1) / ATTENTION_STEP_TOKENS;
   const uint32_t items = plan.blocks() * geometry.kvHeads, places = 2 * computeUnits;
   uint64_t splits = 1;
@@ -319,7 +322,8 @@ void PagedAttention::addPromptProjection(hip::CommandGraph &graph, const Attenti
   requireBytes(w.querySums, need.querySums, "staged query sums");
   requirePromptPages(plan, params, pages);
   const hip::Buffer &spare = b.qkv;
-  // From about 25 blocks on a workgroup a block is faster than one a row (14.5 us + 0.5 a block against 4 + 0.85).
+  // A workgroup a block is the faster of the two from about 20 blocks on, and beyond the noise from here: of 64 / 8 heads
+  // 31 against 33 us at 32 blocks, 46 against 58 at 64 (24.3 against 24.0 at 16).
   const bool blocks = plan.blocks() >= 32;
   const hip::DispatchSize grid = blocks ? hip::DispatchSize{g.qHeads + g.kvHeads, plan.blocks(), 1}
                                     : hip::DispatchSize{g.qHeads + g.kvHeads, ATTENTION_MAXIMUM_ROWS, plan.blocks()};
