@@ -351,13 +351,14 @@ def test_a_chunks_blocks_attend_whole_histories(backend, geometry, tokens, commi
     want = np.concatenate(want)
     if gated:
         want = want / (1 + np.exp(-orc.bf16_to_f32(heads[:, :, 1]).astype(np.float64)))
-    error = {}
+    error, rows_of_label = {}, {}
 
     def check(label, out):
         got = out.download(np.uint16).reshape(tokens, q_heads, D)
         cos, err = tolerance(got, want)
         assert cos >= 0.9999 and err < 0.02, (label, cos, err)
         error[label] = float(np.sqrt(((orc.bf16_to_f32(got) - want) ** 2).mean()))
+        rows_of_label[label] = got
         for a, b in zip(kv.unpack_pages(kv.download()), (kc, ks, vc, vs)):
             assert np.array_equal(a[table], b[table]), label
     plan = ops.AttentionChunkPlan(q_heads, kv_heads, D, [(0, tokens, committed, 0)], rotary_pairs=pairs, normalize=True, gated=gated)
@@ -393,3 +394,4 @@ def test_a_chunks_blocks_attend_whole_histories(backend, geometry, tokens, commi
         check(f"{prepare} {p.splits}", out)
     print("  rms error: " + ", ".join(f"{k} {v:.3e}" for k, v in error.items()), flush=True)
     assert all(v <= 1.01 * error["chunked"] for v in error.values())
+    assert np.array_equal(rows_of_label["rows 1"], rows_of_label["chunk 1"])      # the two prepare kernels stage the same bytes
