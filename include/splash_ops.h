@@ -702,7 +702,8 @@ sp_status spo_dense_verify_set_capture(spo_dense_verify *verify, const uint32_t 
 /* The step's buffers; each call returns a new reference (release it). `index` is the layer for KV pools and the
    stream (0 or 1) for the hidden rows. The last three hold what the layer that ran last left in them: its fused
    q|k|v rows before the head norms, its attention rows before the output projection, its SwiGLU rows before the
-   down projection (what a layer-by-layer check of the step reads). */
+   down projection (what a layer-by-layer check of the step reads; of a prompt chunk longer than a step the first two hold
+   every row, the SwiGLU rows are the last window's, or another chunk's where none ran in windows). */
 typedef enum spo_verify_buffer {
   SPO_VERIFY_INPUT_TOKENS = 0, SPO_VERIFY_TREE_ROWS, SPO_VERIFY_DEPTHS, SPO_VERIFY_UNIFORMS, SPO_VERIFY_TOKENS,
   SPO_VERIFY_RETAINED, SPO_VERIFY_ACCEPTED, SPO_VERIFY_RETAINED_ROWS, SPO_VERIFY_PAGE_TABLE, SPO_VERIFY_KV_POOL,
