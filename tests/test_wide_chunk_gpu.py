@@ -405,3 +405,17 @@ def test_a_wide_hybrid_chunk_layer_by_layer(backend, tokens, experts, q_heads, k
         ok, detail = close_bf16(hidden_of()[sure], want[sure])
         print(f"  layer {layer} ffn {detail}, sure {sure.mean():.3f}", flush=True)
         assert ok, ("ffn", layer, detail)
+
+
+@pytest.mark.parametrize("experts", [16, 0])
+def test_encoding_a_wide_hybrid_chunk_allocates_nothing(backend, experts):
+    """The hybrid driver's wide buffers come with the last layer's weights (HybridVerify::prepareChunks)."""
+    from tests.hybrid_reference import HybridModel
+    print(f"case wide hybrid memory experts={experts}", flush=True)
+    model = HybridModel(seed=71, hidden=2048, vocabulary=512, layers=4, q_heads=8, kv_heads=2, head_dim=128, gdn_key_heads=2, gdn_value_heads=4,
+                        experts=experts, top_k=2 if experts else 0, expert_ffn=256 if experts else 0, dense_ffn=0 if experts else 512)
+    gpu = model.build_gpu(backend, max_lanes=1, pages_per_lane=3, prefill_rows=300)
+    held = backend.memory_stats().allocated_bytes
+    for rows, wide in ((256, False), (300, True)):
+        assert any("wide" in name for name in gpu.encode_prefill(0, 0, 0, rows).kernels()) == wide
+        assert backend.memory_stats().allocated_bytes == held
