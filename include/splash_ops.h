@@ -344,6 +344,13 @@ typedef struct spo_gdn_prefill_capture { /* ops::GdnPrefillCapture (GDN.hpp:95-1
 sp_status spo_gdn_add_prefill(spo_graph *graph, const spo_gdn_prefill_buffers *buffers, const spo_gdn_shape *shape, uint32_t layer,
                               uint32_t tokens, const spo_gdn_state_strides *state, uint32_t tiled_heads,
                               const spo_gdn_prefill_capture *captures, uint32_t count);
+/* The same with the scan in blocks of sixteen tokens on the matrix cores, whose terms pass through `blocks`
+ * (spo_gdn_prefill_blocks_bytes of the chunk's rows): the cells hold the accepted blocks' to fp32 rounding, not bit for bit.
+ * A chunk's row buffers stay under 2 GiB each. */
+uint64_t spo_gdn_prefill_blocks_bytes(const spo_gdn_shape *shape, uint32_t tokens);
+sp_status spo_gdn_add_prefill_blocks(spo_graph *graph, const spo_gdn_prefill_buffers *buffers, sp_buffer *blocks, const spo_gdn_shape *shape,
+                                     uint32_t layer, uint32_t tokens, const spo_gdn_state_strides *state, uint32_t tiled_heads,
+                                     const spo_gdn_prefill_capture *captures, uint32_t count);
 
 /* ---- StateCodec (runtime/ops/StateCodec.hpp:11-49; runtime/metal/abi/StateCodec.h): the cached form of the
  *      recurrent layers, int8 codes row by row and then a bf16 scale per block of 32 values ---- */

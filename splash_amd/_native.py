@@ -307,6 +307,8 @@ _sig("spo_float_projection_add", c_int, c_p, c_p, c_p, c_u32, c_u32, c_u32, c_p,
 _sig("spo_gdn_layout", c_int, P(GdnShape), c_u32, P(GdnStateStrides), P(c_u64), P(c_u64))
 _sig("spo_gdn_add_decode", c_int, c_p, P(GdnDecodeBuffers), P(GdnShape), c_u32, P(GdnStateStrides), c_u32, P(GdnLane), c_u32)
 _sig("spo_gdn_add_prefill", c_int, c_p, P(GdnPrefillBuffers), P(GdnShape), c_u32, c_u32, P(GdnStateStrides), c_u32, P(GdnPrefillCapture), c_u32)
+_sig("spo_gdn_prefill_blocks_bytes", c_u64, P(GdnShape), c_u32)
+_sig("spo_gdn_add_prefill_blocks", c_int, c_p, P(GdnPrefillBuffers), c_p, P(GdnShape), c_u32, c_u32, P(GdnStateStrides), c_u32, P(GdnPrefillCapture), c_u32)
 _sig("spo_gdn_add_fold", c_int, c_p, c_p, c_p, c_p, c_u64, c_u64, c_u64, P(GdnShape), c_u32, c_u32, P(GdnStateStrides))
 _sig("spo_state_codec_layer_bytes", c_u64, c_u32, c_u32)
 for _name in ("spo_state_codec_add_quantize", "spo_state_codec_add_dequantize", "spo_state_codec_add_copy"):

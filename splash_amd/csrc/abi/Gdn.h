@@ -106,6 +106,19 @@ struct GdnFoldParams {
 // `next_cell`, another cell. No tape: a prompt's rows are never rolled back.
 #define GDN_SCAN_STATE_ROWS 16u   // state rows of one scan workgroup (the reference's SPLASH_GDN_SCAN_STATE_ROWS)
 #define GDN_SCAN_BLOCK 16u        // tokens a scan workgroup stages at a time
+// A run in blocks of GDN_SCAN_BLOCK tokens (gdn_prefill_blocks, gdn_prefill_block_scan): what a block needs that its rows and
+// gates alone decide. Per block and value head, fp32: T [16][16], the block's triangular system solved (its unknowns' right
+// sides weighed by their betas), A [16][16], the rows' decayed products with the queries, the decay from the block's start to
+// each row and from each row to the block's end. Then per block and key head the keys as operands of the state's update.
+#define GDN_BLOCK_TERMS 576u          // floats: T, A, the two decays, the betas, the betas times the first decays
+#define GDN_BLOCK_KEYS_BYTES 8192u
+GDN_INLINE uint64_t gdn_prefill_block_keys_offset(uint32_t tokens, uint32_t value_heads) {
+  return uint64_t((tokens + GDN_SCAN_BLOCK - 1u) / GDN_SCAN_BLOCK) * value_heads * (GDN_BLOCK_TERMS * 4u);
+}
+GDN_INLINE uint64_t gdn_prefill_blocks_bytes(uint32_t tokens, uint32_t key_heads, uint32_t value_heads) {
+  return gdn_prefill_block_keys_offset(tokens, value_heads) +
+         uint64_t((tokens + GDN_SCAN_BLOCK - 1u) / GDN_SCAN_BLOCK) * key_heads * GDN_BLOCK_KEYS_BYTES;
+}
 struct GdnPrefillParams {
   struct GdnShapeParams shape;
   uint32_t flags;

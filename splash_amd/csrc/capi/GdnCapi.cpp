@@ -21,6 +21,18 @@ ops::GdnShape shapeOf(const spo_gdn_shape &s) {
 ops::GdnStateStrides stridesOf(const spo_gdn_state_strides &s) {
   return {s.convolution_layer_bytes, s.recurrent_layer_bytes, s.convolution_state_bytes};
 }
+void addPrefill(spo_graph *graph, const spo_gdn_prefill_buffers *b, sp_buffer *blocks, const spo_gdn_shape *shape, uint32_t layer,
+                uint32_t tokens, const spo_gdn_state_strides *state, uint32_t tiled_heads, const spo_gdn_prefill_capture *captures, uint32_t count) {
+  capi::require(graph && b && shape && state && (captures || !count), "graph, buffers, shape, strides or captures");
+  ops::GdnPrefillBuffers buffers{B(b->packed), B(b->convolution_weights), B(b->states), B(b->decay_weights), B(b->time_bias),
+                                 B(b->mixer_norm), b->float_norm != 0, B(b->queries), B(b->keys), B(b->values), B(b->decay),
+                                 B(b->beta), B(b->recurrent_rows), B(b->hidden), b->current_cell, b->next_cell};
+  if (blocks) buffers.blocks = B(blocks);
+  std::vector<ops::GdnPrefillCapture> list;
+  for (uint32_t i = 0; i < count; ++i) list.push_back({captures[i].tokens, captures[i].cell});
+  ops::GDN::addPrefill(capi::graphOf(graph), buffers, shapeOf(*shape), layer, tokens, stridesOf(*state),
+                       tiled_heads ? ops::GdnHeadOrder::Tiled : ops::GdnHeadOrder::Grouped, list);
+}
 } // namespace
 
 extern "C" {
@@ -64,21 +76,23 @@ sp_status spo_gdn_add_fold(spo_graph *graph, sp_buffer *states, sp_buffer *tape,
   });
 }
 
+uint64_t spo_gdn_prefill_blocks_bytes(const spo_gdn_shape *shape, uint32_t tokens) {
+  return shape ? gdn_prefill_blocks_bytes(tokens, shape->key_heads, shape->value_heads) : 0;
+}
+
+sp_status spo_gdn_add_prefill_blocks(spo_graph *graph, const spo_gdn_prefill_buffers *b, sp_buffer *blocks, const spo_gdn_shape *shape,
+                                     uint32_t layer, uint32_t tokens, const spo_gdn_state_strides *state, uint32_t tiled_heads,
+                                     const spo_gdn_prefill_capture *captures, uint32_t count) {
+  return capi::guard([&] {
+    capi::require(blocks, "block terms");
+    addPrefill(graph, b, blocks, shape, layer, tokens, state, tiled_heads, captures, count);
+  });
+}
 sp_status spo_gdn_add_prefill(spo_graph *graph, const spo_gdn_prefill_buffers *b, const spo_gdn_shape *shape, uint32_t layer,
                               uint32_t tokens, const spo_gdn_state_strides *state, uint32_t tiled_heads,
                               const spo_gdn_prefill_capture *captures, uint32_t count) {
-  return capi::guard([&] {
-    capi::require(graph && b && shape && state && (captures || !count), "graph, buffers, shape, strides or captures");
-    ops::GdnPrefillBuffers buffers{B(b->packed), B(b->convolution_weights), B(b->states), B(b->decay_weights), B(b->time_bias),
-                                   B(b->mixer_norm), b->float_norm != 0, B(b->queries), B(b->keys), B(b->values), B(b->decay),
-                                   B(b->beta), B(b->recurrent_rows), B(b->hidden), b->current_cell, b->next_cell};
-    std::vector<ops::GdnPrefillCapture> list;
-    for (uint32_t i = 0; i < count; ++i) list.push_back({captures[i].tokens, captures[i].cell});
-    ops::GDN::addPrefill(capi::graphOf(graph), buffers, shapeOf(*shape), layer, tokens, stridesOf(*state),
-                         tiled_heads ? ops::GdnHeadOrder::Tiled : ops::GdnHeadOrder::Grouped, list);
-  });
+  return capi::guard([&] { addPrefill(graph, b, nullptr, shape, layer, tokens, state, tiled_heads, captures, count); });
 }
-
 uint64_t spo_state_codec_layer_bytes(uint32_t rows, uint32_t columns) { return state_codec_layer_bytes(rows, columns); }
 
 extern "C++" {

@@ -22,7 +22,7 @@
 #include "abi/Gguf.h"
 #include "abi/PagedAttention.h"  // AttentionTreeRow
 #include "backend/KernelRegistry.hpp"
-#include "kernels/device_common.hpp"
+#include "kernels/gguf_records.hpp"   // buffer resources
 
 namespace splash::kernels {
 
@@ -725,6 +725,361 @@ __global__ __launch_bounds__(256) void gdn_prefill_scan(const uint16_t *__restri
     *reinterpret_cast<float4 *>(stateOut + stateAt + 4u * h) = make_float4(state[h][0], state[h][1], state[h][2], state[h][3]);
 }
 SP_REGISTER_KERNEL("gdn_prefill_scan", &gdn_prefill_scan);
+
+// ---- prefill in blocks of sixteen tokens, on the matrix cores ----
+//
+// Within a block that starts from the state S, with g_t the decay from its start to row t and D_tj that from row j to row t,
+// the state after row t is g_t S + sum_{j <= t} D_tj u_j k_j', where the corrections u solve the triangular system
+//   u_t + beta_t sum_{j < t} D_tj (k_t . k_j) u_j = beta_t (v_t - g_t S k_t).
+// Its inverse (with the betas folded in, T) and the products A_tj = D_tj (q_t . k_j) of the outputs
+//   o_t = g_t S q_t + sum_{j <= t} A_tj u_j
+// depend on the block's rows alone: gdn_prefill_blocks works them out for every block at once, and what is left to do in
+// order, gdn_prefill_block_scan, is per block two products with the state, one with T and the state's update, all MFMAs.
+// A token is one dependent chain in gdn_prefill_scan (0.2 us each); here sixteen are: 2048 tokens of 16 / 32 heads 402 us there,
+// 13 + 93 us here (0.72 us a block). The sums' order differs from the fold's, so a chunk through these kernels leaves the accepted blocks' cell to rounding, not bit for bit.
+// Precision: keys and queries are bf16, as they are; the state and the corrections enter their products as three bf16 parts
+// each, which hold all 24 bits, and every sum is fp32. Against 64-bit arithmetic the state of 32 heads is off by 5.0e-8 of
+// its norm where the scan's is by 5.7e-8, and the rows by the same rounding to bf16 (tests/test_gdn_blocks_gpu.py). A row that is not finite makes the rows of its own block that lie
+// before it NaN too (the triangle's zeros multiply it), where the scan would have kept those finite.
+__device__ __forceinline__ uint32_t upper_halves(float low, float high) {
+  return __builtin_amdgcn_perm(__float_as_uint(high), __float_as_uint(low), 0x07060302u);
+}
+__device__ __forceinline__ float cut(float v) { return __uint_as_float(__float_as_uint(v) & 0xFFFF0000u); }
+// Two values as three pairs of bf16 whose sums they are (each part the eight leading bits of what is left).
+__device__ __forceinline__ void split3(float a, float b, uint32_t &high, uint32_t &middle, uint32_t &low) {
+  high = upper_halves(a, b);
+  const float a1 = a - cut(a), b1 = b - cut(b);
+  middle = upper_halves(a1, b1);
+  low = upper_halves(a1 - cut(a1), b1 - cut(b1));
+}
+
+// gdn_prefill_blocks: grid (value_heads, ceil(blocks / 4)), 256 threads, a wave per (block, value head). A run's last block
+// may be short: rows past it repeat the last one with a decay of 1 and a beta of 0, which makes their corrections zero.
+__global__ __launch_bounds__(256) void gdn_prefill_blocks(const uint16_t *__restrict__ queries, const uint16_t *__restrict__ keys,
+                                                          const float *__restrict__ decay, const uint16_t *__restrict__ beta,
+                                                          uint8_t *__restrict__ work, GdnPrefillParams p) {
+  constexpr uint32_t B = GDN_SCAN_BLOCK;
+  __shared__ __align__(16) uint16_t stagedKeys[4][B][kDim + 8];
+  __shared__ __align__(16) float system[4][B][B];
+  __shared__ __align__(16) float gates[4][2][B];
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, row = lane & 15u, kq = lane >> 4;
+  const GdnShapeParams s = p.shape;
+  const uint32_t head = blockIdx.x, block = blockIdx.y * 4u + wave, start = block * B;
+  const uint32_t perKey = s.value_heads / s.key_heads, keyHead = head / perKey, keyWidth = s.key_heads * kDim;
+  if (start >= p.tokens) return;   // (no barrier below: a wave's LDS is its own)
+  const uint32_t token = min(start + row, p.tokens - 1u);
+  const size_t at = (size_t(p.first) + token) * keyWidth + keyHead * kDim + 8u * kq;
+  uint4 key[4], query[4];
+#pragma unroll
+  for (uint32_t w = 0; w < 4; ++w) {
+    key[w] = *reinterpret_cast<const uint4 *>(keys + at + 32u * w);
+    query[w] = *reinterpret_cast<const uint4 *>(queries + at + 32u * w);
+  }
+  if (kq == 0) {
+    const size_t gate = (size_t(p.first) + token) * s.value_heads + head;
+    const bool live = start + row < p.tokens;
+    gates[wave][0][row] = live ? decay[gate] : 1.f;
+    gates[wave][1][row] = live ? bf16_bits_to_float(beta[gate]) : 0.f;
+  }
+  // rows t = 4 kq + i, columns j = row
+  f32x4 kk = {0.f, 0.f, 0.f, 0.f}, qk = kk;
+#pragma unroll
+  for (uint32_t w = 0; w < 4; ++w) {
+    kk = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(key[w]), as_bf16x8(key[w]), kk, 0, 0, 0);
+    qk = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(query[w]), as_bf16x8(key[w]), qk, 0, 0, 0);
+  }
+  wave_lds_fence();
+  float between[4], sinceStart[4], toEnd = 1.f, running = 1.f;
+#pragma unroll
+  for (uint32_t t = 0; t < B; ++t) {
+    const float d = gates[wave][0][t];
+    toEnd = t > row ? toEnd * d : 1.f;
+    running *= d;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i)
+      if (4u * kq + i == t) {
+        between[i] = toEnd;
+        sinceStart[i] = running;
+      }
+  }
+  float *terms = reinterpret_cast<float *>(work) + (size_t(block) * s.value_heads + head) * GDN_BLOCK_TERMS;
+#pragma unroll
+  for (uint32_t i = 0; i < 4; ++i) {
+    const uint32_t t = 4u * kq + i;
+    system[wave][t][row] = t > row ? gates[wave][1][t] * (between[i] * kk[i]) : 0.f;
+    terms[B * B + t * B + row] = t >= row ? between[i] * qk[i] : 0.f;
+    if (row == 0) {
+      terms[2 * B * B + t] = sinceStart[i];
+      terms[2 * B * B + 3 * B + t] = sinceStart[i] * gates[wave][1][t];
+    }
+  }
+  if (kq == 0) {
+    terms[2 * B * B + B + row] = toEnd;
+    terms[2 * B * B + 2 * B + row] = gates[wave][1][row];
+  }
+  wave_lds_fence();
+  // column j = row of the inverse, top down
+  float x[B];
+#pragma unroll
+  for (uint32_t t = 0; t < B; ++t) {
+    float sum = t == row ? 1.f : 0.f;
+#pragma unroll
+    for (uint32_t j = 0; j < t; ++j) sum = __fmaf_rn(-system[wave][t][j], x[j], sum);
+    x[t] = sum;
+    if (kq == t / 4u) terms[t * B + row] = t == row ? 0.f : sum;
+  }
+  if (head % perKey) return;
+  // The keys as the update's operands: lane (r, kq) of wave w's tile m holds tokens 4 kq .. + 3 of dimension
+  // 32 w + 8 (r / 4) + 4 m + r % 4, the dimension that row r of the tile's part of the state holds, twice over: the update
+  // multiplies them by the corrections' leading parts and by what is left of those.
+#pragma unroll
+  for (uint32_t w = 0; w < 4; ++w) *reinterpret_cast<uint4 *>(&stagedKeys[wave][row][32u * w + 8u * kq]) = key[w];
+  wave_lds_fence();
+  uint4 *out = reinterpret_cast<uint4 *>(work + gdn_prefill_block_keys_offset(p.tokens, s.value_heads) +
+                                         (size_t(block) * s.key_heads + keyHead) * GDN_BLOCK_KEYS_BYTES);
+#pragma unroll
+  for (uint32_t w = 0; w < 4; ++w) {
+#pragma unroll
+    for (uint32_t m = 0; m < 2; ++m) {
+      const uint32_t dimension = 32u * w + 8u * (row >> 2) + 4u * m + (row & 3u);
+      uint32_t words[2];
+#pragma unroll
+      for (uint32_t e = 0; e < 2; ++e)
+        words[e] = uint32_t(stagedKeys[wave][4u * kq + 2u * e][dimension]) | (uint32_t(stagedKeys[wave][4u * kq + 2u * e + 1u][dimension]) << 16);
+      out[w * 128u + m * 64u + lane] = make_uint4(words[0], words[1], words[0], words[1]);
+    }
+  }
+}
+SP_REGISTER_KERNEL("gdn_prefill_blocks", &gdn_prefill_blocks);
+
+// gdn_prefill_block_scan: grid (value_heads * 8), 320 threads. A workgroup carries sixteen rows (value dimensions) of a head's
+// state through the run's blocks. Four waves hold it, wave w the key dimensions 32 w .. + 31: lane (r, kq) row r's dimensions
+// 32 w + 8 kq .. + 7, which are both the result of the update and, cut in three, the operand of the next block's products, so
+// the state never moves between lanes. Their shares of S k and S q meet in LDS, one barrier a block; every wave then solves
+// for all sixteen rows' corrections (four fp32 MFMAs), the four update their columns and the fifth writes the outputs. What a
+// block needs from memory is in flight three blocks ahead (all of it issued at a block's end: 113 us, the compiler's own order:
+// 124; the outputs by the four waves in turn: 118). One workgroup a compute unit: the pass is the latency of a block's
+// chain. The workgroups of a head read the same keys and terms: head h's run on die h % 8 (workgroup b runs on die b % 8)
+// wherever the heads fill the dies.
+struct BlockTerms {
+  uint4 solve, started, weight;   // of rows `row` (solve), 4 kq .. + 3
+  uint32_t value[4];              // of token 4 kq + i, value dimensions rowBase + (row & ~1) and the next
+};
+__global__ __launch_bounds__(320, 1) void gdn_prefill_block_scan(const uint16_t *__restrict__ queries, const uint16_t *__restrict__ keys,
+                                                                 const uint16_t *__restrict__ values, const uint8_t *__restrict__ work,
+                                                                 uint8_t *__restrict__ states, uint16_t *__restrict__ recurrent_rows,
+                                                                 GdnPrefillParams p) {
+  constexpr uint32_t B = GDN_SCAN_BLOCK, kAhead = 4;
+  __shared__ __align__(16) float4 shares[2][2][4][64];   // [block parity][S k, S q][wave][lane]
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, row = lane & 15u, kq = lane >> 4;
+  const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(int(tid >> 6)));
+  const GdnShapeParams s = p.shape;
+  const uint32_t head = blockIdx.x % s.value_heads, rowBase = blockIdx.x / s.value_heads * 16u;
+  const uint32_t keyHead = head / (s.value_heads / s.key_heads), keyWidth = s.key_heads * kDim, valueWidth = s.value_heads * kDim;
+  const uint32_t blocks = (p.tokens + B - 1u) / B, rounds = (blocks + kAhead - 1u) / kAhead;
+  // Every stream through a buffer resource of the run's rows: rows past them, and blocks past the last, read as zeros (which
+  // correct nothing), and writes there go nowhere.
+  const uint32_t keyRow = keyWidth * 2u, valueRow = valueWidth * 2u, keysAt = uint32_t(gdn_prefill_block_keys_offset(p.tokens, s.value_heads));
+  const uint32_t termsBlock = s.value_heads * (GDN_BLOCK_TERMS * 4u), keysBlock = s.key_heads * GDN_BLOCK_KEYS_BYTES;
+  const Resource valueRows = make_resource(values + size_t(p.first) * valueWidth, p.tokens * valueRow);
+  const Resource terms = make_resource(work, blocks * termsBlock);
+  uint32_t valueAt[4];
+#pragma unroll
+  for (uint32_t i = 0; i < 4; ++i) valueAt[i] = (4u * kq + i) * valueRow + (head * kDim + rowBase + (row & ~1u)) * 2u;
+  uint32_t termAt = head * (GDN_BLOCK_TERMS * 4u) + (row * B + 4u * kq) * 4u, rowsAt = head * (GDN_BLOCK_TERMS * 4u) + 2u * B * B * 4u + 16u * kq;
+  auto fetchValues = [&](BlockTerms &f) __attribute__((always_inline)) {
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) f.value[i] = __builtin_amdgcn_raw_buffer_load_b32(valueRows, int(valueAt[i]), 0, 0);
+  };
+  auto fetchSolve = [&](BlockTerms &f) __attribute__((always_inline)) { f.solve = load128<0>(terms, termAt); };
+  auto fetchWeights = [&](BlockTerms &f) __attribute__((always_inline)) {
+    f.weight = load128<0>(terms, rowsAt + 2u * B * 4u);
+    f.started = load128<0>(terms, rowsAt + 3u * B * 4u);
+  };
+  auto advanceTerms = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) valueAt[i] += B * valueRow;
+    termAt += termsBlock;
+    rowsAt += termsBlock;
+  };
+  // A fetched word where it is used: what is computed from it, and with that the wait for it, stays there.
+  auto used = [](uint32_t v) __attribute__((always_inline)) {
+    asm volatile("" : "+v"(v));
+    return v;
+  };
+  auto floats = [](const uint4 &v) __attribute__((always_inline)) { return __builtin_bit_cast(f32x4, v); };
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  auto whole = [&](uint32_t parity, uint32_t which) __attribute__((always_inline)) {   // the waves' shares added
+    f32x4 part[4], sum;
+#pragma unroll
+    for (uint32_t w = 0; w < 4; ++w) part[w] = __builtin_bit_cast(f32x4, shares[parity][which][w][lane]);
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) sum[i] = (part[0][i] + part[1][i]) + (part[2][i] + part[3][i]);
+    return sum;
+  };
+  const uint32_t valueShift = row & 1u ? 0u : 16u;
+  // `between(i)` is issued behind the i-th product, each of which waits for the one before.
+  auto correctionsOf = [&](const BlockTerms &f, const f32x4 &memory, auto &&between) __attribute__((always_inline)) {
+    const f32x4 solve = floats(f.solve), started = floats(f.started), weight = floats(f.weight);
+    f32x4 own, sum = zero;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i)
+      own[i] = __fmaf_rn(-started[i], memory[i], weight[i] * __uint_as_float((used(f.value[i]) << valueShift) & 0xFFFF0000u));   // (the last product is exact)
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {   // token 4 kq + i in place kq
+      sum = __builtin_amdgcn_mfma_f32_16x16x4f32(solve[i], own[i], sum, 0, 0, 0);
+      between(i);
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) sum[i] += own[i];
+    return sum;
+  };
+  // (A block's shares are written over those of two blocks before, which every wave has read once it is past the barrier of
+  // the block between. Both kinds of wave below pass rounds * kAhead barriers.)
+  if (wave == 4u) {
+    const Resource outputRows = make_resource(recurrent_rows + size_t(p.first) * valueWidth, p.tokens * valueRow);
+    struct Fetched {
+      BlockTerms terms;
+      uint4 outputs, sinceStart;
+    };
+    uint32_t outputAt[4];
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) outputAt[i] = valueAt[i] + (row & 1u) * 2u;
+    auto fetch = [&](Fetched &f) __attribute__((always_inline)) {
+      fetchValues(f.terms);
+      fetchSolve(f.terms);
+      fetchWeights(f.terms);
+      f.sinceStart = load128<0>(terms, rowsAt);
+      f.outputs = load128<0>(terms, termAt + B * B * 4u);
+      advanceTerms();
+    };
+    auto run = [&](uint32_t parity, const Fetched &f) __attribute__((always_inline)) {
+      __syncthreads();
+      const f32x4 memory = whole(parity, 0);
+      f32x4 out = whole(parity, 1);
+      const f32x4 corrections = correctionsOf(f.terms, memory, [](uint32_t) {}), sinceStart = floats(f.sinceStart), outputs = floats(f.outputs);
+#pragma unroll
+      for (uint32_t i = 0; i < 4; ++i) out[i] *= sinceStart[i];
+#pragma unroll
+      for (uint32_t i = 0; i < 4; ++i) out = __builtin_amdgcn_mfma_f32_16x16x4f32(outputs[i], corrections[i], out, 0, 0, 0);
+#pragma unroll
+      for (uint32_t i = 0; i < 4; ++i) {
+        __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, static_cast<__bf16>(out[i])), outputRows, int(outputAt[i]), 0, 0);
+        outputAt[i] += B * valueRow;
+      }
+    };
+    Fetched ahead[kAhead];
+#pragma unroll
+    for (uint32_t a = 0; a < kAhead; ++a) {
+      fetch(ahead[a]);
+      __builtin_amdgcn_sched_barrier(0);   // (in the order the loop waits for them)
+    }
+    for (uint32_t round = 0, parity = 0; round < rounds; ++round) {
+#pragma unroll
+      for (uint32_t a = 0; a < kAhead; ++a, parity ^= 1u) {
+        run(parity, ahead[a]);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(ahead[a]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    return;
+  }
+  const float *stateIn = reinterpret_cast<const float *>(states + p.current_cell + p.convolution_state_bytes + uint64_t(p.layer) * p.recurrent_layer_bytes);
+  float *stateOut = reinterpret_cast<float *>(states + p.next_cell + p.convolution_state_bytes + uint64_t(p.layer) * p.recurrent_layer_bytes);
+  const size_t stateAt = (size_t(head) * kDim + rowBase + row) * kDim + 32u * wave + 8u * kq;
+  f32x4 state[2];
+#pragma unroll
+  for (uint32_t m = 0; m < 2; ++m) state[m] = *reinterpret_cast<const f32x4 *>(stateIn + stateAt + 4u * m);
+  const Resource keyRows = make_resource(keys + size_t(p.first) * keyWidth, p.tokens * keyRow);
+  const Resource queryRows = make_resource(queries + size_t(p.first) * keyWidth, p.tokens * keyRow);
+  const Resource operands = make_resource(work + keysAt, blocks * keysBlock);
+  uint32_t keyAt = row * keyRow + (keyHead * kDim + 32u * wave + 8u * kq) * 2u, operandAt = keyHead * GDN_BLOCK_KEYS_BYTES + wave * 2048u + lane * 16u;
+  uint32_t decayAt = head * (GDN_BLOCK_TERMS * 4u) + (2u * B * B + B - 1u) * 4u;
+  struct Fetched {
+    BlockTerms terms;
+    uint4 key, query;             // this wave's 32 dimensions of token `row`
+    uint4 update[2];              // and of tokens 4 kq .. + 3, twice over
+    uint4 toEnd;
+    uint32_t decay;               // the whole block's
+  };
+  // The next block's loads in six pieces, which leave between the products of a block: all at once they fill the address
+  // unit that the four waves share, and a wave that waits there runs nothing else.
+  auto fetch = [&](Fetched &f, uint32_t piece) __attribute__((always_inline)) {
+    if (piece == 0) {
+      f.key = load128<0>(keyRows, keyAt);
+      f.query = load128<0>(queryRows, keyAt);
+      keyAt += B * keyRow;
+    } else if (piece == 1) {
+      fetchSolve(f.terms);
+    } else if (piece == 2) {
+      fetchWeights(f.terms);
+    } else if (piece == 3) {
+      fetchValues(f.terms);
+    } else if (piece == 4) {
+      f.toEnd = load128<0>(terms, rowsAt + B * 4u);
+      f.decay = __builtin_amdgcn_raw_buffer_load_b32(terms, int(decayAt), 0, 0);
+      advanceTerms();
+      decayAt += termsBlock;
+    } else {
+#pragma unroll
+      for (uint32_t m = 0; m < 2; ++m) f.update[m] = load128<0>(operands, operandAt + 1024u * m);
+      operandAt += keysBlock;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto run = [&](uint32_t block, uint32_t parity, const Fetched &f, Fetched &next) __attribute__((always_inline)) {
+    uint32_t high[4], middle[4], low[4];
+#pragma unroll
+    for (uint32_t e = 0; e < 4; ++e) split3(state[e >> 1][2u * (e & 1u)], state[e >> 1][2u * (e & 1u) + 1u], high[e], middle[e], low[e]);
+    const bf16x8 parts[3] = {as_bf16x8(make_uint4(low[0], low[1], low[2], low[3])), as_bf16x8(make_uint4(middle[0], middle[1], middle[2], middle[3])),
+                             as_bf16x8(make_uint4(high[0], high[1], high[2], high[3]))};
+    f32x4 sk = zero, sq = zero;   // rows are tokens 4 kq + i, column `row` a value dimension
+#pragma unroll
+    for (uint32_t e = 0; e < 3; ++e) {
+      sk = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(f.key), parts[e], sk, 0, 0, 0);
+      sq = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(f.query), parts[e], sq, 0, 0, 0);
+    }
+    shares[parity][0][wave][lane] = __builtin_bit_cast(float4, sk);
+    shares[parity][1][wave][lane] = __builtin_bit_cast(float4, sq);
+    __syncthreads();
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(next, 0);
+    const f32x4 corrections = correctionsOf(f.terms, whole(parity, 0), [&](uint32_t i) __attribute__((always_inline)) { fetch(next, 1u + i); });
+    const f32x4 toEnd = floats(f.toEnd);
+    // the update: places 0..3 of an operand's eight the corrections' leading parts, and apart from them the two parts left
+    uint32_t uh[2], um[2], ul[2];
+#pragma unroll
+    for (uint32_t e = 0; e < 2; ++e)
+      split3(corrections[2u * e] * toEnd[2u * e], corrections[2u * e + 1u] * toEnd[2u * e + 1u], uh[e], um[e], ul[e]);
+    const bf16x8 leading = as_bf16x8(make_uint4(uh[0], uh[1], 0u, 0u)), last = as_bf16x8(make_uint4(um[0], um[1], ul[0], ul[1]));
+    const float decay = block < blocks ? __uint_as_float(f.decay) : 1.f;
+#pragma unroll
+    for (uint32_t m = 0; m < 2; ++m) {
+      const bf16x8 key = as_bf16x8(f.update[m]);
+      const f32x4 most = __builtin_amdgcn_mfma_f32_16x16x32_bf16(key, leading, zero, 0, 0, 0);
+      const f32x4 rest = __builtin_amdgcn_mfma_f32_16x16x32_bf16(key, last, zero, 0, 0, 0);
+      if (m == 0) fetch(next, 5);
+#pragma unroll
+      for (uint32_t i = 0; i < 4; ++i) state[m][i] = __fmaf_rn(state[m][i], decay, rest[i]) + most[i];
+    }
+  };
+  Fetched ahead[kAhead];
+#pragma unroll
+  for (uint32_t a = 0; a + 1 < kAhead; ++a)
+#pragma unroll
+    for (uint32_t piece = 0; piece < 6; ++piece) fetch(ahead[a], piece);   // (in the order the loop waits for them)
+  for (uint32_t round = 0, parity = 0; round < rounds; ++round) {
+#pragma unroll
+    for (uint32_t a = 0; a < kAhead; ++a, parity ^= 1u) {
+      run(round * kAhead + a, parity, ahead[a], ahead[(a + kAhead - 1u) % kAhead]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (uint32_t m = 0; m < 2; ++m) *reinterpret_cast<f32x4 *>(stateOut + stateAt + 4u * m) = state[m];
+}
+SP_REGISTER_KERNEL("gdn_prefill_block_scan", &gdn_prefill_block_scan);
 
 // gdn_prefill_gate: grid (value_heads, ceil(tokens / 4)), 256 threads, a wave per (row, value head): the gated
 // output norm of the scan's rows (prefill/gdn.metal:312-341, gdn.metal:489-526).

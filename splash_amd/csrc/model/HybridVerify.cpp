@@ -169,6 +169,7 @@ void HybridVerify::prepareChunks() {
                  device(chunk.totals, "moe chunk totals"), device(chunk.table, "moe chunk tables"), device(chunk.intermediate, "moe chunk SwiGLU rows"),
                  device(chunk.expertOutput, "moe chunk expert outputs")};
   }
+  if (d.gdnLayers()) gdnBlocks_ = device(gdn_prefill_blocks_bytes(rowCapacity_, d.gdnKeyHeads, d.gdnValueHeads), "GDN block terms");
   // last: what says that the others are there
   const uint32_t widest = std::max({d.hidden, d.attentionWidth(), d.gdnWidth(), d.dense() ? d.denseFfn : 0u});
   wideTable_ = device(ops::Linear::wideTableBytes(widest, rowCapacity_), "wide table");
@@ -435,7 +436,7 @@ void HybridVerify::encodeWidePrefillLayer(hip::CommandGraph &graph, uint32_t lay
     ops::PagedAttention::addPromptProjection(graph, plan, {packed_, w.queryNorm, w.keyNorm, ropeCos_, ropeSin_}, attentionWorkspace_, pages);
     ops::PagedAttention::addPromptAttention(graph, plan, attentionWorkspace_, treeRows_, pages, mixed_, packed_);
   } else {
-    addGdnPrefill(graph, w, index, tokens, currentCell, nextCell);
+    addGdnPrefill(graph, w, index, tokens, currentCell, nextCell, gdnBlocks_);
   }
   ops::Linear::addWideTable(graph, mixed_, wideTable_, mixedWidth, tokens);
   linear_.addWide(graph, w.mixerOutput, wideTable_, next, residual, widePartials_, tokens);
@@ -451,8 +452,10 @@ void HybridVerify::encodeWidePrefillLayer(hip::CommandGraph &graph, uint32_t lay
   ops::MoE::addChunk(graph, wideScores_, dims_.experts, normalized_, next, residual, w.experts, moeChunk_, dims_.moeShape(), tokens, w.sharedScalarGate);
 }
 
-void HybridVerify::addGdnPrefill(hip::CommandGraph &graph, const HybridLayer &w, uint32_t index, uint32_t tokens, uint64_t currentCell, uint64_t nextCell) {
+void HybridVerify::addGdnPrefill(hip::CommandGraph &graph, const HybridLayer &w, uint32_t index, uint32_t tokens, uint64_t currentCell, uint64_t nextCell,
+                                 const hip::Buffer &blocks) {
   ops::GdnPrefillBuffers buffers = gdnPrefill_;
+  buffers.blocks = blocks;
   buffers.packed = packed_;
   buffers.convolutionWeights = w.convolutionWeights;
   buffers.states = states_;

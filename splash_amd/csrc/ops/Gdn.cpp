@@ -107,6 +107,12 @@ void GDN::addPrefill(hip::CommandGraph &graph, const GdnPrefillBuffers &b, const
   requireBytes(b.beta, uint64_t{tokens} * shape.valueHeads * 2, "GDN beta rows");
   requireBytes(b.recurrentRows, tokens * valueWidth * 2, "GDN recurrent rows");
   requireBytes(b.hidden, tokens * valueWidth * 2, "GDN hidden rows");
+  if (b.blocks) {
+    // (offsets into a run's rows are 32-bit)
+    if (std::max<uint64_t>(tokens * valueWidth * 2, gdn_prefill_blocks_bytes(tokens, shape.keyHeads, shape.valueHeads)) >> 31)
+      throw std::invalid_argument("the rows of a GDN prompt chunk in blocks are too many");
+    requireBytes(b.blocks, gdn_prefill_blocks_bytes(tokens, shape.keyHeads, shape.valueHeads), "GDN block terms");
+  }
   GdnPrefillParams params{};
   params.shape = shape.params();
   params.flags = (order == GdnHeadOrder::Tiled ? GDN_TILED_HEADS : 0u) | (shape.sigmoidGate ? GDN_SIGMOID_GATE : 0u) |
@@ -130,7 +136,12 @@ void GDN::addPrefill(hip::CommandGraph &graph, const GdnPrefillBuffers &b, const
     graph.add("gdn_prefill_prepare",
               {b.packed, b.convolutionWeights, b.states, b.decayWeights, b.timeBias, b.queries, b.keys, b.values, b.decay, b.beta}, params,
               {shape.valueHeads, (params.tokens + 3) / 4, 1}, {256, 1, 1});
-    graph.add("gdn_prefill_scan", {b.queries, b.keys, b.values, b.decay, b.beta, b.states, b.recurrentRows}, params,
+    if (b.blocks) {
+      graph.add("gdn_prefill_blocks", {b.queries, b.keys, b.decay, b.beta, b.blocks}, params,
+                {shape.valueHeads, ((params.tokens + GDN_SCAN_BLOCK - 1) / GDN_SCAN_BLOCK + 3) / 4, 1}, {256, 1, 1});
+      graph.add("gdn_prefill_block_scan", {b.queries, b.keys, b.values, b.blocks, b.states, b.recurrentRows}, params,
+                {shape.valueHeads * (GDN_HEAD_DIMENSION / 16), 1, 1}, {320, 1, 1});
+    } else graph.add("gdn_prefill_scan", {b.queries, b.keys, b.values, b.decay, b.beta, b.states, b.recurrentRows}, params,
               {shape.valueHeads * (GDN_HEAD_DIMENSION / GDN_SCAN_STATE_ROWS), 1, 1}, {256, 1, 1});
     begin = end;
     cell = out;

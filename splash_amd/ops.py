@@ -680,14 +680,23 @@ class GDN:
                      recurrent_rows=tokens * vw * 2, hidden=tokens * vw * 2)
         return {n: backend.allocate_buffer(max(b, 16), STORAGE_PRIVATE, "gdn prefill " + n) for n, b in sizes.items()}
 
-    def add_prefill(self, graph, buffers, layer, tokens, current_cell, next_cell, captures=(), tiled_heads=False, float_norm=False):
+    def prefill_blocks_bytes(self, tokens):
+        return lib.spo_gdn_prefill_blocks_bytes(ctypes.byref(self.shape), tokens)
+
+    def add_prefill(self, graph, buffers, layer, tokens, current_cell, next_cell, captures=(), tiled_heads=False, float_norm=False, blocks=None):
         """GDN::addPrefill: a prompt chunk of one lane and layer. buffers: dict of Buffer by the names of
-        spo_gdn_prefill_buffers; captures: [(tokens, cell)], ascending inside the rows."""
+        spo_gdn_prefill_buffers; captures: [(tokens, cell)], ascending inside the rows; blocks: a Buffer of
+        prefill_blocks_bytes(tokens) for the scan in blocks on the matrix cores, equal to the scan to rounding."""
         b = nat.GdnPrefillBuffers(**{k: v.handle for k, v in buffers.items()}, float_norm=int(float_norm), current_cell=current_cell,
                                   next_cell=next_cell)
         arr = (nat.GdnPrefillCapture * max(1, len(captures)))(*[nat.GdnPrefillCapture(t, 0, c) for t, c in captures])
-        check(lib.spo_gdn_add_prefill(graph.handle, ctypes.byref(b), ctypes.byref(self.shape), layer, tokens, ctypes.byref(self.strides),
-                                      int(tiled_heads), arr, len(captures)))
+        if blocks is None:
+            check(lib.spo_gdn_add_prefill(graph.handle, ctypes.byref(b), ctypes.byref(self.shape), layer, tokens, ctypes.byref(self.strides),
+                                          int(tiled_heads), arr, len(captures)))
+        else:
+            check(lib.spo_gdn_add_prefill_blocks(graph.handle, ctypes.byref(b), blocks.handle, ctypes.byref(self.shape), layer, tokens,
+                                                 ctypes.byref(self.strides), int(tiled_heads), arr, len(captures)))
+            graph._keep.append(blocks)
         graph._keep.extend(list(buffers.values()))
 
     def add_fold(self, graph, states, tape, retained_rows, step_tape, state_cell, fold_cell, rows):
