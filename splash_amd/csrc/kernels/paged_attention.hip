@@ -6,6 +6,7 @@
 //                             query rows, quantize k and v into the row's page slot.
 //   attention_q8_split_d<D>_g<G>  per (KV head, history split, sequence): flash-decoding page loop
 //                             over the split's 64-token steps for all 16 G fused rows of the head.
+//   attention_q8_few_d<D>_g<G>_t<T>  the same for blocks of up to eight rows, a wave a split.
 //   attention_reduce_d<D>     per (query head, row, sequence): merge the splits in split order.
 //   attention_q8_commit_d<D>  per (KV head, sequence): move the retained path's slots to their depths.
 //
@@ -21,7 +22,7 @@
 #include "abi/Gguf.h"
 #include "abi/PagedAttention.h"
 #include "backend/KernelRegistry.hpp"
-#include "kernels/device_common.hpp"
+#include "kernels/gguf_records.hpp"   // buffer resources
 #include <type_traits>
 
 namespace splash::kernels {
@@ -671,6 +672,271 @@ SP_REGISTER_KERNEL("attention_q8_split_chunk_d64_g2", (&attention_q8_split<64, 2
 SP_REGISTER_KERNEL("attention_q8q_split_d128_g8", &attention_q8_split<128, 8, true>);
 SP_REGISTER_KERNEL("attention_q8q_split_d128_g4", &attention_q8_split<128, 4, true>);
 SP_REGISTER_KERNEL("attention_q8q_split_d64_g2", &attention_q8_split<64, 2, true>);
+
+// ---------------------------------------------------------------------------------------------
+// attention_q8_few: grid (parts * kv_heads, splits, sequences), 64 threads: the same partials, bit for bit, for blocks of at
+// most 16 T parts / G rows, whose (row, head) pairs fill T tiles of sixteen a part where attention_q8_split always computes G
+// tiles. The parts of a head read its keys and values each for itself, on one die, whose L2 answers all but the first.
+//
+// A wave walks its split alone: no staging, no barrier. Keys and values go from the cache's pages straight into registers in
+// whole 16-byte loads, and lane-row swaps put them in operand order: of a token's key codes lane quarter a loads chunk a with
+// its bits exchanged, and one v_permlane16_swap of the chunk's halves leaves unit 4 j + a of eight codes in quarter a; of a
+// dimension's 64 values quarter a loads tokens 16 a .. + 15, and a 4 x 4 transpose (two v_permlane32_swap, two
+// v_permlane16_swap) leaves tokens 16 j + 4 a .. + 3. Loads run `Ahead` steps ahead through a buffer resource of their page,
+// which past the split's last step is empty (zeros, no traffic), so nothing branches around them.
+//
+// Bound by memory latency at two waves a compute unit: one row of 64 / 8 heads behind 100000 tokens takes 48 us (4.3 TB/s of
+// keys and values, a copy 5.2) against 77 in attention_q8_split, which computes 128 pairs for its eight.
+// ---------------------------------------------------------------------------------------------
+__device__ __forceinline__ void swap_rows16(uint32_t &a, uint32_t &b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
+}
+__device__ __forceinline__ void swap_rows32(uint32_t &a, uint32_t &b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
+}
+template <int D, int G, int T, int Ahead>
+__global__ __launch_bounds__(64, 1) void attention_q8_few(const _Float16 *__restrict__ queries, const float *__restrict__ qsums,
+                                                                      const AttentionTreeRow *__restrict__ tree,
+                                                                      const uint64_t *__restrict__ page_table, uint8_t *__restrict__ pool,
+                                                                      _Float16 *__restrict__ partialO, float *__restrict__ partialML,
+                                                                      AttentionParams p) {
+  constexpr uint32_t kStep = ATTENTION_STEP_TOKENS;
+  constexpr int JD = D / 32, DT = D / 16, KL = D / 64;
+  __shared__ __align__(16) float scales[2][kStep];
+  const uint32_t lane = threadIdx.x, column = lane & 15u, kq = lane >> 4, h = blockIdx.x % p.kv_heads, part = blockIdx.x / p.kv_heads, split = blockIdx.y, z = blockIdx.z;
+  const AttentionSequence seq = p.sequence[z];
+  const uint32_t total = seq.committed + seq.rows, span = uint32_t(seq.steps_per_split) * kStep;
+  const uint32_t first = min(total, split * span), last = min(total, (split + 1) * span);
+  const uint32_t steps = first < last ? (last - first + kStep - 1) / kStep : 0;
+  const float scale2 = kLog2e / sqrtf(float(D));
+
+  // Column c of all parts' tiles is row c % rowsHeld of head c / rowsHeld (rowsHeld a power of two).
+  const uint32_t rowsShift = uint32_t(__builtin_ctz(gridDim.x / p.kv_heads * (16u * T) / G));
+  auto headOf = [&](uint32_t k) { return (16u * (part * T + k) + column) >> rowsShift; };
+  const uint32_t row = column & ((1u << rowsShift) - 1u);
+  f16x8 q[T][JD];
+  float qsum[T];
+  uint32_t ancestors[T];
+#pragma unroll
+  for (int k = 0; k < T; ++k) {
+    const size_t at = ((size_t(z) * p.kv_heads + h) * G + headOf(k)) * 16u + row;
+#pragma unroll
+    for (int j = 0; j < JD; ++j) q[k][j] = *reinterpret_cast<const f16x8 *>(queries + at * D + 32 * j + 8 * kq);
+    qsum[k] = -(qsums[at] * kCodeOffset);
+    ancestors[k] = row < seq.rows ? tree[seq.first_row + row].ancestors : 0u;
+  }
+  float m[T], l[T];
+  f32x4 o[T][DT + 1];
+#pragma unroll
+  for (int k = 0; k < T; ++k) {
+    m[k] = -INFINITY;
+    l[k] = 0.f;
+#pragma unroll
+    for (int dt = 0; dt <= DT; ++dt) o[k][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+
+  struct Raw {
+    uint4 key[4][KL], value[DT];
+    uint32_t keyScale, valueScale;   // of token `lane`
+  };
+  const uint64_t *entries = page_table + seq.table_first;
+  const uint32_t lastPage = total ? (total - 1u) / ATTENTION_PAGE_TOKENS : 0u;
+  uint32_t heldPage = min(first / ATTENTION_PAGE_TOKENS, lastPage);
+  uint64_t heldEntry = entries[heldPage], nextEntry = entries[min(heldPage + 1u, lastPage)];   // (read one page ahead)
+  struct Page {
+    Resource bytes;
+    uint32_t inPage;
+  };
+  auto pageOf = [&](uint32_t step) __attribute__((always_inline)) {
+    const uint32_t token0 = first + step * kStep;
+    if (step < steps && token0 / ATTENTION_PAGE_TOKENS != heldPage) {
+      heldPage = token0 / ATTENTION_PAGE_TOKENS;
+      heldEntry = nextEntry;
+      nextEntry = entries[min(heldPage + 1u, lastPage)];
+    }
+    return Page{make_resource(pool + heldEntry * p.page_bytes, step < steps ? uint32_t(attention_page_bytes(p.kv_heads, D)) : 0u), token0 % ATTENTION_PAGE_TOKENS};
+  };
+  const uint32_t keyLane = column * D + 16u * (((kq & 1u) << 1) | (kq >> 1)), valueLane = column * kStep + 16u * kq;
+  auto loadKeys = [&](Raw &raw, const Page &page) __attribute__((always_inline)) {
+    const uint32_t at = uint32_t(attention_key_index(h, page.inPage, 0, D)) + keyLane;
+#pragma unroll
+    for (uint32_t tt = 0; tt < 4; ++tt)
+#pragma unroll
+      for (uint32_t n = 0; n < KL; ++n) raw.key[tt][n] = load128<0>(page.bytes, at + tt * (16u * D) + 64u * n);
+    raw.keyScale = __builtin_amdgcn_raw_buffer_load_b16(
+        page.bytes, int(uint32_t(attention_page_key_scales_offset(p.kv_heads, D)) + 2u * (uint32_t(attention_scale_index(h, page.inPage)) + lane)), 0, 0);
+    raw.valueScale = __builtin_amdgcn_raw_buffer_load_b16(
+        page.bytes, int(uint32_t(attention_page_value_scales_offset(p.kv_heads, D)) + 2u * (uint32_t(attention_scale_index(h, page.inPage)) + lane)), 0, 0);
+  };
+  auto loadValues = [&](Raw &raw, const Page &page) __attribute__((always_inline)) {
+    const uint32_t at = uint32_t(attention_page_values_offset(p.kv_heads, D)) + uint32_t(attention_value_index(h, page.inPage, 0, D)) + valueLane;
+#pragma unroll
+    for (uint32_t dt = 0; dt < uint32_t(DT); ++dt) raw.value[dt] = load128<kStreamOnce>(page.bytes, at + dt * (16u * kStep));
+  };
+  const f16x8 ones = {_Float16(1.f), _Float16(1.f), _Float16(1.f), _Float16(1.f), _Float16(1.f), _Float16(1.f), _Float16(1.f), _Float16(1.f)};
+  auto operand = [](uint32_t a, uint32_t b) __attribute__((always_inline)) {   // two words of codes as 1152 + code
+    const uint2 x = bytes_to_f16(a ^ 0x80808080u), y = bytes_to_f16(b ^ 0x80808080u);
+    return __builtin_bit_cast(f16x8, make_uint4(x.x, x.y, y.x, y.y));
+  };
+
+  // One step, its arithmetic attention_split's (see there); `raw` then takes the step `Ahead` after it.
+  auto run = [&](uint32_t step, Raw &raw, auto maskedTag) __attribute__((always_inline)) {
+    constexpr bool kMasked = decltype(maskedTag)::value;
+    const Page next = pageOf(step + Ahead);
+    wave_lds_fence();
+    scales[0][lane] = half_bits_to_float(raw.keyScale) * scale2;
+    scales[1][lane] = half_bits_to_float(raw.valueScale) * kPScale;
+    wave_lds_fence();
+    f32x4 s[T][4];
+#pragma unroll
+    for (uint32_t tt = 0; tt < 4; ++tt) {
+      f16x8 key[JD];
+#pragma unroll
+      for (uint32_t n = 0; n < KL; ++n) {
+        uint4 x = raw.key[tt][n];
+        swap_rows16(x.x, x.z);
+        swap_rows16(x.y, x.w);
+        key[2 * n] = operand(x.x, x.y);
+        key[2 * n + 1] = operand(x.z, x.w);
+      }
+#pragma unroll
+      for (int k = 0; k < T; ++k) {
+        f32x4 acc = {qsum[k], qsum[k], qsum[k], qsum[k]};
+#pragma unroll
+        for (int j = 0; j < JD; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(key[j], q[k][j], acc, 0, 0, 0);
+        s[k][tt] = acc;
+      }
+    }
+    loadKeys(raw, next);
+    f32x4 keyScale[4], valueScale[4];
+#pragma unroll
+    for (int tt = 0; tt < 4; ++tt) {
+      keyScale[tt] = *reinterpret_cast<const f32x4 *>(&scales[0][16 * tt + 4 * kq]);
+      valueScale[tt] = *reinterpret_cast<const f32x4 *>(&scales[1][16 * tt + 4 * kq]);
+    }
+    f16x8 pOperand[T][2];
+#pragma unroll
+    for (int k = 0; k < T; ++k) {
+      float stepMax = -INFINITY;
+#pragma unroll
+      for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float score = s[k][tt][i] * keyScale[tt][i];
+          if constexpr (kMasked) {
+            const uint32_t token = first + step * kStep + 16u * tt + 4u * kq + i;
+            const bool visible = token < seq.committed || (token < total && ((ancestors[k] >> (token - seq.committed)) & 1u));
+            score = visible ? score : -INFINITY;
+          }
+          s[k][tt][i] = score;
+          stepMax = fmaxf(stepMax, score);
+        }
+      stepMax = fmaxf(stepMax, __shfl_xor(stepMax, 16, 64));
+      stepMax = fmaxf(stepMax, __shfl_xor(stepMax, 32, 64));
+      const float newMax = fmaxf(m[k], stepMax), safeMax = newMax == -INFINITY ? 0.f : newMax;
+      const float alpha = __builtin_amdgcn_exp2f(m[k] - safeMax);
+      m[k] = newMax;
+      float sum = 0.f, folded[16];
+#pragma unroll
+      for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float pr = __builtin_amdgcn_exp2f(s[k][tt][i] - safeMax);
+          sum += pr;
+          const float f = pr * valueScale[tt][i];
+          folded[4 * tt + i] = kMasked ? (pr > 0.f ? f : 0.f) : f;
+        }
+      l[k] = l[k] * alpha + sum;
+      if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {
+#pragma unroll
+        for (int dt = 0; dt <= DT; ++dt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[k][dt][i] *= alpha;
+      }
+#pragma unroll
+      for (int pair = 0; pair < 2; ++pair)
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+          typedef __attribute__((ext_vector_type(2))) float f32x2;
+          typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
+          const f16x2 two = __builtin_convertvector(f32x2{folded[8 * pair + e], folded[8 * pair + e + 1]}, f16x2);
+          pOperand[k][pair][e] = two[0];
+          pOperand[k][pair][e + 1] = two[1];
+        }
+    }
+#pragma unroll
+    for (uint32_t dt = 0; dt < uint32_t(DT); ++dt) {
+      uint4 x = raw.value[dt];
+      swap_rows32(x.x, x.z);
+      swap_rows32(x.y, x.w);
+      swap_rows16(x.x, x.y);
+      swap_rows16(x.z, x.w);
+      const f16x8 value[2] = {operand(x.x, x.y), operand(x.z, x.w)};
+#pragma unroll
+      for (int k = 0; k < T; ++k)
+#pragma unroll
+        for (int pair = 0; pair < 2; ++pair) o[k][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(value[pair], pOperand[k][pair], o[k][dt], 0, 0, 0);
+    }
+#pragma unroll
+    for (int k = 0; k < T; ++k)
+#pragma unroll
+      for (int pair = 0; pair < 2; ++pair) o[k][DT] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, pOperand[k][pair], o[k][DT], 0, 0, 0);
+    loadValues(raw, next);
+  };
+  Raw raw[Ahead];
+#pragma unroll
+  for (uint32_t a = 0; a < uint32_t(Ahead); ++a) {
+    const Page page = pageOf(a);
+    loadKeys(raw[a], page);
+    loadValues(raw[a], page);
+    __builtin_amdgcn_sched_barrier(0);   // (in the order the loop waits for them)
+  }
+  // Steps wholly inside the committed history, then those that reach the block's own rows or the sequence's end.
+  const uint32_t plain = first < seq.committed ? min(steps, (seq.committed - first) / kStep) : 0u;
+  for (uint32_t step = 0; step < steps; step += Ahead) {
+#pragma unroll
+    for (uint32_t a = 0; a < uint32_t(Ahead); ++a) {
+      if (step + a < plain) run(step + a, raw[a], std::false_type{});
+      else if (step + a < steps) run(step + a, raw[a], std::true_type{});
+    }
+  }
+
+  // The partials, as attention_split leaves them.
+#pragma unroll
+  for (int k = 0; k < T; ++k) {
+    const uint32_t g = headOf(k);
+    float sum = l[k];
+    sum += __shfl_xor(sum, 16, 64);
+    sum += __shfl_xor(sum, 32, 64);
+    if (row >= seq.rows) continue;
+    const size_t fused = ((size_t(z) * p.kv_heads + h) * p.splits + split) * (16u * G) + 16u * g + row;
+    const float rowSum = o[k][DT][0] * kCodeOffset, norm = sum > 0.f ? 1.0f / (sum * kPScale) : 0.f;
+    uint4 *mine = reinterpret_cast<uint4 *>(partialO + fused * D + 4u * DT * kq);
+#pragma unroll
+    for (int dt = 0; dt < DT; dt += 2) {
+      f16x8 out;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        out[i] = _Float16((o[k][dt][i] - rowSum) * norm);
+        out[4 + i] = _Float16((o[k][dt + 1][i] - rowSum) * norm);
+      }
+      mine[dt / 2] = __builtin_bit_cast(uint4, out);
+    }
+    if (kq == 0) {
+      partialML[2 * fused] = m[k];
+      partialML[2 * fused + 1] = sum;
+    }
+  }
+}
+SP_REGISTER_KERNEL("attention_q8_few_d128_g8_t1", (&attention_q8_few<128, 8, 1, 2>));
+SP_REGISTER_KERNEL("attention_q8_few_d128_g8_t2", (&attention_q8_few<128, 8, 2, 2>));
+SP_REGISTER_KERNEL("attention_q8_few_d128_g4_t1", (&attention_q8_few<128, 4, 1, 2>));
+SP_REGISTER_KERNEL("attention_q8_few_d128_g4_t2", (&attention_q8_few<128, 4, 2, 2>));
+SP_REGISTER_KERNEL("attention_q8_few_d64_g2_t1", (&attention_q8_few<64, 2, 1, 2>));
 
 // ---------------------------------------------------------------------------------------------
 // attention_reduce: grid (q_heads, 16, sequences), 256 threads. Merges the splits of one (head,

@@ -2,6 +2,7 @@
 #include "ops/Linear.hpp"  // requireBytes
 
 #include <algorithm>
+#include <bit>
 #include <stdexcept>
 #include <string>
 
@@ -28,6 +29,28 @@ uint32_t totalRows(const std::vector<AttentionRows> &sequences) {
   uint32_t rows = 0;
   for (const AttentionRows &s : sequences) rows = std::max(rows, s.firstRow + s.rows);
   return rows;
+}
+// Which steps attend a wave a split (attention_q8_few) and how: the tiles of (row, head) pairs of a wave, and the waves (parts)
+// that share a split's pairs; no tiles: attention_q8_split, whose workgroups compute sixteen rows whatever the block has.
+// The widest block's rows, rounded up to a power of two, decide. Between events, split against few, us: 64 / 8 heads behind 100003
+// tokens 1 row 92 / 58, 4 rows 93 / 61 in two parts (76 as two tiles of one), 8 rows 92 / 80, 16 rows 90 / 144; 8 sequences behind
+// 16368 tokens 1 row 180 / 64, 4 rows 160 / 80 (100 in two parts), 8 rows 169 / 134, 16 rows 172 / 246; behind 4000 tokens and less
+// all of them lie within the fixed cost (23 / 22). So: up to eight rows; a tile a part while every part has a SIMD of its own
+// (4 x 256), then two tiles a part, which widen the keys and values they share once. 16 / 8 heads of 64, 8 rows: 8 sequences behind
+// 16368 tokens 54 / 37; 16 rows 54 / 51 in two parts, within 1 us of each other elsewhere.
+struct FewRows {
+  uint32_t tiles = 0, parts = 0;
+};
+FewRows fewRows(const AttentionPlan &plan) {
+  const AttentionGeometry &g = plan.geometry();
+  uint32_t most = 1;
+  for (const AttentionRows &s : plan.sequences()) most = std::max(most, s.rows);
+  const uint32_t all = std::max(1u, std::bit_ceil(most) * g.group() / 16u);
+  if (g.int8Queries || most > 8) return {};
+  constexpr uint64_t kSimds = 4 * 256;
+  const uint64_t waves = uint64_t{g.kvHeads} * plan.splits() * plan.sequences().size();
+  if (all == 1 || waves * all <= kSimds) return {1, all};
+  return {2, all / 2};
 }
 void requirePages(const AttentionPlan &plan, const KvPages &pages) {
   const uint64_t need = plan.geometry().layout().bytesPerLayerPage();
@@ -155,9 +178,16 @@ void PagedAttention::addAttention(hip::CommandGraph &graph, const AttentionPlan 
     params.table_tiles = gguf_row_tiles(tableRows ? tableRows : rows);
     requireBytes(outputTable, gguf_tables_bytes(width, params.table_tiles), "attention output table");
   }
-  graph.add(std::string(g.int8Queries ? "attention_q8q_split" : "attention_q8_split") + kernelSuffix(g) + "_g" + std::to_string(g.group()),
-            {w.queries, w.querySums, treeRows, pages.pageTable, pages.pool, w.partials, w.partialSums}, params,
-            {g.kvHeads, plan.splits(), plan.sequences().size()}, {256, 1, 1});
+  const std::string suffix = kernelSuffix(g) + "_g" + std::to_string(g.group());
+  const FewRows few = fewRows(plan);
+  if (few.tiles)
+    graph.add("attention_q8_few" + suffix + "_t" + std::to_string(few.tiles),
+              {w.queries, w.querySums, treeRows, pages.pageTable, pages.pool, w.partials, w.partialSums}, params,
+              {few.parts * g.kvHeads, plan.splits(), plan.sequences().size()}, {64, 1, 1});
+  else
+    graph.add((g.int8Queries ? "attention_q8q_split" : "attention_q8_split") + suffix,
+              {w.queries, w.querySums, treeRows, pages.pageTable, pages.pool, w.partials, w.partialSums}, params,
+              {g.kvHeads, plan.splits(), plan.sequences().size()}, {256, 1, 1});
   graph.add("attention_reduce" + kernelSuffix(g) + (outputTable ? "_t" : ""),
             {w.partials, w.partialSums, output, outputTable ? outputTable : output, g.gated ? packed : output}, params,
             {g.qHeads, ATTENTION_MAXIMUM_ROWS, plan.sequences().size()}, {256, 1, 1});
