@@ -10,10 +10,11 @@
 #include <chrono>
 #include <cstdio>
 #include <cstring>
-#include <map>
 #include <mutex>
 #include <string>
+#include <string_view>
 #include <thread>
+#include <unordered_map>
 #include <vector>
 
 namespace splash::hipbackend {
@@ -23,8 +24,13 @@ std::vector<KernelEntry> &registry() {
   static std::vector<KernelEntry> entries;
   return entries;
 }
-std::map<std::string, size_t> &registryIndex() {
-  static std::map<std::string, size_t> index;
+// (looked up once a dispatch, before the first of a command is launched: by the caller's characters, not by a copy of them)
+struct NameHash {
+  using is_transparent = void;
+  size_t operator()(std::string_view name) const noexcept { return std::hash<std::string_view>{}(name); }
+};
+std::unordered_map<std::string, size_t, NameHash, std::equal_to<>> &registryIndex() {
+  static std::unordered_map<std::string, size_t, NameHash, std::equal_to<>> index;
   return index;
 }
 } // namespace
@@ -41,7 +47,7 @@ void registerKernel(KernelEntry entry) {
 const KernelEntry *findKernel(const char *name) {
   if (!name) return nullptr;
   const auto &index = registryIndex();
-  const auto it = index.find(name);
+  const auto it = index.find(std::string_view(name));
   return it == index.end() ? nullptr : &registry()[it->second];
 }
 const std::vector<KernelEntry> &allKernels() { return registry(); }
@@ -81,6 +87,31 @@ struct sp_backend {
   uint64_t allocated = 0, peak = 0, deviceCurrent = 0, devicePeak = 0;
   uint64_t deviceBaseline = 0;  // bytes in use on the device before this backend allocated
   std::atomic<int> liveBuffers{0};
+  // Events of finished commands, for the next ones (creating and destroying a command's two costs more than recording them):
+  // at most kSpareEvents, destroyed with the backend's stream.
+  static constexpr size_t kSpareEvents = 8;
+  std::vector<hipEvent_t> spareEvents;   // under `mutex`
+  hipError_t takeEvent(hipEvent_t *event) {
+    {
+      std::lock_guard<std::mutex> lock(mutex);
+      if (!spareEvents.empty()) {
+        *event = spareEvents.back();
+        spareEvents.pop_back();
+        return hipSuccess;
+      }
+    }
+    return hipEventCreate(event);
+  }
+  void giveEvent(hipEvent_t event) {
+    {
+      std::lock_guard<std::mutex> lock(mutex);
+      if (stream && spareEvents.size() < kSpareEvents) {
+        spareEvents.push_back(event);
+        return;
+      }
+    }
+    (void)hipEventDestroy(event);
+  }
   // The backend's memory outlives sp_backend_destroy while buffers, tickets or commands still name it.
   std::atomic<int> refs{1};
   void retain() { ++refs; }
@@ -140,9 +171,20 @@ struct sp_command {
 
 namespace {
 
-sp_status validateDispatch(const sp_dispatch &d, uint32_t index, RecordedDispatch &out, std::vector<sp_buffer *> &retained,
+// Every kernel of the registry binds fewer (checked where a dispatch is validated).
+constexpr uint32_t kMostBuffers = 32;
+
+sp_status validateDispatch(const sp_dispatch &d, uint32_t index, const KernelEntry *&found, std::vector<sp_buffer *> &retained,
                            sp_backend *backend) {
-  const std::string at = "dispatch " + std::to_string(index) + " (" + (d.kernel ? d.kernel : "<null>") + ")";
+  // (the words of a message are put together only where there is one)
+  struct Where {
+    const sp_dispatch &d;
+    uint32_t index;
+    std::string operator+(const std::string &rest) const {
+      return "dispatch " + std::to_string(index) + " (" + (d.kernel ? d.kernel : "<null>") + ")" + rest;
+    }
+  };
+  const Where at{d, index};
   const KernelEntry *kernel = findKernel(d.kernel);
   if (!kernel) return fail(SP_UNKNOWN_KERNEL, at + ": no kernel of that name");
   if (d.buffer_count != kernel->buffers)
@@ -157,17 +199,13 @@ sp_status validateDispatch(const sp_dispatch &d, uint32_t index, RecordedDispatc
   if (uint64_t(d.block[0]) * d.block[1] * d.block[2] > 1024)
     return fail(SP_INVALID_ARGUMENT, at + ": more than 1024 threads per workgroup");
   if (d.grid[1] > 65535 || d.grid[2] > 65535) return fail(SP_INVALID_ARGUMENT, at + ": grid y or z beyond 65535");
-  out.kernel = kernel;
-  out.grid = dim3(d.grid[0], d.grid[1], d.grid[2]);
-  out.block = dim3(d.block[0], d.block[1], d.block[2]);
-  out.params.assign(static_cast<const unsigned char *>(d.params), static_cast<const unsigned char *>(d.params) + d.params_bytes);
-  out.pointers.resize(d.buffer_count);
+  if (d.buffer_count > kMostBuffers) return fail(SP_INVALID_ARGUMENT, at + ": more buffers than a dispatch takes");
+  found = kernel;
   for (uint32_t b = 0; b < d.buffer_count; ++b) {
     sp_buffer *buffer = d.buffers[b];
     if (!buffer) return fail(SP_INVALID_ARGUMENT, at + ": buffer " + std::to_string(b) + " is null");
     if (buffer->backend != backend)
       return fail(SP_INVALID_ARGUMENT, at + ": buffer " + std::to_string(b) + " belongs to another backend");
-    out.pointers[b] = buffer->device;
     retained.push_back(buffer);
   }
   return SP_OK;
@@ -181,6 +219,23 @@ void releaseAll(std::vector<sp_buffer *> &buffers) {
   buffers.clear();
 }
 
+RecordedDispatch recordDispatch(const sp_dispatch &d, const KernelEntry *kernel) {
+  RecordedDispatch out;
+  out.kernel = kernel;
+  out.grid = dim3(d.grid[0], d.grid[1], d.grid[2]);
+  out.block = dim3(d.block[0], d.block[1], d.block[2]);
+  out.params.assign(static_cast<const unsigned char *>(d.params), static_cast<const unsigned char *>(d.params) + d.params_bytes);
+  for (uint32_t b = 0; b < d.buffer_count; ++b) out.pointers.push_back(d.buffers[b]->device);
+  return out;
+}
+// A validated dispatch from the caller's own records.
+hipError_t launchDispatch(sp_backend *backend, const sp_dispatch &d, const KernelEntry *kernel) {
+  void *pointers[kMostBuffers];
+  for (uint32_t b = 0; b < d.buffer_count; ++b) pointers[b] = d.buffers[b]->device;
+  LaunchArgs args{backend->stream, dim3(d.grid[0], d.grid[1], d.grid[2]), dim3(d.block[0], d.block[1], d.block[2]), pointers, d.buffer_count,
+                  d.params, d.params_bytes};
+  return kernel->launch(args);
+}
 hipError_t launchRecorded(sp_backend *backend, const RecordedDispatch &d) {
   LaunchArgs args{backend->stream, d.grid, d.block, d.pointers.data(), uint32_t(d.pointers.size()), d.params.data(),
                   uint32_t(d.params.size())};
@@ -205,9 +260,9 @@ sp_status beginTicket(sp_backend *backend, sp_completion completion, void *user,
   ticket->backend = backend;
   ticket->completion = completion;
   ticket->user = user;
-  hipError_t e = hipEventCreate(&ticket->start);
-  if (e == hipSuccess) e = hipEventCreate(&ticket->end);
-  if (e == hipSuccess && completion) e = hipEventCreate(&ticket->fence);
+  hipError_t e = backend->takeEvent(&ticket->start);
+  if (e == hipSuccess) e = backend->takeEvent(&ticket->end);
+  if (e == hipSuccess && completion) e = backend->takeEvent(&ticket->fence);
   for (size_t i = 0; e == hipSuccess && i < marks; ++i) {
     hipEvent_t mark = nullptr;
     e = hipEventCreate(&mark);
@@ -227,9 +282,8 @@ sp_status beginTicket(sp_backend *backend, sp_completion completion, void *user,
 
 void destroyTicket(sp_ticket *ticket) {
   for (hipEvent_t m : ticket->marks) (void)hipEventDestroy(m);
-  (void)hipEventDestroy(ticket->start);
-  (void)hipEventDestroy(ticket->end);
-  if (ticket->fence) (void)hipEventDestroy(ticket->fence);
+  for (hipEvent_t event : {ticket->start, ticket->end, ticket->fence})
+    if (event) ticket->backend->giveEvent(event);
   releaseAll(ticket->retained);
   delete ticket;
 }
@@ -237,8 +291,11 @@ void destroyTicket(sp_ticket *ticket) {
 // Waits for the ticket's end event under the command watchdog (CommandWatchdog.hpp:16-44).
 sp_status awaitTicket(sp_ticket *ticket) {
   sp_backend *backend = ticket->backend;
+  // A step is waited for by its caller, and a sleep ends up to 70 us late: the wait polls for as long as a step or a prompt
+  // chunk takes before it sleeps.
+  constexpr auto kPolls = std::chrono::milliseconds(20);
   const auto begin = Clock::now();
-  uint32_t spins = 0;
+  uint32_t sleeps = 0;
   for (;;) {
     const hipError_t e = hipEventQuery(ticket->fence ? ticket->fence : ticket->end);
     if (e == hipSuccess) return SP_OK;
@@ -246,12 +303,13 @@ sp_status awaitTicket(sp_ticket *ticket) {
       backend->markUnhealthy(std::string("command failed: ") + hipGetErrorString(e));
       return hipFail(e, "command");
     }
-    if (std::chrono::duration<double>(Clock::now() - begin).count() > backend->timeout) {
+    const auto waited = Clock::now() - begin;
+    if (std::chrono::duration<double>(waited).count() > backend->timeout) {
       backend->markUnhealthy("command watchdog: no completion within the command timeout");
       return fail(SP_TIMEOUT, "command watchdog: no completion within the command timeout");
     }
-    if (++spins < 2000) std::this_thread::yield();
-    else std::this_thread::sleep_for(std::chrono::microseconds(spins < 20000 ? 20 : 500));
+    if (waited < kPolls) std::this_thread::yield();
+    else std::this_thread::sleep_for(std::chrono::microseconds(++sleeps < 20000 ? 20 : 500));
   }
 }
 
@@ -304,7 +362,12 @@ void sp_backend_destroy(sp_backend *backend) {
   (void)hipSetDevice(backend->device);
   (void)hipStreamSynchronize(backend->stream);
   (void)hipStreamDestroy(backend->stream);
-  backend->stream = nullptr;
+  {
+    std::lock_guard<std::mutex> lock(backend->mutex);
+    backend->stream = nullptr;
+    for (hipEvent_t event : backend->spareEvents) (void)hipEventDestroy(event);
+    backend->spareEvents.clear();
+  }
   backend->stopped = true;
   // Buffers still alive keep the backend's bookkeeping; their memory is freed as they are released.
   backend->release();
@@ -485,10 +548,11 @@ sp_status sp_submit(sp_backend *backend, const sp_dispatch *dispatches, uint32_t
   if (!dispatches && count) return fail(SP_INVALID_ARGUMENT, "null dispatches");
   // Every dispatch is validated before any is launched (the reference's operators and backend
   // throw before anything is encoded).
-  std::vector<RecordedDispatch> recorded(count);
+  std::vector<const KernelEntry *> kernels(count);
   std::vector<sp_buffer *> retained;
+  retained.reserve(size_t{count} * 8);
   for (uint32_t i = 0; i < count; ++i)
-    if (sp_status s = validateDispatch(dispatches[i], i, recorded[i], retained, backend)) return s;
+    if (sp_status s = validateDispatch(dispatches[i], i, kernels[i], retained, backend)) return s;
   (void)hipSetDevice(backend->device);
   const bool profile = backend->profiling;
   sp_ticket *ticket = nullptr;
@@ -499,7 +563,7 @@ sp_status sp_submit(sp_backend *backend, const sp_dispatch *dispatches, uint32_t
   hipError_t e = hipEventRecord(ticket->start, backend->stream);
   for (uint32_t i = 0; e == hipSuccess && i < count; ++i) {
     if (profile) e = hipEventRecord(ticket->marks[i], backend->stream);
-    if (e == hipSuccess) e = launchRecorded(backend, recorded[i]);
+    if (e == hipSuccess) e = launchDispatch(backend, dispatches[i], kernels[i]);
   }
   if (e == hipSuccess && profile) e = hipEventRecord(ticket->marks[count], backend->stream);
   if (e == hipSuccess) e = hipEventRecord(ticket->end, backend->stream);
@@ -556,11 +620,14 @@ sp_status sp_command_create(sp_backend *backend, const sp_dispatch *dispatches, 
   auto *command = new sp_command;
   command->backend = backend;
   command->dispatches.resize(count);
-  for (uint32_t i = 0; i < count; ++i)
-    if (sp_status s = validateDispatch(dispatches[i], i, command->dispatches[i], command->retained, backend)) {
+  for (uint32_t i = 0; i < count; ++i) {
+    const KernelEntry *kernel = nullptr;
+    if (sp_status s = validateDispatch(dispatches[i], i, kernel, command->retained, backend)) {
       delete command;
       return s;
     }
+    command->dispatches[i] = recordDispatch(dispatches[i], kernel);
+  }
   retainAll(command->retained);
   (void)hipSetDevice(backend->device);
   hipError_t e = hipStreamBeginCapture(backend->stream, hipStreamCaptureModeThreadLocal);

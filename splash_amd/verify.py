@@ -142,7 +142,7 @@ class DenseVerify:
         """A prompt chunk's inputs: its tokens, a chain of tree rows a block of sixteen, each row's depth in its block."""
         tokens = np.asarray(tokens, dtype=np.uint32)
         blocks = [min(16, tokens.size - at) for at in range(0, tokens.size, 16)]
-        self.set_block([Lane(rows, 0) for rows in blocks], tokens)
+        self._write_block(tokens, ops.chain_tree_rows(blocks))
 
     def set_block(self, lanes, tokens, tree_rows=None, uniforms=None):
         """Writes the step's host-visible inputs: packed input tokens, tree rows (chains by default), depths."""
@@ -150,11 +150,23 @@ class DenseVerify:
         tokens = np.asarray(tokens, dtype=np.uint32)
         assert tokens.size == rows
         tree = tree_rows if tree_rows is not None else ops.chain_tree_rows([l.rows for l in lanes])
-        self.buffer(INPUT_TOKENS).contents()[:rows * 4] = tokens.view(np.uint8)
-        self.buffer(TREE_ROWS).contents()[:rows * 8] = tree.view(np.uint8)
-        self.buffer(DEPTHS).contents()[:rows * 4] = tree["depth"].astype(np.uint32).view(np.uint8)
+        self._write_block(tokens, tree)
         if uniforms is not None:
-            self.buffer(UNIFORMS).contents()[:rows * 8] = np.asarray(uniforms, dtype=np.float32).reshape(rows, 2).view(np.uint8).ravel()
+            self._input(UNIFORMS)[:rows * 8] = np.asarray(uniforms, dtype=np.float32).reshape(rows, 2).view(np.uint8).ravel()
+
+    def _input(self, which):
+        """The host view of one of the driver's input buffers, which are allocated with it and stay where they are."""
+        views = self.__dict__.setdefault("_inputs", {})
+        if which not in views:
+            buffer = self.buffer(which)
+            views[which] = (buffer.contents(), buffer)
+        return views[which][0]
+
+    def _write_block(self, tokens, tree):
+        rows = tokens.size
+        self._input(INPUT_TOKENS)[:rows * 4] = tokens.view(np.uint8)
+        self._input(TREE_ROWS)[:rows * 8] = tree.view(np.uint8)
+        self._input(DEPTHS)[:rows * 4] = tree["depth"].astype(np.uint32).view(np.uint8)
 
     _results_call = "spo_dense_verify_results"
 
@@ -193,11 +205,10 @@ class DenseVerify:
         from the driver's buffers after the step's command completed and checked as Runtime::finalizeDecode checks them
         (a SplashError names the lane and the rule a result breaks)."""
         rows, n = sum(l.rows for l in lanes), len(lanes)
-        tokens = np.zeros(rows, np.uint32)
-        retained, accepted, mask = (np.zeros(n, np.uint32) for _ in range(3))
-        p = lambda a: a.ctypes.data_as(ctypes.POINTER(ctypes.c_uint32))
-        check(getattr(lib, self._results_call)(self.handle, self._lanes(lanes), n, p(tokens), p(retained), p(accepted), p(mask)))
-        return tokens, retained, accepted, mask
+        tokens, per_lane = np.zeros(rows, np.uint32), np.zeros((3, n), np.uint32)
+        t, p = (ctypes.c_uint32 * rows).from_buffer(tokens), [(ctypes.c_uint32 * n).from_buffer(per_lane, 4 * n * i) for i in range(3)]
+        check(getattr(lib, self._results_call)(self.handle, self._lanes(lanes), n, t, *p))
+        return tokens, *per_lane
 
 
 class HybridLane(Lane):
@@ -359,6 +370,8 @@ class HybridVerify:
 
     set_block = DenseVerify.set_block
     set_prefill_block = DenseVerify.set_prefill_block
+    _input = DenseVerify._input
+    _write_block = DenseVerify._write_block
     results = DenseVerify.results
     _results_call = "spo_hybrid_verify_results"
 
