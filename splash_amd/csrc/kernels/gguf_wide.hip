@@ -10,11 +10,15 @@
 // 2^-28 of its row's largest. The fp32 sums of 768 inputs lie 4 to 12 times closer to 64-bit ones than the decode kernels'.
 //
 // Split: a wave owns 32 columns (a record of two column tiles each super-block, dequantized once in its registers) of
-// all of the workgroup's 128 rows, whose operands pass through LDS two groups at a time, double-buffered, one barrier
-// each. Two waves a SIMD (256 registers) overlap the conversion of one with the MFMAs of the other. At 2048 rows of the
-// 5120 x 2 x 25600 Q4_K gate/up pair a launch takes 1.25 ms (860 TFLOP/s of the projection's own operations; the 64-row
-// windows of the decode kernels took 2.38 ms), at 25600 x 5120 Q6_K 0.96 ms (2.2 ms): the matrix cores are busy 47 % and
-// 56 % of the cycles of a clock that the card's power limit holds at 2.0 and 1.9 GHz.
+// all of the workgroup's 128 rows, whose operands go from memory straight into LDS, three stages of two groups ahead of
+// their use in four buffers, one barrier a stage. (Through registers, one stage ahead, which is what 256 of them leave
+// room for, waves waited a quarter of their time: gate/up 1.27, the SwiGLU rows' projection 0.97 ms where it is 1.18 and
+// 0.91 now; an expert's tiles, whose rows come from further away, 215 and 158 us where they take 192 and 149. A row
+// tile's operands read two tiles ahead, or waves of a priority that follows the phase, changed nothing.) Two waves a SIMD
+// overlap the conversion of one with the MFMAs of the other. At 2048 rows of the 5120 x 2 x 25600 Q4_K gate/up pair a
+// launch takes 1.18 ms (906 TFLOP/s of the projection's own operations; the 64-row windows of the decode kernels took
+// 2.38 ms), at 25600 x 5120 Q6_K 0.91 ms (2.2 ms): with the constant terms and the second product that is 1.02 and 1.18
+// PFLOP/s of MFMAs, where a large library product reaches 1.19 under the card's power limit.
 #include "abi/Gguf.h"
 #include "abi/Moe.h"
 #include "backend/KernelRegistry.hpp"
@@ -330,10 +334,16 @@ __device__ __forceinline__ WideOperands<FMT> wide_staged_operands(const WideReco
   return out;
 }
 
-template <uint32_t T> struct WideShared {
-  uint4 rows[2][(T + 1) / 2 * 2][2][64];   // [buffer][row tile][group][lane]
-  uint4 sums[(T + 3) / 4 * 4][64];
-};
+// Sixteen bytes a lane of a wave, from memory straight into LDS (`to` the wave's first lane's, the others after it).
+typedef __attribute__((address_space(3))) void LdsVoid;
+__device__ __forceinline__ void load_to_lds(Resource r, uint32_t offset, uint4 *to) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LdsVoid *)to, 16, int(offset), 0, 0, 0);
+}
+// Vector-memory instructions that may be in flight behind a wait (s_waitcnt's vmcnt alone).
+template <uint32_t N> __device__ __forceinline__ void wait_loads() {
+  static_assert(N < 64, "vmcnt has six bits");
+  __builtin_amdgcn_s_waitcnt((N & 15u) | ((N >> 4) << 14) | 0x0F70u);
+}
 
 // What a workgroup computes: its wave's two column tiles (image null: a tile past the last), its row tiles, its part of K.
 struct WideTile {
@@ -384,7 +394,10 @@ __device__ __forceinline__ void wide_workgroup(const WideTile &w, const uint8_t 
                                                const uint16_t *__restrict__ residual, const GgufWideParams &p) {
   constexpr uint32_t kRecord = gguf_record_bytes(FMT);
   constexpr bool kSums = FMT != GGUF_FMT_Q6K && !Staged, kTwice = FMT == GGUF_FMT_Q6K && !Staged, kGateUp = EP == GGUF_WIDE_GATE_UP;
-  __shared__ WideShared<T> shared;
+  // A super-block's four stages, each [row tile][group][lane], and its sums: objects of their own, so that a read of one
+  // does not wait for what is on its way into another.
+  constexpr uint32_t kTiles = (T + 1) / 2 * 2, kStageVectors = kTiles * 2 * 64;
+  __shared__ uint4 rows0[kStageVectors], rows1[kStageVectors], rows2[kStageVectors], rows3[kStageVectors], sums[kSums ? (T + 3) / 4 * 4 * 64 : 1];
   const uint32_t lane = threadIdx.x & 63u, c = lane & 15u, kq = lane >> 4;
   const uint32_t tile0 = w.tile0, tilesHere = w.tilesHere, b0 = w.b0, count = w.count, split = w.split;
   const uint32_t column[2] = {w.column[0], w.column[1]};
@@ -404,32 +417,24 @@ __device__ __forceinline__ void wide_workgroup(const WideTile &w, const uint8_t 
     for (uint32_t t = 0; t < T; ++t) acc[r][t] = dot[r][t] = zero;
 
   // Stage n holds groups 2 (n % 4), 2 (n % 4) + 1 of super-block n / 4 (and with a super-block's last, its sums): this
-  // thread's vectors of it, four (six) of 16 bytes.
-  constexpr uint32_t kShare = (T + 1) / 2, kSumShare = (T + 3) / 4;
-  uint4 held[kShare], heldSums[kSumShare];
+  // wave's share of it, four (six) kilobytes, on its way into LDS three stages ahead of its use.
+  constexpr uint32_t kShare = (T + 1) / 2, kSumShare = kSums ? (T + 3) / 4 : 0;
+  const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)));
   const uint32_t mineAt = (threadIdx.x >> 7) * tileBytes + (threadIdx.x & 127u) * 16u;
   const uint32_t sumsAt = (threadIdx.x >> 6) * tileBytes + lane * 16u;
-  auto fetch = [&](uint32_t block, uint32_t stage) {   // block counts from b0
-    const uint32_t at = (b0 + block) * (GGUF_WIDE_OPERANDS * 1024u) + stage * 2048u;
-#pragma unroll
-    for (uint32_t i = 0; i < kShare; ++i) {
-      const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rowValues, int(mineAt + (at + 2u * i * tileBytes)), 0, 0);
-      held[i] = make_uint4(v.x, v.y, v.z, v.w);
-    }
-    if (kSums && stage == 3u) {
-#pragma unroll
-      for (uint32_t i = 0; i < kSumShare; ++i) {
-        const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rowValues, int(sumsAt + (at + 2048u + 4u * i * tileBytes)), 0, 0);
-        heldSums[i] = make_uint4(v.x, v.y, v.z, v.w);
-      }
-    }
+  auto stageRows = [&](auto stageConstant) __attribute__((always_inline)) -> uint4 * {
+    constexpr uint32_t S = decltype(stageConstant)::value;
+    return S == 0 ? rows0 : S == 1 ? rows1 : S == 2 ? rows2 : rows3;
   };
-  auto store = [&](uint32_t buffer, uint32_t stage) {
+  auto fetch = [&](uint32_t block, auto stageConstant) __attribute__((always_inline)) {   // block counts from b0
+    constexpr uint32_t S = decltype(stageConstant)::value;
+    const uint32_t at = block < count ? (b0 + block) * (GGUF_WIDE_OPERANDS * 1024u) + S * 2048u : 0x80000000u;   // (past the part of K: zeros, no traffic)
+    uint4 *to = stageRows(stageConstant) + 64u * wave;
 #pragma unroll
-    for (uint32_t i = 0; i < kShare; ++i) (&shared.rows[buffer][0][0][0])[threadIdx.x + 256u * i] = held[i];
-    if (kSums && stage == 3u) {
+    for (uint32_t i = 0; i < kShare; ++i) load_to_lds(rowValues, mineAt + (at + 2u * i * tileBytes), to + 256u * i);
+    if constexpr (S == 3u) {
 #pragma unroll
-      for (uint32_t i = 0; i < kSumShare; ++i) (&shared.sums[0][0])[threadIdx.x + 256u * i] = heldSums[i];
+      for (uint32_t i = 0; i < kSumShare; ++i) load_to_lds(rowValues, sumsAt + (at + 2048u + 4u * i * tileBytes), sums + 64u * wave + 256u * i);
     }
   };
   // A record's first half (and what both share) is fetched two stages ahead of its use, and so is its second.
@@ -448,22 +453,40 @@ __device__ __forceinline__ void wide_workgroup(const WideTile &w, const uint8_t 
     for (uint32_t r = 0; r < 2; ++r) rec[r].codes[1] = load128<kStreamOnce>(weights[r], mine + 1024u);
     mine += kRecord;
   };
+  // What a stage's loads are: its rows' (three stages ahead), then the weights'. A stage's rows are there when at most what
+  // was asked for after them is on its way.
+  constexpr uint32_t kFirst = FMT == GGUF_FMT_Q6K ? 6u : 4u, kLate = FMT == GGUF_FMT_Q4K ? 0u : 2u, kSecond = 2u;
+  constexpr auto weightLoads = [](uint32_t stage) constexpr { return stage == 0 ? kSecond : stage == 2u ? kFirst : stage == 3u ? kLate : 0u; };
+  constexpr auto rowLoads = [](uint32_t stage) constexpr { return kShare + (stage == 3u ? kSumShare : 0u); };
+  // (the loads before the first stage in the order of the stages that would have asked for them)
+  fetch(0, std::integral_constant<uint32_t, 0>{});
+  __builtin_amdgcn_sched_barrier(0);
+  fetch(0, std::integral_constant<uint32_t, 1>{});
+  __builtin_amdgcn_sched_barrier(0);
   fetchFirst();
+  __builtin_amdgcn_sched_barrier(0);
+  fetch(0, std::integral_constant<uint32_t, 2>{});
+  __builtin_amdgcn_sched_barrier(0);
   fetchLate();
-  fetch(0, 0);
-  store(0, 0);
-  fetch(0, 1);
-  __syncthreads();
+  __builtin_amdgcn_sched_barrier(0);
   for (uint32_t block = 0; block < count; ++block) {
     WideScales<FMT> scales[2];
 #pragma unroll
     for (uint32_t r = 0; r < 2; ++r) scales[r] = wide_scales(rec[r]);
     auto run = [&](auto stageConstant) {
       constexpr uint32_t S = decltype(stageConstant)::value;
-      store((S + 1u) & 1u, (S + 1u) & 3u);
-      fetch(block + (S >= 2u ? 1u : 0u), (S + 2u) & 3u);
+      // (behind stage S's rows: the weights of that stage and the two after it, and the two stages' rows between)
+      wait_loads<weightLoads((S + 1u) & 3u) + rowLoads((S + 1u) & 3u) + weightLoads((S + 2u) & 3u) + rowLoads((S + 2u) & 3u) + weightLoads((S + 3u) & 3u)>();
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      fetch(block + (S >= 1u ? 1u : 0u), std::integral_constant<uint32_t, (S + 3u) & 3u>{});
+      __builtin_amdgcn_sched_barrier(0);
       if constexpr (S == 0) fetchSecond();
       if constexpr (S == 2u) fetchFirst();
+      __builtin_amdgcn_sched_barrier(0);
+      const uint4 *rows = stageRows(stageConstant);
       WideOperands<FMT> operands[2];
 #pragma unroll
       for (uint32_t r = 0; r < 2; ++r) {
@@ -475,14 +498,14 @@ __device__ __forceinline__ void wide_workgroup(const WideTile &w, const uint8_t 
 #pragma unroll
         for (uint32_t r = 0; r < 2; ++r) mins[r] = wide_mins(scales[r]);
       }
-      if constexpr (S == 3u) fetchLate();
+      if constexpr (S == 3u) fetchLate();   // (over the bits that the last operands were made of)
       // A row tile's operands leave LDS while the tile before it is multiplied.
       constexpr uint32_t kReads = S == 3u && kSums ? 3u : 2u;
       f16x8 a[2][3];
       auto read = [&](uint32_t t) {
 #pragma unroll
-        for (uint32_t g = 0; g < 2; ++g) a[t & 1u][g] = as_f16x8(shared.rows[S & 1u][t][g][lane]);
-        if constexpr (kReads == 3u) a[t & 1u][2] = as_f16x8(shared.sums[t][lane]);
+        for (uint32_t g = 0; g < 2; ++g) a[t & 1u][g] = as_f16x8(rows[(t * 2u + g) * 64u + lane]);
+        if constexpr (kReads == 3u) a[t & 1u][2] = as_f16x8(sums[t * 64u + lane]);
       };
       read(0);
 #pragma unroll
@@ -520,7 +543,6 @@ __device__ __forceinline__ void wide_workgroup(const WideTile &w, const uint8_t 
         if (t + 1 < T) __builtin_amdgcn_sched_group_barrier(0x100, kReads, 0);
         __builtin_amdgcn_sched_group_barrier(0x008, kProducts, 0);
       }
-      __syncthreads();
       __builtin_amdgcn_sched_barrier(0);
     };
     run(std::integral_constant<uint32_t, 0>{});
@@ -534,6 +556,7 @@ __device__ __forceinline__ void wide_workgroup(const WideTile &w, const uint8_t 
 #pragma unroll
       for (uint32_t t = 0; t < T; ++t) acc[r][t] = dot[r][t];
   }
+  wait_loads<0>();   // (nothing is on its way into LDS when the workgroup gives it up)
   // Element (t, v) of this lane is row 16 (tile0 + t) + 4 kq + v, column column[r] + c.
   const float *inverse = reinterpret_cast<const float *>(table + gguf_wide_scales_offset(p.input_size, p.tiles));
 #pragma unroll
