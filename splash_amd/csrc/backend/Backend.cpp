@@ -171,9 +171,6 @@ struct sp_command {
 
 namespace {
 
-// Every kernel of the registry binds fewer (checked where a dispatch is validated).
-constexpr uint32_t kMostBuffers = 32;
-
 sp_status validateDispatch(const sp_dispatch &d, uint32_t index, const KernelEntry *&found, std::vector<sp_buffer *> &retained,
                            sp_backend *backend) {
   // (the words of a message are put together only where there is one)
@@ -199,7 +196,6 @@ sp_status validateDispatch(const sp_dispatch &d, uint32_t index, const KernelEnt
   if (uint64_t(d.block[0]) * d.block[1] * d.block[2] > 1024)
     return fail(SP_INVALID_ARGUMENT, at + ": more than 1024 threads per workgroup");
   if (d.grid[1] > 65535 || d.grid[2] > 65535) return fail(SP_INVALID_ARGUMENT, at + ": grid y or z beyond 65535");
-  if (d.buffer_count > kMostBuffers) return fail(SP_INVALID_ARGUMENT, at + ": more buffers than a dispatch takes");
   found = kernel;
   for (uint32_t b = 0; b < d.buffer_count; ++b) {
     sp_buffer *buffer = d.buffers[b];
@@ -228,12 +224,12 @@ RecordedDispatch recordDispatch(const sp_dispatch &d, const KernelEntry *kernel)
   for (uint32_t b = 0; b < d.buffer_count; ++b) out.pointers.push_back(d.buffers[b]->device);
   return out;
 }
-// A validated dispatch from the caller's own records.
-hipError_t launchDispatch(sp_backend *backend, const sp_dispatch &d, const KernelEntry *kernel) {
-  void *pointers[kMostBuffers];
-  for (uint32_t b = 0; b < d.buffer_count; ++b) pointers[b] = d.buffers[b]->device;
-  LaunchArgs args{backend->stream, dim3(d.grid[0], d.grid[1], d.grid[2]), dim3(d.block[0], d.block[1], d.block[2]), pointers, d.buffer_count,
-                  d.params, d.params_bytes};
+// A validated dispatch from the caller's own records; `pointers` is the submission's, reused by its dispatches.
+hipError_t launchDispatch(sp_backend *backend, const sp_dispatch &d, const KernelEntry *kernel, std::vector<void *> &pointers) {
+  pointers.clear();
+  for (uint32_t b = 0; b < d.buffer_count; ++b) pointers.push_back(d.buffers[b]->device);
+  LaunchArgs args{backend->stream, dim3(d.grid[0], d.grid[1], d.grid[2]), dim3(d.block[0], d.block[1], d.block[2]), pointers.data(),
+                  d.buffer_count, d.params, d.params_bytes};
   return kernel->launch(args);
 }
 hipError_t launchRecorded(sp_backend *backend, const RecordedDispatch &d) {
@@ -561,9 +557,10 @@ sp_status sp_submit(sp_backend *backend, const sp_dispatch *dispatches, uint32_t
   retainAll(ticket->retained);
   ticket->wallStart = Clock::now();
   hipError_t e = hipEventRecord(ticket->start, backend->stream);
+  std::vector<void *> pointers;
   for (uint32_t i = 0; e == hipSuccess && i < count; ++i) {
     if (profile) e = hipEventRecord(ticket->marks[i], backend->stream);
-    if (e == hipSuccess) e = launchDispatch(backend, dispatches[i], kernels[i]);
+    if (e == hipSuccess) e = launchDispatch(backend, dispatches[i], kernels[i], pointers);
   }
   if (e == hipSuccess && profile) e = hipEventRecord(ticket->marks[count], backend->stream);
   if (e == hipSuccess) e = hipEventRecord(ticket->end, backend->stream);
