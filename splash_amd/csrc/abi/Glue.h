@@ -2,8 +2,10 @@
 // (the reference's abi/RoPE.h, abi/Embedding.h and the `uint width` of its norm kernels).
 #pragma once
 #include <stdint.h>
+#include "abi/Gguf.h"
 
 #define SPLASH_RMS_EPSILON 1e-6f
+#define NORM_STAGED_WIDTH 8192u  // columns of a row that a norm holds in LDS
 
 // norm_rms / norm_rms_table16: one workgroup of 256 threads per row. norm_rms_table16 also writes
 // the projection activation table of the normalized rows (abi/Gguf.h), as the reference's
@@ -25,6 +27,13 @@ struct RopeTreeParams {
   uint32_t first_row[8];  // per sequence
   uint32_t row_count[8];
   uint32_t anchor[8];     // position of the sequence's row 0
+};
+
+// gguf_embed_norm_<fmt>: the embedding, first norm and RoPE tables of a step's rows (kernels/glue.hip).
+struct EmbedNormParams {
+  struct GgufEmbedParams embed;
+  uint32_t tiles;  // row tiles of the table
+  struct RopeTreeParams rope;  // pairs 0: no tables
 };
 
 // copy_rows_bf16: `rows` rows of `width` bf16 values between two row regions (the reference's
@@ -57,6 +66,7 @@ struct GgufFloatParams {
 };
 
 #ifdef __cplusplus
+static_assert(sizeof(EmbedNormParams) == 12 + 4 + 16 + 96, "embedding and norm parameters are 128 bytes on both sides");
 static_assert(sizeof(GgufFloatParams) == 32, "float projection parameters are 32 bytes on both sides");
 static_assert(sizeof(RowCopyParams) == 32, "row copy parameters are 32 bytes on both sides");
 static_assert(sizeof(NormParams) == 16, "norm parameters are 16 bytes on both sides");

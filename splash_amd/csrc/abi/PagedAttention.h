@@ -15,6 +15,7 @@
 // sequence's logical pages to physical ones; its entries are 64-bit (physical page index).
 #pragma once
 #include <stdint.h>
+#include "abi/Sampling.h"
 
 #define ATTENTION_PAGE_TOKENS 256u
 #define ATTENTION_STEP_TOKENS 64u    // tokens the split kernel takes at a time; history splits hold whole steps
@@ -113,9 +114,17 @@ struct AttentionCommitParams {
   struct AttentionSequence sequence[ATTENTION_MAXIMUM_SEQUENCES];
 };
 
+// attention_q8_accept_commit_d<D>: the acceptance of a step's greedy rows and the commit of the path it keeps.
+struct AttentionAcceptCommitParams {
+  struct AttentionCommitParams commit;
+  uint32_t remaining[ATTENTION_MAXIMUM_SEQUENCES];  // AcceptBatchParams of the lanes that are the sequences
+  uint32_t stop_tokens[SAMPLING_STOP_TOKENS];
+};
+
 #ifdef __cplusplus
 static_assert(sizeof(AttentionTreeRow) == 8, "a tree row is 8 bytes on both sides");
 static_assert(sizeof(AttentionSequence) == 16, "an attention sequence is 16 bytes on both sides");
 static_assert(sizeof(AttentionParams) == 56 + 16 * ATTENTION_MAXIMUM_SEQUENCES, "attention parameters are 184 bytes on both sides");
 static_assert(sizeof(AttentionCommitParams) == 32 + 16 * ATTENTION_MAXIMUM_SEQUENCES, "commit parameters are 160 bytes on both sides");
+static_assert(sizeof(AttentionAcceptCommitParams) == 160 + 32 + 16, "accepting commit parameters are 208 bytes on both sides");
 #endif

@@ -7,11 +7,13 @@
 #include "backend/KernelRegistry.hpp"
 #include "kernels/device_common.hpp"
 
+#include <type_traits>
+
 namespace splash::kernels {
 
 // Rows of up to kStagedWidth columns are staged in LDS with every global load in flight at once
 // (a row's columns are read twice, in an order no vector load gives directly).
-constexpr uint32_t kStagedWidth = 8192;
+constexpr uint32_t kStagedWidth = NORM_STAGED_WIDTH;
 
 // Copies `width` bf16 values (a multiple of 8, 16-byte aligned) to LDS; no barrier.
 __device__ __forceinline__ void stage_row(const uint16_t *__restrict__ source, uint32_t width, uint16_t *lds) {
@@ -19,8 +21,8 @@ __device__ __forceinline__ void stage_row(const uint16_t *__restrict__ source, u
   uint4 held[kStagedWidth / 8u / 256u];
 #pragma unroll
   for (uint32_t i = 0; i < kStagedWidth / 8u / 256u; ++i) {
-    const uint32_t v = threadIdx.x + 256u * i;
-    if (v < vectors) held[i] = reinterpret_cast<const uint4 *>(source)[v];
+    // (the last vector again past the row's end: a read under a condition is waited for before the next and kept in scratch)
+    held[i] = reinterpret_cast<const uint4 *>(source)[min(threadIdx.x + 256u * i, vectors - 1u)];
   }
 #pragma unroll
   for (uint32_t i = 0; i < kStagedWidth / 8u / 256u; ++i) {
@@ -133,7 +135,7 @@ __device__ __forceinline__ void write_table_row(const uint16_t *x, const uint16_
 
 // The same, and the activation table of the normalized rows: grid (tiles * 16) so that the rows
 // past the live ones are written as zeros. A handful of workgroups that only wait: every loop keeps several reads in
-// flight (8.7 us at 8 rows of 5120 either way).
+// flight (6.4 us at 128 rows of 2048 while a staged row's reads waited for one another, 5.8 since).
 __global__ __launch_bounds__(256) void norm_rms_table16(const uint16_t *__restrict__ input, const uint16_t *__restrict__ weight,
                                                         uint16_t *__restrict__ output, uint8_t *__restrict__ table, NormParams p) {
   __shared__ float scratch[4];
@@ -159,8 +161,8 @@ SP_REGISTER_KERNEL("norm_rms_table16", &norm_rms_table16);
 // draft_conv (draft_attention.hip) and the pass that reads its rows, one workgroup a row: a Prepare stage's rows and their
 // activation table; a Residual stage's rows, their RMS norm (of `norm_weight`, into `normalized`) and its table. Each
 // convolution was a launch of its own before a launch of as few workgroups. Values and their order are the two kernels'.
-// The rows' 16-byte accesses are the host's rule (DraftAttention::addConvolutionTable). 8 rows of 5120: 5.3 us
-// for 3.1 + 3.0, 8.9 us for 3.1 + 8.7, and a launch less each: the draft model's pass of one lane 928, 923 and 938 us
+// The rows' 16-byte accesses are the host's rule (DraftAttention::addConvolutionTable). 8 rows of 5120: 5.2 us
+// for 3.1 + 3.0, 8.3 us for 3.1 + 8.7, and a launch less each: the draft model's pass of one lane 928, 923 and 938 us
 // before, 869, 888 and 889 after, in three runs of both sides in turn whose repeats differ by 1 to 2 %.
 template <bool Residual>
 __global__ __launch_bounds__(256) void draft_conv_table(const uint16_t *__restrict__ input, const uint16_t *__restrict__ dynamic,
@@ -261,16 +263,20 @@ __global__ __launch_bounds__(256) void swiglu_rows(const uint16_t *__restrict__ 
 }
 SP_REGISTER_KERNEL("swiglu_rows", &swiglu_rows);
 
-__global__ void rope_build_tree_tables(const float *__restrict__ inverse_frequency, const uint32_t *__restrict__ depth,
-                                       float *__restrict__ cosines, float *__restrict__ sines, RopeTreeParams p) {
-  const uint32_t row = blockIdx.x, pair = threadIdx.x;
-  if (row >= p.rows || pair >= p.pairs) return;
+__device__ __forceinline__ void rope_entry(uint32_t row, uint32_t pair, const float *__restrict__ inverse_frequency,
+                                           const uint32_t *__restrict__ depth, float *__restrict__ cosines, float *__restrict__ sines,
+                                           const RopeTreeParams &p) {
   uint32_t anchor = 0;
   for (uint32_t s = 0; s < p.sequences; ++s)
     if (row >= p.first_row[s] && row < p.first_row[s] + p.row_count[s]) anchor = p.anchor[s];
   const float angle = float(anchor + depth[row]) * inverse_frequency[pair];
   cosines[size_t(row) * p.pairs + pair] = cosf(angle);
   sines[size_t(row) * p.pairs + pair] = sinf(angle);
+}
+__global__ void rope_build_tree_tables(const float *__restrict__ inverse_frequency, const uint32_t *__restrict__ depth,
+                                       float *__restrict__ cosines, float *__restrict__ sines, RopeTreeParams p) {
+  const uint32_t row = blockIdx.x, pair = threadIdx.x;
+  if (row < p.rows && pair < p.pairs) rope_entry(row, pair, inverse_frequency, depth, cosines, sines, p);
 }
 SP_REGISTER_KERNEL("rope_build_tree_tables", &rope_build_tree_tables);
 
@@ -324,47 +330,30 @@ SP_REGISTER_KERNEL("gguf_float_f32_bf16", (&gguf_float<false, true>));
 SP_REGISTER_KERNEL("gguf_float_bf16_f32", (&gguf_float<true, false>));
 SP_REGISTER_KERNEL("gguf_float_bf16_bf16", (&gguf_float<true, true>));
 
-// gguf_embed_<fmt>: out[r][:] = bf16(decode(native row tokens[r])); a token at or past the
-// vocabulary gives zeros (embedding.metal:10-18). Grid (rows, hidden / 256), 64 threads: a thread
-// decodes four values of a super-block.
-template <uint32_t FMT>
-__global__ __launch_bounds__(64) void gguf_embed(const uint8_t *__restrict__ table, const uint32_t *__restrict__ tokens,
-                                                 uint16_t *__restrict__ out, GgufEmbedParams p) {
-  const uint32_t row = blockIdx.x, block = blockIdx.y, tid = threadIdx.x;
-  const uint32_t token = tokens[row];
-  uint16_t *o = out + size_t(row) * p.hidden + size_t(block) * 256u;
-  if (token >= p.vocabulary) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) o[tid + 64 * i] = 0;
-    return;
-  }
-  const uint32_t blocks = p.hidden / 256u;
-  if constexpr (FMT == GGUF_FMT_Q4K || FMT == GGUF_FMT_Q5K) {
-    constexpr bool kFifth = FMT == GGUF_FMT_Q5K;   // Q5_K: 32 bytes of fifth bits between the scales and the nibbles
-    const uint8_t *blk = table + (size_t(token) * blocks + block) * (kFifth ? GGUF_Q5K_NATIVE : GGUF_Q4K_NATIVE);
-    const float d = half_bits_to_float(blk[0] | (blk[1] << 8)), dmin = half_bits_to_float(blk[2] | (blk[3] << 8));
-    const uint8_t *sc = blk + 4, *qh = blk + 16, *qs = blk + (kFifth ? 48 : 16);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t k = tid + 64u * i, j = k / 32u, e = k % 32u;
-      uint32_t s, m;
-      if (j < 4) { s = sc[j] & 63u; m = sc[j + 4] & 63u; }
-      else { s = (sc[j + 4] & 0xFu) | ((sc[j - 4] >> 6) << 4); m = (sc[j + 4] >> 4) | ((sc[j] >> 6) << 4); }
+// Input k of a native super-block of 256 (embedding.metal:10-18).
+template <uint32_t FMT> struct EmbedBlock {
+  static constexpr uint32_t kBytes = FMT == GGUF_FMT_Q4K ? GGUF_Q4K_NATIVE : FMT == GGUF_FMT_Q5K ? GGUF_Q5K_NATIVE : FMT == GGUF_FMT_Q6K ? GGUF_Q6K_NATIVE
+                                   : FMT == GGUF_FMT_Q80 ? GGUF_Q80_NATIVE : FMT == GGUF_FMT_IQ4XS ? GGUF_IQ4XS_NATIVE : GGUF_IQ4NL_NATIVE;
+  static __device__ __forceinline__ uint32_t bits(const uint8_t *__restrict__ blk, uint32_t k) {
+    const uint32_t j = k / 32u, e = k % 32u;
+    if constexpr (FMT == GGUF_FMT_Q4K || FMT == GGUF_FMT_Q5K) {
+      constexpr bool kFifth = FMT == GGUF_FMT_Q5K;   // Q5_K: 32 bytes of fifth bits between the scales and the nibbles
+      const float d = half_bits_to_float(blk[0] | (blk[1] << 8)), dmin = half_bits_to_float(blk[2] | (blk[3] << 8));
+      const uint8_t *sc = blk + 4, *qh = blk + 16, *qs = blk + (kFifth ? 48 : 16);
+      // groups 0..3: six bits of bytes j and j + 4; groups 4..7: the halves of byte j + 4 and two bits of bytes j - 4 and j
+      // (by masks, so that no branch stands between a thread's loads)
+      const bool low = j < 4u;
+      const uint32_t keep = low ? 63u : 15u, top = low ? 0u : 48u, shift = low ? 0u : 4u, both = sc[j + 4u];
+      const uint32_t s = (sc[j + shift] & keep) | ((sc[j & 3u] >> 2) & top), m = ((both >> shift) & keep) | ((sc[(j & 3u) + 4u] >> 2) & top);
       uint32_t code = (qs[32u * (j / 2u) + e] >> (4u * (j % 2u))) & 15u;
       if constexpr (kFifth) code |= ((qh[e] >> j) & 1u) << 4;
-      o[k] = uint16_t(float_to_bf16_bits(__fmaf_rn(d * float(s), float(code), -(dmin * float(m)))));
-    }
-  } else if constexpr (FMT == GGUF_FMT_IQ4XS || FMT == GGUF_FMT_IQ4NL) {
-    // value = scale * codebook[nibble]: byte e % 16 of the group's 16 holds inputs e (low nibble) and 16 + e (high)
-    constexpr int kCodebook[16] = {-127, -104, -83, -65, -49, -35, -22, -10, 1, 13, 25, 38, 53, 69, 89, 113};
-    constexpr bool kXs = FMT == GGUF_FMT_IQ4XS;
-    const uint8_t *blk = table + (size_t(token) * blocks + block) * (kXs ? GGUF_IQ4XS_NATIVE : GGUF_IQ4NL_NATIVE);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t k = tid + 64u * i, j = k / 32u, e = k % 32u;
+      return float_to_bf16_bits(__fmaf_rn(d * float(s), float(code), -(dmin * float(m))));
+    } else if constexpr (FMT == GGUF_FMT_IQ4XS || FMT == GGUF_FMT_IQ4NL) {
+      // value = scale * codebook[nibble]: byte e % 16 of the group's 16 holds inputs e (low nibble) and 16 + e (high)
+      constexpr int kCodebook[16] = {-127, -104, -83, -65, -49, -35, -22, -10, 1, 13, 25, 38, 53, 69, 89, 113};
       float scale;
       const uint8_t *qs;
-      if constexpr (kXs) {
+      if constexpr (FMT == GGUF_FMT_IQ4XS) {
         const uint32_t high = blk[2] | (blk[3] << 8), ls = ((blk[4u + j / 2u] >> (4u * (j % 2u))) & 15u) | (((high >> (2u * j)) & 3u) << 4);
         scale = half_bits_to_float(blk[0] | (blk[1] << 8)) * float(int(ls) - 32);
         qs = blk + 8u + 16u * j;
@@ -373,29 +362,33 @@ __global__ __launch_bounds__(64) void gguf_embed(const uint8_t *__restrict__ tab
         qs = blk + 18u * j + 2u;
       }
       const uint32_t code = e < 16u ? qs[e] & 15u : qs[e - 16u] >> 4;
-      o[k] = uint16_t(float_to_bf16_bits(scale * float(kCodebook[code])));
-    }
-  } else if constexpr (FMT == GGUF_FMT_Q80) {
-    const uint8_t *blk = table + (size_t(token) * blocks + block) * GGUF_Q80_NATIVE;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t k = tid + 64u * i, j = k / 32u, e = k % 32u;
+      return float_to_bf16_bits(scale * float(kCodebook[code]));
+    } else if constexpr (FMT == GGUF_FMT_Q80) {
       const uint8_t *group = blk + 34u * j;
       const float d = half_bits_to_float(group[0] | (group[1] << 8));
-      o[k] = uint16_t(float_to_bf16_bits(d * float(int(int8_t(group[2u + e])))));
-    }
-  } else {
-    const uint8_t *blk = table + (size_t(token) * blocks + block) * GGUF_Q6K_NATIVE;
-    const float d = half_bits_to_float(blk[208] | (blk[209] << 8));
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t k = tid + 64u * i, n = k / 128u, r = (k % 128u) / 32u, e = k % 32u;
+      return float_to_bf16_bits(d * float(int(int8_t(group[2u + e]))));
+    } else {
+      const float d = half_bits_to_float(blk[208] | (blk[209] << 8));
+      const uint32_t n = k / 128u, r = (k % 128u) / 32u;
       const uint32_t l4 = (blk[64u * n + e + 32u * (r & 1u)] >> (4u * (r >> 1))) & 15u, h2 = (blk[128u + 32u * n + e] >> (2u * r)) & 3u;
       const int q = int(l4 | (h2 << 4)) - 32;
       const float scale = float(int(int8_t(blk[192u + 8u * n + 2u * r + e / 16u])));
-      o[k] = uint16_t(float_to_bf16_bits(d * scale * float(q)));
+      return float_to_bf16_bits(d * scale * float(q));
     }
   }
+};
+
+// gguf_embed_<fmt>: out[r][:] = bf16(decode(native row tokens[r])); a token at or past the
+// vocabulary gives zeros. Grid (rows, hidden / 256), 64 threads: a thread decodes four values of a super-block.
+template <uint32_t FMT>
+__global__ __launch_bounds__(64) void gguf_embed(const uint8_t *__restrict__ table, const uint32_t *__restrict__ tokens,
+                                                 uint16_t *__restrict__ out, GgufEmbedParams p) {
+  const uint32_t row = blockIdx.x, block = blockIdx.y, tid = threadIdx.x;
+  const uint32_t token = tokens[row];
+  uint16_t *o = out + size_t(row) * p.hidden + size_t(block) * 256u;
+  const uint8_t *blk = table + (size_t(token) * (p.hidden / 256u) + block) * EmbedBlock<FMT>::kBytes;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) o[tid + 64 * i] = token < p.vocabulary ? uint16_t(EmbedBlock<FMT>::bits(blk, tid + 64u * i)) : uint16_t(0);
 }
 SP_REGISTER_KERNEL("gguf_embed_q4k", &gguf_embed<GGUF_FMT_Q4K>);
 SP_REGISTER_KERNEL("gguf_embed_q6k", &gguf_embed<GGUF_FMT_Q6K>);
@@ -403,5 +396,62 @@ SP_REGISTER_KERNEL("gguf_embed_q5k", &gguf_embed<GGUF_FMT_Q5K>);
 SP_REGISTER_KERNEL("gguf_embed_q80", &gguf_embed<GGUF_FMT_Q80>);
 SP_REGISTER_KERNEL("gguf_embed_iq4xs", &gguf_embed<GGUF_FMT_IQ4XS>);
 SP_REGISTER_KERNEL("gguf_embed_iq4nl", &gguf_embed<GGUF_FMT_IQ4NL>);
+
+// gguf_embed_norm_<fmt>: the first passes of a step as one: rope_build_tree_tables, gguf_embed and norm_rms_table16 of
+// its rows, each the values of its own kernel. Grid (tiles * 16, 2 or 1 without rotary pairs), 256 threads: a workgroup
+// of y = 0 gathers a row into LDS (thread t input t of every super-block), stores it, norms it and writes its part of
+// the activation table (zeros past the live rows); one of y = 1 writes the row's RoPE tables. Rows of up to kStagedWidth
+// columns. Three launches of a few workgroups each that only waited on one another: 3.7 + 4.1 + 5.6 us at 16 rows of 1024
+// columns, 8.3 together (the gather, the sum and the table are one chain of waits), and two launches less a step.
+template <uint32_t FMT>
+__global__ __launch_bounds__(256) void gguf_embed_norm(const uint8_t *__restrict__ embedding, const uint32_t *__restrict__ tokens,
+                                                       const uint16_t *__restrict__ weight, uint16_t *__restrict__ hidden,
+                                                       uint16_t *__restrict__ output, uint8_t *__restrict__ table,
+                                                       const float *__restrict__ inverse_frequency, const uint32_t *__restrict__ depth,
+                                                       float *__restrict__ cosines, float *__restrict__ sines, EmbedNormParams p) {
+  __shared__ float scratch[4];
+  __shared__ __align__(16) uint16_t rowX[kStagedWidth], rowW[kStagedWidth];
+  // a native row in pieces that every format's rows are whole numbers of (a Q6_K block is 210 bytes)
+  using Piece = std::conditional_t<FMT == GGUF_FMT_Q6K, uint16_t, uint32_t>;
+  constexpr uint32_t kNative = kStagedWidth / 256u * EmbedBlock<FMT>::kBytes / sizeof(Piece), kPieces = (kNative + 255u) / 256u;
+  __shared__ __align__(16) Piece native[kNative];
+  const uint32_t row = blockIdx.x, tid = threadIdx.x;
+  const bool live = row < p.embed.rows;
+  if (blockIdx.y) {
+    if (live)
+      for (uint32_t pair = tid; pair < p.rope.pairs; pair += 256u) rope_entry(row, pair, inverse_frequency, depth, cosines, sines, p.rope);
+    return;
+  }
+  float inverse = 0.f;
+  if (live) {
+    const uint32_t token = tokens[row], blocks = p.embed.hidden / 256u;
+    const bool inside = token < p.embed.vocabulary;
+    // the native row whole, with every load in flight at once (a decode's byte loads from memory wait for one another)
+    const uint8_t *source = embedding + size_t(inside ? token : 0u) * blocks * EmbedBlock<FMT>::kBytes;
+    const uint32_t pieces = blocks * EmbedBlock<FMT>::kBytes / uint32_t(sizeof(Piece));
+    Piece held[kPieces];
+#pragma unroll
+    for (uint32_t i = 0; i < kPieces; ++i) __builtin_memcpy(&held[i], source + min(tid + 256u * i, pieces - 1u) * sizeof(Piece), sizeof(Piece));
+    stage_row(weight, p.embed.hidden, rowW);
+#pragma unroll
+    for (uint32_t i = 0; i < kPieces; ++i)
+      if (tid + 256u * i < pieces) native[tid + 256u * i] = held[i];
+    __syncthreads();
+    for (uint32_t b = 0; b < blocks; ++b) {
+      const uint16_t value = inside ? uint16_t(EmbedBlock<FMT>::bits(reinterpret_cast<const uint8_t *>(native) + b * EmbedBlock<FMT>::kBytes, tid)) : uint16_t(0);
+      rowX[b * 256u + tid] = value;
+      hidden[size_t(row) * p.embed.hidden + b * 256u + tid] = value;
+    }
+  }
+  __syncthreads();
+  if (live) inverse = rms_inverse(rowX, p.embed.hidden, scratch);
+  write_table_row<true>(rowX, rowW, inverse, live, row, output, table, p.embed.hidden, p.tiles);
+}
+SP_REGISTER_KERNEL("gguf_embed_norm_q4k", &gguf_embed_norm<GGUF_FMT_Q4K>);
+SP_REGISTER_KERNEL("gguf_embed_norm_q6k", &gguf_embed_norm<GGUF_FMT_Q6K>);
+SP_REGISTER_KERNEL("gguf_embed_norm_q5k", &gguf_embed_norm<GGUF_FMT_Q5K>);
+SP_REGISTER_KERNEL("gguf_embed_norm_q80", &gguf_embed_norm<GGUF_FMT_Q80>);
+SP_REGISTER_KERNEL("gguf_embed_norm_iq4xs", &gguf_embed_norm<GGUF_FMT_IQ4XS>);
+SP_REGISTER_KERNEL("gguf_embed_norm_iq4nl", &gguf_embed_norm<GGUF_FMT_IQ4NL>);
 
 } // namespace splash::kernels

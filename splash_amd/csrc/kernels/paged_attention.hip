@@ -22,6 +22,7 @@
 #include "abi/Gguf.h"
 #include "abi/PagedAttention.h"
 #include "backend/KernelRegistry.hpp"
+#include "kernels/acceptance.hpp"
 #include "kernels/gguf_records.hpp"   // buffer resources
 #include <type_traits>
 
@@ -1056,13 +1057,11 @@ SP_REGISTER_KERNEL("attention_reduce_d64_t", &attention_reduce<64, true>);
 // rows on the accepted path; its k-th set bit (row r) moves from slot committed + r to committed + k.
 // ---------------------------------------------------------------------------------------------
 template <int D>
-__global__ __launch_bounds__(D) void attention_q8_commit(const uint32_t *__restrict__ retained,
-                                                         const uint64_t *__restrict__ page_table, uint8_t *__restrict__ pool,
-                                                         AttentionCommitParams p) {
+__device__ __forceinline__ void commit_path(uint32_t mask, const uint64_t *__restrict__ page_table, uint8_t *__restrict__ pool,
+                                            const AttentionCommitParams &p) {
   const uint32_t tid = threadIdx.x, h = blockIdx.x, z = blockIdx.y;
   const AttentionSequence seq = p.sequence[z];
   pool += uint64_t(blockIdx.z) * p.layer_bytes;
-  uint32_t mask = retained[z];
   uint32_t depth = 0;
   while (mask) {
     const uint32_t r = uint32_t(__builtin_ctz(mask));
@@ -1085,6 +1084,67 @@ __global__ __launch_bounds__(D) void attention_q8_commit(const uint32_t *__restr
     __syncthreads();
   }
 }
+template <int D>
+__global__ __launch_bounds__(D) void attention_q8_commit(const uint32_t *__restrict__ retained,
+                                                         const uint64_t *__restrict__ page_table, uint8_t *__restrict__ pool,
+                                                         AttentionCommitParams p) {
+  commit_path<D>(retained[blockIdx.y], page_table, pool, p);
+}
+
+// attention_q8_accept_commit: decode_sample_argmax_reduce, decode_accept_tree and attention_q8_commit of a step whose
+// rows are all greedy, on the commit's grid: every workgroup reduces the shards' partials of its lane's rows (half a
+// wavefront a row, 4 KB from L2 at most) and walks the block itself, and the first of a lane writes the results the other
+// two kernels leave. Two launches of a few waiting wavefronts less a step:
+// 6.8 us for 2.8 + 4.5 + 4.1 at 16 rows of one lane. (With the ends' other launches, a step of 8 layers of 5120 columns
+// 1296 -> 1286 us.)
+template <int D>
+__global__ __launch_bounds__(D) void attention_q8_accept_commit(const float *__restrict__ partial_values, const uint32_t *__restrict__ partial_indices,
+                                                                const uint32_t *__restrict__ input_tokens, const AttentionTreeRow *__restrict__ tree,
+                                                                uint32_t *__restrict__ tokens, uint32_t *__restrict__ retained,
+                                                                uint32_t *__restrict__ accepted_count, uint32_t *__restrict__ retained_rows,
+                                                                const uint64_t *__restrict__ page_table, uint8_t *__restrict__ pool,
+                                                                AttentionAcceptCommitParams p) {
+  static_assert(SAMPLING_SHARDS == 32, "half a wavefront holds a row's shards");
+  constexpr uint32_t kTogether = D / SAMPLING_SHARDS;   // rows reduced at a time
+  __shared__ uint32_t selections[SAMPLING_MAXIMUM_ROWS];
+  const uint32_t tid = threadIdx.x, z = blockIdx.y;
+  const uint32_t first = p.commit.sequence[z].first_row, rows = min(uint32_t(p.commit.sequence[z].rows), SAMPLING_MAXIMUM_ROWS);
+  const uint32_t row = tid & 63u;   // each wavefront walks the whole block
+  const bool live = row < rows;
+  const AttentionTreeRow node = live ? tree[first + row] : AttentionTreeRow{0u, 0u, 0u};
+  const uint32_t input = live ? input_tokens[first + row] : 0u;
+  Best best[SAMPLING_MAXIMUM_ROWS / kTogether];
+#pragma unroll
+  for (uint32_t i = 0; i < SAMPLING_MAXIMUM_ROWS / kTogether; ++i) {
+    const uint32_t r = i * kTogether + tid / SAMPLING_SHARDS, at = (first + min(r, rows - 1u)) * SAMPLING_SHARDS + tid % SAMPLING_SHARDS;
+    best[i] = {partial_values[at], partial_indices[at]};
+  }
+#pragma unroll
+  for (uint32_t i = 0; i < SAMPLING_MAXIMUM_ROWS / kTogether; ++i) {
+    if (unselectable(best[i].value)) best[i] = {-INFINITY, SAMPLING_NO_TOKEN};
+    best[i] = wave_best<SAMPLING_SHARDS>(best[i]);
+    if (tid % SAMPLING_SHARDS == 0) selections[i * kTogether + tid / SAMPLING_SHARDS] = best[i].index;
+  }
+  __syncthreads();
+  const uint32_t selection = live ? selections[row] : 0u;
+  const Acceptance a = accept_rows(row, live, node, input, selection, p.remaining[z], p.stop_tokens);
+  if (tid < 64u && blockIdx.x == 0 && blockIdx.z == 0) {
+    // the kept path's selections from the lane's first row on, every row past them its own
+    if (live && row >= a.kept) tokens[first + row] = selection;
+    if (a.retains) tokens[first + a.depth] = selection;
+    if (a.last) {
+      retained_rows[z] = node.ancestors;
+      retained[z] = a.kept;
+      accepted_count[z] = a.accepted;
+    }
+  }
+  // a block that keeps no row (its anchor is not its own ancestor) writes no results: the commit reads those that are there
+  const uint64_t keeps = __builtin_amdgcn_ballot_w64(a.last);
+  const uint32_t mask = keeps ? uint32_t(__shfl(node.ancestors, int(__builtin_ctzll(keeps)), 64)) : retained_rows[z];
+  commit_path<D>(mask, page_table, pool, p.commit);
+}
+SP_REGISTER_KERNEL("attention_q8_accept_commit_d128", &attention_q8_accept_commit<128>);
+SP_REGISTER_KERNEL("attention_q8_accept_commit_d64", &attention_q8_accept_commit<64>);
 SP_REGISTER_KERNEL("attention_q8_commit_d128", &attention_q8_commit<128>);
 SP_REGISTER_KERNEL("attention_q8_commit_d64", &attention_q8_commit<64>);
 

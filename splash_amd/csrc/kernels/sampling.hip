@@ -27,29 +27,11 @@
 #include "abi/Sampling.h"
 #include "abi/PagedAttention.h"
 #include "backend/KernelRegistry.hpp"
-#include "kernels/device_common.hpp"
+#include "kernels/acceptance.hpp"
 
 #include <cfloat>
 
 namespace splash::kernels {
-
-__device__ __forceinline__ bool unselectable(float v) { return !(v > -INFINITY); }  // NaN or -inf (sampling.metal:986-989)
-
-struct Best {
-  float value;
-  uint32_t index;
-};
-__device__ __forceinline__ Best better(Best a, Best b) {
-  return (b.value > a.value || (b.value == a.value && b.index < a.index)) ? b : a;
-}
-__device__ __forceinline__ Best wave_best(Best v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    Best other{__shfl_xor(v.value, o, 64), __shfl_xor(v.index, o, 64)};
-    v = better(v, other);
-  }
-  return v;
-}
 
 __device__ __forceinline__ uint32_t lane_of(const TargetSamplingParams &p, uint32_t row) {
   uint32_t lane = 0;
@@ -348,12 +330,7 @@ __global__ __launch_bounds__(64) void decode_sample_argmax_reduce(const float *_
 SP_REGISTER_KERNEL("decode_sample_argmax_reduce", &decode_sample_argmax_reduce);
 
 // decode_accept_tree (what the reference's sampling.metal:2044-2083 decides): grid (lanes), one wavefront a lane, a
-// thread a row. tokens: in, each row's selection; out, the lane's retained tokens from its first row.
-// A row follows its parent when its input token is the parent's selection and no earlier row of the same parent
-// does (one ballot); a row lies on the accepted path when every row of its ancestor mask follows its parent. The
-// path's rows, by depth, are the accepted draft tokens' rows; each selects the next token of the output, the last
-// the target's own. The output is cut to what the lane may still keep and after its first stop token (a second
-// ballot); the retained rows are the ancestor mask of the last kept row.
+// thread a row (accept_rows). tokens: in, each row's selection; out, the lane's retained tokens from its first row.
 __global__ __launch_bounds__(64) void decode_accept_tree(const uint32_t *__restrict__ input_tokens, const AttentionTreeRow *__restrict__ tree,
                                                          uint32_t *__restrict__ tokens, uint32_t *__restrict__ retained,
                                                          uint32_t *__restrict__ accepted_count, uint32_t *__restrict__ retained_rows,
@@ -364,33 +341,12 @@ __global__ __launch_bounds__(64) void decode_accept_tree(const uint32_t *__restr
   const bool live = row < rows;
   const AttentionTreeRow node = live ? tree[first + row] : AttentionTreeRow{0u, 0u, 0u};
   const uint32_t input = live ? input_tokens[first + row] : 0u, selection = live ? tokens[first + row] : 0u;
-  const uint32_t parent = live && row ? min(uint32_t(node.parent), SAMPLING_MAXIMUM_ROWS - 1u) : 0u;
-  const uint32_t parentSelection = __shfl(selection, int(parent), 64);
-  const bool matches = live && row && node.parent < row && input == parentSelection;
-  // the matching rows of this row's parent before it
-  uint32_t siblingsBefore = 0;
-  for (uint32_t other = 1; other < rows; ++other) {
-    const bool sameParent = __shfl(matches ? int(parent) : -1, int(other), 64) == int(parent);
-    siblingsBefore += other < row && sameParent ? 1u : 0u;
-  }
-  const bool follows = matches && !siblingsBefore;
-  const uint32_t following = uint32_t(__builtin_amdgcn_ballot_w64(follows)) | 1u;   // the anchor starts the path
-  const bool onPath = live && (node.ancestors & ~following) == 0u && ((node.ancestors >> row) & 1u);
-  const uint32_t path = uint32_t(__builtin_amdgcn_ballot_w64(onPath));
-  const uint32_t accepted = uint32_t(__builtin_popcount(path)) - 1u;
-  const uint32_t depth = live ? uint32_t(__builtin_popcount(path & ((1u << row) - 1u))) : 0u;   // the path's rows rise with depth
-  uint32_t kept = min(accepted + 1u, max(p.remaining[lane], 1u));
-  bool stop = false;
-#pragma unroll
-  for (int s = 0; s < int(SAMPLING_STOP_TOKENS); ++s) stop = stop || (p.stop_tokens[s] != SAMPLING_NO_TOKEN && selection == p.stop_tokens[s]);
-  // the shallowest path row within the kept ones that selects a stop token ends the output
-  const uint32_t stops = uint32_t(__builtin_amdgcn_ballot_w64(onPath && depth < kept && stop));
-  if (stops) kept = uint32_t(__builtin_popcount(path & ((2u << __builtin_ctz(stops)) - 1u)));
-  if (onPath && depth < kept) tokens[first + depth] = selection;   // every selection was read before any is written
-  if (onPath && depth + 1u == kept) {
+  const Acceptance a = accept_rows(row, live, node, input, selection, p.remaining[lane], p.stop_tokens);
+  if (a.retains) tokens[first + a.depth] = selection;   // every selection was read before any is written
+  if (a.last) {
     retained_rows[lane] = node.ancestors;
-    retained[lane] = kept;
-    accepted_count[lane] = min(accepted, kept);
+    retained[lane] = a.kept;
+    accepted_count[lane] = a.accepted;
   }
 }
 SP_REGISTER_KERNEL("decode_accept_tree", &decode_accept_tree);

@@ -169,15 +169,16 @@ void DenseVerify::encodeEmbedding(hip::CommandGraph &graph, uint32_t rows) {
 }
 
 void DenseVerify::encodeLayer(hip::CommandGraph &graph, uint32_t layer, const ops::AttentionPlan &plan, uint32_t rows,
-                              bool inputReady, bool feedsNext) {
+                              ops::LinearInput input, bool feedsNext) {
   const DenseLayer &w = weights_.layers.at(layer);
   const hip::Buffer &residual = hidden_[0], &next = hidden_[1];
   // Attention block: hidden[1] = hidden[0] + o(attention(qkv(norm(hidden[0])))).
   // A table a residual projection's epilogue wrote stands for the normalized rows, which are then
   // never stored; their inverse RMS is applied by the projection that reads the table.
   const ops::PreparedInput ready{normalized_, ops::LinearInput::TableUnscaled};
-  ops::PreparedInput prepared =
-      inputReady ? ready : ops::Normalization::addRmsTable(graph, residual, w.inputNorm, normalized_, scratch_, dims_.hidden, rows);
+  ops::PreparedInput prepared{normalized_, input};
+  if (input == ops::LinearInput::Plain)
+    prepared = ops::Normalization::addRmsTable(graph, residual, w.inputNorm, normalized_, scratch_, dims_.hidden, rows);
   ops::LinearBuffers qkv;
   qkv.input = normalized_;
   qkv.output = qkv_;
@@ -255,7 +256,7 @@ uint32_t DenseVerify::takeChainStatus() {
 // The layers with their projections chained: the first layer's q|k|v on its own, then a layer's head norms, RoPE and
 // cache store, its attention, and one dispatch of its output projection, gate/up pair, down projection and the q|k|v
 // projection of the layer after it (after the last layer, the LM head).
-void DenseVerify::encodeChainedLayers(hip::CommandGraph &graph, const ops::AttentionPlan &plan, uint32_t rows) {
+void DenseVerify::encodeChainedLayers(hip::CommandGraph &graph, const ops::AttentionPlan &plan, const ops::PreparedInput &entry, uint32_t rows) {
   const hip::Buffer &tableQkv = scratch_.input, &tableOutput = nextTable_, &tableGateUp = chainTables_[0], &tableDown = chainTables_[1];
   const ops::PreparedInput ready{normalized_, ops::LinearInput::TableUnscaled};
   auto scratchOf = [&](uint32_t link, const hip::Buffer &table) {
@@ -269,7 +270,7 @@ void DenseVerify::encodeChainedLayers(hip::CommandGraph &graph, const ops::Atten
     qkv.input = normalized_;
     qkv.output = qkv_;
     qkv.scratch = scratch_;
-    qkv.prepared = ops::Normalization::addRmsTable(graph, hidden_[0], first.inputNorm, normalized_, scratch_, dims_.hidden, rows);
+    qkv.prepared = entry;
     linear_.add(graph, qkv, first.qkv, linear_.plan(first.qkv, rows));
   }
   for (uint32_t layer = 0; layer < dims_.layers; ++layer) {
@@ -532,7 +533,8 @@ void DenseVerify::encodePrefill(hip::CommandGraph &graph, uint32_t tableFirst, u
   encodeEmbedding(graph, tokens);
   const bool feeds = layersFeedNext(tokens);
   for (uint32_t layer = 0; layer < dims_.layers; ++layer) {
-    encodeLayer(graph, layer, plan, tokens, feeds && layer > 0, feeds && layer + 1 < dims_.layers);
+    encodeLayer(graph, layer, plan, tokens, feeds && layer > 0 ? ops::LinearInput::TableUnscaled : ops::LinearInput::Plain,
+                feeds && layer + 1 < dims_.layers);
     encodeCapture(graph, layer, tokens);
   }
 }
@@ -558,15 +560,17 @@ void DenseVerify::encode(hip::CommandGraph &graph, const std::vector<VerifyLane>
   const ops::AttentionGeometry geometry{dims_.qHeads, dims_.kvHeads, dims_.headDimension, dims_.rotaryPairs, dims_.normalizeHeads};
   const ops::AttentionPlan plan = ops::PagedAttention::plan(geometry, sequences);
   if (samples && !testChildren_) (void)draftProbabilities();
-  if (dims_.rotaryPairs)
-    ops::RoPE::addTreeTables(graph, inverseFrequency_, depths_, ropeCos_, ropeSin_, dims_.rotaryPairs, rope);
-  encodeEmbedding(graph, rows);
+  const ops::PreparedInput entry = ops::Embedding::addNormTable(
+      graph, weights_.embedding, inputTokens_, hidden_[0], weights_.layers.front().inputNorm, normalized_, scratch_,
+      {inverseFrequency_, depths_, ropeCos_, ropeSin_, dims_.rotaryPairs, rope}, rows);
   if (chains(rows)) {
-    encodeChainedLayers(graph, plan, rows);
+    encodeChainedLayers(graph, plan, entry, rows);
   } else {
     const bool feeds = layersFeedNext(rows);
+    ops::LinearInput input = entry.layout;
     for (uint32_t layer = 0; layer < dims_.layers; ++layer) {
-      encodeLayer(graph, layer, plan, rows, feeds && layer > 0, feeds);
+      encodeLayer(graph, layer, plan, rows, input, feeds);
+      input = feeds ? ops::LinearInput::TableUnscaled : ops::LinearInput::Plain;
       encodeCapture(graph, layer, rows);
     }
     encodeHead(graph, rows, feeds);
@@ -586,13 +590,21 @@ void DenseVerify::encode(hip::CommandGraph &graph, const std::vector<VerifyLane>
     sampling.maskWords = lanePolicies_.maskWords();
   }
   if (penalized) ops::Sampling::addPenalties(graph, sampling, dims_.vocabulary, dims_.vocabulary, laneRows, policies, lanePolicies_.table());
-  ops::Sampling::addVerify(graph, sampling, dims_.vocabulary, dims_.vocabulary, laneRows, policies, lanePolicies_.stopTokens());
+  // a step of greedy rows that commits selects, accepts and commits in one dispatch
+  const bool together = commit && ops::Sampling::selectsGreedily(laneRows, policies);
+  ops::Sampling::addVerify(graph, sampling, dims_.vocabulary, dims_.vocabulary, laneRows, policies, lanePolicies_.stopTokens(),
+                           together ? ops::GreedySelection::Partials : ops::GreedySelection::Tokens);
   const ops::AcceptanceBuffers acceptance{inputTokens_, treeRows_, tokens_, retained_, acceptedCount_, retainedRows_};
-  ops::Sampling::addAcceptance(graph, acceptance, laneRows, remaining, lanePolicies_.stopTokens());
+  if (together)
+    ops::PagedAttention::addAcceptCommit(graph, plan, sampling, acceptance,
+                                         ops::Sampling::acceptance(acceptance, laneRows, remaining, lanePolicies_.stopTokens()),
+                                         {pageTable_, kvAll_, pageBytes_}, dims_.layers, layerBytes_);
+  else
+    ops::Sampling::addAcceptance(graph, acceptance, laneRows, remaining, lanePolicies_.stopTokens());
   // a step that commits counts the tokens its penalized lanes keep, for the next step's penalties
   if (penalized && commit)
     ops::Sampling::addPenaltyCount(graph, acceptance, dims_.vocabulary, laneRows, lanePolicies_.penalized(lanes.size()), lanePolicies_.table());
-  if (commit)
+  if (commit && !together)
     ops::PagedAttention::addPathCommit(graph, plan, retainedRows_, {pageTable_, kvAll_, pageBytes_}, dims_.layers, layerBytes_);
 }
 

@@ -115,11 +115,12 @@ public:
   void encode(hip::CommandGraph &graph, const std::vector<VerifyLane> &lanes, bool commit = true);
   // Its parts, for per-kernel timing and tests.
   void encodeEmbedding(hip::CommandGraph &graph, uint32_t rows);
-  // A layer (or the head) whose predecessor in the same graph left the table of its normalized input
-  // in the projection scratch passes `inputReady`; a layer that passes `feedsNext` leaves that table
-  // for its successor. A part encoded on its own passes neither.
+  // A layer whose predecessor in the same graph left the table of its normalized input in the projection scratch
+  // passes the table's layout as `input` (TableUnscaled: a layer's, less the rows' inverse RMS; Table16: a step's first
+  // pass), the head `inputReady` for a layer's; a layer that passes `feedsNext` leaves that table for its successor. A
+  // part encoded on its own passes none of them.
   void encodeLayer(hip::CommandGraph &graph, uint32_t layer, const ops::AttentionPlan &plan, uint32_t rows,
-                   bool inputReady = false, bool feedsNext = false);
+                   ops::LinearInput input = ops::LinearInput::Plain, bool feedsNext = false);
   void encodeHead(hip::CommandGraph &graph, uint32_t rows, bool inputReady = false);
   // Whether every layer's down projection can norm its rows for the layer after it.
   [[nodiscard]] bool layersFeedNext(uint32_t rows) const noexcept;
@@ -214,7 +215,7 @@ private:
   hip::Buffer chunkAttentionTable_;  // a long chunk's attention rows as the output projection's tables, every window's
   void encodeChunkLayer(hip::CommandGraph &graph, uint32_t layer, const ops::AttentionChunkPlan &plan, uint32_t tokens, bool first,
                         bool feedsNext);
-  void encodeChainedLayers(hip::CommandGraph &graph, const ops::AttentionPlan &plan, uint32_t rows);
+  void encodeChainedLayers(hip::CommandGraph &graph, const ops::AttentionPlan &plan, const ops::PreparedInput &entry, uint32_t rows);
   [[nodiscard]] bool chains(uint32_t rows) const noexcept;
   ops::AttentionWorkspace attentionWorkspace_;
   ops::SamplingBuffers sampling_;

@@ -221,7 +221,7 @@ void HybridVerify::encodeEmbedding(hip::CommandGraph &graph, uint32_t rows) {
   ops::Embedding::add(graph, weights_.embedding, inputTokens_, hidden_[0], rows);
 }
 
-void HybridVerify::encodeLayer(hip::CommandGraph &graph, uint32_t layer, const std::vector<HybridLane> &lanes, bool inputReady,
+void HybridVerify::encodeLayer(hip::CommandGraph &graph, uint32_t layer, const std::vector<HybridLane> &lanes, ops::LinearInput input,
                                bool feedsNext) {
   if (lanes.empty() || lanes.size() > maxLanes_) throw std::invalid_argument("the step takes 1 to its most lanes");
   const HybridLayer &w = weights_.layers.at(layer);
@@ -251,14 +251,16 @@ void HybridVerify::encodeLayer(hip::CommandGraph &graph, uint32_t layer, const s
     in.input = normalized;
     in.output = rowsOf(packed_, first, count, uint64_t{inputWidth} * 2);
     in.scratch = scratch_;
-    // The layer before may have left the table of these rows, less their inverse RMS, from its combine.
-    in.prepared = inputReady ? ops::PreparedInput{normalized, ops::LinearInput::TableUnscaled}
-                             : ops::Normalization::addRmsTable(graph, rowsOf(residual, first, count, hiddenBytes), w.inputNorm, normalized,
-                                                               scratch_, dims_.hidden, count);
+    // The layer before may have left the table of these rows, less their inverse RMS, from its combine; the step's first
+    // pass leaves the first layer's whole.
+    in.prepared = {normalized, input};
+    if (input == ops::LinearInput::Plain)
+      in.prepared = ops::Normalization::addRmsTable(graph, rowsOf(residual, first, count, hiddenBytes), w.inputNorm, normalized, scratch_,
+                                                    dims_.hidden, count);
     linear_.add(graph, in, w.mixerInput, linear_.plan(w.mixerInput, count));
     if (!attends && w.gateRows) {
       // beta | alpha from rows of floats: the packed row's columns after q, k, v and z
-      if (inputReady) throw std::invalid_argument("float gate rows read the normalized rows, which a deferred norm does not store");
+      if (input == ops::LinearInput::TableUnscaled) throw std::invalid_argument("float gate rows read the normalized rows, which a deferred norm does not store");
       const ops::GdnShape shape = dims_.gdnShape();
       if (w.gateRows.outputSize != 2 * shape.valueHeads || w.gateRows.inputSize != dims_.hidden)
         throw std::invalid_argument("a GDN layer's gate rows are beta then alpha, a row a value head each");
@@ -386,9 +388,17 @@ void HybridVerify::encode(hip::CommandGraph &graph, const std::vector<HybridLane
     rows += lane.block.rows;
   }
   if (samples) (void)draftProbabilities();
-  if (dims_.rotaryPairs)
-    ops::RoPE::addTreeTables(graph, inverseFrequency_, depths_, ropeCos_, ropeSin_, dims_.rotaryPairs, rope);
-  encodeEmbedding(graph, rows);
+  // A step of one piece of rows: its tables, gather and first norm are one pass.
+  ops::LinearInput input = ops::LinearInput::Plain;
+  if (rows <= kProjectionRows) {
+    input = ops::Embedding::addNormTable(graph, weights_.embedding, inputTokens_, hidden_[0], weights_.layers.front().inputNorm, normalized_,
+                                         scratch_, {inverseFrequency_, depths_, ropeCos_, ropeSin_, dims_.rotaryPairs, rope}, rows)
+                .layout;
+  } else {
+    if (dims_.rotaryPairs)
+      ops::RoPE::addTreeTables(graph, inverseFrequency_, depths_, ropeCos_, ropeSin_, dims_.rotaryPairs, rope);
+    encodeEmbedding(graph, rows);
+  }
   // One piece of rows: a layer's combine can write the table the next layer's (or the head's) first projection reads.
   bool feeds = rows <= kProjectionRows && dims_.hidden % GGUF_BLOCK == 0;
   if (dims_.dense())
@@ -396,7 +406,8 @@ void HybridVerify::encode(hip::CommandGraph &graph, const std::vector<HybridLane
   // float gate rows read the normalized rows themselves, which a layer fed by the combine before it never stores
   for (const HybridLayer &l : weights_.layers) feeds = feeds && !l.gateRows;
   for (uint32_t layer = 0; layer < dims_.layers; ++layer) {
-    encodeLayer(graph, layer, lanes, feeds && layer > 0, feeds);
+    encodeLayer(graph, layer, lanes, input, feeds);
+    input = feeds ? ops::LinearInput::TableUnscaled : ops::LinearInput::Plain;
     encodeCapture(graph, layer, rows);
   }
   encodeHead(graph, rows, feeds);
@@ -408,13 +419,21 @@ void HybridVerify::encode(hip::CommandGraph &graph, const std::vector<HybridLane
     selection.maskWords = lanePolicies_.maskWords();
   }
   if (penalized) ops::Sampling::addPenalties(graph, selection, dims_.vocabulary, dims_.vocabulary, laneRows, policies, lanePolicies_.table());
-  ops::Sampling::addVerify(graph, selection, dims_.vocabulary, dims_.vocabulary, laneRows, policies, lanePolicies_.stopTokens());
+  // a step of greedy rows that commits keys and values selects, accepts and commits in one dispatch
+  const bool together = commit && dims_.attentionLayers() && ops::Sampling::selectsGreedily(laneRows, policies);
+  ops::Sampling::addVerify(graph, selection, dims_.vocabulary, dims_.vocabulary, laneRows, policies, lanePolicies_.stopTokens(),
+                           together ? ops::GreedySelection::Partials : ops::GreedySelection::Tokens);
   const ops::AcceptanceBuffers acceptance{inputTokens_, treeRows_, tokens_, retained_, acceptedCount_, retainedRows_};
-  ops::Sampling::addAcceptance(graph, acceptance, laneRows, remaining, lanePolicies_.stopTokens());
+  if (together)
+    ops::PagedAttention::addAcceptCommit(graph, planOf(lanes), selection, acceptance,
+                                         ops::Sampling::acceptance(acceptance, laneRows, remaining, lanePolicies_.stopTokens()),
+                                         {pageTable_, kvAll_, pageBytes_}, dims_.attentionLayers(), layerBytes_);
+  else
+    ops::Sampling::addAcceptance(graph, acceptance, laneRows, remaining, lanePolicies_.stopTokens());
   // a step that commits counts the tokens its penalized lanes keep, for the next step's penalties
   if (penalized && commit)
     ops::Sampling::addPenaltyCount(graph, acceptance, dims_.vocabulary, laneRows, lanePolicies_.penalized(lanes.size()), lanePolicies_.table());
-  if (commit && dims_.attentionLayers())
+  if (commit && !together && dims_.attentionLayers())
     ops::PagedAttention::addPathCommit(graph, planOf(lanes), retainedRows_, {pageTable_, kvAll_, pageBytes_}, dims_.attentionLayers(),
                                        layerBytes_);
 }

@@ -170,11 +170,12 @@ public:
 
   void encode(hip::CommandGraph &graph, const std::vector<HybridLane> &lanes, bool commit = true);
   void encodeEmbedding(hip::CommandGraph &graph, uint32_t rows);
-  // A layer (or the head) whose predecessor in the same graph left the table of its input rows, less their inverse
-  // RMS, in the projection scratch passes `inputReady`; a layer that passes `feedsNext` leaves that table from its
-  // combine. A part encoded on its own passes neither.
-  void encodeLayer(hip::CommandGraph &graph, uint32_t layer, const std::vector<HybridLane> &lanes, bool inputReady = false,
-                   bool feedsNext = false);
+  // A layer whose predecessor in the same graph left the table of its input rows in the projection scratch passes the
+  // table's layout as `input` (TableUnscaled: a layer's, less the rows' inverse RMS; Table16: a step's first pass, whose
+  // rows are one piece), the head `inputReady` for a layer's; a layer that passes `feedsNext` leaves that table from its
+  // combine. A part encoded on its own passes none of them.
+  void encodeLayer(hip::CommandGraph &graph, uint32_t layer, const std::vector<HybridLane> &lanes,
+                   ops::LinearInput input = ops::LinearInput::Plain, bool feedsNext = false);
   void encodeHead(hip::CommandGraph &graph, uint32_t rows, bool inputReady = false);
   // A chunk of `tokens` prompt tokens (1 to prefillRows(); inputs where a step's are: tokens, a chain of tree rows a block
   // of sixteen, each row's depth in its block) of the sequence of lane `lane`, `committed` tokens already cached, through

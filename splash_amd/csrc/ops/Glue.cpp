@@ -13,6 +13,34 @@ void requireNorm(const hip::Buffer &input, const hip::Buffer &weight, const hip:
   requireBytes(weight, uint64_t{width} * 2, "norm weight");
   requireBytes(output, uint64_t{rows} * width * 2, "norm output");
 }
+
+RopeTreeParams ropeParams(const RopeTables &t) {
+  if (!t.pairs || t.pairs > 1024) throw std::invalid_argument("RoPE tables take 1 to 1024 pairs");
+  if (t.sequences.empty() || t.sequences.size() > 8) throw std::invalid_argument("RoPE tables take 1 to 8 sequences");
+  RopeTreeParams params{};
+  params.pairs = t.pairs;
+  params.sequences = uint32_t(t.sequences.size());
+  for (size_t i = 0; i < t.sequences.size(); ++i) {
+    params.first_row[i] = t.sequences[i].firstRow;
+    params.row_count[i] = t.sequences[i].rows;
+    params.anchor[i] = t.sequences[i].anchor;
+    params.rows = std::max(params.rows, t.sequences[i].firstRow + t.sequences[i].rows);
+  }
+  requireBytes(t.inverseFrequency, uint64_t{t.pairs} * 4, "RoPE inverse frequencies");
+  requireBytes(t.depth, uint64_t{params.rows} * 4, "row depths");
+  requireBytes(t.cosines, uint64_t{params.rows} * t.pairs * 4, "RoPE cosine table");
+  requireBytes(t.sines, uint64_t{params.rows} * t.pairs * 4, "RoPE sine table");
+  return params;
+}
+
+void requireTable(const EmbeddingTable &table, const hip::Buffer &tokens, const hip::Buffer &output, uint32_t rows) {
+  if (!gguf_native_bytes(table.formatId)) throw std::invalid_argument("no token gather for this table format");
+  if (!rows || !table.hidden || table.hidden % GGUF_BLOCK || !table.vocabulary)
+    throw std::invalid_argument("a token table holds whole native blocks");
+  requireBytes(table.rows, uint64_t{table.vocabulary} * (table.hidden / GGUF_BLOCK) * gguf_native_bytes(table.formatId), "token table");
+  requireBytes(tokens, uint64_t{rows} * 4, "input tokens");
+  requireBytes(output, uint64_t{rows} * table.hidden * 2, "embedding output");
+}
 } // namespace
 
 void Normalization::addRms(hip::CommandGraph &graph, const hip::Buffer &input, const hip::Buffer &weight, const hip::Buffer &output,
@@ -35,14 +63,32 @@ PreparedInput Normalization::addRmsTable(hip::CommandGraph &graph, const hip::Bu
 
 void Embedding::add(hip::CommandGraph &graph, const EmbeddingTable &table, const hip::Buffer &tokens, const hip::Buffer &output,
                     uint32_t rows) {
-  if (!gguf_native_bytes(table.formatId)) throw std::invalid_argument("no token gather for this table format");
-  if (!rows || !table.hidden || table.hidden % GGUF_BLOCK || !table.vocabulary)
-    throw std::invalid_argument("a token table holds whole native blocks");
-  requireBytes(table.rows, uint64_t{table.vocabulary} * (table.hidden / GGUF_BLOCK) * gguf_native_bytes(table.formatId), "token table");
-  requireBytes(tokens, uint64_t{rows} * 4, "input tokens");
-  requireBytes(output, uint64_t{rows} * table.hidden * 2, "embedding output");
+  requireTable(table, tokens, output, rows);
   graph.add(std::string("gguf_embed_") + gguf_format_name(table.formatId), {table.rows, tokens, output},
             GgufEmbedParams{rows, table.vocabulary, table.hidden}, {rows, table.hidden / GGUF_BLOCK, 1}, {64, 1, 1});
+}
+
+PreparedInput Embedding::addNormTable(hip::CommandGraph &graph, const EmbeddingTable &table, const hip::Buffer &tokens,
+                                      const hip::Buffer &hidden, const hip::Buffer &weight, const hip::Buffer &normalized,
+                                      const LinearScratch &scratch, const RopeTables &rope, uint32_t rows) {
+  const uint32_t tiles = gguf_row_tiles(rows);
+  EmbedNormParams params{{rows, table.vocabulary, table.hidden}, tiles, {}};
+  if (rope.pairs) params.rope = ropeParams(rope);
+  if (table.hidden > NORM_STAGED_WIDTH || rows > kMaximumDispatchRows || (rope.pairs && params.rope.rows != rows)) {
+    if (rope.pairs) RoPE::addTreeTables(graph, rope.inverseFrequency, rope.depth, rope.cosines, rope.sines, rope.pairs, rope.sequences);
+    add(graph, table, tokens, hidden, rows);
+    return Normalization::addRmsTable(graph, hidden, weight, normalized, scratch, table.hidden, rows);
+  }
+  requireTable(table, tokens, hidden, rows);
+  requireNorm(hidden, weight, normalized, table.hidden, rows);
+  requireBytes(scratch.input, gguf_tables_bytes(table.hidden, tiles), "projection table");
+  // without tables the hidden rows stand in for their bindings, which are then not touched
+  const bool rotates = rope.pairs != 0;
+  graph.add(std::string("gguf_embed_norm_") + gguf_format_name(table.formatId),
+            {table.rows, tokens, weight, hidden, normalized, scratch.input, rotates ? rope.inverseFrequency : hidden,
+             rotates ? rope.depth : hidden, rotates ? rope.cosines : hidden, rotates ? rope.sines : hidden},
+            params, {tiles * GGUF_ROW_TILE, rotates ? 2u : 1u, 1}, {256, 1, 1});
+  return {normalized, LinearInput::Table16};
 }
 
 void FloatProjection::add(hip::CommandGraph &graph, const hip::Buffer &input, const FloatRows &w, const hip::Buffer &output, uint32_t rows,
@@ -61,21 +107,7 @@ void FloatProjection::add(hip::CommandGraph &graph, const hip::Buffer &input, co
 void RoPE::addTreeTables(hip::CommandGraph &graph, const hip::Buffer &inverseFrequency, const hip::Buffer &depth,
                          const hip::Buffer &cosines, const hip::Buffer &sines, uint32_t pairs,
                          const std::vector<RopeSequence> &sequences) {
-  if (!pairs || pairs > 1024) throw std::invalid_argument("RoPE tables take 1 to 1024 pairs");
-  if (sequences.empty() || sequences.size() > 8) throw std::invalid_argument("RoPE tables take 1 to 8 sequences");
-  RopeTreeParams params{};
-  params.pairs = pairs;
-  params.sequences = uint32_t(sequences.size());
-  for (size_t i = 0; i < sequences.size(); ++i) {
-    params.first_row[i] = sequences[i].firstRow;
-    params.row_count[i] = sequences[i].rows;
-    params.anchor[i] = sequences[i].anchor;
-    params.rows = std::max(params.rows, sequences[i].firstRow + sequences[i].rows);
-  }
-  requireBytes(inverseFrequency, uint64_t{pairs} * 4, "RoPE inverse frequencies");
-  requireBytes(depth, uint64_t{params.rows} * 4, "row depths");
-  requireBytes(cosines, uint64_t{params.rows} * pairs * 4, "RoPE cosine table");
-  requireBytes(sines, uint64_t{params.rows} * pairs * 4, "RoPE sine table");
+  const RopeTreeParams params = ropeParams({inverseFrequency, depth, cosines, sines, pairs, sequences});
   graph.add("rope_build_tree_tables", {inverseFrequency, depth, cosines, sines}, params, {params.rows, 1, 1}, {pairs, 1, 1});
 }
 

@@ -22,6 +22,16 @@ public:
                                    const hip::Buffer &output, const LinearScratch &scratch, uint32_t width, uint32_t rows);
 };
 
+struct RopeSequence final {
+  uint32_t firstRow = 0, rows = 0, anchor = 0;
+};
+// What a step's RoPE tables are built from and where (no pairs: the model rotates nothing).
+struct RopeTables final {
+  const hip::Buffer &inverseFrequency, &depth, &cosines, &sines;
+  uint32_t pairs = 0;
+  const std::vector<RopeSequence> &sequences;
+};
+
 // A token table's rows as stored: native K-quant blocks, gathered, never multiplied (Weights.hpp:227-260).
 struct EmbeddingTable final {
   hip::Buffer rows;
@@ -33,6 +43,12 @@ class Embedding final {
 public:
   static void add(hip::CommandGraph &graph, const EmbeddingTable &table, const hip::Buffer &tokens, const hip::Buffer &output,
                   uint32_t rows);
+  // The first passes of a step's rows: their RoPE tables, this gather into `hidden` and the table of the rows normed
+  // with `weight` (RoPE::addTreeTables, add and Normalization::addRmsTable, whose values these are), as one dispatch
+  // where a row is whole super-blocks that fit a workgroup's LDS.
+  static PreparedInput addNormTable(hip::CommandGraph &graph, const EmbeddingTable &table, const hip::Buffer &tokens, const hip::Buffer &hidden,
+                                    const hip::Buffer &weight, const hip::Buffer &normalized, const LinearScratch &scratch,
+                                    const RopeTables &rope, uint32_t rows);
 };
 
 // The fp32 projection of weights kept as rows (the reference's addGgufFloat, LinearGguf.cpp:545-612): output row r's
@@ -50,9 +66,6 @@ public:
   static void add(hip::CommandGraph &graph, const hip::Buffer &gate, const hip::Buffer &up, const hip::Buffer &output, uint64_t count);
 };
 
-struct RopeSequence final {
-  uint32_t firstRow = 0, rows = 0, anchor = 0;
-};
 class RoPE final {
 public:
   // cos/sin of (anchor + depth[row]) * inverseFrequency[pair] per packed row.

@@ -392,10 +392,9 @@ void PagedAttention::addPromptAttention(hip::CommandGraph &graph, const Attentio
             {g.qHeads, ATTENTION_MAXIMUM_ROWS, plan.blocks()}, {256, 1, 1});
 }
 
-void PagedAttention::addPathCommit(hip::CommandGraph &graph, const AttentionPlan &plan, const hip::Buffer &retained,
-                                   const KvPages &pages, uint32_t layers, uint64_t layerBytes) {
+namespace {
+AttentionCommitParams commitParams(const AttentionPlan &plan, const KvPages &pages, uint32_t layers, uint64_t layerBytes) {
   const AttentionGeometry &g = plan.geometry();
-  requireBytes(retained, plan.sequences().size() * 4, "retained rows");
   requirePages(plan, pages);
   if (!layers || (layers > 1 && (layerBytes < pages.pageBytes || pages.pool.sizeBytes() < layerBytes * layers)))
     throw std::invalid_argument("KV pool buffer does not hold the layers' pools");
@@ -408,8 +407,39 @@ void PagedAttention::addPathCommit(hip::CommandGraph &graph, const AttentionPlan
   params.page_bytes = pages.pageBytes;
   params.layer_bytes = layerBytes;
   for (uint32_t i = 0; i < full.sequences; ++i) params.sequence[i] = full.sequence[i];
-  graph.add("attention_q8_commit" + kernelSuffix(g), {retained, pages.pageTable, pages.pool}, params,
+  return params;
+}
+} // namespace
+
+void PagedAttention::addPathCommit(hip::CommandGraph &graph, const AttentionPlan &plan, const hip::Buffer &retained,
+                                   const KvPages &pages, uint32_t layers, uint64_t layerBytes) {
+  const AttentionGeometry &g = plan.geometry();
+  requireBytes(retained, plan.sequences().size() * 4, "retained rows");
+  graph.add("attention_q8_commit" + kernelSuffix(g), {retained, pages.pageTable, pages.pool}, commitParams(plan, pages, layers, layerBytes),
             {g.kvHeads, plan.sequences().size(), layers}, {g.headDimension, 1, 1});
+}
+
+void PagedAttention::addAcceptCommit(hip::CommandGraph &graph, const AttentionPlan &plan, const SamplingBuffers &sampling,
+                                     const AcceptanceBuffers &acceptance, const AcceptBatchParams &accept, const KvPages &pages,
+                                     uint32_t layers, uint64_t layerBytes) {
+  const AttentionGeometry &g = plan.geometry();
+  uint32_t rows = 0;
+  if (accept.lanes != plan.sequences().size()) throw std::invalid_argument("an accepting commit takes a lane a sequence");
+  for (uint32_t i = 0; i < accept.lanes; ++i) {
+    if (accept.lane[i].first != plan.sequences()[i].firstRow || accept.lane[i].rows != plan.sequences()[i].rows)
+      throw std::invalid_argument("an accepting commit's lanes are the plan's sequences");
+    rows = std::max(rows, accept.lane[i].first + accept.lane[i].rows);
+  }
+  const SamplingWorkspaceSize need = Sampling::workspace(rows);
+  requireBytes(sampling.partialValues, need.partialValues, "argmax partial values");
+  requireBytes(sampling.partialIndices, need.partialIndices, "argmax partial indices");
+  AttentionAcceptCommitParams params{commitParams(plan, pages, layers, layerBytes), {}, {}};
+  std::copy(std::begin(accept.remaining), std::end(accept.remaining), params.remaining);
+  std::copy(std::begin(accept.stop_tokens), std::end(accept.stop_tokens), params.stop_tokens);
+  graph.add("attention_q8_accept_commit" + kernelSuffix(g),
+            {sampling.partialValues, sampling.partialIndices, acceptance.inputTokens, acceptance.treeRows, acceptance.tokens,
+             acceptance.retained, acceptance.acceptedCount, acceptance.retainedRows, pages.pageTable, pages.pool},
+            params, {g.kvHeads, accept.lanes, layers}, {g.headDimension, 1, 1});
 }
 
 } // namespace splash::ops

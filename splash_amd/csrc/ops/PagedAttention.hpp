@@ -7,6 +7,7 @@
 #include "abi/PagedAttention.h"
 #include "hip/Backend.hpp"
 #include "ops/Linear.hpp"
+#include "ops/Sampling.hpp"
 
 #include <cstdint>
 #include <vector>
@@ -190,6 +191,12 @@ public:
   // reference's grid of layers x KV heads does).
   static void addPathCommit(hip::CommandGraph &graph, const AttentionPlan &plan, const hip::Buffer &retained,
                             const KvPages &pages, uint32_t layers = 1, uint64_t layerBytes = 0);
+  // The same for a step of greedy rows whose selections are still their shards' partials (addVerify with
+  // GreedySelection::Partials): the dispatch also selects, accepts the block and leaves what addAcceptance leaves.
+  // `accept`'s lanes are the plan's sequences.
+  static void addAcceptCommit(hip::CommandGraph &graph, const AttentionPlan &plan, const SamplingBuffers &sampling,
+                              const AcceptanceBuffers &acceptance, const AcceptBatchParams &accept, const KvPages &pages, uint32_t layers,
+                              uint64_t layerBytes);
 };
 
 } // namespace splash::ops

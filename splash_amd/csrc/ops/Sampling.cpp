@@ -34,9 +34,11 @@ SamplingWorkspaceSize Sampling::workspace(uint32_t rows) noexcept {
 
 void Sampling::addVerify(hip::CommandGraph &graph, const SamplingBuffers &b, uint32_t vocabulary, uint32_t logitsStride,
                          const std::vector<LaneRows> &lanes, const std::vector<SamplingPolicy> &policies,
-                         const std::array<uint32_t, SAMPLING_STOP_TOKENS> &stopTokens) {
+                         const std::array<uint32_t, SAMPLING_STOP_TOKENS> &stopTokens, GreedySelection greedy) {
   const uint32_t rows = packedRows(lanes);
   if (policies.size() != lanes.size()) throw std::invalid_argument("acceptance takes one policy per lane");
+  if (greedy == GreedySelection::Partials && !selectsGreedily(lanes, policies))
+    throw std::invalid_argument("only rows that are all greedy can leave their selections as partials");
   if (!vocabulary || logitsStride < vocabulary) throw std::invalid_argument("logits rows hold the vocabulary");
   TargetSamplingParams params{};
   params.vocabulary = vocabulary;
@@ -92,6 +94,7 @@ void Sampling::addVerify(hip::CommandGraph &graph, const SamplingBuffers &b, uin
   // Every row gets its argmax; the sampled lanes' rows are then overwritten by their draw.
   graph.add("decode_sample_argmax_sharded", {b.logits, b.partialValues, b.partialIndices}, params, {rows * SAMPLING_SHARDS, 1, 1},
             {SAMPLING_THREADS, 1, 1});
+  if (greedy == GreedySelection::Partials) return;
   graph.add("decode_sample_argmax_reduce", {b.partialValues, b.partialIndices, b.tokens}, params, {rows, 1, 1}, {64, 1, 1});
   if (!params.sampling_mask) {
     addThinkingCutoff(graph, b, vocabulary, lanes, policies);
@@ -113,6 +116,13 @@ void Sampling::addVerify(hip::CommandGraph &graph, const SamplingBuffers &b, uin
     graph.add("decode_sample_draw", {b.logits, b.draftProbabilities, b.masses, b.uniforms, b.ranges, b.decisions, b.tokens}, params,
               {rows, 1, 1}, {64, 1, 1});
   addThinkingCutoff(graph, b, vocabulary, lanes, policies);
+}
+
+bool Sampling::selectsGreedily(const std::vector<LaneRows> &lanes, const std::vector<SamplingPolicy> &policies) noexcept {
+  if (policies.size() != lanes.size()) return false;
+  for (size_t l = 0; l < lanes.size(); ++l)
+    if (policies[l].samples() || (policies[l].thinkingCutoff && policies[l].thinkingCutoff->row < lanes[l].rows)) return false;
+  return true;
 }
 
 void Sampling::addThinkingCutoff(hip::CommandGraph &graph, const SamplingBuffers &b, uint32_t vocabulary, const std::vector<LaneRows> &lanes,
@@ -225,8 +235,8 @@ void Sampling::addPenaltyCount(hip::CommandGraph &graph, const AcceptanceBuffers
   graph.add("decode_sample_count_tokens", {table.words, b.tokens, b.retained}, params, {params.entries, 1, 1}, {64, 1, 1});
 }
 
-void Sampling::addAcceptance(hip::CommandGraph &graph, const AcceptanceBuffers &b, const std::vector<LaneRows> &lanes,
-                             const std::vector<uint32_t> &remaining, const std::array<uint32_t, SAMPLING_STOP_TOKENS> &stopTokens) {
+AcceptBatchParams Sampling::acceptance(const AcceptanceBuffers &b, const std::vector<LaneRows> &lanes, const std::vector<uint32_t> &remaining,
+                                       const std::array<uint32_t, SAMPLING_STOP_TOKENS> &stopTokens) {
   const uint32_t rows = packedRows(lanes);
   if (remaining.size() != lanes.size()) throw std::invalid_argument("acceptance takes one remaining count per lane");
   AcceptBatchParams params{};
@@ -242,6 +252,12 @@ void Sampling::addAcceptance(hip::CommandGraph &graph, const AcceptanceBuffers &
   requireBytes(b.retained, lanes.size() * 4, "retained counts");
   requireBytes(b.acceptedCount, lanes.size() * 4, "accepted counts");
   requireBytes(b.retainedRows, lanes.size() * 4, "retained rows");
+  return params;
+}
+
+void Sampling::addAcceptance(hip::CommandGraph &graph, const AcceptanceBuffers &b, const std::vector<LaneRows> &lanes,
+                             const std::vector<uint32_t> &remaining, const std::array<uint32_t, SAMPLING_STOP_TOKENS> &stopTokens) {
+  const AcceptBatchParams params = acceptance(b, lanes, remaining, stopTokens);
   graph.add("decode_accept_tree", {b.inputTokens, b.treeRows, b.tokens, b.retained, b.acceptedCount, b.retainedRows}, params,
             {lanes.size(), 1, 1}, {64, 1, 1});
 }

@@ -109,6 +109,9 @@ struct AcceptanceBuffers final {
   hip::Buffer retainedRows;   // uint32 [lanes]: mask of the block rows retained
 };
 
+// What addVerify leaves of the greedy rows: their tokens, or their shards' partial maxima for a kernel that reduces them.
+enum class GreedySelection : uint8_t { Tokens, Partials };
+
 class Sampling final {
 public:
   [[nodiscard]] static SamplingWorkspaceSize workspace(uint32_t rows) noexcept;
@@ -118,7 +121,14 @@ public:
   static void addVerify(hip::CommandGraph &graph, const SamplingBuffers &buffers, uint32_t vocabulary, uint32_t logitsStride,
                         const std::vector<LaneRows> &lanes, const std::vector<SamplingPolicy> &policies,
                         const std::array<uint32_t, SAMPLING_STOP_TOKENS> &stopTokens = {SAMPLING_NO_TOKEN, SAMPLING_NO_TOKEN,
-                                                                                       SAMPLING_NO_TOKEN, SAMPLING_NO_TOKEN});
+                                                                                       SAMPLING_NO_TOKEN, SAMPLING_NO_TOKEN},
+                        GreedySelection greedy = GreedySelection::Tokens);
+  // Whether the lanes' selections are their rows' argmax and nothing else: no lane samples and no cutoff lies in its block.
+  [[nodiscard]] static bool selectsGreedily(const std::vector<LaneRows> &lanes, const std::vector<SamplingPolicy> &policies) noexcept;
+  // The parameters of a step's acceptance; throws for buffers that do not hold it.
+  [[nodiscard]] static AcceptBatchParams acceptance(const AcceptanceBuffers &buffers, const std::vector<LaneRows> &lanes,
+                                                    const std::vector<uint32_t> &remaining,
+                                                    const std::array<uint32_t, SAMPLING_STOP_TOKENS> &stopTokens);
   static void addAcceptance(hip::CommandGraph &graph, const AcceptanceBuffers &buffers, const std::vector<LaneRows> &lanes,
                             const std::vector<uint32_t> &remaining, const std::array<uint32_t, SAMPLING_STOP_TOKENS> &stopTokens);
 
