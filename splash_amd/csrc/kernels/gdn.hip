@@ -6,18 +6,18 @@
 //
 // Sixteen waves. In the prologue and the gate a wave takes a row: lane l holds channels l and 64 + l,
 // and a sum over the head's 128 channels is four tree sums over 32 lanes added in channel
-// order, the reference's simdgroup sums (gdn.metal:215-222). In the recurrence a wave advances
+// order, the reference's simdgroup sums (gdn.metal:215-222). In the fold a wave advances
 // two state rows at once, one per half-wave, lane j of a half holding key columns 4 j .. 4 j + 3;
-// the row's products with k and q are tree sums over the half's 32 lanes, and each token keeps
-// the decay, memory, delta, update, output order of gdn.metal:270-298.
+// the row's products with k are tree sums over the half's 32 lanes, and each token keeps
+// the decay, memory, delta, update order of gdn.metal:270-298.
 //
 // The block's rows never advance the state: every row, of a chain block as of a tree block, takes its
 // output from the committed state (the reference does so for tree blocks, gdn.metal:417-478; a chain is
 // the tree whose every row follows the row before it): with S_j the state after the j-th token of a
 // row's path, S_j z = S_j-1 (d_j (z - c k_j)) + c v_j for c = beta_j (k_j . z), so the row's output is
-// S_-1 z_-1 + sum_j c_j v_j; a wave per row walks its path upward for z_-1 and the coefficients, and
-// the recurrence's waves add the path terms to the state's product with z_-1: one product with the
-// state a row instead of the four passes over it that advancing it takes.
+// S_-1 z_-1 + sum_j c_j v_j; a wave per row walks its path upward for z_-1 and the coefficients, the
+// folded state goes to LDS and meets the transformed queries of all rows on the matrix cores, and the
+// row's wave adds the path terms before it norms and gates them.
 #include "abi/Gdn.h"
 #include "abi/Gguf.h"
 #include "abi/PagedAttention.h"  // AttentionTreeRow
@@ -103,6 +103,8 @@ __device__ __forceinline__ void load_pending(const Tape &tape, Pending &pending,
 // `path` of `rows` (gdn_primitives.h:20-35).
 struct History {
   const uint16_t *row[kTaps - 1];
+  // Row `index` by selects: an indexed read would keep the rows in scratch.
+  __device__ __forceinline__ const uint16_t *at(uint32_t index) const { return index == 0 ? row[0] : index == 1 ? row[1] : row[2]; }
 };
 __device__ __forceinline__ History history_of(const uint16_t *carried, const uint16_t *rows, uint32_t conv_dim, uint32_t consumed,
                                               uint32_t path) {
@@ -236,8 +238,8 @@ __global__ __launch_bounds__(64 * kWaves) void gdn_decode(const uint16_t *__rest
                                                   const AttentionTreeRow *__restrict__ tree, uint8_t *__restrict__ table,
                                                   GdnDecodeParams p) {
   __shared__ __align__(16) uint16_t queries[kRows][kDim], keys[kRows][kDim], values[kRows][kDim], outputs[kRows][kDim];
-  __shared__ __align__(16) float transformed[kRows][kDim];
-  __shared__ float coefficients[kRows][kRows];
+  __shared__ __align__(16) float transformed[kRows][kDim + 4], committed[kDim][kDim + 4];   // rows of sixteen lanes in sixteen bank groups
+  __shared__ float products[2][kRows][kDim + 4], coefficients[kRows][kRows];
   __shared__ float decays[kRows];
   __shared__ uint16_t betas[kRows];
   __shared__ uint32_t paths[kRows];
@@ -271,10 +273,10 @@ __global__ __launch_bounds__(64 * kWaves) void gdn_decode(const uint16_t *__rest
 #pragma unroll
     for (uint32_t part = 0; part < 2; ++part) {
       const uint32_t d = lane + 64u * part;
-      carryV[part] = history.row[wave][vChannel + d];
+      carryV[part] = history.at(wave)[vChannel + d];
       if (sharedWriter) {
-        carryQ[part] = history.row[wave][qChannel + d];
-        carryK[part] = history.row[wave][kChannel + d];
+        carryQ[part] = history.at(wave)[qChannel + d];
+        carryK[part] = history.at(wave)[kChannel + d];
       }
     }
   }
@@ -292,7 +294,7 @@ __global__ __launch_bounds__(64 * kWaves) void gdn_decode(const uint16_t *__rest
       for (uint32_t tap = kTaps; tap-- > 0;) {
         const uint32_t row = up ? 31u - uint32_t(__builtin_clz(up)) : 0u;
         up &= ~(1u << row);
-        taps[tap] = depth + tap < kTaps - 1 ? history.row[depth + tap] : rowsIn + size_t(row) * P;
+        taps[tap] = depth + tap < kTaps - 1 ? history.at(depth + tap) : rowsIn + size_t(row) * P;
       }
     }
     const HeadRow row = head_row(taps, conv_weights, qChannel, kChannel, vChannel, lane);
@@ -369,7 +371,7 @@ __global__ __launch_bounds__(64 * kWaves) void gdn_decode(const uint16_t *__rest
     const uint32_t half = lane >> 5, column = 4u * (lane & 31u);
     for (uint32_t batch = 0; batch < kDim / (2u * kWaves); batch += kInFlight) {
       uint32_t valueDim[kInFlight];
-      float state[kInFlight][4], result[kInFlight];
+      float state[kInFlight][4];
 #pragma unroll
       for (int r = 0; r < kInFlight; ++r) {
         valueDim[r] = (batch + r) * 2u * kWaves + wave * 2u + half;
@@ -386,37 +388,50 @@ __global__ __launch_bounds__(64 * kWaves) void gdn_decode(const uint16_t *__rest
       for (int r = 0; r < kInFlight; ++r)
         *reinterpret_cast<float4 *>(stateOut + (size_t(head) * kDim + valueDim[r]) * kDim + column) =
             make_float4(state[r][0], state[r][1], state[r][2], state[r][3]);
-      for (uint32_t token = 0; token < rows; ++token) {
-        // The path's terms, a lane per block row, beside the committed state's product with the
-        // transformed query (gdn.metal:363-377).
-        const uint32_t j = lane & 31u, pathRowIndex = j & (kRows - 1u);
-        const bool onPath = j < kRows && ((paths[token] >> j) & 1u);
-        const float coefficient = coefficients[token][pathRowIndex];
-        const float4 zq = *reinterpret_cast<const float4 *>(&transformed[token][column]);
 #pragma unroll
-        for (int r = 0; r < kInFlight; ++r) {
-          result[r] = onPath ? coefficient * bf16_bits_to_float(values[pathRowIndex][valueDim[r]]) : 0.0f;
-          result[r] += state[r][0] * zq.x;
-          result[r] += state[r][1] * zq.y;
-          result[r] += state[r][2] * zq.z;
-          result[r] += state[r][3] * zq.w;
-          result[r] = half_sum(result[r]);
-        }
-        if ((lane & 31u) == 0) {
-#pragma unroll
-          for (int r = 0; r < kInFlight; ++r) outputs[token][valueDim[r]] = uint16_t(float_to_bf16_bits(result[r]));
-        }
-      }
+      for (int r = 0; r < kInFlight; ++r)
+        *reinterpret_cast<float4 *>(&committed[valueDim[r]][column]) = make_float4(state[r][0], state[r][1], state[r][2], state[r][3]);
     }
+  }
+  __syncthreads();
+
+  // ---- the committed state's products with the transformed queries (gdn.metal:363-377): wave w sixteen of the state's
+  // rows over half of their columns, for all the block's tokens (a token past them is a product that nothing reads). One matrix instruction's sums of
+  // four products each, added as a tree: against 64 bits 7.3e-8 of the terms' norm where a half-wave's tree of four-term
+  // chains was off by 7.6e-8 (with sixteen path terms 7.8e-8 for 8.1e-8). A block's rows were 0.8 us each in the state's
+  // registers, four 32-lane sums a wave; the kernel at 32 heads, as many pending rows as rows: 8 lanes of 16 rows 42.0 -> 32.8 us, of 4
+  // 19.2 -> 17.5, of 1 13.3 -> 13.7 (one form for every count, so that a row's bits do not depend on its block's). ----
+  {
+    const uint32_t tile = wave >> 1, from = (kDim / 2u) * (wave & 1u), line = lane & 15u, quarter = lane >> 4;
+    const f32x4 none = {};
+    f32x4 sums[4];
+#pragma unroll
+    for (uint32_t c = 0; c < 4; ++c) {
+      const float4 z = *reinterpret_cast<const float4 *>(&transformed[line][from + 16u * c + 4u * quarter]);
+      const float4 m = *reinterpret_cast<const float4 *>(&committed[16u * tile + line][from + 16u * c + 4u * quarter]);
+      sums[c] = (__builtin_amdgcn_mfma_f32_16x16x4f32(z.x, m.x, none, 0, 0, 0) + __builtin_amdgcn_mfma_f32_16x16x4f32(z.y, m.y, none, 0, 0, 0)) +
+                (__builtin_amdgcn_mfma_f32_16x16x4f32(z.z, m.z, none, 0, 0, 0) + __builtin_amdgcn_mfma_f32_16x16x4f32(z.w, m.w, none, 0, 0, 0));
+    }
+    const f32x4 sum = (sums[0] + sums[1]) + (sums[2] + sums[3]);
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) products[wave & 1u][4u * quarter + i][16u * tile + line] = sum[i];
   }
   __syncthreads();
 
   // ---- gated output norm (gdn.metal:489-526) ----
   const uint32_t outHead = (p.flags & GDN_TILED_HEADS) ? (head % perKey) * s.key_heads + head / perKey : head;
   for (uint32_t token = wave; token < rows; token += kWaves) {
-    float value[2];
+    // beside the products the path's terms, in block order: rows off the path are not touched, whatever they hold
+    float value[2] = {0.f, 0.f};
+    for (uint32_t path = paths[token]; path; path &= path - 1u) {
+      const uint32_t row = uint32_t(__builtin_ctz(path));
 #pragma unroll
-    for (uint32_t part = 0; part < 2; ++part) value[part] = bf16_bits_to_float(outputs[token][lane + 64u * part]);
+      for (uint32_t part = 0; part < 2; ++part)
+        value[part] = __fmaf_rn(coefficients[token][row], bf16_bits_to_float(values[row][lane + 64u * part]), value[part]);
+    }
+#pragma unroll
+    for (uint32_t part = 0; part < 2; ++part)
+      value[part] = round_bf16(value[part] + (products[0][token][lane + 64u * part] + products[1][token][lane + 64u * part]));
     uint32_t gated[2];
     gated_norm(value, norm_weight, p.flags, rowsIn + size_t(token) * P + zOffset + head * kDim, lane, gated);
 #pragma unroll
