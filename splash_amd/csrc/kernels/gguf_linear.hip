@@ -711,36 +711,56 @@ __device__ __forceinline__ void decode_workgroup(DecodeShared<RT> &shared, const
     const uint32_t sumsAt = kSums32 && !kPairSums ? gguf_table_sums32_offset(p.input_size, tiles) : gguf_table_sums16_offset(p.input_size, tiles);
     const uint32_t sumGroups = kSums32 ? G : 2u * G;  // row-sum entries per row tile
     const Resource sums = make_resource(table + sumsAt, tiles * (kPairSums ? 2u * G : sumGroups) * 64u);
-    // Threads past the staged sums repeat an earlier thread's (same value to the same slot).
-    uint32_t sumShare[kSumShare], sumSlot[kSumShare];
-#pragma unroll
-    for (int q = 0; q < kSumShare; ++q) {
-      const uint32_t at = (threadIdx.x + 256u * q) % kSumFloats;
+    // Threads past the staged sums repeat an earlier thread's (same value to the same slot). A thread's q-th sum lies
+    // whole row tiles past its first: its place and its address are the first's and a uniform step.
+    constexpr uint32_t kTileStep = 256u / (kSumsPerBlock * 64u);
+    static_assert(kSumShare == 1 || kSumFloats % 256u == 0, "a thread's sums lie whole row tiles apart");
+    uint32_t sumShare, sumSlot;
+    {
+      const uint32_t at = threadIdx.x % kSumFloats;
       const uint32_t t = at / (kSumsPerBlock * 64u), j = (at / 64u) % kSumsPerBlock, l = at % 64u;
-      sumShare[q] = ((t * sumGroups + kSumsPerBlock * 4u * b0 + 4u * j + (l >> 4)) * 16u * (kPairSums ? 2u : 1u) + (l & 15u)) * 4u;
-      sumSlot[q] = (t * 4u + j) * 64u + l;
+      sumShare = ((t * sumGroups + kSumsPerBlock * 4u * b0 + 4u * j + (l >> 4)) * 16u * (kPairSums ? 2u : 1u) + (l & 15u)) * 4u;
+      sumSlot = (t * 4u + j) * 64u + l;
     }
+    const uint32_t sumStep = kTileStep * sumGroups * 64u * (kPairSums ? 2u : 1u);
     auto issueTable = [&](Stage &st) {
 #pragma unroll
       for (int j = 0; j < 2 * RT; ++j) st.a[j] = load128<0>(values[j / 2], share[j % 2]);
 #pragma unroll
       for (int q = 0; q < kSumShare; ++q)
-        st.sum[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sums, int(sumShare[q]), 0, 0));
+        st.sum[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sums, int(sumShare + q * sumStep), 0, 0));
       if constexpr (kPairSums) {
 #pragma unroll
         for (int q = 0; q < kSumShare; ++q)
-          st.second[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sums, int(sumShare[q] + 64u), 0, 0));
+          st.second[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sums, int(sumShare + q * sumStep + 64u), 0, 0));
       }
 #pragma unroll
       for (int j = 0; j < 2; ++j) share[j] += 8192u;
       // Sums past the range are the next range's or, past the table, zeros: staged and never used.
-#pragma unroll
-      for (int q = 0; q < kSumShare; ++q) sumShare[q] += kSumsPerBlock * 4u * 16u * 4u * (kPairSums ? 2u : 1u);
+      sumShare += kSumsPerBlock * 4u * 16u * 4u * (kPairSums ? 2u : 1u);
     };
+    // A Q6_K wave of four row tiles has no register left for its lane's three places in a record: it works them out for
+    // each. (Kept, one was spilled and read back behind the loads just issued, and the wait for it was the wait for all
+    // of them: the vector-memory counter is one queue. 64 rows of 17408 -> 5120 57.1 -> 53.3 us, 5120 -> 17408 59.5 -> 52.7,
+    // 5120 -> 8192 Q4_K and 6144 Q6_K columns in one dispatch, at two waves a SIMD before and three now, 44.0 -> 38.9.)
+    constexpr bool kFreshLane = FMT == GGUF_FMT_Q6K && RT > 2;
+    uint32_t record = 0;
     auto issueWeights = [&](Stage &st) {
-      load_record(st.rec, weights, mine, column);
-      mine += kRecord;
-      column += kRecord;
+      if constexpr (kFreshLane) {
+        uint32_t l;
+        asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+        const uint32_t first = record + 16u * l, mine16 = record + kColumnPart + 16u * (l & 15u);
+        st.rec.n0 = load128<kStreamOnce>(weights, first);
+        st.rec.n1 = load128<kStreamOnce>(weights, first + 1024u);
+        st.rec.high = load128<kStreamOnce>(weights, first + 2048u);
+        st.rec.scales = load128<kStreamOnce>(weights, mine16);
+        st.rec.d = __builtin_amdgcn_raw_buffer_load_b16(weights, int(record + GGUF_Q6K_D + 2u * (l & 15u)), 0, kStreamOnce);
+        record += kRecord;
+      } else {
+        load_record(st.rec, weights, mine, column);
+        mine += kRecord;
+        column += kRecord;
+      }
     };
     auto issue = [&](Stage &st) {
       issueTable(st);
@@ -831,7 +851,7 @@ __device__ __forceinline__ void decode_workgroup(DecodeShared<RT> &shared, const
         for (int j = 0; j < 2 * RT; ++j) (&ldsA[buffer][0][0][0])[threadIdx.x + 256u * j] = stage[u].a[j];
 #pragma unroll
         for (int q = 0; q < kSumShare; ++q)
-          (&ldsSums[buffer][0][0][0])[sumSlot[q]] = kPairSums ? stage[u].sum[q] + stage[u].second[q] : stage[u].sum[q];
+          (&ldsSums[buffer][0][0][0])[sumSlot + q * kTileStep * 256u] = kPairSums ? stage[u].sum[q] + stage[u].second[q] : stage[u].sum[q];
         __syncthreads();
         issue(stage[(u + kStages - 1) % kStages]);
         if (now < count) {
@@ -1176,8 +1196,12 @@ __device__ __forceinline__ void decode_workgroup(DecodeShared<RT> &shared, const
   }
 }
 
+// Three waves a SIMD (168 registers) where a kernel would take a few registers more and run two: every format's four row
+// tiles, and Q6_K's two under some epilogues (a step of 8 layers and 24 rows in three lanes, whose down projections take the residual
+// and norm, 1755 -> 1670 us). Four (128) for Q6_K's one row tile spill outside the loop and are slower (16 rows 1307 ->
+// 1342 us a step).
 template <uint32_t FMT, int RT, uint32_t EP, bool Staged = false>
-__global__ __launch_bounds__(256, RT > 2 ? 3 : 1) void gguf_decode(const uint8_t *__restrict__ seg0, const uint8_t *__restrict__ seg1,
+__global__ __launch_bounds__(256, RT > 2 || (RT == 2 && FMT == GGUF_FMT_Q6K) ? 3 : 1) void gguf_decode(const uint8_t *__restrict__ seg0, const uint8_t *__restrict__ seg1,
                                                    const uint8_t *__restrict__ seg2, const uint8_t *__restrict__ table,
                                                    void *__restrict__ out, const uint16_t *__restrict__ residual,
                                                    float *__restrict__ partials, uint32_t *__restrict__ counters,
@@ -1206,7 +1230,7 @@ __global__ __launch_bounds__(256, RT > 2 ? 3 : 1) void gguf_decode(const uint8_t
 // columns), every workgroup takes one of p.splits parts of K (whole_groups 0), and a workgroup runs its segment's
 // format as a projection of that segment alone, its partials and counters after those of the segments before it.
 template <int RT>
-__global__ __launch_bounds__(256) void gguf_decode_mixed(const uint8_t *__restrict__ seg0, const uint8_t *__restrict__ seg1,
+__global__ __launch_bounds__(256, RT > 2 ? 3 : 1) void gguf_decode_mixed(const uint8_t *__restrict__ seg0, const uint8_t *__restrict__ seg1,
                                                          const uint8_t *__restrict__ seg2, const uint8_t *__restrict__ table,
                                                          void *__restrict__ out, const uint16_t *__restrict__ residual,
                                                          float *__restrict__ partials, uint32_t *__restrict__ counters,
