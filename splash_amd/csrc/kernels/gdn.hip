@@ -532,25 +532,26 @@ SP_REGISTER_KERNEL("gdn_fold", &gdn_fold);
 // blocks. Only the outputs differ in form: here a row reads the state after its own token, o = S_t q_t
 // (gdn.metal:291-298), where a verify block's rows read the state before the block.
 
-// gdn_prefill_prepare: grid (value_heads, ceil(tokens / 4)), 256 threads, a wave per (row, value head),
-// lane l the dimensions l and 64 + l: convolution + SiLU, q/k norms, gates (prefill/gdn.metal:196-262).
-// The head's value rows, its gates and, from the first value head of a key head, the key head's query
-// and key rows leave to the run's buffers; the workgroups of the first rows also write the convolution
-// carry after the run's last row.
+// gdn_prefill_prepare: grid (2 key_heads + value_heads, ceil(tokens / (4 GDN_PREPARE_ROWS))), 256 threads, a wave per run
+// of GDN_PREPARE_ROWS rows and head of the convolution's channels (the query heads, the key heads, then the value heads),
+// lane l the dimensions l and 64 + l: convolution + SiLU, the norm of a query or key head, a value head's gates with a
+// lane a row (prefill/gdn.metal:196-262). The workgroups of the first rows also write the convolution carry after the
+// run's last row. Bound by its vector instructions (silu's correctly rounded division, the roundings): a wave reads a
+// row's inputs and widens them once for the four taps that use them, and a key head that two value heads share is worked
+// out once, where a wave per (row, value head) did both over again. 2048 rows of 16 / 32 heads: 63 us that way, 34 so.
 __global__ __launch_bounds__(256) void gdn_prefill_prepare(const uint16_t *__restrict__ packed, const uint16_t *__restrict__ conv_weights,
                                                            uint8_t *__restrict__ states, const float *__restrict__ a_scale,
                                                            const uint16_t *__restrict__ dt_bias, uint16_t *__restrict__ queries,
                                                            uint16_t *__restrict__ keys, uint16_t *__restrict__ values,
                                                            float *__restrict__ decay, uint16_t *__restrict__ beta, GdnPrefillParams p) {
-  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, head = blockIdx.x, token = blockIdx.y * 4u + wave;
+  constexpr uint32_t R = GDN_PREPARE_ROWS;
+  const uint32_t lane = threadIdx.x & 63u, wave = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6))), unit = blockIdx.x;
+  const uint32_t firstRow = (blockIdx.y * 4u + wave) * R;
   const GdnShapeParams s = p.shape;
-  const uint32_t perKey = s.value_heads / s.key_heads, keyHead = head / perKey, keyWidth = s.key_heads * kDim;
-  const uint32_t valueWidth = s.value_heads * kDim, C = s.conv_dim, P = s.packed_width;
-  const uint32_t bOffset = C + valueWidth, aOffset = bOffset + s.value_heads;
-  const bool sharedWriter = head % perKey == 0;
+  const uint32_t keyWidth = s.key_heads * kDim, valueWidth = s.value_heads * kDim, C = s.conv_dim, P = s.packed_width;
+  const uint32_t bOffset = C + valueWidth, aOffset = bOffset + s.value_heads, channel = unit * kDim;
   const uint16_t *convIn = reinterpret_cast<const uint16_t *>(states + p.current_cell + uint64_t(p.layer) * p.conv_layer_bytes);
   uint16_t *convOut = reinterpret_cast<uint16_t *>(states + p.next_cell + uint64_t(p.layer) * p.conv_layer_bytes);
-  const uint32_t qChannel = keyHead * kDim, kChannel = keyWidth + keyHead * kDim, vChannel = 2 * keyWidth + head * kDim;
   // input position i of the run's history: the carried rows, then the run's own (gdn_primitives.h:20-35)
   auto input = [&](uint32_t position) __attribute__((always_inline)) -> const uint16_t * {
     return position < kTaps - 1 ? convIn + size_t(position) * C : packed + size_t(p.first + position - (kTaps - 1)) * P;
@@ -558,34 +559,51 @@ __global__ __launch_bounds__(256) void gdn_prefill_prepare(const uint16_t *__res
   if (blockIdx.y == 0 && wave < kTaps - 1) {
     const uint16_t *source = input(p.tokens + wave);
 #pragma unroll
-    for (uint32_t part = 0; part < 2; ++part) {
-      const uint32_t d = lane + 64u * part;
-      convOut[size_t(wave) * C + vChannel + d] = source[vChannel + d];
-      if (sharedWriter) {
-        convOut[size_t(wave) * C + qChannel + d] = source[qChannel + d];
-        convOut[size_t(wave) * C + kChannel + d] = source[kChannel + d];
-      }
-    }
+    for (uint32_t part = 0; part < 2; ++part) convOut[size_t(wave) * C + channel + lane + 64u * part] = source[channel + lane + 64u * part];
   }
-  if (token >= p.tokens) return;
-  const uint16_t *taps[kTaps];
-#pragma unroll
-  for (uint32_t tap = 0; tap < kTaps; ++tap) taps[tap] = input(token + tap);
-  const HeadRow row = head_row(taps, conv_weights, qChannel, kChannel, vChannel, lane);
-  const size_t at = size_t(p.first) + token;  // the row's place in the chunk's buffers
+  if (firstRow >= p.tokens) return;
+  const uint32_t rows = min(R, p.tokens - firstRow);
+  float taps[2][kTaps], inputs[2][R + kTaps - 1];
 #pragma unroll
   for (uint32_t part = 0; part < 2; ++part) {
-    const uint32_t d = lane + 64u * part;
-    values[at * valueWidth + head * kDim + d] = uint16_t(row.value[part]);
-    if (sharedWriter) {
-      queries[at * keyWidth + keyHead * kDim + d] = uint16_t(row.query[part]);
-      keys[at * keyWidth + keyHead * kDim + d] = uint16_t(row.key[part]);
-    }
+    const uint32_t d = channel + lane + 64u * part;
+#pragma unroll
+    for (uint32_t i = 0; i < R + kTaps - 1; ++i)   // the last row's last input again past the run's end
+      inputs[part][i] = bf16_bits_to_float(input(firstRow + min(i, rows + kTaps - 2u))[d]);
+#pragma unroll
+    for (uint32_t tap = 0; tap < kTaps; ++tap) taps[part][tap] = bf16_bits_to_float(conv_weights[size_t(d) * kTaps + tap]);
   }
-  if (lane == 0) {
-    const Gates gates = gates_of(packed + at * P, bOffset, aOffset, head, a_scale, dt_bias);
-    beta[at * s.value_heads + head] = uint16_t(gates.beta);
-    decay[at * s.value_heads + head] = gates.decay;
+  const size_t at = size_t(p.first) + firstRow;  // the run of rows' place in the chunk's buffers
+  const bool query = unit < s.key_heads, key = !query && unit < 2u * s.key_heads;
+  uint16_t *out = (query ? queries + at * keyWidth + channel : key ? keys + at * keyWidth + (channel - keyWidth)
+                                                                  : values + at * valueWidth + (channel - 2u * keyWidth)) + lane;
+  const uint32_t width = query || key ? keyWidth : valueWidth;
+  const float scaleAfter = query ? 0.0078125f : 0.08838834765f;
+#pragma unroll
+  for (uint32_t r = 0; r < R; ++r) {
+    if (r >= rows) break;
+    float x[2];
+#pragma unroll
+    for (uint32_t part = 0; part < 2; ++part) {
+      float value = 0.f;   // conv_silu's sum
+#pragma unroll
+      for (uint32_t tap = 0; tap < kTaps; ++tap) value += inputs[part][r + tap] * taps[part][tap];
+      x[part] = round_bf16(silu_of(round_bf16(value)));
+    }
+    if (query || key) {
+      const float scale = 1.0f / sqrtf(head_sum(x[0] * x[0], x[1] * x[1]) / float(kDim) + 1e-6f);
+#pragma unroll
+      for (uint32_t part = 0; part < 2; ++part) x[part] = round_bf16(x[part] * scale) * scaleAfter;
+    }
+#pragma unroll
+    for (uint32_t part = 0; part < 2; ++part) out[size_t(r) * width + 64u * part] = uint16_t(float_to_bf16_bits(x[part]));
+  }
+  if (!query && !key && lane < rows) {
+    const uint32_t head = unit - 2u * s.key_heads;
+    const size_t row = at + lane;
+    const Gates gates = gates_of(packed + row * P, bOffset, aOffset, head, a_scale, dt_bias);
+    beta[row * s.value_heads + head] = uint16_t(gates.beta);
+    decay[row * s.value_heads + head] = gates.decay;
   }
 }
 SP_REGISTER_KERNEL("gdn_prefill_prepare", &gdn_prefill_prepare);

@@ -135,7 +135,7 @@ void GDN::addPrefill(hip::CommandGraph &graph, const GdnPrefillBuffers &b, const
     params.next_cell = out;
     graph.add("gdn_prefill_prepare",
               {b.packed, b.convolutionWeights, b.states, b.decayWeights, b.timeBias, b.queries, b.keys, b.values, b.decay, b.beta}, params,
-              {shape.valueHeads, (params.tokens + 3) / 4, 1}, {256, 1, 1});
+              {2 * shape.keyHeads + shape.valueHeads, (params.tokens + 4 * GDN_PREPARE_ROWS - 1) / (4 * GDN_PREPARE_ROWS), 1}, {256, 1, 1});
     if (b.blocks) {
       graph.add("gdn_prefill_blocks", {b.queries, b.keys, b.decay, b.beta, b.blocks}, params,
                 {shape.valueHeads, ((params.tokens + GDN_SCAN_BLOCK - 1) / GDN_SCAN_BLOCK + 3) / 4, 1}, {256, 1, 1});
