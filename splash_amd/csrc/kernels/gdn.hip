@@ -174,19 +174,28 @@ __device__ __forceinline__ Gates gates_of(const uint16_t *inputs, uint32_t bOffs
 // The gated output norm of a row's 128 recurrent values of one head, lane l the dimensions l and
 // 64 + l, as bf16 bits (gdn.metal:489-526): RMS norm with the mixer's weight, rounded, times silu(z)
 // (or sigmoid(z)) of the row's gate columns `z`.
-__device__ __forceinline__ void gated_norm(const float (&value)[2], const void *norm_weight, uint32_t flags, const uint16_t *z_row,
-                                           uint32_t lane, uint32_t (&bits)[2]) {
+__device__ __forceinline__ float norm_weight_of(const void *norm_weight, uint32_t flags, uint32_t d) {
+  return (flags & GDN_FLOAT_NORM) ? static_cast<const float *>(norm_weight)[d] : bf16_bits_to_float(static_cast<const uint16_t *>(norm_weight)[d]);
+}
+__device__ __forceinline__ void gated_values(const float (&value)[2], const float (&weight)[2], const float (&z)[2], uint32_t flags,
+                                             uint32_t (&bits)[2]) {
   const float inverse = 1.0f / sqrtf(head_sum(value[0] * value[0], value[1] * value[1]) / float(kDim) + 1e-6f);
 #pragma unroll
   for (uint32_t part = 0; part < 2; ++part) {
-    const uint32_t d = lane + 64u * part;
-    const float weight = (flags & GDN_FLOAT_NORM) ? static_cast<const float *>(norm_weight)[d]
-                                                  : bf16_bits_to_float(static_cast<const uint16_t *>(norm_weight)[d]);
-    const float normalized = round_bf16((value[part] * inverse) * weight);
-    const float z = bf16_bits_to_float(z_row[d]);
-    const float gated = (normalized * ((flags & GDN_SIGMOID_GATE) ? 1.0f : z)) / (1.0f + exp2_fast(-kLog2e * z));
+    const float normalized = round_bf16((value[part] * inverse) * weight[part]);
+    const float gated = (normalized * ((flags & GDN_SIGMOID_GATE) ? 1.0f : z[part])) / (1.0f + exp2_fast(-kLog2e * z[part]));
     bits[part] = float_to_bf16_bits(gated);
   }
+}
+__device__ __forceinline__ void gated_norm(const float (&value)[2], const void *norm_weight, uint32_t flags, const uint16_t *z_row,
+                                           uint32_t lane, uint32_t (&bits)[2]) {
+  float weight[2], z[2];
+#pragma unroll
+  for (uint32_t part = 0; part < 2; ++part) {
+    weight[part] = norm_weight_of(norm_weight, flags, lane + 64u * part);
+    z[part] = bf16_bits_to_float(z_row[lane + 64u * part]);
+  }
+  gated_values(value, weight, z, flags, bits);
 }
 
 // One token's delta-rule step on the wave's state rows (R pairs, a row per half-wave): decay,
@@ -1114,26 +1123,41 @@ __global__ __launch_bounds__(320, 1) void gdn_prefill_block_scan(const uint16_t 
 }
 SP_REGISTER_KERNEL("gdn_prefill_block_scan", &gdn_prefill_block_scan);
 
-// gdn_prefill_gate: grid (value_heads, ceil(tokens / 4)), 256 threads, a wave per (row, value head): the gated
-// output norm of the scan's rows (prefill/gdn.metal:312-341, gdn.metal:489-526).
+// gdn_prefill_gate: grid (value_heads, ceil(tokens / (4 GDN_GATE_ROWS))), 256 threads, a wave per GDN_GATE_ROWS rows of a
+// value head: the gated output norm of the scan's rows (prefill/gdn.metal:312-341, gdn.metal:489-526). A wave of one row
+// only waited for its four loads: 2048 rows of 32 heads 28 us so, 17.6 with the rows' loads out together.
 __global__ __launch_bounds__(256) void gdn_prefill_gate(const uint16_t *__restrict__ recurrent_rows, const uint16_t *__restrict__ packed,
                                                         const void *__restrict__ norm_weight, uint16_t *__restrict__ hidden,
                                                         GdnPrefillParams p) {
-  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, head = blockIdx.x;
-  if (blockIdx.y * 4u + wave >= p.tokens) return;
-  const size_t token = size_t(p.first) + blockIdx.y * 4u + wave;
+  constexpr uint32_t R = GDN_GATE_ROWS;
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, head = blockIdx.x, firstRow = (blockIdx.y * 4u + wave) * R;
+  if (firstRow >= p.tokens) return;
+  const uint32_t rows = min(R, p.tokens - firstRow);
+  const size_t first = size_t(p.first) + firstRow;
   const GdnShapeParams s = p.shape;
   const uint32_t perKey = s.value_heads / s.key_heads, valueWidth = s.value_heads * kDim;
   const uint32_t outHead = (p.flags & GDN_TILED_HEADS) ? (head % perKey) * s.key_heads + head / perKey : head;
-  float value[2];
+  float value[R][2], z[R][2], weight[2];
 #pragma unroll
-  for (uint32_t part = 0; part < 2; ++part)
-    value[part] = bf16_bits_to_float(recurrent_rows[token * valueWidth + head * kDim + lane + 64u * part]);
-  uint32_t gated[2];
-  gated_norm(value, norm_weight, p.flags, packed + token * s.packed_width + s.conv_dim + head * kDim, lane, gated);
+  for (uint32_t r = 0; r < R; ++r) {
+    const size_t token = first + min(r, rows - 1u);   // the last row again past the run's end
 #pragma unroll
-  for (uint32_t part = 0; part < 2; ++part)
-    hidden[(token * s.value_heads + outHead) * kDim + lane + 64u * part] = uint16_t(gated[part]);
+    for (uint32_t part = 0; part < 2; ++part) {
+      value[r][part] = bf16_bits_to_float(recurrent_rows[token * valueWidth + head * kDim + lane + 64u * part]);
+      z[r][part] = bf16_bits_to_float(packed[token * s.packed_width + s.conv_dim + head * kDim + lane + 64u * part]);
+    }
+  }
+#pragma unroll
+  for (uint32_t part = 0; part < 2; ++part) weight[part] = norm_weight_of(norm_weight, p.flags, lane + 64u * part);
+#pragma unroll
+  for (uint32_t r = 0; r < R; ++r) {
+    if (r >= rows) break;
+    uint32_t gated[2];
+    gated_values(value[r], weight, z[r], p.flags, gated);
+#pragma unroll
+    for (uint32_t part = 0; part < 2; ++part)
+      hidden[((first + r) * s.value_heads + outHead) * kDim + lane + 64u * part] = uint16_t(gated[part]);
+  }
 }
 SP_REGISTER_KERNEL("gdn_prefill_gate", &gdn_prefill_gate);
 

@@ -148,8 +148,8 @@ void GDN::addPrefill(hip::CommandGraph &graph, const GdnPrefillBuffers &b, const
   }
   params.first = 0;
   params.tokens = tokens;
-  graph.add("gdn_prefill_gate", {b.recurrentRows, b.packed, b.mixerNorm, b.hidden}, params, {shape.valueHeads, (tokens + 3) / 4, 1},
-            {256, 1, 1});
+  graph.add("gdn_prefill_gate", {b.recurrentRows, b.packed, b.mixerNorm, b.hidden}, params,
+            {shape.valueHeads, (tokens + 4 * GDN_GATE_ROWS - 1) / (4 * GDN_GATE_ROWS), 1}, {256, 1, 1});
 }
 
 void GDN::addFold(hip::CommandGraph &graph, const GdnFoldBuffers &b, const GdnShape &shape, uint32_t layers, uint32_t rows,

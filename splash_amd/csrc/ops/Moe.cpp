@@ -220,8 +220,14 @@ void MoE::addChunk(hip::CommandGraph &graph, const hip::Buffer &scores, uint32_t
   project("gguf_wide_moe_gather", normalized, rows, shape.hidden, shape.ffn, experts.format, pairBytes, experts.gate, experts.up, w.intermediate, true);
   project("gguf_wide_moe_rows", w.intermediate, 16 * tiles, shape.ffn, shape.hidden, experts.downFormat, downBytes, experts.down, experts.down,
           w.expertOutput, false);
-  graph.add("moe_combine", {w.expertOutput, w.routeSlot, w.weights, residual, output, output, output},
-            MoeCombineParams{rows, shape.hidden, shape.routesPerRow(), 0u}, {rows, (shape.hidden + 255) / 256, 1}, {256, 1, 1});
+  // whole 16-byte vectors of a row, or a column a thread
+  const MoeCombineParams combine{rows, shape.hidden, shape.routesPerRow(), 0u};
+  if (shape.hidden % 8 == 0 && w.expertOutput.gpuAddress() % 16 == 0 && residual.gpuAddress() % 16 == 0 && output.gpuAddress() % 16 == 0)
+    graph.add("moe_combine_rows", {w.expertOutput, w.routeSlot, w.weights, residual, output}, combine,
+              {rows, (shape.hidden + 2047) / 2048, 1}, {256, 1, 1});
+  else
+    graph.add("moe_combine", {w.expertOutput, w.routeSlot, w.weights, residual, output, output, output}, combine,
+              {rows, (shape.hidden + 255) / 256, 1}, {256, 1, 1});
 }
 
 } // namespace splash::ops
