@@ -71,6 +71,13 @@ struct DraftLanesParams {
   uint32_t lanes;
 };
 
+// draft_attention_merge: grid (8 KV heads, lanes), 1024 threads. `table_tiles` row tiles of the merged rows' activation
+// table (abi/Gguf.h), 0 for none.
+struct DraftMergeParams {
+  uint32_t lanes;
+  uint32_t table_tiles;
+};
+
 // draft_attention_split: grid (8 KV heads, lanes, 17), 256 threads.
 // Lane l's key ring starts keys[l] bytes into the bound rings buffer, its value ring values[l] bytes.
 struct DraftAttentionParams {

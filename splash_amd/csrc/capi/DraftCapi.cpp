@@ -145,6 +145,8 @@ struct spo_dflash_draft {
       decode.scratch = {device(size.input, "draft linear table"), device(size.partials, "draft linear partials"),
                         device(size.counters, "draft linear counters")};
       context.scratch = decode.scratch;
+      decode.intermediateTable = device(gguf_tables_bytes(weights.layout.intermediateSize, gguf_row_tiles(maxLanes * DRAFT_ATTENTION_QUERY_ROWS)),
+                                        "draft intermediate table");
     }
     return *draft;
   }

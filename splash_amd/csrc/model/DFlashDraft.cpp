@@ -110,8 +110,8 @@ void DFlashDraft::addDecode(hip::CommandGraph &graph, const DFlashDecodeBuffers 
     ops::DraftAttention::addPrepare(graph, {b.proposalQkv, b.attention, w.queryNorm, w.keyNorm, b.ropeCos, b.ropeSin, b.queryKeys, b.queryValues},
                                     plan);
     ops::DraftAttention::addDecode(graph, {b.attention, ringsOf(b.rings, lanes, index, keys, values), b.queryKeys, b.queryValues}, cacheLengths,
-                                   plan);
-    linear_.addProjection(graph, b.attention, w.outputProjection, b.projected, rows, b.scratch);
+                                   plan, b.scratch.input);
+    project(b.attention, w.outputProjection, b.projected, {b.attention, ops::LinearInput::Table16});
     normalized = ops::DraftAttention::addConvolutionTable(graph, {b.projected, b.dynamic, w.attentionConvolution, current, b.residual}, plan,
                                                           ops::DraftConvolutionStage::Residual, w.postAttentionNorm, b.normalized, b.scratch);
     // MLP: norm -> dynamic weights -> convolution -> SwiGLU -> down -> convolution with the residual
@@ -123,8 +123,17 @@ void DFlashDraft::addDecode(hip::CommandGraph &graph, const DFlashDecodeBuffers 
     pair.output = b.intermediate;
     pair.scratch = b.scratch;
     pair.prepared = convolved;
+    pair.nextTable = b.intermediateTable;
     linear_.add(graph, pair, w.upProjection, linear_.plan(w.upProjection, rows, ops::LinearEpilogue::GateUp), &w.gateProjection);
-    linear_.addProjection(graph, b.intermediate, w.downProjection, b.projected, rows, b.scratch);
+    ops::LinearBuffers down;
+    down.input = b.intermediate;
+    down.output = b.projected;
+    down.scratch = b.scratch;
+    if (b.intermediateTable) {
+      down.scratch.input = b.intermediateTable;
+      down.prepared = {b.intermediate, ops::LinearInput::Table16};
+    }
+    linear_.add(graph, down, w.downProjection, linear_.plan(w.downProjection, rows));
     // (the last layer's rows take the final norm, into the head's input)
     normalized = ops::DraftAttention::addConvolutionTable(
         graph, {b.projected, b.dynamic, w.mlpConvolution, b.residual, next}, plan, ops::DraftConvolutionStage::Residual,

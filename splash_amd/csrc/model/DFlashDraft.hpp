@@ -75,6 +75,9 @@ struct DFlashDecodeBuffers final {
   ops::LinearScratch scratch;
   std::array<hip::Buffer, 2> hidden;  // bf16 [lanes * 8][hidden]: layer l reads hidden[l & 1]
   hip::Buffer normalized, dynamic, convolved, proposalQkv, attention, projected, residual, intermediate;
+  // The activation table of the intermediate rows, beside scratch.input (which the gate/up pass reads): written by that
+  // pass's epilogue, where given, instead of by a pass of its own.
+  hip::Buffer intermediateTable;
   hip::Buffer finalHidden;     // bf16 [lanes * 8][hidden]
   hip::Buffer logits;          // fp32 [lanes * 8][vocabulary]
   hip::Buffer selectorHidden;  // bf16 [lanes * 8][DRAFT_SELECTOR_RANK]

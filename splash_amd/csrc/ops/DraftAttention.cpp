@@ -139,9 +139,11 @@ void DraftAttention::addPrepare(hip::CommandGraph &graph, const DraftPrepareBuff
 }
 
 void DraftAttention::addDecode(hip::CommandGraph &graph, const DraftDecodeAttentionBuffers &buffers, std::span<const uint32_t> cacheLengths,
-                               const DraftAttentionPlan &plan) {
+                               const DraftAttentionPlan &plan, const hip::Buffer &table) {
   const DraftAttentionWorkspace workspace = plan.workspace();
-  const uint32_t lanes = plan.lanes();
+  const uint32_t lanes = plan.lanes(), tiles = gguf_row_tiles(lanes * DRAFT_ATTENTION_QUERY_ROWS);
+  static_assert(DRAFT_ATTENTION_MAXIMUM_LANES * DRAFT_ATTENTION_QUERY_ROWS <= 16u * GGUF_PIECE_TILES, "the lanes' rows are one piece of a table");
+  if (table) requireBytes(table, gguf_tables_bytes(DRAFT_ATTENTION_WIDTH, tiles), "draft attention table");
   if (cacheLengths.size() != lanes) throw std::invalid_argument("invalid draft attention geometry");
   requireBytes(buffers.groupedQueries, workspace.groupedQueriesBytes, "draft grouped queries");
   requireBytes(buffers.queryKeys, workspace.queryKeysBytes, "draft query keys");
@@ -158,8 +160,8 @@ void DraftAttention::addDecode(hip::CommandGraph &graph, const DraftDecodeAttent
   const hip::Buffer partials = buffers.groupedQueries.slice(queryRowsBytes(plan), workspace.groupedQueriesBytes - queryRowsBytes(plan));
   graph.add("draft_attention_split", {buffers.groupedQueries, buffers.rings.buffer, buffers.queryKeys, buffers.queryValues, partials}, params,
             {DRAFT_ATTENTION_KV_HEADS, lanes, DRAFT_ATTENTION_SPLITS});
-  graph.add("draft_attention_merge", {partials, buffers.groupedQueries}, DraftLanesParams{lanes}, {DRAFT_ATTENTION_KV_HEADS, lanes, 1},
-            {1024, 1, 1});
+  graph.add("draft_attention_merge", {partials, buffers.groupedQueries, table ? table : buffers.groupedQueries},
+            DraftMergeParams{lanes, table ? tiles : 0u}, {DRAFT_ATTENTION_KV_HEADS, lanes, 1}, {1024, 1, 1});
 }
 
 void DraftAttention::addContextPrefill(hip::CommandGraph &graph, const hip::Buffer &contextKv, const hip::Buffer &keyNorm,

@@ -103,8 +103,9 @@ public:
                                            DraftConvolutionStage stage, const hip::Buffer &normWeight, const hip::Buffer &normalized,
                                            const LinearScratch &scratch);
   static void addPrepare(hip::CommandGraph &graph, const DraftPrepareBuffers &buffers, const DraftAttentionPlan &plan);
+  // With a `table`, the merged rows also leave as the activation table of the projection that reads them.
   static void addDecode(hip::CommandGraph &graph, const DraftDecodeAttentionBuffers &buffers, std::span<const uint32_t> cacheLengths,
-                        const DraftAttentionPlan &plan);
+                        const DraftAttentionPlan &plan, const hip::Buffer &table = {});
   // The context writers. A row of contextKv holds its keys, then its values (1024 each); its normalized, rotated keys
   // and its values go to its position's slot of the ring. The prefill writes `tokens` rows of one lane from
   // startPosition on, row r rotated by RoPE row r.
