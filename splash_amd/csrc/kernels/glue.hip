@@ -15,21 +15,32 @@ namespace splash::kernels {
 // (a row's columns are read twice, in an order no vector load gives directly).
 constexpr uint32_t kStagedWidth = NORM_STAGED_WIDTH;
 
-// Copies `width` bf16 values (a multiple of 8, 16-byte aligned) to LDS; no barrier.
-__device__ __forceinline__ void stage_row(const uint16_t *__restrict__ source, uint32_t width, uint16_t *lds) {
-  const uint32_t vectors = width / 8u;
-  uint4 held[kStagedWidth / 8u / 256u];
+// `v` has arrived: nothing that uses it moves above this, and its load does not move below. A load that is sunk to its use
+// under a condition is waited for alone, one round trip each.
+__device__ __forceinline__ void arrived(uint4 &v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)); }
+__device__ __forceinline__ void arrived(uint32_t &v) { asm volatile("" : "+v"(v)); }
+
+// `width` bf16 values (a multiple of 8, 16-byte aligned) on their way to LDS: every load of it goes out before any is stored,
+// and those of several rows before the first row's stores. No barrier. (With the loads sunk
+// to their stores the norm and its table were 7.9 us at 8 rows of 5120, 6.6 so; at 128 rows of 2048 5.8 either way.)
+struct StagedRow {
+  static constexpr uint32_t kHeld = kStagedWidth / 8u / 256u;
+  uint4 held[kHeld];
+  __device__ __forceinline__ void load(const uint16_t *__restrict__ source, uint32_t width) {
 #pragma unroll
-  for (uint32_t i = 0; i < kStagedWidth / 8u / 256u; ++i) {
-    // (the last vector again past the row's end: a read under a condition is waited for before the next and kept in scratch)
-    held[i] = reinterpret_cast<const uint4 *>(source)[min(threadIdx.x + 256u * i, vectors - 1u)];
+    for (uint32_t i = 0; i < kHeld; ++i)   // (the last vector again past the row's end)
+      held[i] = reinterpret_cast<const uint4 *>(source)[min(threadIdx.x + 256u * i, width / 8u - 1u)];
   }
+  __device__ __forceinline__ void store(uint32_t width, uint16_t *lds) {
 #pragma unroll
-  for (uint32_t i = 0; i < kStagedWidth / 8u / 256u; ++i) {
-    const uint32_t v = threadIdx.x + 256u * i;
-    if (v < vectors) reinterpret_cast<uint4 *>(lds)[v] = held[i];
+    for (uint32_t i = 0; i < kHeld; ++i) arrived(held[i]);
+#pragma unroll
+    for (uint32_t i = 0; i < kHeld; ++i) {
+      const uint32_t v = threadIdx.x + 256u * i;
+      if (v < width / 8u) reinterpret_cast<uint4 *>(lds)[v] = held[i];
+    }
   }
-}
+};
 
 // The row's inverse RMS: 256 threads sum the squares of columns tid, tid + 256, ... in column
 // order; a wavefront sums its lanes by butterfly, the four wavefronts' sums are added in order
@@ -59,8 +70,11 @@ __global__ __launch_bounds__(256) void norm_rms(const uint16_t *__restrict__ inp
   const uint32_t row = blockIdx.x;
   const uint16_t *x = input + size_t(row) * p.width, *w = weight;
   if (p.width <= kStagedWidth && p.width % 8u == 0) {
-    stage_row(x, p.width, rowX);
-    stage_row(w, p.width, rowW);
+    StagedRow stagedX, stagedW;
+    stagedX.load(x, p.width);
+    stagedW.load(w, p.width);
+    stagedX.store(p.width, rowX);
+    stagedW.store(p.width, rowW);
     __syncthreads();
     x = rowX;
     w = rowW;
@@ -145,8 +159,11 @@ __global__ __launch_bounds__(256) void norm_rms_table16(const uint16_t *__restri
   const uint16_t *x = input + size_t(live ? row : 0) * p.width;
   if (p.width <= kStagedWidth) {  // the width is a multiple of 256
     if (live) {
-      stage_row(x, p.width, rowX);
-      stage_row(weight, p.width, rowW);
+      StagedRow stagedX, stagedW;
+      stagedX.load(x, p.width);
+      stagedW.load(weight, p.width);
+      stagedX.store(p.width, rowX);
+      stagedW.store(p.width, rowW);
     }
     __syncthreads();
     const float inverse = live ? rms_inverse(rowX, p.width, scratch) : 0.f;
@@ -162,7 +179,7 @@ SP_REGISTER_KERNEL("norm_rms_table16", &norm_rms_table16);
 // activation table; a Residual stage's rows, their RMS norm (of `norm_weight`, into `normalized`) and its table. Each
 // convolution was a launch of its own before a launch of as few workgroups. Values and their order are the two kernels'.
 // The rows' 16-byte accesses are the host's rule (DraftAttention::addConvolutionTable). 8 rows of 5120: 5.2 us
-// for 3.1 + 3.0, 8.3 us for 3.1 + 8.7, and a launch less each: the draft model's pass of one lane 928, 923 and 938 us
+// for 3.1 + 3.0, 7.9 us for 3.1 + 8.7, and a launch less each: the draft model's pass of one lane 928, 923 and 938 us
 // before, 869, 888 and 889 after, in three runs of both sides in turn whose repeats differ by 1 to 2 %.
 template <bool Residual>
 __global__ __launch_bounds__(256) void draft_conv_table(const uint16_t *__restrict__ input, const uint16_t *__restrict__ dynamic,
@@ -185,8 +202,7 @@ __global__ __launch_bounds__(256) void draft_conv_table(const uint16_t *__restri
     uint32_t dynamic0[kHeld], dynamic1[kHeld];
 #pragma unroll
     for (uint32_t i = 0; i < kHeld; ++i) {
-      const uint32_t v = threadIdx.x + 256u * i;
-      if (v >= vectors) continue;
+      const uint32_t v = min(threadIdx.x + 256u * i, vectors - 1u);   // the last vector again past the row's end
       now[i] = vector(input + size_t(row) * width, v);
       last[i] = vector(input + before * width, v);
       tap0[i] = vector(taps, v);
@@ -195,7 +211,19 @@ __global__ __launch_bounds__(256) void draft_conv_table(const uint16_t *__restri
       dynamic0[i] = mine[v / (DRAFT_CONVOLUTION_GROUP / 8u)];
       dynamic1[i] = mine[groups + v / (DRAFT_CONVOLUTION_GROUP / 8u)];
     }
-    if constexpr (Residual) stage_row(norm_weight, width, rowW);
+    StagedRow norms;
+    if constexpr (Residual) norms.load(norm_weight, width);
+#pragma unroll
+    for (uint32_t i = 0; i < kHeld; ++i) {
+      arrived(now[i]);
+      arrived(last[i]);
+      arrived(tap0[i]);
+      arrived(tap1[i]);
+      if constexpr (Residual) arrived(added[i]);
+      arrived(dynamic0[i]);
+      arrived(dynamic1[i]);
+    }
+    if constexpr (Residual) norms.store(width, rowW);
 #pragma unroll
     for (uint32_t i = 0; i < kHeld; ++i) {
       const uint32_t v = threadIdx.x + 256u * i;
@@ -429,13 +457,21 @@ __global__ __launch_bounds__(256) void gguf_embed_norm(const uint8_t *__restrict
     // the native row whole, with every load in flight at once (a decode's byte loads from memory wait for one another)
     const uint8_t *source = embedding + size_t(inside ? token : 0u) * blocks * EmbedBlock<FMT>::kBytes;
     const uint32_t pieces = blocks * EmbedBlock<FMT>::kBytes / uint32_t(sizeof(Piece));
-    Piece held[kPieces];
+    uint32_t held[kPieces];
 #pragma unroll
-    for (uint32_t i = 0; i < kPieces; ++i) __builtin_memcpy(&held[i], source + min(tid + 256u * i, pieces - 1u) * sizeof(Piece), sizeof(Piece));
-    stage_row(weight, p.embed.hidden, rowW);
+    for (uint32_t i = 0; i < kPieces; ++i) {
+      Piece piece;
+      __builtin_memcpy(&piece, source + min(tid + 256u * i, pieces - 1u) * sizeof(Piece), sizeof(Piece));
+      held[i] = piece;
+    }
+    StagedRow norms;
+    norms.load(weight, p.embed.hidden);
+#pragma unroll
+    for (uint32_t i = 0; i < kPieces; ++i) arrived(held[i]);
 #pragma unroll
     for (uint32_t i = 0; i < kPieces; ++i)
-      if (tid + 256u * i < pieces) native[tid + 256u * i] = held[i];
+      if (tid + 256u * i < pieces) native[tid + 256u * i] = Piece(held[i]);
+    norms.store(p.embed.hidden, rowW);
     __syncthreads();
     for (uint32_t b = 0; b < blocks; ++b) {
       const uint16_t value = inside ? uint16_t(EmbedBlock<FMT>::bits(reinterpret_cast<const uint8_t *>(native) + b * EmbedBlock<FMT>::kBytes, tid)) : uint16_t(0);
