@@ -346,6 +346,7 @@ sp_status spo_gdn_add_prefill(spo_graph *graph, const spo_gdn_prefill_buffers *b
                               const spo_gdn_prefill_capture *captures, uint32_t count);
 /* The same with the scan in blocks of sixteen tokens on the matrix cores, whose terms pass through `blocks`
  * (spo_gdn_prefill_blocks_bytes of the chunk's rows): the cells hold the accepted blocks' to fp32 rounding, not bit for bit.
+ * A value that is not finite reaches the rows and state rows that it reaches token by token, and no others.
  * A chunk's row buffers stay under 2 GiB each. */
 uint64_t spo_gdn_prefill_blocks_bytes(const spo_gdn_shape *shape, uint32_t tokens);
 sp_status spo_gdn_add_prefill_blocks(spo_graph *graph, const spo_gdn_prefill_buffers *buffers, sp_buffer *blocks, const spo_gdn_shape *shape,

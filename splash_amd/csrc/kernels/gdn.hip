@@ -633,19 +633,27 @@ __device__ __forceinline__ float sixteen_sum(float v) {
   v += dpp_of<0x140>(v);  // row_mirror
   return v;
 }
-__global__ __launch_bounds__(256) void gdn_prefill_scan(const uint16_t *__restrict__ queries, const uint16_t *__restrict__ keys,
-                                                        const uint16_t *__restrict__ values, const float *__restrict__ decay,
-                                                        const uint16_t *__restrict__ beta, uint8_t *__restrict__ states,
-                                                        uint16_t *__restrict__ recurrent_rows, GdnPrefillParams p) {
-  constexpr uint32_t B = GDN_SCAN_BLOCK, R = GDN_SCAN_STATE_ROWS, kGroups = kDim / R, kPieces = R / 8;
+struct ScanStaging {
+  __align__(16) float keys[2][GDN_SCAN_BLOCK][kDim], queries[2][GDN_SCAN_BLOCK][kDim];
+  __align__(16) uint16_t values[2][GDN_SCAN_BLOCK][GDN_SCAN_STATE_ROWS], outputs[GDN_SCAN_BLOCK][GDN_SCAN_STATE_ROWS];
+  float2 gates[2][GDN_SCAN_BLOCK];   // decay, beta
+};
+// One head's state rows rowBase .. + GDN_SCAN_STATE_ROWS - 1 through the run, by the first 256 threads of a workgroup.
+// It passes scan_barriers(tokens) barriers.
+__device__ __forceinline__ uint32_t scan_barriers(uint32_t tokens) { return 1u + 2u * ((tokens + GDN_SCAN_BLOCK - 1u) / GDN_SCAN_BLOCK); }
+__device__ __forceinline__ void scan_state_rows(ScanStaging &staging, const uint16_t *__restrict__ queries, const uint16_t *__restrict__ keys,
+                                                const uint16_t *__restrict__ values, const float *__restrict__ decay,
+                                                const uint16_t *__restrict__ beta, uint8_t *__restrict__ states,
+                                                uint16_t *__restrict__ recurrent_rows, const GdnPrefillParams &p, uint32_t head, uint32_t rowBase) {
+  constexpr uint32_t B = GDN_SCAN_BLOCK, R = GDN_SCAN_STATE_ROWS, kPieces = R / 8;
   static_assert(B * kDim * 2 == 256 * 16, "a thread stages sixteen bytes of a block's keys and of its queries");
   static_assert(R == 16, "four waves of four rows hold a workgroup's state rows");
-  __shared__ __align__(16) float sk[2][B][kDim], sq[2][B][kDim];
-  __shared__ __align__(16) uint16_t sv[2][B][R], so[B][R];
-  __shared__ float2 gates[2][B];   // decay, beta
+  auto &sk = staging.keys, &sq = staging.queries;
+  auto &sv = staging.values;
+  auto &so = staging.outputs;
+  auto &gates = staging.gates;
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-  const GdnShapeParams s = p.shape;
-  const uint32_t head = blockIdx.x / kGroups, rowBase = (blockIdx.x % kGroups) * R;
+  const GdnShapeParams &s = p.shape;
   const uint32_t keyHead = head / (s.value_heads / s.key_heads), keyWidth = s.key_heads * kDim, valueWidth = s.value_heads * kDim;
   const uint32_t local = wave * 4u + (lane >> 4), column = 8u * (lane & 15u), tokens = p.tokens;
   const float *stateIn = reinterpret_cast<const float *>(states + p.current_cell + p.convolution_state_bytes + uint64_t(p.layer) * p.recurrent_layer_bytes);
@@ -766,6 +774,14 @@ __global__ __launch_bounds__(256) void gdn_prefill_scan(const uint16_t *__restri
   for (uint32_t h = 0; h < 2; ++h)
     *reinterpret_cast<float4 *>(stateOut + stateAt + 4u * h) = make_float4(state[h][0], state[h][1], state[h][2], state[h][3]);
 }
+__global__ __launch_bounds__(256) void gdn_prefill_scan(const uint16_t *__restrict__ queries, const uint16_t *__restrict__ keys,
+                                                        const uint16_t *__restrict__ values, const float *__restrict__ decay,
+                                                        const uint16_t *__restrict__ beta, uint8_t *__restrict__ states,
+                                                        uint16_t *__restrict__ recurrent_rows, GdnPrefillParams p) {
+  constexpr uint32_t kGroups = kDim / GDN_SCAN_STATE_ROWS;
+  __shared__ ScanStaging staging;
+  scan_state_rows(staging, queries, keys, values, decay, beta, states, recurrent_rows, p, blockIdx.x / kGroups, (blockIdx.x % kGroups) * GDN_SCAN_STATE_ROWS);
+}
 SP_REGISTER_KERNEL("gdn_prefill_scan", &gdn_prefill_scan);
 
 // ---- prefill in blocks of sixteen tokens, on the matrix cores ----
@@ -781,8 +797,11 @@ SP_REGISTER_KERNEL("gdn_prefill_scan", &gdn_prefill_scan);
 // 13 + 93 us here (0.72 us a block). The sums' order differs from the fold's, so a chunk through these kernels leaves the accepted blocks' cell to rounding, not bit for bit.
 // Precision: keys and queries are bf16, as they are; the state and the corrections enter their products as three bf16 parts
 // each, which hold all 24 bits, and every sum is fp32. Against 64-bit arithmetic the state of 32 heads is off by 5.0e-8 of
-// its norm where the scan's is by 5.7e-8, and the rows by the same rounding to bf16 (tests/test_gdn_blocks_gpu.py). A row that is not finite makes the rows of its own block that lie
-// before it NaN too (the triangle's zeros multiply it), where the scan would have kept those finite.
+// its norm where the scan's is by 5.7e-8, and the rows by the same rounding to bf16 (tests/test_gdn_blocks_gpu.py).
+// Values that are not finite: in these products a row of them would reach the rows of its block before it (the triangle's
+// zeros multiply it) and an infinite state would be NaN (its parts are inf - inf). Either stays in the state's row to the
+// run's end, where a workgroup that finds one in its rows takes the run again token by token, as the scan does and bit for
+// bit. (A query that is not finite reaches its own output alone, here as there.)
 __device__ __forceinline__ uint32_t upper_halves(float low, float high) {
   return __builtin_amdgcn_perm(__float_as_uint(high), __float_as_uint(low), 0x07060302u);
 }
@@ -908,14 +927,18 @@ struct BlockTerms {
   uint32_t value[4];              // of token 4 kq + i, value dimensions rowBase + (row & ~1) and the next
 };
 __global__ __launch_bounds__(320, 1) void gdn_prefill_block_scan(const uint16_t *__restrict__ queries, const uint16_t *__restrict__ keys,
-                                                                 const uint16_t *__restrict__ values, const uint8_t *__restrict__ work,
+                                                                 const uint16_t *__restrict__ values, const float *__restrict__ decay,
+                                                                 const uint16_t *__restrict__ beta, const uint8_t *__restrict__ work,
                                                                  uint8_t *__restrict__ states, uint16_t *__restrict__ recurrent_rows,
                                                                  GdnPrefillParams p) {
   constexpr uint32_t B = GDN_SCAN_BLOCK, kAhead = 4;
   __shared__ __align__(16) float4 shares[2][2][4][64];   // [block parity][S k, S q][wave][lane]
+  __shared__ ScanStaging staging;                        // of the run again
+  __shared__ uint32_t unbounded;                         // the state after the run is not finite
   const uint32_t tid = threadIdx.x, lane = tid & 63u, row = lane & 15u, kq = lane >> 4;
   const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(int(tid >> 6)));
   const GdnShapeParams s = p.shape;
+  if (tid == 0) unbounded = 0;   // (set behind the blocks' barriers)
   const uint32_t head = blockIdx.x % s.value_heads, rowBase = blockIdx.x / s.value_heads * 16u;
   const uint32_t keyHead = head / (s.value_heads / s.key_heads), keyWidth = s.key_heads * kDim, valueWidth = s.value_heads * kDim;
   const uint32_t blocks = (p.tokens + B - 1u) / B, rounds = (blocks + kAhead - 1u) / kAhead;
@@ -977,7 +1000,8 @@ __global__ __launch_bounds__(320, 1) void gdn_prefill_block_scan(const uint16_t 
     return sum;
   };
   // (A block's shares are written over those of two blocks before, which every wave has read once it is past the barrier of
-  // the block between. Both kinds of wave below pass rounds * kAhead barriers.)
+  // the block between. Both kinds of wave below pass rounds * kAhead barriers, one that ends the run, and those of the run
+  // again where there is one.)
   if (wave == 4u) {
     const Resource outputRows = make_resource(recurrent_rows + size_t(p.first) * valueWidth, p.tokens * valueRow);
     struct Fetched {
@@ -1025,6 +1049,10 @@ __global__ __launch_bounds__(320, 1) void gdn_prefill_block_scan(const uint16_t 
         __builtin_amdgcn_sched_barrier(0);
       }
     }
+    __threadfence();   // (the outputs of this run, before those of the run again)
+    __syncthreads();
+    if (unbounded)
+      for (uint32_t n = scan_barriers(p.tokens); n; --n) __syncthreads();
     return;
   }
   const float *stateIn = reinterpret_cast<const float *>(states + p.current_cell + p.convolution_state_bytes + uint64_t(p.layer) * p.recurrent_layer_bytes);
@@ -1095,7 +1123,7 @@ __global__ __launch_bounds__(320, 1) void gdn_prefill_block_scan(const uint16_t 
     for (uint32_t e = 0; e < 2; ++e)
       split3(corrections[2u * e] * toEnd[2u * e], corrections[2u * e + 1u] * toEnd[2u * e + 1u], uh[e], um[e], ul[e]);
     const bf16x8 leading = as_bf16x8(make_uint4(uh[0], uh[1], 0u, 0u)), last = as_bf16x8(make_uint4(um[0], um[1], ul[0], ul[1]));
-    const float decay = block < blocks ? __uint_as_float(f.decay) : 1.f;
+    const float kept = block < blocks ? __uint_as_float(f.decay) : 1.f;
 #pragma unroll
     for (uint32_t m = 0; m < 2; ++m) {
       const bf16x8 key = as_bf16x8(f.update[m]);
@@ -1103,7 +1131,7 @@ __global__ __launch_bounds__(320, 1) void gdn_prefill_block_scan(const uint16_t 
       const f32x4 rest = __builtin_amdgcn_mfma_f32_16x16x32_bf16(key, last, zero, 0, 0, 0);
       if (m == 0) fetch(next, 5);
 #pragma unroll
-      for (uint32_t i = 0; i < 4; ++i) state[m][i] = __fmaf_rn(state[m][i], decay, rest[i]) + most[i];
+      for (uint32_t i = 0; i < 4; ++i) state[m][i] = __fmaf_rn(state[m][i], kept, rest[i]) + most[i];
     }
   };
   Fetched ahead[kAhead];
@@ -1117,6 +1145,17 @@ __global__ __launch_bounds__(320, 1) void gdn_prefill_block_scan(const uint16_t 
       run(round * kAhead + a, parity, ahead[a], ahead[(a + kAhead - 1u) % kAhead]);
       __builtin_amdgcn_sched_barrier(0);
     }
+  }
+  uint32_t most = 0;   // the magnitudes' bits order as the magnitudes do, those past the infinity's are NaNs
+#pragma unroll
+  for (uint32_t m = 0; m < 2; ++m)
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) most = max(most, __float_as_uint(state[m][i]) & 0x7FFFFFFFu);
+  if (most >= 0x7F800000u) unbounded = 1;
+  __syncthreads();
+  if (unbounded) {
+    scan_state_rows(staging, queries, keys, values, decay, beta, states, recurrent_rows, p, head, rowBase);
+    return;
   }
 #pragma unroll
   for (uint32_t m = 0; m < 2; ++m) *reinterpret_cast<f32x4 *>(stateOut + stateAt + 4u * m) = state[m];

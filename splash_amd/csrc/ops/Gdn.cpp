@@ -139,7 +139,7 @@ void GDN::addPrefill(hip::CommandGraph &graph, const GdnPrefillBuffers &b, const
     if (b.blocks) {
       graph.add("gdn_prefill_blocks", {b.queries, b.keys, b.decay, b.beta, b.blocks}, params,
                 {shape.valueHeads, ((params.tokens + GDN_SCAN_BLOCK - 1) / GDN_SCAN_BLOCK + 3) / 4, 1}, {256, 1, 1});
-      graph.add("gdn_prefill_block_scan", {b.queries, b.keys, b.values, b.blocks, b.states, b.recurrentRows}, params,
+      graph.add("gdn_prefill_block_scan", {b.queries, b.keys, b.values, b.decay, b.beta, b.blocks, b.states, b.recurrentRows}, params,
                 {shape.valueHeads * (GDN_HEAD_DIMENSION / 16), 1, 1}, {320, 1, 1});
     } else graph.add("gdn_prefill_scan", {b.queries, b.keys, b.values, b.decay, b.beta, b.states, b.recurrentRows}, params,
               {shape.valueHeads * (GDN_HEAD_DIMENSION / GDN_SCAN_STATE_ROWS), 1, 1}, {256, 1, 1});

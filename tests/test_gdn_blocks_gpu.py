@@ -116,3 +116,47 @@ def test_blocks_in_runs_and_refusals(backend):
     with pytest.raises(ValueError):
         layer.gdn.add_prefill(graph, buffers, 0, 45, layer.cell(0, 0), layer.cell(0, 1), blocks=small)
     assert len(graph) == 0
+
+
+@pytest.mark.parametrize("place", ["value", "key", "query", "beta", "decay", "infinite value", "infinite state", "state", "last row"])
+def test_blocks_keep_what_is_not_finite_where_the_scan_keeps_it(backend, place):
+    """Rows and states that are not finite reach through the blocks what they reach token by token, and nothing else: not the
+    rows of their block before them, not the state's other rows. Where they reach, the sixteen state rows of a workgroup are
+    the scan's bit for bit."""
+    print(f"case gdn blocks not finite: {place}", flush=True)
+    tokens, row, dimension = 45, 21, 37
+    nan, inf = 0x7FC0, 0x7F80
+
+    def change(shape, packed):
+        packed, values = packed.copy(), 2 * shape.key_heads * 128
+        gate = shape.conv_dim + shape.value_heads * 128
+        at = {"value": values + 128 + dimension, "infinite value": values + 128 + dimension, "last row": values + 128 + dimension,
+              "query": dimension, "key": (shape.key_heads + 1) * 128 + dimension, "beta": gate + 1, "decay": gate + shape.value_heads + 1}
+        if place in at:
+            packed[tokens - 1 if place == "last row" else row, at[place]] = inf if place == "infinite value" else nan
+        return packed
+
+    layer, packed, conv_in, state_in = _case(backend, (2, 4), tokens, 54, change)
+    if "state" in place:
+        state_in = state_in.copy()
+        state_in[1, dimension, 5] = np.inf if place == "infinite state" else np.nan
+        layer.write_cell(0, 0, conv_in, state_in)
+    scan = Chunk(layer, tokens).run(packed, 0, 0, 1)
+    got = BlockChunk(layer, tokens).run(packed, 0, 0, 1)
+    widen = lambda run: (orc.bf16_to_f32(run["recurrent"]).reshape(tokens, 4, 128), run["state_out"])
+    (rows, state), (want, want_state) = widen(got), widen(scan)
+    broken = ~np.isfinite(want_state).all(axis=2)                   # [head][dimension]
+    first = 0 if "state" in place else tokens - 1 if place == "last row" else row
+    assert np.isfinite(want[:first]).all() and not np.isfinite(want[first:]).all()
+    assert broken.any() == (place != "query") and not broken.all()
+    for a, b in ((rows, want), (state, want_state)):
+        assert np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(np.where(np.isinf(a), a, 0), np.where(np.isinf(b), b, 0))
+    groups = broken.reshape(4, 8, 16).any(axis=2)
+    for head, group in zip(*np.nonzero(groups)):
+        part = slice(16 * group, 16 * group + 16)
+        assert rows[:, head, part].tobytes() == want[:, head, part].tobytes()
+        assert state[head, part].tobytes() == want_state[head, part].tobytes()
+    # elsewhere each form is within a bf16 step and 1e-5 of the recurrence (check_prefill_against_fp64's bound), its state within 1e-5
+    finite, stays = np.isfinite(want), np.isfinite(want_state)
+    assert np.all(np.abs(rows - want)[finite] <= 2 * (0.0078125 * np.abs(want[finite]) + 1e-5))
+    assert np.abs(state - want_state)[stays].max() <= 2e-5
