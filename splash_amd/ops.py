@@ -614,7 +614,7 @@ def chain_tree_rows(rows_per_sequence):
     rows = list(rows_per_sequence)
     if max(rows, default=0) > _CHAIN.size:
         raise OverflowError("a tree row's ancestors are 32 bits")
-    return np.concatenate([_CHAIN[:0]] + [_CHAIN[:r] for r in rows]).view(_TREE_ROW)
+    return np.concatenate([_CHAIN[:0]] + [_CHAIN[:max(r, 0)] for r in rows]).view(_TREE_ROW)
 
 
 # ---------------------------------------------------------------------------------------------

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 import splash_amd
-from splash_amd import verify
+from splash_amd import ops, verify
 
 V = 1000
 
@@ -81,3 +81,16 @@ def test_penalty_words_are_rebuilt_from_a_history():
         ops.Sampling.rebuild_penalty_words(V, [3, V], 0)
     with pytest.raises(ValueError):
         ops.Sampling.rebuild_penalty_words(V, [3], 0, pending_token=V)
+
+
+@pytest.mark.parametrize("counts", [[], [0], [1], [3, 0, 2], [-1], [2, -40, 1], [32, 32], (n for n in (4, 5))])
+def test_chain_rows_hold_each_sequences_chain(counts):
+    """A sequence's rows in order; a count of none or below leaves none, more than 32 bits of ancestors are refused."""
+    counts = list(counts)
+    rows = ops.chain_tree_rows(iter(counts))
+    want = [((2 << r) - 1, 0xFFFF if r == 0 else r - 1, r) for n in counts for r in range(n)]
+    assert rows.tolist() == want and rows.dtype.names == ("ancestors", "parent", "depth") and rows.dtype.itemsize == 8
+    rows[:1] = 0   # the caller's own
+    assert ops.chain_tree_rows(counts).tolist() == want
+    with pytest.raises(OverflowError):
+        ops.chain_tree_rows(counts + [33])
