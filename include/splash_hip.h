@@ -119,6 +119,11 @@ sp_status sp_submit(sp_backend *backend, const sp_dispatch *dispatches, uint32_t
 int sp_ticket_ready(const sp_ticket *ticket);
 sp_status sp_ticket_wait(sp_ticket *ticket, double *gpu_seconds, double *wall_seconds);
 void sp_ticket_release(sp_ticket *ticket);
+/* How long sp_ticket_wait and sp_ticket_release poll the GPU before they sleep between their looks. While a wait polls it
+ * holds a host core (a whole verify step long, by default); one that sleeps takes a few per cent of it and returns up to
+ * 70 us later. 0 sleeps at once. Applies to the backend's waits that begin later, of any thread. */
+#define SP_DEFAULT_POLL_SECONDS 0.02
+sp_status sp_backend_set_poll_seconds(sp_backend *backend, double seconds);
 
 /* BackendInstrumentation::setDispatchProfiling (runtime/metal/BackendInstrumentation.hpp:23-37):
  * while on, every dispatch of a submitted command is bracketed by its own event pair and

@@ -235,6 +235,7 @@ _sig("sp_submit", c_int, c_p, P(Dispatch), c_u32, c_p, c_p, P(c_p))
 _sig("sp_ticket_ready", c_int, c_p)
 _sig("sp_ticket_wait", c_int, c_p, P(c_double), P(c_double))
 _sig("sp_ticket_release", None, c_p)
+_sig("sp_backend_set_poll_seconds", c_int, c_p, c_double)
 _sig("sp_backend_set_dispatch_profiling", None, c_p, c_int)
 _sig("sp_ticket_wait_profiled", c_int, c_p, P(c_double), P(c_double), P(c_double), c_u32)
 _sig("sp_command_create", c_int, c_p, P(Dispatch), c_u32, P(c_p))

@@ -196,6 +196,10 @@ class Backend:
         check(lib.spo_graph_record(self.handle, graph.handle, ctypes.byref(c)))
         return RecordedCommand(c.value, graph)
 
+    def set_poll_seconds(self, seconds):
+        """How long a wait polls, holding a host core, before it sleeps between its looks (0.02 unless set)."""
+        check(lib.sp_backend_set_poll_seconds(self.handle, seconds))
+
     def set_dispatch_profiling(self, on):
         lib.sp_backend_set_dispatch_profiling(self.handle, int(bool(on)))
 

@@ -272,6 +272,7 @@ public:
     for (const ComputeDispatch &d : dispatches)
       if (!sp_kernel_exists(d.pipelineName.c_str())) throw std::invalid_argument("no kernel named " + d.pipelineName);
   }
+  void setPollSeconds(double seconds) const { throwStatus(sp_backend_set_poll_seconds(backend_, seconds)); }
   void setDispatchProfiling(bool on) const { sp_backend_set_dispatch_profiling(backend_, on); }
   [[nodiscard]] MemoryStats memoryStats() const {
     sp_memory_stats_t s{};
