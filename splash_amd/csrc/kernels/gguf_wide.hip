@@ -23,6 +23,8 @@
 #include "abi/Moe.h"
 #include "backend/KernelRegistry.hpp"
 #include "kernels/gguf_records.hpp"
+#include <type_traits>
+#include <utility>
 
 namespace splash::kernels {
 
@@ -191,19 +193,43 @@ template <uint32_t FMT> struct WideRecord {
   uint2 fifth;        // Q5_K: the fifth bits
   uint32_t d;         // Q6_K
 };
-// What a record's first two stages need, and (`late`) the bits its last stage reads too.
+// The loads of a record in three parts: what its first two stages need (and what all share), the codes of its last two, and
+// the bits its last stage reads too. A part's count is the loop that issues it and what the waits for the rows count by: a
+// load is one vector-memory instruction.
+template <uint32_t FMT> constexpr uint32_t kWideFirstLoads = FMT == GGUF_FMT_Q6K ? 3u : 2u;
+template <uint32_t FMT> constexpr uint32_t kWideSecondLoads = 1u;
+template <uint32_t FMT> constexpr uint32_t kWideLateLoads = FMT == GGUF_FMT_Q4K ? 0u : 1u;
+template <uint32_t N, typename F> __device__ __forceinline__ void each_load(F &&load) {
+  [&]<uint32_t... I>(std::integer_sequence<uint32_t, I...>) __attribute__((always_inline)) {
+    (load(std::integral_constant<uint32_t, I>{}), ...);
+  }(std::make_integer_sequence<uint32_t, N>{});
+}
 template <uint32_t FMT> __device__ __forceinline__ void load_first(WideRecord<FMT> &rec, Resource r, uint32_t mine, uint32_t lane) {
   const uint32_t record = mine - 16u * lane, c = lane & 15u;
-  rec.codes[0] = load128<kStreamOnce>(r, mine);
-  rec.meta = load128<kStreamOnce>(r, record + Cursor<FMT>::kColumnPart + 16u * c);
-  if constexpr (FMT == GGUF_FMT_Q6K) rec.d = __builtin_amdgcn_raw_buffer_load_b16(r, int(record + GGUF_Q6K_D + 2u * c), 0, kStreamOnce);
+  each_load<kWideFirstLoads<FMT>>([&](auto i) __attribute__((always_inline)) {
+    if constexpr (i == 0u) rec.codes[0] = load128<kStreamOnce>(r, mine);
+    else if constexpr (i == 1u) rec.meta = load128<kStreamOnce>(r, record + Cursor<FMT>::kColumnPart + 16u * c);
+    else {
+      static_assert(i == 2u && FMT == GGUF_FMT_Q6K);
+      rec.d = __builtin_amdgcn_raw_buffer_load_b16(r, int(record + GGUF_Q6K_D + 2u * c), 0, kStreamOnce);
+    }
+  });
+}
+template <uint32_t FMT> __device__ __forceinline__ void load_second(WideRecord<FMT> &rec, Resource r, uint32_t mine) {
+  each_load<kWideSecondLoads<FMT>>([&](auto i) __attribute__((always_inline)) {
+    static_assert(i == 0u);
+    rec.codes[1] = load128<kStreamOnce>(r, mine + 1024u);
+  });
 }
 template <uint32_t FMT> __device__ __forceinline__ void load_late(WideRecord<FMT> &rec, Resource r, uint32_t mine, uint32_t lane) {
-  if constexpr (FMT == GGUF_FMT_Q6K) rec.high = load128<kStreamOnce>(r, mine + GGUF_Q6K_HIGH);
-  if constexpr (FMT == GGUF_FMT_Q5K) {
-    const u32x2 fifth = __builtin_amdgcn_raw_buffer_load_b64(r, int(mine - 8u * lane + GGUF_Q5K_HIGH), 0, kStreamOnce);
-    rec.fifth = make_uint2(fifth.x, fifth.y);
-  }
+  each_load<kWideLateLoads<FMT>>([&](auto i) __attribute__((always_inline)) {
+    static_assert(i == 0u && (FMT == GGUF_FMT_Q6K || FMT == GGUF_FMT_Q5K));
+    if constexpr (FMT == GGUF_FMT_Q6K) rec.high = load128<kStreamOnce>(r, mine + GGUF_Q6K_HIGH);
+    else {
+      const u32x2 fifth = __builtin_amdgcn_raw_buffer_load_b64(r, int(mine - 8u * lane + GGUF_Q5K_HIGH), 0, kStreamOnce);
+      rec.fifth = make_uint2(fifth.x, fifth.y);
+    }
+  });
 }
 // What its operands need of `meta` once a super-block.
 template <uint32_t FMT> struct WideScales {
@@ -450,13 +476,14 @@ __device__ __forceinline__ void wide_workgroup(const WideTile &w, const uint8_t 
   };
   auto fetchSecond = [&] {
 #pragma unroll
-    for (uint32_t r = 0; r < 2; ++r) rec[r].codes[1] = load128<kStreamOnce>(weights[r], mine + 1024u);
+    for (uint32_t r = 0; r < 2; ++r) load_second<FMT>(rec[r], weights[r], mine);
     mine += kRecord;
   };
   // What a stage's loads are: its rows' (three stages ahead), then the weights'. A stage's rows are there when at most what
-  // was asked for after them is on its way.
-  constexpr uint32_t kFirst = FMT == GGUF_FMT_Q6K ? 6u : 4u, kLate = FMT == GGUF_FMT_Q4K ? 0u : 2u, kSecond = 2u;
-  constexpr auto weightLoads = [](uint32_t stage) constexpr { return stage == 0 ? kSecond : stage == 2u ? kFirst : stage == 3u ? kLate : 0u; };
+  // was asked for after them is on its way. (Counted by what issues them: the parts' own counts, of the lane's two records.)
+  constexpr auto weightLoads = [](uint32_t stage) constexpr {
+    return 2u * (stage == 0 ? kWideSecondLoads<FMT> : stage == 2u ? kWideFirstLoads<FMT> : stage == 3u ? kWideLateLoads<FMT> : 0u);
+  };
   constexpr auto rowLoads = [](uint32_t stage) constexpr { return kShare + (stage == 3u ? kSumShare : 0u); };
   // (the loads before the first stage in the order of the stages that would have asked for them)
   fetch(0, std::integral_constant<uint32_t, 0>{});
