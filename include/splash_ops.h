@@ -199,6 +199,10 @@ uint64_t spo_kv_value_index(uint32_t head, uint32_t token, uint32_t dim, uint32_
 /* PagedAttention::plan (PagedAttention.cpp:351-389). */
 sp_status spo_attention_plan_create(const spo_attention_geometry *geometry, const spo_attention_rows *sequences,
                                     uint32_t count, spo_attention_plan **out);
+/* The same for a device of `compute_units` (256 otherwise), by which a dispatch of few rows is split over waves: whatever is
+ * given, the results are the same bits. */
+sp_status spo_attention_plan_create_calibrated(const spo_attention_geometry *geometry, const spo_attention_rows *sequences,
+                                               uint32_t count, uint32_t compute_units, spo_attention_plan **out);
 void spo_attention_plan_destroy(spo_attention_plan *plan);
 uint32_t spo_attention_plan_splits(const spo_attention_plan *plan);
 /* PagedAttention::workspace: bytes of the staged queries, their sums, the split partials, their sums. */

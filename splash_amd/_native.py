@@ -285,6 +285,7 @@ _sig("spo_kv_page_bytes", c_u64, c_u32, c_u32)
 _sig("spo_kv_key_index", c_u64, c_u32, c_u32, c_u32, c_u32)
 _sig("spo_kv_value_index", c_u64, c_u32, c_u32, c_u32, c_u32)
 _sig("spo_attention_plan_create", c_int, P(AttentionGeometry), P(AttentionRows), c_u32, P(c_p))
+_sig("spo_attention_plan_create_calibrated", c_int, P(AttentionGeometry), P(AttentionRows), c_u32, c_u32, P(c_p))
 _sig("spo_attention_plan_destroy", None, c_p)
 _sig("spo_attention_plan_splits", c_u32, c_p)
 _sig("spo_attention_workspace", c_int, c_p, P(c_u64))

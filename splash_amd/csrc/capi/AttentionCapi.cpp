@@ -25,6 +25,10 @@ uint64_t spo_kv_value_index(uint32_t head, uint32_t token, uint32_t dim, uint32_
 
 sp_status spo_attention_plan_create(const spo_attention_geometry *geometry, const spo_attention_rows *sequences, uint32_t count,
                                     spo_attention_plan **out) {
+  return spo_attention_plan_create_calibrated(geometry, sequences, count, ops::KernelCalibration{}.computeUnits, out);
+}
+sp_status spo_attention_plan_create_calibrated(const spo_attention_geometry *geometry, const spo_attention_rows *sequences, uint32_t count,
+                                               uint32_t compute_units, spo_attention_plan **out) {
   return capi::guard([&] {
     capi::require(geometry && sequences && out, "geometry, sequences or result");
     std::vector<ops::AttentionRows> rows;
@@ -32,7 +36,7 @@ sp_status spo_attention_plan_create(const spo_attention_geometry *geometry, cons
       rows.push_back({sequences[i].first_row, sequences[i].rows, sequences[i].committed, sequences[i].table_first});
     const ops::AttentionGeometry g{geometry->q_heads, geometry->kv_heads, geometry->head_dim, geometry->rotary_pairs,
                                    geometry->normalize != 0, geometry->gated != 0, geometry->int8_queries != 0};
-    *out = new spo_attention_plan{ops::PagedAttention::plan(g, std::move(rows))};
+    *out = new spo_attention_plan{ops::PagedAttention::plan(g, std::move(rows), compute_units)};
   });
 }
 void spo_attention_plan_destroy(spo_attention_plan *plan) { delete plan; }

@@ -38,7 +38,8 @@ ops::AttentionPlan planOf(const model::DenseVerify &v, const std::vector<model::
   std::vector<ops::AttentionRows> sequences;
   uint32_t rows = 0;
   for (const model::VerifyLane &l : lanes) { sequences.push_back({rows, l.rows, l.committed, l.tableFirst}); rows += l.rows; }
-  return ops::PagedAttention::plan({d.qHeads, d.kvHeads, d.headDimension, d.rotaryPairs, d.normalizeHeads}, sequences);
+  return ops::PagedAttention::plan({d.qHeads, d.kvHeads, d.headDimension, d.rotaryPairs, d.normalizeHeads}, sequences,
+                                   v.calibration().computeUnits);
 }
 } // namespace
 

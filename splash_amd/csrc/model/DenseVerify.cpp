@@ -494,7 +494,7 @@ void DenseVerify::encodePrefill(hip::CommandGraph &graph, uint32_t tableFirst, u
     ops::AttentionChunkPlan plan;
     ops::AttentionPromptPlan widePlan;
     if (wide) widePlan = ops::PagedAttention::planPrompt(geometry, {0, tokens, committed, tableFirst}, linear_.calibration().computeUnits);
-    else plan = ops::PagedAttention::planChunks(geometry, {{0, tokens, committed, tableFirst}});
+    else plan = ops::PagedAttention::planChunks(geometry, {{0, tokens, committed, tableFirst}}, linear_.calibration().computeUnits);
     if (dims_.rotaryPairs) {
       // the RoPE tables eight blocks a dispatch, each dispatch over its own rows of the depths and tables
       const uint32_t span = ATTENTION_MAXIMUM_SEQUENCES * ATTENTION_MAXIMUM_ROWS;
@@ -527,7 +527,7 @@ void DenseVerify::encodePrefill(hip::CommandGraph &graph, uint32_t tableFirst, u
     rope.push_back({first, rows, committed + first});
   }
   const ops::AttentionGeometry geometry{dims_.qHeads, dims_.kvHeads, dims_.headDimension, dims_.rotaryPairs, dims_.normalizeHeads};
-  const ops::AttentionPlan plan = ops::PagedAttention::plan(geometry, sequences);
+  const ops::AttentionPlan plan = ops::PagedAttention::plan(geometry, sequences, linear_.calibration().computeUnits);
   if (dims_.rotaryPairs)
     ops::RoPE::addTreeTables(graph, inverseFrequency_, depths_, ropeCos_, ropeSin_, dims_.rotaryPairs, rope);
   encodeEmbedding(graph, tokens);
@@ -558,7 +558,7 @@ void DenseVerify::encode(hip::CommandGraph &graph, const std::vector<VerifyLane>
     rows += lane.rows;
   }
   const ops::AttentionGeometry geometry{dims_.qHeads, dims_.kvHeads, dims_.headDimension, dims_.rotaryPairs, dims_.normalizeHeads};
-  const ops::AttentionPlan plan = ops::PagedAttention::plan(geometry, sequences);
+  const ops::AttentionPlan plan = ops::PagedAttention::plan(geometry, sequences, linear_.calibration().computeUnits);
   if (samples && !testChildren_) (void)draftProbabilities();
   const ops::PreparedInput entry = ops::Embedding::addNormTable(
       graph, weights_.embedding, inputTokens_, hidden_[0], weights_.layers.front().inputNorm, normalized_, scratch_,

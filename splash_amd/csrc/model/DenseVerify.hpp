@@ -59,6 +59,7 @@ public:
   [[nodiscard]] uint32_t prefillRows() const noexcept { return rowCapacity_; }
 
   [[nodiscard]] const DenseDimensions &dimensions() const noexcept { return dims_; }
+  [[nodiscard]] const ops::KernelCalibration &calibration() const noexcept { return linear_.calibration(); }
   DenseWeights &weights() noexcept { return weights_; }
   // Allocates what the model's long prompt chunks hold beyond a step's rows, where they take the wide kernels
   // (encodePrefill): a table, SwiGLU rows and partial sums, 420 MB at the 27B shape and 2048 rows. For whoever set the

@@ -214,7 +214,7 @@ ops::AttentionPlan HybridVerify::planOf(const std::vector<HybridLane> &lanes) co
   }
   return ops::PagedAttention::plan({dims_.qHeads, dims_.kvHeads, dims_.headDimension, dims_.rotaryPairs, dims_.normalizeHeads,
                                     dims_.gatedAttention},
-                                   sequences);
+                                   sequences, linear_.calibration().computeUnits);
 }
 
 void HybridVerify::encodeEmbedding(hip::CommandGraph &graph, uint32_t rows) {
@@ -564,7 +564,7 @@ void HybridVerify::encodePrefill(hip::CommandGraph &graph, uint32_t lane, uint32
   ops::AttentionChunkPlan plan;
   ops::AttentionPromptPlan widePlan;
   if (wide) widePlan = ops::PagedAttention::planPrompt(geometry, {0, tokens, committed, tableFirst}, linear_.calibration().computeUnits);
-  else plan = ops::PagedAttention::planChunks(geometry, {{0, tokens, committed, tableFirst}});
+  else plan = ops::PagedAttention::planChunks(geometry, {{0, tokens, committed, tableFirst}}, linear_.calibration().computeUnits);
   if (firstLayer == 0) {
     if (dims_.rotaryPairs) {
       // the RoPE tables eight blocks a dispatch, each dispatch over its own rows of the depths and tables

@@ -36,7 +36,7 @@ uint32_t totalRows(const std::vector<AttentionRows> &sequences) {
 // tokens 1 row 92 / 58, 4 rows 93 / 61 in two parts (76 as two tiles of one), 8 rows 92 / 80, 16 rows 90 / 144; 8 sequences behind
 // 16368 tokens 1 row 180 / 64, 4 rows 160 / 80 (100 in two parts), 8 rows 169 / 134, 16 rows 172 / 246; behind 4000 tokens and less
 // all of them lie within the fixed cost (23 / 22). So: up to eight rows; a tile a part while every part has a SIMD of its own
-// (4 x 256), then two tiles a part, which widen the keys and values they share once. 16 / 8 heads of 64, 8 rows: 8 sequences behind
+// (four a compute unit), then two tiles a part, which widen the keys and values they share once. 16 / 8 heads of 64, 8 rows: 8 sequences behind
 // 16368 tokens 54 / 37; 16 rows 54 / 51 in two parts, within 1 us of each other elsewhere.
 struct FewRows {
   uint32_t tiles = 0, parts = 0;
@@ -47,9 +47,8 @@ FewRows fewRows(const AttentionPlan &plan) {
   for (const AttentionRows &s : plan.sequences()) most = std::max(most, s.rows);
   const uint32_t all = std::max(1u, std::bit_ceil(most) * g.group() / 16u);
   if (g.int8Queries || most > 8) return {};
-  constexpr uint64_t kSimds = 4 * 256;
-  const uint64_t waves = uint64_t{g.kvHeads} * plan.splits() * plan.sequences().size();
-  if (all == 1 || waves * all <= kSimds) return {1, all};
+  const uint64_t simds = uint64_t{4} * plan.computeUnits(), waves = uint64_t{g.kvHeads} * plan.splits() * plan.sequences().size();
+  if (all == 1 || waves * all <= simds) return {1, all};
   return {2, all / 2};
 }
 void requirePages(const AttentionPlan &plan, const KvPages &pages) {
@@ -92,14 +91,16 @@ AttentionParams AttentionPlan::params(uint64_t pageBytes) const noexcept {
   return p;
 }
 
-AttentionPlan PagedAttention::plan(const AttentionGeometry &geometry, std::vector<AttentionRows> sequences) {
+AttentionPlan PagedAttention::plan(const AttentionGeometry &geometry, std::vector<AttentionRows> sequences, uint32_t computeUnits) {
   if (!geometry.kvHeads || geometry.qHeads % geometry.kvHeads || !compiled(geometry))
     throw std::invalid_argument("no attention kernel for this head geometry");
   if (2 * geometry.rotaryPairs > geometry.headDimension) throw std::invalid_argument("the rotated pairs are dimensions of the head");
   if (sequences.empty() || sequences.size() > ATTENTION_MAXIMUM_SEQUENCES)
     throw std::invalid_argument("an attention dispatch takes 1 to 8 sequences");
+  if (!computeUnits) throw std::invalid_argument("a device has compute units");
   AttentionPlan plan;
   plan.geometry_ = geometry;
+  plan.computeUnits_ = computeUnits;
   for (const AttentionRows &s : sequences) {
     if (!s.rows || s.rows > ATTENTION_MAXIMUM_ROWS) throw std::invalid_argument("a sequence's verify block holds 1 to 16 rows");
     const AttentionSplits part = attentionSplits(uint64_t{s.committed} + s.rows);
@@ -205,7 +206,7 @@ AttentionWorkspaceSize AttentionChunkPlan::workspace() const noexcept {
   return size;
 }
 
-AttentionChunkPlan PagedAttention::planChunks(const AttentionGeometry &geometry, const std::vector<AttentionChunk> &chunks) {
+AttentionChunkPlan PagedAttention::planChunks(const AttentionGeometry &geometry, const std::vector<AttentionChunk> &chunks, uint32_t computeUnits) {
   if (chunks.empty()) throw std::invalid_argument("a chunked attention takes at least one chunk");
   std::vector<AttentionRows> tiles;
   AttentionChunkPlan plan;
@@ -221,7 +222,7 @@ AttentionChunkPlan PagedAttention::planChunks(const AttentionGeometry &geometry,
   plan.tiles_ = uint32_t(tiles.size());
   for (size_t first = 0; first < tiles.size(); first += ATTENTION_MAXIMUM_SEQUENCES)
     plan.dispatches_.push_back(PagedAttention::plan(
-        geometry, {tiles.begin() + first, tiles.begin() + std::min(tiles.size(), first + ATTENTION_MAXIMUM_SEQUENCES)}));
+        geometry, {tiles.begin() + first, tiles.begin() + std::min(tiles.size(), first + ATTENTION_MAXIMUM_SEQUENCES)}, computeUnits));
   return plan;
 }
 

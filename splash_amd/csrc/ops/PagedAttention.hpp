@@ -73,6 +73,7 @@ public:
   [[nodiscard]] const AttentionGeometry &geometry() const noexcept { return geometry_; }
   [[nodiscard]] const std::vector<AttentionRows> &sequences() const noexcept { return sequences_; }
   [[nodiscard]] uint32_t splits() const noexcept { return splits_; }
+  [[nodiscard]] uint32_t computeUnits() const noexcept { return computeUnits_; }
   [[nodiscard]] AttentionWorkspaceSize workspace() const noexcept;
   [[nodiscard]] AttentionParams params(uint64_t pageBytes) const noexcept;
 
@@ -81,7 +82,7 @@ private:
   AttentionGeometry geometry_;
   std::vector<AttentionRows> sequences_;
   std::vector<AttentionSplits> partition_;
-  uint32_t splits_ = 1;
+  uint32_t splits_ = 1, computeUnits_ = 0;
 };
 
 // A prompt chunk of one sequence (the reference's kv::ChunkedPrefillParams with its rows' place in the command,
@@ -148,7 +149,9 @@ struct KvPages final {
 class PagedAttention final {
 public:
   // Throws for a geometry no kernel is compiled for, no or too many sequences, or rows outside 1..16.
-  [[nodiscard]] static AttentionPlan plan(const AttentionGeometry &geometry, std::vector<AttentionRows> sequences);
+  // computeUnits: the device's, by which a dispatch of few rows is split over waves; every choice computes the same bits.
+  [[nodiscard]] static AttentionPlan plan(const AttentionGeometry &geometry, std::vector<AttentionRows> sequences,
+                                          uint32_t computeUnits = KernelCalibration{}.computeUnits);
   // q/k norm + RoPE + query staging + INT8 store of the block's K and V (PagedAttention.cpp:441-464).
   static void addProjection(hip::CommandGraph &graph, const AttentionPlan &plan, const AttentionProjectionBuffers &buffers,
                             const AttentionWorkspace &workspace, const KvPages &pages);
@@ -172,7 +175,8 @@ public:
   // throws for a chunk of no or more than kMaximumChunkRows rows. addChunkProjection runs the projection pass of every
   // dispatch, so that every row's K and V are stored before any row attends; addChunkAttention then splits and merges
   // dispatch by dispatch. Buffers as addProjection's and addAttention's, over all the chunks' rows.
-  [[nodiscard]] static AttentionChunkPlan planChunks(const AttentionGeometry &geometry, const std::vector<AttentionChunk> &chunks);
+  [[nodiscard]] static AttentionChunkPlan planChunks(const AttentionGeometry &geometry, const std::vector<AttentionChunk> &chunks,
+                                                     uint32_t computeUnits = KernelCalibration{}.computeUnits);
   static void addChunkProjection(hip::CommandGraph &graph, const AttentionChunkPlan &plan, const AttentionProjectionBuffers &buffers,
                                  const AttentionWorkspace &workspace, const KvPages &pages);
   static void addChunkAttention(hip::CommandGraph &graph, const AttentionChunkPlan &plan, const AttentionWorkspace &workspace,

@@ -298,13 +298,13 @@ class KvPages:
 class AttentionPlan:
     """ops::AttentionPlan: geometry + sequences + history splits."""
 
-    def __init__(self, q_heads, kv_heads, head_dim, sequences, rotary_pairs=0, normalize=False, gated=False, int8_queries=False):
+    def __init__(self, q_heads, kv_heads, head_dim, sequences, rotary_pairs=0, normalize=False, gated=False, int8_queries=False, compute_units=256):
         """sequences: [(first_row, rows, committed, table_first)]; gated: a projection row holds each query head's
-        queries, then its gate, and the output rows are multiplied by the gates' sigmoids."""
+        queries, then its gate, and the output rows are multiplied by the gates' sigmoids; compute_units: the device's."""
         g = nat.AttentionGeometry(q_heads, kv_heads, head_dim, rotary_pairs, int(normalize), int(gated), int(int8_queries))
         rows = (nat.AttentionRows * len(sequences))(*[nat.AttentionRows(*s) for s in sequences])
         h = ctypes.c_void_p()
-        check(lib.spo_attention_plan_create(ctypes.byref(g), rows, len(sequences), ctypes.byref(h)))
+        check(lib.spo_attention_plan_create_calibrated(ctypes.byref(g), rows, len(sequences), compute_units, ctypes.byref(h)))
         self.handle = h
         self.geometry = g
         self.sequences = sequences

@@ -4,6 +4,7 @@ import pytest
 
 import splash_amd
 from splash_amd import ops, synthetic
+from tests import oracle as orc
 from tests.test_wide_kernels_gpu import AttentionParams, Sequence
 
 pytestmark = pytest.mark.gpu
@@ -93,3 +94,32 @@ def test_the_rule_takes_blocks_of_up_to_eight_rows(backend, rows, sequences, int
                                      backend.allocate_buffer(n * 64 * 128 * 2))
     assert kernel in graph.kernels()[0], graph.kernels()
     backend.run(graph)
+
+
+@pytest.mark.parametrize("heads,rows,tiles", [((64, 8, 128), 3, 2), ((64, 8, 128), 8, 4), ((32, 8, 128), 5, 2)])
+def test_two_tiles_a_wave_once_the_parts_outnumber_the_simds(backend, heads, rows, tiles):
+    """A tile a wave while every part has one of the device's SIMDs, four a compute unit, then two: the same rows, bit for bit."""
+    print(f"case few parts {heads} rows={rows}", flush=True)
+    Q, K, D = heads
+    rng = np.random.default_rng(rows)
+    lanes = [(0, rows, 700, 0), (rows, 2, 129, 3)]
+    kv = ops.KvPages(backend, K, D, 4, rng.permutation(4))
+    kv.upload(synthetic.kv_pages(rng, K, D, 4).reshape(4, -1))
+    tree = backend.from_array(_tree(rng, [rows, 2]))
+    queries = rng.standard_normal((2, Q, 16, D)).astype(np.float16)
+    splits = ops.AttentionPlan(Q, K, D, lanes).splits
+    enough = K * splits * len(lanes) * tiles // 4
+    got = []
+    for units, kernel in ((enough, "t1"), (enough - 1, "t2"), (1, "t2")):
+        plan = ops.AttentionPlan(Q, K, D, lanes, compute_units=units)
+        workspace = ops.AttentionWorkspace(backend, plan)
+        workspace.queries.upload(queries)
+        workspace.query_sums.upload(queries.astype(np.float32).sum(-1))
+        graph, out = splash_amd.CommandGraph(), backend.from_array(np.full((rows + 2) * Q * D, 0x7FC0, np.uint16))
+        ops.PagedAttention.add_attention(graph, plan, workspace, tree, kv, out)
+        assert graph.kernels()[0].endswith(kernel), (units, graph.kernels())
+        backend.run(graph)
+        got.append(out.download(np.uint16))
+    assert np.isfinite(orc.bf16_to_f32(got[0])).all() and all(np.array_equal(got[0], g) for g in got[1:])
+    with pytest.raises(ValueError):
+        ops.AttentionPlan(Q, K, D, lanes, compute_units=0)
