@@ -405,11 +405,12 @@ __global__ __launch_bounds__(64 * kWaves) void gdn_decode(const uint16_t *__rest
   __syncthreads();
 
   // ---- the committed state's products with the transformed queries (gdn.metal:363-377): wave w sixteen of the state's
-  // rows over half of their columns, for all the block's tokens (a token past them is a product that nothing reads). One matrix instruction's sums of
-  // four products each, added as a tree: against 64 bits 7.3e-8 of the terms' norm where a half-wave's tree of four-term
-  // chains was off by 7.6e-8 (with sixteen path terms 7.8e-8 for 8.1e-8). A block's rows were 0.8 us each in the state's
-  // registers, four 32-lane sums a wave; the kernel at 32 heads, as many pending rows as rows: 8 lanes of 16 rows 42.0 -> 32.8 us, of 4
-  // 19.2 -> 17.5, of 1 13.3 -> 13.7 (one form for every count, so that a row's bits do not depend on its block's). ----
+  // rows over half of their columns, for all the block's tokens (a token past them is a product that nothing reads). One
+  // matrix instruction's sums of four products each, added as a tree: against 64 bits 6.2e-8 of the terms' norm where a
+  // half-wave's tree of four-term chains is off by 6.6e-8 (tests/test_gdn_products_gpu.py). A block's rows were 0.8 us each
+  // in the state's registers, four 32-lane sums a wave; the kernel at 32 heads, as many pending rows as rows: 8 lanes of 16
+  // rows 42.0 -> 32.8 us, of 4 19.2 -> 17.5, of 1 13.3 -> 13.7 (one form for every count, so that a row's bits do not depend
+  // on its block's). ----
   {
     const uint32_t tile = wave >> 1, from = (kDim / 2u) * (wave & 1u), line = lane & 15u, quarter = lane >> 4;
     const f32x4 none = {};
