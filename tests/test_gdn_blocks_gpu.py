@@ -107,6 +107,14 @@ def test_blocks_in_runs_and_refusals(backend):
     runs = BlockChunk(layer, 45).run(packed, 0, 0, 1, captures=[(7, 2), (32, 3)])
     scale = np.abs(whole["state_out"]).max()
     assert np.abs(runs["state_out"] - whole["state_out"]).max() <= 2e-6 * scale
+    # the outputs of every run: bf16 of sums as far apart as the states, each row the gate pass's of its own values, and the
+    # runs' own convolution carry
+    wide = lambda run: orc.bf16_to_f32(run["recurrent"])
+    assert np.all(np.abs(wide(runs) - wide(whole)) <= 0.0078125 * np.abs(wide(whole)) + 1e-5)
+    same = (runs["recurrent"] == whole["recurrent"]).reshape(45, 4, 128).all(axis=2)
+    assert same[7:32].mean() > 0.9 and same[32:].mean() > 0.9
+    assert np.array_equal(runs["hidden"].reshape(45, 4, 128)[same], whole["hidden"].reshape(45, 4, 128)[same])
+    assert runs["conv_out"].tobytes() == whole["conv_out"].tobytes()
     _, state = layer.read_cell(0, 3)
     alone = Chunk(layer, 32).run(packed[:32], 0, 0, 1)
     assert np.abs(state - alone["state_out"]).max() <= 2e-6 * scale
