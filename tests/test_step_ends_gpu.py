@@ -66,7 +66,8 @@ class AcceptCommit(ctypes.Structure):
 
 @pytest.mark.parametrize("dimension,kv_heads", [(64, 2), (128, 3)])
 def test_selection_acceptance_and_commit_in_one_dispatch(backend, dimension, kv_heads):
-    """Chains and trees of 1 to 16 rows, caps, stop tokens, paths across a page's end, rows with no selectable logit."""
+    """Chains and trees of 1 to 16 rows, caps, stop tokens, paths across a page's end, rows with no selectable logit, lanes
+    that keep no row."""
     from tests.test_oracle_sampling import random_tree
     from tests.test_glue_sampling_gpu import sampling_buffers
     rng = np.random.default_rng(dimension)
@@ -79,6 +80,8 @@ def test_selection_acceptance_and_commit_in_one_dispatch(backend, dimension, kv_
         rows = int(first[-1])
         lanes = [(int(first[i]), n) for i, n in enumerate(counts)]
         tree = np.concatenate([random_tree(rng, n) if trial % 2 else ops.chain_tree_rows([n]) for n in counts])
+        if trial > 8:   # a lane whose anchor is not its own ancestor keeps no row: its commit takes the rows left there before
+            tree["ancestors"][first[int(rng.integers(0, len(counts)))]] = 0
         tokens = rng.integers(0, 3, rows).astype(np.uint32)
         logits = rng.standard_normal((rows, vocabulary)).astype(np.float32)
         logits[np.arange(rows), rng.integers(0, 3, rows)] = 9.0
@@ -93,11 +96,12 @@ def test_selection_acceptance_and_commit_in_one_dispatch(backend, dimension, kv_
             p.stop_tokens[i] = s
         table = backend.from_array(rng.permutation(2 * len(counts)).astype(np.uint64))
         pool = rng.integers(0, 256, layers * 2 * len(counts) * page_bytes, dtype=np.uint8)
+        before = [np.array([int(rng.integers(0, 1 << n)) for n in counts], np.uint32) for _ in range(3)]
         results = []
         for together in (False, True):
             b = sampling_buffers(backend, rows, vocabulary, logits, tokens=tokens, tree=tree)
             kv = backend.from_array(pool)
-            left = [backend.from_array(np.full(len(counts) * 4, 0, np.uint8)) for _ in range(3)]
+            left = [backend.from_array(x) for x in before]
             graph = splash_amd.CommandGraph()
             ops.Sampling.add_verify(graph, b, vocabulary, vocabulary, lanes, [0.0] * len(counts))
             if together:
@@ -113,3 +117,36 @@ def test_selection_acceptance_and_commit_in_one_dispatch(backend, dimension, kv_
             results.append([b["tokens"].download(), *(x.download() for x in left), kv.download()])
         for a, b in zip(*results):
             assert np.array_equal(a, b)
+
+
+# a workgroup's LDS holds a row's last column, the first row it does not hold, and a model without rotary pairs
+@pytest.mark.parametrize("hidden,pairs,entry", [(8192, 32, ["gguf_embed_norm_q4k"]), (512, 0, ["gguf_embed_norm_q4k"]),
+                                                (8448, 32, ["rope_build_tree_tables", "gguf_embed_q4k", "norm_rms_table16"]),
+                                                (8448, 0, ["gguf_embed_q4k", "norm_rms_table16"])])
+def test_a_steps_entry_takes_one_pass_where_a_row_fits(backend, hidden, pairs, entry):
+    """The first layer's projection of a step's rows is, bit for bit, that of the embedding and the layer on their own."""
+    print(f"case entry rule hidden={hidden} pairs={pairs}", flush=True)
+    from splash_amd import verify
+    from tests.dense_reference import DenseModel
+    Q, K, D, ffn, vocabulary = 4, 2, 64, 256, 512
+    m = DenseModel(3, hidden, Q, K, D, ffn, vocabulary, 1)
+    gpu = verify.DenseVerify(backend, hidden, Q, K, D, ffn, vocabulary, 1, rotary_pairs=pairs, max_lanes=2, physical_pages=2)
+    gpu.buffer(verify.PAGE_TABLE).upload(np.arange(2, dtype=np.uint64))
+    P, w, f = ops.Projection.from_native, m.layers[0], orc.FMT_Q4K
+    gpu.set_layer(0, P(backend, [(f, Q * D, w["q"]), (f, K * D, w["k"]), (f, K * D, w["v"])], hidden), P(backend, [(f, hidden, w["o"])], Q * D),
+                  P(backend, [(f, ffn, w["gate"])], hidden), P(backend, [(f, ffn, w["up"])], hidden), P(backend, [(f, hidden, w["down"])], ffn),
+                  *(backend.from_array(w[n]) for n in ("input_norm", "post_norm", "q_norm", "k_norm")))
+    gpu.set_head(f, backend.from_array(m.embedding), backend.from_array(m.final_norm), P(backend, [(orc.FMT_Q6K, vocabulary, m.head)], hidden, float32=True))
+    lanes = [verify.Lane(16, 0), verify.Lane(3, 0, table_first=1)]
+    gpu.set_block(lanes, np.random.default_rng(1).integers(0, vocabulary + 1, 19).astype(np.uint32))
+    got = []
+    graph = gpu.encode(lanes, commit=False)
+    assert graph.kernels()[:len(entry)] == entry, graph.kernels()
+    for run in (graph, gpu.encode_part(1, 0, lanes, gpu.encode_part(0, 0, lanes))):
+        for which in (verify.QKV_ROWS, verify.ATTENTION_ROWS):
+            rows = gpu.buffer(which)
+            rows.upload(np.full(rows.size_bytes // 2, 0x7FC0, np.uint16))
+        backend.run(run)
+        got.append([gpu.buffer(which).download(np.uint16) for which in (verify.QKV_ROWS, verify.ATTENTION_ROWS)])
+    for whole, parts, width in zip(*got, ((Q + 2 * K) * D, Q * D)):
+        assert np.isfinite(orc.bf16_to_f32(whole[:19 * width])).all() and np.array_equal(whole, parts)
