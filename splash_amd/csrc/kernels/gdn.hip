@@ -794,8 +794,11 @@ SP_REGISTER_KERNEL("gdn_prefill_scan", &gdn_prefill_scan);
 //   o_t = g_t S q_t + sum_{j <= t} A_tj u_j
 // depend on the block's rows alone: gdn_prefill_blocks works them out for every block at once, and what is left to do in
 // order, gdn_prefill_block_scan, is per block two products with the state, one with T and the state's update, all MFMAs.
-// A token is one dependent chain in gdn_prefill_scan (0.2 us each); here sixteen are: 2048 tokens of 16 / 32 heads 402 us there,
-// 13 + 93 us here (0.72 us a block). The sums' order differs from the fold's, so a chunk through these kernels leaves the accepted blocks' cell to rounding, not bit for bit.
+// (The chunkwise form of the gated delta rule: Yang, Kautz and Hatamizadeh, Gated Delta Networks, 2024, after Yang et al.,
+// Parallelizing Linear Transformers with the Delta Rule over Sequence Length, 2024; here with the system solved per block.)
+// A token is one dependent chain in gdn_prefill_scan (0.2 us each); here sixteen are: 2048 tokens of 16 / 32 heads 402 us
+// there, 13 + 93 us here (0.72 us a block). The sums' order differs from the fold's, so a chunk through these kernels leaves
+// the accepted blocks' cell to rounding, not bit for bit.
 // Precision: keys and queries are bf16, as they are; the state and the corrections enter their products as three bf16 parts
 // each, which hold all 24 bits, and every sum is fp32. Against 64-bit arithmetic the state of 32 heads is off by 5.0e-8 of
 // its norm where the scan's is by 5.7e-8, and the rows by the same rounding to bf16 (tests/test_gdn_blocks_gpu.py).
@@ -990,7 +993,8 @@ __global__ __launch_bounds__(320, 1) void gdn_prefill_block_scan(const uint16_t 
     f32x4 own, sum = zero;
 #pragma unroll
     for (uint32_t i = 0; i < 4; ++i)
-      own[i] = __fmaf_rn(-started[i], memory[i], weight[i] * __uint_as_float((used(f.value[i]) << valueShift) & 0xFFFF0000u));   // (the last product is exact)
+      // (the last product is exact)
+      own[i] = __fmaf_rn(-started[i], memory[i], weight[i] * __uint_as_float((used(f.value[i]) << valueShift) & 0xFFFF0000u));
 #pragma unroll
     for (uint32_t i = 0; i < 4; ++i) {   // token 4 kq + i in place kq
       sum = __builtin_amdgcn_mfma_f32_16x16x4f32(solve[i], own[i], sum, 0, 0, 0);

@@ -454,7 +454,8 @@ __device__ __forceinline__ void wide_workgroup(const WideTile &w, const uint8_t 
   };
   auto fetch = [&](uint32_t block, auto stageConstant) __attribute__((always_inline)) {   // block counts from b0
     constexpr uint32_t S = decltype(stageConstant)::value;
-    const uint32_t at = block < count ? (b0 + block) * (GGUF_WIDE_OPERANDS * 1024u) + S * 2048u : 0x80000000u;   // (past the part of K: zeros, no traffic)
+    // (past the part of K: zeros, no traffic)
+    const uint32_t at = block < count ? (b0 + block) * (GGUF_WIDE_OPERANDS * 1024u) + S * 2048u : 0x80000000u;
     uint4 *to = stageRows(stageConstant) + 64u * wave;
 #pragma unroll
     for (uint32_t i = 0; i < kShare; ++i) load_to_lds(rowValues, mineAt + (at + 2u * i * tileBytes), to + 256u * i);

@@ -21,8 +21,9 @@ __device__ __forceinline__ void arrived(uint4 &v) { asm volatile("" : "+v"(v.x),
 __device__ __forceinline__ void arrived(uint32_t &v) { asm volatile("" : "+v"(v)); }
 
 // `width` bf16 values (a multiple of 8, 16-byte aligned) on their way to LDS: every load of it goes out before any is stored,
-// and those of several rows before the first row's stores. No barrier. (With the loads sunk
-// to their stores the norm and its table were 7.9 us at 8 rows of 5120, 6.6 so; at 128 rows of 2048 5.8 either way.)
+// and those of several rows before the first row's stores. No barrier. (The norm and its table: 8.7 us at 8 rows of 5120 and
+// 6.4 at 128 of 2048 where each load was waited for; 7.9 and 5.8 with the loads unconditional but sunk to their stores; 6.6
+// and 5.8 so.)
 struct StagedRow {
   static constexpr uint32_t kHeld = kStagedWidth / 8u / 256u;
   uint4 held[kHeld];
@@ -149,7 +150,7 @@ __device__ __forceinline__ void write_table_row(const uint16_t *x, const uint16_
 
 // The same, and the activation table of the normalized rows: grid (tiles * 16) so that the rows
 // past the live ones are written as zeros. A handful of workgroups that only wait: every loop keeps several reads in
-// flight (6.4 us at 128 rows of 2048 while a staged row's reads waited for one another, 5.8 since).
+// flight (what that gives: at StagedRow).
 __global__ __launch_bounds__(256) void norm_rms_table16(const uint16_t *__restrict__ input, const uint16_t *__restrict__ weight,
                                                         uint16_t *__restrict__ output, uint8_t *__restrict__ table, NormParams p) {
   __shared__ float scratch[4];
@@ -178,8 +179,9 @@ SP_REGISTER_KERNEL("norm_rms_table16", &norm_rms_table16);
 // draft_conv (draft_attention.hip) and the pass that reads its rows, one workgroup a row: a Prepare stage's rows and their
 // activation table; a Residual stage's rows, their RMS norm (of `norm_weight`, into `normalized`) and its table. Each
 // convolution was a launch of its own before a launch of as few workgroups. Values and their order are the two kernels'.
-// The rows' 16-byte accesses are the host's rule (DraftAttention::addConvolutionTable). 8 rows of 5120: 5.2 us
-// for 3.1 + 3.0, 7.9 us for 3.1 + 8.7, and a launch less each: the draft model's pass of one lane 928, 923 and 938 us
+// The rows' 16-byte accesses are the host's rule (DraftAttention::addConvolutionTable). 8 rows of 5120, inside a draft
+// model's pass: 5.2 us for 3.1 + 3.0 and 7.5 for 3.1 + 6.6 (the norm's passes as they are now; 8.9 for 3.1 + 8.7 before
+// StagedRow's loads went out together), and a launch less each. The pass of one lane when it was fused: 928, 923 and 938 us
 // before, 869, 888 and 889 after, in three runs of both sides in turn whose repeats differ by 1 to 2 %.
 template <bool Residual>
 __global__ __launch_bounds__(256) void draft_conv_table(const uint16_t *__restrict__ input, const uint16_t *__restrict__ dynamic,

@@ -1,8 +1,9 @@
 // What a driver's lanes add to their sampling policies between steps: each dispatch lane's thinking cutoff
 // (ops::ThinkingCutoff), whether it is constrained by its rows of the token mask and whether it ignores end-of-sequence,
 // the step's stop tokens, the lane's penalties (ops::SamplingPenalties) and its row of the penalty table the driver owns,
-// `vocabulary` words a lane in device memory, allocated (zeroed) when a lane first takes active penalties. The reference's model keeps the table per state lane and the engine counts a step's tokens into it
-// on the host (Sampling.hpp:85-91, Sampling::countPenaltyTokens); here a step that commits counts them on the device.
+// `vocabulary` words a lane in device memory, allocated (zeroed) when a lane first takes active penalties. The reference's
+// model keeps the table per state lane and the engine counts a step's tokens into it on the host (Sampling.hpp:85-91,
+// Sampling::countPenaltyTokens); here a step that commits counts them on the device.
 #pragma once
 #include "hip/Backend.hpp"
 #include "ops/Sampling.hpp"

@@ -104,7 +104,8 @@ public:
   // A chunk of `tokens` rows of one lane, in runs that end at the captures (ascending, inside the rows): each run is
   // a prepare and a scan dispatch that continue from the cell the run before wrote, and one gate dispatch covers all
   // rows (GDN.cpp:176-222). The scan is sequential, so the runs compute bit for bit what one run computes. With buffers.blocks
-  // a run is a prepare, a blocks and a block scan dispatch, equal to the scan's results to fp32 rounding (however it is cut).
+  // a run is a prepare, a blocks and a block scan dispatch, equal to the scan's results to fp32 rounding (however it is cut);
+  // a value that is not finite reaches what it reaches in the scan.
   // 2048 tokens of 16 / 32 heads: 106 us for the two against 400 for the scan, which a caller keeps for its bits alone.
   static void addPrefill(hip::CommandGraph &graph, const GdnPrefillBuffers &buffers, const GdnShape &shape, uint32_t layer,
                          uint32_t tokens, const GdnStateStrides &state, GdnHeadOrder order,
