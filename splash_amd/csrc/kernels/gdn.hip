@@ -1054,10 +1054,11 @@ __global__ __launch_bounds__(320, 1) void gdn_prefill_block_scan(const uint16_t 
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    __threadfence();   // (the outputs of this run, before those of the run again)
     __syncthreads();
-    if (unbounded)
+    if (unbounded) {
+      __threadfence();   // (this run's outputs are out before the run again stores its first, behind two more barriers)
       for (uint32_t n = scan_barriers(p.tokens); n; --n) __syncthreads();
+    }
     return;
   }
   const float *stateIn = reinterpret_cast<const float *>(states + p.current_cell + p.convolution_state_bytes + uint64_t(p.layer) * p.recurrent_layer_bytes);
