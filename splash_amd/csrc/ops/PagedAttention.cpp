@@ -36,8 +36,8 @@ uint32_t totalRows(const std::vector<AttentionRows> &sequences) {
 // tokens 1 row 92 / 58, 4 rows 93 / 61 in two parts (76 as two tiles of one), 8 rows 92 / 80, 16 rows 90 / 144; 8 sequences behind
 // 16368 tokens 1 row 180 / 64, 4 rows 160 / 80 (100 in two parts), 8 rows 169 / 134, 16 rows 172 / 246; behind 4000 tokens and less
 // all of them lie within the fixed cost (23 / 22). So: up to eight rows; a tile a part while every part has a SIMD of its own
-// (four a compute unit), then two tiles a part, which widen the keys and values they share once. 16 / 8 heads of 64, 8 rows: 8 sequences behind
-// 16368 tokens 54 / 37; 16 rows 54 / 51 in two parts, within 1 us of each other elsewhere.
+// (four a compute unit), then two tiles a part, which widen the keys and values they share once. 16 / 8 heads of 64, 8 rows: 8
+// sequences behind 16368 tokens 54 / 37; 16 rows 54 / 51 in two parts, within 1 us of each other elsewhere.
 struct FewRows {
   uint32_t tiles = 0, parts = 0;
 };
