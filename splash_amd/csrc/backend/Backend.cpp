@@ -255,6 +255,7 @@ sp_status guardSubmit(sp_backend *backend) {
 sp_status beginTicket(sp_backend *backend, sp_completion completion, void *user, size_t marks, sp_ticket **out) {
   auto *ticket = new sp_ticket;
   ticket->backend = backend;
+  backend->retain();
   ticket->completion = completion;
   ticket->user = user;
   hipError_t e = backend->takeEvent(&ticket->start);
@@ -271,18 +272,22 @@ sp_status beginTicket(sp_backend *backend, sp_completion completion, void *user,
     if (ticket->end) (void)hipEventDestroy(ticket->end);
     if (ticket->fence) (void)hipEventDestroy(ticket->fence);
     delete ticket;
+    backend->release();
     return hipFail(e, "hipEventCreate");
   }
   *out = ticket;
   return SP_OK;
 }
 
+// (the last use of the ticket's backend, which may end with it: what else there is to do with it comes before)
 void destroyTicket(sp_ticket *ticket) {
+  sp_backend *backend = ticket->backend;
   for (hipEvent_t m : ticket->marks) (void)hipEventDestroy(m);
   for (hipEvent_t event : {ticket->start, ticket->end, ticket->fence})
-    if (event) ticket->backend->giveEvent(event);
+    if (event) backend->giveEvent(event);
   releaseAll(ticket->retained);
   delete ticket;
+  backend->release();
 }
 
 // Waits for the ticket's end event under the command watchdog (CommandWatchdog.hpp:16-44).
@@ -316,8 +321,8 @@ sp_status awaitTicket(sp_ticket *ticket) {
 sp_status finishSubmit(sp_backend *backend, sp_ticket *ticket, hipError_t launchError, sp_ticket **out) {
   if (launchError != hipSuccess) {
     (void)hipStreamSynchronize(backend->stream);
-    destroyTicket(ticket);
     backend->markUnhealthy(std::string("launch failed: ") + hipGetErrorString(launchError));
+    destroyTicket(ticket);
     return hipFail(launchError, "kernel launch");
   }
   if (ticket->completion) {
@@ -597,8 +602,8 @@ sp_status sp_ticket_wait_profiled(sp_ticket *ticket, double *gpu_seconds, double
   }
   if (status != SP_TIMEOUT) {
     // A command the watchdog gave up may still run: its buffers stay retained (leaked with the ticket).
-    destroyTicket(ticket);
     backend->inFlight = false;
+    destroyTicket(ticket);
   }
   return status;
 }
