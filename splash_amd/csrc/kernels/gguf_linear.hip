@@ -1197,11 +1197,12 @@ __device__ __forceinline__ void decode_workgroup(DecodeShared<RT> &shared, const
 }
 
 // Three waves a SIMD (168 registers) where a kernel would take a few registers more and run two: every format's four row
-// tiles, and Q6_K's two under some epilogues (a step of 8 layers and 24 rows in three lanes, whose down projections take the residual
-// and norm, 1755 -> 1670 us). Four (128) for Q6_K's one row tile spill outside the loop and are slower (16 rows 1307 ->
-// 1342 us a step).
+// tiles, and Q6_K's two under some epilogues (a step of 8 layers and 24 rows in three lanes, whose down projections take the
+// residual and norm, 1755 -> 1670 us). Four (128) for Q6_K's one row tile spill outside the loop and are slower (16 rows
+// 1307 -> 1342 us a step).
 template <uint32_t FMT, int RT, uint32_t EP, bool Staged = false>
-__global__ __launch_bounds__(256, RT > 2 || (RT == 2 && FMT == GGUF_FMT_Q6K) ? 3 : 1) void gguf_decode(const uint8_t *__restrict__ seg0, const uint8_t *__restrict__ seg1,
+__global__ __launch_bounds__(256, RT > 2 || (RT == 2 && FMT == GGUF_FMT_Q6K) ? 3 : 1)
+                                  void gguf_decode(const uint8_t *__restrict__ seg0, const uint8_t *__restrict__ seg1,
                                                    const uint8_t *__restrict__ seg2, const uint8_t *__restrict__ table,
                                                    void *__restrict__ out, const uint16_t *__restrict__ residual,
                                                    float *__restrict__ partials, uint32_t *__restrict__ counters,
