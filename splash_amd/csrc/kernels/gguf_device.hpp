@@ -27,12 +27,15 @@ __device__ __forceinline__ float byte_of(uint32_t word, uint32_t index) { return
 
 // Register j (0..3) of a group's bf16 operands 128 + code, from the two words that hold the
 // lane's eight codes of that group in their low (high = false) or high nibbles.
-// (a & mask) | base in one instruction: the mask rides the scalar bus, the base a register (on
-// this ISA a three-operand vector instruction takes no literal, so the compiler would emit two).
+// (a & mask) | base in one instruction: the mask rides the scalar bus, the base a register (on this ISA a three-operand
+// vector instruction takes no literal: the two are made opaque, or the compiler would emit two instructions). The
+// instruction itself is the compiler's: a matrix instruction that reads a vector instruction's result needs two wait states
+// behind it, which the compiler does not count behind inline assembly.
 __device__ __forceinline__ uint32_t and_or(uint32_t a, uint32_t mask, uint32_t base) {
-  uint32_t r;
-  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(mask), "v"(base));
-  return r;
+  uint32_t m = mask;
+  asm("" : "+s"(m));
+  asm("" : "+v"(base));
+  return (a & m) | base;
 }
 template <bool High, uint32_t Base = 0x43004300u> __device__ __forceinline__ uint4 q4_operands(uint32_t wa, uint32_t wb) {
   constexpr uint32_t kMask = 0x000F000Fu, kBase = Base;  // bf16 0x4300 = 128, ulp 1 (fp16 0x6400 = 1024, ulp 1)
