@@ -82,6 +82,13 @@ template <class T> __device__ __forceinline__ T wave_max_dpp(T v) {
 __device__ __forceinline__ uint32_t row_max_dpp(uint32_t v) {
   return dpp_max<kRowMirror>(dpp_max<kRowHalfMirror>(dpp_max<kQuadSwap2>(dpp_max<kQuadSwap1>(v))));
 }
+// The sum of each row of sixteen lanes, in every lane of the row: the additions of a butterfly over lanes 1, 2, 4 and 8 apart
+// (behind the first two steps a quad's lanes hold the same sum, behind the third an octet's, so a mirrored lane holds what
+// the lane 4 or 8 away does), without the LDS crossbar's latency a step.
+template <int Control> __device__ __forceinline__ float dpp_add(float v) { return v + __uint_as_float(dpp_move<Control>(__float_as_uint(v))); }
+__device__ __forceinline__ float row_sum_dpp(float v) {
+  return dpp_add<kRowMirror>(dpp_add<kRowHalfMirror>(dpp_add<kQuadSwap2>(dpp_add<kQuadSwap1>(v))));
+}
 // A wavefront's LDS writes before its later reads (its LDS operations are carried out in order).
 __device__ __forceinline__ void wave_lds_fence() { __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront"); }
 
