@@ -27,13 +27,9 @@ __device__ __forceinline__ float half_bits_to_float(uint32_t bits) {
 }
 __device__ __forceinline__ uint32_t float_to_half_bits(float v) { return __half_as_ushort(__float2half_rn(v)); }
 __device__ __forceinline__ float bf16_bits_to_float(uint32_t bits) { return __uint_as_float(bits << 16); }
-// Round to nearest even; NaN stays NaN.
-__device__ __forceinline__ uint32_t float_to_bf16_bits(float v) {
-  uint32_t u = __float_as_uint(v);
-  if ((u & 0x7FFFFFFFu) > 0x7F800000u) return (u >> 16) | 0x40u;
-  u += 0x7FFFu + ((u >> 16) & 1u);
-  return u >> 16;
-}
+// Round to nearest even; NaN stays NaN (its upper bits, quiet): the machine's own conversion, of all 2^32 values the same
+// bits as adding 0x7FFF and the last kept bit.
+__device__ __forceinline__ uint32_t float_to_bf16_bits(float v) { return __builtin_bit_cast(uint16_t, static_cast<__bf16>(v)); }
 __device__ __forceinline__ float round_bf16(float v) { return bf16_bits_to_float(float_to_bf16_bits(v)); }
 
 // x / (1 + 2^(-log2(e) x)), the reference's silu (kernels/common/activation.h:8-16).
