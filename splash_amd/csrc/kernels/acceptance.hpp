@@ -18,11 +18,12 @@ __device__ __forceinline__ Best better(Best a, Best b) {
 }
 // The best of `Lanes` neighbouring lanes, in each of them.
 template <int Lanes = 64> __device__ __forceinline__ Best wave_best(Best v) {
-#pragma unroll
-  for (int o = Lanes / 2; o > 0; o >>= 1) {
-    Best other{__shfl_xor(v.value, o, 64), __shfl_xor(v.index, o, 64)};
-    v = better(v, other);
-  }
+  if constexpr (Lanes > 32) v = better(v, Best{lane_xor<32>(v.value), lane_xor<32>(v.index)});
+  if constexpr (Lanes > 16) v = better(v, Best{lane_xor<16>(v.value), lane_xor<16>(v.index)});
+  if constexpr (Lanes > 8) v = better(v, Best{lane_xor<8>(v.value), lane_xor<8>(v.index)});
+  if constexpr (Lanes > 4) v = better(v, Best{lane_xor<4>(v.value), lane_xor<4>(v.index)});
+  if constexpr (Lanes > 2) v = better(v, Best{lane_xor<2>(v.value), lane_xor<2>(v.index)});
+  if constexpr (Lanes > 1) v = better(v, Best{lane_xor<1>(v.value), lane_xor<1>(v.index)});
   return v;
 }
 

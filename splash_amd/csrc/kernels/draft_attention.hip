@@ -157,9 +157,9 @@ __global__ __launch_bounds__(256) void draft_attention_split(const uint16_t *__r
       float dot = 0.f;
 #pragma unroll
       for (int i = 0; i < 16; ++i) dot += query[i] * bf16_bits_to_float(keys[j * kD + 16u * c + i]);
-      dot += __shfl_xor(dot, 1, 64);
-      dot += __shfl_xor(dot, 2, 64);
-      dot += __shfl_xor(dot, 4, 64);
+      dot += lane_xor<1>(dot);
+      dot += lane_xor<2>(dot);
+      dot += lane_xor<4>(dot);
       score[j] = dot * kScoreScale;
       best = fmaxf(best, score[j]);
     }
@@ -235,8 +235,8 @@ __global__ __launch_bounds__(256) void draft_attention_split(const uint16_t *__r
         s[g][t][i] = visible ? s[g][t][i] * kScoreScale : -INFINITY;
         most = fmaxf(most, s[g][t][i]);
       }
-    most = fmaxf(most, __shfl_xor(most, 16, 64));
-    most = fmaxf(most, __shfl_xor(most, 32, 64));
+    most = fmaxf(most, lane_xor<16>(most));
+    most = fmaxf(most, lane_xor<32>(most));
     const float safe = most == -INFINITY ? 0.f : most;
     float total = 0.f;
 #pragma unroll
@@ -247,8 +247,8 @@ __global__ __launch_bounds__(256) void draft_attention_split(const uint16_t *__r
         total += weight;
         weights[g][4 * t + i] = __bf16(weight);
       }
-    total += __shfl_xor(total, 16, 64);
-    total += __shfl_xor(total, 32, 64);
+    total += lane_xor<16>(total);
+    total += lane_xor<32>(total);
     best[g] = most;
     sum[g] = total;
     if (kq == 0) {
@@ -344,9 +344,9 @@ __global__ __launch_bounds__(1024) void draft_attention_merge(const float *__res
   const uint32_t packedRow = batch * kRows + queryRow, r = packedRow % 16u, tile = packedRow / 16u, G = DRAFT_ATTENTION_WIDTH / 32u;
   const uint32_t q = queryHead * (kD / 4u) + c, g = q / 8u, half = (q / 4u) % 2u, kq = q % 4u;
   float sum = (bf16_bits_to_float(low & 0xFFFFu) + bf16_bits_to_float(low >> 16)) + (bf16_bits_to_float(high & 0xFFFFu) + bf16_bits_to_float(high >> 16));
-  const float s1 = __shfl_down(sum, 1, 64), s2 = __shfl_down(sum, 2, 64), s3 = __shfl_down(sum, 3, 64);
+  const float s1 = lane_down<1>(sum), s2 = lane_down<2>(sum), s3 = lane_down<3>(sum);
   sum = ((sum + s1) + s2) + s3;
-  const float other = __shfl_down(sum, 4, 64);
+  const float other = lane_down<4>(sum);
   // operand elements 4 half + {0,1,2,3} are inputs 4 kq + {0,2,1,3} of the half
   reinterpret_cast<uint2 *>(table)[((size_t(tile) * G + g) * 64u + kq * 16u + r) * 2u + half] =
       make_uint2((low & 0xFFFFu) | (high << 16), (low >> 16) | (high & 0xFFFF0000u));

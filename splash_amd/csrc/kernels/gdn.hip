@@ -49,7 +49,7 @@ __device__ __forceinline__ float half_sum(float v) {
 // 32-channel groups' sums added in channel order.
 __device__ __forceinline__ float head_sum(float a, float b) {
   const float first = half_sum(a), second = half_sum(b);
-  const float s0 = __shfl(first, 0, 64), s1 = __shfl(first, 32, 64), s2 = __shfl(second, 0, 64), s3 = __shfl(second, 32, 64);
+  const float s0 = lane_value_of(first, 0), s1 = lane_value_of(first, 32), s2 = lane_value_of(second, 0), s3 = lane_value_of(second, 32);
   return ((s0 + s1) + s2) + s3;
 }
 __device__ __forceinline__ uint32_t path_row(uint32_t path, uint32_t depth) {
@@ -461,9 +461,9 @@ __global__ __launch_bounds__(64 * kWaves) void gdn_decode(const uint16_t *__rest
       const uint2 raw = *reinterpret_cast<const uint2 *>(&outputs[token][4u * run]);
       const uint32_t x0 = raw.x & 0xFFFFu, x1 = raw.x >> 16, x2 = raw.y & 0xFFFFu, x3 = raw.y >> 16;
       float sum = (bf16_bits_to_float(x0) + bf16_bits_to_float(x1)) + (bf16_bits_to_float(x2) + bf16_bits_to_float(x3));
-      const float s1 = __shfl_down(sum, 1, 64), s2 = __shfl_down(sum, 2, 64), s3 = __shfl_down(sum, 3, 64);
+      const float s1 = lane_down<1>(sum), s2 = lane_down<2>(sum), s3 = lane_down<3>(sum);
       sum = ((sum + s1) + s2) + s3;
-      const float other = __shfl_down(sum, 4, 64);
+      const float other = lane_down<4>(sum);
       if (lane < 32u) {
         // operand elements 4 half + {0,1,2,3} are inputs 4 kq + {0,2,1,3} of the half
         reinterpret_cast<uint2 *>(mine)[((size_t(tile) * G + g) * 64u + kq * 16u + r) * 2u + half] = make_uint2(x0 | (x2 << 16), x1 | (x3 << 16));

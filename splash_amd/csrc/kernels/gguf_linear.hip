@@ -1100,9 +1100,7 @@ __device__ __forceinline__ void decode_workgroup(DecodeShared<RT> &shared, const
         store_result<Chain>(&values[((size_t(t2) * G2 + g) * 64u + q4 * 16u + r) * 2u + h2],
                             uint64_t(x0 | (x2 << 16)) | uint64_t(x1 | (x3 << 16)) << 32);
         const float run = (bf16_bits_to_float(x0) + bf16_bits_to_float(x1)) + (bf16_bits_to_float(x2) + bf16_bits_to_float(x3));
-        const float r0 = __shfl(run, int(r), 64), r1 = __shfl(run, int(r) + 16, 64), r2 = __shfl(run, int(r) + 32, 64),
-                    r3 = __shfl(run, int(r) + 48, 64);
-        const float sum = ((r0 + r1) + r2) + r3;
+        const float sum = quarters_sum(run);   // (of quarter 0)
         if (q4 == 0) {
           store_result<Chain>(&sums16[(size_t(t2) * 2u * G2 + 2u * g + h2) * 16u + r], sum);
           halfSums[(t2 * 2u + h2) * 16u + r] = sum;
@@ -1170,9 +1168,7 @@ __device__ __forceinline__ void decode_workgroup(DecodeShared<RT> &shared, const
       store_result<Chain>(&values[((size_t(t2) * G2 + g2) * 64u + q4 * 16u + r) * 2u + h2],
                           uint64_t(x0 | (x2 << 16)) | uint64_t(x1 | (x3 << 16)) << 32);
       const float run = (bf16_bits_to_float(x0) + bf16_bits_to_float(x1)) + (bf16_bits_to_float(x2) + bf16_bits_to_float(x3));
-      const float r0 = __shfl(run, int(r), 64), r1 = __shfl(run, int(r) + 16, 64), r2 = __shfl(run, int(r) + 32, 64),
-                  r3 = __shfl(run, int(r) + 48, 64);
-      const float sum = ((r0 + r1) + r2) + r3;
+      const float sum = quarters_sum(run);   // (of quarter 0)
       if (q4 == 0) {
         store_result<Chain>(&sums16[(size_t(t2) * 2u * G2 + 2u * g2 + h2) * 16u + r], sum);
         halfSums[(t2 * 4u + w2) * 16u + r] = sum;

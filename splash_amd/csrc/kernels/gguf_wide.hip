@@ -137,15 +137,15 @@ __device__ __forceinline__ void wide_table_row(const uint16_t *__restrict__ inpu
       float s = 0.f;
 #pragma unroll
       for (int e = 0; e < 4; ++e) s += float(operand[e].x) + float(operand[e].y);
-      s += __shfl_xor(s, 1, 64);
-      s += __shfl_xor(s, 2, 64);
+      s += lane_xor<1>(s);
+      s += lane_xor<2>(s);
       s *= 0.03125f;
       const float first = float(_Float16(s)), second = float(_Float16(s - first)), third = float(_Float16((s - first) - second));
       const float mine = kq == 0u ? first : kq == 1u ? second : kq == 2u ? third : 0.f;
       // element g % 8 of the super-block's operand: the halves of eight threads into one 16-byte store
       const uint32_t part = as_word(f16x2{_Float16(mine), _Float16(0.f)}) & 0xFFFFu;
-      const uint32_t two = part | (uint32_t(__shfl_down(int(part), 4, 64)) << 16);
-      const uint32_t b = uint32_t(__shfl_down(int(two), 8, 64)), c = uint32_t(__shfl_down(int(two), 16, 64)), d = uint32_t(__shfl_down(int(two), 24, 64));
+      const uint32_t two = part | (lane_down<4>(part) << 16);
+      const uint32_t b = lane_down<8>(two), c = uint32_t(__shfl_down(int(two), 16, 64)), d = uint32_t(__shfl_down(int(two), 24, 64));
       if ((g & 7u) == 0 && g < groups) values[(size_t(g >> 3) * GGUF_WIDE_OPERANDS + 8u) * 64u + kq * 16u + r] = make_uint4(two, b, c, d);
     }
   if (tid == 0) reinterpret_cast<float *>(table + gguf_wide_scales_offset(p.input_size, p.tiles))[row] = inverseScale;

@@ -128,9 +128,9 @@ __device__ __forceinline__ void write_table_row(const uint16_t *x, const uint16_
     for (uint32_t j = 0; j < kRuns; ++j) {
       const uint32_t q = first + 256u * j + threadIdx.x;
       // run q: group g = q / 8, half = (q / 4) % 2, kq = q % 4; the four runs of a half sit in four consecutive lanes
-      const float s1 = __shfl_down(sum[j], 1, 64), s2 = __shfl_down(sum[j], 2, 64), s3 = __shfl_down(sum[j], 3, 64);
+      const float s1 = lane_down<1>(sum[j]), s2 = lane_down<2>(sum[j]), s3 = lane_down<3>(sum[j]);
       const float s = ((sum[j] + s1) + s2) + s3;   // of 16 inputs, in input order
-      const float other = __shfl_down(s, 4, 64);
+      const float other = lane_down<4>(s);
       if (q >= runs) continue;
       if constexpr (Normed)
         if (live)

@@ -49,8 +49,12 @@ __global__ __launch_bounds__(64) void moe_route_select(const float *__restrict__
     const float rowBest = wave_max(best);
     uint32_t candidate = best == rowBest ? lane + 64u * bestSlot : 0xFFFFFFFFu;
     uint32_t winner = candidate;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) winner = min(winner, uint32_t(__shfl_xor(int(winner), o, 64)));
+    winner = min(winner, lane_xor<32>(winner));
+    winner = min(winner, lane_xor<16>(winner));
+    winner = min(winner, lane_xor<8>(winner));
+    winner = min(winner, lane_xor<4>(winner));
+    winner = min(winner, lane_xor<2>(winner));
+    winner = min(winner, lane_xor<1>(winner));
     if (candidate == winner) {
 #pragma unroll
       for (uint32_t slot = 0; slot < kPerLane; ++slot)
@@ -266,13 +270,8 @@ __global__ __launch_bounds__(64) void moe_gather_table(const uint16_t *__restric
   reinterpret_cast<uint4 *>(table)[size_t(g) * 64u + lane] =
       make_uint4(bits[0] | (bits[1] << 16), bits[2] | (bits[3] << 16), bits[4] | (bits[5] << 16), bits[6] | (bits[7] << 16));
   const float half0 = (v[0] + v[2]) + (v[1] + v[3]), half1 = (v[4] + v[6]) + (v[5] + v[7]);
-  float h0[4], h1[4];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    h0[q] = __shfl(half0, int(r) + 16 * q, 64);
-    h1[q] = __shfl(half1, int(r) + 16 * q, 64);
-  }
-  const float s0 = ((h0[0] + h0[1]) + h0[2]) + h0[3], s1 = ((h1[0] + h1[1]) + h1[2]) + h1[3];
+  // (of quarter 0's lanes, the only ones that store them)
+  const float s0 = quarters_sum(half0), s1 = quarters_sum(half1);
   if (kq == 0) {
     float *sums32 = reinterpret_cast<float *>(table + gguf_table_sums32_offset(p.hidden, 1));
     float *sums16 = reinterpret_cast<float *>(table + gguf_table_sums16_offset(p.hidden, 1));
@@ -310,17 +309,17 @@ __global__ __launch_bounds__(256) void moe_combine(const uint16_t *__restrict__ 
   const float hidden = bf16_bits_to_float(bits);
   const uint32_t scaled = float_to_bf16_bits(hidden * bf16_bits_to_float(norm_weight[d]));
   const float v = bf16_bits_to_float(scaled);
-  const uint32_t b1 = uint32_t(__shfl_down(int(scaled), 1, 64)), b2 = uint32_t(__shfl_down(int(scaled), 2, 64)),
-                 b3 = uint32_t(__shfl_down(int(scaled), 3, 64));
-  const float v1 = __shfl_down(v, 1, 64), v2 = __shfl_down(v, 2, 64), v3 = __shfl_down(v, 3, 64);
+  const uint32_t b1 = lane_down<1>(scaled), b2 = lane_down<2>(scaled), b3 = lane_down<3>(scaled);
+  const float v1 = lane_down<1>(v), v2 = lane_down<2>(v), v3 = lane_down<3>(v);
   // sums of 16 inputs in input order: the four runs of a half are led by lanes 4 apart
   float s = (v + v1) + (v2 + v3);
-  const float s1 = __shfl_down(s, 4, 64), s2 = __shfl_down(s, 8, 64), s3 = __shfl_down(s, 12, 64);
+  const float s1 = lane_down<4>(s), s2 = lane_down<8>(s), s3 = lane_down<12>(s);
   s = ((s + s1) + s2) + s3;
-  const float other = __shfl_down(s, 16, 64);
+  const float other = lane_xor<16>(s);
   float square = hidden * hidden;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) square += __shfl_xor(square, o, 64);
+  square = row_sum_dpp(square);
+  square += lane_xor<16>(square);
+  square += lane_xor<32>(square);
   const uint32_t q = d / 4u, g = q / 8u, half = (q / 4u) % 2u, kq = q % 4u;  // the run of input d
   if ((lane & 3u) == 0) {
     // operand elements 4 half + {0,1,2,3} are inputs 4 kq + {0,2,1,3} of the half

@@ -593,8 +593,8 @@ __device__ __forceinline__ void attention_split(const _Float16 *__restrict__ que
     if (!owns[k]) continue;
     const uint32_t g = wave + 4u * k;
     float sum = l[k];
-    sum += __shfl_xor(sum, 16, 64);
-    sum += __shfl_xor(sum, 32, 64);
+    sum += lane_xor<16>(sum);
+    sum += lane_xor<32>(sum);
     const size_t fused = ((size_t(z) * p.kv_heads + h) * p.splits + split) * (16u * G) + 16u * g + row;
     const float rowSum = o[k][DT][0] * kCodeOffset;
     const float norm = sum > 0.f ? 1.0f / (sum * kPScale) : 0.f;
@@ -911,8 +911,8 @@ __global__ __launch_bounds__(64, 1) void attention_q8_few(const _Float16 *__rest
   for (int k = 0; k < T; ++k) {
     const uint32_t g = headOf(k);
     float sum = l[k];
-    sum += __shfl_xor(sum, 16, 64);
-    sum += __shfl_xor(sum, 32, 64);
+    sum += lane_xor<16>(sum);
+    sum += lane_xor<32>(sum);
     if (row >= seq.rows) continue;
     const size_t fused = ((size_t(z) * p.kv_heads + h) * p.splits + split) * (16u * G) + 16u * g + row;
     const float rowSum = o[k][DT][0] * kCodeOffset, norm = sum > 0.f ? 1.0f / (sum * kPScale) : 0.f;
@@ -1033,9 +1033,9 @@ __global__ __launch_bounds__(256) void attention_reduce(const _Float16 *__restri
       const uint32_t g = q / 8u, half = (q / 4u) % 2u, kq = q % 4u;
       reinterpret_cast<uint2 *>(mine)[((size_t(tile) * G + g) * 64u + kq * 16u + r) * 2u + half] = make_uint2(x0 | (x2 << 16), x1 | (x3 << 16));
       float s = (bf16_bits_to_float(x0) + bf16_bits_to_float(x1)) + (bf16_bits_to_float(x2) + bf16_bits_to_float(x3));
-      const float s1 = __shfl_down(s, 1, 64), s2 = __shfl_down(s, 2, 64), s3 = __shfl_down(s, 3, 64);
+      const float s1 = lane_down<1>(s), s2 = lane_down<2>(s), s3 = lane_down<3>(s);
       s = ((s + s1) + s2) + s3;
-      const float other = __shfl_down(s, 4, 64);
+      const float other = lane_down<4>(s);
       if (kq == 0) {
         float *sums32 = reinterpret_cast<float *>(mine + gguf_table_sums32_offset(width, tiles));
         float *sums16 = reinterpret_cast<float *>(mine + gguf_table_sums16_offset(width, tiles));

@@ -388,8 +388,12 @@ __global__ __launch_bounds__(256) void decode_sample_mass_sharded(const float *_
     mine = merge(mine, Mass{value, 1.0f}, inverse);
   }
   // lanes in a fixed butterfly, then the four wavefronts in order
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) mine = merge(mine, Mass{__shfl_xor(mine.maximum, o, 64), __shfl_xor(mine.sum, o, 64)}, inverse);
+  mine = merge(mine, Mass{lane_xor<32>(mine.maximum), lane_xor<32>(mine.sum)}, inverse);
+  mine = merge(mine, Mass{lane_xor<16>(mine.maximum), lane_xor<16>(mine.sum)}, inverse);
+  mine = merge(mine, Mass{lane_xor<8>(mine.maximum), lane_xor<8>(mine.sum)}, inverse);
+  mine = merge(mine, Mass{lane_xor<4>(mine.maximum), lane_xor<4>(mine.sum)}, inverse);
+  mine = merge(mine, Mass{lane_xor<2>(mine.maximum), lane_xor<2>(mine.sum)}, inverse);
+  mine = merge(mine, Mass{lane_xor<1>(mine.maximum), lane_xor<1>(mine.sum)}, inverse);
   if ((tid & 63u) == 0) {
     shared[tid >> 6][0] = mine.maximum;
     shared[tid >> 6][1] = mine.sum;
@@ -409,9 +413,9 @@ SP_REGISTER_KERNEL("decode_sample_mass_sharded", &decode_sample_mass_sharded);
 __device__ __forceinline__ Mass row_mass(const float *masses, uint32_t row, float inverse) {
   const uint32_t shard = (threadIdx.x & 63u) % SAMPLING_SHARDS;
   const float2 mine = reinterpret_cast<const float2 *>(masses)[row * SAMPLING_SHARDS + shard];
-  Mass all{__shfl(mine.x, 0, 64), __shfl(mine.y, 0, 64)};
+  Mass all{lane_value_of(mine.x, 0), lane_value_of(mine.y, 0)};
 #pragma unroll
-  for (int s = 1; s < int(SAMPLING_SHARDS); ++s) all = merge(all, Mass{__shfl(mine.x, s, 64), __shfl(mine.y, s, 64)}, inverse);
+  for (int s = 1; s < int(SAMPLING_SHARDS); ++s) all = merge(all, Mass{lane_value_of(mine.x, s), lane_value_of(mine.y, s)}, inverse);
   return all;
 }
 // The child of `row` in its lane's block: the first later row whose parent it is; none: SAMPLING_NO_TOKEN.
@@ -467,6 +471,26 @@ __device__ __forceinline__ float kept_weight(float logit, uint32_t token, const 
 __device__ __forceinline__ float residual_of(float logit, uint32_t token, float q, const Kept &kept, float inverse, bool rejected) {
   const float w = kept_weight(logit, token, kept, inverse);
   return rejected ? fmaxf(w / kept.mass.sum - q, 0.f) : w;
+}
+// The residual weights of tokens first .. first + count, below end, summed in order; eight tokens' loads are on their way
+// together (one past the end reads the last and adds nothing).
+__device__ __forceinline__ float lane_residual(const float *x, const float *q, uint32_t first, uint32_t count, uint32_t end, const Kept &kept,
+                                               float inverse, bool rejected) {
+  constexpr uint32_t kAhead = 8;
+  float sum = 0.f;
+  for (uint32_t i0 = 0; i0 < count; i0 += kAhead) {
+    float logits[kAhead], drafted[kAhead];
+#pragma unroll
+    for (uint32_t i = 0; i < kAhead; ++i) {
+      const uint32_t at = min(first + i0 + i, end - 1u);
+      logits[i] = x[at];
+      drafted[i] = rejected ? q[at] : 0.f;
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < kAhead; ++i)
+      if (i0 + i < count && first + i0 + i < end) sum += residual_of(logits[i], first + i0 + i, drafted[i], kept, inverse, rejected);
+  }
+  return sum;
 }
 // ---------------------------------------------------------------------------------------------
 // decode_sample_distribution_end: grid (rows), 1024 threads. Writes the row's end words of the
@@ -874,16 +898,29 @@ __global__ __launch_bounds__(256) void decode_sample_residual_ranges(const float
   // the range's residual: a lane sums its tokens in id order, the lanes are added in order
   const uint32_t size = range_tokens(p.vocabulary), begin = range * size, end = min(p.vocabulary, begin + size);
   const uint32_t per = (size + 63u) / 64u;
-  float sum = 0.f;
-  for (uint32_t i = 0; i < per; ++i) {
-    const uint32_t token = begin + lane * per + i;
-    if (token < end) sum += residual_of(x[token], token, rejected ? q[token] : 0.f, kept, inverse, rejected);
-  }
+  const float sum = lane_residual(x, q, begin + lane * per, per, end, kept, inverse, rejected);
   float total = 0.f;
-  for (int l = 0; l < 64; ++l) total += __shfl(sum, l, 64);
+#pragma unroll
+  for (int l = 0; l < 64; ++l) total += lane_value_of(sum, l);
   if (lane == 0) ranges[row * SAMPLING_RANGES + range] = total;
 }
 SP_REGISTER_KERNEL("decode_sample_residual_ranges", &decode_sample_residual_ranges);
+
+// The wavefront's 64 values, in every lane, for a walk in lane order: once through LDS, where a shuffle a step would wait for
+// each. `staged` is the wavefront's own.
+__device__ __forceinline__ void wave_values(float mine, float *staged, float (&values)[64]) {
+  wave_lds_fence();   // (what the walk before read)
+  staged[threadIdx.x & 63u] = mine;
+  wave_lds_fence();
+#pragma unroll
+  for (uint32_t i = 0; i < 16; ++i) {
+    const float4 v = reinterpret_cast<const float4 *>(staged)[i];
+    values[4 * i] = v.x;
+    values[4 * i + 1] = v.y;
+    values[4 * i + 2] = v.z;
+    values[4 * i + 3] = v.w;
+  }
+}
 
 // Grid (rows), 64 threads: the row's selection. A sampled row whose child was accepted selects it;
 // otherwise it draws at point = u_row * sum of the ranges, from the residual when its child was
@@ -907,6 +944,7 @@ __global__ __launch_bounds__(64) void decode_sample_draw(const float *__restrict
   const float *r = ranges + row * SAMPLING_RANGES;
   // the ranges in LDS: the sums walk them in order without a trip to memory each
   __shared__ float weights[SAMPLING_RANGES];
+  __shared__ __align__(16) float staged[64];
 #pragma unroll
   for (uint32_t i = 0; i < SAMPLING_RANGES / 64u; ++i) weights[lane + 64u * i] = r[lane + 64u * i];
   __syncthreads();
@@ -936,16 +974,14 @@ __global__ __launch_bounds__(64) void decode_sample_draw(const float *__restrict
   // Its lanes' chunks, as the ranges kernel summed them, walked in lane order.
   const uint32_t size = range_tokens(p.vocabulary), begin = hit * size, end = min(p.vocabulary, begin + size);
   const uint32_t per = (size + 63u) / 64u;
-  float sum = 0.f;
-  for (uint32_t i = 0; i < per; ++i) {
-    const uint32_t token = begin + lane * per + i;
-    if (token < end) sum += residual_of(x[token], token, rejected ? q[token] : 0.f, kept, inverse, rejected);
-  }
+  const float sum = lane_residual(x, q, begin + lane * per, per, end, kept, inverse, rejected);
   uint32_t chunk = 64, lastChunk = 0;
   float chunkBefore = 0.f, lastChunkBefore = 0.f, cumulative = 0.f;
+  float sums[64];
+  wave_values(sum, staged, sums);
 #pragma unroll
   for (int l = 0; l < 64; ++l) {
-    const float c = __shfl(sum, l, 64);
+    const float c = sums[l];
     if (c > 0.f) { lastChunk = uint32_t(l); lastChunkBefore = cumulative; }
     if (chunk == 64 && target < cumulative + c) { chunk = uint32_t(l); chunkBefore = cumulative; }
     cumulative += c;
@@ -959,8 +995,12 @@ __global__ __launch_bounds__(64) void decode_sample_draw(const float *__restrict
     const uint32_t own = begin + chunk * per + i0 + lane;
     const bool live = i0 + lane < per && own < end;
     const float weight = live ? residual_of(x[own], own, rejected ? q[own] : 0.f, kept, inverse, rejected) : 0.f;
-    for (uint32_t i = 0; i < 64u && i0 + i < per; ++i) {
-      const float w = __shfl(weight, int(i), 64);
+    float token_weights[64];
+    wave_values(weight, staged, token_weights);
+#pragma unroll
+    for (uint32_t i = 0; i < 64u; ++i) {
+      if (i0 + i >= per) break;
+      const float w = token_weights[i];
       const uint32_t token = begin + chunk * per + i0 + i;
       if (w > 0.f) lastToken = token;
       walked += w;
@@ -992,6 +1032,7 @@ __global__ __launch_bounds__(64) void decode_sample_draw_children(const float *_
   constexpr uint32_t K = SAMPLING_CANDIDATES;
   __shared__ float rangeWeight[SAMPLING_RANGES];
   __shared__ float candidateWeight[K];
+  __shared__ __align__(16) float staged[64];
   __shared__ uint32_t excludedIds[K];
   __shared__ uint32_t decided[4];  // selected (1) or walking (0), token or range, target bits, excluding
   const uint32_t row = blockIdx.x, lane = threadIdx.x;
@@ -1111,8 +1152,11 @@ __global__ __launch_bounds__(64) void decode_sample_draw_children(const float *_
   }
   uint32_t chunk = 64, lastChunk = 0;
   float chunkBefore = 0.f, lastChunkBefore = 0.f, cumulative = 0.f;
+  float sums[64];
+  wave_values(sum, staged, sums);
+#pragma unroll
   for (int l = 0; l < 64; ++l) {
-    const float c = __shfl(sum, l, 64);
+    const float c = sums[l];
     if (c > 0.f) { lastChunk = uint32_t(l); lastChunkBefore = cumulative; }
     if (chunk == 64 && c > 0.f && target < cumulative + c) { chunk = uint32_t(l); chunkBefore = cumulative; }
     cumulative += c;
