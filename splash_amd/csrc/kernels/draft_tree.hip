@@ -10,7 +10,8 @@
 // exactly "the largest estimate, the earlier entry among equal ones"; a draw is a 16-lane maximum over the Gumbel keys (a
 // hash of the row's key and the candidate's token a lane). Sums whose order decides a float's bits (a distribution's mass)
 // are taken in candidate order, as a sequential statement takes them, so the values agree with it to the rounding of exp
-// and log alone. Eight lanes' trees of 16 rows: 61 -> 36 us (all of it in one wavefront, with LDS between the steps, before).
+// and log alone. Eight lanes' trees of 16 rows: 61 -> 36 us (all of it in one wavefront, with LDS between the steps, before),
+// -> 31.6 with four teams of threads on the distributions (6 us of the pass by now; a step of the growth is 1.6).
 #include "abi/PagedAttention.h"
 #include "abi/Sampling.h"
 #include "backend/KernelRegistry.hpp"
@@ -55,6 +56,7 @@ __device__ __forceinline__ float ordered_sum(const float *values) {
 struct TreeState {
   float probability[kPositions][kCandidates][kCandidates];
   float drafted[kPositions][kCandidates][kCandidates];
+  float logDrafted[kPositions][kCandidates][kCandidates];
   float estimate[kPositions][kCandidates][kCandidates];
   uint32_t order[kPositions][kCandidates][kCandidates];
   uint8_t likeliest[kPositions][kCandidates][kChildren];
@@ -63,7 +65,8 @@ struct TreeState {
 
 } // namespace
 
-__global__ __launch_bounds__(256) void draft_select_tree(const uint32_t *__restrict__ candidates, const float *__restrict__ unary,
+constexpr uint32_t kTreeThreads = 1024, kLatticeThreads = kCandidates * kCandidates, kTeams = kTreeThreads / kLatticeThreads;
+__global__ __launch_bounds__(kTreeThreads) void draft_select_tree(const uint32_t *__restrict__ candidates, const float *__restrict__ unary,
                                                          const float *__restrict__ edges, const uint32_t *__restrict__ chain_tokens,
                                                          const float *__restrict__ chain_rates, uint32_t *__restrict__ tokens,
                                                          AttentionTreeRow *__restrict__ tree, float *__restrict__ scores,
@@ -78,16 +81,21 @@ __global__ __launch_bounds__(256) void draft_select_tree(const uint32_t *__restr
   const float rates = tid < kRates ? chain_rates[size_t(lane) * kRates + tid] : 0.f;
 
   // ---- The lattice: sixteen threads, a candidate each, a predecessor (position 0 follows the anchor alone, predecessor 0;
-  // what the others compute there is not read), all positions side by side. Sixteen threads share a wavefront, whose LDS
-  // operations are in order, so nothing here waits for the workgroup.
+  // what the others compute there is not read); a team of 256 threads every fourth position, its two side by side (one team,
+  // seven positions a thread, took the longer half of the kernel). Sixteen threads share a wavefront, whose LDS operations
+  // are in order, so nothing here waits for the workgroup.
   {
-    const uint32_t predecessor = tid / kCandidates;
-    float score[kPositions], weight[kPositions];
+    constexpr uint32_t kEach = (kPositions + kTeams - 1u) / kTeams;
+    const uint32_t predecessor = tid % kLatticeThreads / kCandidates, team = tid / kLatticeThreads;
+    uint32_t positions[kEach];   // (one past the last: not worked, by whole wavefronts)
+    float score[kEach], weight[kEach];
 #pragma unroll
-    for (uint32_t position = 0; position < kPositions; ++position) {
+    for (uint32_t e = 0; e < kEach; ++e) {
+      const uint32_t position = positions[e] = team + kTeams * e;
+      if (position >= kPositions) break;
       const size_t at = origin + position * kCandidates;
-      if (tid < kCandidates) s.ids[position][i] = candidates[at + i];
-      score[position] = unary[at + i] + edges[(at + predecessor) * kCandidates + i];
+      if (predecessor == 0) s.ids[position][i] = candidates[at + i];
+      score[e] = unary[at + i] + edges[(at + predecessor) * kCandidates + i];
     }
     auto largest = [](float v) {   // of sixteen, as fmaxf has it
       v = fmaxf(v, __uint_as_float(dpp_move<kQuadSwap1>(__float_as_uint(v))));
@@ -96,41 +104,51 @@ __global__ __launch_bounds__(256) void draft_select_tree(const uint32_t *__restr
       return fmaxf(v, __uint_as_float(dpp_move<kRowMirror>(__float_as_uint(v))));
     };
 #pragma unroll
-    for (uint32_t position = 0; position < kPositions; ++position) {
-      weight[position] = expf(score[position] - largest(score[position]));
-      s.probability[position][predecessor][i] = weight[position];
-      s.order[position][predecessor][i] = order_bits(score[position] + 0.0f);
+    for (uint32_t e = 0; e < kEach; ++e) {
+      const uint32_t position = positions[e];
+      if (position >= kPositions) break;
+      weight[e] = expf(score[e] - largest(score[e]));
+      s.probability[position][predecessor][i] = weight[e];
+      s.order[position][predecessor][i] = order_bits(score[e] + 0.0f);
     }
     wave_lds_fence();
 #pragma unroll
-    for (uint32_t position = 0; position < kPositions; ++position) {
+    for (uint32_t e = 0; e < kEach; ++e) {
+      const uint32_t position = positions[e];
+      if (position >= kPositions) break;
       // the four likeliest, the lower index first among equal scores
       uint32_t rank = 0;
-      const uint32_t mine = order_bits(score[position] + 0.0f);
+      const uint32_t mine = order_bits(score[e] + 0.0f);
 #pragma unroll
       for (uint32_t c = 0; c < kCandidates; ++c) {
         const uint32_t other = s.order[position][predecessor][c];
         rank += other > mine || (other == mine && c < i) ? 1u : 0u;
       }
       if (rank < kChildren) s.likeliest[position][predecessor][rank] = uint8_t(i);
-      weight[position] /= ordered_sum(s.probability[position][predecessor]);
+      weight[e] /= ordered_sum(s.probability[position][predecessor]);
     }
     wave_lds_fence();
 #pragma unroll
-    for (uint32_t position = 0; position < kPositions; ++position) {
-      const float q = weight[position], top = largest(q);
+    for (uint32_t e = 0; e < kEach; ++e) {
+      const uint32_t position = positions[e];
+      if (position >= kPositions) break;
+      const float q = weight[e], top = largest(q);
       s.probability[position][predecessor][i] = q;
-      weight[position] = temperature == 0.0f || !(q > 0.0f) ? q : expf((logf(q) - logf(top)) / temperature);
-      s.drafted[position][predecessor][i] = weight[position];
+      weight[e] = temperature == 0.0f || !(q > 0.0f) ? q : expf((logf(q) - logf(top)) / temperature);
+      s.drafted[position][predecessor][i] = weight[e];
     }
     wave_lds_fence();
 #pragma unroll
-    for (uint32_t position = 0; position < kPositions; ++position) weight[position] /= ordered_sum(s.drafted[position][predecessor]);
+    for (uint32_t e = 0; e < kEach; ++e)
+      if (positions[e] < kPositions) weight[e] /= ordered_sum(s.drafted[positions[e]][predecessor]);
     wave_lds_fence();
 #pragma unroll
-    for (uint32_t position = 0; position < kPositions; ++position) {
-      s.drafted[position][predecessor][i] = weight[position];
-      const float q = fminf(fmaxf(weight[position], 1.0e-6f), 1.0f - 1.0e-6f);
+    for (uint32_t e = 0; e < kEach; ++e) {
+      const uint32_t position = positions[e];
+      if (position >= kPositions) break;
+      s.drafted[position][predecessor][i] = weight[e];
+      s.logDrafted[position][predecessor][i] = logf(weight[e]);
+      const float q = fminf(fmaxf(weight[e], 1.0e-6f), 1.0f - 1.0e-6f);
       const float z = slope * logf(q / (1.0f - q)) + p.intercept[lane][position];
       s.estimate[position][predecessor][i] = 1.0f / (1.0f + expf(-z));
     }
@@ -187,6 +205,7 @@ __global__ __launch_bounds__(256) void draft_select_tree(const uint32_t *__restr
                     float chainRateHere) __attribute__((always_inline)) {
     const float q = s.probability[position][predecessor][i], mine = s.drafted[position][predecessor][i];
     const float estimate = s.estimate[position][predecessor][i];
+    const float logMine = s.logDrafted[position][predecessor][i];
     const uint32_t id = s.ids[position][i], likeliest = *reinterpret_cast<const uint32_t *>(s.likeliest[position][predecessor]);
     if (tid < kCandidates) next[(size_t(lane) * kRows + row) * kCandidates + i] = mine;
     expanded |= 1u << row;
@@ -194,7 +213,7 @@ __global__ __launch_bounds__(256) void draft_select_tree(const uint32_t *__restr
     float key = -INFINITY;
     if (temperature > 0.0f) {
       const uint64_t rowKey = uint64_t(lane_value(rowKeyHigh, row)) << 32 | lane_value(rowKeyLow, row);
-      if (mine > 0.0f) key = logf(mine) + gumbel_of(rowKey, id);
+      if (mine > 0.0f) key = logMine + gumbel_of(rowKey, id);
     }
     uint32_t taken = 0;
     float bound = score, left = 1.0f - chainRateHere, reserved = chainRateHere;

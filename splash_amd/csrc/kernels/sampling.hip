@@ -184,13 +184,18 @@ __global__ __launch_bounds__(128) void draft_verify_rows(const uint32_t *__restr
                                                          SamplingLaneRows *__restrict__ lane_rows, uint32_t *__restrict__ sources,
                                                          VerifyRowsParams p) {
   constexpr uint32_t kLanes = SAMPLING_MAXIMUM_LANES, kRows = SAMPLING_MAXIMUM_ROWS, kAll = kLanes * kRows;
-  __shared__ float estimateOf[kAll];
+  __shared__ __align__(16) float estimateOf[kAll];
   __shared__ uint32_t rankedOwner[kAll];   // the lane of the candidate at each place of the order, kLanes for none
   __shared__ float rankedEstimate[kAll];
   __shared__ uint32_t eligibleBefore[2];   // eligible candidates in the first wave's places
-  __shared__ uint32_t takenOf[kLanes];
-  __shared__ uint32_t pathOf[kAll];        // a row's ancestors and itself, in its tree's own numbering
-  __shared__ uint32_t placeOf[kAll];       // a row's place in its lane's preorder
+  __shared__ __align__(16) uint32_t takenOf[kLanes];
+  __shared__ __align__(16) uint32_t pathOf[kAll];   // a row's ancestors and itself, in its tree's own numbering
+  __shared__ __align__(16) uint32_t placeOf[kAll];  // a row's place in its lane's preorder
+  // (the lists are read whole, sixteen bytes at a time, before the first of them is used: entry by entry each would be waited for)
+  auto four = [](const uint32_t *from, uint32_t i, uint32_t (&to)[4]) {
+    const uint4 v = reinterpret_cast<const uint4 *>(from)[i];
+    to[0] = v.x, to[1] = v.y, to[2] = v.z, to[3] = v.w;
+  };
   if (blockIdx.x) return;
   const uint32_t t = threadIdx.x, lane = t / kRows, row = t % kRows, lanes = min(p.lanes, kLanes);
   const uint32_t size = lane < lanes ? min(sizes[lane], kRows) : 0u;
@@ -208,10 +213,12 @@ __global__ __launch_bounds__(128) void draft_verify_rows(const uint32_t *__restr
   __syncthreads();
   if (candidate) {
     uint32_t rank = 0;
-#pragma unroll 16
-    for (uint32_t other = 0; other < kAll; ++other) {   // (no candidate: -infinity)
-      const float e = estimateOf[other];
-      rank += (e > estimate || (e == estimate && other < t)) && e != -INFINITY ? 1u : 0u;
+#pragma unroll
+    for (uint32_t i = 0; i < kAll / 4u; ++i) {   // (no candidate: -infinity)
+      const float4 e4 = reinterpret_cast<const float4 *>(estimateOf)[i];
+      const float e[4] = {e4.x, e4.y, e4.z, e4.w};
+#pragma unroll
+      for (uint32_t k = 0; k < 4; ++k) rank += (e[k] > estimate || (e[k] == estimate && 4u * i + k < t)) && e[k] != -INFINITY ? 1u : 0u;
     }
     rankedOwner[rank] = lane;
     rankedEstimate[rank] = estimate;
@@ -236,33 +243,52 @@ __global__ __launch_bounds__(128) void draft_verify_rows(const uint32_t *__restr
   if (eligible && earlier < budget) atomicAdd(&takenOf[owner], 1u);
   __syncthreads();
   // Back to thread (lane, row): the lane keeps its anchor and its first taken rows.
-  const uint32_t mine = lane < lanes ? takenOf[lane] + 1u : 0u;
-  uint32_t first = 0, total = 0;
-  for (uint32_t l = 0; l < lanes; ++l) {
-    first += l < lane ? takenOf[l] + 1u : 0u;
-    total += takenOf[l] + 1u;
+  uint32_t mine = 0, first = 0, total = 0;
+#pragma unroll
+  for (uint32_t i = 0; i < kLanes / 4u; ++i) {
+    uint32_t taken[4];
+    four(takenOf, i, taken);
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+      const uint32_t l = 4u * i + k, here = l < lanes ? taken[k] + 1u : 0u;
+      mine = l == lane ? here : mine;
+      first += l < lane ? here : 0u;
+      total += here;
+    }
   }
   if (p.slots) first = lane * p.lane_cap;
   const bool placed = row < mine;
   const AttentionTreeRow node = placed ? read : AttentionTreeRow{0u, 0u, 0u};
   pathOf[t] = placed ? node.ancestors : 0u;
   __syncthreads();
+  static_assert(kRows == 16 && kLanes % 4 == 0, "a lane's rows are four reads");
   uint32_t place = 0;
   if (placed) {
     const uint32_t path = node.ancestors;
-    for (uint32_t x = 0; x < mine; ++x) {
-      if (x == row) continue;
-      const uint32_t other = pathOf[lane * kRows + x], common = other & path;
-      const bool ancestor = (path >> x) & 1u, descendant = (other >> row) & 1u;
-      const bool earlierBranch = __builtin_ctz((other & ~common) | 0x10000u) < __builtin_ctz((path & ~common) | 0x10000u);
-      place += ancestor || (!descendant && earlierBranch) ? 1u : 0u;
+#pragma unroll
+    for (uint32_t i = 0; i < kRows / 4u; ++i) {
+      uint32_t paths[4];
+      four(pathOf + lane * kRows, i, paths);
+#pragma unroll
+      for (uint32_t k = 0; k < 4; ++k) {
+        const uint32_t x = 4u * i + k, other = paths[k], common = other & path;
+        const bool ancestor = (path >> x) & 1u, descendant = (other >> row) & 1u;
+        const bool earlierBranch = __builtin_ctz((other & ~common) | 0x10000u) < __builtin_ctz((path & ~common) | 0x10000u);
+        place += x < mine && x != row && (ancestor || (!descendant && earlierBranch)) ? 1u : 0u;
+      }
     }
   }
   placeOf[t] = place;
   __syncthreads();
   if (placed) {
     uint32_t ancestors = 0;
-    for (uint32_t walk = node.ancestors; walk; walk &= walk - 1u) ancestors |= 1u << placeOf[lane * kRows + uint32_t(__builtin_ctz(walk))];
+#pragma unroll
+    for (uint32_t i = 0; i < kRows / 4u; ++i) {
+      uint32_t places[4];
+      four(placeOf + lane * kRows, i, places);
+#pragma unroll
+      for (uint32_t k = 0; k < 4; ++k) ancestors |= (node.ancestors >> (4u * i + k) & 1u) << (places[k] & 31u);
+    }
     const uint32_t depth = uint32_t(__builtin_popcount(node.ancestors)) - 1u;
     const uint32_t up = row ? placeOf[lane * kRows + node.parent] : SAMPLING_TREE_ROOT;
     tokens[first + place] = token;

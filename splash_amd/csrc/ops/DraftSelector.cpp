@@ -78,7 +78,7 @@ void DraftSelector::addTree(hip::CommandGraph &graph, const DraftTreeBuffers &b,
   graph.add("draft_select_tree",
             {b.candidates, b.unary, b.edges, b.chainTokens, b.chainRates, b.treeTokens, b.trees, b.treeScores, b.treeSizes, b.treeDraws,
              b.treeNext, b.treeCaps},
-            params, {params.lanes, 1, 1}, {256, 1, 1});
+            params, {params.lanes, 1, 1}, {1024, 1, 1});
 }
 
 void DraftSelector::addVerifyChildren(hip::CommandGraph &graph, const DraftVerifyChildrenBuffers &b, const StepRows &step) {
