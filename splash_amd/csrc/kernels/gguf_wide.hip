@@ -414,16 +414,20 @@ __device__ __forceinline__ void wide_columns(WideTile &w, const uint8_t *seg0, c
   }
 }
 
+// A workgroup's LDS: a super-block's four stages, each [row tile][group][lane], and its sums. Objects of their own, so that a
+// read of one does not wait for what is on its way into another.
+struct WideLds {
+  uint4 *rows0, *rows1, *rows2, *rows3, *sums;
+};
+template <uint32_t T> constexpr uint32_t kWideStageVectors = (T + 1) / 2 * 2 * 2 * 64;
+template <uint32_t FMT, uint32_t T, bool Staged> constexpr uint32_t kWideSumVectors = FMT != GGUF_FMT_Q6K && !Staged ? (T + 3) / 4 * 4 * 64 : 1;
+
 // T: the row tiles a workgroup computes, at least those it takes (a tile past them multiplies zeros).
 template <uint32_t FMT, uint32_t EP, uint32_t T, bool Staged>
-__device__ __forceinline__ void wide_workgroup(const WideTile &w, const uint8_t *__restrict__ table, void *__restrict__ out,
+__device__ __forceinline__ void wide_workgroup(const WideLds lds, const WideTile &w, const uint8_t *__restrict__ table, void *__restrict__ out,
                                                const uint16_t *__restrict__ residual, const GgufWideParams &p) {
   constexpr uint32_t kRecord = gguf_record_bytes(FMT);
   constexpr bool kSums = FMT != GGUF_FMT_Q6K && !Staged, kTwice = FMT == GGUF_FMT_Q6K && !Staged, kGateUp = EP == GGUF_WIDE_GATE_UP;
-  // A super-block's four stages, each [row tile][group][lane], and its sums: objects of their own, so that a read of one
-  // does not wait for what is on its way into another.
-  constexpr uint32_t kTiles = (T + 1) / 2 * 2, kStageVectors = kTiles * 2 * 64;
-  __shared__ uint4 rows0[kStageVectors], rows1[kStageVectors], rows2[kStageVectors], rows3[kStageVectors], sums[kSums ? (T + 3) / 4 * 4 * 64 : 1];
   const uint32_t lane = threadIdx.x & 63u, c = lane & 15u, kq = lane >> 4;
   const uint32_t tile0 = w.tile0, tilesHere = w.tilesHere, b0 = w.b0, count = w.count, split = w.split;
   const uint32_t column[2] = {w.column[0], w.column[1]};
@@ -450,7 +454,7 @@ __device__ __forceinline__ void wide_workgroup(const WideTile &w, const uint8_t 
   const uint32_t sumsAt = (threadIdx.x >> 6) * tileBytes + lane * 16u;
   auto stageRows = [&](auto stageConstant) __attribute__((always_inline)) -> uint4 * {
     constexpr uint32_t S = decltype(stageConstant)::value;
-    return S == 0 ? rows0 : S == 1 ? rows1 : S == 2 ? rows2 : rows3;
+    return S == 0 ? lds.rows0 : S == 1 ? lds.rows1 : S == 2 ? lds.rows2 : lds.rows3;
   };
   auto fetch = [&](uint32_t block, auto stageConstant) __attribute__((always_inline)) {   // block counts from b0
     constexpr uint32_t S = decltype(stageConstant)::value;
@@ -461,7 +465,7 @@ __device__ __forceinline__ void wide_workgroup(const WideTile &w, const uint8_t 
     for (uint32_t i = 0; i < kShare; ++i) load_to_lds(rowValues, mineAt + (at + 2u * i * tileBytes), to + 256u * i);
     if constexpr (S == 3u) {
 #pragma unroll
-      for (uint32_t i = 0; i < kSumShare; ++i) load_to_lds(rowValues, sumsAt + (at + 2048u + 4u * i * tileBytes), sums + 64u * wave + 256u * i);
+      for (uint32_t i = 0; i < kSumShare; ++i) load_to_lds(rowValues, sumsAt + (at + 2048u + 4u * i * tileBytes), lds.sums + 64u * wave + 256u * i);
     }
   };
   // A record's first half (and what both share) is fetched two stages ahead of its use, and so is its second.
@@ -533,7 +537,7 @@ __device__ __forceinline__ void wide_workgroup(const WideTile &w, const uint8_t 
       auto read = [&](uint32_t t) {
 #pragma unroll
         for (uint32_t g = 0; g < 2; ++g) a[t & 1u][g] = as_f16x8(rows[(t * 2u + g) * 64u + lane]);
-        if constexpr (kReads == 3u) a[t & 1u][2] = as_f16x8(sums[t * 64u + lane]);
+        if constexpr (kReads == 3u) a[t & 1u][2] = as_f16x8(lds.sums[t * 64u + lane]);
       };
       read(0);
 #pragma unroll
@@ -631,10 +635,16 @@ __global__ __launch_bounds__(256, 2) void gguf_wide(const uint8_t *__restrict__ 
   w.b0 = blocks * w.split / p.splits;
   w.count = blocks * (w.split + 1u) / p.splits - w.b0;
   wide_columns<FMT, EP == GGUF_WIDE_GATE_UP>(w, seg0, seg1, seg2, p, rest / p.splits, wave);
-  wide_workgroup<FMT, EP, T, Staged>(w, table, out, residual, p);
+  __shared__ uint4 rows0[kWideStageVectors<T>], rows1[kWideStageVectors<T>], rows2[kWideStageVectors<T>], rows3[kWideStageVectors<T>],
+      sums[kWideSumVectors<FMT, T, Staged>];
+  wide_workgroup<FMT, EP, T, Staged>(WideLds{rows0, rows1, rows2, rows3, sums}, w, table, out, residual, p);
 }
 // The routed experts of a prompt chunk: a task is up to T of an expert's row tiles (moe_chunk_place lists them), an item a
-// task's column group, the groups of a task side by side. Output rows are the slots'.
+// task's column group, the groups of a task side by side. Output rows are the slots'. A workgroup computes whole bodies of
+// row tiles, and a tile past the task's multiplies zeros: a kernel of tall tasks holds the bodies of its shorter ones and
+// takes the one that fits. A task's weights are converted once, whatever its height: 2048 rows of 128 experts, 8 a row,
+// 7 to 10 tiles an expert, in tasks of up to eight 164 and 130 us a layer's gate/up and down, in tasks of five that were
+// always computed as five 195 and 151.
 template <uint32_t FMT, uint32_t EP, uint32_t T>
 __global__ __launch_bounds__(256, 2) void gguf_wide_moe(const uint8_t *__restrict__ seg0, const uint8_t *__restrict__ seg1, const uint8_t *__restrict__ table,
                                                         void *__restrict__ out, const MoeChunkTask *__restrict__ tasks,
@@ -653,7 +663,18 @@ __global__ __launch_bounds__(256, 2) void gguf_wide_moe(const uint8_t *__restric
   w.count = p.input_size / GGUF_BLOCK;
   const uint64_t expertAt = task.expert * m.expert_bytes;
   wide_columns<FMT, EP == GGUF_WIDE_GATE_UP>(w, seg0 + expertAt, seg1 + expertAt, seg0 + expertAt, p, item % p.groups, wave);
-  wide_workgroup<FMT, EP, T, false>(w, table, out, nullptr, p);
+  __shared__ uint4 rows0[kWideStageVectors<T>], rows1[kWideStageVectors<T>], rows2[kWideStageVectors<T>], rows3[kWideStageVectors<T>],
+      sums[kWideSumVectors<FMT, T, false>];
+  const WideLds lds{rows0, rows1, rows2, rows3, sums};
+  if constexpr (T > 4u) {
+    if (w.tilesHere <= 4u) return wide_workgroup<FMT, EP, 4, false>(lds, w, table, out, nullptr, p);
+  }
+  if constexpr (T == 8u) {
+    if (w.tilesHere == 5u) return wide_workgroup<FMT, EP, 5, false>(lds, w, table, out, nullptr, p);
+    if (w.tilesHere == 6u) return wide_workgroup<FMT, EP, 6, false>(lds, w, table, out, nullptr, p);
+    if (w.tilesHere == 7u) return wide_workgroup<FMT, EP, 7, false>(lds, w, table, out, nullptr, p);
+  }
+  wide_workgroup<FMT, EP, T, false>(lds, w, table, out, nullptr, p);
 }
 #define SP_GGUF_WIDE_T(fmt, FMT, T)                                                          \
   SP_REGISTER_KERNEL("gguf_wide_" fmt "_t" #T "_a", (&gguf_wide<FMT, GGUF_WIDE_PLAIN, T>));        \
@@ -684,12 +705,15 @@ SP_GGUF_WIDE("q6k", GGUF_FMT_Q6K);
 SP_GGUF_WIDE_MOE("q4k", GGUF_FMT_Q4K, 2);
 SP_GGUF_WIDE_MOE("q4k", GGUF_FMT_Q4K, 4);
 SP_GGUF_WIDE_MOE("q4k", GGUF_FMT_Q4K, 5);
+SP_GGUF_WIDE_MOE("q4k", GGUF_FMT_Q4K, 8);
 SP_GGUF_WIDE_MOE("q5k", GGUF_FMT_Q5K, 2);
 SP_GGUF_WIDE_MOE("q5k", GGUF_FMT_Q5K, 4);
 SP_GGUF_WIDE_MOE("q5k", GGUF_FMT_Q5K, 5);
+SP_GGUF_WIDE_MOE("q5k", GGUF_FMT_Q5K, 8);
 SP_GGUF_WIDE_MOE("q6k", GGUF_FMT_Q6K, 2);
 SP_GGUF_WIDE_MOE("q6k", GGUF_FMT_Q6K, 4);
 SP_GGUF_WIDE_MOE("q6k", GGUF_FMT_Q6K, 5);
+SP_GGUF_WIDE_MOE("q6k", GGUF_FMT_Q6K, 8);
 
 template <bool Residual, bool Float = false>
 __global__ __launch_bounds__(256) void gguf_wide_reduce(const float4 *__restrict__ partials, void *__restrict__ out,

@@ -136,13 +136,11 @@ void MoE::addRouted(hip::CommandGraph &graph, const hip::Buffer &normalized, con
 
 namespace {
 bool wideFormat(uint32_t format) { return format == GGUF_FMT_Q4K || format == GGUF_FMT_Q5K || format == GGUF_FMT_Q6K; }
-// The row tiles of a task: what an expert's share of the routes comes to, and a tile more, in as few tasks as hold it.
-// (The kernels compute all of a task's tiles, live or not.)
+// The most row tiles of a task: what an expert's share of the routes comes to, and a tile more, in one task as far as the
+// kernels' tallest holds it (its weights are converted once a task).
 uint32_t taskTiles(uint32_t routes, uint32_t experts) {
   const uint32_t expected = (routes + experts * MOE_TILE_ROWS - 1) / (experts * MOE_TILE_ROWS) + 1;
-  if (expected <= 2) return 2;
-  const uint32_t parts = (expected + 4) / 5;
-  return (expected + parts - 1) / parts <= 4 ? 4 : 5;
+  return expected <= 2 ? 2 : expected <= 4 ? 4 : expected <= 5 ? 5 : 8;
 }
 } // namespace
 

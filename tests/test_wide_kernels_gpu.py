@@ -313,6 +313,12 @@ def test_expert_tiles_lie_in_the_interval(backend, name, T):
                     assert np.all(np.abs(g - w) <= 2.0 ** -6 * np.abs(w) + 1e-6) and (got[at] != expected).mean() < 0.03
 
 
+@pytest.mark.parametrize("name", list(FORMATS))
+def test_expert_tiles_of_tall_tasks_lie_in_the_interval(backend, name):
+    """The same of tasks of up to eight row tiles, whose kernels hold a body for each height of four and more."""
+    test_expert_tiles_lie_in_the_interval(backend, name, 8)
+
+
 @pytest.mark.parametrize("geometry,tokens,committed,gated", [((64, 8, 128), 200, 300, False), ((64, 8, 128), 53, 0, True), ((32, 8, 128), 200, 250, True),
                                                              ((32, 8, 128), 64, 1000, False), ((16, 8, 64), 200, 300, False), ((16, 8, 64), 37, 700, True)])
 def test_a_chunks_blocks_attend_whole_histories(backend, geometry, tokens, committed, gated):
