@@ -237,7 +237,10 @@ struct GgufWideParams {
   uint32_t groups;      // column groups of GGUF_WIDE_COLUMNS over the segments
   uint32_t cols[3];     // columns per segment: multiples of 16; each segment starts a column group of its own
   uint32_t offset[3];   // first destination column per segment
-  uint32_t reserved[3];
+  // The last tail_groups column groups' rows dealt over tail_row_groups workgroups of up to four row tiles each (splits 1;
+  // not the kernels of four), whose items are a second part of the grid: 8 * ceil(tail_row_groups * tail_groups / 8) more.
+  uint32_t tail_groups, tail_row_groups;
+  uint32_t reserved;
 };
 // gguf_wide_moe_<fmt>_t<T>_{a,g}: the routed experts of a chunk (abi/Moe.h, MoeChunkTask): wide.rows, .row_groups and
 // .splits are unused. Binds the experts' images (gate and up, or down twice), the slots' wide table, the slots' output rows,

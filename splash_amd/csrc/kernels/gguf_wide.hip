@@ -622,22 +622,28 @@ template <uint32_t FMT, uint32_t EP, uint32_t T, bool Staged = false>
 __global__ __launch_bounds__(256, 2) void gguf_wide(const uint8_t *__restrict__ seg0, const uint8_t *__restrict__ seg1, const uint8_t *__restrict__ seg2,
                                                     const uint8_t *__restrict__ table, void *__restrict__ out, const uint16_t *__restrict__ residual,
                                                     GgufWideParams p) {
-  const uint32_t perDie = gridDim.x / 8u, item = (blockIdx.x % 8u) * perDie + blockIdx.x / 8u;
-  if (item >= p.row_groups * p.splits * p.groups) return;
-  const uint32_t rowGroup = item % p.row_groups, rest = item / p.row_groups;
+  // The last p.tail_groups column groups are a second part of the grid, in workgroups of four row tiles.
+  const uint32_t tallGroups = p.groups - p.tail_groups, tallItems = p.row_groups * p.splits * tallGroups, tallBlocks = (tallItems + 7u) / 8u * 8u;
+  const bool tail = T > 4u && blockIdx.x >= tallBlocks;
+  const uint32_t block = tail ? blockIdx.x - tallBlocks : blockIdx.x, blocksHere = tail ? gridDim.x - tallBlocks : tallBlocks;
+  const uint32_t item = (block % 8u) * (blocksHere / 8u) + block / 8u, rowGroups = tail ? p.tail_row_groups : p.row_groups;
+  if (item >= (tail ? p.tail_row_groups * p.tail_groups : tallItems)) return;
+  const uint32_t rowGroup = item % rowGroups, rest = item / rowGroups;
   const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)));
   const uint32_t blocks = p.input_size / GGUF_BLOCK, liveTiles = (p.rows + 15u) / 16u;
   WideTile w;
-  w.split = rest % p.splits;
-  w.tile0 = liveTiles * rowGroup / p.row_groups;
-  w.tilesHere = liveTiles * (rowGroup + 1u) / p.row_groups - w.tile0;
+  w.split = tail ? 0u : rest % p.splits;
+  w.tile0 = liveTiles * rowGroup / rowGroups;
+  w.tilesHere = liveTiles * (rowGroup + 1u) / rowGroups - w.tile0;
   w.rows = p.rows;
   w.b0 = blocks * w.split / p.splits;
   w.count = blocks * (w.split + 1u) / p.splits - w.b0;
-  wide_columns<FMT, EP == GGUF_WIDE_GATE_UP>(w, seg0, seg1, seg2, p, rest / p.splits, wave);
+  wide_columns<FMT, EP == GGUF_WIDE_GATE_UP>(w, seg0, seg1, seg2, p, tail ? tallGroups + rest : rest / p.splits, wave);
   __shared__ uint4 rows0[kWideStageVectors<T>], rows1[kWideStageVectors<T>], rows2[kWideStageVectors<T>], rows3[kWideStageVectors<T>],
       sums[kWideSumVectors<FMT, T, Staged>];
-  wide_workgroup<FMT, EP, T, Staged>(WideLds{rows0, rows1, rows2, rows3, sums}, w, table, out, residual, p);
+  const WideLds lds{rows0, rows1, rows2, rows3, sums};
+  if (tail) wide_workgroup<FMT, EP, 4, Staged>(lds, w, table, out, residual, p);
+  else wide_workgroup<FMT, EP, T, Staged>(lds, w, table, out, residual, p);
 }
 // The routed experts of a prompt chunk: a task is up to T of an expert's row tiles (moe_chunk_place lists them), an item a
 // task's column group, the groups of a task side by side. Output rows are the slots'. A workgroup computes whole bodies of

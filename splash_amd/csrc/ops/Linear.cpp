@@ -503,10 +503,11 @@ uint64_t Linear::wideTableBytes(uint32_t inputSize, uint32_t rows) noexcept { re
 // fill the device's rounds best, in microseconds. A compute unit holds two workgroups, so `items` workgroups take
 // ceil(items / (2 units)) rounds of 1 / splits of K each; a super-block of a round takes 0.55 for each row tile and for the
 // conversion of its weights as much as 2.2 of them (5.6 measured at eight tiles); parts cost a launch and their partials'
-// trip to memory and back.
+// trip to memory and back. Where a last round would be far from full, the column groups past the full rounds go in
+// workgroups of four row tiles instead, a second part of the grid that starts as the first one's last workgroups end.
 Linear::WideSplit Linear::wideSplit(uint32_t columnGroups, uint32_t blocks, uint32_t rows, bool splittable) const noexcept {
   const uint32_t liveTiles = gguf_row_tiles(rows), slots = 2 * calibration_.computeUnits;
-  WideSplit chosen{1, GGUF_WIDE_TILES, 1};
+  WideSplit chosen{1, GGUF_WIDE_TILES, 1, 0, 0};
   double best = 0;
   for (uint32_t tallest : {8u, 7u, 6u, 4u}) {
     const uint32_t rowGroups = (liveTiles + tallest - 1) / tallest, items = rowGroups * columnGroups;
@@ -515,8 +516,21 @@ Linear::WideSplit Linear::wideSplit(uint32_t columnGroups, uint32_t blocks, uint
                           (s > 1 ? 5.0 + double(s) * rows * columnGroups * GGUF_WIDE_COLUMNS * 8 / 4.5e6 : 0.0);
       if (!best || cost < best) {
         best = cost;
-        chosen = {rowGroups, tallest, s};
+        chosen = {rowGroups, tallest, s, 0, 0};
       }
+    }
+  }
+  for (uint32_t tallest : {8u, 7u, 6u}) {
+    const uint32_t rowGroups = (liveTiles + tallest - 1) / tallest, full = rowGroups * columnGroups / slots;
+    const uint32_t tail = full ? columnGroups - full * slots / rowGroups : 0;
+    if (!tail) continue;
+    // (a round of one workgroup a compute unit is two thirds as long as one of two)
+    const uint32_t tailRowGroups = (liveTiles + 3) / 4, tailItems = tailRowGroups * tail;
+    const double tailRounds = tailItems <= calibration_.computeUnits ? 0.67 : double((tailItems + slots - 1) / slots);
+    const double cost = (full * (2.2 + tallest) + tailRounds * (2.2 + 4)) * blocks * 0.55;
+    if (cost < 0.999 * best) {
+      best = cost;
+      chosen = {rowGroups, tallest, 1, tail, tailRowGroups};
     }
   }
   return chosen;
@@ -559,7 +573,8 @@ void Linear::addWideNormTable(hip::CommandGraph &graph, const hip::Buffer &input
 }
 
 namespace {
-GgufWideParams wideParams(uint32_t k, uint32_t rows, uint32_t outStride, uint32_t groups, uint32_t rowGroups, uint32_t splits) {
+GgufWideParams wideParams(uint32_t k, uint32_t rows, uint32_t outStride, uint32_t groups, uint32_t rowGroups, uint32_t splits, uint32_t tailGroups,
+                          uint32_t tailRowGroups) {
   GgufWideParams params{};
   params.input_size = k;
   params.rows = rows;
@@ -568,9 +583,13 @@ GgufWideParams wideParams(uint32_t k, uint32_t rows, uint32_t outStride, uint32_
   params.splits = splits;
   params.out_stride = outStride;
   params.groups = groups;
+  params.tail_groups = tailGroups;
+  params.tail_row_groups = tailRowGroups;
   return params;
 }
-uint32_t wideGrid(const GgufWideParams &p) { return 8 * ((p.row_groups * p.splits * p.groups + 7) / 8); }
+uint32_t wideGrid(const GgufWideParams &p) {
+  return 8 * ((p.row_groups * p.splits * (p.groups - p.tail_groups) + 7) / 8) + 8 * ((p.tail_row_groups * p.tail_groups + 7) / 8);
+}
 std::string wideName(const char *format, bool staged, uint32_t tiles, const char *suffix) {
   return std::string(staged ? "gguf_wide_staged_" : "gguf_wide_") + format + "_t" + std::to_string(staged ? GGUF_WIDE_TILES : tiles) + suffix;
 }
@@ -594,7 +613,7 @@ void Linear::addWide(hip::CommandGraph &graph, const Projection &p, const hip::B
   // (unsplit fp32 rows are the partials of one part)
   const WideSplit split = wideSplit(groups, k / GGUF_BLOCK, rows, bool(partials) && n % 4 == 0);
   if (split.splits > 1) requireBytes(partials, uint64_t{split.splits} * rows * n * 4, "projection partials");
-  GgufWideParams params = wideParams(k, rows, n, groups, split.rowGroups, split.splits);
+  GgufWideParams params = wideParams(k, rows, n, groups, split.rowGroups, split.splits, split.tailGroups, split.tailRowGroups);
   hip::Buffer images[3];
   for (size_t s = 0; s < 3; ++s) {
     const QuantizedSegment &segment = segments[std::min(s, segments.size() - 1)];
@@ -630,7 +649,7 @@ void Linear::addWideGateUp(hip::CommandGraph &graph, const Projection &gate, con
   requireBytes(output, uint64_t{rows} * n * 2, "projection output");
   const uint32_t groups = (n + GGUF_WIDE_COLUMNS / 2 - 1) / (GGUF_WIDE_COLUMNS / 2);
   const WideSplit split = wideSplit(groups, k / GGUF_BLOCK, rows, false);
-  GgufWideParams params = wideParams(k, rows, n, groups, split.rowGroups, 1);
+  GgufWideParams params = wideParams(k, rows, n, groups, split.rowGroups, 1, split.tailGroups, split.tailRowGroups);
   params.cols[0] = n;
   const hip::Buffer &first = gate.blocks().segments.front().image, &second = up.blocks().segments.front().image;
   graph.add(wideName(up.blocks().segments.front().name(), staged, split.tiles, "_g"), {first, second, second, table, output, table}, params,

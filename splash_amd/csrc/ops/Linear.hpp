@@ -262,7 +262,7 @@ public:
 
 private:
   struct Resolved;
-  struct WideSplit { uint32_t rowGroups, tiles, splits; };
+  struct WideSplit { uint32_t rowGroups, tiles, splits, tailGroups, tailRowGroups; };
   [[nodiscard]] WideSplit wideSplit(uint32_t columnGroups, uint32_t blocks, uint32_t rows, bool splittable) const noexcept;
   PreparedInput addColumn(hip::CommandGraph &graph, LinearBuffers buffers, const Projection &projection, const LinearPlan &plan,
                           const Projection *gate) const;

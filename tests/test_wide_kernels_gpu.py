@@ -189,6 +189,44 @@ def test_every_tile_height_lies_in_the_interval(backend, name, T):
                 assert np.all(np.abs(g - w) <= 2.0 ** -7 * np.abs(w) + 1e-38) and (got != expected).mean() < 0.03      # (exp2's last bit)
 
 
+@pytest.mark.parametrize("T", [6, 7, 8])
+@pytest.mark.parametrize("name", ["q4k", "q6k", "staged_q4k"])
+def test_tail_columns_in_shorter_workgroups_change_nothing(backend, name, T):
+    """The last column groups in workgroups of four row tiles, one group to all but one of them, tensors that end inside a
+    group, rows that leave the last workgroup short: every epilogue's bits are those of the same columns in tall ones."""
+    fmt, K, cols = FORMATS[name[-3:]], 768, [144, 128, 16]
+    if name.startswith("staged"):
+        if T < 8:
+            pytest.skip("the staged rule has the tallest tile alone")
+        cols = [256, 128, 128]
+    print(f"case wide tail {name} T={T}", flush=True)
+    rng = np.random.default_rng(T)
+    N = sum(cols)
+    images = [backend.from_array(ops.pack_gguf_image(fmt, orc.make_native(fmt, n, K, 10 * T + n), n, K)) for n in cols]
+    for rows in (5, 16 * (2 * T - 1) - 5):
+        residual = backend.from_array(orc.f32_to_bf16(rng.standard_normal((rows, N)).astype(np.float32)))
+        graph = splash_amd.CommandGraph()
+        table = add_table(graph, backend, rows_of(rng, rows, K))
+        backend.run(graph)
+        tiles = (rows + 15) // 16
+        for kind, size, widths, columns in (("p", 4, cols, 128), ("a", 2, cols, 128), ("r", 2, cols, 128), ("g", 2, cols[1:2], 64)):
+            weights = images if kind != "g" else [images[1], images[1]]
+            groups, span, got = sum(-(-n // columns) for n in widths), sum(widths), []
+            for tail in (0, 1, groups - 1):
+                p = WideParams(K, rows, wide_tiles(rows), -(-tiles // T), 1, span, groups)
+                for s, n in enumerate(widths):
+                    p.cols[s], p.offset[s] = n, sum(widths[:s])
+                p.reserved[0], p.reserved[1] = tail, -(-tiles // 4)
+                out = backend.allocate_buffer(rows * span * size)
+                out.fill(0xFF)
+                graph = splash_amd.CommandGraph()
+                blocks = 8 * -(-p.row_groups * (groups - tail) // 8) + 8 * -(-p.reserved[1] * tail // 8)
+                graph.add(f"gguf_wide_{name}_t{T}_{kind}", (weights + weights[-1:] * 2)[:3] + [table, out, residual], p, (blocks, 1, 1))
+                backend.run(graph)
+                got.append(out.download(np.uint8).tobytes())
+            assert got[1] == got[0] and got[2] == got[0], (kind, rows)
+
+
 @pytest.mark.parametrize("name", list(FORMATS))
 def test_a_staged_projection_lies_in_the_staged_interval(backend, name):
     """The staged rule's tile, K whole and in parts."""
