@@ -292,9 +292,20 @@ __global__ __launch_bounds__(256) void moe_combine(const uint16_t *__restrict__ 
   uint32_t bits = 0;
   if (live) {
     float value = bf16_bits_to_float(residual[size_t(row) * p.hidden + d]);
-    for (uint32_t rank = 0; rank < p.top_k; ++rank) {
-      const size_t route = size_t(row) * p.top_k + rank;
-      value += weights[route] * bf16_bits_to_float(expert_output[size_t(route_slot[route]) * p.hidden + d]);
+    // (eight routes' outputs are on their way together; one past the last reads the last and adds nothing)
+    constexpr uint32_t kAhead = 8;
+    for (uint32_t first = 0; first < p.top_k; first += kAhead) {
+      float weight[kAhead];
+      uint32_t y[kAhead];
+#pragma unroll
+      for (uint32_t i = 0; i < kAhead; ++i) {
+        const size_t route = size_t(row) * p.top_k + min(first + i, p.top_k - 1u);
+        weight[i] = weights[route];
+        y[i] = expert_output[size_t(route_slot[route]) * p.hidden + d];
+      }
+#pragma unroll
+      for (uint32_t i = 0; i < kAhead; ++i)
+        if (first + i < p.top_k) value += weight[i] * bf16_bits_to_float(y[i]);
     }
     bits = float_to_bf16_bits(value);
     output[size_t(row) * p.hidden + d] = uint16_t(bits);
