@@ -7,8 +7,8 @@
 #define SPLASH_RMS_EPSILON 1e-6f
 #define NORM_STAGED_WIDTH 8192u  // columns of a row that a norm holds in LDS
 
-// norm_rms / norm_rms_table16: one workgroup of 256 threads per row. norm_rms_table16 also writes
-// the projection activation table of the normalized rows (abi/Gguf.h), as the reference's
+// norm_rms / norm_rms_table16: one workgroup per row, of 256 threads / of norm_row_threads(width). norm_rms_table16 also
+// writes the projection activation table of the normalized rows (abi/Gguf.h), as the reference's
 // norm_rms_table16_decode does for its register tile.
 struct NormParams {
   uint32_t width;
@@ -16,6 +16,14 @@ struct NormParams {
   uint32_t tiles;  // row tiles of the table (norm_rms_table16)
   uint32_t reserved;
 };
+#if defined(__cplusplus)
+// Threads of a workgroup that norms a row of whole super-blocks and writes its part of a table: one a vector of eight
+// columns where the row is held in LDS, and the 256 that sum its squares at least.
+inline uint32_t norm_row_threads(uint32_t width) {
+  const uint32_t vectors = width / 8u;
+  return width > NORM_STAGED_WIDTH || vectors <= 256u ? 256u : (vectors + 63u) / 64u * 64u;
+}
+#endif
 
 // rope_build_tree_tables: cos and sin of (anchor[sequence] + depth[row]) * inverse_frequency[pair]
 // per packed row (the reference's RopeTreeParams, abi/RoPE.h). Grid (rows), `pairs` threads.

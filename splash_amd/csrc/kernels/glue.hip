@@ -21,9 +21,8 @@ __device__ __forceinline__ void arrived(uint4 &v) { asm volatile("" : "+v"(v.x),
 __device__ __forceinline__ void arrived(uint32_t &v) { asm volatile("" : "+v"(v)); }
 
 // `width` bf16 values (a multiple of 8, 16-byte aligned) on their way to LDS: every load of it goes out before any is stored,
-// and those of several rows before the first row's stores. No barrier. (The norm and its table: 8.7 us at 8 rows of 5120 and
-// 6.4 at 128 of 2048 where each load was waited for; 7.9 and 5.8 with the loads unconditional but sunk to their stores; 6.6
-// and 5.8 so.)
+// and those of several rows before the first row's stores. No barrier. (A norm of 8 rows of 5120: 8.7 us where each load was
+// waited for, 7.9 with the loads unconditional but sunk to their stores, 6.6 so.)
 struct StagedRow {
   static constexpr uint32_t kHeld = kStagedWidth / 8u / 256u;
   uint4 held[kHeld];
@@ -43,22 +42,25 @@ struct StagedRow {
   }
 };
 
-// The row's inverse RMS: 256 threads sum the squares of columns tid, tid + 256, ... in column
+// The row's inverse RMS: a workgroup's first 256 threads sum the squares of columns tid, tid + 256, ... in column
 // order; a wavefront sums its lanes by butterfly, the four wavefronts' sums are added in order
-// (normalization.metal:59-99 and common/rms_inverse.h:15-33, on 64-lane wavefronts).
+// (normalization.metal:59-99 and common/rms_inverse.h:15-33, on 64-lane wavefronts). The order is the same whatever the
+// workgroup's size is.
 __device__ __forceinline__ float rms_inverse(const uint16_t *row, uint32_t width, float *scratch) {
   // (ten reads at a time: a column past the row adds a zero)
   constexpr uint32_t kAhead = 10;
-  float sum = 0.f;
-  for (uint32_t first = threadIdx.x; first < width; first += 256u * kAhead) {
-    float v[kAhead];
+  if (threadIdx.x < 256u) {
+    float sum = 0.f;
+    for (uint32_t first = threadIdx.x; first < width; first += 256u * kAhead) {
+      float v[kAhead];
 #pragma unroll
-    for (uint32_t j = 0; j < kAhead; ++j) v[j] = bf16_bits_to_float(row[min(first + 256u * j, width - 1u)]);
+      for (uint32_t j = 0; j < kAhead; ++j) v[j] = bf16_bits_to_float(row[min(first + 256u * j, width - 1u)]);
 #pragma unroll
-    for (uint32_t j = 0; j < kAhead; ++j) sum += first + 256u * j < width ? v[j] * v[j] : 0.f;
+      for (uint32_t j = 0; j < kAhead; ++j) sum += first + 256u * j < width ? v[j] * v[j] : 0.f;
+    }
+    sum = wave_sum(sum);
+    if ((threadIdx.x & 63u) == 0) scratch[threadIdx.x >> 6] = sum;
   }
-  sum = wave_sum(sum);
-  if ((threadIdx.x & 63u) == 0) scratch[threadIdx.x >> 6] = sum;
   __syncthreads();
   const float total = ((scratch[0] + scratch[1]) + scratch[2]) + scratch[3];
   return 1.0f / sqrtf(total / float(width) + SPLASH_RMS_EPSILON);
@@ -86,11 +88,10 @@ __global__ __launch_bounds__(256) void norm_rms(const uint16_t *__restrict__ inp
 }
 SP_REGISTER_KERNEL("norm_rms", &norm_rms);
 
-// A row's part of an activation table, and (Normed) the normalized row it describes: 256 threads, each the runs of four
-// inputs q = t, t + 256, ... (4 kq .. 4 kq + 3 of a group's half, one 8-byte piece of a table entry), kRuns of them in
-// flight together. A row past the live ones is zeros. The width is a multiple of 256, so a wavefront's runs are all inside
-// the row or all past it.
-template <bool Normed>
+// A row's part of an activation table, and the normalized row it describes, of rows wider than kStagedWidth: 256 threads,
+// each the runs of four inputs q = t, t + 256, ... (4 kq .. 4 kq + 3 of a group's half, one 8-byte piece of a table entry),
+// kRuns of them in flight together. A row past the live ones is zeros. The width is a multiple of 256, so a wavefront's runs
+// are all inside the row or all past it.
 __device__ __forceinline__ void write_table_row(const uint16_t *x, const uint16_t *w, float inverse, bool live, uint32_t row,
                                                 uint16_t *__restrict__ output, uint8_t *__restrict__ table, uint32_t width, uint32_t allTiles) {
   constexpr uint32_t kRuns = 5;
@@ -111,15 +112,14 @@ __device__ __forceinline__ void write_table_row(const uint16_t *x, const uint16_
       uint2 xs = make_uint2(0u, 0u), ws = xs;
       if (live) {
         xs = *reinterpret_cast<const uint2 *>(x + 4u * q);
-        if constexpr (Normed) ws = *reinterpret_cast<const uint2 *>(w + 4u * q);
+        ws = *reinterpret_cast<const uint2 *>(w + 4u * q);
       }
       const uint32_t xb[4] = {xs.x & 0xFFFFu, xs.x >> 16, xs.y & 0xFFFFu, xs.y >> 16};
       const uint32_t wb[4] = {ws.x & 0xFFFFu, ws.x >> 16, ws.y & 0xFFFFu, ws.y >> 16};
       float v[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        bits[j][i] = xb[i];
-        if constexpr (Normed) bits[j][i] = live ? float_to_bf16_bits((bf16_bits_to_float(xb[i]) * inverse) * bf16_bits_to_float(wb[i])) : 0u;
+        bits[j][i] = live ? float_to_bf16_bits((bf16_bits_to_float(xb[i]) * inverse) * bf16_bits_to_float(wb[i])) : 0u;
         v[i] = bf16_bits_to_float(bits[j][i]);
       }
       sum[j] = (v[0] + v[1]) + (v[2] + v[3]);
@@ -132,10 +132,9 @@ __device__ __forceinline__ void write_table_row(const uint16_t *x, const uint16_
       const float s = ((sum[j] + s1) + s2) + s3;   // of 16 inputs, in input order
       const float other = lane_down<4>(s);
       if (q >= runs) continue;
-      if constexpr (Normed)
-        if (live)
-          *reinterpret_cast<uint2 *>(output + size_t(row) * width + 4u * q) =
-              make_uint2(bits[j][0] | (bits[j][1] << 16), bits[j][2] | (bits[j][3] << 16));
+      if (live)
+        *reinterpret_cast<uint2 *>(output + size_t(row) * width + 4u * q) =
+            make_uint2(bits[j][0] | (bits[j][1] << 16), bits[j][2] | (bits[j][3] << 16));
       const uint32_t g = q / 8u, half = (q / 4u) % 2u, kq = q % 4u;
       // operand elements 4 half + {0,1,2,3} are inputs 4 kq + {0,2,1,3} of the half
       values[((size_t(tile) * G + g) * 64u + kq * 16u + r) * 2u + half] =
@@ -148,114 +147,145 @@ __device__ __forceinline__ void write_table_row(const uint16_t *x, const uint16_
   }
 }
 
-// The same, and the activation table of the normalized rows: grid (tiles * 16) so that the rows
-// past the live ones are written as zeros. A handful of workgroups that only wait: every loop keeps several reads in
-// flight (what that gives: at StagedRow).
-__global__ __launch_bounds__(256) void norm_rms_table16(const uint16_t *__restrict__ input, const uint16_t *__restrict__ weight,
-                                                        uint16_t *__restrict__ output, uint8_t *__restrict__ table, NormParams p) {
+// Eight inputs 8 v .. 8 v + 7 of a row, a thread of its own for each v: their two pieces of the row's activation table and
+// their parts of its sums, the values and the order of additions of write_table_row. Lanes 4 l .. 4 l + 3 hold consecutive v
+// of one group of 32 inputs.
+__device__ __forceinline__ void write_table_vector(uint4 bits, uint32_t row, uint32_t v, uint8_t *__restrict__ table, uint32_t width, uint32_t allTiles) {
+  const uint32_t r = row % 16u, G = width / 32u;
+  const uint32_t piece = row / 16u / GGUF_PIECE_TILES, tile = row / 16u % GGUF_PIECE_TILES;
+  const uint32_t tiles = min(uint32_t(GGUF_PIECE_TILES), allTiles - piece * GGUF_PIECE_TILES);
+  table += piece * gguf_table_bytes(width, GGUF_PIECE_TILES);
+  uint2 *values = reinterpret_cast<uint2 *>(table);
+  const uint32_t g = v / 4u, half = (v / 2u) % 2u, kq = 2u * (v % 2u);
+  auto four = [](uint32_t low, uint32_t high) {
+    return (bf16_bits_to_float(low & 0xFFFFu) + bf16_bits_to_float(low >> 16)) + (bf16_bits_to_float(high & 0xFFFFu) + bf16_bits_to_float(high >> 16));
+  };
+  const float a = four(bits.x, bits.y), b = four(bits.z, bits.w), a1 = lane_down<1>(a), b1 = lane_down<1>(b);
+  const float s = ((a + b) + a1) + b1;   // of 16 inputs, in input order
+  const float other = lane_down<2>(s);
+  // operand elements 4 half + {0,1,2,3} are inputs 4 kq + {0,2,1,3} of the half
+  auto operand = [](uint32_t low, uint32_t high) { return make_uint2((low & 0xFFFFu) | (high << 16), (low >> 16) | (high & 0xFFFF0000u)); };
+  uint2 *at = values + ((size_t(tile) * G + g) * 64u + kq * 16u + r) * 2u + half;
+  at[0] = operand(bits.x, bits.y);
+  at[32] = operand(bits.z, bits.w);
+  if (kq == 0) {
+    float *sums32 = reinterpret_cast<float *>(table + gguf_table_sums32_offset(width, tiles));
+    float *sums16 = reinterpret_cast<float *>(table + gguf_table_sums16_offset(width, tiles));
+    sums16[(size_t(tile) * 2u * G + 2u * g + half) * 16u + r] = s;
+    if (half == 0) sums32[(size_t(tile) * G + g) * 16u + r] = s + other;
+  }
+}
+
+// Eight values of a normalized row.
+__device__ __forceinline__ uint4 norm_vector(uint4 x, uint4 w, float inverse) {
+  auto two = [&](uint32_t xs, uint32_t ws) {
+    const uint32_t low = float_to_bf16_bits((bf16_bits_to_float(xs & 0xFFFFu) * inverse) * bf16_bits_to_float(ws & 0xFFFFu));
+    return low | (float_to_bf16_bits((bf16_bits_to_float(xs >> 16) * inverse) * bf16_bits_to_float(ws >> 16)) << 16);
+  };
+  return make_uint4(two(x.x, w.x), two(x.y, w.y), two(x.z, w.z), two(x.w, w.w));
+}
+// Eight values of a normalized row and their part of the table; zeros in the table for a row past the live ones. (Eight bytes
+// a store: all that the rows' buffers promise.)
+__device__ __forceinline__ void write_norm_vector(uint4 x, uint4 w, float inverse, bool live, uint32_t row, uint32_t v, uint16_t *__restrict__ output,
+                                                  uint8_t *__restrict__ table, uint32_t width, uint32_t tiles) {
+  uint4 bits = make_uint4(0u, 0u, 0u, 0u);
+  if (live) {
+    bits = norm_vector(x, w, inverse);
+    uint2 *to = reinterpret_cast<uint2 *>(output + size_t(row) * width + 8u * v);
+    to[0] = make_uint2(bits.x, bits.y);
+    to[1] = make_uint2(bits.z, bits.w);
+  }
+  write_table_vector(bits, row, v, table, width, tiles);
+}
+
+// The same, and the activation table of the normalized rows: grid (tiles * 16) so that the rows past the live ones are
+// written as zeros, norm_row_threads(width) threads. A handful of workgroups that only wait, so what counts is the chain one
+// thread runs: a row of up to kStagedWidth columns has a thread a vector of eight, which holds it and its weights in
+// registers from the load to the stores, and LDS serves the sum alone. (8 rows of 5120: 7.4 us by 256 threads, 4.3 so; 128 of
+// 2048: 6.0 and 5.6.)
+__global__ __launch_bounds__(1024) void norm_rms_table16(const uint16_t *__restrict__ input, const uint16_t *__restrict__ weight,
+                                                         uint16_t *__restrict__ output, uint8_t *__restrict__ table, NormParams p) {
   __shared__ float scratch[4];
-  __shared__ __align__(16) uint16_t rowX[kStagedWidth], rowW[kStagedWidth];
+  __shared__ __align__(16) uint16_t rowX[kStagedWidth];
   const uint32_t row = blockIdx.x;
   const bool live = row < p.rows;
   const uint16_t *x = input + size_t(live ? row : 0) * p.width;
   if (p.width <= kStagedWidth) {  // the width is a multiple of 256
-    if (live) {
-      StagedRow stagedX, stagedW;
-      stagedX.load(x, p.width);
-      stagedW.load(weight, p.width);
-      stagedX.store(p.width, rowX);
-      stagedW.store(p.width, rowW);
+    const uint32_t v = threadIdx.x;
+    uint4 mine = make_uint4(0u, 0u, 0u, 0u), norm = mine;
+    if (live && v < p.width / 8u) {
+      mine = reinterpret_cast<const uint4 *>(x)[v];
+      norm = reinterpret_cast<const uint4 *>(weight)[v];
+      reinterpret_cast<uint4 *>(rowX)[v] = mine;
     }
     __syncthreads();
     const float inverse = live ? rms_inverse(rowX, p.width, scratch) : 0.f;
-    write_table_row<true>(rowX, rowW, inverse, live, row, output, table, p.width, p.tiles);
+    if (v < p.width / 8u) write_norm_vector(mine, norm, inverse, live, row, v, output, table, p.width, p.tiles);
   } else {
     const float inverse = live ? rms_inverse(x, p.width, scratch) : 0.f;
-    write_table_row<true>(x, weight, inverse, live, row, output, table, p.width, p.tiles);
+    write_table_row(x, weight, inverse, live, row, output, table, p.width, p.tiles);
   }
 }
 SP_REGISTER_KERNEL("norm_rms_table16", &norm_rms_table16);
 
-// draft_conv (draft_attention.hip) and the pass that reads its rows, one workgroup a row: a Prepare stage's rows and their
-// activation table; a Residual stage's rows, their RMS norm (of `norm_weight`, into `normalized`) and its table. Each
-// convolution was a launch of its own before a launch of as few workgroups. Values and their order are the two kernels'.
-// The rows' 16-byte accesses are the host's rule (DraftAttention::addConvolutionTable). 8 rows of 5120, inside a draft
-// model's pass: 5.2 us for 3.1 + 3.0 and 7.5 for 3.1 + 6.6 (the norm's passes as they are now; 8.9 for 3.1 + 8.7 before
-// StagedRow's loads went out together), and a launch less each. The pass of one lane when it was fused: 928, 923 and 938 us
-// before, 869, 888 and 889 after, in three runs of both sides in turn whose repeats differ by 1 to 2 %.
+// draft_conv (draft_attention.hip) and the pass that reads its rows, a thread a vector of eight channels: a Prepare stage's
+// rows and their activation table, grid (tiles * 16, the row's vectors by 64), 64 threads, since nothing there needs the
+// row's other channels; a Residual stage's rows, their RMS norm (of `norm_weight`, into `normalized`) and its table, a
+// workgroup of norm_row_threads(width) a row. Each convolution was a launch of its own before a launch of as few workgroups.
+// 8 rows of 5120, inside a draft model's pass: 3.1 us (a workgroup of 256 a row, 5.3) and 4.7 (8.3).
+// Values and their order are the two kernels'. The rows' 16-byte accesses are the host's rule
+// (DraftAttention::addConvolutionTable).
 template <bool Residual>
-__global__ __launch_bounds__(256) void draft_conv_table(const uint16_t *__restrict__ input, const uint16_t *__restrict__ dynamic,
-                                                        const uint16_t *__restrict__ base, const uint16_t *__restrict__ residual,
-                                                        const uint16_t *__restrict__ norm_weight, uint16_t *__restrict__ output,
-                                                        uint16_t *__restrict__ normalized, uint8_t *__restrict__ table, DraftConvTableParams p) {
-  constexpr uint32_t kHeld = kStagedWidth / 8u / 256u;
+__global__ __launch_bounds__(Residual ? 1024 : 64) void draft_conv_table(
+    const uint16_t *__restrict__ input, const uint16_t *__restrict__ dynamic, const uint16_t *__restrict__ base,
+    const uint16_t *__restrict__ residual, const uint16_t *__restrict__ norm_weight, uint16_t *__restrict__ output,
+    uint16_t *__restrict__ normalized, uint8_t *__restrict__ table, DraftConvTableParams p) {
   static_assert(DRAFT_CONVOLUTION_TABLE_WIDTH <= kStagedWidth && DRAFT_CONVOLUTION_GROUP % 8u == 0, "eight channels share their dynamic weights");
   __shared__ float scratch[4];
-  __shared__ __align__(16) uint16_t rowX[kStagedWidth], rowW[Residual ? kStagedWidth : 8];
+  __shared__ __align__(16) uint16_t rowX[Residual ? kStagedWidth : 8];
   const uint32_t row = blockIdx.x, width = p.hidden, vectors = width / 8u, groups = width / DRAFT_CONVOLUTION_GROUP;
+  const uint32_t v = Residual ? threadIdx.x : blockIdx.y * 64u + threadIdx.x;
   const bool live = row < p.rows;
-  if (live) {
+  uint4 packed = make_uint4(0u, 0u, 0u, 0u), norm = packed;
+  if (live && v < vectors) {
     const bool follows = row % DRAFT_ATTENTION_QUERY_ROWS > 0;   // a lane's first row has none before it
     const size_t before = row - (follows ? 1u : 0u);
     const uint16_t *mine = dynamic + size_t(row) * draft_dynamic_width(width) + (Residual ? DRAFT_CONVOLUTION_TAPS : 0u) * groups;
     const uint16_t *taps = base + (Residual ? DRAFT_CONVOLUTION_TAPS : 0u) * size_t(width);
-    auto vector = [](const uint16_t *from, uint32_t v) { return reinterpret_cast<const uint4 *>(from)[v]; };
-    uint4 now[kHeld], last[kHeld], tap0[kHeld], tap1[kHeld], added[kHeld];
-    uint32_t dynamic0[kHeld], dynamic1[kHeld];
-#pragma unroll
-    for (uint32_t i = 0; i < kHeld; ++i) {
-      const uint32_t v = min(threadIdx.x + 256u * i, vectors - 1u);   // the last vector again past the row's end
-      now[i] = vector(input + size_t(row) * width, v);
-      last[i] = vector(input + before * width, v);
-      tap0[i] = vector(taps, v);
-      tap1[i] = vector(taps + width, v);
-      if constexpr (Residual) added[i] = vector(residual + size_t(row) * width, v);
-      dynamic0[i] = mine[v / (DRAFT_CONVOLUTION_GROUP / 8u)];
-      dynamic1[i] = mine[groups + v / (DRAFT_CONVOLUTION_GROUP / 8u)];
-    }
-    StagedRow norms;
-    if constexpr (Residual) norms.load(norm_weight, width);
-#pragma unroll
-    for (uint32_t i = 0; i < kHeld; ++i) {
-      arrived(now[i]);
-      arrived(last[i]);
-      arrived(tap0[i]);
-      arrived(tap1[i]);
-      if constexpr (Residual) arrived(added[i]);
-      arrived(dynamic0[i]);
-      arrived(dynamic1[i]);
-    }
-    if constexpr (Residual) norms.store(width, rowW);
-#pragma unroll
-    for (uint32_t i = 0; i < kHeld; ++i) {
-      const uint32_t v = threadIdx.x + 256u * i;
-      if (v >= vectors) continue;
-      const float d0 = bf16_bits_to_float(dynamic0[i]), d1 = bf16_bits_to_float(dynamic1[i]);
-      auto channel = [&](uint32_t x, uint32_t y, uint32_t t0, uint32_t t1, uint32_t a) {
-        float value = bf16_bits_to_float(x) * (bf16_bits_to_float(t0) + d0);
-        if (follows) value += bf16_bits_to_float(y) * (bf16_bits_to_float(t1) + d1);
-        if constexpr (Residual) value += bf16_bits_to_float(a);
-        return float_to_bf16_bits(value);
-      };
-      const uint32_t x[4] = {now[i].x, now[i].y, now[i].z, now[i].w}, y[4] = {last[i].x, last[i].y, last[i].z, last[i].w};
-      const uint32_t t0[4] = {tap0[i].x, tap0[i].y, tap0[i].z, tap0[i].w}, t1[4] = {tap1[i].x, tap1[i].y, tap1[i].z, tap1[i].w};
-      uint32_t a[4] = {}, out[4];
-      if constexpr (Residual) a[0] = added[i].x, a[1] = added[i].y, a[2] = added[i].z, a[3] = added[i].w;
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        out[e] = channel(x[e] & 0xFFFFu, y[e] & 0xFFFFu, t0[e] & 0xFFFFu, t1[e] & 0xFFFFu, a[e] & 0xFFFFu) |
-                 (channel(x[e] >> 16, y[e] >> 16, t0[e] >> 16, t1[e] >> 16, a[e] >> 16) << 16);
-      const uint4 packed = make_uint4(out[0], out[1], out[2], out[3]);
-      reinterpret_cast<uint4 *>(output + size_t(row) * width)[v] = packed;
-      reinterpret_cast<uint4 *>(rowX)[v] = packed;
-    }
+    auto vector = [&](const uint16_t *from) { return reinterpret_cast<const uint4 *>(from)[v]; };
+    uint4 now = vector(input + size_t(row) * width), last = vector(input + before * width), tap0 = vector(taps), tap1 = vector(taps + width);
+    uint4 added = packed;
+    if constexpr (Residual) added = vector(residual + size_t(row) * width);
+    uint32_t dynamic0 = mine[v / (DRAFT_CONVOLUTION_GROUP / 8u)], dynamic1 = mine[groups + v / (DRAFT_CONVOLUTION_GROUP / 8u)];
+    if constexpr (Residual) norm = vector(norm_weight);
+    arrived(now);
+    arrived(last);
+    arrived(tap0);
+    arrived(tap1);
+    if constexpr (Residual) arrived(added);
+    arrived(dynamic0);
+    arrived(dynamic1);
+    const float d0 = bf16_bits_to_float(dynamic0), d1 = bf16_bits_to_float(dynamic1);
+    auto channel = [&](uint32_t x, uint32_t y, uint32_t t0, uint32_t t1, uint32_t a) {
+      float value = bf16_bits_to_float(x) * (bf16_bits_to_float(t0) + d0);
+      if (follows) value += bf16_bits_to_float(y) * (bf16_bits_to_float(t1) + d1);
+      if constexpr (Residual) value += bf16_bits_to_float(a);
+      return float_to_bf16_bits(value);
+    };
+    auto pair = [&](uint32_t x, uint32_t y, uint32_t t0, uint32_t t1, uint32_t a) {
+      return channel(x & 0xFFFFu, y & 0xFFFFu, t0 & 0xFFFFu, t1 & 0xFFFFu, a & 0xFFFFu) | (channel(x >> 16, y >> 16, t0 >> 16, t1 >> 16, a >> 16) << 16);
+    };
+    packed = make_uint4(pair(now.x, last.x, tap0.x, tap1.x, added.x), pair(now.y, last.y, tap0.y, tap1.y, added.y),
+                        pair(now.z, last.z, tap0.z, tap1.z, added.z), pair(now.w, last.w, tap0.w, tap1.w, added.w));
+    reinterpret_cast<uint4 *>(output + size_t(row) * width)[v] = packed;
+    if constexpr (Residual) reinterpret_cast<uint4 *>(rowX)[v] = packed;
   }
-  __syncthreads();
   if constexpr (Residual) {
+    __syncthreads();
     const float inverse = live ? rms_inverse(rowX, width, scratch) : 0.f;
-    write_table_row<true>(rowX, rowW, inverse, live, row, normalized, table, width, p.tiles);
-  } else {
-    write_table_row<false>(rowX, rowW, 0.f, live, row, normalized, table, width, p.tiles);
+    if (v < vectors) write_norm_vector(packed, norm, inverse, live, row, v, normalized, table, width, p.tiles);
+  } else if (v < vectors) {
+    write_table_vector(packed, row, v, table, width, p.tiles);
   }
 }
 SP_REGISTER_KERNEL("draft_conv_table", &draft_conv_table<false>);
@@ -428,62 +458,67 @@ SP_REGISTER_KERNEL("gguf_embed_iq4xs", &gguf_embed<GGUF_FMT_IQ4XS>);
 SP_REGISTER_KERNEL("gguf_embed_iq4nl", &gguf_embed<GGUF_FMT_IQ4NL>);
 
 // gguf_embed_norm_<fmt>: the first passes of a step as one: rope_build_tree_tables, gguf_embed and norm_rms_table16 of
-// its rows, each the values of its own kernel. Grid (tiles * 16, 2 or 1 without rotary pairs), 256 threads: a workgroup
-// of y = 0 gathers a row into LDS (thread t input t of every super-block), stores it, norms it and writes its part of
-// the activation table (zeros past the live rows); one of y = 1 writes the row's RoPE tables. Rows of up to kStagedWidth
-// columns. Three launches of a few workgroups each that only waited on one another: 3.7 + 4.1 + 5.6 us at 16 rows of 1024
-// columns, 8.3 together (the gather, the sum and the table are one chain of waits), and two launches less a step.
+// its rows, each the values of its own kernel. Grid (tiles * 16, 2 or 1 without rotary pairs), 256 threads
+// or more (the host: a thread an input, up to 1024): a workgroup of y = 0 gathers a row into LDS, stores it, norms it and
+// writes its part of the activation table, a thread a vector of eight (zeros past the live rows); one of y = 1 writes the
+// row's RoPE tables. Rows of up to kStagedWidth columns. Three launches of a few workgroups each that only waited on one
+// another: 3.7 + 4.1 + 5.6 us at 16 rows of 1024 columns, 8.0 together by 256 threads (the gather, the sum and the table are
+// one chain of waits), 5.7 by 1024; at 16 rows of 5120 columns 12.9 -> 9.2. And two launches less a step.
 template <uint32_t FMT>
-__global__ __launch_bounds__(256) void gguf_embed_norm(const uint8_t *__restrict__ embedding, const uint32_t *__restrict__ tokens,
+__global__ __launch_bounds__(1024) void gguf_embed_norm(const uint8_t *__restrict__ embedding, const uint32_t *__restrict__ tokens,
                                                        const uint16_t *__restrict__ weight, uint16_t *__restrict__ hidden,
                                                        uint16_t *__restrict__ output, uint8_t *__restrict__ table,
                                                        const float *__restrict__ inverse_frequency, const uint32_t *__restrict__ depth,
                                                        float *__restrict__ cosines, float *__restrict__ sines, EmbedNormParams p) {
   __shared__ float scratch[4];
-  __shared__ __align__(16) uint16_t rowX[kStagedWidth], rowW[kStagedWidth];
+  __shared__ __align__(16) uint16_t rowX[kStagedWidth];
   // a native row in pieces that every format's rows are whole numbers of (a Q6_K block is 210 bytes)
   using Piece = std::conditional_t<FMT == GGUF_FMT_Q6K, uint16_t, uint32_t>;
-  constexpr uint32_t kNative = kStagedWidth / 256u * EmbedBlock<FMT>::kBytes / sizeof(Piece), kPieces = (kNative + 255u) / 256u;
+  constexpr uint32_t kNative = kStagedWidth / 256u * EmbedBlock<FMT>::kBytes / sizeof(Piece), kPieces = (kNative + 1023u) / 1024u;
   __shared__ __align__(16) Piece native[kNative];
-  const uint32_t row = blockIdx.x, tid = threadIdx.x;
+  const uint32_t row = blockIdx.x, tid = threadIdx.x, threads = blockDim.x, vectors = p.embed.hidden / 8u;
   const bool live = row < p.embed.rows;
   if (blockIdx.y) {
     if (live)
-      for (uint32_t pair = tid; pair < p.rope.pairs; pair += 256u) rope_entry(row, pair, inverse_frequency, depth, cosines, sines, p.rope);
+      for (uint32_t pair = tid; pair < p.rope.pairs; pair += threads) rope_entry(row, pair, inverse_frequency, depth, cosines, sines, p.rope);
     return;
   }
-  float inverse = 0.f;
+  uint4 norm = make_uint4(0u, 0u, 0u, 0u);
   if (live) {
     const uint32_t token = tokens[row], blocks = p.embed.hidden / 256u;
     const bool inside = token < p.embed.vocabulary;
     // the native row whole, with every load in flight at once (a decode's byte loads from memory wait for one another)
     const uint8_t *source = embedding + size_t(inside ? token : 0u) * blocks * EmbedBlock<FMT>::kBytes;
     const uint32_t pieces = blocks * EmbedBlock<FMT>::kBytes / uint32_t(sizeof(Piece));
-    uint32_t held[kPieces];
+    norm = reinterpret_cast<const uint4 *>(weight)[min(tid, vectors - 1u)];
+    for (uint32_t first = tid; first < pieces; first += threads * kPieces) {
+      uint32_t held[kPieces];
 #pragma unroll
-    for (uint32_t i = 0; i < kPieces; ++i) {
-      Piece piece;
-      __builtin_memcpy(&piece, source + min(tid + 256u * i, pieces - 1u) * sizeof(Piece), sizeof(Piece));
-      held[i] = piece;
+      for (uint32_t i = 0; i < kPieces; ++i) {
+        Piece piece;
+        __builtin_memcpy(&piece, source + min(first + threads * i, pieces - 1u) * sizeof(Piece), sizeof(Piece));
+        held[i] = piece;
+      }
+#pragma unroll
+      for (uint32_t i = 0; i < kPieces; ++i) arrived(held[i]);
+#pragma unroll
+      for (uint32_t i = 0; i < kPieces; ++i)
+        if (first + threads * i < pieces) native[first + threads * i] = Piece(held[i]);
     }
-    StagedRow norms;
-    norms.load(weight, p.embed.hidden);
-#pragma unroll
-    for (uint32_t i = 0; i < kPieces; ++i) arrived(held[i]);
-#pragma unroll
-    for (uint32_t i = 0; i < kPieces; ++i)
-      if (tid + 256u * i < pieces) native[tid + 256u * i] = Piece(held[i]);
-    norms.store(p.embed.hidden, rowW);
     __syncthreads();
-    for (uint32_t b = 0; b < blocks; ++b) {
-      const uint16_t value = inside ? uint16_t(EmbedBlock<FMT>::bits(reinterpret_cast<const uint8_t *>(native) + b * EmbedBlock<FMT>::kBytes, tid)) : uint16_t(0);
-      rowX[b * 256u + tid] = value;
-      hidden[size_t(row) * p.embed.hidden + b * 256u + tid] = value;
+    for (uint32_t at = tid; at < p.embed.hidden; at += threads) {
+      const uint8_t *block = reinterpret_cast<const uint8_t *>(native) + at / 256u * EmbedBlock<FMT>::kBytes;
+      const uint16_t value = inside ? uint16_t(EmbedBlock<FMT>::bits(block, at % 256u)) : uint16_t(0);
+      rowX[at] = value;
+      hidden[size_t(row) * p.embed.hidden + at] = value;
     }
   }
   __syncthreads();
-  if (live) inverse = rms_inverse(rowX, p.embed.hidden, scratch);
-  write_table_row<true>(rowX, rowW, inverse, live, row, output, table, p.embed.hidden, p.tiles);
+  const float inverse = live ? rms_inverse(rowX, p.embed.hidden, scratch) : 0.f;
+  for (uint32_t v = tid; v < vectors; v += threads) {   // (once where the host's rule gives the threads)
+    if (live && v != tid) norm = reinterpret_cast<const uint4 *>(weight)[v];
+    write_norm_vector(reinterpret_cast<const uint4 *>(rowX)[v], norm, inverse, live, row, v, output, table, p.embed.hidden, p.tiles);
+  }
 }
 SP_REGISTER_KERNEL("gguf_embed_norm_q4k", &gguf_embed_norm<GGUF_FMT_Q4K>);
 SP_REGISTER_KERNEL("gguf_embed_norm_q6k", &gguf_embed_norm<GGUF_FMT_Q6K>);

@@ -115,7 +115,8 @@ PreparedInput DraftAttention::addConvolutionTable(hip::CommandGraph &graph, cons
                     &after = finish ? normalized : buffers.output;
   graph.add(finish ? "draft_conv_norm_table" : "draft_conv_table",
             {buffers.input, buffers.dynamic, buffers.weights, residual, norm, buffers.output, after, scratch.input},
-            DraftConvTableParams{width, rows, tiles}, {tiles * GGUF_ROW_TILE, 1, 1}, {256, 1, 1});
+            DraftConvTableParams{width, rows, tiles}, {tiles * GGUF_ROW_TILE, finish ? 1u : (width / 8 + 63) / 64, 1},
+            {finish ? norm_row_threads(width) : 64u, 1, 1});
   return {after, LinearInput::Table16};
 }
 

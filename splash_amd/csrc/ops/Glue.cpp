@@ -2,6 +2,7 @@
 
 #include <string>
 
+#include <algorithm>
 #include <stdexcept>
 
 namespace splash::ops {
@@ -57,7 +58,7 @@ PreparedInput Normalization::addRmsTable(hip::CommandGraph &graph, const hip::Bu
   const uint32_t tiles = gguf_row_tiles(rows);
   requireBytes(scratch.input, gguf_tables_bytes(width, tiles), "projection table");
   graph.add("norm_rms_table16", {input, weight, output, scratch.input}, NormParams{width, rows, tiles, 0},
-            {tiles * GGUF_ROW_TILE, 1, 1}, {256, 1, 1});
+            {tiles * GGUF_ROW_TILE, 1, 1}, {norm_row_threads(width), 1, 1});
   return {output, LinearInput::Table16};
 }
 
@@ -87,7 +88,7 @@ PreparedInput Embedding::addNormTable(hip::CommandGraph &graph, const EmbeddingT
   graph.add(std::string("gguf_embed_norm_") + gguf_format_name(table.formatId),
             {table.rows, tokens, weight, hidden, normalized, scratch.input, rotates ? rope.inverseFrequency : hidden,
              rotates ? rope.depth : hidden, rotates ? rope.cosines : hidden, rotates ? rope.sines : hidden},
-            params, {tiles * GGUF_ROW_TILE, rotates ? 2u : 1u, 1}, {256, 1, 1});
+            params, {tiles * GGUF_ROW_TILE, rotates ? 2u : 1u, 1}, {std::min(table.hidden, 1024u), 1, 1});
   return {normalized, LinearInput::Table16};
 }
 
