@@ -674,7 +674,7 @@ __device__ OrderEnd select_last(const float *x, uint32_t vocabulary, Mass mass, 
 // (logit, id) in LDS; the count and the running mass in that order are what top_k and top_p cut. Any other row (a
 // nucleus of many thousand tokens) takes the descent above, a scan of the row a digit. What bounds the pass is one
 // compute unit's reading of the row: 24 rows of 151936 logits under min_p 0.02, top_k 64 and top_p 0.95 took 1244 us by
-// the descent of 256 threads, and 42 us this way.
+// the descent of 256 threads, 39 us this way with every token keyed and 27 as it is.
 constexpr uint32_t kEndCandidates = 8192, kEndBins = 512;
 constexpr float kEndBinsPerFold = 16.f;
 struct EndSelection {
@@ -688,11 +688,23 @@ union EndShared {
   EndScratch descent;
   EndSelection selection;
 };
-// Calls take(value, token) of every token of the row, four a load whatever the row's alignment.
-template <class Take> __device__ __forceinline__ void end_scan(const float *x, uint32_t vocabulary, uint32_t tid, Take take) {
+// Calls all(four) of every four tokens of the row, a load whatever the row's alignment, and take(value, token) of the tokens
+// of a four that holds a value at or above `floor` (past the row's end the values are -infinity). Few tokens pass a floor, so
+// a scan costs what it does of every token: with the row's key, its comparison and a branch for each of them a row of 151936
+// logits took 10 us a scan of its compute unit's vector ALUs, more than the 4 us of reading it.
+template <class All, class Take>
+__device__ __forceinline__ void end_scan(const float *x, uint32_t vocabulary, uint32_t tid, float floor, All all, Take take) {
   typedef __attribute__((ext_vector_type(4), aligned(4))) float f32x4_unaligned;
   const f32x4_unaligned *v = reinterpret_cast<const f32x4_unaligned *>(x);
   const uint32_t vectors = vocabulary / 4u;
+  auto four = [&](f32x4_unaligned held, uint32_t first) {
+    all(held);
+    if (!(fmaxf(fmaxf(held.x, held.y), fmaxf(held.z, held.w)) >= floor)) return;   // (a NaN is no maximum of others)
+    take(held.x, first);
+    take(held.y, first + 1u);
+    take(held.z, first + 2u);
+    take(held.w, first + 3u);
+  };
   constexpr uint32_t kAhead = 8;
   for (uint32_t base = tid; base < vectors; base += kAhead * kEndThreads) {
     f32x4_unaligned held[kAhead];
@@ -702,11 +714,9 @@ template <class Take> __device__ __forceinline__ void end_scan(const float *x, u
       held[i] = at < vectors ? v[at] : f32x4_unaligned{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
     }
 #pragma unroll
-    for (uint32_t i = 0; i < kAhead; ++i)
-#pragma unroll
-      for (uint32_t e = 0; e < 4; ++e) take(held[i][e], 4u * (base + i * kEndThreads) + e);
+    for (uint32_t i = 0; i < kAhead; ++i) four(held[i], 4u * (base + i * kEndThreads));
   }
-  if (tid < vocabulary % 4u) take(x[4u * vectors + tid], 4u * vectors + tid);
+  if (tid < vocabulary % 4u) four(f32x4_unaligned{x[4u * vectors + tid], -INFINITY, -INFINITY, -INFINITY}, 4u * vectors + tid);
 }
 __device__ __forceinline__ uint32_t end_bin(float value, float maximum, float inverse) {
   return uint32_t(min(int((maximum - value) * inverse * kEndBinsPerFold), int(kEndBins) - 1));  // rises as the logit falls
@@ -725,7 +735,8 @@ __global__ __launch_bounds__(kEndThreads) void decode_sample_distribution_end(co
   const uint32_t topK = p.top_k[laneIndex];
   const float maximum = wave_max(masses[2u * (row * SAMPLING_SHARDS + lane % SAMPLING_SHARDS)]);
   // what min_p keeps: the tokens at or above the logit that weighs min_p of the heaviest
-  const uint32_t lowest = minP > 0.f ? logit_key(fminf(maximum + temperature * logf(minP), maximum)) : kLowestKey;
+  const float floor = minP > 0.f ? fminf(maximum + temperature * logf(minP), maximum) : -INFINITY;
+  const uint32_t lowest = logit_key(floor);
   for (uint32_t b = tid; b < kEndBins; b += kEndThreads) s.bins[b] = 0;
   if (wave == 0) {
     const float total = row_mass(masses, row, inverse).sum;
@@ -737,11 +748,15 @@ __global__ __launch_bounds__(kEndThreads) void decode_sample_distribution_end(co
   }
   __syncthreads();
   uint32_t selectable = 0;
-  end_scan(x, p.vocabulary, tid, [&](float value, uint32_t) {
-    if (unselectable(value)) return;
-    ++selectable;
-    if (logit_key(value) >= lowest) atomicAdd(&s.bins[end_bin(value, maximum, inverse)], 1u);
-  });
+  end_scan(x, p.vocabulary, tid, floor,
+           [&](auto held) {
+#pragma unroll
+             for (int e = 0; e < 4; ++e) selectable += unselectable(held[e]) ? 0u : 1u;
+           },
+           [&](float value, uint32_t) {
+             if (unselectable(value)) return;
+             if (logit_key(value) >= lowest) atomicAdd(&s.bins[end_bin(value, maximum, inverse)], 1u);
+           });
   selectable = wave_sum(selectable);
   if (lane == 0) atomicAdd(&s.selectable, selectable);
   __syncthreads();
@@ -799,12 +814,16 @@ __global__ __launch_bounds__(kEndThreads) void decode_sample_distribution_end(co
   if (candidates <= kEndCandidates) {
     const uint32_t slots = candidates <= 1u ? 1u : 1u << (32u - uint32_t(__builtin_clz(candidates - 1u)));
     for (uint32_t i = candidates + tid; i < slots; i += kEndThreads) s.order[i] = 0;
-    end_scan(x, p.vocabulary, tid, [&](float value, uint32_t token) {
-      if (unselectable(value)) return;
-      const uint32_t key = logit_key(value);
-      if (key < lowest || end_bin(value, maximum, inverse) > cut) return;
-      s.order[atomicAdd(&s.gathered, 1u)] = uint64_t(key) << 32 | uint64_t(~token);
-    });
+    // A token of bin `cut` or before lies at or above this: the bin's far edge, and further out by more than the roundings of
+    // end_bin and of this line move it. (An infinite maximum makes it NaN, which fmaxf drops.)
+    const float edge = cut + 1u < kEndBins ? maximum - float(cut + 1u) / kEndBinsPerFold * temperature * 1.0001f - fabsf(maximum) * 1e-6f : -INFINITY;
+    end_scan(x, p.vocabulary, tid, fmaxf(floor, edge), [](auto) {},
+             [&](float value, uint32_t token) {
+               if (unselectable(value)) return;
+               const uint32_t key = logit_key(value);
+               if (key < lowest || end_bin(value, maximum, inverse) > cut) return;
+               s.order[atomicAdd(&s.gathered, 1u)] = uint64_t(key) << 32 | uint64_t(~token);
+             });
     __syncthreads();
     // bitonic, descending (the order they were gathered in leaves no trace: no two are equal)
     for (uint32_t size = 2; size <= slots; size <<= 1)
@@ -963,6 +982,42 @@ __device__ __forceinline__ void wave_values(float mine, float *staged, float (&v
   }
 }
 
+// The running sums of `count` values of LDS, a multiple of four, in their order and from `start`: before[i] what lies before
+// value i, before[count] all of it. One lane's chain of additions and nothing else: what a walk in order asks of each step
+// (is the point passed, is this the last with weight) the lanes then ask of all of them at once. (24 rows' draws: 27 us with
+// walks that asked at each step, unrolled into 20 KB of instructions; 10.6 so. The same sums and the same token.)
+__device__ __forceinline__ void running_sums(const float *values, float *before, uint32_t count, float start) {
+  wave_lds_fence();   // (the values are written, and what was read of `before`)
+  if ((threadIdx.x & 63u) == 0) {
+    float sum = start;
+#pragma unroll 4
+    for (uint32_t i = 0; i < count / 4u; ++i) {
+      const float4 v = reinterpret_cast<const float4 *>(values)[i];
+      float4 b;
+      b.x = sum;
+      b.y = b.x + v.x;
+      b.z = b.y + v.y;
+      b.w = b.z + v.z;
+      sum = b.w + v.w;
+      reinterpret_cast<float4 *>(before)[i] = b;
+    }
+    before[count] = sum;
+  }
+  wave_lds_fence();
+}
+// Of values whose running sums are `before`: the first that the point lies inside, or the last that has weight (0 if none has).
+template <uint32_t Count> __device__ __forceinline__ uint32_t value_at(const float *values, const float *before, float point) {
+  uint32_t hit = Count, lastWeighted = 0;
+#pragma unroll
+  for (uint32_t i = 0; i < Count; i += 64u) {
+    const uint32_t j = i + (threadIdx.x & 63u);
+    const uint64_t passed = __ballot(point < before[j] + values[j]), weighted = __ballot(values[j] > 0.f);
+    if (hit == Count && passed) hit = i + uint32_t(__builtin_ctzll(passed));
+    if (weighted) lastWeighted = i + 63u - uint32_t(__builtin_clzll(weighted));
+  }
+  return hit == Count ? lastWeighted : hit;
+}
+
 // Grid (rows), 64 threads: the row's selection. A sampled row whose child was accepted selects it;
 // otherwise it draws at point = u_row * sum of the ranges, from the residual when its child was
 // rejected (decisions[2 row + 1] == 1) and from p itself when it has no child.
@@ -984,69 +1039,42 @@ __global__ __launch_bounds__(64) void decode_sample_draw(const float *__restrict
   const float *x = logits + size_t(row) * p.logits_stride, *q = draft + size_t(row) * p.logits_stride;
   const float *r = ranges + row * SAMPLING_RANGES;
   // the ranges in LDS: the sums walk them in order without a trip to memory each
-  __shared__ float weights[SAMPLING_RANGES];
-  __shared__ __align__(16) float staged[64];
+  __shared__ __align__(16) float weights[SAMPLING_RANGES], before[SAMPLING_RANGES + 4];
 #pragma unroll
   for (uint32_t i = 0; i < SAMPLING_RANGES / 64u; ++i) weights[lane + 64u * i] = r[lane + 64u * i];
-  __syncthreads();
-  float total = 0.f;
-#pragma unroll 32
-  for (uint32_t j = 0; j < SAMPLING_RANGES; ++j) total += weights[j];
+  running_sums(weights, before, SAMPLING_RANGES, 0.f);
+  const float total = before[SAMPLING_RANGES];
   if (!(total > 0.f)) {
     if (lane == 0) tokens[row] = SAMPLING_NO_TOKEN;
     return;
   }
-  const float point = uniforms[2 * row] * total;
   // The range that holds the point; the last weighted range on a rounding shortfall.
-  uint32_t hit = SAMPLING_RANGES, lastWeighted = 0;
-  float before = 0.f, lastBefore = 0.f;
-  {
-    float cumulative = 0.f;
-#pragma unroll 32
-    for (uint32_t j = 0; j < SAMPLING_RANGES; ++j) {
-      const float w = weights[j];
-      if (w > 0.f) { lastWeighted = j; lastBefore = cumulative; }
-      if (hit == SAMPLING_RANGES && point < cumulative + w) { hit = j; before = cumulative; }
-      cumulative += w;
-    }
-  }
-  if (hit == SAMPLING_RANGES) { hit = lastWeighted; before = lastBefore; }
-  float target = point - before;
+  const float point = uniforms[2 * row] * total;
+  const uint32_t hit = value_at<SAMPLING_RANGES>(weights, before, point);
+  float target = point - before[hit];
   // Its lanes' chunks, as the ranges kernel summed them, walked in lane order.
   const uint32_t size = range_tokens(p.vocabulary), begin = hit * size, end = min(p.vocabulary, begin + size);
   const uint32_t per = (size + 63u) / 64u;
   const float sum = lane_residual(x, q, begin + lane * per, per, end, kept, inverse, rejected);
-  uint32_t chunk = 64, lastChunk = 0;
-  float chunkBefore = 0.f, lastChunkBefore = 0.f, cumulative = 0.f;
-  float sums[64];
-  wave_values(sum, staged, sums);
-#pragma unroll
-  for (int l = 0; l < 64; ++l) {
-    const float c = sums[l];
-    if (c > 0.f) { lastChunk = uint32_t(l); lastChunkBefore = cumulative; }
-    if (chunk == 64 && target < cumulative + c) { chunk = uint32_t(l); chunkBefore = cumulative; }
-    cumulative += c;
-  }
-  if (chunk == 64) { chunk = lastChunk; chunkBefore = lastChunkBefore; }
-  target -= chunkBefore;
+  wave_lds_fence();
+  weights[lane] = sum;
+  running_sums(weights, before, 64u, 0.f);
+  const uint32_t chunk = value_at<64u>(weights, before, target);
+  target -= before[chunk];
   // The chunk's tokens, weighed a lane each and walked in id order.
   uint32_t selected = SAMPLING_NO_TOKEN, lastToken = SAMPLING_NO_TOKEN;
   float walked = 0.f;
-  for (uint32_t i0 = 0; i0 < per; i0 += 64u) {
-    const uint32_t own = begin + chunk * per + i0 + lane;
+  for (uint32_t i0 = 0; i0 < per && selected == SAMPLING_NO_TOKEN; i0 += 64u) {
+    const uint32_t first = begin + chunk * per + i0, own = first + lane;
     const bool live = i0 + lane < per && own < end;
     const float weight = live ? residual_of(x[own], own, rejected ? q[own] : 0.f, kept, inverse, rejected) : 0.f;
-    float token_weights[64];
-    wave_values(weight, staged, token_weights);
-#pragma unroll
-    for (uint32_t i = 0; i < 64u; ++i) {
-      if (i0 + i >= per) break;
-      const float w = token_weights[i];
-      const uint32_t token = begin + chunk * per + i0 + i;
-      if (w > 0.f) lastToken = token;
-      walked += w;
-      if (selected == SAMPLING_NO_TOKEN && w > 0.f && target < walked) selected = token;
-    }
+    wave_lds_fence();
+    weights[lane] = weight;
+    running_sums(weights, before, 64u, walked);
+    const uint64_t weighted = __ballot(weight > 0.f), passed = __ballot(weight > 0.f && target < before[lane] + weight);
+    if (passed) selected = first + uint32_t(__builtin_ctzll(passed));
+    if (weighted) lastToken = first + 63u - uint32_t(__builtin_clzll(weighted));
+    walked = before[64];
   }
   if (lane == 0) tokens[row] = selected != SAMPLING_NO_TOKEN ? selected : lastToken;
 }

@@ -374,6 +374,36 @@ def test_distribution_ends_at_the_candidate_limit(backend, V):
     assert checked >= 6
 
 
+def test_distribution_ends_far_from_zero(backend):
+    """decode_sample_distribution_end passes over tokens below an edge that it derives from the row's maximum: logits so large
+    that their own spacing is a bin's width or many, and temperatures a bin of which is finer or wider than that."""
+    print("case distribution ends far from zero", flush=True)
+    rng = np.random.default_rng(17)
+    V = 20011
+    policies = [(0.7, 0.0, 40, 1.0), (0.01, 0.0, 0, 0.9), (50.0, 0.0, 100, 0.99), (0.7, 0.05, 300, 0.95)]
+    lanes = [(4 * i, 4) for i in range(len(policies))]
+    rows = 16
+    logits = (rng.standard_normal((rows, V)) * 2).astype(np.float32)
+    for r in range(rows):
+        logits[r] = (logits[r] * (1, 1, 20, 1)[r // 4] + (0, 1e4, -1e6, 3e7)[r % 4]).astype(np.float32)
+    draft = np.full((rows, V), 1.0 / V, np.float32)
+    b = sampling_buffers(backend, rows, V, logits, draft, rng.random((rows, 2)).astype(np.float32), np.zeros(rows, np.uint32),
+                         ops.chain_tree_rows([n for _, n in lanes]))
+    g = splash_amd.CommandGraph()
+    ops.Sampling.add_verify(g, b, V, V, lanes, policies)
+    backend.run(g)
+    words = b["decisions"].download(np.uint32).reshape(rows, 8)
+    checked = 0
+    for (first, n), (T, min_p, top_k, top_p) in zip(lanes, policies):
+        for r in range(first, first + n):
+            key, last, mass, count, close_end = orc.distribution_end(logits[r], T, min_p, top_k, top_p)
+            if close_end > 1e-5:
+                assert (words[r, 2], words[r, 3], words[r, 5]) == (key, last, count), (r, top_k, top_p)
+                assert abs(words[r, 4:5].view(np.float32)[0] - mass) <= 1e-5 * mass
+                checked += 1
+    assert checked >= 10
+
+
 def test_constraint_masks_and_stop_exclusion(backend):
     """TargetRow::admits (sampling.metal:42-46): a constrained lane's rows select only tokens of their mask rows, a lane
     that ignores end-of-sequence never a stop token, greedy or sampled; the other lanes' rows are untouched. The
