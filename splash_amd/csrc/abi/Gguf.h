@@ -221,6 +221,7 @@ struct GgufWideTableParams {
   uint32_t tiles;  // gguf_wide_tiles(rows)
   uint32_t reserved;
 };
+#define GGUF_WIDE_TILE_INPUTS 2048u  // inputs of the rows whose tile a workgroup puts together in LDS (gguf_wide_moe_*_tile)
 // gguf_wide_<fmt>_{a,r,g,p} (and gguf_wide_staged_*, weights rounded once to half): a chunk of rows, a workgroup up to 128
 // of them x 128 columns. Binds up to three segments of one format (a gate/up pair: gate, up), the wide table, out and the
 // residual rows (any buffer when unused). _p writes fp32 partials of its part of K to out, [part][rows][out_stride], which

@@ -202,8 +202,11 @@ void MoE::addChunk(hip::CommandGraph &graph, const hip::Buffer &scores, uint32_t
   graph.add("moe_chunk_place", {w.selected, w.counts, w.routeSlot, w.slotRow, w.tasks, w.totals}, grouping, {windows, 1, 1}, {1024, 1, 1});
   auto project = [&](const char *table, const hip::Buffer &input, uint32_t inputRows, uint32_t k, uint32_t n, uint32_t format, uint64_t expertBytes,
                      const hip::Buffer &first, const hip::Buffer &second, const hip::Buffer &out, bool gateUp) {
-    graph.add(table, {input, w.slotRow, w.totals, w.table}, GgufWideTableParams{k, inputRows, tiles, 0}, {64 * ((16 * tiles + 63) / 64), 1, 1},
-              {256, 1, 1});
+    const GgufWideTableParams slots{k, inputRows, tiles, 0};
+    if (k <= GGUF_WIDE_TILE_INPUTS)
+      graph.add(std::string(table) + "_tile", {input, w.slotRow, w.totals, w.table}, slots, {tiles, 1, 1}, {1024, 1, 1});
+    else
+      graph.add(table, {input, w.slotRow, w.totals, w.table}, slots, {64 * ((16 * tiles + 63) / 64), 1, 1}, {256, 1, 1});
     GgufWideMoeParams params{};
     params.wide.input_size = k;
     params.wide.tiles = tiles;

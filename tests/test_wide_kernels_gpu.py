@@ -357,6 +357,33 @@ def test_expert_tiles_of_tall_tasks_lie_in_the_interval(backend, name):
     test_expert_tiles_lie_in_the_interval(backend, name, 8)
 
 
+# half a wave's piece, one and a half, three and a half, and the four that a wave holds
+@pytest.mark.parametrize("K", [256, 768, 1792, 2048])
+@pytest.mark.parametrize("kind", ["gather", "rows"])
+def test_slots_tables_by_the_tile_are_those_by_the_row(backend, K, kind):
+    """The slots' tables put together in LDS and those that the rows write are the same bytes: rows of ordinary values, of
+    zeros, subnormals and the largest ones, with infinities and NaN, empty slots, and tiles past the count left alone."""
+    print(f"case slot tables by the tile {kind} K={K}", flush=True)
+    rng = np.random.default_rng(K)
+    tiles, live, rows = 7, 5, 61
+    slots = 16 * tiles
+    source = orc.f32_to_bf16((rng.standard_normal((rows if kind == "gather" else slots, K)) * 10.0 ** rng.integers(-6, 7, (1, K))).astype(np.float32))
+    source[1], source[2], source[3] = 0, 1, 0x7F7F
+    source[4, 5], source[5, K - 1], source[6, :3] = 0x7F80, 0x7FC1, (0xFF80, 0x8000, 0xFFFF)
+    slot_row = np.where(rng.random(slots) < 0.2, 0xFFFFFFFF, rng.integers(0, rows, slots)).astype(np.uint32)
+    slot_row[:7] = np.arange(7)
+    x, s, totals = backend.from_array(source), backend.from_array(slot_row), backend.from_array(np.array([live, 0, 0, 0], np.uint32))
+    got = []
+    for suffix, grid, threads in (("", 64 * -(-slots // 64), 256), ("_tile", tiles, 1024)):
+        table = backend.allocate_buffer(table_bytes(K, tiles))
+        table.fill(0xA5)
+        graph = splash_amd.CommandGraph()
+        graph.add(f"gguf_wide_moe_{kind}{suffix}", [x, s, totals, table], TableParams(K, len(source), tiles, 0), (grid, 1, 1), (threads, 1, 1))
+        backend.run(graph)
+        got.append(table.download())
+    assert np.array_equal(got[0], got[1]) and (got[0] != 0xA5).any()
+
+
 @pytest.mark.parametrize("geometry,tokens,committed,gated", [((64, 8, 128), 200, 300, False), ((64, 8, 128), 53, 0, True), ((32, 8, 128), 200, 250, True),
                                                              ((32, 8, 128), 64, 1000, False), ((16, 8, 64), 200, 300, False), ((16, 8, 64), 37, 700, True)])
 def test_a_chunks_blocks_attend_whole_histories(backend, geometry, tokens, committed, gated):
