@@ -374,6 +374,34 @@ def test_distribution_ends_at_the_candidate_limit(backend, V):
     assert checked >= 6
 
 
+# fewer tokens than ranges, ranges that end inside a round of loads, the longest range that LDS holds and one past it
+@pytest.mark.parametrize("V", [33, 8191, 262144, 262145])
+def test_rejection_sampling_rows_of_short_and_long_ranges(backend, V):
+    """The draws of a row whose 256 ranges are summed through LDS, and past it, equal the oracle's as above."""
+    print(f"case sampled ranges V={V}", flush=True)
+    rng = np.random.default_rng(V)
+    rows, T = 6, 0.9
+    logits = (rng.standard_normal((rows, V)) * 2.5).astype(np.float32)
+    draft = np.exp(rng.standard_normal((rows, V)) * 2)
+    draft = (draft / draft.sum(axis=1, keepdims=True)).astype(np.float32)
+    tokens = np.array([int(np.argmax(draft[max(r - 1, 0)])) for r in range(rows)], np.uint32)
+    uniforms = rng.random((rows, 2)).astype(np.float32)
+    b = sampling_buffers(backend, rows, V, logits, draft, uniforms, tokens, ops.chain_tree_rows([rows]))
+    g = splash_amd.CommandGraph()
+    ops.Sampling.add_verify(g, b, V, V, [(0, rows)], [T])
+    backend.run(g)
+    got = b["tokens"].download(np.uint32)
+    checked = 0
+    for r in range(rows):
+        child = int(tokens[r + 1]) if r + 1 < rows else orc.NO_TOKEN
+        want, accepted, close = orc.rejection_row(logits[r], T, draft[r] if child != orc.NO_TOKEN else None, child,
+                                                  float(uniforms[r, 1]), float(uniforms[r, 0]))
+        if close > 1e-5:
+            assert got[r] == want, (r, got[r], want, accepted)
+            checked += 1
+    assert checked >= 3
+
+
 def test_distribution_ends_far_from_zero(backend):
     """decode_sample_distribution_end passes over tokens below an edge that it derives from the row's maximum: logits so large
     that their own spacing is a bin's width or many, and temperatures a bin of which is finer or wider than that."""
