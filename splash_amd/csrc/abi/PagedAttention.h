@@ -21,6 +21,7 @@
 #define ATTENTION_STEP_TOKENS 64u    // tokens the split kernel takes at a time; history splits hold whole steps
 #define ATTENTION_VALUE_BLOCK 64u
 #define ATTENTION_MAXIMUM_ROWS 16u      // rows of one sequence's verify block (SPLASH_TARGET_VERIFY_ROWS)
+#define ATTENTION_VECTOR_HEADS(D) (512u / (D))  // query heads of a workgroup of attention_q8_qkv_vectors
 #define ATTENTION_MAXIMUM_SEQUENCES 8u  // sequences of one dispatch
 #define ATTENTION_MAXIMUM_SPLITS 128u   // SPLASH_ATTENTION_MAXIMUM_SPLITS
 

@@ -187,14 +187,13 @@ SP_REGISTER_KERNEL("attention_q8_qkv_chunk_d64", (&attention_q8_qkv<64, true>));
 // A workgroup a row is bound by how fast workgroups start (147456 of them for 2048 rows of 64 / 8 heads): 114 us there, 45 at
 // 777 rows, against 76 and 36 here. Four rows one after the other take 14.5 us however few the blocks are.
 template <int D>
-__global__ __launch_bounds__(256) void attention_q8_qkv_rows(const uint16_t *__restrict__ qkv, const uint16_t *__restrict__ q_norm,
-                                                            const uint16_t *__restrict__ k_norm, const float *__restrict__ rope_cos,
-                                                            const float *__restrict__ rope_sin, _Float16 *__restrict__ queries,
-                                                            float *__restrict__ qsums, const uint64_t *__restrict__ page_table,
-                                                            uint8_t *__restrict__ pool, AttentionParams p) {
+__device__ __forceinline__ void qkv_rows_of_head(const uint32_t head, const uint16_t *__restrict__ qkv, const uint16_t *__restrict__ q_norm,
+                                                 const uint16_t *__restrict__ k_norm, const float *__restrict__ rope_cos,
+                                                 const float *__restrict__ rope_sin, _Float16 *__restrict__ queries, float *__restrict__ qsums,
+                                                 const uint64_t *__restrict__ page_table, uint8_t *__restrict__ pool, const AttentionParams &p) {
   constexpr uint32_t E = D / 64, kRows = 4;
   __shared__ float normalized[4][D];
-  const uint32_t l = threadIdx.x & 63u, wave = threadIdx.x >> 6, head = blockIdx.x, z = blockIdx.y;
+  const uint32_t l = threadIdx.x & 63u, wave = threadIdx.x >> 6, z = blockIdx.y;
   const AttentionSequence seq = block_sequence<true>(p, z);
   const bool query = head < p.q_heads;
   const uint32_t group = p.q_heads / p.kv_heads, index = query ? head : head - p.q_heads, pairs = p.rotary_pairs;
@@ -307,8 +306,127 @@ __global__ __launch_bounds__(256) void attention_q8_qkv_rows(const uint16_t *__r
     }
   }
 }
+template <int D>
+__global__ __launch_bounds__(256) void attention_q8_qkv_rows(const uint16_t *__restrict__ qkv, const uint16_t *__restrict__ q_norm,
+                                                            const uint16_t *__restrict__ k_norm, const float *__restrict__ rope_cos,
+                                                            const float *__restrict__ rope_sin, _Float16 *__restrict__ queries,
+                                                            float *__restrict__ qsums, const uint64_t *__restrict__ page_table,
+                                                            uint8_t *__restrict__ pool, AttentionParams p) {
+  qkv_rows_of_head<D>(blockIdx.x, qkv, q_norm, k_norm, rope_cos, rope_sin, queries, qsums, page_table, pool, p);
+}
 SP_REGISTER_KERNEL("attention_q8_qkv_rows_d128", &attention_q8_qkv_rows<128>);
 SP_REGISTER_KERNEL("attention_q8_qkv_rows_d64", &attention_q8_qkv_rows<64>);
+
+// The sum that a wavefront's butterfly over 64 elements gives, of eight lanes that hold eight elements each: lane bits 0, 1 and
+// 2 are the elements' bits 5, 4 and 3, so that the lanes are added first, and what a lane holds last. In all eight lanes.
+__device__ __forceinline__ float sum_of_eights(const float (&v)[8]) {
+  float s[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) s[i] = dpp_add<kRowHalfMirror>(dpp_add<kQuadSwap2>(dpp_add<kQuadSwap1>(v[i])));
+  return ((s[0] + s[4]) + (s[2] + s[6])) + ((s[1] + s[5]) + (s[3] + s[7]));
+}
+// The same where a row's vectors are whole (rotary pairs a multiple of eight, sixteen-byte rows, weights and tables): a query
+// head's row is D / 8 lanes of eight elements, so that a sum is three steps between lanes for several rows at once, loads and
+// stores are sixteen bytes, and a row's cosines and sines serve kHeads heads. Grid (groups of query heads, then the key heads,
+// sequences): a key head's workgroup is attention_q8_qkv_rows'. Every byte is the same. A row a wave spent its time in its sums'
+// steps, a square root and a division for 128 values: 2048 rows of 64 / 8 heads 68.4 us so and 42.8 here, 777 33.0 and 20.7.
+template <int D>
+__global__ __launch_bounds__(256) void attention_q8_qkv_vectors(const uint16_t *__restrict__ qkv, const uint16_t *__restrict__ q_norm,
+                                                               const uint16_t *__restrict__ k_norm, const float *__restrict__ rope_cos,
+                                                               const float *__restrict__ rope_sin, _Float16 *__restrict__ queries,
+                                                               float *__restrict__ qsums, const uint64_t *__restrict__ page_table,
+                                                               uint8_t *__restrict__ pool, AttentionParams p) {
+  constexpr uint32_t kLanes = D / 8, kRows = 64 / kLanes, kWaves = 16 / kRows, kHeads = 4, kGroup = kHeads * (4 / kWaves);
+  static_assert(kGroup == ATTENTION_VECTOR_HEADS(D));
+  const uint32_t groups = (p.q_heads + kGroup - 1u) / kGroup;
+  if (blockIdx.x >= groups) {
+    qkv_rows_of_head<D>(p.q_heads + blockIdx.x - groups, qkv, q_norm, k_norm, rope_cos, rope_sin, queries, qsums, page_table, pool, p);
+    return;
+  }
+  __shared__ __align__(16) float normalized[4][kRows][D];
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, z = blockIdx.y, k = lane % kLanes;
+  const AttentionSequence seq = block_sequence<true>(p, z);
+  const uint32_t row = wave % kWaves * kRows + lane / kLanes, firstHead = blockIdx.x * kGroup + wave / kWaves * kHeads, pairs = p.rotary_pairs;
+  const bool live = row < seq.rows;
+  const size_t packed = size_t(seq.first_row) + row;
+  const uint32_t d = 64u * (k >> 3) + 32u * (k & 1u) + 8u * (k & 2u) + 2u * (k & 4u), queryStride = p.gated ? 2u * D : uint32_t(D);
+  const bool turns = d < 2u * pairs;
+  const uint32_t pair = d < pairs ? d : d - pairs;
+  auto vector = [](const uint16_t *from) { return *reinterpret_cast<const uint4 *>(from); };
+  uint4 held[kHeads], weights = make_uint4(0u, 0u, 0u, 0u);
+  float4 cosine[2] = {}, sine[2] = {};
+#pragma unroll
+  for (uint32_t h = 0; h < kHeads; ++h)
+    held[h] = live && firstHead + h < p.q_heads ? vector(qkv + packed * p.qkv_stride + (firstHead + h) * queryStride + d) : weights;
+  if (live && turns) {
+#pragma unroll
+    for (uint32_t i = 0; i < 2; ++i) {
+      cosine[i] = *reinterpret_cast<const float4 *>(rope_cos + packed * pairs + pair + 4u * i);
+      sine[i] = *reinterpret_cast<const float4 *>(rope_sin + packed * pairs + pair + 4u * i);
+    }
+  }
+  if (p.normalize) weights = vector(q_norm + d);
+  auto each = [](const uint4 &v, float (&out)[8]) {
+    const uint32_t words[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      out[2 * i] = bf16_bits_to_float(words[i] & 0xFFFFu);
+      out[2 * i + 1] = bf16_bits_to_float(words[i] >> 16);
+    }
+  };
+  auto sumOf = [&](const float (&v)[8]) {
+    const float mine = sum_of_eights(v);
+    if constexpr (kLanes == 8) return mine;
+    const float other = lane_xor<8>(mine), first = k < 8u ? mine : other, second = k < 8u ? other : mine;
+    return (0.f + first) + second;
+  };
+  const float cosines[8] = {cosine[0].x, cosine[0].y, cosine[0].z, cosine[0].w, cosine[1].x, cosine[1].y, cosine[1].z, cosine[1].w};
+  const float sines[8] = {sine[0].x, sine[0].y, sine[0].z, sine[0].w, sine[1].x, sine[1].y, sine[1].z, sine[1].w};
+  float weight[8], *mine = normalized[wave][lane / kLanes];
+  each(weights, weight);
+#pragma unroll
+  for (uint32_t h = 0; h < kHeads; ++h) {
+    const uint32_t head = firstHead + h, group = p.q_heads / p.kv_heads;
+    if (head >= p.q_heads) break;
+    float result[8];
+    each(held[h], result);
+    if (p.normalize) {
+      float squares[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) squares[i] = result[i] * result[i];
+      const float inverse = 1.0f / sqrtf(sumOf(squares) / float(D) + 1e-6f);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) result[i] = round_bf16(result[i] * inverse * weight[i]);
+    }
+    if (pairs) {
+      wave_lds_fence();
+      reinterpret_cast<float4 *>(mine + d)[0] = make_float4(result[0], result[1], result[2], result[3]);
+      reinterpret_cast<float4 *>(mine + d)[1] = make_float4(result[4], result[5], result[6], result[7]);
+      wave_lds_fence();
+      if (turns) {
+        const float4 *partner = reinterpret_cast<const float4 *>(mine + (d < pairs ? d + pairs : pair));
+        const float4 a = partner[0], b = partner[1];
+        const float others[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          result[i] = d < pairs ? round_bf16(result[i] * cosines[i] - others[i] * sines[i]) : round_bf16(result[i] * cosines[i] + others[i] * sines[i]);
+      }
+    }
+    f16x8 halves;
+    float staged[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      halves[i] = live ? _Float16(result[i]) : _Float16(0.f);
+      staged[i] = float(halves[i]);
+    }
+    const float sum = sumOf(staged);
+    const size_t at = ((size_t(z) * p.kv_heads + head / group) * group + head % group) * 16u + row;
+    *reinterpret_cast<f16x8 *>(queries + at * D + d) = halves;
+    if (k == 0) qsums[at] = live ? sum : 0.f;
+  }
+}
+SP_REGISTER_KERNEL("attention_q8_qkv_vectors_d128", &attention_q8_qkv_vectors<128>);
+SP_REGISTER_KERNEL("attention_q8_qkv_vectors_d64", &attention_q8_qkv_vectors<64>);
 
 // ---------------------------------------------------------------------------------------------
 // attention_q8_split: grid (kv_heads, splits, sequences), 256 threads.

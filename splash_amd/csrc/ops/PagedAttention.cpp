@@ -356,9 +356,15 @@ void PagedAttention::addPromptProjection(hip::CommandGraph &graph, const Attenti
   // A workgroup a block is the faster of the two from about 20 blocks on, and beyond the noise from here: of 64 / 8 heads
   // 31 against 33 us at 32 blocks, 46 against 58 at 64 (24.3 against 24.0 at 16).
   const bool blocks = plan.blocks() >= 32;
-  const hip::DispatchSize grid = blocks ? hip::DispatchSize{g.qHeads + g.kvHeads, plan.blocks(), 1}
-                                    : hip::DispatchSize{g.qHeads + g.kvHeads, ATTENTION_MAXIMUM_ROWS, plan.blocks()};
-  graph.add((blocks ? "attention_q8_qkv_rows" : "attention_q8_qkv_chunk") + kernelSuffix(g),
+  // Its query heads' rows go by whole vectors where they are whole.
+  auto aligned = [](const hip::Buffer &buffer) { return buffer.gpuAddress() % 16 == 0; };
+  const bool vectors = blocks && g.rotaryPairs % 8 == 0 && g.packedWidth() % 8 == 0 && aligned(b.qkv) && aligned(w.queries) &&
+                       (!g.normalize || aligned(b.queryNorm)) && (!g.rotaryPairs || (aligned(b.ropeCos) && aligned(b.ropeSin)));
+  const uint32_t perGroup = ATTENTION_VECTOR_HEADS(g.headDimension);
+  const hip::DispatchSize grid = vectors  ? hip::DispatchSize{(g.qHeads + perGroup - 1) / perGroup + g.kvHeads, plan.blocks(), 1}
+                                 : blocks ? hip::DispatchSize{g.qHeads + g.kvHeads, plan.blocks(), 1}
+                                          : hip::DispatchSize{g.qHeads + g.kvHeads, ATTENTION_MAXIMUM_ROWS, plan.blocks()};
+  graph.add((vectors ? "attention_q8_qkv_vectors" : blocks ? "attention_q8_qkv_rows" : "attention_q8_qkv_chunk") + kernelSuffix(g),
             {b.qkv, g.normalize ? b.queryNorm : spare, g.normalize ? b.keyNorm : spare, g.rotaryPairs ? b.ropeCos : spare,
              g.rotaryPairs ? b.ropeSin : spare, w.queries, w.querySums, pages.pageTable, pages.pool},
             params, grid, {blocks ? 256u : g.headDimension, 1, 1});

@@ -384,6 +384,43 @@ def test_slots_tables_by_the_tile_are_those_by_the_row(backend, K, kind):
     assert np.array_equal(got[0], got[1]) and (got[0] != 0xA5).any()
 
 
+# head counts that end inside a workgroup's group of heads, every kind of rotation, a ragged last block
+@pytest.mark.parametrize("geometry,pairs,gated,normalize", [((64, 8, 128), 64, False, True), ((6, 2, 128), 32, True, True), ((3, 1, 128), 0, False, True),
+                                                            ((8, 8, 128), 8, True, False), ((16, 8, 64), 32, False, True), ((9, 3, 64), 24, True, True)])
+def test_a_chunks_heads_by_vectors_are_those_by_rows(backend, geometry, pairs, gated, normalize):
+    """attention_q8_qkv_vectors leaves the bytes of attention_q8_qkv_rows: queries, their sums, keys, values and scales, with
+    rows of zeros, of large values and of an infinity and a NaN."""
+    q_heads, kv_heads, D = geometry
+    print(f"case heads by vectors {geometry} pairs={pairs} gated={gated} normalize={normalize}", flush=True)
+    rng = np.random.default_rng(q_heads + pairs)
+    tokens, committed, first = 45, 250, 3
+    blocks = -(-tokens // 16)
+    width = ((2 if gated else 1) * q_heads + 2 * kv_heads) * D
+    qkv = orc.f32_to_bf16(rng.standard_normal((first + tokens, width)).astype(np.float32) * 2)
+    qkv[first + 1] = 0
+    qkv[first + 2] = orc.f32_to_bf16(np.full(width, 2.0 ** 60, np.float32))
+    qkv[first + 3, 5], qkv[first + 4, D - 1] = 0x7F80, 0x7FC0    # (of the first query head: a key head's scale is a comparison)
+    weights = [orc.f32_to_bf16((1 + 0.1 * rng.standard_normal(D)).astype(np.float32)) for _ in range(2)]
+    angles = rng.uniform(0, 6.28, (first + tokens, max(pairs, 1))).astype(np.float32)
+    inputs = [backend.from_array(a) for a in (qkv, *weights, np.cos(angles), np.sin(angles))]
+    pages = -(-(committed + tokens) // ops.PAGE_TOKENS)
+    table = backend.from_array(rng.permutation(pages).astype(np.uint64))
+    p = AttentionParams(q_heads, kv_heads, D, pairs, normalize, width, 1, blocks, 0, gated, 0, tokens, ops.kv_page_bytes(kv_heads, D))
+    s = p.sequence[0]
+    s.first_row, s.committed, s.table_first, s.rows, s.steps_per_split = first, committed, 0, 16, 1
+    got = []
+    for name, grid in (("rows", q_heads + kv_heads), ("vectors", -(-q_heads // (512 // D)) + kv_heads)):
+        out = [backend.from_array(np.full(n, 0xA5, np.uint8)) for n in (blocks * q_heads * 16 * D * 2, blocks * q_heads * 16 * 4, pages * p.page_bytes)]
+        graph = splash_amd.CommandGraph()
+        graph.add(f"attention_q8_qkv_{name}_d{D}", [*inputs, *out[:2], table, out[2]], p, (grid, blocks, 1))
+        backend.run(graph)
+        queries, sums, pool = out[0].download(np.uint16).copy(), out[1].download(np.uint32).copy(), out[2].download()
+        for values, low, mask in ((queries, 0x7C00, 0x7FFF), (sums, 0x7F800000, 0x7FFFFFFF)):    # (one NaN is as good as another)
+            values[(values & mask) > low] = low + 1
+        got.append((queries, sums, pool))
+    assert all(np.array_equal(a, b) for a, b in zip(*got))
+
+
 @pytest.mark.parametrize("geometry,tokens,committed,gated", [((64, 8, 128), 200, 300, False), ((64, 8, 128), 53, 0, True), ((32, 8, 128), 200, 250, True),
                                                              ((32, 8, 128), 64, 1000, False), ((16, 8, 64), 200, 300, False), ((16, 8, 64), 37, 700, True)])
 def test_a_chunks_blocks_attend_whole_histories(backend, geometry, tokens, committed, gated):
