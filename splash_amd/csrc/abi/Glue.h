@@ -37,6 +37,15 @@ struct RopeTreeParams {
   uint32_t anchor[8];     // position of the sequence's row 0
 };
 
+// rope_build_chunk_tables: the same of a prompt chunk's rows, blocks of `block_rows` one after the other behind `anchor`
+// tokens, a row's position its block's first plus its depth. Grid (ceil(rows * pairs / 256)), 256 threads.
+struct RopeChunkParams {
+  uint32_t pairs;
+  uint32_t rows;
+  uint32_t anchor;
+  uint32_t block_rows;
+};
+
 // gguf_embed_norm_<fmt>: the embedding, first norm and RoPE tables of a step's rows (kernels/glue.hip).
 struct EmbedNormParams {
   struct GgufEmbedParams embed;

@@ -477,7 +477,6 @@ __device__ __forceinline__ uint32_t logit_key(float value) {
 __device__ __forceinline__ float key_logit(uint32_t key) {
   return __builtin_bit_cast(float, (key & 0x80000000u) ? key & 0x7FFFFFFFu : ~key);
 }
-constexpr uint32_t kLowestKey = 0x007FFFFFu;  // of -infinity
 // A position in the order: the tokens at or before it have a larger key, or its key and an id at
 // most `last`. {0, 0} lies after every token.
 struct OrderEnd {

@@ -495,19 +495,8 @@ void DenseVerify::encodePrefill(hip::CommandGraph &graph, uint32_t tableFirst, u
     ops::AttentionPromptPlan widePlan;
     if (wide) widePlan = ops::PagedAttention::planPrompt(geometry, {0, tokens, committed, tableFirst}, linear_.calibration().computeUnits);
     else plan = ops::PagedAttention::planChunks(geometry, {{0, tokens, committed, tableFirst}}, linear_.calibration().computeUnits);
-    if (dims_.rotaryPairs) {
-      // the RoPE tables eight blocks a dispatch, each dispatch over its own rows of the depths and tables
-      const uint32_t span = ATTENTION_MAXIMUM_SEQUENCES * ATTENTION_MAXIMUM_ROWS;
-      for (uint32_t first = 0; first < tokens; first += span) {
-        const uint32_t count = std::min(span, tokens - first);
-        std::vector<ops::RopeSequence> rope;
-        for (uint32_t at = 0; at < count; at += ATTENTION_MAXIMUM_ROWS)
-          rope.push_back({at, std::min<uint32_t>(ATTENTION_MAXIMUM_ROWS, count - at), committed + first + at});
-        const uint64_t tableBytes = uint64_t{dims_.rotaryPairs} * 4;
-        ops::RoPE::addTreeTables(graph, inverseFrequency_, rowsOf(depths_, first, count, 4), rowsOf(ropeCos_, first, count, tableBytes),
-                                 rowsOf(ropeSin_, first, count, tableBytes), dims_.rotaryPairs, rope);
-      }
-    }
+    if (dims_.rotaryPairs)
+      ops::RoPE::addChunkTables(graph, inverseFrequency_, depths_, ropeCos_, ropeSin_, dims_.rotaryPairs, tokens, committed, ATTENTION_MAXIMUM_ROWS);
     encodeEmbedding(graph, tokens);
     // every window is a step's worth of rows at most, so what holds for one holds for all
     const bool feeds = layersFeedNext(std::min(tokens, kWindowRows));

@@ -566,19 +566,8 @@ void HybridVerify::encodePrefill(hip::CommandGraph &graph, uint32_t lane, uint32
   if (wide) widePlan = ops::PagedAttention::planPrompt(geometry, {0, tokens, committed, tableFirst}, linear_.calibration().computeUnits);
   else plan = ops::PagedAttention::planChunks(geometry, {{0, tokens, committed, tableFirst}}, linear_.calibration().computeUnits);
   if (firstLayer == 0) {
-    if (dims_.rotaryPairs) {
-      // the RoPE tables eight blocks a dispatch, each dispatch over its own rows of the depths and tables
-      const uint32_t span = ATTENTION_MAXIMUM_SEQUENCES * ATTENTION_MAXIMUM_ROWS;
-      const uint64_t tableBytes = uint64_t{dims_.rotaryPairs} * 4;
-      for (uint32_t first = 0; first < tokens; first += span) {
-        const uint32_t count = std::min(span, tokens - first);
-        std::vector<ops::RopeSequence> rope;
-        for (uint32_t at = 0; at < count; at += ATTENTION_MAXIMUM_ROWS)
-          rope.push_back({at, std::min<uint32_t>(ATTENTION_MAXIMUM_ROWS, count - at), committed + first + at});
-        ops::RoPE::addTreeTables(graph, inverseFrequency_, rowsOf(depths_, first, count, 4), rowsOf(ropeCos_, first, count, tableBytes),
-                                 rowsOf(ropeSin_, first, count, tableBytes), dims_.rotaryPairs, rope);
-      }
-    }
+    if (dims_.rotaryPairs)
+      ops::RoPE::addChunkTables(graph, inverseFrequency_, depths_, ropeCos_, ropeSin_, dims_.rotaryPairs, tokens, committed, ATTENTION_MAXIMUM_ROWS);
     encodeEmbedding(graph, tokens);
   }
   const uint32_t end = layerCount ? firstLayer + layerCount : dims_.layers;

@@ -112,6 +112,18 @@ void RoPE::addTreeTables(hip::CommandGraph &graph, const hip::Buffer &inverseFre
   graph.add("rope_build_tree_tables", {inverseFrequency, depth, cosines, sines}, params, {params.rows, 1, 1}, {pairs, 1, 1});
 }
 
+void RoPE::addChunkTables(hip::CommandGraph &graph, const hip::Buffer &inverseFrequency, const hip::Buffer &depth,
+                          const hip::Buffer &cosines, const hip::Buffer &sines, uint32_t pairs, uint32_t rows, uint32_t anchor, uint32_t blockRows) {
+  if (!pairs || pairs > 1024) throw std::invalid_argument("RoPE tables take 1 to 1024 pairs");
+  if (!rows || !blockRows) throw std::invalid_argument("RoPE tables of a chunk take blocks of rows");
+  requireBytes(inverseFrequency, uint64_t{pairs} * 4, "RoPE inverse frequencies");
+  requireBytes(depth, uint64_t{rows} * 4, "row depths");
+  requireBytes(cosines, uint64_t{rows} * pairs * 4, "RoPE cosine table");
+  requireBytes(sines, uint64_t{rows} * pairs * 4, "RoPE sine table");
+  graph.add("rope_build_chunk_tables", {inverseFrequency, depth, cosines, sines}, RopeChunkParams{pairs, rows, anchor, blockRows},
+            {(uint64_t{rows} * pairs + 255) / 256, 1, 1}, {256, 1, 1});
+}
+
 void SwiGlu::add(hip::CommandGraph &graph, const hip::Buffer &gate, const hip::Buffer &up, const hip::Buffer &output, uint64_t count) {
   if (!count || count % 8) throw std::invalid_argument("a SwiGLU pass takes whole vectors of eight values");
   requireBytes(gate, count * 2, "SwiGLU gate rows");

@@ -72,6 +72,9 @@ public:
   static void addTreeTables(hip::CommandGraph &graph, const hip::Buffer &inverseFrequency, const hip::Buffer &depth,
                             const hip::Buffer &cosines, const hip::Buffer &sines, uint32_t pairs,
                             const std::vector<RopeSequence> &sequences);
+  // The tables of a prompt chunk: blocks of `blockRows` rows one after the other from position `anchor`, a row `depth` into its own.
+  static void addChunkTables(hip::CommandGraph &graph, const hip::Buffer &inverseFrequency, const hip::Buffer &depth,
+                             const hip::Buffer &cosines, const hip::Buffer &sines, uint32_t pairs, uint32_t rows, uint32_t anchor, uint32_t blockRows);
 };
 
 // Rows of `stride` bf16 values from row `row` of a buffer, of which a copy reads or writes the values

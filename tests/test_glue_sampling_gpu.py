@@ -100,6 +100,31 @@ def test_rope_tree_tables(backend):
     assert np.abs(sin.download(np.float32).reshape(7, pairs) - np.sin(angle)).max() < 2e-6
 
 
+@pytest.mark.parametrize("rows,pairs", [(1, 1), (45, 24), (130, 64), (17, 300)])
+def test_a_chunks_rope_tables_are_its_blocks(backend, rows, pairs):
+    """rope_build_chunk_tables leaves the bits of rope_build_tree_tables over the chunk's blocks, and nothing past its rows."""
+    print(f"case chunk RoPE tables rows={rows} pairs={pairs}", flush=True)
+    import ctypes
+
+    class Chunk(ctypes.Structure):
+        _fields_ = [(n, ctypes.c_uint32) for n in ("pairs", "rows", "anchor", "block_rows")]
+    rng = np.random.default_rng(rows)
+    inv = backend.from_array((1e6 ** (-np.arange(pairs) / pairs)).astype(np.float32))
+    depths = rng.integers(0, 16, rows).astype(np.uint32)
+    depth, anchor = backend.from_array(depths), 32741
+    tables = [[backend.from_array(np.full((rows + 1) * pairs, 7, np.float32)) for _ in range(2)] for _ in range(2)]
+    g = splash_amd.CommandGraph()
+    for first in range(0, rows, 128):    # (eight blocks a dispatch)
+        count = min(128, rows - first)
+        part = lambda buffer, width: buffer.view(first * width * 4, count * width * 4)
+        ops.RoPE.add_tree_tables(g, inv, part(depth, 1), part(tables[0][0], pairs), part(tables[0][1], pairs), pairs,
+                                 [(at, min(16, count - at), anchor + first + at) for at in range(0, count, 16)])
+    g.add("rope_build_chunk_tables", [inv, depth, *tables[1]], Chunk(pairs, rows, anchor, 16), (-(-rows * pairs // 256), 1, 1))
+    backend.run(g)
+    for a, b in zip(*tables):
+        assert np.array_equal(a.download(np.uint32), b.download(np.uint32))
+
+
 def test_row_copy(backend):
     """RowCopy.hpp:17-28: a capture copies a layer's output rows into its slot of wider rows."""
     rng = np.random.default_rng(5)
