@@ -503,8 +503,11 @@ uint64_t Linear::wideTableBytes(uint32_t inputSize, uint32_t rows) noexcept { re
 // fill the device's rounds best, in microseconds. A compute unit holds two workgroups, so `items` workgroups take
 // ceil(items / (2 units)) rounds of 1 / splits of K each; a super-block of a round takes 0.55 for each row tile and for the
 // conversion of its weights as much as 2.2 of them (5.6 measured at eight tiles); parts cost a launch and their partials'
-// trip to memory and back. Where a last round would be far from full, the column groups past the full rounds go in
-// workgroups of four row tiles instead, a second part of the grid that starts as the first one's last workgroups end.
+// trip to memory and back. Where K is whole and a last round would be far from full, the column groups past the full rounds
+// go in workgroups of four row tiles instead, a second part of the grid that starts as the first one's last workgroups end.
+// A tail does not take the place of parts of K, even where it is the faster (2048 rows of 8192 -> 5120: 248 + 20 us in two
+// parts, 212 with a tail): a row's sum over K in one run is rounded otherwise than the sum of its parts, and what shares
+// the work leaves the results as they are.
 Linear::WideSplit Linear::wideSplit(uint32_t columnGroups, uint32_t blocks, uint32_t rows, bool splittable) const noexcept {
   const uint32_t liveTiles = gguf_row_tiles(rows), slots = 2 * calibration_.computeUnits;
   WideSplit chosen{1, GGUF_WIDE_TILES, 1, 0, 0};
@@ -520,6 +523,7 @@ Linear::WideSplit Linear::wideSplit(uint32_t columnGroups, uint32_t blocks, uint
       }
     }
   }
+  if (chosen.splits > 1) return chosen;
   for (uint32_t tallest : {8u, 7u, 6u}) {
     const uint32_t rowGroups = (liveTiles + tallest - 1) / tallest, full = rowGroups * columnGroups / slots;
     const uint32_t tail = full ? columnGroups - full * slots / rowGroups : 0;
