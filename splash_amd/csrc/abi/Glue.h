@@ -7,9 +7,9 @@
 #define SPLASH_RMS_EPSILON 1e-6f
 #define NORM_STAGED_WIDTH 8192u  // columns of a row that a norm holds in LDS
 
-// norm_rms / norm_rms_table16: one workgroup per row, of 256 threads / of norm_row_threads(width). norm_rms_table16 also
-// writes the projection activation table of the normalized rows (abi/Gguf.h), as the reference's
-// norm_rms_table16_decode does for its register tile.
+// norm_rms / norm_rms_table16: one workgroup per row, of 256 threads / of norm_row_threads(width), where 256 threads are
+// right as well. norm_rms_table16 also writes the projection activation table of the normalized rows (abi/Gguf.h), as the
+// reference's norm_rms_table16_decode does for its register tile.
 struct NormParams {
   uint32_t width;
   uint32_t rows;

@@ -152,7 +152,8 @@ struct DraftSelectParams {
 // candidates, none, past its positions). The tree grows best first by estimate, a draft row taking children[l]
 // candidates (a greedy lane's likeliest; a sampled lane's Gumbel-top-k draws from the probabilities at its temperature,
 // with noise[l] as the anchor's key) and a chain row the chain's next token, one row a token path, until it holds
-// DRAFT_TREE_ROWS rows, depth[l] + 1 rows, or nothing no deeper than depth[l] is left. Grid (lanes), 1024 threads.
+// DRAFT_TREE_ROWS rows, depth[l] + 1 rows, or nothing no deeper than depth[l] is left. Grid (lanes), 1024 threads
+// (or 512 or 256).
 #define DRAFT_TREE_ROWS 16u
 #define DRAFT_CHAIN_TOKENS (DRAFT_TREE_ROWS - 1u)
 #define DRAFT_CHAIN_AGREEMENTS 4u

@@ -82,11 +82,11 @@ __global__ __launch_bounds__(kTreeThreads) void draft_select_tree(const uint32_t
 
   // ---- The lattice: sixteen threads, a candidate each, a predecessor (position 0 follows the anchor alone, predecessor 0;
   // what the others compute there is not read); a team of 256 threads every fourth position, its two side by side (one team,
-  // seven positions a thread, took the longer half of the kernel). Sixteen threads share a wavefront, whose LDS operations
-  // are in order, so nothing here waits for the workgroup.
-  {
+  // seven positions a thread, took the longer half of the kernel; a launch of fewer threads has its teams' work done in
+  // turns). Sixteen threads share a wavefront, whose LDS operations are in order, so nothing here waits for the workgroup.
+  for (uint32_t team = tid / kLatticeThreads; team < kTeams; team += max(1u, blockDim.x / kLatticeThreads)) {
     constexpr uint32_t kEach = (kPositions + kTeams - 1u) / kTeams;
-    const uint32_t predecessor = tid % kLatticeThreads / kCandidates, team = tid / kLatticeThreads;
+    const uint32_t predecessor = tid % kLatticeThreads / kCandidates;
     uint32_t positions[kEach];   // (one past the last: not worked, by whole wavefronts)
     float score[kEach], weight[kEach];
 #pragma unroll

@@ -198,8 +198,21 @@ __device__ __forceinline__ void write_norm_vector(uint4 x, uint4 w, float invers
   write_table_vector(bits, row, v, table, width, tiles);
 }
 
+// A row's normalized vectors by a workgroup: a thread's first from its registers (its values and weights), those past it, where
+// the workgroup has fewer threads than the row has vectors, from LDS and memory.
+__device__ __forceinline__ void write_norm_vectors(uint4 mine, uint4 norm, const uint16_t *row_x, const uint16_t *__restrict__ weight, float inverse,
+                                                   bool live, uint32_t row, uint16_t *__restrict__ output, uint8_t *__restrict__ table,
+                                                   uint32_t width, uint32_t tiles) {
+  const uint32_t vectors = width / 8u, first = threadIdx.x;
+  if (first < vectors) write_norm_vector(mine, norm, inverse, live, row, first, output, table, width, tiles);
+  for (uint32_t v = first + blockDim.x; v < vectors; v += blockDim.x) {
+    if (live) norm = reinterpret_cast<const uint4 *>(weight)[v];
+    write_norm_vector(reinterpret_cast<const uint4 *>(row_x)[v], norm, inverse, live, row, v, output, table, width, tiles);
+  }
+}
+
 // The same, and the activation table of the normalized rows: grid (tiles * 16) so that the rows past the live ones are
-// written as zeros, norm_row_threads(width) threads. A handful of workgroups that only wait, so what counts is the chain one
+// written as zeros, norm_row_threads(width) threads (any whole wavefronts from 256 threads on are right). A handful of workgroups that only wait, so what counts is the chain one
 // thread runs: a row of up to kStagedWidth columns has a thread a vector of eight, which holds it and its weights in
 // registers from the load to the stores, and LDS serves the sum alone. (8 rows of 5120: 7.4 us by 256 threads, 4.3 so; 128 of
 // 2048: 6.0 and 5.6.)
@@ -211,16 +224,19 @@ __global__ __launch_bounds__(1024) void norm_rms_table16(const uint16_t *__restr
   const bool live = row < p.rows;
   const uint16_t *x = input + size_t(live ? row : 0) * p.width;
   if (p.width <= kStagedWidth) {  // the width is a multiple of 256
-    const uint32_t v = threadIdx.x;
+    const uint32_t vectors = p.width / 8u, first = threadIdx.x;
     uint4 mine = make_uint4(0u, 0u, 0u, 0u), norm = mine;
-    if (live && v < p.width / 8u) {
-      mine = reinterpret_cast<const uint4 *>(x)[v];
-      norm = reinterpret_cast<const uint4 *>(weight)[v];
-      reinterpret_cast<uint4 *>(rowX)[v] = mine;
+    if (live) {
+      if (first < vectors) {
+        mine = reinterpret_cast<const uint4 *>(x)[first];
+        norm = reinterpret_cast<const uint4 *>(weight)[first];
+        reinterpret_cast<uint4 *>(rowX)[first] = mine;
+      }
+      for (uint32_t v = first + blockDim.x; v < vectors; v += blockDim.x) reinterpret_cast<uint4 *>(rowX)[v] = reinterpret_cast<const uint4 *>(x)[v];
     }
     __syncthreads();
     const float inverse = live ? rms_inverse(rowX, p.width, scratch) : 0.f;
-    if (v < p.width / 8u) write_norm_vector(mine, norm, inverse, live, row, v, output, table, p.width, p.tiles);
+    write_norm_vectors(mine, norm, rowX, weight, inverse, live, row, output, table, p.width, p.tiles);
   } else {
     const float inverse = live ? rms_inverse(x, p.width, scratch) : 0.f;
     write_table_row(x, weight, inverse, live, row, output, table, p.width, p.tiles);
@@ -231,12 +247,13 @@ SP_REGISTER_KERNEL("norm_rms_table16", &norm_rms_table16);
 // draft_conv (draft_attention.hip) and the pass that reads its rows, a thread a vector of eight channels: a Prepare stage's
 // rows and their activation table, grid (tiles * 16, the row's vectors by 64), 64 threads, since nothing there needs the
 // row's other channels; a Residual stage's rows, their RMS norm (of `norm_weight`, into `normalized`) and its table, a
-// workgroup of norm_row_threads(width) a row. Each convolution was a launch of its own before a launch of as few workgroups.
+// workgroup of norm_row_threads(width) a row. (A launch of fewer threads, of the one any, of the other whole 256, takes its
+// vectors in turns.) Each convolution was a launch of its own before a launch of as few workgroups.
 // 8 rows of 5120, inside a draft model's pass: 3.1 us (a workgroup of 256 a row, 5.3) and 4.7 (8.3).
 // Values and their order are the two kernels'. The rows' 16-byte accesses are the host's rule
 // (DraftAttention::addConvolutionTable).
 template <bool Residual>
-__global__ __launch_bounds__(Residual ? 1024 : 64) void draft_conv_table(
+__global__ __launch_bounds__(Residual ? 1024 : 256) void draft_conv_table(
     const uint16_t *__restrict__ input, const uint16_t *__restrict__ dynamic, const uint16_t *__restrict__ base,
     const uint16_t *__restrict__ residual, const uint16_t *__restrict__ norm_weight, uint16_t *__restrict__ output,
     uint16_t *__restrict__ normalized, uint8_t *__restrict__ table, DraftConvTableParams p) {
@@ -244,20 +261,21 @@ __global__ __launch_bounds__(Residual ? 1024 : 64) void draft_conv_table(
   __shared__ float scratch[4];
   __shared__ __align__(16) uint16_t rowX[Residual ? kStagedWidth : 8];
   const uint32_t row = blockIdx.x, width = p.hidden, vectors = width / 8u, groups = width / DRAFT_CONVOLUTION_GROUP;
-  const uint32_t v = Residual ? threadIdx.x : blockIdx.y * 64u + threadIdx.x;
+  const uint32_t start = Residual ? threadIdx.x : blockIdx.y * blockDim.x + threadIdx.x, step = Residual ? blockDim.x : gridDim.y * blockDim.x;
   const bool live = row < p.rows;
-  uint4 packed = make_uint4(0u, 0u, 0u, 0u), norm = packed;
-  if (live && v < vectors) {
+  uint4 norm = make_uint4(0u, 0u, 0u, 0u);
+  auto convolve = [&](uint32_t v) __attribute__((always_inline)) {
     const bool follows = row % DRAFT_ATTENTION_QUERY_ROWS > 0;   // a lane's first row has none before it
     const size_t before = row - (follows ? 1u : 0u);
     const uint16_t *mine = dynamic + size_t(row) * draft_dynamic_width(width) + (Residual ? DRAFT_CONVOLUTION_TAPS : 0u) * groups;
     const uint16_t *taps = base + (Residual ? DRAFT_CONVOLUTION_TAPS : 0u) * size_t(width);
     auto vector = [&](const uint16_t *from) { return reinterpret_cast<const uint4 *>(from)[v]; };
     uint4 now = vector(input + size_t(row) * width), last = vector(input + before * width), tap0 = vector(taps), tap1 = vector(taps + width);
-    uint4 added = packed;
+    uint4 added = make_uint4(0u, 0u, 0u, 0u);
     if constexpr (Residual) added = vector(residual + size_t(row) * width);
     uint32_t dynamic0 = mine[v / (DRAFT_CONVOLUTION_GROUP / 8u)], dynamic1 = mine[groups + v / (DRAFT_CONVOLUTION_GROUP / 8u)];
-    if constexpr (Residual) norm = vector(norm_weight);
+    if constexpr (Residual)
+      if (v == start) norm = vector(norm_weight);
     arrived(now);
     arrived(last);
     arrived(tap0);
@@ -275,17 +293,22 @@ __global__ __launch_bounds__(Residual ? 1024 : 64) void draft_conv_table(
     auto pair = [&](uint32_t x, uint32_t y, uint32_t t0, uint32_t t1, uint32_t a) {
       return channel(x & 0xFFFFu, y & 0xFFFFu, t0 & 0xFFFFu, t1 & 0xFFFFu, a & 0xFFFFu) | (channel(x >> 16, y >> 16, t0 >> 16, t1 >> 16, a >> 16) << 16);
     };
-    packed = make_uint4(pair(now.x, last.x, tap0.x, tap1.x, added.x), pair(now.y, last.y, tap0.y, tap1.y, added.y),
-                        pair(now.z, last.z, tap0.z, tap1.z, added.z), pair(now.w, last.w, tap0.w, tap1.w, added.w));
+    const uint4 packed = make_uint4(pair(now.x, last.x, tap0.x, tap1.x, added.x), pair(now.y, last.y, tap0.y, tap1.y, added.y),
+                                    pair(now.z, last.z, tap0.z, tap1.z, added.z), pair(now.w, last.w, tap0.w, tap1.w, added.w));
     reinterpret_cast<uint4 *>(output + size_t(row) * width)[v] = packed;
     if constexpr (Residual) reinterpret_cast<uint4 *>(rowX)[v] = packed;
-  }
+    return packed;
+  };
+  const uint4 none = make_uint4(0u, 0u, 0u, 0u);
   if constexpr (Residual) {
+    const uint4 mine = live && start < vectors ? convolve(start) : none;
+    if (live)
+      for (uint32_t v = start + step; v < vectors; v += step) convolve(v);
     __syncthreads();
     const float inverse = live ? rms_inverse(rowX, width, scratch) : 0.f;
-    if (v < vectors) write_norm_vector(packed, norm, inverse, live, row, v, normalized, table, width, p.tiles);
-  } else if (v < vectors) {
-    write_table_vector(packed, row, v, table, width, p.tiles);
+    write_norm_vectors(mine, norm, rowX, norm_weight, inverse, live, row, normalized, table, width, p.tiles);
+  } else {
+    for (uint32_t v = start; v < vectors; v += step) write_table_vector(live ? convolve(v) : none, row, v, table, width, p.tiles);
   }
 }
 SP_REGISTER_KERNEL("draft_conv_table", &draft_conv_table<false>);
@@ -530,10 +553,8 @@ __global__ __launch_bounds__(1024) void gguf_embed_norm(const uint8_t *__restric
   }
   __syncthreads();
   const float inverse = live ? rms_inverse(rowX, p.embed.hidden, scratch) : 0.f;
-  for (uint32_t v = tid; v < vectors; v += threads) {   // (once where the host's rule gives the threads)
-    if (live && v != tid) norm = reinterpret_cast<const uint4 *>(weight)[v];
-    write_norm_vector(reinterpret_cast<const uint4 *>(rowX)[v], norm, inverse, live, row, v, output, table, p.embed.hidden, p.tiles);
-  }
+  const uint4 mine = reinterpret_cast<const uint4 *>(rowX)[min(tid, vectors - 1u)];
+  write_norm_vectors(mine, norm, rowX, weight, inverse, live, row, output, table, p.embed.hidden, p.tiles);
 }
 SP_REGISTER_KERNEL("gguf_embed_norm_q4k", &gguf_embed_norm<GGUF_FMT_Q4K>);
 SP_REGISTER_KERNEL("gguf_embed_norm_q6k", &gguf_embed_norm<GGUF_FMT_Q6K>);
