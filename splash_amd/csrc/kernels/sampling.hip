@@ -453,7 +453,8 @@ __device__ __forceinline__ Mass row_mass(const float *masses, uint32_t row, floa
   const uint32_t shard = (threadIdx.x & 63u) % SAMPLING_SHARDS;
   const float2 mine = reinterpret_cast<const float2 *>(masses)[row * SAMPLING_SHARDS + shard];
   const float maximum = wave_max(mine.x);
-  const float sum = mine.x == -INFINITY ? 0.f : mine.y * expf((mine.x - maximum) * inverse);
+  // (a shard at the maximum weighs 1 as it is: of an infinite maximum, or divided by the least temperatures, 0 is no number)
+  const float sum = mine.x == maximum ? mine.y : mine.x == -INFINITY ? 0.f : mine.y * expf((mine.x - maximum) * inverse);
   float total = 0.f;
 #pragma unroll
   for (int s = 0; s < int(SAMPLING_SHARDS); ++s) total += lane_value_of(sum, s);

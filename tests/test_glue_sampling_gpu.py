@@ -457,6 +457,23 @@ def test_distribution_ends_far_from_zero(backend):
     assert checked >= 10
 
 
+def test_a_row_with_an_infinite_logit_has_a_finite_mass(backend):
+    """The row's mass is its shards' at the row's maximum: one shard holds it and weighs 1, the others' tokens nothing. A
+    nucleus that no token's own weight (0 / 0) exceeds keeps the row whole, with that mass."""
+    print("case infinite logit", flush=True)
+    rng = np.random.default_rng(3)
+    V, rows = 5000, 4
+    logits = rng.standard_normal((rows, V)).astype(np.float32)
+    logits[np.arange(rows), [0, 77, 3000, V - 1]] = np.inf
+    draft = np.full((rows, V), 1.0 / V, np.float32)
+    b = sampling_buffers(backend, rows, V, logits, draft, rng.random((rows, 2)).astype(np.float32), np.zeros(rows, np.uint32), ops.chain_tree_rows([rows]))
+    g = splash_amd.CommandGraph()
+    ops.Sampling.add_verify(g, b, V, V, [(0, rows)], [(0.7, 0.0, 0, 0.5)])
+    backend.run(g)
+    words = b["decisions"].download(np.uint32).reshape(rows, 8)
+    assert np.array_equal(words[:, 4].view(np.float32), np.ones(rows, np.float32)) and np.array_equal(words[:, 5], np.full(rows, V))
+
+
 def test_constraint_masks_and_stop_exclusion(backend):
     """TargetRow::admits (sampling.metal:42-46): a constrained lane's rows select only tokens of their mask rows, a lane
     that ignores end-of-sequence never a stop token, greedy or sampled; the other lanes' rows are untouched. The
