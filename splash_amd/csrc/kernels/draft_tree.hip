@@ -84,7 +84,7 @@ __global__ __launch_bounds__(kTreeThreads) void draft_select_tree(const uint32_t
   // what the others compute there is not read); a team of 256 threads every fourth position, its two side by side (one team,
   // seven positions a thread, took the longer half of the kernel; a launch of fewer threads has its teams' work done in
   // turns). Sixteen threads share a wavefront, whose LDS operations are in order, so nothing here waits for the workgroup.
-  for (uint32_t team = tid / kLatticeThreads; team < kTeams; team += max(1u, blockDim.x / kLatticeThreads)) {
+  auto lattice = [&](uint32_t team) __attribute__((always_inline)) {
     constexpr uint32_t kEach = (kPositions + kTeams - 1u) / kTeams;
     const uint32_t predecessor = tid % kLatticeThreads / kCandidates;
     uint32_t positions[kEach];   // (one past the last: not worked, by whole wavefronts)
@@ -152,7 +152,11 @@ __global__ __launch_bounds__(kTreeThreads) void draft_select_tree(const uint32_t
       const float z = slope * logf(q / (1.0f - q)) + p.intercept[lane][position];
       s.estimate[position][predecessor][i] = 1.0f / (1.0f + expf(-z));
     }
-  }
+  };
+  lattice(tid / kLatticeThreads);
+  if (__builtin_expect(blockDim.x < kTreeThreads, 0))
+    for (uint32_t team = tid / kLatticeThreads + max(1u, blockDim.x / kLatticeThreads); team < kTeams; team += max(1u, blockDim.x / kLatticeThreads))
+      lattice(team);
   __syncthreads();
   if (tid >= 64u) return;
 

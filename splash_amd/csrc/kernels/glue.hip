@@ -261,7 +261,7 @@ __global__ __launch_bounds__(Residual ? 1024 : 256) void draft_conv_table(
   __shared__ float scratch[4];
   __shared__ __align__(16) uint16_t rowX[Residual ? kStagedWidth : 8];
   const uint32_t row = blockIdx.x, width = p.hidden, vectors = width / 8u, groups = width / DRAFT_CONVOLUTION_GROUP;
-  const uint32_t start = Residual ? threadIdx.x : blockIdx.y * blockDim.x + threadIdx.x, step = Residual ? blockDim.x : gridDim.y * blockDim.x;
+  const uint32_t start = Residual ? threadIdx.x : blockIdx.y * 64u + threadIdx.x;
   const bool live = row < p.rows;
   uint4 norm = make_uint4(0u, 0u, 0u, 0u);
   auto convolve = [&](uint32_t v) __attribute__((always_inline)) {
@@ -303,12 +303,15 @@ __global__ __launch_bounds__(Residual ? 1024 : 256) void draft_conv_table(
   if constexpr (Residual) {
     const uint4 mine = live && start < vectors ? convolve(start) : none;
     if (live)
-      for (uint32_t v = start + step; v < vectors; v += step) convolve(v);
+      for (uint32_t v = start + blockDim.x; v < vectors; v += blockDim.x) convolve(v);
     __syncthreads();
     const float inverse = live ? rms_inverse(rowX, width, scratch) : 0.f;
     write_norm_vectors(mine, norm, rowX, norm_weight, inverse, live, row, normalized, table, width, p.tiles);
   } else {
-    for (uint32_t v = start; v < vectors; v += step) write_table_vector(live ? convolve(v) : none, row, v, table, width, p.tiles);
+    // (64 vectors a workgroup and turn, whatever its threads: more of them than 64 do the next turn's again)
+    if (start < vectors) write_table_vector(live ? convolve(start) : none, row, start, table, width, p.tiles);
+    for (uint32_t v = start + 64u * gridDim.y; v < vectors; v += 64u * gridDim.y)
+      write_table_vector(live ? convolve(v) : none, row, v, table, width, p.tiles);
   }
 }
 SP_REGISTER_KERNEL("draft_conv_table", &draft_conv_table<false>);
