@@ -17,11 +17,14 @@ class Embed(ctypes.Structure):
         ("first_row", U32 * 8), ("row_count", U32 * 8), ("anchor", U32 * 8)]
 
 
-# one super-block; a step's rows; a second row tile; the widest row a workgroup holds, without rotary pairs; more pairs than threads
-@pytest.mark.parametrize("rows,hidden,pairs", [(1, 256, 32), (16, 5120, 64), (17, 2304, 1), (33, 8192, 0), (5, 1024, 300)])
+# one super-block; a step's rows; a second row tile; the widest row a workgroup holds, without rotary pairs; more pairs than
+# threads; a last wave half filled with vectors. By the threads that a step's entry has, and by 256.
+@pytest.mark.parametrize("threads", ["the entry's", 256])
+@pytest.mark.parametrize("rows,hidden,pairs", [(1, 256, 32), (16, 5120, 64), (17, 2304, 1), (33, 8192, 0), (5, 1024, 300), (3, 768, 64)])
 @pytest.mark.parametrize("fmt", ops.FORMATS)
-def test_gather_norm_and_rope_tables_in_one_pass(backend, fmt, rows, hidden, pairs):
-    print(f"case entry fmt={fmt} rows={rows} hidden={hidden} pairs={pairs}", flush=True)
+def test_gather_norm_and_rope_tables_in_one_pass(backend, fmt, rows, hidden, pairs, threads):
+    threads = min(hidden, 1024) if threads != 256 else threads
+    print(f"case entry fmt={fmt} rows={rows} hidden={hidden} pairs={pairs} threads={threads}", flush=True)
     vocabulary = 40
     rng = np.random.default_rng(rows)
     table = backend.from_array(orc.make_native(fmt, vocabulary, hidden, 3))
@@ -46,7 +49,7 @@ def test_gather_norm_and_rope_tables_in_one_pass(backend, fmt, rows, hidden, pai
     for i, (first, count, anchor) in enumerate(sequences):
         p.first_row[i], p.row_count[i], p.anchor[i] = first, count, anchor
     graph.add(name.replace("gguf_embed_", "gguf_embed_norm_"), [table, tokens, weight, *together[:3], inverse, depth, *together[3:]], p,
-              (tiles * 16, 2 if pairs else 1, 1), (256, 1, 1))
+              (tiles * 16, 2 if pairs else 1, 1), (threads, 1, 1))
     backend.run(graph)
     for a, b in zip(apart, together):
         assert np.array_equal(a.download(), b.download())

@@ -355,10 +355,10 @@ def test_a_wide_chunks_stages_are_as_close_to_64_bits_as_the_steps(backend, toke
         assert b <= 1.03 * a and worst_b <= 1.5 * worst_a, stage
 
 
-@pytest.mark.parametrize("tokens,experts,q_heads,kv_heads", [(300, 80, 8, 2), (784, 0, 32, 8)])
+@pytest.mark.parametrize("tokens,experts,q_heads,kv_heads", [(300, 80, 8, 2), (300, 16, 8, 2), (784, 0, 32, 8)])
 def test_a_wide_hybrid_chunk_layer_by_layer(backend, tokens, experts, q_heads, kv_heads):
     """HybridVerify::encodeWidePrefillLayer against the oracle from the GPU's own layer input, every row: a mixture whose
-    routes take two windows, with a shared expert; gated attention over whole histories (784 rows of eight KV heads)."""
+    routes take two windows, with a shared expert, a few tiles an expert and (16 experts) tasks of the tallest; gated attention over whole histories (784 rows of eight KV heads)."""
     from tests.hybrid_reference import HybridModel
     from tests.test_hybrid_step_gpu import close_bf16, sure_routes, ulps
     print(f"case wide hybrid layers tokens={tokens} experts={experts}", flush=True)
@@ -383,6 +383,7 @@ def test_a_wide_hybrid_chunk_layer_by_layer(backend, tokens, experts, q_heads, k
         graph = gpu.encode_prefill(0, 0, committed, tokens, parity=0, first_layer=layer, layer_count=1)
         names = graph.kernels()
         assert any("gguf_wide_moe" in name for name in names) == bool(experts) and any("gguf_wide_q" in name for name in names)
+        assert sum("gguf_wide_moe" in name and "_t8_" in name for name in names) == (2 if experts == 16 else 0), names
         assert any("attention_q8_whole" in name for name in names) == (model.attends(layer) and tokens == 784)
         backend.run(graph)
         packed = model.oracle_mixer_input(before, layer)

@@ -285,7 +285,8 @@ def skewed(rng, routes, experts):
     return selected
 
 
-@pytest.mark.parametrize("rows,top_k,experts,T", [(1, 1, 2, 2), (256, 8, 128, 4), (257, 8, 128, 5), (640, 9, 80, 5), (2048, 9, 129, 5), (2048, 16, 256, 4)])
+@pytest.mark.parametrize("rows,top_k,experts,T", [(1, 1, 2, 2), (256, 8, 128, 4), (257, 8, 128, 5), (640, 9, 80, 5), (2048, 9, 129, 5), (2048, 16, 256, 4),
+                                                  (2048, 8, 128, 8)])
 def test_a_chunks_routes_are_placed_across_windows(backend, rows, top_k, experts, T):
     """One window of 2048 routes, one route more, several, the last one short: every route's slot follows those of the windows
     before it, an expert's slots are whole tiles, its tasks even."""
@@ -304,13 +305,16 @@ def test_a_chunks_routes_are_placed_across_windows(backend, rows, top_k, experts
 def test_expert_tiles_lie_in_the_interval(backend, name, T):
     """The experts' projections over gathered rows and over the slots' own, tasks of every height up to T, two windows of
     routes, columns that end inside a column group: each slot's row in the interval of its row through its expert."""
-    fmt, K, N, experts, top_k, rows = FORMATS[name], 512, 272, 6, 3, 700
+    fmt, K, N, experts, top_k, rows = FORMATS[name], 512, 272, T + 2, 3, 700
     print(f"case wide experts {name} T={T}", flush=True)
     rng = np.random.default_rng(T)
     routes = rows * top_k
-    selected = skewed(rng, routes, experts)
+    # an expert of each height, its last tile short; one without a row; one of many tasks with the routes left
+    counts = [16 * height - int(rng.integers(0, 16)) for height in range(1, T + 1)] + [0]
+    selected = rng.permutation(np.repeat(np.arange(experts), counts + [routes - sum(counts)]))
     b = place(backend, selected, experts, top_k, T)
     route_slot, slot_row, tasks, live = expected_places(selected, experts, top_k, T)
+    assert set(tasks[:, 2]) == set(range(1, T + 1)) and len(tasks) >= T + 3
     tiles = routes // 16 + experts
     gate, up = ([orc.make_native(fmt, N, K, seed + e) for e in range(experts)] for seed in (1, 50))
     image_of = lambda natives: backend.from_array(np.concatenate([ops.pack_gguf_image(fmt, n, N, K) for n in natives]))
@@ -355,6 +359,19 @@ def test_expert_tiles_lie_in_the_interval(backend, name, T):
 def test_expert_tiles_of_tall_tasks_lie_in_the_interval(backend, name):
     """The same of tasks of up to eight row tiles, whose kernels hold a body for each height of four and more."""
     test_expert_tiles_lie_in_the_interval(backend, name, 8)
+
+
+def test_the_conversion_to_bf16_is_the_integer_rule(backend):
+    """Round to nearest even of every upper half with lower halves at a tie and beside it, at the ends and between: zeros,
+    subnormals, every exponent's carries, the overflow to infinity, infinities and NaN payloads."""
+    print("case bf16 conversion", flush=True)
+    lower = np.array([0, 1, 0x4000, 0x7FFF, 0x8000, 0x8001, 0xC000, 0xFFFF], np.uint32)
+    values = ((np.arange(1 << 16, dtype=np.uint32) << 16)[:, None] | lower).view(np.float32)
+    out = backend.allocate_buffer(values.size * 2)
+    graph = splash_amd.CommandGraph()
+    graph.add("gguf_wide_reduce_a", [backend.from_array(values), out, out], ReduceParams(*values.shape, 1, 0), (values.size // 1024, 1, 1))
+    backend.run(graph)
+    assert np.array_equal(out.download(np.uint16), orc.f32_to_bf16(values).ravel())
 
 
 # half a wave's piece, one and a half, three and a half, and the four that a wave holds
