@@ -191,6 +191,9 @@ __global__ __launch_bounds__(256) void gguf_wide_moe_table(const uint16_t *__res
 // store; the tile's are 1 KB. In LDS a line's sixteen places are turned by its number, or the lanes of a row's store would all
 // meet in the same four banks. 16384 slots and what fills their tiles: 2048 gathered inputs 32.5 us by the row, 34.1 by a wave
 // a row without the tile, 28.1 so (5 TB/s of rows read and tables written); 768 of the slots' own 24.3, 16.9 and 16.1.
+// Up to 2048 inputs, of which two workgroups fit a compute unit: with LDS for 4096 (144 KB, one a unit) 17408 gathered slots
+// took 35.7 us of 2048 inputs (27.2 so), 43.2 of 2304 and 64.4 of 4096 where the rows' kernel takes 35.8 and 56.7. (4096 slots
+// of 2304 11.4 for 12.2; the slots' own rows past 3072 inputs, 17408 of 3584, 58 for 84: not built for.)
 template <bool Gathers>
 __global__ __launch_bounds__(1024) void gguf_wide_moe_tile(const uint16_t *__restrict__ input, const uint32_t *__restrict__ slot_row,
                                                            const uint32_t *__restrict__ tile_total, uint8_t *__restrict__ table,

@@ -353,8 +353,11 @@ void PagedAttention::addPromptProjection(hip::CommandGraph &graph, const Attenti
   requireBytes(w.querySums, need.querySums, "staged query sums");
   requirePromptPages(plan, params, pages);
   const hip::Buffer &spare = b.qkv;
-  // A workgroup a block is the faster of the two from about 20 blocks on, and beyond the noise from here: of 64 / 8 heads
-  // 31 against 33 us at 32 blocks, 46 against 58 at 64 (24.3 against 24.0 at 16).
+  // A workgroup a row takes what its rows do, a workgroup a block at least the chain of its sixteen rows. us at 16, 32 and 64
+  // blocks, by the row, by blocks and by blocks whose heads go by vectors: 64 / 8 heads of 128 13.2, 13.3, 11.1; 22.3, 20.3,
+  // 13.0; 43.6, 35.3, 20.3. 32 / 4 of 128: 8.5, 11.5, 10.2; 13.4, 13.2, 11.2; 22.6, 20.7, 13.3. 16 / 8 of 64: 4.9, 7.2, 7.1;
+  // 6.9, 7.9, 8.3; 10.6, 10.7, 10.1. The line is where blocks without vectors are the faster for heads of 128; those by
+  // vectors are from 12 (64 / 8) or 24 blocks (32 / 4) on.
   const bool blocks = plan.blocks() >= 32;
   // Its query heads' rows go by whole vectors where they are whole.
   auto aligned = [](const hip::Buffer &buffer) { return buffer.gpuAddress() % 16 == 0; };
