@@ -20,6 +20,7 @@
 #include "abi/Moe.h"
 #include "backend/KernelRegistry.hpp"
 #include "kernels/gguf_records.hpp"
+#include <type_traits>
 
 namespace splash::kernels {
 
@@ -200,71 +201,67 @@ __device__ __forceinline__ void scaled_groups(f32x4 (&acc)[RT], Dot dot, Scale s
   }
 }
 
+// What a record's scales and constant terms are made of. A step is a group, of Q6_K half a group (16 inputs under one scale).
+template <uint32_t FMT> struct RecordTerms {
+  static constexpr uint32_t kSteps = FMT == GGUF_FMT_Q6K ? 16 : 8;
+  static constexpr uint32_t kConstants = FMT == GGUF_FMT_Q6K ? 4 : 2;   // K = 4 MFMAs of the rows' sums
+  Q4KScales sc{};
+  float d6 = 0.f;
+  __device__ __forceinline__ explicit RecordTerms(const Record<FMT> &rec) {
+    if constexpr (FMT == GGUF_FMT_Q4K || FMT == GGUF_FMT_Q5K) sc = q4k_scales(rec.meta);
+    if constexpr (FMT == GGUF_FMT_Q6K) d6 = half_bits_to_float(rec.d);
+  }
+  // The coefficient of the sums of groups 4 j + kq (Q6_K: of 16-input blocks 4 j + kq).
+  __device__ __forceinline__ float constant(const Record<FMT> &rec, uint32_t j, uint32_t kq) const {
+    if constexpr (FMT == GGUF_FMT_Q4K || FMT == GGUF_FMT_Q5K) {
+      // m - 128 s
+      const float s = sc.d * byte_of(j == 0 ? sc.sc_lo : sc.sc_hi, kq);
+      return __fmaf_rn(-128.f, s, -(sc.dmin * byte_of(j == 0 ? sc.mn_lo : sc.mn_hi, kq)));
+    } else if constexpr (FMT == GGUF_FMT_Q6K) {
+      // -160 d sc (operand 128 + q, value q - 32)
+      const uint32_t word = j == 0 ? rec.scales.x : j == 1 ? rec.scales.y : j == 2 ? rec.scales.z : rec.scales.w;
+      return -160.f * (d6 * float(int(int8_t((word >> (8u * kq)) & 0xFFu))));
+    } else if constexpr (FMT == GGUF_FMT_IQ4XS) {
+      return -128.f * iq4xs_scale(rec.meta, 4u * j + kq);   // one scale a group; the operands' 128 leaves through the row sums
+    } else {
+      const uint32_t first = j == 0 ? rec.scales.x : rec.scales.z, second = j == 0 ? rec.scales.y : rec.scales.w;
+      const uint32_t word = kq == 0 ? first : kq == 1 ? first >> 16 : kq == 2 ? second : second >> 16;
+      return -128.f * half_bits_to_float(word & 0xFFFFu);
+    }
+  }
+  __device__ __forceinline__ float scale(const Record<FMT> &rec, uint32_t step) const {
+    if constexpr (FMT == GGUF_FMT_Q4K || FMT == GGUF_FMT_Q5K) return sc.d * byte_of(step < 4 ? sc.sc_lo : sc.sc_hi, step & 3u);
+    else if constexpr (FMT == GGUF_FMT_Q6K) return d6 * q6_scale(rec.scales, step);
+    else return group_scale(rec, step);
+  }
+  // A step's product of a row tile's operand of its group with the column tile's.
+  static __device__ __forceinline__ f32x4 product(uint32_t step, const uint4 &av, const uint4 &bv) {
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (FMT == GGUF_FMT_Q6K) {
+      const uint2 bw = step & 1u ? make_uint2(bv.z, bv.w) : make_uint2(bv.x, bv.y);
+      const uint2 aw = step & 1u ? make_uint2(av.z, av.w) : make_uint2(av.x, av.y);
+      return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, aw), __builtin_bit_cast(s16x4, bw), zero, 0, 0, 0);
+    } else {
+      return __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(av), as_bf16x8(bv), zero, 0, 0, 0);
+    }
+  }
+};
 template <uint32_t FMT, int RT>
 __device__ __forceinline__ void accumulate_record(const Record<FMT> &rec, const uint4 (*a)[8][64], const float (*sums)[4][64],
                                                   f32x4 (&acc)[RT], uint32_t lane, uint32_t kq) {
   uint4 ops[8];
   record_operands(rec, ops);
-  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-  if constexpr (FMT == GGUF_FMT_Q80 || FMT == GGUF_FMT_IQ4XS || FMT == GGUF_FMT_IQ4NL) {
-    // One scale a group; the operands' 128 leaves through the row sums: -128 s of groups kq and 4 + kq.
-    float s[8];
+  const RecordTerms<FMT> terms(rec);
 #pragma unroll
-    for (uint32_t g = 0; g < 8; ++g) s[g] = group_scale(rec, g);
-    float c_lo, c_hi;
-    if constexpr (FMT == GGUF_FMT_IQ4XS) {
-      c_lo = -128.f * iq4xs_scale(rec.meta, kq);
-      c_hi = -128.f * iq4xs_scale(rec.meta, 4u + kq);
-    } else {
-      const uint32_t lowWord = kq == 0 ? rec.scales.x : kq == 1 ? rec.scales.x >> 16 : kq == 2 ? rec.scales.y : rec.scales.y >> 16;
-      const uint32_t highWord = kq == 0 ? rec.scales.z : kq == 1 ? rec.scales.z >> 16 : kq == 2 ? rec.scales.w : rec.scales.w >> 16;
-      c_lo = -128.f * half_bits_to_float(lowWord & 0xFFFFu);
-      c_hi = -128.f * half_bits_to_float(highWord & 0xFFFFu);
-    }
+  for (uint32_t j = 0; j < RecordTerms<FMT>::kConstants; ++j) {
+    const float coefficient = terms.constant(rec, j, kq);
 #pragma unroll
-    for (int t = 0; t < RT; ++t) {
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(sums[t][0][lane], c_lo, acc[t], 0, 0, 0);
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(sums[t][1][lane], c_hi, acc[t], 0, 0, 0);
-    }
-    scaled_groups<RT, 8>(acc, [&](uint32_t g, int t) {
-      return __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a[t][g][lane]), as_bf16x8(ops[g]), zero, 0, 0, 0);
-    }, [&](uint32_t g) { return s[g]; });
-  } else if constexpr (FMT == GGUF_FMT_Q4K || FMT == GGUF_FMT_Q5K) {
-    const Q4KScales sc = q4k_scales(rec.meta);
-    float s[8];
-#pragma unroll
-    for (uint32_t g = 0; g < 8; ++g) s[g] = sc.d * byte_of(g < 4 ? sc.sc_lo : sc.sc_hi, g & 3u);
-    // Constant terms of groups kq and 4 + kq: m - 128 s.
-    const float s_lo = sc.d * byte_of(sc.sc_lo, kq), s_hi = sc.d * byte_of(sc.sc_hi, kq);
-    const float c_lo = __fmaf_rn(-128.f, s_lo, -(sc.dmin * byte_of(sc.mn_lo, kq)));
-    const float c_hi = __fmaf_rn(-128.f, s_hi, -(sc.dmin * byte_of(sc.mn_hi, kq)));
-#pragma unroll
-    for (int t = 0; t < RT; ++t) {
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(sums[t][0][lane], c_lo, acc[t], 0, 0, 0);
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(sums[t][1][lane], c_hi, acc[t], 0, 0, 0);
-    }
-    scaled_groups<RT, 8>(acc, [&](uint32_t g, int t) {
-      return __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a[t][g][lane]), as_bf16x8(ops[g]), zero, 0, 0, 0);
-    }, [&](uint32_t g) { return s[g]; });
-  } else {
-    const float d = half_bits_to_float(rec.d);
-    // Constant terms of 16-input blocks 4 j + kq: -160 d sc (operand 128 + q, value q - 32).
-#pragma unroll
-    for (uint32_t j = 0; j < 4; ++j) {
-      const uint32_t word = j == 0 ? rec.scales.x : j == 1 ? rec.scales.y : j == 2 ? rec.scales.z : rec.scales.w;
-      const float coef = -160.f * (d * float(int(int8_t((word >> (8u * kq)) & 0xFFu))));
-#pragma unroll
-      for (int t = 0; t < RT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(sums[t][j][lane], coef, acc[t], 0, 0, 0);
-    }
-    // a step is half a group: 16 inputs under one scale
-    scaled_groups<RT, 16>(acc, [&](uint32_t j, int t) {
-      const uint32_t g = j >> 1;
-      const uint4 av = a[t][g][lane];
-      const uint2 bw = j & 1u ? make_uint2(ops[g].z, ops[g].w) : make_uint2(ops[g].x, ops[g].y);
-      const uint2 aw = j & 1u ? make_uint2(av.z, av.w) : make_uint2(av.x, av.y);
-      return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, aw), __builtin_bit_cast(s16x4, bw), zero, 0, 0, 0);
-    }, [&](uint32_t j) { return d * q6_scale(rec.scales, j); });
+    for (int t = 0; t < RT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(sums[t][j][lane], coefficient, acc[t], 0, 0, 0);
   }
+  constexpr uint32_t kGroupSteps = RecordTerms<FMT>::kSteps / 8u;
+  scaled_groups<RT, RecordTerms<FMT>::kSteps>(acc, [&](uint32_t j, int t) {
+    return RecordTerms<FMT>::product(j, a[t][j / kGroupSteps][lane], ops[j / kGroupSteps]);
+  }, [&](uint32_t j) { return terms.scale(rec, j); });
 }
 
 // The staged rule (the reference's staged tile, kernels/common/gguf_staged.h:12-66: every weight decoded with fp32 group
@@ -353,18 +350,49 @@ __device__ __forceinline__ void accumulate_record_staged(const Record<FMT> &rec,
 // is tile u of its concatenated segments; of a gate/up pair, unit 2 j is gate tile j and unit
 // 2 j + 1 up tile j, so the two halves of a pair sit in neighbouring waves of one workgroup.
 // `item` is the workgroup's place in the dispatch (blockIdx.x of gguf_decode).
-// A workgroup's LDS, which the kernel declares once whatever formats its workgroups decode.
-// The four-tile kernels keep ONE buffer of a super-block's activations (two barriers a super-block instead of one): at
-// 32 KiB instead of 64 a compute unit holds three of their workgroups, not two, which their waits on LDS and on the
-// weight stream need more than they need the barrier. `spare` extends the buffer for the epilogues that lay rows out in it.
+// A workgroup's LDS, which the kernel declares once whatever formats its workgroups decode: what the loops that stage a
+// super-block's activations through registers use. The kernels of a chain and of q|k|v with its preparation keep ONE buffer
+// at four row tiles (two barriers a super-block instead of one): at 32 KiB instead of 64 a compute unit holds three of
+// their workgroups, not two. `spare` extends the buffer for the epilogues that lay rows out in it.
 template <int RT> struct DecodeShared {
+  static constexpr bool kRing = false;
   static constexpr int kBuffers = RT > 2 ? 1 : 2;
   uint4 a[kBuffers][RT][8][64];
   uint4 spare[RT > 2 ? 512 : 1];
   float sums[kBuffers][RT][4][64];
-  uint32_t arrived;
+  uint32_t arrivedWord;
   float scaleParts[256 * RT], rowScale[16 * RT];  // of a table with a deferred scale
+  __device__ __forceinline__ uint32_t &arrived() { return arrivedWord; }
+  // The staging buffers once the loop is done: sums, rows and halves an epilogue hands between its waves.
+  __device__ __forceinline__ float *epilogueSums() { return reinterpret_cast<float *>(&a[0][0][0][0]); }
+  __device__ __forceinline__ uint16_t *epilogueRows() { return reinterpret_cast<uint16_t *>(epilogueSums() + 2u * RT * 256u); }
+  __device__ __forceinline__ float *epilogueHalves() { return reinterpret_cast<float *>(epilogueRows() + 4u * RT * 256u); }
 };
+// The ring's: a stage is two groups of a super-block's activations, [row tile][group][lane], and four of them are a
+// super-block. Objects of their own, so that a read of one does not wait for what is on its way into another.
+template <int RT> struct DecodeRing {
+  static constexpr bool kRing = true;
+  static constexpr uint32_t kStageGroups = RT == 1 ? 4 : 2;
+  uint4 *rows0, *rows1, *rows2, *rows3;
+  float *sums0, *sums1;           // [row tile][K = 4 MFMA][lane]; a ring of two super-blocks has two
+  float *scaleParts, *rowScale;   // of a table with a deferred scale
+  uint32_t *arrivedWord;
+  __device__ __forceinline__ uint32_t &arrived() { return *arrivedWord; }
+  // (a stage holds 2 KiB a row tile)
+  __device__ __forceinline__ float *epilogueSums() { return reinterpret_cast<float *>(rows0); }
+  __device__ __forceinline__ uint16_t *epilogueRows() { return reinterpret_cast<uint16_t *>(rows1); }
+  __device__ __forceinline__ float *epilogueHalves() { return reinterpret_cast<float *>(rows2); }
+};
+// (FMT: the format of the workgroup's records; of several, any of those with most sums, which is Q6_K)
+#define SP_DECODE_RING(name, RT, FMT)                                                                                         \
+  constexpr uint32_t name##Stage = RT * DecodeRing<RT>::kStageGroups * 64, name##Sum = RT * RecordTerms<FMT>::kConstants * 64;  \
+  __shared__ uint4 name##Rows0[name##Stage], name##Rows1[name##Stage], name##Rows2[name##Stage], name##Rows3[name##Stage];    \
+  __shared__ float name##Sums0[name##Sum], name##Sums1[RT == 1 ? name##Sum : 1], name##Parts[256 * RT], name##Scale[16 * RT]; \
+  __shared__ uint32_t name##Arrived;                                                                                          \
+  DecodeRing<RT> name{name##Rows0, name##Rows1, name##Rows2, name##Rows3, name##Sums0, name##Sums1, name##Parts, name##Scale, &name##Arrived}
+
+// Vector-memory instructions of a record's load.
+template <uint32_t FMT> constexpr uint32_t kRecordLoads = FMT == GGUF_FMT_Q6K || FMT == GGUF_FMT_Q80 ? 5u : FMT == GGUF_FMT_Q5K ? 4u : 3u;
 
 // A projection's place in a chain of projections that share one dispatch (gguf_decode_chain): link i + 1 reads what link
 // i's epilogues wrote, so its workgroups, which the device starts after every workgroup of link i, fetch their first
@@ -620,8 +648,8 @@ __device__ __forceinline__ void qkv_clear_rows(const QkvHead &head, const QkvPre
     }
 }
 
-template <uint32_t FMT, int RT, uint32_t EP, bool Chain = false, bool Staged = false>
-__device__ __forceinline__ void decode_workgroup(DecodeShared<RT> &shared, const uint8_t *__restrict__ seg0,
+template <uint32_t FMT, int RT, uint32_t EP, bool Chain = false, bool Staged = false, class Shared>
+__device__ __forceinline__ void decode_workgroup(Shared &shared, const uint8_t *__restrict__ seg0,
                                                  const uint8_t *__restrict__ seg1, const uint8_t *__restrict__ seg2,
                                                  const uint8_t *__restrict__ table, void *__restrict__ out,
                                                  const uint16_t *__restrict__ residual, float *__restrict__ partials,
@@ -636,12 +664,10 @@ __device__ __forceinline__ void decode_workgroup(DecodeShared<RT> &shared, const
   constexpr uint32_t kColumnPart = Cursor<FMT>::kColumnPart;
   constexpr bool kSums32 = FMT != GGUF_FMT_Q6K;                // the constant term rides on 32-input sums (Q6_K: 16)
   constexpr uint32_t kSumsPerBlock = kSums32 ? 2 : 4;          // K = 4 MFMAs of row sums per super-block
-  // The range's activations pass through LDS one super-block at a time (two buffers, one barrier
-  // per super-block), each wave fetching a quarter of them, so a wave's vector-memory queue holds
+  // The range's activations pass through LDS, each wave fetching a quarter of them, so a wave's vector-memory queue holds
   // almost only weights and the MFMA operands arrive on the LDS counter instead.
-  auto &ldsA = shared.a;
-  auto &ldsSums = shared.sums;
-  uint32_t &arrived = shared.arrived;
+  constexpr bool kRing = Shared::kRing;
+  uint32_t &arrived = shared.arrived();
   auto &scaleParts = shared.scaleParts;
   auto &rowScale = shared.rowScale;
 
@@ -683,89 +709,8 @@ __device__ __forceinline__ void decode_workgroup(DecodeShared<RT> &shared, const
   for (int t = 0; t < RT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   {
-    // A software pipeline of kStages super-blocks in registers: the loads of super-block
-    // b + kStages - 1 are issued before the MFMAs of super-block b, so kStages - 1 super-blocks of
-    // weights per wave stay in flight (loads return in issue order, so waiting for b's never
-    // waits for a later one's). Loads past the range return zeros without touching memory.
-    constexpr int kStages = RT > 2 ? 2 : 3;
-    constexpr uint32_t kSumFloats = RT * kSumsPerBlock * 64u;  // staged row sums per super-block
-    constexpr int kSumShare = (kSumFloats + 255u) / 256u;
-    struct Stage {
-      Record<FMT> rec;
-      uint4 a[2 * RT];       // this thread's share of the super-block's RT * 8 * 64 operand vectors
-      float sum[kSumShare];  // and of its row sums
-      float second[kPairSums ? kSumShare : 1];  // a chained link: the other 16-input half of a 32-input sum
-    };
-    Stage stage[kStages];
     // A wave without a tile reads an empty range.
     const Resource weights = make_resource(tile.image ? tile.image + size_t(b0) * kRecord : seg0, tile.image ? count * kRecord : 0u);
-    uint32_t mine = 16u * lane, column = kColumnPart + 16u * c;
-    // The table's values of row tile t, super-blocks b0..b1: one resource per row tile.
-    Resource values[RT];
-#pragma unroll
-    for (int t = 0; t < RT; ++t)  // a row tile past the table's reads as zeros
-      values[t] = make_resource(table + (size_t(uint32_t(t) < tiles ? t : 0) * G + 8u * b0) * 1024u, uint32_t(t) < tiles ? count * 8192u : 0u);
-    uint32_t share[2];  // vector j of a row tile's super-block: byte offset of this thread's
-#pragma unroll
-    for (int j = 0; j < 2; ++j) share[j] = (threadIdx.x + 256u * j) * 16u;
-    const uint32_t sumsAt = kSums32 && !kPairSums ? gguf_table_sums32_offset(p.input_size, tiles) : gguf_table_sums16_offset(p.input_size, tiles);
-    const uint32_t sumGroups = kSums32 ? G : 2u * G;  // row-sum entries per row tile
-    const Resource sums = make_resource(table + sumsAt, tiles * (kPairSums ? 2u * G : sumGroups) * 64u);
-    // Threads past the staged sums repeat an earlier thread's (same value to the same slot). A thread's q-th sum lies
-    // whole row tiles past its first: its place and its address are the first's and a uniform step.
-    constexpr uint32_t kTileStep = 256u / (kSumsPerBlock * 64u);
-    static_assert(kSumShare == 1 || kSumFloats % 256u == 0, "a thread's sums lie whole row tiles apart");
-    uint32_t sumShare, sumSlot;
-    {
-      const uint32_t at = threadIdx.x % kSumFloats;
-      const uint32_t t = at / (kSumsPerBlock * 64u), j = (at / 64u) % kSumsPerBlock, l = at % 64u;
-      sumShare = ((t * sumGroups + kSumsPerBlock * 4u * b0 + 4u * j + (l >> 4)) * 16u * (kPairSums ? 2u : 1u) + (l & 15u)) * 4u;
-      sumSlot = (t * 4u + j) * 64u + l;
-    }
-    const uint32_t sumStep = kTileStep * sumGroups * 64u * (kPairSums ? 2u : 1u);
-    auto issueTable = [&](Stage &st) {
-#pragma unroll
-      for (int j = 0; j < 2 * RT; ++j) st.a[j] = load128<0>(values[j / 2], share[j % 2]);
-#pragma unroll
-      for (int q = 0; q < kSumShare; ++q)
-        st.sum[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sums, int(sumShare + q * sumStep), 0, 0));
-      if constexpr (kPairSums) {
-#pragma unroll
-        for (int q = 0; q < kSumShare; ++q)
-          st.second[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sums, int(sumShare + q * sumStep + 64u), 0, 0));
-      }
-#pragma unroll
-      for (int j = 0; j < 2; ++j) share[j] += 8192u;
-      // Sums past the range are the next range's or, past the table, zeros: staged and never used.
-      sumShare += kSumsPerBlock * 4u * 16u * 4u * (kPairSums ? 2u : 1u);
-    };
-    // A Q6_K wave of four row tiles has no register left for its lane's three places in a record: it works them out for
-    // each. (Kept, one was spilled and read back behind the loads just issued, and the wait for it was the wait for all
-    // of them: the vector-memory counter is one queue. 64 rows of 17408 -> 5120 57.1 -> 53.3 us, 5120 -> 17408 59.5 -> 52.7,
-    // 5120 -> 8192 Q4_K and 6144 Q6_K columns in one dispatch, at two waves a SIMD before and three now, 44.0 -> 38.9.)
-    constexpr bool kFreshLane = FMT == GGUF_FMT_Q6K && RT > 2;
-    uint32_t record = 0;
-    auto issueWeights = [&](Stage &st) {
-      if constexpr (kFreshLane) {
-        uint32_t l;
-        asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
-        const uint32_t first = record + 16u * l, mine16 = record + kColumnPart + 16u * (l & 15u);
-        st.rec.n0 = load128<kStreamOnce>(weights, first);
-        st.rec.n1 = load128<kStreamOnce>(weights, first + 1024u);
-        st.rec.high = load128<kStreamOnce>(weights, first + 2048u);
-        st.rec.scales = load128<kStreamOnce>(weights, mine16);
-        st.rec.d = __builtin_amdgcn_raw_buffer_load_b16(weights, int(record + GGUF_Q6K_D + 2u * (l & 15u)), 0, kStreamOnce);
-        record += kRecord;
-      } else {
-        load_record(st.rec, weights, mine, column);
-        mine += kRecord;
-        column += kRecord;
-      }
-    };
-    auto issue = [&](Stage &st) {
-      issueTable(st);
-      issueWeights(st);
-    };
     // Every row's inverse RMS from the squares the table's writer left, one entry a 64-column group:
     // part q of 16 adds entries q, q + 16, ... in order, then the 16 parts are added in order -- the same
     // sums whatever the kernel's row tiles, so a row's result does not depend on the block's height. A
@@ -793,72 +738,311 @@ __device__ __forceinline__ void decode_workgroup(DecodeShared<RT> &shared, const
 #pragma unroll
       for (uint32_t e = 0; e < kChunk; ++e) squareSum[i] += loaded[i][e];
     };
-    if constexpr (Chain) {
-      // The first stages' weights go out, then the wait for the link before, then what that link wrote.
-#pragma unroll
-      for (int s = 0; s < kStages - 1; ++s) {
-        issueWeights(stage[s]);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      chain_wait(chain);
+    auto loadFirstSquares = [&] {
 #pragma unroll
       for (int i = 0; i < RT; ++i) loadSquares(i, threadIdx.x / kRows + kThreadParts * i);
       __builtin_amdgcn_sched_barrier(0);
+    };
+    auto setRowScales = [&] {
 #pragma unroll
-      for (int s = 0; s < kStages - 1; ++s) {
-        issueTable(stage[s]);
-        __builtin_amdgcn_sched_barrier(0);
+      for (int i = 0; i < RT; ++i) {
+        addSquares(i);
+        // a wider table: the part's further entries, eight at a time (these waits do reach the weights')
+        if (p.deferred_scale)
+          for (uint32_t base = threadIdx.x / kRows + kThreadParts * i + kParts * kChunk; base < squareEntries; base += kParts * kChunk) {
+            loadSquares(i, base);
+            addSquares(i);
+          }
       }
-    } else {
+      if (p.deferred_scale) {
 #pragma unroll
-      for (int i = 0; i < RT; ++i) loadSquares(i, threadIdx.x / kRows + kThreadParts * i);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int s = 0; s < kStages - 1; ++s) {
-        issue(stage[s]);
-        // Keep the stages' loads in issue order: the loop's counted waits assume it on entry too.
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < RT; ++i) {
-      addSquares(i);
-      // a wider table: the part's further entries, eight at a time (these waits do reach the weights')
-      if (p.deferred_scale)
-        for (uint32_t base = threadIdx.x / kRows + kThreadParts * i + kParts * kChunk; base < squareEntries; base += kParts * kChunk) {
-          loadSquares(i, base);
-          addSquares(i);
+        for (int i = 0; i < RT; ++i) scaleParts[256u * i + threadIdx.x] = squareSum[i];   // part (threadIdx.x / kRows + kThreadParts i) of row threadIdx.x % kRows
+        __syncthreads();
+        if (threadIdx.x < kRows) {
+          float total = 0.f;
+          for (uint32_t q = 0; q < kParts; ++q) total += scaleParts[q * kRows + threadIdx.x];
+          rowScale[threadIdx.x] = 1.0f / sqrtf(total / float(p.input_size) + 1e-6f);
         }
-    }
-    if (p.deferred_scale) {
-#pragma unroll
-      for (int i = 0; i < RT; ++i) scaleParts[256u * i + threadIdx.x] = squareSum[i];   // part (threadIdx.x / kRows + kThreadParts i) of row threadIdx.x % kRows
-      __syncthreads();
-      if (threadIdx.x < kRows) {
-        float total = 0.f;
-        for (uint32_t q = 0; q < kParts; ++q) total += scaleParts[q * kRows + threadIdx.x];
-        rowScale[threadIdx.x] = 1.0f / sqrtf(total / float(p.input_size) + 1e-6f);
+        __syncthreads();
       }
-      __syncthreads();
-    }
-    const uint32_t rounds = (count + kStages - 1) / kStages;
-    uint32_t now = 0;
-    for (uint32_t round = 0; round < rounds; ++round) {
+    };
+    uint32_t mine = 16u * lane, column = kColumnPart + 16u * c;
+    // A staging Q6_K wave of four row tiles has no register left for its lane's three places in a record: it works them out for
+    // each. (Kept, one was spilled and read back behind the loads just issued, and the wait for it was the wait for all
+    // of them: the vector-memory counter is one queue. 64 rows of 17408 -> 5120 57.1 -> 53.3 us, 5120 -> 17408 59.5 -> 52.7,
+    // 5120 -> 8192 Q4_K and 6144 Q6_K columns in one dispatch, at two waves a SIMD before and three now, 44.0 -> 38.9.)
+    constexpr bool kFreshLane = !kRing && FMT == GGUF_FMT_Q6K && RT > 2;
+    uint32_t record = 0;
+    auto issueWeights = [&](Record<FMT> &rec) {
+      if constexpr (kFreshLane) {
+        uint32_t l;
+        asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+        const uint32_t first = record + 16u * l, mine16 = record + kColumnPart + 16u * (l & 15u);
+        rec.n0 = load128<kStreamOnce>(weights, first);
+        rec.n1 = load128<kStreamOnce>(weights, first + 1024u);
+        rec.high = load128<kStreamOnce>(weights, first + 2048u);
+        rec.scales = load128<kStreamOnce>(weights, mine16);
+        rec.d = __builtin_amdgcn_raw_buffer_load_b16(weights, int(record + GGUF_Q6K_D + 2u * (l & 15u)), 0, kStreamOnce);
+        record += kRecord;
+      } else {
+        load_record(rec, weights, mine, column);
+        mine += kRecord;
+        column += kRecord;
+      }
+    };
+    if constexpr (kRing) {
+      // The rows go from memory straight into LDS, three stages ahead of their use in four buffers, one barrier a stage: a
+      // wave has no register for them on the way and no store of them to wait for. What bounds the loop is issue and the
+      // LDS reads of operands; without the staging registers (32 of 165 at four row tiles of Q4_K, and what they kept the
+      // compiler from holding) a SIMD takes a wave more, and the arithmetic between two barriers is a stage's and not a
+      // super-block's. Through registers a super-block ahead (the loop below), against this, us a launch, weights past the
+      // caches: 5120 x 2 x 25600 Q4_K gate/up 34.9 -> 34.1 at 16 rows, 48.6 -> 43.0 at 32, 78.2 -> 67.2 at 64; 25600 x 5120
+      // Q6_K 33.6 -> 31.0, 47.3 -> 41.3, 77.5 -> 64.0; 5120 x 151936 Q6_K 134 -> 119, 198 -> 165, 366 -> 278; 5120 x 10240 Q4_K
+      // 15.3 -> 14.1, 19.5 -> 17.3, 28.0 -> 25.1. A third record in flight (87 -> 97 registers at two row tiles) is slower
+      // everywhere (down at 64 rows 69), five waves a SIMD spill (head at 16 rows 155).
+      using Ring = DecodeRing<RT>;
+      constexpr uint32_t kStages = 8u / Ring::kStageGroups;   // of a super-block
+      constexpr uint32_t kRowLoads = RT * Ring::kStageGroups / 4, kSumChunks = RT * kSumsPerBlock;
+      // a wave's sums: kSumLoads times 256 bytes, or a kilobyte at once; of fewer chunks than waves, two load the same
+      constexpr uint32_t kSumBytes = kSumChunks == 16 ? 16u : 4u, kSumLoads = kSumChunks == 16 || kSumChunks < 4 ? 1 : kSumChunks / 4;
+      constexpr uint32_t kWeightLoads = kRecordLoads<FMT>;
+      const uint32_t waveIndex = uint32_t(__builtin_amdgcn_readfirstlane(int(wave)));
+      const uint32_t rowChunk = kRowLoads * waveIndex, rowTile = rowChunk / Ring::kStageGroups;   // its kilobytes of a stage, one row tile's
+      // (a row tile past the table's, and a super-block past the range, read as zeros)
+      const Resource values = make_resource(table + (size_t(rowTile < tiles ? rowTile : 0) * G + 8u * b0) * 1024u, rowTile < tiles ? count * 8192u : 0u);
+      const uint32_t sumsAt = kSums32 ? gguf_table_sums32_offset(p.input_size, tiles) : gguf_table_sums16_offset(p.input_size, tiles);
+      const uint32_t sumGroups = kSums32 ? G : 2u * G;   // row-sum entries per row tile
+      const Resource sums = make_resource(table + sumsAt, tiles * sumGroups * 64u);
+      uint32_t rowsAt = lane * 16u + rowChunk % Ring::kStageGroups * 1024u;
+      // chunk j of a row tile: the sums of entries 4 j .. + 3 of the super-block, 64 floats
+      const uint32_t sumChunk = kSumBytes == 16u ? waveIndex * 4u : waveIndex * kSumLoads % kSumChunks;
+      uint32_t sumsFrom = (sumChunk / kSumsPerBlock * sumGroups + kSumsPerBlock * 4u * b0 + sumChunk % kSumsPerBlock * 4u) * 64u + lane * kSumBytes;
+      auto stageRows = [&](auto stageConstant) __attribute__((always_inline)) -> uint4 * {
+        constexpr uint32_t S = decltype(stageConstant)::value & 3u;
+        return S == 0 ? shared.rows0 : S == 1 ? shared.rows1 : S == 2 ? shared.rows2 : shared.rows3;
+      };
+      auto fetchRows = [&](auto stageConstant) __attribute__((always_inline)) {   // the ring's stage, of the super-block at rowsAt
+        constexpr uint32_t S = decltype(stageConstant)::value % kStages;
+        uint4 *to = stageRows(stageConstant) + kRowLoads * 64u * waveIndex;
 #pragma unroll
-      for (int u = 0; u < kStages; ++u, ++now) {
-        const uint32_t buffer = DecodeShared<RT>::kBuffers == 2 ? (now & 1u) : 0u;
+        for (uint32_t i = 0; i < kRowLoads; ++i) load_to_lds<16>(values, rowsAt + S * Ring::kStageGroups * 1024u + i * 1024u, to + 64u * i);
+        if constexpr (S + 1u == kStages) rowsAt += 8192u;
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      auto sumsOf = [&](auto stageConstant) __attribute__((always_inline)) -> float * {   // of the super-block that starts at the ring's stage
+        return (decltype(stageConstant)::value & 3u) / kStages ? shared.sums1 : shared.sums0;
+      };
+      auto fetchSums = [&](auto stageConstant) __attribute__((always_inline)) {
+        float *to = sumsOf(stageConstant) + sumChunk * 64u;
 #pragma unroll
-        for (int j = 0; j < 2 * RT; ++j) (&ldsA[buffer][0][0][0])[threadIdx.x + 256u * j] = stage[u].a[j];
+        for (uint32_t i = 0; i < kSumLoads; ++i) load_to_lds<kSumBytes>(sums, sumsFrom + i * 256u, to + 64u * i);
+        sumsFrom += kSumsPerBlock * 4u * 64u;   // (sums past the range are the next range's or, past the table, zeros: never used)
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      constexpr uint32_t kRecords = 2;   // a record's loads leave kRecords - 1 super-blocks ahead of its use
+      static_assert(kRecords * kStages % 4u == 0, "a turn of the records is whole turns of the ring");
+      Record<FMT> rec[kRecords];
+      using Terms = RecordTerms<FMT>;
+      constexpr uint32_t kStageSteps = Terms::kSteps / kStages, kGroupSteps = Terms::kSteps / 8u;
+      // (the loads before the first stage in the order of the stages that would have asked for them)
+      loadFirstSquares();
+#pragma unroll
+      for (uint32_t i = 0; i + 1 < kRecords; ++i) {
+        if (kStages == 2u && i + 2 == kRecords) break;
+        issueWeights(rec[i]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      fetchRows(std::integral_constant<uint32_t, 0>{});
+      fetchSums(std::integral_constant<uint32_t, 0>{});
+      fetchRows(std::integral_constant<uint32_t, 1>{});
+      if constexpr (kStages == 2u) {
+        issueWeights(rec[kRecords - 2]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      fetchRows(std::integral_constant<uint32_t, 2>{});
+      if constexpr (kStages == 2u) fetchSums(std::integral_constant<uint32_t, 2>{});
+      setRowScales();
+      auto superBlock = [&](const Record<FMT> &now, Record<FMT> &next, auto firstStage) __attribute__((always_inline)) {
+        constexpr uint32_t F = decltype(firstStage)::value;   // the ring's stage of the super-block's first
+        f32x4 held[2][RT];
+        auto run = [&](auto stageConstant) __attribute__((always_inline)) {
+          constexpr uint32_t S = decltype(stageConstant)::value;
+          // What left behind stage S's rows: what else its stage asked for (the first stage's: a super-block's sums, which it
+          // needs as well), and all that the two stages after it did.
+          constexpr auto others = [](uint32_t stage) constexpr { return (stage % kStages == 0 ? kWeightLoads : 0u) + (stage % kStages == 1u ? kSumLoads : 0u); };
+          wait_loads<(S == 0 ? 0u : others(S + 1u)) + kRowLoads + others(S + 2u) + kRowLoads + others(S + 3u)>();
+          asm volatile("" ::: "memory");
+          __builtin_amdgcn_s_barrier();
+          asm volatile("" ::: "memory");
+          __builtin_amdgcn_sched_barrier(0);
+          fetchRows(std::integral_constant<uint32_t, (F + S + 3u) & 3u>{});
+          if constexpr (S == 0) issueWeights(next);
+          if constexpr (S == 1) fetchSums(std::integral_constant<uint32_t, (F + S + 3u) & 3u>{});
+          __builtin_amdgcn_sched_barrier(0);
+          const uint4 *rows = stageRows(std::integral_constant<uint32_t, F + S>{});
+          uint4 ops[8];
+          record_operands(now, ops);   // (this stage's)
+          const Terms terms(now);
+          if constexpr (S == 0 && !Staged) {
+            const float *rowSums = sumsOf(firstStage);
+#pragma unroll
+            for (uint32_t j = 0; j < Terms::kConstants; ++j) {
+              const float coefficient = terms.constant(now, j, kq);
+#pragma unroll
+              for (int t = 0; t < RT; ++t)
+                acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(rowSums[(t * Terms::kConstants + j) * 64u + lane], coefficient, acc[t], 0, 0, 0);
+            }
+          }
+          if constexpr (Staged) {
+            const StagedCoefficients<FMT> k(now);
+#pragma unroll
+            for (uint32_t g = 0; g < Ring::kStageGroups; ++g) {
+              bf16x8 high, low;
+              staged_group(now, k, ops[Ring::kStageGroups * S + g], Ring::kStageGroups * S + g, high, low);
+#pragma unroll
+              for (int t = 0; t < RT; ++t) {
+                const bf16x8 a = as_bf16x8(rows[(t * Ring::kStageGroups + g) * 64u + lane]);
+                acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, high, acc[t], 0, 0, 0);
+                acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, low, acc[t], 0, 0, 0);
+              }
+            }
+          } else {
+            // as scaled_groups: a step's products leave before the multiply-adds of the step before it
+            auto multiplyAdd = [&](uint32_t step) __attribute__((always_inline)) {
+              const float scale = terms.scale(now, step);
+#pragma unroll
+              for (int t = 0; t < RT; ++t)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) acc[t][v] = __fmaf_rn(held[step & 1u][t][v], scale, acc[t][v]);
+            };
+#pragma unroll
+            for (uint32_t i = 0; i < kStageSteps; ++i) {
+              const uint32_t step = kStageSteps * S + i, g = step / kGroupSteps;
+#pragma unroll
+              for (int t = 0; t < RT; ++t)
+                held[step & 1u][t] = Terms::product(step, rows[(t * Ring::kStageGroups + g % Ring::kStageGroups) * 64u + lane], ops[g]);
+              if (step) multiplyAdd(step - 1u);
+            }
+            if constexpr (S + 1u == kStages) multiplyAdd(Terms::kSteps - 1u);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        };
+        run(std::integral_constant<uint32_t, 0>{});
+        run(std::integral_constant<uint32_t, 1>{});
+        if constexpr (kStages == 4u) {
+          run(std::integral_constant<uint32_t, 2>{});
+          run(std::integral_constant<uint32_t, 3>{});
+        }
+      };
+      for (uint32_t block = 0; block < count; block += kRecords) {
+        [&]<uint32_t... I>(std::integer_sequence<uint32_t, I...>) __attribute__((always_inline)) {
+          ((block + I < count ? superBlock(rec[I], rec[(I + kRecords - 1u) % kRecords], std::integral_constant<uint32_t, I * kStages & 3u>{}) : void()), ...);
+        }(std::make_integer_sequence<uint32_t, kRecords>{});
+      }
+      wait_loads<0>();   // nothing is on its way into LDS when the epilogue takes it
+    } else {
+      auto &ldsA = shared.a;
+      auto &ldsSums = shared.sums;
+      // A software pipeline of kStages super-blocks in registers: the loads of super-block
+      // b + kStages - 1 are issued before the MFMAs of super-block b, so kStages - 1 super-blocks of
+      // weights per wave stay in flight (loads return in issue order, so waiting for b's never
+      // waits for a later one's). Loads past the range return zeros without touching memory.
+      constexpr int kStages = RT > 2 ? 2 : 3;
+      constexpr uint32_t kSumFloats = RT * kSumsPerBlock * 64u;  // staged row sums per super-block
+      constexpr int kSumShare = (kSumFloats + 255u) / 256u;
+      struct Stage {
+        Record<FMT> rec;
+        uint4 a[2 * RT];       // this thread's share of the super-block's RT * 8 * 64 operand vectors
+        float sum[kSumShare];  // and of its row sums
+        float second[kPairSums ? kSumShare : 1];  // a chained link: the other 16-input half of a 32-input sum
+      };
+      Stage stage[kStages];
+      // The table's values of row tile t, super-blocks b0..b1: one resource per row tile.
+      Resource values[RT];
+#pragma unroll
+      for (int t = 0; t < RT; ++t)  // a row tile past the table's reads as zeros
+        values[t] = make_resource(table + (size_t(uint32_t(t) < tiles ? t : 0) * G + 8u * b0) * 1024u, uint32_t(t) < tiles ? count * 8192u : 0u);
+      uint32_t share[2];  // vector j of a row tile's super-block: byte offset of this thread's
+#pragma unroll
+      for (int j = 0; j < 2; ++j) share[j] = (threadIdx.x + 256u * j) * 16u;
+      const uint32_t sumsAt = kSums32 && !kPairSums ? gguf_table_sums32_offset(p.input_size, tiles) : gguf_table_sums16_offset(p.input_size, tiles);
+      const uint32_t sumGroups = kSums32 ? G : 2u * G;  // row-sum entries per row tile
+      const Resource sums = make_resource(table + sumsAt, tiles * (kPairSums ? 2u * G : sumGroups) * 64u);
+      // Threads past the staged sums repeat an earlier thread's (same value to the same slot). A thread's q-th sum lies
+      // whole row tiles past its first: its place and its address are the first's and a uniform step.
+      constexpr uint32_t kTileStep = 256u / (kSumsPerBlock * 64u);
+      static_assert(kSumShare == 1 || kSumFloats % 256u == 0, "a thread's sums lie whole row tiles apart");
+      uint32_t sumShare, sumSlot;
+      {
+        const uint32_t at = threadIdx.x % kSumFloats;
+        const uint32_t t = at / (kSumsPerBlock * 64u), j = (at / 64u) % kSumsPerBlock, l = at % 64u;
+        sumShare = ((t * sumGroups + kSumsPerBlock * 4u * b0 + 4u * j + (l >> 4)) * 16u * (kPairSums ? 2u : 1u) + (l & 15u)) * 4u;
+        sumSlot = (t * 4u + j) * 64u + l;
+      }
+      const uint32_t sumStep = kTileStep * sumGroups * 64u * (kPairSums ? 2u : 1u);
+      auto issueTable = [&](Stage &st) {
+#pragma unroll
+        for (int j = 0; j < 2 * RT; ++j) st.a[j] = load128<0>(values[j / 2], share[j % 2]);
 #pragma unroll
         for (int q = 0; q < kSumShare; ++q)
-          (&ldsSums[buffer][0][0][0])[sumSlot + q * kTileStep * 256u] = kPairSums ? stage[u].sum[q] + stage[u].second[q] : stage[u].sum[q];
-        __syncthreads();
-        issue(stage[(u + kStages - 1) % kStages]);
-        if (now < count) {
-          if constexpr (Staged) accumulate_record_staged<FMT, RT>(stage[u].rec, ldsA[buffer], acc, lane, kq);
-          else accumulate_record<FMT, RT>(stage[u].rec, ldsA[buffer], ldsSums[buffer], acc, lane, kq);
+          st.sum[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sums, int(sumShare + q * sumStep), 0, 0));
+        if constexpr (kPairSums) {
+#pragma unroll
+          for (int q = 0; q < kSumShare; ++q)
+            st.second[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sums, int(sumShare + q * sumStep + 64u), 0, 0));
         }
-        if constexpr (DecodeShared<RT>::kBuffers == 1) __syncthreads();   // every wave has read the buffer before the next super-block lands in it
+#pragma unroll
+        for (int j = 0; j < 2; ++j) share[j] += 8192u;
+        // Sums past the range are the next range's or, past the table, zeros: staged and never used.
+        sumShare += kSumsPerBlock * 4u * 16u * 4u * (kPairSums ? 2u : 1u);
+      };
+      auto issue = [&](Stage &st) {
+        issueTable(st);
+        issueWeights(st.rec);
+      };
+      if constexpr (Chain) {
+        // The first stages' weights go out, then the wait for the link before, then what that link wrote.
+#pragma unroll
+        for (int s = 0; s < kStages - 1; ++s) {
+          issueWeights(stage[s].rec);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        chain_wait(chain);
+        loadFirstSquares();
+#pragma unroll
+        for (int s = 0; s < kStages - 1; ++s) {
+          issueTable(stage[s]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      } else {
+        loadFirstSquares();
+#pragma unroll
+        for (int s = 0; s < kStages - 1; ++s) {
+          issue(stage[s]);
+          // Keep the stages' loads in issue order: the loop's counted waits assume it on entry too.
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      setRowScales();
+      const uint32_t rounds = (count + kStages - 1) / kStages;
+      uint32_t now = 0;
+      for (uint32_t round = 0; round < rounds; ++round) {
+#pragma unroll
+        for (int u = 0; u < kStages; ++u, ++now) {
+          const uint32_t buffer = DecodeShared<RT>::kBuffers == 2 ? (now & 1u) : 0u;
+#pragma unroll
+          for (int j = 0; j < 2 * RT; ++j) (&ldsA[buffer][0][0][0])[threadIdx.x + 256u * j] = stage[u].a[j];
+#pragma unroll
+          for (int q = 0; q < kSumShare; ++q)
+            (&ldsSums[buffer][0][0][0])[sumSlot + q * kTileStep * 256u] = kPairSums ? stage[u].sum[q] + stage[u].second[q] : stage[u].sum[q];
+          __syncthreads();
+          issue(stage[(u + kStages - 1) % kStages]);
+          if (now < count) {
+            if constexpr (Staged) accumulate_record_staged<FMT, RT>(stage[u].rec, ldsA[buffer], acc, lane, kq);
+            else accumulate_record<FMT, RT>(stage[u].rec, ldsA[buffer], ldsSums[buffer], acc, lane, kq);
+          }
+          if constexpr (DecodeShared<RT>::kBuffers == 1) __syncthreads();   // every wave has read the buffer before the next super-block lands in it
+        }
       }
     }
   }
@@ -945,6 +1129,7 @@ __device__ __forceinline__ void decode_workgroup(DecodeShared<RT> &shared, const
     if (arrived != halves * splits - 1u) return;
     if (threadIdx.x == 0) __hip_atomic_store(counters + headOf, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     // the staging buffers are free: the head's rows as floats, then a row a wave for the RoPE exchange
+    auto &ldsA = shared.a;
     float (*headRows)[128] = reinterpret_cast<float (*)[128]>(&ldsA[0][0][0][0]);
     float (*waveRows)[4][128] = reinterpret_cast<float (*)[4][128]>(reinterpret_cast<char *>(&ldsA[0][0][0][0]) + 16u * RT * 128u * 4u);
     static_assert(sizeof(shared.a) + (RT > 2 ? sizeof(shared.spare) : 0u) >= 16u * RT * 128u * 4u + 4u * 4u * 128u * 4u,
@@ -1053,7 +1238,7 @@ __device__ __forceinline__ void decode_workgroup(DecodeShared<RT> &shared, const
 
   if constexpr (kGateUp) {
     // The up wave hands its sums to the gate wave beside it through LDS (the staging buffers are free).
-    float *exchange = reinterpret_cast<float *>(&ldsA[0][0][0][0]);
+    float *exchange = shared.epilogueSums();
     __syncthreads();
     if (wave & 1u) {
 #pragma unroll
@@ -1065,8 +1250,8 @@ __device__ __forceinline__ void decode_workgroup(DecodeShared<RT> &shared, const
     // With the table epilogue the workgroup's 32 columns, one group of the next projection's
     // inputs, also leave as that projection's activation table (abi/Gguf.h), as gguf_prepare_table
     // would write them: tileOut[half][row tile][row][column] collects the bf16 results.
-    uint16_t *tileOut = reinterpret_cast<uint16_t *>(exchange + 2u * RT * 256u);
-    float *halfSums = reinterpret_cast<float *>(tileOut + 2u * RT * 256u);
+    uint16_t *tileOut = shared.epilogueRows();
+    float *halfSums = shared.epilogueHalves();
     const uint32_t half = wave >> 1;
     if (!(wave & 1u)) {
       uint16_t *o = static_cast<uint16_t *>(out);
@@ -1121,9 +1306,9 @@ __device__ __forceinline__ void decode_workgroup(DecodeShared<RT> &shared, const
     const float weight = bf16_bits_to_float(normBits);
     // The staging buffers are free once every wave has left the loop.
     __syncthreads();
-    float *waveSquares = reinterpret_cast<float *>(&ldsA[0][0][0][0]);          // [wave][row]
-    uint16_t *tileOut = reinterpret_cast<uint16_t *>(waveSquares + 4u * kRows);  // [wave][row tile][row][column]
-    float *halfSums = reinterpret_cast<float *>(tileOut + 4u * RT * 256u);       // [row tile][wave][row]
+    float *waveSquares = shared.epilogueSums();       // [wave][row]
+    uint16_t *tileOut = shared.epilogueRows();        // [wave][row tile][row][column]
+    float *halfSums = shared.epilogueHalves();        // [row tile][wave][row]
 #pragma unroll
     for (int t = 0; t < RT; ++t) {
       uint32_t bits[4];
@@ -1219,12 +1404,12 @@ __device__ __forceinline__ void decode_workgroup(DecodeShared<RT> &shared, const
   }
 }
 
-// Three waves a SIMD (168 registers) where a kernel would take a few registers more and run two: every format's four row
-// tiles, and Q6_K's two under some epilogues (a step of 8 layers and 24 rows in three lanes, whose down projections take the
-// residual and norm, 1755 -> 1670 us). Four (128) for Q6_K's one row tile spill outside the loop and are slower (16 rows
-// 1307 -> 1342 us a step).
+// Waves a SIMD: four (128 registers); three where those would spill in the loop (Q6_K's taller tiles, and four row tiles of
+// the formats with a scale of 16 bits a group).
+template <uint32_t FMT, int RT>
+constexpr uint32_t kDecodeWaves = (RT > 1 && FMT == GGUF_FMT_Q6K) || (RT > 2 && (FMT == GGUF_FMT_Q80 || FMT == GGUF_FMT_IQ4NL)) ? 3 : 4;
 template <uint32_t FMT, int RT, uint32_t EP, bool Staged = false>
-__global__ __launch_bounds__(256, RT > 2 || (RT == 2 && FMT == GGUF_FMT_Q6K) ? 3 : 1)
+__global__ __launch_bounds__(256, kDecodeWaves<FMT, RT>)
                                   void gguf_decode(const uint8_t *__restrict__ seg0, const uint8_t *__restrict__ seg1,
                                                    const uint8_t *__restrict__ seg2, const uint8_t *__restrict__ table,
                                                    void *__restrict__ out, const uint16_t *__restrict__ residual,
@@ -1245,7 +1430,7 @@ __global__ __launch_bounds__(256, RT > 2 || (RT == 2 && FMT == GGUF_FMT_Q6K) ? 3
     p.rows -= first;
   }
   p.rows = min(p.rows, uint32_t(GGUF_MAXIMUM_ROWS));
-  __shared__ DecodeShared<RT> shared;
+  SP_DECODE_RING(shared, RT, FMT);
   decode_workgroup<FMT, RT, EP, false, Staged>(shared, seg0, seg1, seg2, table, out, residual, partials, counters, p, blockIdx.x);
 }
 
@@ -1254,7 +1439,7 @@ __global__ __launch_bounds__(256, RT > 2 || (RT == 2 && FMT == GGUF_FMT_Q6K) ? 3
 // columns), every workgroup takes one of p.splits parts of K (whole_groups 0), and a workgroup runs its segment's
 // format as a projection of that segment alone, its partials and counters after those of the segments before it.
 template <int RT>
-__global__ __launch_bounds__(256, RT > 2 ? 3 : 1) void gguf_decode_mixed(const uint8_t *__restrict__ seg0, const uint8_t *__restrict__ seg1,
+__global__ __launch_bounds__(256, 3) void gguf_decode_mixed(const uint8_t *__restrict__ seg0, const uint8_t *__restrict__ seg1,
                                                          const uint8_t *__restrict__ seg2, const uint8_t *__restrict__ table,
                                                          void *__restrict__ out, const uint16_t *__restrict__ residual,
                                                          float *__restrict__ partials, uint32_t *__restrict__ counters,
@@ -1290,28 +1475,21 @@ __global__ __launch_bounds__(256, RT > 2 ? 3 : 1) void gguf_decode_mixed(const u
   partials += size_t(before) * p.splits * kGroupFloats;
   counters += before;
   const uint32_t item = (group - before) * p.splits + split;
-  __shared__ DecodeShared<RT> shared;
+  SP_DECODE_RING(shared, RT, GGUF_FMT_Q6K);
+#define SP_MIXED_FORMAT(F)                                                                                                             \
+  case F:                                                                                                                              \
+    decode_workgroup<F, RT, GGUF_EPILOGUE_PLAIN>(shared, image, image, image, table, out, residual, partials, counters, mine, item);   \
+    break
   switch (format) {
-  case GGUF_FMT_Q4K:
-    decode_workgroup<GGUF_FMT_Q4K, RT, GGUF_EPILOGUE_PLAIN>(shared, image, image, image, table, out, residual, partials, counters, mine, item);
-    break;
-  case GGUF_FMT_Q5K:
-    decode_workgroup<GGUF_FMT_Q5K, RT, GGUF_EPILOGUE_PLAIN>(shared, image, image, image, table, out, residual, partials, counters, mine, item);
-    break;
-  case GGUF_FMT_Q6K:
-    decode_workgroup<GGUF_FMT_Q6K, RT, GGUF_EPILOGUE_PLAIN>(shared, image, image, image, table, out, residual, partials, counters, mine, item);
-    break;
-  case GGUF_FMT_Q80:
-    decode_workgroup<GGUF_FMT_Q80, RT, GGUF_EPILOGUE_PLAIN>(shared, image, image, image, table, out, residual, partials, counters, mine, item);
-    break;
-  case GGUF_FMT_IQ4XS:
-    decode_workgroup<GGUF_FMT_IQ4XS, RT, GGUF_EPILOGUE_PLAIN>(shared, image, image, image, table, out, residual, partials, counters, mine, item);
-    break;
-  case GGUF_FMT_IQ4NL:
-    decode_workgroup<GGUF_FMT_IQ4NL, RT, GGUF_EPILOGUE_PLAIN>(shared, image, image, image, table, out, residual, partials, counters, mine, item);
-    break;
+    SP_MIXED_FORMAT(GGUF_FMT_Q4K);
+    SP_MIXED_FORMAT(GGUF_FMT_Q5K);
+    SP_MIXED_FORMAT(GGUF_FMT_Q6K);
+    SP_MIXED_FORMAT(GGUF_FMT_Q80);
+    SP_MIXED_FORMAT(GGUF_FMT_IQ4XS);
+    SP_MIXED_FORMAT(GGUF_FMT_IQ4NL);
   default: break;
   }
+#undef SP_MIXED_FORMAT
 }
 SP_REGISTER_KERNEL("gguf_decode_mixed_m16_a", &gguf_decode_mixed<1>);
 SP_REGISTER_KERNEL("gguf_decode_mixed_m32_a", &gguf_decode_mixed<2>);
@@ -1488,7 +1666,7 @@ SP_REGISTER_KERNEL("gguf_decode_chain_m64", &gguf_decode_chain<4>);
 // own activation table (table_bytes apart) and writes its own 16 output rows (and, with the table
 // epilogue, its own next table). Slots at or past tile_total[0] are empty.
 template <uint32_t FMT, uint32_t EP>
-__global__ __launch_bounds__(256) void gguf_moe_decode(const uint8_t *__restrict__ seg0, const uint8_t *__restrict__ seg1,
+__global__ __launch_bounds__(256, 4) void gguf_moe_decode(const uint8_t *__restrict__ seg0, const uint8_t *__restrict__ seg1,
                                                        const uint8_t *__restrict__ tables, uint8_t *__restrict__ out,
                                                        uint8_t *__restrict__ next_tables, const uint32_t *__restrict__ tile_expert,
                                                        const uint32_t *__restrict__ tile_rows, const uint32_t *__restrict__ tile_total,
@@ -1498,7 +1676,7 @@ __global__ __launch_bounds__(256) void gguf_moe_decode(const uint8_t *__restrict
   const uint32_t expert = tile_expert[tile];
   GgufDecodeParams p = m.decode;
   p.rows = tile_rows[tile];
-  __shared__ DecodeShared<1> shared;
+  SP_DECODE_RING(shared, 1, FMT);
   decode_workgroup<FMT, 1, EP>(shared, seg0 + expert * m.expert_bytes, seg1 + expert * m.expert_bytes, seg0 + expert * m.expert_bytes,
                                tables + tile * m.table_bytes, out + size_t(tile) * 16u * m.out_row_bytes,
                                reinterpret_cast<const uint16_t *>(next_tables + tile * m.next_table_bytes), nullptr, nullptr, p,

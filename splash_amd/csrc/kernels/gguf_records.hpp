@@ -190,6 +190,18 @@ template <int Aux> __device__ __forceinline__ uint4 load128(Resource r, uint32_t
   const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, int(offset), 0, Aux);
   return make_uint4(v.x, v.y, v.z, v.w);
 }
+// Sixteen (four) bytes a lane of a wave, from memory straight into LDS (`to` the wave's first lane's, the others after it).
+typedef __attribute__((address_space(3))) void LdsVoid;
+template <uint32_t Bytes> __device__ __forceinline__ void load_to_lds(Resource r, uint32_t offset, void *to) {
+  static_assert(Bytes == 16u || Bytes == 4u);
+  if constexpr (Bytes == 16u) __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LdsVoid *)to, 16, int(offset), 0, 0, 0);
+  else __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LdsVoid *)to, 4, int(offset), 0, 0, 0);
+}
+// Vector-memory instructions that may be in flight behind a wait (s_waitcnt's vmcnt alone).
+template <uint32_t N> __device__ __forceinline__ void wait_loads() {
+  static_assert(N < 64, "vmcnt has six bits");
+  __builtin_amdgcn_s_waitcnt((N & 15u) | ((N >> 4) << 14) | 0x0F70u);
+}
 // `mine` is the lane's 16 bytes of the record's first 1024-byte part, `column` its column's scale
 // field, both as byte offsets into the resource.
 __device__ __forceinline__ void load_record(Record<GGUF_FMT_Q4K> &rec, Resource r, uint32_t mine, uint32_t column) {

@@ -403,17 +403,6 @@ __device__ __forceinline__ WideOperands<FMT> wide_staged_operands(const WideReco
   return out;
 }
 
-// Sixteen bytes a lane of a wave, from memory straight into LDS (`to` the wave's first lane's, the others after it).
-typedef __attribute__((address_space(3))) void LdsVoid;
-__device__ __forceinline__ void load_to_lds(Resource r, uint32_t offset, uint4 *to) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LdsVoid *)to, 16, int(offset), 0, 0, 0);
-}
-// Vector-memory instructions that may be in flight behind a wait (s_waitcnt's vmcnt alone).
-template <uint32_t N> __device__ __forceinline__ void wait_loads() {
-  static_assert(N < 64, "vmcnt has six bits");
-  __builtin_amdgcn_s_waitcnt((N & 15u) | ((N >> 4) << 14) | 0x0F70u);
-}
-
 // What a workgroup computes: its wave's two column tiles (image null: a tile past the last), its row tiles, its part of K.
 struct WideTile {
   const uint8_t *image[2];
@@ -505,10 +494,10 @@ __device__ __forceinline__ void wide_workgroup(const WideLds lds, const WideTile
     const uint32_t at = block < count ? (b0 + block) * (GGUF_WIDE_OPERANDS * 1024u) + S * 2048u : 0x80000000u;
     uint4 *to = stageRows(stageConstant) + 64u * wave;
 #pragma unroll
-    for (uint32_t i = 0; i < kShare; ++i) load_to_lds(rowValues, mineAt + (at + 2u * i * tileBytes), to + 256u * i);
+    for (uint32_t i = 0; i < kShare; ++i) load_to_lds<16>(rowValues, mineAt + (at + 2u * i * tileBytes), to + 256u * i);
     if constexpr (S == 3u) {
 #pragma unroll
-      for (uint32_t i = 0; i < kSumShare; ++i) load_to_lds(rowValues, sumsAt + (at + 2048u + 4u * i * tileBytes), lds.sums + 64u * wave + 256u * i);
+      for (uint32_t i = 0; i < kSumShare; ++i) load_to_lds<16>(rowValues, sumsAt + (at + 2048u + 4u * i * tileBytes), lds.sums + 64u * wave + 256u * i);
     }
   };
   // A record's first half (and what both share) is fetched two stages ahead of its use, and so is its second.
