@@ -1409,7 +1409,7 @@ __device__ __forceinline__ void decode_workgroup(Shared &shared, const uint8_t *
 template <uint32_t FMT, int RT>
 constexpr uint32_t kDecodeWaves = (RT > 1 && FMT == GGUF_FMT_Q6K) || (RT > 2 && (FMT == GGUF_FMT_Q80 || FMT == GGUF_FMT_IQ4NL)) ? 3 : 4;
 template <uint32_t FMT, int RT, uint32_t EP, bool Staged = false>
-__global__ __launch_bounds__(256, kDecodeWaves<FMT, RT>)
+__global__ __launch_bounds__(256, (kDecodeWaves<FMT, RT>))
                                   void gguf_decode(const uint8_t *__restrict__ seg0, const uint8_t *__restrict__ seg1,
                                                    const uint8_t *__restrict__ seg2, const uint8_t *__restrict__ table,
                                                    void *__restrict__ out, const uint16_t *__restrict__ residual,
