@@ -12,12 +12,12 @@
 // Split: a wave owns 32 columns (a record of two column tiles each super-block, dequantized once in its registers) of
 // all of the workgroup's 128 rows, whose operands go from memory straight into LDS, three stages of two groups ahead of
 // their use in four buffers, one barrier a stage. (Through registers, one stage ahead, which is what 256 of them leave
-// room for, waves waited a quarter of their time: gate/up 1.27, the SwiGLU rows' projection 0.97 ms where it is 1.18 and
-// 0.91 now; an expert's tiles, whose rows come from further away, 215 and 158 us where they take 192 and 149. A row
+// room for, waves waited a quarter of their time: gate/up 1.27, the SwiGLU rows' projection 0.97 ms where it was 1.18 and
+// 0.91; an expert's tiles, whose rows come from further away, 215 and 158 us where they take 192 and 149. A row
 // tile's operands read two tiles ahead, or waves of a priority that follows the phase, changed nothing.) Two waves a SIMD
 // overlap the conversion of one with the MFMAs of the other. At 2048 rows of the 5120 x 2 x 25600 Q4_K gate/up pair a
-// launch takes 1.18 ms (906 TFLOP/s of the projection's own operations; the 64-row windows of the decode kernels took
-// 2.38 ms), at 25600 x 5120 Q6_K 0.91 ms (2.2 ms): with the constant terms and the second product that is 1.02 and 1.18
+// launch takes 1.09 ms (985 TFLOP/s of the projection's own operations; the 64-row windows of the decode kernels took
+// 2.38 ms), at 25600 x 5120 Q6_K 0.86 ms (2.2 ms): with the constant terms and the second product that is 1.11 and 1.25
 // PFLOP/s of MFMAs, where a large library product reaches 1.19 under the card's power limit.
 #include "abi/Gguf.h"
 #include "abi/Moe.h"
@@ -450,10 +450,15 @@ __device__ __forceinline__ void wide_columns(WideTile &w, const uint8_t *seg0, c
 // read of one does not wait for what is on its way into another.
 struct WideLds {
   uint4 *rows0, *rows1, *rows2, *rows3, *sums;
+  float *scales;   // the row tiles' scales
 };
+template <uint32_t T> constexpr uint32_t kWideScales = (T + 3) / 4 * 64;
 template <uint32_t T> constexpr uint32_t kWideStageVectors = (T + 1) / 2 * 2 * 2 * 64;
 template <uint32_t FMT, uint32_t T, bool Staged> constexpr uint32_t kWideSumVectors = FMT != GGUF_FMT_Q6K && !Staged ? (T + 3) / 4 * 4 * 64 : 1;
 
+// Two neighbouring columns in memory, aligned as one is.
+typedef uint32_t __attribute__((aligned(2), may_alias)) PairBits;
+typedef float __attribute__((ext_vector_type(2), aligned(4), may_alias)) PairFloats;
 // T: the row tiles a workgroup computes, at least those it takes (a tile past them multiplies zeros).
 template <uint32_t FMT, uint32_t EP, uint32_t T, bool Staged>
 __device__ __forceinline__ void wide_workgroup(const WideLds lds, const WideTile &w, const uint8_t *__restrict__ table, void *__restrict__ out,
@@ -522,6 +527,11 @@ __device__ __forceinline__ void wide_workgroup(const WideLds lds, const WideTile
     return 2u * (stage == 0 ? kWideSecondLoads<FMT> : stage == 2u ? kWideFirstLoads<FMT> : stage == 3u ? kWideLateLoads<FMT> : 0u);
   };
   constexpr auto rowLoads = [](uint32_t stage) constexpr { return kShare + (stage == 3u ? kSumShare : 0u); };
+  // (first of all loads, so that the first stage's wait and barrier are these's too)
+  if (wave < kWideScales<T> / 64u)
+    load_to_lds<4>(make_resource(table + gguf_wide_scales_offset(p.input_size, p.tiles) + tile0 * 64u, tilesHere * 64u), threadIdx.x * 4u,
+                   lds.scales + 64u * wave);
+  __builtin_amdgcn_sched_barrier(0);
   // (the loads before the first stage in the order of the stages that would have asked for them)
   fetch(0, std::integral_constant<uint32_t, 0>{});
   __builtin_amdgcn_sched_barrier(0);
@@ -621,30 +631,62 @@ __device__ __forceinline__ void wide_workgroup(const WideLds lds, const WideTile
       for (uint32_t t = 0; t < T; ++t) acc[r][t] = dot[r][t];
   }
   wait_loads<0>();   // (nothing is on its way into LDS when the workgroup gives it up)
-  // Element (t, v) of this lane is row 16 (tile0 + t) + 4 kq + v, column column[r] + c.
-  const float *inverse = reinterpret_cast<const float *>(table + gguf_wide_scales_offset(p.input_size, p.tiles));
+  // Element (t, v) of this lane is row 16 (tile0 + t) + 4 kq + v, column column[r] + c. Neighbouring lanes trade one of every
+  // two rows, so that a lane stores two columns of a row: half the stores, of twice the bytes. What a residual adds leaves
+  // memory for all of the tiles at once. (The scales were loaded here, a row's behind the test that the row is there, and a
+  // residual's values the same way: up to 32 waits for memory one after the other, about 10 us a workgroup. 2048 rows, us a
+  // launch before and now: the experts' gate/up 157 and 146, their down projection of three super-blocks 126 and 89, a
+  // 2048-wide hybrid's mixer inputs on average 131 and 106, 4096 -> 2048 with its residual 56 and 48; 777 rows of 25600 ->
+  // 5120 Q6_K 395 and 377, 5120 -> 10240 136 and 118.)
+  const uint32_t odd = c & 1u, pairColumn = c - odd;
+  constexpr bool kResidual = EP == GGUF_WIDE_RESIDUAL;
+  uint32_t residuals[kResidual ? T : 1][2][2];
+  if constexpr (kResidual) {
+    const uint32_t last = w.rows - 1u;   // (rows past the last read the last)
+#pragma unroll
+    for (uint32_t t = 0; t < T; ++t)
+#pragma unroll
+      for (uint32_t r = 0; r < 2; ++r)
+#pragma unroll
+        for (uint32_t pair = 0; pair < 2; ++pair)
+          if (t < tilesHere && w.image[r])
+            residuals[t][r][pair] = *reinterpret_cast<const PairBits *>(
+                &residual[size_t(min(16u * (tile0 + t) + 4u * kq + 2u * pair + odd, last)) * p.out_stride + column[r] + pairColumn]);
+  }
+  // a pair's values of the row that this lane stores: its own column's and its neighbour's, in order
+  auto trade = [&](float first, float second, float (&out)[2]) __attribute__((always_inline)) {
+    const float mine = odd ? second : first, theirs = lane_xor<1>(odd ? first : second);
+    out[0] = odd ? theirs : mine;
+    out[1] = odd ? mine : theirs;
+  };
 #pragma unroll
   for (uint32_t t = 0; t < T; ++t) {
     if (t >= tilesHere) break;
+    const f32x4 scale = *reinterpret_cast<const f32x4 *>(lds.scales + 16u * t + 4u * kq);
 #pragma unroll
-    for (uint32_t v = 0; v < 4; ++v) {
-      const uint32_t row = 16u * (tile0 + t) + 4u * kq + v;
-      if (row >= w.rows) continue;
-      const float scale = inverse[row];
-      if constexpr (kGateUp) {
-        if (!w.image[0]) continue;
-        const float gate = round_bf16(acc[0][t][v] * scale), up = round_bf16(acc[1][t][v] * scale);
-        static_cast<uint16_t *>(out)[size_t(row) * p.out_stride + column[0] + c] = uint16_t(float_to_bf16_bits(up * silu(gate)));
-      } else {
+    for (uint32_t pair = 0; pair < 2; ++pair) {
+      const uint32_t row = 16u * (tile0 + t) + 4u * kq + 2u * pair + odd;
 #pragma unroll
-        for (uint32_t r = 0; r < 2; ++r) {
-          if (!w.image[r]) continue;
-          const float value = acc[r][t][v] * scale;
-          const size_t at = size_t(row) * p.out_stride + column[r] + c;
-          if constexpr (EP == GGUF_WIDE_PARTIAL) static_cast<float *>(out)[size_t(split) * w.rows * p.out_stride + at] = value;
-          else if constexpr (EP == GGUF_WIDE_RESIDUAL)
-            static_cast<uint16_t *>(out)[at] = uint16_t(float_to_bf16_bits(value + bf16_bits_to_float(residual[at])));
-          else static_cast<uint16_t *>(out)[at] = uint16_t(float_to_bf16_bits(value));
+      for (uint32_t r = 0; r < (kGateUp ? 1u : 2u); ++r) {
+        if (!w.image[r]) continue;
+        float value[2], two[2];
+#pragma unroll
+        for (uint32_t i = 0; i < 2; ++i) {
+          const uint32_t v = 2u * pair + i;
+          value[i] = acc[r][t][v] * scale[v];
+          if constexpr (kGateUp) value[i] = round_bf16(acc[1][t][v] * scale[v]) * silu(round_bf16(value[i]));
+        }
+        trade(value[0], value[1], two);
+        if (row >= w.rows) continue;
+        const size_t at = size_t(row) * p.out_stride + column[r] + pairColumn;
+        if constexpr (EP == GGUF_WIDE_PARTIAL) {
+          *reinterpret_cast<PairFloats *>(static_cast<float *>(out) + size_t(split) * w.rows * p.out_stride + at) = PairFloats{two[0], two[1]};
+        } else {
+          if constexpr (kResidual) {
+            two[0] += bf16_bits_to_float(residuals[t][r][pair] & 0xFFFFu);
+            two[1] += bf16_bits_to_float(residuals[t][r][pair] >> 16);
+          }
+          *reinterpret_cast<PairBits *>(static_cast<uint16_t *>(out) + at) = float_to_bf16_bits(two[0]) | (float_to_bf16_bits(two[1]) << 16);
         }
       }
     }
@@ -673,7 +715,8 @@ __global__ __launch_bounds__(256, 2) void gguf_wide(const uint8_t *__restrict__ 
   wide_columns<FMT, EP == GGUF_WIDE_GATE_UP>(w, seg0, seg1, seg2, p, tail ? tallGroups + rest : rest / p.splits, wave);
   __shared__ uint4 rows0[kWideStageVectors<T>], rows1[kWideStageVectors<T>], rows2[kWideStageVectors<T>], rows3[kWideStageVectors<T>],
       sums[kWideSumVectors<FMT, T, Staged>];
-  const WideLds lds{rows0, rows1, rows2, rows3, sums};
+  __shared__ float scales[kWideScales<T>];
+  const WideLds lds{rows0, rows1, rows2, rows3, sums, scales};
   if (tail) wide_workgroup<FMT, EP, 4, Staged>(lds, w, table, out, residual, p);
   else wide_workgroup<FMT, EP, T, Staged>(lds, w, table, out, residual, p);
 }
@@ -703,7 +746,8 @@ __global__ __launch_bounds__(256, 2) void gguf_wide_moe(const uint8_t *__restric
   wide_columns<FMT, EP == GGUF_WIDE_GATE_UP>(w, seg0 + expertAt, seg1 + expertAt, seg0 + expertAt, p, item % p.groups, wave);
   __shared__ uint4 rows0[kWideStageVectors<T>], rows1[kWideStageVectors<T>], rows2[kWideStageVectors<T>], rows3[kWideStageVectors<T>],
       sums[kWideSumVectors<FMT, T, false>];
-  const WideLds lds{rows0, rows1, rows2, rows3, sums};
+  __shared__ float scales[kWideScales<T>];
+  const WideLds lds{rows0, rows1, rows2, rows3, sums, scales};
   if constexpr (T > 4u) {
     if (w.tilesHere <= 4u) return wide_workgroup<FMT, EP, 4, false>(lds, w, table, out, nullptr, p);
   }
