@@ -716,36 +716,37 @@ __device__ __forceinline__ void decode_workgroup(Shared &shared, const uint8_t *
     // sums whatever the kernel's row tiles, so a row's result does not depend on the block's height. A
     // thread takes RT parts of its row. The loads go out before the first weights', so the wait for
     // them leaves those in flight.
-    constexpr uint32_t kRows = 16u * RT, kParts = 16u, kThreadParts = 256u / kRows;
+    // (of three row tiles, 240 threads take five parts a turn)
+    constexpr uint32_t kRows = 16u * RT, kParts = 16u, kThreadParts = 256u / kRows, kTurns = (kParts + kThreadParts - 1u) / kThreadParts;
     // Eight entries of a part are loaded together and added in their order afterwards, so a part costs one round trip
     // to the cache, not one an entry; the first eight go out before the first weights and are added once those are
     // on their way. The squares are read through a resource of their own: an entry past the table's, a row past its
     // rows and every entry of a table without a deferred scale read as zero without touching memory (a squares entry
     // is a sum of squares: adding 0 changes nothing).
     constexpr uint32_t kChunk = 8u;
-    float squareSum[RT], loaded[RT][kChunk];
+    float squareSum[kTurns], loaded[kTurns][kChunk];
 #pragma unroll
-    for (int i = 0; i < RT; ++i) squareSum[i] = 0.f;
+    for (uint32_t i = 0; i < kTurns; ++i) squareSum[i] = 0.f;
     const uint32_t squareRow = threadIdx.x % kRows, squareEntries = p.input_size / 64u, squareStride = gguf_squares_stride(tiles) * 4u;
     const Resource squares = make_resource(table + gguf_table_squares_offset(p.input_size, tiles),
                                            p.deferred_scale && squareRow < 16u * tiles ? squareEntries * squareStride : 0u);
-    auto loadSquares = [&](int i, uint32_t base) {
+    auto loadSquares = [&](uint32_t i, uint32_t base) {
 #pragma unroll
       for (uint32_t e = 0; e < kChunk; ++e)
         loaded[i][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(squares, int((base + kParts * e) * squareStride + squareRow * 4u), 0, 0));
     };
-    auto addSquares = [&](int i) {
+    auto addSquares = [&](uint32_t i) {
 #pragma unroll
       for (uint32_t e = 0; e < kChunk; ++e) squareSum[i] += loaded[i][e];
     };
     auto loadFirstSquares = [&] {
 #pragma unroll
-      for (int i = 0; i < RT; ++i) loadSquares(i, threadIdx.x / kRows + kThreadParts * i);
+      for (uint32_t i = 0; i < kTurns; ++i) loadSquares(i, threadIdx.x / kRows + kThreadParts * i);
       __builtin_amdgcn_sched_barrier(0);
     };
     auto setRowScales = [&] {
 #pragma unroll
-      for (int i = 0; i < RT; ++i) {
+      for (uint32_t i = 0; i < kTurns; ++i) {
         addSquares(i);
         // a wider table: the part's further entries, eight at a time (these waits do reach the weights')
         if (p.deferred_scale)
@@ -756,7 +757,9 @@ __device__ __forceinline__ void decode_workgroup(Shared &shared, const uint8_t *
       }
       if (p.deferred_scale) {
 #pragma unroll
-        for (int i = 0; i < RT; ++i) scaleParts[256u * i + threadIdx.x] = squareSum[i];   // part (threadIdx.x / kRows + kThreadParts i) of row threadIdx.x % kRows
+        for (uint32_t i = 0; i < kTurns; ++i)
+          if (const uint32_t part = threadIdx.x / kRows + kThreadParts * i; (kThreadParts * kRows == 256u) || (threadIdx.x < kThreadParts * kRows && part < kParts))
+            scaleParts[part * kRows + squareRow] = squareSum[i];
         __syncthreads();
         if (threadIdx.x < kRows) {
           float total = 0.f;
@@ -802,11 +805,12 @@ __device__ __forceinline__ void decode_workgroup(Shared &shared, const uint8_t *
       // everywhere (down at 64 rows 69), five waves a SIMD spill (head at 16 rows 155).
       using Ring = DecodeRing<RT>;
       constexpr uint32_t kStages = 8u / Ring::kStageGroups;   // of a super-block
-      constexpr uint32_t kRowLoads = RT * Ring::kStageGroups / 4, kSumChunks = RT * kSumsPerBlock;
+      // (of three row tiles a wave takes what it would of four, and the fourth repeats the third's)
+      constexpr uint32_t kTall = RT == 3 ? 4 : RT, kRowLoads = kTall * Ring::kStageGroups / 4, kSumChunks = kTall * kSumsPerBlock;
       // a wave's sums: kSumLoads times 256 bytes, or a kilobyte at once; of fewer chunks than waves, two load the same
       constexpr uint32_t kSumBytes = kSumChunks == 16 ? 16u : 4u, kSumLoads = kSumChunks == 16 || kSumChunks < 4 ? 1 : kSumChunks / 4;
       constexpr uint32_t kWeightLoads = kRecordLoads<FMT>;
-      const uint32_t waveIndex = uint32_t(__builtin_amdgcn_readfirstlane(int(wave)));
+      const uint32_t waveIndex = min(uint32_t(__builtin_amdgcn_readfirstlane(int(wave))), RT == 3 ? 2u : 3u);
       const uint32_t rowChunk = kRowLoads * waveIndex, rowTile = rowChunk / Ring::kStageGroups;   // its kilobytes of a stage, one row tile's
       // (a row tile past the table's, and a super-block past the range, read as zeros)
       const Resource values = make_resource(table + (size_t(rowTile < tiles ? rowTile : 0) * G + 8u * b0) * 1024u, rowTile < tiles ? count * 8192u : 0u);
@@ -1493,6 +1497,7 @@ __global__ __launch_bounds__(256, 3) void gguf_decode_mixed(const uint8_t *__res
 }
 SP_REGISTER_KERNEL("gguf_decode_mixed_m16_a", &gguf_decode_mixed<1>);
 SP_REGISTER_KERNEL("gguf_decode_mixed_m32_a", &gguf_decode_mixed<2>);
+SP_REGISTER_KERNEL("gguf_decode_mixed_m48_a", &gguf_decode_mixed<3>);
 SP_REGISTER_KERNEL("gguf_decode_mixed_m64_a", &gguf_decode_mixed<4>);
 
 // The fused q|k|v projection that also prepares the attention block (GGUF_EPILOGUE_QKV_PREPARE): one format, or a format
@@ -1693,34 +1698,43 @@ SP_GGUF_MOE_DECODE("q80", GGUF_FMT_Q80);
 SP_GGUF_MOE_DECODE("iq4xs", GGUF_FMT_IQ4XS);
 SP_GGUF_MOE_DECODE("iq4nl", GGUF_FMT_IQ4NL);
 
-#define SP_GGUF_DECODE(fmt, FMT, rows, RT)                                                              \
+// (three row tiles: the projections of a step of 33 to 48 rows; what else takes such rows runs four)
+#define SP_GGUF_DECODE_TILES(fmt, FMT, rows, RT)                                                        \
   SP_REGISTER_KERNEL("gguf_decode_" fmt "_m" #rows "_a", &gguf_decode<FMT, RT, GGUF_EPILOGUE_PLAIN>);   \
   SP_REGISTER_KERNEL("gguf_decode_" fmt "_m" #rows "_a_f32", &gguf_decode<FMT, RT, GGUF_EPILOGUE_PLAIN_F32>); \
   SP_REGISTER_KERNEL("gguf_decode_" fmt "_m" #rows "_r", &gguf_decode<FMT, RT, GGUF_EPILOGUE_RESIDUAL>); \
   SP_REGISTER_KERNEL("gguf_decode_" fmt "_m" #rows "_g", &gguf_decode<FMT, RT, GGUF_EPILOGUE_GATE_UP>);  \
   SP_REGISTER_KERNEL("gguf_decode_" fmt "_m" #rows "_gt", &gguf_decode<FMT, RT, GGUF_EPILOGUE_GATE_UP_TABLE>); \
-  SP_REGISTER_KERNEL("gguf_decode_" fmt "_m" #rows "_rn", &gguf_decode<FMT, RT, GGUF_EPILOGUE_RESIDUAL_NORM>);                             \
+  SP_REGISTER_KERNEL("gguf_decode_" fmt "_m" #rows "_rn", &gguf_decode<FMT, RT, GGUF_EPILOGUE_RESIDUAL_NORM>)
+#define SP_GGUF_DECODE(fmt, FMT, rows, RT)                                                              \
+  SP_GGUF_DECODE_TILES(fmt, FMT, rows, RT);                                                             \
   SP_REGISTER_KERNEL("gguf_decode_qkv_" fmt "_m" #rows, &gguf_decode_qkv<FMT, RT>);                     \
   SP_REGISTER_KERNEL("gguf_staged_" fmt "_m" #rows "_a", &gguf_decode<FMT, RT, GGUF_EPILOGUE_PLAIN, true>); \
   SP_REGISTER_KERNEL("gguf_staged_" fmt "_m" #rows "_a_f32", &gguf_decode<FMT, RT, GGUF_EPILOGUE_PLAIN_F32, true>); \
   SP_REGISTER_KERNEL("gguf_staged_" fmt "_m" #rows "_r", &gguf_decode<FMT, RT, GGUF_EPILOGUE_RESIDUAL, true>)
 SP_GGUF_DECODE("q4k", GGUF_FMT_Q4K, 16, 1);
 SP_GGUF_DECODE("q4k", GGUF_FMT_Q4K, 32, 2);
+SP_GGUF_DECODE_TILES("q4k", GGUF_FMT_Q4K, 48, 3);
 SP_GGUF_DECODE("q4k", GGUF_FMT_Q4K, 64, 4);
 SP_GGUF_DECODE("q6k", GGUF_FMT_Q6K, 16, 1);
 SP_GGUF_DECODE("q6k", GGUF_FMT_Q6K, 32, 2);
+SP_GGUF_DECODE_TILES("q6k", GGUF_FMT_Q6K, 48, 3);
 SP_GGUF_DECODE("q6k", GGUF_FMT_Q6K, 64, 4);
 SP_GGUF_DECODE("q5k", GGUF_FMT_Q5K, 16, 1);
 SP_GGUF_DECODE("q5k", GGUF_FMT_Q5K, 32, 2);
+SP_GGUF_DECODE_TILES("q5k", GGUF_FMT_Q5K, 48, 3);
 SP_GGUF_DECODE("q5k", GGUF_FMT_Q5K, 64, 4);
 SP_GGUF_DECODE("q80", GGUF_FMT_Q80, 16, 1);
 SP_GGUF_DECODE("q80", GGUF_FMT_Q80, 32, 2);
+SP_GGUF_DECODE_TILES("q80", GGUF_FMT_Q80, 48, 3);
 SP_GGUF_DECODE("q80", GGUF_FMT_Q80, 64, 4);
 SP_GGUF_DECODE("iq4xs", GGUF_FMT_IQ4XS, 16, 1);
 SP_GGUF_DECODE("iq4xs", GGUF_FMT_IQ4XS, 32, 2);
+SP_GGUF_DECODE_TILES("iq4xs", GGUF_FMT_IQ4XS, 48, 3);
 SP_GGUF_DECODE("iq4xs", GGUF_FMT_IQ4XS, 64, 4);
 SP_GGUF_DECODE("iq4nl", GGUF_FMT_IQ4NL, 16, 1);
 SP_GGUF_DECODE("iq4nl", GGUF_FMT_IQ4NL, 32, 2);
+SP_GGUF_DECODE_TILES("iq4nl", GGUF_FMT_IQ4NL, 48, 3);
 SP_GGUF_DECODE("iq4nl", GGUF_FMT_IQ4NL, 64, 4);
 
 // ---------------------------------------------------------------------------------------------

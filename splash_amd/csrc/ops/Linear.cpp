@@ -299,8 +299,12 @@ Linear::Resolved Linear::resolve(LinearBuffers b, const Projection &p, const Lin
   // Unused bindings still name a buffer: the table stands in for them.
   const hip::Buffer &spare = b.scratch.input;
   const bool staged = c.tile == LinearTile::GgufStaged;
+  // A step of 33 to 48 rows runs three row tiles (scratch is sized for the four that a chain of such rows runs). 40 rows by
+  // four and by three, us a launch: 5120 x 2 x 25600 Q4_K gate/up 64.3 and 56.0, 25600 x 5120 Q6_K 62.1 and 53.9, 5120 -> 10240
+  // 25.0 and 21.8, 5120 -> 151936 Q6_K 321 and 253, 2048 -> 12288 16.0 and 14.4.
+  const uint32_t kernelRows = !staged && w.rows > 32 && w.rows <= 48 ? 48 : plan.storageRows();
   const std::string name = std::string(staged ? "gguf_staged_" : "gguf_decode_") + (mixed ? "mixed" : segments.front().name()) + "_m" +
-                           std::to_string(plan.storageRows()) + epilogueSuffix(w.epilogue, plan.destination(), writesTable);
+                           std::to_string(kernelRows) + epilogueSuffix(w.epilogue, plan.destination(), writesTable);
   if (norms) {
     images[1] = b.normWeight;
     images[2] = b.nextTable;

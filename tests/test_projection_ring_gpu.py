@@ -5,6 +5,8 @@ import pytest
 from splash_amd import ops
 from tests import oracle as orc
 from tests.test_gguf_gpu import ALL_FORMATS, run_projection
+from tests.test_gguf_gpu import test_gate_up_table_epilogue_equals_the_table_pass as gate_up_table
+from tests.test_gguf_gpu import test_residual_norm_epilogue as residual_norm
 
 pytestmark = pytest.mark.gpu
 
@@ -28,3 +30,26 @@ def test_short_ranges_at_every_height(backend, fmt, blocks):
         for rows in (1, 16, 17, 32, 33, 48):
             part, _, _ = run_projection(backend, linear, fmt, [(N, native)], K, x[:rows], float32=True, splits=splits, whole_groups=0)
             assert part.tobytes() == full[:rows].tobytes(), rows
+
+
+@pytest.mark.parametrize("M", [33, 40, 48])
+def test_three_row_tiles_write_what_four_do(backend, M):
+    """Steps of 33 to 48 rows: the residual and gate/up rows, whole and in parts, are those of a 64-row block bit for bit; the
+    tables that gate/up and the norming residual leave are held to what they are at other heights."""
+    print(f"case three row tiles M={M}", flush=True)
+    rng = np.random.default_rng(M)
+    N, K = 320, 1280
+    linear = ops.Linear(backend)
+    for fmt in (ops.FMT_Q4K, ops.FMT_Q6K):
+        native, gate = orc.make_native(fmt, N, K, 70), orc.make_native(fmt, N, K, 71)
+        x, residual = (orc.f32_to_bf16(rng.standard_normal((64, width)).astype(np.float32)) for width in (K, N))
+        for splits, whole in ((1, 0), (3, 1)):
+            for extra in (dict(epilogue=ops.EPILOGUE_RESIDUAL, residual_bits=residual), dict(epilogue=ops.EPILOGUE_GATE_UP, gate_native=gate)):
+                full, _, _ = run_projection(backend, linear, fmt, [(N, native)], K, x, splits=splits, whole_groups=whole, **extra)
+                if "residual_bits" in extra:
+                    extra["residual_bits"] = residual[:M]
+                part, _, _ = run_projection(backend, linear, fmt, [(N, native)], K, x[:M], splits=splits, whole_groups=whole, **extra)
+                assert part.tobytes() == full[:M].tobytes()
+    gate_up_table(backend, M)
+    for fmt, n, k, config in ((ops.FMT_Q4K, 512, 768, None), (ops.FMT_Q6K, 512, 2048, None)):
+        residual_norm(backend, fmt, n, k, M, config)
