@@ -211,10 +211,16 @@ GGUF_INLINE uint64_t gguf_wide_table_bytes(uint32_t k, uint32_t rows) {
   const uint32_t tiles = gguf_wide_tiles(rows);
   return gguf_wide_scales_offset(k, tiles) + tiles * GGUF_ROW_TILE * 4u;
 }
+// The rows' tables: a wide table's operands and sums row by row, so that a row can be gathered by lines of its own: the values
+// fp16 [K / 256][8 groups][4 quarters][8], then the sums' [K / 256][4][8], up to whole 128-byte lines. After the rows fp32
+// [rows]: 2^-e.
+GGUF_INLINE uint32_t gguf_wide_row_bytes(uint32_t k) { return (k * 2u + k / GGUF_BLOCK * 64u + 127u) / 128u * 128u; }
+GGUF_INLINE uint64_t gguf_wide_rows_bytes(uint32_t k, uint32_t rows) { return uint64_t(rows) * (gguf_wide_row_bytes(k) + 4u); }
 #endif
 // gguf_wide_table: bf16 rows of up to 8192 inputs -> the wide table (_long: up to 32768); gguf_wide_table_norm: the rows'
-// RMS norm (weights bf16 [K]) on the way, bf16((x * inverse) * weight) as norm_rms writes it. Grid (64 * ceil(16 tiles /
-// 64)), 256 threads: a workgroup a row.
+// RMS norm (weights bf16 [K]) on the way, bf16((x * inverse) * weight) as norm_rms writes it; gguf_wide_table_norm_rows: that
+// and the rows' tables beside it. Grid (64 * ceil(16 tiles / 64)), 256 threads: a workgroup a row. gguf_wide_rows: the rows'
+// tables of bf16 rows of up to 8192 inputs, grid (rows), 256 threads.
 struct GgufWideTableParams {
   uint32_t input_size;
   uint32_t rows;
@@ -245,7 +251,8 @@ struct GgufWideParams {
 };
 // gguf_wide_moe_<fmt>_t<T>_{a,g}: the routed experts of a chunk (abi/Moe.h, MoeChunkTask): wide.rows, .row_groups and
 // .splits are unused. Binds the experts' images (gate and up, or down twice), the slots' wide table, the slots' output rows,
-// the tasks and their totals. Grid (8 * ceil(most tasks * groups / 8)).
+// the tasks and their totals. _x: the gate/up pair of rows that the slots gather; wide.rows rows, their tables in the wide
+// table's place, and the slots' rows bound last. Grid (8 * ceil(most tasks * groups / 8)).
 struct GgufWideMoeParams {
   struct GgufWideParams wide;
   uint64_t expert_bytes;  // between experts' images of a tensor

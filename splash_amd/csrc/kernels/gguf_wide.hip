@@ -41,11 +41,12 @@ __device__ __forceinline__ f16x2 both(float v) { return f16x2{_Float16(v), _Floa
 // `Waves` waves a row, whose values stay in registers from their one load to where `put` stores them: thread t of them holds
 // the eight inputs of quarter t % 4 of groups t / 4, 16 Waves + t / 4, ... in `Held` pieces. put(line, g, kq, entry): the
 // row's place among the sixteen of line `line` of its tile (a line: one quarter of one operand, sixteen rows of 16 bytes).
+// Returns the row's scale.
 // (The operands, the parts of their sums and the scale are the same bits whatever Waves is; a norm's sum of squares is added
 // over four waves.)
 template <bool Norm, uint32_t Held, uint32_t Waves, class Put>
-__device__ __forceinline__ void wide_table_row(const uint16_t *__restrict__ input, const uint16_t *__restrict__ weight, uint8_t *__restrict__ table,
-                                               const GgufWideTableParams &p, const uint32_t row, const uint32_t source, Put &&put) {
+__device__ __forceinline__ float wide_table_row(const uint16_t *__restrict__ input, const uint16_t *__restrict__ weight, const GgufWideTableParams &p,
+                                                const uint32_t source, Put &&put) {
   static_assert(Waves == 4u || (Waves == 1u && !Norm), "a row of one wave has no other wave's sums to add");
   __shared__ float scratch[8];
   constexpr uint32_t kPiece = 16u * Waves;   // groups of 32 inputs a piece
@@ -153,7 +154,10 @@ __device__ __forceinline__ void wide_table_row(const uint16_t *__restrict__ inpu
       const uint32_t b = lane_down<8>(two), c = uint32_t(__shfl_down(int(two), 16, 64)), d = uint32_t(__shfl_down(int(two), 24, 64));
       if ((g & 7u) == 0 && g < groups) put(((g >> 3) * GGUF_WIDE_OPERANDS + 8u) * 4u + kq, 8u, kq, make_uint4(two, b, c, d));
     }
-  if (tid == 0) reinterpret_cast<float *>(table + gguf_wide_scales_offset(p.input_size, p.tiles))[row] = inverseScale;
+  return inverseScale;
+}
+__device__ __forceinline__ float *wide_scales_of(uint8_t *table, const GgufWideTableParams &p) {
+  return reinterpret_cast<float *>(table + gguf_wide_scales_offset(p.input_size, p.tiles));
 }
 __device__ __forceinline__ uint32_t wide_table_row_of(uint32_t block) {
   const uint32_t die = block % 8u, slot = block / 8u;
@@ -165,9 +169,10 @@ template <bool Norm, uint32_t Held>
 __device__ __forceinline__ void wide_table_row_out(const uint16_t *__restrict__ input, const uint16_t *__restrict__ weight, uint8_t *__restrict__ table,
                                                    const GgufWideTableParams &p, const uint32_t row, const uint32_t source) {
   uint4 *values = reinterpret_cast<uint4 *>(table + row / 16u * gguf_wide_tile_bytes(p.input_size)) + row % 16u;
-  wide_table_row<Norm, Held, 4>(input, weight, table, p, row, source, [&](uint32_t line, uint32_t, uint32_t, uint4 entry) __attribute__((always_inline)) {
+  const float scale = wide_table_row<Norm, Held, 4>(input, weight, p, source, [&](uint32_t line, uint32_t, uint32_t, uint4 entry) __attribute__((always_inline)) {
     values[size_t(line) * 16u] = entry;
   });
+  if (threadIdx.x == 0) wide_scales_of(table, p)[row] = scale;
 }
 template <bool Norm, uint32_t Held>
 __global__ __launch_bounds__(256) void gguf_wide_table(const uint16_t *__restrict__ input, const uint16_t *__restrict__ weight,
@@ -175,8 +180,40 @@ __global__ __launch_bounds__(256) void gguf_wide_table(const uint16_t *__restric
   const uint32_t row = wide_table_row_of(blockIdx.x);
   if (row < 16u * p.tiles) wide_table_row_out<Norm, Held>(input, weight, table, p, row, row);
 }
-// The table of the rows that a mixture's slots gather (or, Gathers false, of the slots' own rows): row s is row slot_row[s]
-// of the input, zeros where the slot is empty, for the slots of the tiles there are.
+// Where a row's table (abi/Gguf.h) has entry `kq` of operand `operand` of the super-block that `line` is of.
+__device__ __forceinline__ uint4 *wide_row_entry(uint8_t *of, uint32_t inputSize, uint32_t line, uint32_t operand, uint32_t kq) {
+  const uint32_t block = (line / 4u - operand) / GGUF_WIDE_OPERANDS;
+  return reinterpret_cast<uint4 *>(of + (operand < 8u ? (block * 8u + operand) * 64u : inputSize * 2u + block * 64u) + 16u * kq);
+}
+// The rows' tables, a workgroup a row: whole lines of the row's own.
+__global__ __launch_bounds__(256) void gguf_wide_rows(const uint16_t *__restrict__ input, uint8_t *__restrict__ rows, GgufWideTableParams p) {
+  const uint32_t row = blockIdx.x, bytes = gguf_wide_row_bytes(p.input_size);
+  if (row >= p.rows) return;
+  uint8_t *of = rows + size_t(row) * bytes;
+  const float scale = wide_table_row<false, 4, 4>(input, nullptr, p, row, [&](uint32_t line, uint32_t operand, uint32_t kq, uint4 entry) __attribute__((always_inline)) {
+    *wide_row_entry(of, p.input_size, line, operand, kq) = entry;
+  });
+  if (threadIdx.x == 0) reinterpret_cast<float *>(rows + size_t(p.rows) * bytes)[row] = scale;
+}
+// The normed rows as both: their wide table, and the rows' tables (2048 rows of 2048 inputs 10.0 us, 8.0 without the latter).
+__global__ __launch_bounds__(256) void gguf_wide_table_norm_rows(const uint16_t *__restrict__ input, const uint16_t *__restrict__ weight,
+                                                                 uint8_t *__restrict__ table, uint8_t *__restrict__ rows, GgufWideTableParams p) {
+  const uint32_t row = wide_table_row_of(blockIdx.x), bytes = gguf_wide_row_bytes(p.input_size);
+  if (row >= 16u * p.tiles) return;
+  uint4 *values = reinterpret_cast<uint4 *>(table + row / 16u * gguf_wide_tile_bytes(p.input_size)) + row % 16u;
+  uint8_t *of = rows + size_t(row) * bytes;
+  const float scale = wide_table_row<true, 4, 4>(input, weight, p, row, [&](uint32_t line, uint32_t operand, uint32_t kq, uint4 entry) __attribute__((always_inline)) {
+    values[size_t(line) * 16u] = entry;
+    if (row < p.rows) *wide_row_entry(of, p.input_size, line, operand, kq) = entry;
+  });
+  if (threadIdx.x == 0) {
+    wide_scales_of(table, p)[row] = scale;
+    if (row < p.rows) reinterpret_cast<float *>(rows + size_t(p.rows) * bytes)[row] = scale;
+  }
+}
+// The table of a mixture's slots' own rows (or, Gathers, of the rows that they gather: row s is row slot_row[s] of the input;
+// a chunk's gate/up pair gathers from the rows' tables instead, and this is what it is held against), zeros where the slot is
+// empty, for the slots of the tiles there are.
 template <bool Gathers>
 __global__ __launch_bounds__(256) void gguf_wide_moe_table(const uint16_t *__restrict__ input, const uint32_t *__restrict__ slot_row,
                                                            const uint32_t *__restrict__ tile_total, uint8_t *__restrict__ table,
@@ -203,9 +240,10 @@ __global__ __launch_bounds__(1024) void gguf_wide_moe_tile(const uint16_t *__res
   if (tile >= min(p.tiles, tile_total[0])) return;
   auto turned = [](uint32_t place, uint32_t operand, uint32_t kq) __attribute__((always_inline)) { return place ^ ((4u * operand + kq) & 15u); };
   const uint32_t source = slot_row[row];
-  wide_table_row<false, GGUF_WIDE_TILE_INPUTS / 512u, 1>(
-      input, nullptr, table, p, row, Gathers || source == MOE_NO_ROW ? source : row,
+  const float scale = wide_table_row<false, GGUF_WIDE_TILE_INPUTS / 512u, 1>(
+      input, nullptr, p, Gathers || source == MOE_NO_ROW ? source : row,
       [&](uint32_t line, uint32_t operand, uint32_t kq, uint4 entry) __attribute__((always_inline)) { staged[line * 16u + turned(r, operand, kq)] = entry; });
+  if ((threadIdx.x & 63u) == 0) wide_scales_of(table, p)[row] = scale;
   __syncthreads();
   uint4 *values = reinterpret_cast<uint4 *>(table + tile * gguf_wide_tile_bytes(p.input_size));
   const uint32_t entries = p.input_size / 256u * GGUF_WIDE_OPERANDS * 64u;
@@ -219,6 +257,8 @@ SP_REGISTER_KERNEL("gguf_wide_moe_rows", &gguf_wide_moe_table<false>);
 SP_REGISTER_KERNEL("gguf_wide_table", (&gguf_wide_table<false, 4>));
 SP_REGISTER_KERNEL("gguf_wide_table_long", (&gguf_wide_table<false, 16>));
 SP_REGISTER_KERNEL("gguf_wide_table_norm", (&gguf_wide_table<true, 4>));
+SP_REGISTER_KERNEL("gguf_wide_rows", &gguf_wide_rows);
+SP_REGISTER_KERNEL("gguf_wide_table_norm_rows", &gguf_wide_table_norm_rows);
 
 // ---------------------------------------------------------------------------------------------
 // The wide projection.
@@ -459,10 +499,14 @@ template <uint32_t FMT, uint32_t T, bool Staged> constexpr uint32_t kWideSumVect
 // Two neighbouring columns in memory, aligned as one is.
 typedef uint32_t __attribute__((aligned(2), may_alias)) PairBits;
 typedef float __attribute__((ext_vector_type(2), aligned(4), may_alias)) PairFloats;
-// T: the row tiles a workgroup computes, at least those it takes (a tile past them multiplies zeros).
-template <uint32_t FMT, uint32_t EP, uint32_t T, bool Staged>
+// T: the row tiles a workgroup computes, at least those it takes (a tile past them multiplies zeros). Gathers: `table` holds
+// the rows' tables (of p.rows rows), and slot s is row slot_row[s]. Eight neighbouring lanes fetch a line of a row, both
+// groups of a stage; in LDS the row's eight places are turned by half the row's number, so that the sixteen rows that a
+// quarter of the wave reads lie in all the banks.
+template <uint32_t FMT, uint32_t EP, uint32_t T, bool Staged, bool Gathers = false>
 __device__ __forceinline__ void wide_workgroup(const WideLds lds, const WideTile &w, const uint8_t *__restrict__ table, void *__restrict__ out,
-                                               const uint16_t *__restrict__ residual, const GgufWideParams &p) {
+                                               const uint16_t *__restrict__ residual, const GgufWideParams &p,
+                                               const uint32_t *__restrict__ slot_row = nullptr) {
   constexpr uint32_t kRecord = gguf_record_bytes(FMT);
   constexpr bool kSums = FMT != GGUF_FMT_Q6K && !Staged, kTwice = FMT == GGUF_FMT_Q6K && !Staged, kGateUp = EP == GGUF_WIDE_GATE_UP;
   const uint32_t lane = threadIdx.x & 63u, c = lane & 15u, kq = lane >> 4;
@@ -474,7 +518,8 @@ __device__ __forceinline__ void wide_workgroup(const WideLds lds, const WideTile
     weights[r] = make_resource(w.image[r] ? w.image[r] + size_t(b0) * kRecord : table, w.image[r] ? count * kRecord : 0u);
   const uint32_t tileBytes = uint32_t(gguf_wide_tile_bytes(p.input_size));
   // (row tiles past the workgroup's, and super-blocks past its range, read as zeros or are not used)
-  const Resource rowValues = make_resource(table + size_t(tile0) * tileBytes, tilesHere * tileBytes);
+  const uint32_t rowBytes = gguf_wide_row_bytes(p.input_size);
+  const Resource rowValues = Gathers ? make_resource(table, p.rows * rowBytes) : make_resource(table + size_t(tile0) * tileBytes, tilesHere * tileBytes);
 
   f32x4 acc[2][T], dot[2][T];
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
@@ -489,15 +534,49 @@ __device__ __forceinline__ void wide_workgroup(const WideLds lds, const WideTile
   const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)));
   const uint32_t mineAt = (threadIdx.x >> 7) * tileBytes + (threadIdx.x & 127u) * 16u;
   const uint32_t sumsAt = (threadIdx.x >> 6) * tileBytes + lane * 16u;
+  // Of gathered rows: where this lane's row begins, a share's tiles; past every row for an empty slot, which reads as zeros.
+  constexpr uint32_t kNowhere = 0xC0000000u;
+  uint32_t rowAt[Gathers ? kShare : 1], rowSumsAt[Gathers && kSums ? kSumShare : 1], scaleAt = 0;
+  if constexpr (Gathers) {
+    auto sourceOf = [&](uint32_t tile, uint32_t r) __attribute__((always_inline)) {
+      const uint32_t source = slot_row[16u * (tile0 + min(tile, tilesHere - 1u)) + r];
+      return tile < tilesHere ? source : MOE_NO_ROW;
+    };
+    const uint32_t r = (threadIdx.x & 127u) >> 3, piece = (threadIdx.x & 7u) ^ (r >> 1), sumRow = lane >> 2, sumPiece = (lane & 3u) ^ (sumRow >> 2);
+#pragma unroll
+    for (uint32_t i = 0; i < kShare; ++i) {
+      const uint32_t source = sourceOf(2u * i + (threadIdx.x >> 7), r);
+      rowAt[i] = source < p.rows ? source * rowBytes + 16u * piece : kNowhere;
+    }
+    if constexpr (kSums) {
+#pragma unroll
+      for (uint32_t i = 0; i < kSumShare; ++i) {
+        const uint32_t source = sourceOf(4u * i + wave, sumRow);
+        rowSumsAt[i] = source < p.rows ? source * rowBytes + p.input_size * 2u + 16u * sumPiece : kNowhere;
+      }
+    }
+    const uint32_t source = sourceOf(threadIdx.x >> 4, threadIdx.x & 15u);
+    scaleAt = source < p.rows ? source * 4u : kNowhere;
+  }
   auto stageRows = [&](auto stageConstant) __attribute__((always_inline)) -> uint4 * {
     constexpr uint32_t S = decltype(stageConstant)::value;
     return S == 0 ? lds.rows0 : S == 1 ? lds.rows1 : S == 2 ? lds.rows2 : lds.rows3;
   };
   auto fetch = [&](uint32_t block, auto stageConstant) __attribute__((always_inline)) {   // block counts from b0
     constexpr uint32_t S = decltype(stageConstant)::value;
-    // (past the part of K: zeros, no traffic)
-    const uint32_t at = block < count ? (b0 + block) * (GGUF_WIDE_OPERANDS * 1024u) + S * 2048u : 0x80000000u;
     uint4 *to = stageRows(stageConstant) + 64u * wave;
+    // (past the part of K: zeros, no traffic)
+    if constexpr (Gathers) {
+      const uint32_t past = block < count ? 0u : 0x80000000u;
+#pragma unroll
+      for (uint32_t i = 0; i < kShare; ++i) load_to_lds<16>(rowValues, rowAt[i] + (past + (b0 + block) * 512u + S * 128u), to + 256u * i);
+      if constexpr (S == 3u && kSums) {
+#pragma unroll
+        for (uint32_t i = 0; i < kSumShare; ++i) load_to_lds<16>(rowValues, rowSumsAt[i] + (past + (b0 + block) * 64u), lds.sums + 64u * wave + 256u * i);
+      }
+      return;
+    }
+    const uint32_t at = block < count ? (b0 + block) * (GGUF_WIDE_OPERANDS * 1024u) + S * 2048u : 0x80000000u;
 #pragma unroll
     for (uint32_t i = 0; i < kShare; ++i) load_to_lds<16>(rowValues, mineAt + (at + 2u * i * tileBytes), to + 256u * i);
     if constexpr (S == 3u) {
@@ -528,7 +607,9 @@ __device__ __forceinline__ void wide_workgroup(const WideLds lds, const WideTile
   };
   constexpr auto rowLoads = [](uint32_t stage) constexpr { return kShare + (stage == 3u ? kSumShare : 0u); };
   // (first of all loads, so that the first stage's wait and barrier are these's too)
-  if (wave < kWideScales<T> / 64u)
+  if (Gathers && wave < kWideScales<T> / 64u)
+    load_to_lds<4>(make_resource(table + size_t(p.rows) * rowBytes, p.rows * 4u), scaleAt, lds.scales + 64u * wave);
+  if (!Gathers && wave < kWideScales<T> / 64u)
     load_to_lds<4>(make_resource(table + gguf_wide_scales_offset(p.input_size, p.tiles) + tile0 * 64u, tilesHere * 64u), threadIdx.x * 4u,
                    lds.scales + 64u * wave);
   __builtin_amdgcn_sched_barrier(0);
@@ -578,8 +659,8 @@ __device__ __forceinline__ void wide_workgroup(const WideLds lds, const WideTile
       f16x8 a[2][3];
       auto read = [&](uint32_t t) {
 #pragma unroll
-        for (uint32_t g = 0; g < 2; ++g) a[t & 1u][g] = as_f16x8(rows[(t * 2u + g) * 64u + lane]);
-        if constexpr (kReads == 3u) a[t & 1u][2] = as_f16x8(lds.sums[t * 64u + lane]);
+        for (uint32_t g = 0; g < 2; ++g) a[t & 1u][g] = as_f16x8(rows[t * 128u + (Gathers ? 8u * c + ((4u * g + kq) ^ (c >> 1)) : g * 64u + lane)]);
+        if constexpr (kReads == 3u) a[t & 1u][2] = as_f16x8(lds.sums[t * 64u + (Gathers ? 4u * c + (kq ^ (c >> 2)) : lane)]);
       };
       read(0);
 #pragma unroll
@@ -726,10 +807,10 @@ __global__ __launch_bounds__(256, 2) void gguf_wide(const uint8_t *__restrict__ 
 // takes the one that fits. A task's weights are converted once, whatever its height: 2048 rows of 128 experts, 8 a row,
 // 7 to 10 tiles an expert, in tasks of up to eight 164 and 130 us a layer's gate/up and down, in tasks of five that were
 // always computed as five 195 and 151.
-template <uint32_t FMT, uint32_t EP, uint32_t T>
-__global__ __launch_bounds__(256, 2) void gguf_wide_moe(const uint8_t *__restrict__ seg0, const uint8_t *__restrict__ seg1, const uint8_t *__restrict__ table,
-                                                        void *__restrict__ out, const MoeChunkTask *__restrict__ tasks,
-                                                        const uint32_t *__restrict__ totals, GgufWideMoeParams m) {
+template <uint32_t FMT, uint32_t EP, uint32_t T, bool Gathers>
+__device__ __forceinline__ void wide_moe(const uint8_t *__restrict__ seg0, const uint8_t *__restrict__ seg1, const uint8_t *__restrict__ table,
+                                         void *__restrict__ out, const MoeChunkTask *__restrict__ tasks, const uint32_t *__restrict__ totals,
+                                         const uint32_t *__restrict__ slot_row, const GgufWideMoeParams &m) {
   const GgufWideParams &p = m.wide;
   const uint32_t items = totals[1] * p.groups, perDie = (items + 7u) / 8u, item = (blockIdx.x % 8u) * perDie + blockIdx.x / 8u;
   if (blockIdx.x / 8u >= perDie || item >= items) return;
@@ -749,14 +830,31 @@ __global__ __launch_bounds__(256, 2) void gguf_wide_moe(const uint8_t *__restric
   __shared__ float scales[kWideScales<T>];
   const WideLds lds{rows0, rows1, rows2, rows3, sums, scales};
   if constexpr (T > 4u) {
-    if (w.tilesHere <= 4u) return wide_workgroup<FMT, EP, 4, false>(lds, w, table, out, nullptr, p);
+    if (w.tilesHere <= 4u) return wide_workgroup<FMT, EP, 4, false, Gathers>(lds, w, table, out, nullptr, p, slot_row);
   }
   if constexpr (T == 8u) {
-    if (w.tilesHere == 5u) return wide_workgroup<FMT, EP, 5, false>(lds, w, table, out, nullptr, p);
-    if (w.tilesHere == 6u) return wide_workgroup<FMT, EP, 6, false>(lds, w, table, out, nullptr, p);
-    if (w.tilesHere == 7u) return wide_workgroup<FMT, EP, 7, false>(lds, w, table, out, nullptr, p);
+    if (w.tilesHere == 5u) return wide_workgroup<FMT, EP, 5, false, Gathers>(lds, w, table, out, nullptr, p, slot_row);
+    if (w.tilesHere == 6u) return wide_workgroup<FMT, EP, 6, false, Gathers>(lds, w, table, out, nullptr, p, slot_row);
+    if (w.tilesHere == 7u) return wide_workgroup<FMT, EP, 7, false, Gathers>(lds, w, table, out, nullptr, p, slot_row);
   }
-  wide_workgroup<FMT, EP, T, false>(lds, w, table, out, nullptr, p);
+  wide_workgroup<FMT, EP, T, false, Gathers>(lds, w, table, out, nullptr, p, slot_row);
+}
+template <uint32_t FMT, uint32_t EP, uint32_t T>
+__global__ __launch_bounds__(256, 2) void gguf_wide_moe(const uint8_t *__restrict__ seg0, const uint8_t *__restrict__ seg1, const uint8_t *__restrict__ table,
+                                                        void *__restrict__ out, const MoeChunkTask *__restrict__ tasks,
+                                                        const uint32_t *__restrict__ totals, GgufWideMoeParams m) {
+  wide_moe<FMT, EP, T, false>(seg0, seg1, table, out, tasks, totals, nullptr, m);
+}
+// The gate/up pair of the rows that the slots gather, from the rows' tables. A table of the slots holds a row as often as it
+// has routes, and writing it was a pass bound by memory (16384 slots of 2048 inputs: 27.8 us behind a norm's 9.5, for the 2.0
+// that the rows' tables add to the norm's own table). The loads fetch a row's whole lines, as the slots' fetch a tile's, so the
+// pair itself takes little longer: 149.3 -> 152.8 us at 2048 rows, 8 of 128 experts, 2048 x 2 x 768 Q4_K.
+template <uint32_t FMT, uint32_t T>
+__global__ __launch_bounds__(256, 2) void gguf_wide_moe_gathered(const uint8_t *__restrict__ seg0, const uint8_t *__restrict__ seg1,
+                                                                 const uint8_t *__restrict__ rows, void *__restrict__ out,
+                                                                 const MoeChunkTask *__restrict__ tasks, const uint32_t *__restrict__ totals,
+                                                                 const uint32_t *__restrict__ slot_row, GgufWideMoeParams m) {
+  wide_moe<FMT, GGUF_WIDE_GATE_UP, T, true>(seg0, seg1, rows, out, tasks, totals, slot_row, m);
 }
 #define SP_GGUF_WIDE_T(fmt, FMT, T)                                                          \
   SP_REGISTER_KERNEL("gguf_wide_" fmt "_t" #T "_a", (&gguf_wide<FMT, GGUF_WIDE_PLAIN, T>));        \
@@ -783,6 +881,7 @@ SP_GGUF_WIDE("q6k", GGUF_FMT_Q6K);
 
 #define SP_GGUF_WIDE_MOE(fmt, FMT, T)                                                             \
   SP_REGISTER_KERNEL("gguf_wide_moe_" fmt "_t" #T "_g", (&gguf_wide_moe<FMT, GGUF_WIDE_GATE_UP, T>)); \
+  SP_REGISTER_KERNEL("gguf_wide_moe_" fmt "_t" #T "_x", (&gguf_wide_moe_gathered<FMT, T>)); \
   SP_REGISTER_KERNEL("gguf_wide_moe_" fmt "_t" #T "_a", (&gguf_wide_moe<FMT, GGUF_WIDE_PLAIN, T>))
 SP_GGUF_WIDE_MOE("q4k", GGUF_FMT_Q4K, 2);
 SP_GGUF_WIDE_MOE("q4k", GGUF_FMT_Q4K, 4);

@@ -459,7 +459,7 @@ void HybridVerify::encodeWidePrefillLayer(hip::CommandGraph &graph, uint32_t lay
   }
   ops::Linear::addWideTable(graph, mixed_, wideTable_, mixedWidth, tokens);
   linear_.addWide(graph, w.mixerOutput, wideTable_, next, residual, widePartials_, tokens);
-  ops::Linear::addWideNormTable(graph, next, w.postNorm, wideTable_, dims_.hidden, tokens);
+  ops::Linear::addWideNormTable(graph, next, w.postNorm, wideTable_, dims_.hidden, tokens, dims_.dense() ? hip::Buffer{} : moeChunk_.table);
   if (dims_.dense()) {
     linear_.addWideGateUp(graph, w.ffnGate, w.ffnUp, wideTable_, wideRows_, tokens);
     ops::Linear::addWideTable(graph, wideRows_, wideTable_, dims_.denseFfn, tokens);
@@ -467,8 +467,9 @@ void HybridVerify::encodeWidePrefillLayer(hip::CommandGraph &graph, uint32_t lay
     return;
   }
   linear_.addWide(graph, w.router, wideTable_, wideScores_, {}, widePartials_, tokens);
-  ops::Normalization::addRms(graph, next, w.postNorm, normalized_, dims_.hidden, tokens);
-  ops::MoE::addChunk(graph, wideScores_, dims_.experts, normalized_, next, residual, w.experts, moeChunk_, dims_.moeShape(), tokens, w.sharedScalarGate);
+  if (dims_.moeShape().sharedGate) ops::Normalization::addRms(graph, next, w.postNorm, normalized_, dims_.hidden, tokens);
+  ops::MoE::addChunk(graph, wideScores_, dims_.experts, normalized_, next, residual, w.experts, moeChunk_, dims_.moeShape(), tokens, w.sharedScalarGate,
+                     true);
 }
 
 void HybridVerify::addGdnPrefill(hip::CommandGraph &graph, const HybridLayer &w, uint32_t index, uint32_t tokens, uint64_t currentCell, uint64_t nextCell,

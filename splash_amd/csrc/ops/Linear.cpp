@@ -568,7 +568,7 @@ void Linear::addWideTable(hip::CommandGraph &graph, const hip::Buffer &input, co
 }
 
 void Linear::addWideNormTable(hip::CommandGraph &graph, const hip::Buffer &input, const hip::Buffer &weight, const hip::Buffer &table,
-                              uint32_t width, uint32_t rows) {
+                              uint32_t width, uint32_t rows, const hip::Buffer &rowTables) {
   if (!rows || rows > kMaximumPrefillRows) throw std::invalid_argument("a prompt chunk takes 1 to 16384 rows");
   if (!width || width % GGUF_BLOCK || width > kMaximumWideNormWidth)
     throw std::invalid_argument("a normed wide table takes whole super-blocks of up to 8192 inputs");
@@ -576,8 +576,14 @@ void Linear::addWideNormTable(hip::CommandGraph &graph, const hip::Buffer &input
   requireBytes(weight, uint64_t{width} * 2, "norm weight");
   requireBytes(table, gguf_wide_table_bytes(width, rows), "wide table");
   const uint32_t tiles = gguf_wide_tiles(rows);
-  graph.add("gguf_wide_table_norm", {input, weight, table}, GgufWideTableParams{width, rows, tiles, 0},
-            {64 * ((16 * tiles + 63) / 64), 1, 1}, {256, 1, 1});
+  const GgufWideTableParams params{width, rows, tiles, 0};
+  const hip::DispatchSize grid{64 * ((16 * tiles + 63) / 64), 1, 1};
+  if (rowTables) {
+    requireBytes(rowTables, gguf_wide_rows_bytes(width, rows), "row tables");
+    graph.add("gguf_wide_table_norm_rows", {input, weight, table, rowTables}, params, grid, {256, 1, 1});
+  } else {
+    graph.add("gguf_wide_table_norm", {input, weight, table}, params, grid, {256, 1, 1});
+  }
 }
 
 namespace {

@@ -1,0 +1,88 @@
+"""The experts' gate/up pair of a prompt chunk from the rows' own tables, gathered (kernels/gguf_wide.hip), against the same
+pair from a table of the slots: the same operands and the same sums, so the same bits."""
+import numpy as np
+import pytest
+
+import splash_amd
+from splash_amd import ops
+from tests import oracle as orc
+from tests.test_wide_kernels_gpu import FORMATS, TableParams, WideMoeParams, add_table, place, table_bytes, wide_tiles
+
+pytestmark = pytest.mark.gpu
+
+
+def row_bytes(K):
+    return -(-(K * 2 + K // 4) // 128) * 128
+
+
+def rows_of_table(table, K, rows):
+    """The rows' tables a wide table's bytes come to, without what fills their last lines."""
+    values = table[:wide_tiles(rows) * K // 256 * 9216].reshape(-1, K // 256, 9, 4, 16, 16)
+    values = values.transpose(0, 4, 1, 2, 3, 5).reshape(-1, K // 256, 9, 64)[:rows]
+    return np.concatenate([values[:, :, :8].reshape(rows, -1), values[:, :, 8].reshape(rows, -1)], axis=1)
+
+
+# tasks of every height up to T; a row of whole lines and rows whose lines are filled up; columns that end inside a group
+@pytest.mark.parametrize("T,K", [(2, 256), (4, 768), (5, 512), (8, 512), (8, 2048)])
+@pytest.mark.parametrize("name", list(FORMATS))
+def test_gathered_rows_give_the_slots_bits(backend, name, T, K):
+    fmt, N, experts, top_k, rows = FORMATS[name], 272, T + 2, 3, 700
+    print(f"case wide gathered {name} T={T} K={K}", flush=True)
+    rng = np.random.default_rng(T * K)
+    routes = rows * top_k
+    counts = [16 * height - int(rng.integers(0, 16)) for height in range(1, T + 1)] + [0]
+    selected = rng.permutation(np.repeat(np.arange(experts), counts + [routes - sum(counts)]))
+    b = place(backend, selected, experts, top_k, T)
+    tiles = routes // 16 + experts
+    images = [backend.from_array(np.concatenate([ops.pack_gguf_image(fmt, orc.make_native(fmt, N, K, seed + e), N, K) for e in range(experts)]))
+              for seed in (1, 50)]
+    x = backend.from_array(orc.f32_to_bf16((rng.standard_normal((rows, K)) * 0.02).astype(np.float32)))
+    p = WideMoeParams()
+    p.wide.input_size, p.wide.rows, p.wide.tiles, p.wide.out_stride, p.expert_bytes = K, rows, tiles, N, images[0].size_bytes // experts
+    p.wide.cols[0], p.wide.groups = N, -(-N // 64)
+    grid = (8 * -(-(tiles // T + experts) * p.wide.groups // 8), 1, 1)
+    got = []
+    for kind in ("slots", "rows"):
+        out = backend.allocate_buffer(16 * tiles * N * 2)
+        out.fill(0xA5)
+        graph = splash_amd.CommandGraph()
+        if kind == "slots":
+            table = backend.allocate_buffer(table_bytes(K, tiles))
+            table.fill(0xA5)
+            graph.add("gguf_wide_moe_gather", [x, b["slot_row"], b["totals"], table], TableParams(K, rows, tiles, 0), (64 * -(-16 * tiles // 64), 1, 1))
+            graph.add(f"gguf_wide_moe_{name}_t{T}_g", [images[0], images[1], table, out, b["tasks"], b["totals"]], p, grid)
+        else:
+            table = backend.allocate_buffer(rows * (row_bytes(K) + 4))
+            table.fill(0xA5)
+            graph.add("gguf_wide_rows", [x, table], TableParams(K, rows, tiles, 0), (rows, 1, 1))
+            graph.add(f"gguf_wide_moe_{name}_t{T}_x", [images[0], images[1], table, out, b["tasks"], b["totals"], b["slot_row"]], p, grid)
+        backend.run(graph)
+        got.append(out.download(np.uint16))
+    assert np.array_equal(got[0], got[1]) and (got[0] != 0xA5A5).any()
+
+
+@pytest.mark.parametrize("rows,K", [(1, 256), (17, 1792), (130, 8192)])
+def test_rows_tables_hold_what_the_wide_table_does(backend, rows, K):
+    """The rows' tables of rows and of their norms, and the wide table written beside the latter."""
+    print(f"case rows' tables {rows} K={K}", flush=True)
+    rng = np.random.default_rng(rows)
+    x = orc.f32_to_bf16((rng.standard_normal((rows, K)) * 10.0 ** rng.integers(-6, 7, (1, K))).astype(np.float32))
+    x[0, 3], x[rows - 1, 0], x[rows // 2, :5] = 0x7F80, 0x7FC1, 0
+    weight, tiles, size = orc.f32_to_bf16((1 + 0.1 * rng.standard_normal(K)).astype(np.float32)), wide_tiles(rows), row_bytes(K)
+    for normed in (False, True):
+        graph = splash_amd.CommandGraph()
+        table = add_table(graph, backend, x, weight if normed else None)
+        out, beside = backend.allocate_buffer(rows * (size + 4)), backend.allocate_buffer(table_bytes(K, tiles))
+        out.fill(0xA5)
+        beside.fill(0xA5)
+        params, source = TableParams(K, rows, tiles, 0), backend.from_array(x)
+        if normed:
+            graph.add("gguf_wide_table_norm_rows", [source, backend.from_array(weight), beside, out], params, (64 * -(-16 * tiles // 64), 1, 1))
+        else:
+            graph.add("gguf_wide_rows", [source, out], params, (rows, 1, 1))
+        backend.run(graph)
+        want, got = table.download(), out.download()
+        assert np.array_equal(got[:rows * size].reshape(rows, size)[:, :K * 2 + K // 4], rows_of_table(want, K, rows))
+        assert np.array_equal(got[rows * size:], want[tiles * (K // 256) * 9216:][:4 * rows])
+        if normed:
+            assert np.array_equal(beside.download(), want)
