@@ -107,6 +107,7 @@ struct GdnFoldParams {
 #define GDN_SCAN_STATE_ROWS 16u   // state rows of one scan workgroup (the reference's SPLASH_GDN_SCAN_STATE_ROWS)
 #define GDN_PREPARE_ROWS 8u   // consecutive rows of a wave of gdn_prefill_prepare
 #define GDN_GATE_ROWS 4u      // and of gdn_prefill_gate
+#define GDN_GATE_TABLE_WIDTH 8192u  // values of a row of gdn_prefill_gate_table, whose rows are a wide table's (abi/Gguf.h)
 #define GDN_SCAN_BLOCK 16u        // tokens a scan workgroup stages at a time
 // A run in blocks of GDN_SCAN_BLOCK tokens (gdn_prefill_blocks, gdn_prefill_block_scan): what a block needs that its rows and
 // gates alone decide. Per block and value head, fp32: T [16][16], the block's triangular system solved (its unknowns' right

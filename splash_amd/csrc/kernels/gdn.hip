@@ -23,6 +23,7 @@
 #include "abi/PagedAttention.h"  // AttentionTreeRow
 #include "backend/KernelRegistry.hpp"
 #include "kernels/gguf_records.hpp"   // buffer resources
+#include "kernels/gguf_wide_table.hpp"
 
 namespace splash::kernels {
 
@@ -1205,5 +1206,58 @@ __global__ __launch_bounds__(256) void gdn_prefill_gate(const uint16_t *__restri
   }
 }
 SP_REGISTER_KERNEL("gdn_prefill_gate", &gdn_prefill_gate);
+
+// gdn_prefill_gate_table: grid (64 * ceil(16 tiles / 64)), 256 threads, a workgroup a row of the chunk's wide table: the row's
+// gated heads, a wave every fourth one, eight heads' loads out together, meet in LDS and leave as the table the output
+// projection reads. The values and the table are the bits of gdn_prefill_gate and gguf_wide_table, whose rows between them
+// went to memory and back: 2048 rows of 32 heads 18.0 + 11.4 us in the two, 21.4 here (21.9 with four heads' loads out). Bound
+// by memory and what follows it in a row's workgroup, the sums and the scale. Up to GDN_GATE_TABLE_WIDTH values a row, 16 KB
+// of LDS: what the norms' tables hold; wider rows and an odd number of heads (half a super-block) take the two.
+__global__ __launch_bounds__(256) void gdn_prefill_gate_table(const uint16_t *__restrict__ recurrent_rows, const uint16_t *__restrict__ packed,
+                                                              const void *__restrict__ norm_weight, uint8_t *__restrict__ table,
+                                                              GdnPrefillParams p) {
+  constexpr uint32_t R = 8;
+  __shared__ __align__(16) uint16_t gatedRow[GDN_GATE_TABLE_WIDTH];
+  const GdnShapeParams s = p.shape;
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, row = wide_table_row_of(blockIdx.x);
+  const uint32_t tiles = gguf_wide_tiles(p.tokens), perKey = s.value_heads / s.key_heads, valueWidth = s.value_heads * kDim;
+  if (row >= 16u * tiles || valueWidth > GDN_GATE_TABLE_WIDTH) return;
+  const bool live = row < p.tokens;
+  if (live) {
+    const uint16_t *values = recurrent_rows + size_t(row) * valueWidth, *gates = packed + size_t(row) * s.packed_width + s.conv_dim;
+    float weight[2];
+#pragma unroll
+    for (uint32_t part = 0; part < 2; ++part) weight[part] = norm_weight_of(norm_weight, p.flags, lane + 64u * part);
+    for (uint32_t first = wave; first < s.value_heads; first += 4u * R) {
+      float value[R][2], z[R][2];
+#pragma unroll
+      for (uint32_t r = 0; r < R; ++r) {
+        const uint32_t head = min(first + 4u * r, s.value_heads - 1u);
+#pragma unroll
+        for (uint32_t part = 0; part < 2; ++part) {
+          value[r][part] = bf16_bits_to_float(values[head * kDim + lane + 64u * part]);
+          z[r][part] = bf16_bits_to_float(gates[head * kDim + lane + 64u * part]);
+        }
+      }
+#pragma unroll
+      for (uint32_t r = 0; r < R; ++r) {
+        const uint32_t head = first + 4u * r;
+        if (head >= s.value_heads) break;
+        const uint32_t outHead = (p.flags & GDN_TILED_HEADS) ? (head % perKey) * s.key_heads + head / perKey : head;
+        uint32_t gated[2];
+        gated_values(value[r], weight, z[r], p.flags, gated);
+#pragma unroll
+        for (uint32_t part = 0; part < 2; ++part) gatedRow[outHead * kDim + lane + 64u * part] = uint16_t(gated[part]);
+      }
+    }
+  }
+  __syncthreads();
+  const GgufWideTableParams t{valueWidth, 1u, tiles, 0u};
+  uint4 *entries = reinterpret_cast<uint4 *>(table + row / 16u * gguf_wide_tile_bytes(valueWidth)) + row % 16u;
+  const float scale = wide_table_row<false, 4, 4>(gatedRow, nullptr, t, live ? 0u : 1u, [&](uint32_t line, uint32_t, uint32_t, uint4 entry)
+                                                  __attribute__((always_inline)) { entries[size_t(line) * 16u] = entry; });
+  if (threadIdx.x == 0) wide_scales_of(table, t)[row] = scale;
+}
+SP_REGISTER_KERNEL("gdn_prefill_gate_table", &gdn_prefill_gate_table);
 
 } // namespace splash::kernels

@@ -448,6 +448,7 @@ void HybridVerify::encodeWidePrefillLayer(hip::CommandGraph &graph, uint32_t lay
   const uint32_t inputWidth = w.mixerInput.outputSize, mixedWidth = w.mixerOutput.inputSize;
   if (inputWidth != (attends ? dims_.qkvWidth() : dims_.gdnPackedWidth) || mixedWidth != (attends ? dims_.attentionWidth() : dims_.gdnWidth()))
     throw std::invalid_argument("the layer's projections do not fit the model");
+  const bool gates = !attends && ops::GDN::takesTable(dims_.gdnShape());   // straight into the output projection's table
   ops::Linear::addWideNormTable(graph, residual, w.inputNorm, wideTable_, dims_.hidden, tokens);
   linear_.addWide(graph, w.mixerInput, wideTable_, packed_, {}, widePartials_, tokens);
   if (attends) {
@@ -455,9 +456,9 @@ void HybridVerify::encodeWidePrefillLayer(hip::CommandGraph &graph, uint32_t lay
     ops::PagedAttention::addPromptProjection(graph, plan, {packed_, w.queryNorm, w.keyNorm, ropeCos_, ropeSin_}, attentionWorkspace_, pages);
     ops::PagedAttention::addPromptAttention(graph, plan, attentionWorkspace_, treeRows_, pages, mixed_, packed_);
   } else {
-    addGdnPrefill(graph, w, index, tokens, currentCell, nextCell, gdnBlocks_);
+    addGdnPrefill(graph, w, index, tokens, currentCell, nextCell, gdnBlocks_, gates ? wideTable_ : hip::Buffer{});
   }
-  ops::Linear::addWideTable(graph, mixed_, wideTable_, mixedWidth, tokens);
+  if (!gates) ops::Linear::addWideTable(graph, mixed_, wideTable_, mixedWidth, tokens);
   linear_.addWide(graph, w.mixerOutput, wideTable_, next, residual, widePartials_, tokens);
   ops::Linear::addWideNormTable(graph, next, w.postNorm, wideTable_, dims_.hidden, tokens, dims_.dense() ? hip::Buffer{} : moeChunk_.table);
   if (dims_.dense()) {
@@ -473,9 +474,10 @@ void HybridVerify::encodeWidePrefillLayer(hip::CommandGraph &graph, uint32_t lay
 }
 
 void HybridVerify::addGdnPrefill(hip::CommandGraph &graph, const HybridLayer &w, uint32_t index, uint32_t tokens, uint64_t currentCell, uint64_t nextCell,
-                                 const hip::Buffer &blocks) {
+                                 const hip::Buffer &blocks, const hip::Buffer &table) {
   ops::GdnPrefillBuffers buffers = gdnPrefill_;
   buffers.blocks = blocks;
+  buffers.hiddenTable = table;
   buffers.packed = packed_;
   buffers.convolutionWeights = w.convolutionWeights;
   buffers.states = states_;

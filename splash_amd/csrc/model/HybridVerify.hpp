@@ -213,7 +213,7 @@ private:
   void encodeWidePrefillLayer(hip::CommandGraph &graph, uint32_t layer, const ops::AttentionPromptPlan &plan, uint32_t tokens, uint64_t currentCell,
                               uint64_t nextCell);
   void addGdnPrefill(hip::CommandGraph &graph, const HybridLayer &layer, uint32_t index, uint32_t tokens, uint64_t currentCell, uint64_t nextCell,
-                     const hip::Buffer &blocks = {});
+                     const hip::Buffer &blocks = {}, const hip::Buffer &table = {});
   hip::Buffer gdnBlocks_;      // the terms of a wide chunk's scan in blocks
   hip::Buffer wideTable_, wideRows_, widePartials_, wideScores_;
   ops::MoeChunkWorkspace moeChunk_;

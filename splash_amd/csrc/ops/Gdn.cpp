@@ -106,7 +106,12 @@ void GDN::addPrefill(hip::CommandGraph &graph, const GdnPrefillBuffers &b, const
   requireBytes(b.decay, uint64_t{tokens} * shape.valueHeads * 4, "GDN decay rows");
   requireBytes(b.beta, uint64_t{tokens} * shape.valueHeads * 2, "GDN beta rows");
   requireBytes(b.recurrentRows, tokens * valueWidth * 2, "GDN recurrent rows");
-  requireBytes(b.hidden, tokens * valueWidth * 2, "GDN hidden rows");
+  if (b.hiddenTable) {
+    if (!takesTable(shape)) throw std::invalid_argument("a GDN row's table holds whole super-blocks of up to 8192 values");
+    requireBytes(b.hiddenTable, gguf_wide_table_bytes(uint32_t(valueWidth), tokens), "GDN hidden table");
+  } else {
+    requireBytes(b.hidden, tokens * valueWidth * 2, "GDN hidden rows");
+  }
   if (b.blocks) {
     // (offsets into a run's rows are 32-bit)
     if (std::max<uint64_t>(tokens * valueWidth * 2, gdn_prefill_blocks_bytes(tokens, shape.keyHeads, shape.valueHeads)) >> 31)
@@ -148,6 +153,11 @@ void GDN::addPrefill(hip::CommandGraph &graph, const GdnPrefillBuffers &b, const
   }
   params.first = 0;
   params.tokens = tokens;
+  if (b.hiddenTable) {
+    const uint32_t rows = 16 * gguf_wide_tiles(tokens);
+    graph.add("gdn_prefill_gate_table", {b.recurrentRows, b.packed, b.mixerNorm, b.hiddenTable}, params, {64 * ((rows + 63) / 64), 1, 1}, {256, 1, 1});
+    return;
+  }
   graph.add("gdn_prefill_gate", {b.recurrentRows, b.packed, b.mixerNorm, b.hidden}, params,
             {shape.valueHeads, (tokens + 4 * GDN_GATE_ROWS - 1) / (4 * GDN_GATE_ROWS), 1}, {256, 1, 1});
 }

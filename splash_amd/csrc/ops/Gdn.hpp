@@ -91,6 +91,8 @@ struct GdnPrefillBuffers final {
   uint64_t nextCell = 0;           // the cell after its last row
   // Optional (gdn_prefill_blocks_bytes of the rows): the terms of the scan in blocks of sixteen tokens on the matrix cores.
   hip::Buffer blocks{};
+  // Optional (takesTable): the chunk's hidden rows leave as their wide table (abi/Gguf.h) and not as `hidden`.
+  hip::Buffer hiddenTable{};
 };
 // A state a chunk leaves on the way (GDN.hpp:95-104): the cell after its first `tokens` rows, convolution carry and
 // recurrent state as a chunk ending there would leave them. What a cached state codes (ops::StateCodec) is such a cell.
@@ -101,6 +103,9 @@ struct GdnPrefillCapture final {
 
 class GDN final {
 public:
+  [[nodiscard]] static bool takesTable(const GdnShape &shape) noexcept {
+    return shape.valueHeads % 2 == 0 && shape.valueHeads * GDN_HEAD_DIMENSION <= GDN_GATE_TABLE_WIDTH;
+  }
   // A chunk of `tokens` rows of one lane, in runs that end at the captures (ascending, inside the rows): each run is
   // a prepare and a scan dispatch that continue from the cell the run before wrote, and one gate dispatch covers all
   // rows (GDN.cpp:176-222). The scan is sequential, so the runs compute bit for bit what one run computes. With buffers.blocks
