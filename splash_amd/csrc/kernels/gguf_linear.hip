@@ -1408,12 +1408,14 @@ __device__ __forceinline__ void decode_workgroup(Shared &shared, const uint8_t *
   }
 }
 
-// Waves a SIMD: four (128 registers); three where those would spill in the loop (Q6_K's taller tiles, and four row tiles of
-// the formats with a scale of 16 bits a group).
-template <uint32_t FMT, int RT>
-constexpr uint32_t kDecodeWaves = (RT > 1 && FMT == GGUF_FMT_Q6K) || (RT > 2 && (FMT == GGUF_FMT_Q80 || FMT == GGUF_FMT_IQ4NL)) ? 3 : 4;
+// Waves a SIMD: four (128 registers); three for Q6_K and Q8_0 from three row tiles on and for four of Q5_K, most of which would
+// spill at four. (A spilled place of a record is read back behind the loads just issued, and waits for all of them. 64 rows of
+// Q5_K, us a launch at four and three: 5120 x 2 x 25600 gate/up 79.8 and 76.4, 25600 x 5120 55.8 and 52.5, 5120 x 10240 26.2
+// and 24.1. Three row tiles of Q8_0 fit four and gain nothing; the staged rule's Q5_K fits.)
+template <uint32_t FMT, int RT, bool Staged>
+constexpr uint32_t kDecodeWaves = (RT > 2 && (FMT == GGUF_FMT_Q6K || FMT == GGUF_FMT_Q80)) || (RT > 3 && FMT == GGUF_FMT_Q5K && !Staged) ? 3 : 4;
 template <uint32_t FMT, int RT, uint32_t EP, bool Staged = false>
-__global__ __launch_bounds__(256, (kDecodeWaves<FMT, RT>))
+__global__ __launch_bounds__(256, (kDecodeWaves<FMT, RT, Staged>))
                                   void gguf_decode(const uint8_t *__restrict__ seg0, const uint8_t *__restrict__ seg1,
                                                    const uint8_t *__restrict__ seg2, const uint8_t *__restrict__ table,
                                                    void *__restrict__ out, const uint16_t *__restrict__ residual,
