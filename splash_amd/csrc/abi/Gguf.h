@@ -225,8 +225,9 @@ struct GgufWideTableParams {
   uint32_t input_size;
   uint32_t rows;
   uint32_t tiles;  // gguf_wide_tiles(rows)
-  uint32_t reserved;
+  uint32_t flags;  // gguf_wide_table_norm_rows
 };
+#define GGUF_WIDE_ROWS_NORM_RMS 1u   // the rows' tables hold norm_rms's rows to the bit (otherwise the wide table's)
 #define GGUF_WIDE_TILE_INPUTS 2048u  // inputs of the rows whose tile a workgroup puts together in LDS (gguf_wide_moe_*_tile)
 // gguf_wide_<fmt>_{a,r,g,p} (and gguf_wide_staged_*, weights rounded once to half): a chunk of rows, a workgroup up to 128
 // of them x 128 columns. Binds up to three segments of one format (a gate/up pair: gate, up), the wide table, out and the

@@ -69,21 +69,44 @@ __global__ __launch_bounds__(256) void gguf_wide_rows(const uint16_t *__restrict
   });
   if (threadIdx.x == 0) reinterpret_cast<float *>(rows + size_t(p.rows) * bytes)[row] = scale;
 }
-// The normed rows as both: their wide table, and the rows' tables (2048 rows of 2048 inputs 10.0 us, 8.0 without the latter).
+// The normed rows as both: their wide table, and the rows' tables. With GGUF_WIDE_ROWS_NORM_RMS the rows' tables hold norm_rms's
+// rows, whose sum of squares is added column by column: the experts' rows are the bits they are in every other path. Where that
+// inverse is another float than the table's, the entries are made again. Bound by memory and a row's chain of sums; 2048 rows of
+// 2048 inputs 10.8 us (8.8 without the flag, 7.0 the wide table alone, which norm_rms and gguf_wide_rows would follow with 8.4 and
+// 4.9).
 __global__ __launch_bounds__(256) void gguf_wide_table_norm_rows(const uint16_t *__restrict__ input, const uint16_t *__restrict__ weight,
                                                                  uint8_t *__restrict__ table, uint8_t *__restrict__ rows, GgufWideTableParams p) {
+  constexpr uint32_t Held = 4;
   const uint32_t row = wide_table_row_of(blockIdx.x), bytes = gguf_wide_row_bytes(p.input_size);
   if (row >= 16u * p.tiles) return;
+  __shared__ float scratch[16];
+  const bool live = row < p.rows;
+  const uint16_t *from = input + size_t(live ? row : 0u) * p.input_size;
+  uint4 v[Held], w[Held], normed[Held];
+  wide_row_load<Held, 4>(v, from, p.input_size, live);
+  wide_row_load<Held, 4>(w, weight, p.input_size, live);
+  const bool apart = live && (p.flags & GGUF_WIDE_ROWS_NORM_RMS);
+  const float own = apart ? rms_inverse(from, p.input_size, scratch) : 0.f;
+  const float inverse = wide_row_inverse(v, p.input_size, scratch + 4);
+  const bool shared = live && (!apart || own == inverse);
   uint4 *values = reinterpret_cast<uint4 *>(table + row / 16u * gguf_wide_tile_bytes(p.input_size)) + row % 16u;
   uint8_t *of = rows + size_t(row) * bytes;
-  const float scale = wide_table_row<true, 4, 4>(input, weight, p, row, [&](uint32_t line, uint32_t operand, uint32_t kq, uint4 entry) __attribute__((always_inline)) {
+  float *rowScales = reinterpret_cast<float *>(rows + size_t(p.rows) * bytes);
+  wide_row_norm(normed, v, w, inverse, p.input_size);
+  const float scale = wide_row_entries<Held, 4>(normed, p.input_size, scratch + 8, [&](uint32_t line, uint32_t operand, uint32_t kq, uint4 entry) __attribute__((always_inline)) {
     values[size_t(line) * 16u] = entry;
-    if (row < p.rows) *wide_row_entry(of, p.input_size, line, operand, kq) = entry;
+    if (shared) *wide_row_entry(of, p.input_size, line, operand, kq) = entry;
   });
   if (threadIdx.x == 0) {
     wide_scales_of(table, p)[row] = scale;
-    if (row < p.rows) reinterpret_cast<float *>(rows + size_t(p.rows) * bytes)[row] = scale;
+    if (shared) rowScales[row] = scale;
   }
+  if (shared || !live) return;
+  wide_row_norm(normed, v, w, own, p.input_size);
+  const float ownScale = wide_row_entries<Held, 4>(normed, p.input_size, scratch + 12, [&](uint32_t line, uint32_t operand, uint32_t kq, uint4 entry) __attribute__((always_inline)) {
+    *wide_row_entry(of, p.input_size, line, operand, kq) = entry;
+  });
+  if (threadIdx.x == 0) rowScales[row] = ownScale;
 }
 // The table of a mixture's slots' own rows (or, Gathers, of the rows that they gather: row s is row slot_row[s] of the input;
 // a chunk's gate/up pair gathers from the rows' tables instead, and this is what it is held against), zeros where the slot is

@@ -2,6 +2,7 @@
 
 // A row of the wide table (abi/Gguf.h): what makes it, for the kernels that put it where it goes.
 #include "abi/Gguf.h"
+#include "abi/Glue.h"
 #include "kernels/gguf_records.hpp"
 
 namespace splash::kernels {
@@ -14,62 +15,67 @@ __device__ __forceinline__ uint32_t as_word(f16x2 v) { return __builtin_bit_cast
 // Returns the row's scale.
 // (The operands, the parts of their sums and the scale are the same bits whatever Waves is; a norm's sum of squares is added
 // over four waves.)
-template <bool Norm, uint32_t Held, uint32_t Waves, class Put>
-__device__ __forceinline__ float wide_table_row(const uint16_t *__restrict__ input, const uint16_t *__restrict__ weight, const GgufWideTableParams &p,
-                                                const uint32_t source, Put &&put) {
-  static_assert(Waves == 4u || (Waves == 1u && !Norm), "a row of one wave has no other wave's sums to add");
-  __shared__ float scratch[8];
-  constexpr uint32_t kPiece = 16u * Waves;   // groups of 32 inputs a piece
-  const uint32_t tid = threadIdx.x % (64u * Waves), lane = tid & 63u, wave = tid >> 6;
-  const uint32_t kq = tid & 3u, groups = p.input_size / 32u, held = (groups + kPiece - 1u) / kPiece;
-  const bool live = source < p.rows;
-  // piece i: inputs 4 kq .. + 3, then 16 + 4 kq .. + 3 of group 16 Waves i + t / 4
-  auto groupOf = [&](uint32_t i) { return kPiece * i + (tid >> 2); };
-  auto load = [&](const uint16_t *from, uint32_t i) {
-    const uint32_t g = groupOf(i);
-    if (!live || g >= groups) return make_uint4(0u, 0u, 0u, 0u);
-    const uint2 a = *reinterpret_cast<const uint2 *>(from + 32u * g + 4u * kq), b = *reinterpret_cast<const uint2 *>(from + 32u * g + 16u + 4u * kq);
-    return make_uint4(a.x, a.y, b.x, b.y);
-  };
-  uint4 v[Held];
+template <uint32_t Waves> constexpr uint32_t kWidePiece = 16u * Waves;   // groups of 32 inputs a piece
+// A thread's part of a row (or of a norm's weights): piece i holds inputs 4 kq .. + 3, then 16 + 4 kq .. + 3 of group
+// 16 Waves i + t / 4, zeros of a row that is not there.
+template <uint32_t Held, uint32_t Waves>
+__device__ __forceinline__ void wide_row_load(uint4 (&v)[Held], const uint16_t *from, uint32_t inputSize, bool live) {
+  const uint32_t tid = threadIdx.x % (64u * Waves), kq = tid & 3u, groups = inputSize / 32u, held = (groups + kWidePiece<Waves> - 1u) / kWidePiece<Waves>;
 #pragma unroll
   for (uint32_t i = 0; i < Held; ++i)
-    if (i < held) v[i] = load(input + size_t(live ? source : 0u) * p.input_size, i);
-  if constexpr (Norm) {
-    uint4 w[Held];
+    if (i < held) {
+      const uint32_t g = kWidePiece<Waves> * i + (tid >> 2);
+      v[i] = make_uint4(0u, 0u, 0u, 0u);
+      if (!live || g >= groups) continue;
+      const uint2 a = *reinterpret_cast<const uint2 *>(from + 32u * g + 4u * kq), b = *reinterpret_cast<const uint2 *>(from + 32u * g + 16u + 4u * kq);
+      v[i] = make_uint4(a.x, a.y, b.x, b.y);
+    }
+}
+// The row's inverse RMS, over the four waves that hold it.
+template <uint32_t Held>
+__device__ __forceinline__ float wide_row_inverse(const uint4 (&v)[Held], uint32_t inputSize, float *scratch) {
+  const uint32_t held = (inputSize / 32u + kWidePiece<4> - 1u) / kWidePiece<4>;
+  float sum = 0.f;
 #pragma unroll
-    for (uint32_t i = 0; i < Held; ++i)
-      if (i < held) w[i] = load(weight, i);
-    float sum = 0.f;
+  for (uint32_t i = 0; i < Held; ++i)
+    if (i < held) {
+      const uint32_t words[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
 #pragma unroll
-    for (uint32_t i = 0; i < Held; ++i)
-      if (i < held) {
-        const uint32_t words[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float low = bf16_bits_to_float(words[e] & 0xFFFFu), high = bf16_bits_to_float(words[e] >> 16);
-          sum += low * low;
-          sum += high * high;
-        }
+      for (int e = 0; e < 4; ++e) {
+        const float low = bf16_bits_to_float(words[e] & 0xFFFFu), high = bf16_bits_to_float(words[e] >> 16);
+        sum += low * low;
+        sum += high * high;
       }
-    sum = wave_sum(sum);
-    if (lane == 0) scratch[wave] = sum;
-    __syncthreads();
-    const float inverse = 1.0f / sqrtf((((scratch[0] + scratch[1]) + scratch[2]) + scratch[3]) / float(p.input_size) + 1e-6f);
+    }
+  sum = wave_sum(sum);
+  if ((threadIdx.x & 63u) == 0) scratch[threadIdx.x >> 6] = sum;
+  __syncthreads();
+  return 1.0f / sqrtf((((scratch[0] + scratch[1]) + scratch[2]) + scratch[3]) / float(inputSize) + SPLASH_RMS_EPSILON);
+}
+// bf16((x * inverse) * weight)
+template <uint32_t Held>
+__device__ __forceinline__ void wide_row_norm(uint4 (&out)[Held], const uint4 (&v)[Held], const uint4 (&w)[Held], float inverse, uint32_t inputSize) {
+  const uint32_t held = (inputSize / 32u + kWidePiece<4> - 1u) / kWidePiece<4>;
 #pragma unroll
-    for (uint32_t i = 0; i < Held; ++i)
-      if (i < held) {
-        const uint32_t words[4] = {v[i].x, v[i].y, v[i].z, v[i].w}, weights[4] = {w[i].x, w[i].y, w[i].z, w[i].w};
-        uint32_t out[4];
+  for (uint32_t i = 0; i < Held; ++i)
+    if (i < held) {
+      const uint32_t words[4] = {v[i].x, v[i].y, v[i].z, v[i].w}, weights[4] = {w[i].x, w[i].y, w[i].z, w[i].w};
+      uint32_t normed[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const uint32_t low = float_to_bf16_bits((bf16_bits_to_float(words[e] & 0xFFFFu) * inverse) * bf16_bits_to_float(weights[e] & 0xFFFFu));
-          const uint32_t high = float_to_bf16_bits((bf16_bits_to_float(words[e] >> 16) * inverse) * bf16_bits_to_float(weights[e] >> 16));
-          out[e] = low | (high << 16);
-        }
-        v[i] = make_uint4(out[0], out[1], out[2], out[3]);
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t low = float_to_bf16_bits((bf16_bits_to_float(words[e] & 0xFFFFu) * inverse) * bf16_bits_to_float(weights[e] & 0xFFFFu));
+        const uint32_t high = float_to_bf16_bits((bf16_bits_to_float(words[e] >> 16) * inverse) * bf16_bits_to_float(weights[e] >> 16));
+        normed[e] = low | (high << 16);
       }
-  }
+      out[i] = make_uint4(normed[0], normed[1], normed[2], normed[3]);
+    }
+}
+// The row's entries of what the threads hold. (scratch: four floats that no earlier row of the workgroup still reads)
+template <uint32_t Held, uint32_t Waves, class Put>
+__device__ __forceinline__ float wide_row_entries(const uint4 (&v)[Held], uint32_t inputSize, float *scratch, Put &&put) {
+  constexpr uint32_t kPiece = kWidePiece<Waves>;
+  const uint32_t tid = threadIdx.x % (64u * Waves), lane = tid & 63u, wave = tid >> 6;
+  const uint32_t kq = tid & 3u, groups = inputSize / 32u, held = (groups + kPiece - 1u) / kPiece;
   uint32_t largest = 0;
 #pragma unroll
   for (uint32_t i = 0; i < Held; ++i)
@@ -84,10 +90,10 @@ __device__ __forceinline__ float wide_table_row(const uint16_t *__restrict__ inp
     }
   largest = wave_max(largest);
   if constexpr (Waves > 1u) {
-    if (lane == 0) scratch[4u + wave] = __uint_as_float(largest);
+    if (lane == 0) scratch[wave] = __uint_as_float(largest);
     __syncthreads();
 #pragma unroll
-    for (int w = 0; w < 4; ++w) largest = max(largest, __float_as_uint(scratch[4 + w]));
+    for (int w = 0; w < 4; ++w) largest = max(largest, __float_as_uint(scratch[w]));
   }
   // 2^e, e = 14 - the exponent of the largest magnitude (a row of zeros or of subnormals: the largest 2^e there is)
   const uint32_t exponent = max(largest >> 7, 15u);
@@ -95,7 +101,7 @@ __device__ __forceinline__ float wide_table_row(const uint16_t *__restrict__ inp
 #pragma unroll
   for (uint32_t i = 0; i < Held; ++i)
     if (i < held) {
-      const uint32_t g = groupOf(i);
+      const uint32_t g = kPiece * i + (tid >> 2);
       const uint32_t words[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
       float f[8];
 #pragma unroll
@@ -125,6 +131,21 @@ __device__ __forceinline__ float wide_table_row(const uint16_t *__restrict__ inp
       if ((g & 7u) == 0 && g < groups) put(((g >> 3) * GGUF_WIDE_OPERANDS + 8u) * 4u + kq, 8u, kq, make_uint4(two, b, c, d));
     }
   return inverseScale;
+}
+template <bool Norm, uint32_t Held, uint32_t Waves, class Put>
+__device__ __forceinline__ float wide_table_row(const uint16_t *__restrict__ input, const uint16_t *__restrict__ weight, const GgufWideTableParams &p,
+                                                const uint32_t source, Put &&put) {
+  static_assert(Waves == 4u || (Waves == 1u && !Norm), "a row of one wave has no other wave's sums to add");
+  __shared__ float scratch[8];
+  const bool live = source < p.rows;
+  uint4 v[Held];
+  wide_row_load<Held, Waves>(v, input + size_t(live ? source : 0u) * p.input_size, p.input_size, live);
+  if constexpr (Norm) {
+    uint4 w[Held];
+    wide_row_load<Held, Waves>(w, weight, p.input_size, live);
+    wide_row_norm(v, v, w, wide_row_inverse(v, p.input_size, scratch), p.input_size);
+  }
+  return wide_row_entries<Held, Waves>(v, p.input_size, scratch + 4, put);
 }
 __device__ __forceinline__ float *wide_scales_of(uint8_t *table, const GgufWideTableParams &p) {
   return reinterpret_cast<float *>(table + gguf_wide_scales_offset(p.input_size, p.tiles));

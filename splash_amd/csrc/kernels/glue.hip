@@ -42,30 +42,6 @@ struct StagedRow {
   }
 };
 
-// The row's inverse RMS: a workgroup's first 256 threads sum the squares of columns tid, tid + 256, ... in column
-// order; a wavefront sums its lanes by butterfly, the four wavefronts' sums are added in order
-// (normalization.metal:59-99 and common/rms_inverse.h:15-33, on 64-lane wavefronts). The order is the same whatever the
-// workgroup's size is.
-__device__ __forceinline__ float rms_inverse(const uint16_t *row, uint32_t width, float *scratch) {
-  // (ten reads at a time: a column past the row adds a zero)
-  constexpr uint32_t kAhead = 10;
-  if (threadIdx.x < 256u) {
-    float sum = 0.f;
-    for (uint32_t first = threadIdx.x; first < width; first += 256u * kAhead) {
-      float v[kAhead];
-#pragma unroll
-      for (uint32_t j = 0; j < kAhead; ++j) v[j] = bf16_bits_to_float(row[min(first + 256u * j, width - 1u)]);
-#pragma unroll
-      for (uint32_t j = 0; j < kAhead; ++j) sum += first + 256u * j < width ? v[j] * v[j] : 0.f;
-    }
-    sum = wave_sum(sum);
-    if ((threadIdx.x & 63u) == 0) scratch[threadIdx.x >> 6] = sum;
-  }
-  __syncthreads();
-  const float total = ((scratch[0] + scratch[1]) + scratch[2]) + scratch[3];
-  return 1.0f / sqrtf(total / float(width) + SPLASH_RMS_EPSILON);
-}
-
 __global__ __launch_bounds__(256) void norm_rms(const uint16_t *__restrict__ input, const uint16_t *__restrict__ weight,
                                                 uint16_t *__restrict__ output, NormParams p) {
   __shared__ float scratch[4];

@@ -576,7 +576,7 @@ void Linear::addWideNormTable(hip::CommandGraph &graph, const hip::Buffer &input
   requireBytes(weight, uint64_t{width} * 2, "norm weight");
   requireBytes(table, gguf_wide_table_bytes(width, rows), "wide table");
   const uint32_t tiles = gguf_wide_tiles(rows);
-  const GgufWideTableParams params{width, rows, tiles, 0};
+  const GgufWideTableParams params{width, rows, tiles, rowTables ? GGUF_WIDE_ROWS_NORM_RMS : 0u};
   const hip::DispatchSize grid{64 * ((16 * tiles + 63) / 64), 1, 1};
   if (rowTables) {
     requireBytes(rowTables, gguf_wide_rows_bytes(width, rows), "row tables");

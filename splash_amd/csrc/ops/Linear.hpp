@@ -236,8 +236,8 @@ public:
   // The projections of a prompt chunk of many rows through the matrix cores' fp16 (kernels gguf_wide_*): the register
   // rule's exact weights, or (staged) each rounded once to half. takesWide: whether the kernels take the projection (tensors
   // of one format, Q4_K, Q5_K or Q6_K, up to 32768 inputs). The rows enter as a wide table,
-  // which addWideTable makes of bf16 rows and addWideNormTable of their RMS norm (rows of up to 8192 values; with the rows'
-  // tables too, where a buffer for them is given).
+  // which addWideTable makes of bf16 rows and addWideNormTable of their RMS norm (rows of up to 8192 values; with the
+  // tables of the rows that Normalization::addRms writes, where a buffer for them is given).
   static constexpr uint32_t kMaximumWideNormWidth = 8192, kMaximumWideWidth = 32768;
   [[nodiscard]] static bool takesWide(const Projection &projection) noexcept;
   [[nodiscard]] static uint64_t wideTableBytes(uint32_t inputSize, uint32_t rows) noexcept;

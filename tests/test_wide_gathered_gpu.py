@@ -86,3 +86,28 @@ def test_rows_tables_hold_what_the_wide_table_does(backend, rows, K):
         assert np.array_equal(got[rows * size:], want[tiles * (K // 256) * 9216:][:4 * rows])
         if normed:
             assert np.array_equal(beside.download(), want)
+
+
+@pytest.mark.parametrize("rows,K", [(1, 256), (130, 2048), (61, 2304), (33, 8192)])
+def test_rows_tables_of_norms_are_those_of_the_norm_pass(backend, rows, K):
+    """GGUF_WIDE_ROWS_NORM_RMS: the experts' rows are norm_rms's to the bit, whose squares are added in another order than the
+    wide table's; the wide table beside them stays what it is."""
+    print(f"case rows' tables of the norm pass {rows} K={K}", flush=True)
+    rng = np.random.default_rng(rows)
+    x = orc.f32_to_bf16((rng.standard_normal((rows, K)) * 10.0 ** rng.integers(-2, 3, (1, K))).astype(np.float32))
+    if rows > 1:
+        x[0, 3], x[rows - 1, 0], x[rows // 2] = 0x7F80, 0x7FC1, 0
+    weight, tiles, size = orc.f32_to_bf16((1 + 0.1 * rng.standard_normal(K)).astype(np.float32)), wide_tiles(rows), row_bytes(K)
+    source, norm = backend.from_array(x), backend.from_array(weight)
+    normed, want, got = (backend.allocate_buffer(n) for n in (rows * K * 2, rows * (size + 4), rows * (size + 4)))
+    beside = backend.allocate_buffer(table_bytes(K, tiles))
+    for buffer in (want, got, beside):
+        buffer.fill(0xA5)
+    graph = splash_amd.CommandGraph()
+    graph.add("norm_rms", [source, norm, normed], TableParams(K, rows, 0, 0), (rows, 1, 1))
+    graph.add("gguf_wide_rows", [normed, want], TableParams(K, rows, tiles, 0), (rows, 1, 1))
+    graph.add("gguf_wide_table_norm_rows", [source, norm, beside, got], TableParams(K, rows, tiles, 1), (64 * -(-16 * tiles // 64), 1, 1))
+    table = add_table(graph, backend, x, weight)
+    backend.run(graph)
+    assert np.array_equal(got.download(), want.download())
+    assert np.array_equal(beside.download(), table.download())
