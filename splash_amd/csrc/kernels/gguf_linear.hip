@@ -374,7 +374,8 @@ template <int RT> struct DecodeRing {
   static constexpr bool kRing = true;
   static constexpr uint32_t kStageGroups = RT == 1 ? 4 : 2;
   uint4 *rows0, *rows1, *rows2, *rows3;
-  float *sums0, *sums1;           // [row tile][K = 4 MFMA][lane]; a ring of two super-blocks has two
+  float *sums0, *sums1;           // [row tile][K = 4 MFMA][lane]; a ring of two super-blocks has two. (Vectors in LDS, as the rows:
+                                  // the loads place up to sixteen bytes a lane.)
   float *scaleParts, *rowScale;   // of a table with a deferred scale
   uint32_t *arrivedWord;
   __device__ __forceinline__ uint32_t &arrived() { return *arrivedWord; }
@@ -387,9 +388,11 @@ template <int RT> struct DecodeRing {
 #define SP_DECODE_RING(name, RT, FMT)                                                                                         \
   constexpr uint32_t name##Stage = RT * DecodeRing<RT>::kStageGroups * 64, name##Sum = RT * RecordTerms<FMT>::kConstants * 64;  \
   __shared__ uint4 name##Rows0[name##Stage], name##Rows1[name##Stage], name##Rows2[name##Stage], name##Rows3[name##Stage];    \
-  __shared__ float name##Sums0[name##Sum], name##Sums1[RT == 1 ? name##Sum : 1], name##Parts[256 * RT], name##Scale[16 * RT]; \
+  __shared__ uint4 name##Sums0[name##Sum / 4], name##Sums1[RT == 1 ? name##Sum / 4 : 1];                                      \
+  __shared__ float name##Parts[256 * RT], name##Scale[16 * RT];                                                               \
   __shared__ uint32_t name##Arrived;                                                                                          \
-  DecodeRing<RT> name{name##Rows0, name##Rows1, name##Rows2, name##Rows3, name##Sums0, name##Sums1, name##Parts, name##Scale, &name##Arrived}
+  DecodeRing<RT> name{name##Rows0, name##Rows1, name##Rows2, name##Rows3, reinterpret_cast<float *>(name##Sums0),             \
+                      reinterpret_cast<float *>(name##Sums1), name##Parts, name##Scale, &name##Arrived}
 
 // Vector-memory instructions of a record's load.
 template <uint32_t FMT> constexpr uint32_t kRecordLoads = FMT == GGUF_FMT_Q6K || FMT == GGUF_FMT_Q80 ? 5u : FMT == GGUF_FMT_Q5K ? 4u : 3u;

@@ -387,9 +387,9 @@ __device__ __forceinline__ void wide_columns(WideTile &w, const uint8_t *seg0, c
 // read of one does not wait for what is on its way into another.
 struct WideLds {
   uint4 *rows0, *rows1, *rows2, *rows3, *sums;
-  float *scales;   // the row tiles' scales
+  f32x4 *scales;   // the row tiles' scales, four rows a vector
 };
-template <uint32_t T> constexpr uint32_t kWideScales = (T + 3) / 4 * 64;
+template <uint32_t T> constexpr uint32_t kWideScales = (T + 3) / 4 * 16;
 template <uint32_t T> constexpr uint32_t kWideStageVectors = (T + 1) / 2 * 2 * 2 * 64;
 template <uint32_t FMT, uint32_t T, bool Staged> constexpr uint32_t kWideSumVectors = FMT != GGUF_FMT_Q6K && !Staged ? (T + 3) / 4 * 4 * 64 : 1;
 
@@ -504,11 +504,11 @@ __device__ __forceinline__ void wide_workgroup(const WideLds lds, const WideTile
   };
   constexpr auto rowLoads = [](uint32_t stage) constexpr { return kShare + (stage == 3u ? kSumShare : 0u); };
   // (first of all loads, so that the first stage's wait and barrier are these's too)
-  if (Gathers && wave < kWideScales<T> / 64u)
-    load_to_lds<4>(make_resource(table + size_t(p.rows) * rowBytes, p.rows * 4u), scaleAt, lds.scales + 64u * wave);
-  if (!Gathers && wave < kWideScales<T> / 64u)
+  if (Gathers && wave < kWideScales<T> / 16u)
+    load_to_lds<4>(make_resource(table + size_t(p.rows) * rowBytes, p.rows * 4u), scaleAt, lds.scales + 16u * wave);
+  if (!Gathers && wave < kWideScales<T> / 16u)
     load_to_lds<4>(make_resource(table + gguf_wide_scales_offset(p.input_size, p.tiles) + tile0 * 64u, tilesHere * 64u), threadIdx.x * 4u,
-                   lds.scales + 64u * wave);
+                   lds.scales + 16u * wave);
   __builtin_amdgcn_sched_barrier(0);
   // (the loads before the first stage in the order of the stages that would have asked for them)
   fetch(0, std::integral_constant<uint32_t, 0>{});
@@ -640,7 +640,7 @@ __device__ __forceinline__ void wide_workgroup(const WideLds lds, const WideTile
 #pragma unroll
   for (uint32_t t = 0; t < T; ++t) {
     if (t >= tilesHere) break;
-    const f32x4 scale = *reinterpret_cast<const f32x4 *>(lds.scales + 16u * t + 4u * kq);
+    const f32x4 scale = lds.scales[4u * t + kq];
 #pragma unroll
     for (uint32_t pair = 0; pair < 2; ++pair) {
       const uint32_t row = 16u * (tile0 + t) + 4u * kq + 2u * pair + odd;
@@ -693,7 +693,7 @@ __global__ __launch_bounds__(256, 2) void gguf_wide(const uint8_t *__restrict__ 
   wide_columns<FMT, EP == GGUF_WIDE_GATE_UP>(w, seg0, seg1, seg2, p, tail ? tallGroups + rest : rest / p.splits, wave);
   __shared__ uint4 rows0[kWideStageVectors<T>], rows1[kWideStageVectors<T>], rows2[kWideStageVectors<T>], rows3[kWideStageVectors<T>],
       sums[kWideSumVectors<FMT, T, Staged>];
-  __shared__ float scales[kWideScales<T>];
+  __shared__ f32x4 scales[kWideScales<T>];
   const WideLds lds{rows0, rows1, rows2, rows3, sums, scales};
   if (tail) wide_workgroup<FMT, EP, 4, Staged>(lds, w, table, out, residual, p);
   else wide_workgroup<FMT, EP, T, Staged>(lds, w, table, out, residual, p);
@@ -724,7 +724,7 @@ __device__ __forceinline__ void wide_moe(const uint8_t *__restrict__ seg0, const
   wide_columns<FMT, EP == GGUF_WIDE_GATE_UP>(w, seg0 + expertAt, seg1 + expertAt, seg0 + expertAt, p, item % p.groups, wave);
   __shared__ uint4 rows0[kWideStageVectors<T>], rows1[kWideStageVectors<T>], rows2[kWideStageVectors<T>], rows3[kWideStageVectors<T>],
       sums[kWideSumVectors<FMT, T, false>];
-  __shared__ float scales[kWideScales<T>];
+  __shared__ f32x4 scales[kWideScales<T>];
   const WideLds lds{rows0, rows1, rows2, rows3, sums, scales};
   if constexpr (T > 4u) {
     if (w.tilesHere <= 4u) return wide_workgroup<FMT, EP, 4, false, Gathers>(lds, w, table, out, nullptr, p, slot_row);
