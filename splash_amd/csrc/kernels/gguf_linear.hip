@@ -394,9 +394,6 @@ template <int RT> struct DecodeRing {
   DecodeRing<RT> name{name##Rows0, name##Rows1, name##Rows2, name##Rows3, reinterpret_cast<float *>(name##Sums0),             \
                       reinterpret_cast<float *>(name##Sums1), name##Parts, name##Scale, &name##Arrived}
 
-// Vector-memory instructions of a record's load.
-template <uint32_t FMT> constexpr uint32_t kRecordLoads = FMT == GGUF_FMT_Q6K || FMT == GGUF_FMT_Q80 ? 5u : FMT == GGUF_FMT_Q5K ? 4u : 3u;
-
 // A projection's place in a chain of projections that share one dispatch (gguf_decode_chain): link i + 1 reads what link
 // i's epilogues wrote, so its workgroups, which the device starts after every workgroup of link i, fetch their first
 // weights, which depend on nothing, and then wait for link i's count of finished workgroups. Results that a later link
@@ -812,7 +809,7 @@ __device__ __forceinline__ void decode_workgroup(Shared &shared, const uint8_t *
       constexpr uint32_t kTall = RT == 3 ? 4 : RT, kRowLoads = kTall * Ring::kStageGroups / 4, kSumChunks = kTall * kSumsPerBlock;
       // a wave's sums: kSumLoads times 256 bytes, or a kilobyte at once; of fewer chunks than waves, two load the same
       constexpr uint32_t kSumBytes = kSumChunks == 16 ? 16u : 4u, kSumLoads = kSumChunks == 16 || kSumChunks < 4 ? 1 : kSumChunks / 4;
-      constexpr uint32_t kWeightLoads = kRecordLoads<FMT>;
+      constexpr uint32_t kWeightLoads = Record<FMT>::kLoads;
       const uint32_t waveIndex = min(uint32_t(__builtin_amdgcn_readfirstlane(int(wave))), RT == 3 ? 2u : 3u);
       const uint32_t rowChunk = kRowLoads * waveIndex, rowTile = rowChunk / Ring::kStageGroups;   // its kilobytes of a stage, one row tile's
       // (a row tile past the table's, and a super-block past the range, read as zeros)

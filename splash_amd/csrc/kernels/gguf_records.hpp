@@ -2,6 +2,7 @@
 // shared by every projection kernel.
 #pragma once
 #include "kernels/gguf_device.hpp"
+#include <utility>
 
 namespace splash::kernels {
 
@@ -41,6 +42,7 @@ template <uint32_t FMT> struct Cursor {
 
 template <uint32_t FMT> struct Record;
 template <> struct Record<GGUF_FMT_Q4K> {
+  static constexpr uint32_t kLoads = 3;   // load_piece
   uint4 n0, n1, meta;
   __device__ __forceinline__ void load(const Cursor<GGUF_FMT_Q4K> &at) {
     n0 = load_stream(at.mine);
@@ -49,6 +51,7 @@ template <> struct Record<GGUF_FMT_Q4K> {
   }
 };
 template <> struct Record<GGUF_FMT_Q6K> {
+  static constexpr uint32_t kLoads = 5;   // load_piece
   uint4 n0, n1, high, scales;
   uint32_t d;
   __device__ __forceinline__ void load(const Cursor<GGUF_FMT_Q6K> &at) {
@@ -61,6 +64,7 @@ template <> struct Record<GGUF_FMT_Q6K> {
 };
 
 template <> struct Record<GGUF_FMT_Q5K> {
+  static constexpr uint32_t kLoads = 4;   // load_piece
   uint4 n0, n1, meta;
   uint2 fifth;
   __device__ __forceinline__ void load(const Cursor<GGUF_FMT_Q5K> &at) {
@@ -71,6 +75,7 @@ template <> struct Record<GGUF_FMT_Q5K> {
   }
 };
 template <> struct Record<GGUF_FMT_Q80> {
+  static constexpr uint32_t kLoads = 5;   // load_piece
   uint4 v[4], scales;
   __device__ __forceinline__ void load(const Cursor<GGUF_FMT_Q80> &at) {
 #pragma unroll
@@ -80,6 +85,7 @@ template <> struct Record<GGUF_FMT_Q80> {
 };
 
 template <> struct Record<GGUF_FMT_IQ4XS> {
+  static constexpr uint32_t kLoads = 3;   // load_piece
   uint4 n0, n1;
   uint2 meta;  // x: d | scales_h << 16; y: the low four bits of the eight groups' scales
   __device__ __forceinline__ void load(const Cursor<GGUF_FMT_IQ4XS> &at) {
@@ -89,6 +95,7 @@ template <> struct Record<GGUF_FMT_IQ4XS> {
   }
 };
 template <> struct Record<GGUF_FMT_IQ4NL> {
+  static constexpr uint32_t kLoads = 3;   // load_piece
   uint4 n0, n1, scales;
   __device__ __forceinline__ void load(const Cursor<GGUF_FMT_IQ4NL> &at) {
     n0 = load_stream(at.mine);
@@ -202,50 +209,65 @@ template <uint32_t N> __device__ __forceinline__ void wait_loads() {
   static_assert(N < 64, "vmcnt has six bits");
   __builtin_amdgcn_s_waitcnt((N & 15u) | ((N >> 4) << 14) | 0x0F70u);
 }
-// `mine` is the lane's 16 bytes of the record's first 1024-byte part, `column` its column's scale
-// field, both as byte offsets into the resource.
-__device__ __forceinline__ void load_record(Record<GGUF_FMT_Q4K> &rec, Resource r, uint32_t mine, uint32_t column) {
-  rec.n0 = load128<kStreamOnce>(r, mine);
-  rec.n1 = load128<kStreamOnce>(r, mine + 1024u);
-  rec.meta = load128<kStreamOnce>(r, column);
+// Piece I of a record's load, one vector-memory instruction each: Record::kLoads of them are a record, which is what the waits of
+// a loop that counts its loads in flight rest on. `mine` is the lane's 16 bytes of the record's first 1024-byte part, `column`
+// its column's scale field, both as byte offsets into the resource.
+__device__ __forceinline__ uint32_t record_lane() { return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
+template <uint32_t I> __device__ __forceinline__ void load_piece(Record<GGUF_FMT_Q4K> &rec, Resource r, uint32_t mine, uint32_t column) {
+  if constexpr (I == 0) rec.n0 = load128<kStreamOnce>(r, mine);
+  else if constexpr (I == 1) rec.n1 = load128<kStreamOnce>(r, mine + 1024u);
+  else rec.meta = load128<kStreamOnce>(r, column);
+  static_assert(I < 3);
 }
-__device__ __forceinline__ void load_record(Record<GGUF_FMT_Q6K> &rec, Resource r, uint32_t mine, uint32_t column) {
-  rec.n0 = load128<kStreamOnce>(r, mine);
-  rec.n1 = load128<kStreamOnce>(r, mine + 1024u);
-  rec.high = load128<kStreamOnce>(r, mine + 2048u);
-  rec.scales = load128<kStreamOnce>(r, column);
-  // The lane's 16 l and the column's 16 c locate the record and c: d sits at record + 3328 + 2 c.
-  const uint32_t lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-  rec.d = __builtin_amdgcn_raw_buffer_load_b16(r, int(mine - 16u * lane + GGUF_Q6K_D + 2u * (lane & 15u)), 0, kStreamOnce);
+template <uint32_t I> __device__ __forceinline__ void load_piece(Record<GGUF_FMT_Q6K> &rec, Resource r, uint32_t mine, uint32_t column) {
+  if constexpr (I == 0) rec.n0 = load128<kStreamOnce>(r, mine);
+  else if constexpr (I == 1) rec.n1 = load128<kStreamOnce>(r, mine + 1024u);
+  else if constexpr (I == 2) rec.high = load128<kStreamOnce>(r, mine + 2048u);
+  else if constexpr (I == 3) rec.scales = load128<kStreamOnce>(r, column);
+  else {
+    // The lane's 16 l and the column's 16 c locate the record and c: d sits at record + 3328 + 2 c.
+    const uint32_t lane = record_lane();
+    rec.d = __builtin_amdgcn_raw_buffer_load_b16(r, int(mine - 16u * lane + GGUF_Q6K_D + 2u * (lane & 15u)), 0, kStreamOnce);
+  }
+  static_assert(I < 5);
 }
-
-__device__ __forceinline__ void load_record(Record<GGUF_FMT_Q5K> &rec, Resource r, uint32_t mine, uint32_t column) {
-  rec.n0 = load128<kStreamOnce>(r, mine);
-  rec.n1 = load128<kStreamOnce>(r, mine + 1024u);
-  rec.meta = load128<kStreamOnce>(r, column);
-  // The lane's 8 bytes of fifth bits sit at record + 2048 + 8 l; `mine` is record + 16 l.
-  const uint32_t lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-  const u32x2 fifth = __builtin_amdgcn_raw_buffer_load_b64(r, int(mine - 8u * lane + GGUF_Q5K_HIGH), 0, kStreamOnce);
-  rec.fifth = make_uint2(fifth.x, fifth.y);
+template <uint32_t I> __device__ __forceinline__ void load_piece(Record<GGUF_FMT_Q5K> &rec, Resource r, uint32_t mine, uint32_t column) {
+  if constexpr (I == 0) rec.n0 = load128<kStreamOnce>(r, mine);
+  else if constexpr (I == 1) rec.n1 = load128<kStreamOnce>(r, mine + 1024u);
+  else if constexpr (I == 2) rec.meta = load128<kStreamOnce>(r, column);
+  else {
+    // The lane's 8 bytes of fifth bits sit at record + 2048 + 8 l; `mine` is record + 16 l.
+    const u32x2 fifth = __builtin_amdgcn_raw_buffer_load_b64(r, int(mine - 8u * record_lane() + GGUF_Q5K_HIGH), 0, kStreamOnce);
+    rec.fifth = make_uint2(fifth.x, fifth.y);
+  }
+  static_assert(I < 4);
 }
-__device__ __forceinline__ void load_record(Record<GGUF_FMT_Q80> &rec, Resource r, uint32_t mine, uint32_t column) {
-#pragma unroll
-  for (uint32_t i = 0; i < 4; ++i) rec.v[i] = load128<kStreamOnce>(r, mine + 1024u * i);
-  rec.scales = load128<kStreamOnce>(r, column);
+template <uint32_t I> __device__ __forceinline__ void load_piece(Record<GGUF_FMT_Q80> &rec, Resource r, uint32_t mine, uint32_t column) {
+  if constexpr (I < 4) rec.v[I] = load128<kStreamOnce>(r, mine + 1024u * I);
+  else rec.scales = load128<kStreamOnce>(r, column);
+  static_assert(I < 5);
 }
-
-__device__ __forceinline__ void load_record(Record<GGUF_FMT_IQ4XS> &rec, Resource r, uint32_t mine, uint32_t) {
-  rec.n0 = load128<kStreamOnce>(r, mine);
-  rec.n1 = load128<kStreamOnce>(r, mine + 1024u);
-  // The column's 8 bytes sit at record + 2048 + 8 c; `mine` is record + 16 l.
-  const uint32_t lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-  const u32x2 meta = __builtin_amdgcn_raw_buffer_load_b64(r, int(mine - 16u * lane + GGUF_IQ4_SCALES + 8u * (lane & 15u)), 0, kStreamOnce);
-  rec.meta = make_uint2(meta.x, meta.y);
+template <uint32_t I> __device__ __forceinline__ void load_piece(Record<GGUF_FMT_IQ4XS> &rec, Resource r, uint32_t mine, uint32_t) {
+  if constexpr (I == 0) rec.n0 = load128<kStreamOnce>(r, mine);
+  else if constexpr (I == 1) rec.n1 = load128<kStreamOnce>(r, mine + 1024u);
+  else {
+    // The column's 8 bytes sit at record + 2048 + 8 c; `mine` is record + 16 l.
+    const uint32_t lane = record_lane();
+    const u32x2 meta = __builtin_amdgcn_raw_buffer_load_b64(r, int(mine - 16u * lane + GGUF_IQ4_SCALES + 8u * (lane & 15u)), 0, kStreamOnce);
+    rec.meta = make_uint2(meta.x, meta.y);
+  }
+  static_assert(I < 3);
 }
-__device__ __forceinline__ void load_record(Record<GGUF_FMT_IQ4NL> &rec, Resource r, uint32_t mine, uint32_t column) {
-  rec.n0 = load128<kStreamOnce>(r, mine);
-  rec.n1 = load128<kStreamOnce>(r, mine + 1024u);
-  rec.scales = load128<kStreamOnce>(r, column);
+template <uint32_t I> __device__ __forceinline__ void load_piece(Record<GGUF_FMT_IQ4NL> &rec, Resource r, uint32_t mine, uint32_t column) {
+  if constexpr (I == 0) rec.n0 = load128<kStreamOnce>(r, mine);
+  else if constexpr (I == 1) rec.n1 = load128<kStreamOnce>(r, mine + 1024u);
+  else rec.scales = load128<kStreamOnce>(r, column);
+  static_assert(I < 3);
+}
+template <uint32_t FMT> __device__ __forceinline__ void load_record(Record<FMT> &rec, Resource r, uint32_t mine, uint32_t column) {
+  [&]<uint32_t... I>(std::integer_sequence<uint32_t, I...>) __attribute__((always_inline)) {
+    (load_piece<I>(rec, r, mine, column), ...);
+  }(std::make_integer_sequence<uint32_t, Record<FMT>::kLoads>{});
 }
 
 } // namespace splash::kernels
