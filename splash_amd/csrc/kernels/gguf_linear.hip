@@ -325,26 +325,6 @@ __device__ __forceinline__ void staged_group(const Record<FMT> &rec, const Stage
   staged_values(rec, k, operand, g, value);
   staged_operands(value, high, low);
 }
-template <uint32_t FMT, int RT>
-__device__ __forceinline__ void accumulate_record_staged(const Record<FMT> &rec, const uint4 (*a)[8][64], f32x4 (&acc)[RT], uint32_t lane,
-                                                         uint32_t kq) {
-  uint4 ops[8];
-  record_operands(rec, ops);
-  const StagedCoefficients<FMT> k(rec);
-#pragma unroll
-  for (uint32_t g = 0; g < 8; ++g) {
-    bf16x8 high, low;
-    staged_group(rec, k, ops[g], g, high, low);
-#pragma unroll
-    for (int t = 0; t < RT; ++t) {
-      const bf16x8 rows = as_bf16x8(a[t][g][lane]);
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rows, high, acc[t], 0, 0, 0);
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rows, low, acc[t], 0, 0, 0);
-    }
-  }
-  (void)kq;
-}
-
 // Work split: a wave owns one column tile over the workgroup's K range; the four waves of a
 // workgroup walk that range in step and share its activations through LDS. Unit u of a dispatch
 // is tile u of its concatenated segments; of a gate/up pair, unit 2 j is gate tile j and unit
@@ -667,6 +647,7 @@ __device__ __forceinline__ void decode_workgroup(Shared &shared, const uint8_t *
   // The range's activations pass through LDS, each wave fetching a quarter of them, so a wave's vector-memory queue holds
   // almost only weights and the MFMA operands arrive on the LDS counter instead.
   constexpr bool kRing = Shared::kRing;
+  static_assert(kRing || !Staged, "the staged rule's kernels are ring kernels");
   uint32_t &arrived = shared.arrived();
   auto &scaleParts = shared.scaleParts;
   auto &rowScale = shared.rowScale;
@@ -1041,10 +1022,7 @@ __device__ __forceinline__ void decode_workgroup(Shared &shared, const uint8_t *
             (&ldsSums[buffer][0][0][0])[sumSlot + q * kTileStep * 256u] = kPairSums ? stage[u].sum[q] + stage[u].second[q] : stage[u].sum[q];
           __syncthreads();
           issue(stage[(u + kStages - 1) % kStages]);
-          if (now < count) {
-            if constexpr (Staged) accumulate_record_staged<FMT, RT>(stage[u].rec, ldsA[buffer], acc, lane, kq);
-            else accumulate_record<FMT, RT>(stage[u].rec, ldsA[buffer], ldsSums[buffer], acc, lane, kq);
-          }
+          if (now < count) accumulate_record<FMT, RT>(stage[u].rec, ldsA[buffer], ldsSums[buffer], acc, lane, kq);
           if constexpr (DecodeShared<RT>::kBuffers == 1) __syncthreads();   // every wave has read the buffer before the next super-block lands in it
         }
       }
