@@ -469,8 +469,7 @@ void HybridVerify::encodeWidePrefillLayer(hip::CommandGraph &graph, uint32_t lay
   }
   linear_.addWide(graph, w.router, wideTable_, wideScores_, {}, widePartials_, tokens);
   if (dims_.moeShape().sharedGate) ops::Normalization::addRms(graph, next, w.postNorm, normalized_, dims_.hidden, tokens);
-  ops::MoE::addChunk(graph, wideScores_, dims_.experts, normalized_, next, residual, w.experts, moeChunk_, dims_.moeShape(), tokens, w.sharedScalarGate,
-                     true);
+  ops::MoE::addChunk(graph, wideScores_, dims_.experts, normalized_, next, residual, w.experts, moeChunk_, dims_.moeShape(), tokens, w.sharedScalarGate);
 }
 
 void HybridVerify::addGdnPrefill(hip::CommandGraph &graph, const HybridLayer &w, uint32_t index, uint32_t tokens, uint64_t currentCell, uint64_t nextCell,

@@ -168,14 +168,14 @@ MoeChunkWorkspaceSize MoE::chunkWorkspace(const MoeShape &shape, uint32_t rows) 
 
 void MoE::addChunk(hip::CommandGraph &graph, const hip::Buffer &scores, uint32_t scoreStride, const hip::Buffer &normalized,
                    const hip::Buffer &residual, const hip::Buffer &output, const MoeExperts &experts, const MoeChunkWorkspace &w,
-                   const MoeShape &shape, uint32_t rows, const hip::Buffer &sharedScalarGate, bool tabled) {
+                   const MoeShape &shape, uint32_t rows, const hip::Buffer &sharedScalarGate) {
   const MoeChunkWorkspaceSize need = chunkWorkspace(shape, rows);
   if (!takesWide(shape, experts)) throw std::invalid_argument("the wide kernels take experts of K-quants, up to 8192 inputs");
   if (scoreStride < shape.experts) throw std::invalid_argument("a row of scores holds every expert's");
   if (shape.sharedGate) requireBytes(sharedScalarGate, uint64_t{shape.hidden} * 4, "shared expert gate");
   const uint64_t pairBytes = gguf_image_bytes(experts.format, shape.ffn, shape.hidden), downBytes = gguf_image_bytes(experts.downFormat, shape.hidden, shape.ffn);
   requireBytes(scores, (uint64_t{rows - 1} * scoreStride + shape.experts) * 4, "router scores");
-  if (!tabled || shape.sharedGate) requireBytes(normalized, uint64_t{rows} * shape.hidden * 2, "normalized rows");
+  if (shape.sharedGate) requireBytes(normalized, uint64_t{rows} * shape.hidden * 2, "normalized rows");
   requireBytes(residual, uint64_t{rows} * shape.hidden * 2, "residual rows");
   requireBytes(output, uint64_t{rows} * shape.hidden * 2, "MoE output");
   requireBytes(experts.gate, pairBytes * shape.allExperts(), "expert gate images");
@@ -200,22 +200,11 @@ void MoE::addChunk(hip::CommandGraph &graph, const hip::Buffer &scores, uint32_t
   const MoeChunkParams grouping{routes, all, shape.routesPerRow(), T};
   graph.add("moe_chunk_count", {w.selected, w.counts}, grouping, {windows, 1, 1}, {1024, 1, 1});
   graph.add("moe_chunk_place", {w.selected, w.counts, w.routeSlot, w.slotRow, w.tasks, w.totals}, grouping, {windows, 1, 1}, {1024, 1, 1});
-  auto project = [&](const hip::Buffer &input, uint32_t inputRows, uint32_t k, uint32_t n, uint32_t format, uint64_t expertBytes,
-                     const hip::Buffer &first, const hip::Buffer &second, const hip::Buffer &out, bool gateUp) {
-    const GgufWideTableParams slots{k, inputRows, tiles, 0};
-    // The gate/up pair gathers from a table of the rows, whatever their number of routes: against a table of the slots, each
-    // with the pass that makes it, 2048 rows 168.7 us for 185.7 at 8 routes a row, 79.5 for 87.1 at 2, 64.0 for 71.6 at 1; 300
-    // rows 67.1 for 79.8 at 8 and 47.5 for 57.5 at 1 (2048 -> 768 of 128 experts); 2048 rows of 4096 -> 1024, 4 of 32, 188.8
-    // for 210.6; 1000 rows of 2304 inputs 103.2 for 116.9.
-    if (gateUp) {
-      if (!tabled) graph.add("gguf_wide_rows", {input, w.table}, slots, {inputRows, 1, 1}, {256, 1, 1});
-    } else if (k <= GGUF_WIDE_TILE_INPUTS)
-      graph.add("gguf_wide_moe_rows_tile", {input, w.slotRow, w.totals, w.table}, slots, {tiles, 1, 1}, {1024, 1, 1});
-    else
-      graph.add("gguf_wide_moe_rows", {input, w.slotRow, w.totals, w.table}, slots, {64 * ((16 * tiles + 63) / 64), 1, 1}, {256, 1, 1});
+  auto project = [&](uint32_t tableRows, uint32_t k, uint32_t n, uint32_t format, uint64_t expertBytes, const hip::Buffer &first,
+                     const hip::Buffer &second, const hip::Buffer &out, bool gateUp) {
     GgufWideMoeParams params{};
     params.wide.input_size = k;
-    params.wide.rows = inputRows;
+    params.wide.rows = tableRows;
     params.wide.tiles = tiles;
     params.wide.out_stride = n;
     const uint32_t span = gateUp ? GGUF_WIDE_COLUMNS / 2 : GGUF_WIDE_COLUMNS;
@@ -227,9 +216,17 @@ void MoE::addChunk(hip::CommandGraph &graph, const hip::Buffer &scores, uint32_t
     if (gateUp) graph.add(kernel + "_x", {first, second, w.table, out, w.tasks, w.totals, w.slotRow}, params, grid, {256, 1, 1});
     else graph.add(kernel + "_a", {first, second, w.table, out, w.tasks, w.totals}, params, grid, {256, 1, 1});
   };
-  project(normalized, rows, shape.hidden, shape.ffn, experts.format, pairBytes, experts.gate, experts.up, w.intermediate, true);
-  project(w.intermediate, 16 * tiles, shape.ffn, shape.hidden, experts.downFormat, downBytes, experts.down, experts.down,
-          w.expertOutput, false);
+  // The gate/up pair gathers from a table of the rows, whatever their number of routes: against a table of the slots, each
+  // with the pass that makes it, 2048 rows 168.7 us for 185.7 at 8 routes a row, 79.5 for 87.1 at 2, 64.0 for 71.6 at 1; 300
+  // rows 67.1 for 79.8 at 8 and 47.5 for 57.5 at 1 (2048 -> 768 of 128 experts); 2048 rows of 4096 -> 1024, 4 of 32, 188.8
+  // for 210.6; 1000 rows of 2304 inputs 103.2 for 116.9.
+  project(rows, shape.hidden, shape.ffn, experts.format, pairBytes, experts.gate, experts.up, w.intermediate, true);
+  const GgufWideTableParams slots{shape.ffn, 16 * tiles, tiles, 0};
+  if (shape.ffn <= GGUF_WIDE_TILE_INPUTS)
+    graph.add("gguf_wide_moe_rows_tile", {w.intermediate, w.slotRow, w.totals, w.table}, slots, {tiles, 1, 1}, {1024, 1, 1});
+  else
+    graph.add("gguf_wide_moe_rows", {w.intermediate, w.slotRow, w.totals, w.table}, slots, {64 * ((16 * tiles + 63) / 64), 1, 1}, {256, 1, 1});
+  project(16 * tiles, shape.ffn, shape.hidden, experts.downFormat, downBytes, experts.down, experts.down, w.expertOutput, false);
   // whole 16-byte vectors of a row, or a column a thread
   const MoeCombineParams combine{rows, shape.hidden, shape.routesPerRow(), 0u};
   if (shape.hidden % 8 == 0 && w.expertOutput.gpuAddress() % 16 == 0 && residual.gpuAddress() % 16 == 0 && output.gpuAddress() % 16 == 0)

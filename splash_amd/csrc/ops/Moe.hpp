@@ -70,13 +70,12 @@ class MoE final {
 public:
   [[nodiscard]] static bool takesWide(const MoeShape &shape, const MoeExperts &experts) noexcept;
   [[nodiscard]] static MoeChunkWorkspaceSize chunkWorkspace(const MoeShape &shape, uint32_t rows);
-  // What addRouting and addRouted do, for up to kMaximumChunkRows rows. The gate/up pair gathers from the rows' tables
-  // (abi/Gguf.h) in the workspace's table; `tabled`: they are there already (Linear::addWideNormTable), and `normalized` is
-  // read for a gated shared expert alone.
+  // What addRouting and addRouted do, for up to kMaximumChunkRows rows, whose tables (abi/Gguf.h) Linear::addWideNormTable has
+  // left in the workspace's table: the gate/up pair gathers from them. `normalized` is read for a gated shared expert alone.
   static constexpr uint32_t kMaximumChunkRows = 2048;
   static void addChunk(hip::CommandGraph &graph, const hip::Buffer &scores, uint32_t scoreStride, const hip::Buffer &normalized,
                        const hip::Buffer &residual, const hip::Buffer &output, const MoeExperts &experts, const MoeChunkWorkspace &workspace,
-                       const MoeShape &shape, uint32_t rows, const hip::Buffer &sharedScalarGate = {}, bool tabled = false);
+                       const MoeShape &shape, uint32_t rows, const hip::Buffer &sharedScalarGate = {});
   [[nodiscard]] static MoeWorkspaceSize workspace(const MoeShape &shape, uint32_t rows);
   // Selects and weighs each row's experts from its fp32 router scores ([rows][scoreStride]), appends the shape's shared
   // slices to every row's routes and groups the routes. `input` (the normalized rows, bf16 [rows][hidden]) and
