@@ -348,8 +348,9 @@ template <int RT> struct DecodeShared {
   __device__ __forceinline__ uint16_t *epilogueRows() { return reinterpret_cast<uint16_t *>(epilogueSums() + 2u * RT * 256u); }
   __device__ __forceinline__ float *epilogueHalves() { return reinterpret_cast<float *>(epilogueRows() + 4u * RT * 256u); }
 };
-// The ring's: a stage is two groups of a super-block's activations, [row tile][group][lane], and four of them are a
-// super-block. Objects of their own, so that a read of one does not wait for what is on its way into another.
+// The ring's: a stage is two groups of a super-block's activations (four at one row tile), [row tile][group][lane], and the ring
+// four stages: a super-block, at one row tile two. Objects of their own, so that a read of one does not wait for what is on its
+// way into another.
 template <int RT> struct DecodeRing {
   static constexpr bool kRing = true;
   static constexpr uint32_t kStageGroups = RT == 1 ? 4 : 2;
@@ -359,7 +360,7 @@ template <int RT> struct DecodeRing {
   float *scaleParts, *rowScale;   // of a table with a deferred scale
   uint32_t *arrivedWord;
   __device__ __forceinline__ uint32_t &arrived() { return *arrivedWord; }
-  // (a stage holds 2 KiB a row tile)
+  // (a stage holds 2 KiB a row tile, 4 KiB at one: the epilogues lay out at most 2 KiB a row tile in each)
   __device__ __forceinline__ float *epilogueSums() { return reinterpret_cast<float *>(rows0); }
   __device__ __forceinline__ uint16_t *epilogueRows() { return reinterpret_cast<uint16_t *>(rows1); }
   __device__ __forceinline__ float *epilogueHalves() { return reinterpret_cast<float *>(rows2); }
@@ -695,9 +696,8 @@ __device__ __forceinline__ void decode_workgroup(Shared &shared, const uint8_t *
     // Every row's inverse RMS from the squares the table's writer left, one entry a 64-column group:
     // part q of 16 adds entries q, q + 16, ... in order, then the 16 parts are added in order -- the same
     // sums whatever the kernel's row tiles, so a row's result does not depend on the block's height. A
-    // thread takes RT parts of its row. The loads go out before the first weights', so the wait for
-    // them leaves those in flight.
-    // (of three row tiles, 240 threads take five parts a turn)
+    // thread takes kTurns parts of its row: one a row tile, of three row tiles, where 240 threads take five parts a turn, four.
+    // The loads go out before the first weights', so the wait for them leaves those in flight.
     constexpr uint32_t kRows = 16u * RT, kParts = 16u, kThreadParts = 256u / kRows, kTurns = (kParts + kThreadParts - 1u) / kThreadParts;
     // Eight entries of a part are loaded together and added in their order afterwards, so a part costs one round trip
     // to the cache, not one an entry; the first eight go out before the first weights and are added once those are
@@ -751,10 +751,10 @@ __device__ __forceinline__ void decode_workgroup(Shared &shared, const uint8_t *
       }
     };
     uint32_t mine = 16u * lane, column = kColumnPart + 16u * c;
-    // A staging Q6_K wave of four row tiles has no register left for its lane's three places in a record: it works them out for
-    // each. (Kept, one was spilled and read back behind the loads just issued, and the wait for it was the wait for all
-    // of them: the vector-memory counter is one queue. 64 rows of 17408 -> 5120 57.1 -> 53.3 us, 5120 -> 17408 59.5 -> 52.7,
-    // 5120 -> 8192 Q4_K and 6144 Q6_K columns in one dispatch, at two waves a SIMD before and three now, 44.0 -> 38.9.)
+    // A staging Q6_K wave of four row tiles (of a chain, or of q|k|v with its preparation) has no register left for its lane's
+    // three places in a record: it works them out for each. (Kept, one was spilled and read back behind the loads just issued,
+    // and the wait for it was the wait for all of them: the vector-memory counter is one queue. The plain kernels, when they
+    // staged so, 64 rows of 17408 -> 5120 57.1 -> 53.3 us, 5120 -> 17408 59.5 -> 52.7.)
     constexpr bool kFreshLane = !kRing && FMT == GGUF_FMT_Q6K && RT > 2;
     uint32_t record = 0;
     auto issueWeights = [&](Record<FMT> &rec) {

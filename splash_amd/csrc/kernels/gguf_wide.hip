@@ -18,7 +18,9 @@
 // overlap the conversion of one with the MFMAs of the other. At 2048 rows of the 5120 x 2 x 25600 Q4_K gate/up pair a
 // launch takes 1.09 ms (985 TFLOP/s of the projection's own operations; the 64-row windows of the decode kernels took
 // 2.38 ms), at 25600 x 5120 Q6_K 0.86 ms (2.2 ms): with the constant terms and the second product that is 1.11 and 1.25
-// PFLOP/s of MFMAs, where a large library product reaches 1.19 under the card's power limit.
+// PFLOP/s of MFMAs, where a large fp16 library product of normally distributed values reaches 1.25 (of zeros 1.74: the card's
+// power limits it). The matrix cores are busy 57 and 64 % of the cycles, a SIMD issues vector instructions in 60 and 54 %, and
+// waves wait 14 to 15 %.
 #include "abi/Gguf.h"
 #include "abi/Moe.h"
 #include "backend/KernelRegistry.hpp"
@@ -59,7 +61,8 @@ __device__ __forceinline__ uint4 *wide_row_entry(uint8_t *of, uint32_t inputSize
   const uint32_t block = (line / 4u - operand) / GGUF_WIDE_OPERANDS;
   return reinterpret_cast<uint4 *>(of + (operand < 8u ? (block * 8u + operand) * 64u : inputSize * 2u + block * 64u) + 16u * kq);
 }
-// The rows' tables, a workgroup a row: whole lines of the row's own.
+// The rows' tables of rows as they are, a workgroup a row: whole lines of the row's own. (What the tables that a norm leaves are
+// held against.)
 __global__ __launch_bounds__(256) void gguf_wide_rows(const uint16_t *__restrict__ input, uint8_t *__restrict__ rows, GgufWideTableParams p) {
   const uint32_t row = blockIdx.x, bytes = gguf_wide_row_bytes(p.input_size);
   if (row >= p.rows) return;
@@ -743,7 +746,7 @@ __global__ __launch_bounds__(256, 2) void gguf_wide_moe(const uint8_t *__restric
   wide_moe<FMT, EP, T, false>(seg0, seg1, table, out, tasks, totals, nullptr, m);
 }
 // The gate/up pair of the rows that the slots gather, from the rows' tables. A table of the slots holds a row as often as it
-// has routes, and writing it was a pass bound by memory (16384 slots of 2048 inputs: 27.8 us behind a norm's 9.5, for the 2.0
+// has routes, and writing it was a pass bound by memory (16384 slots of 2048 inputs: 27.8 us behind a norm's 9.5, for the 3.8
 // that the rows' tables add to the norm's own table). The loads fetch a row's whole lines, as the slots' fetch a tile's, so the
 // pair itself takes little longer: 149.3 -> 152.8 us at 2048 rows, 8 of 128 experts, 2048 x 2 x 768 Q4_K.
 template <uint32_t FMT, uint32_t T>

@@ -96,7 +96,7 @@ LinearScratchSize LinearPlan::scratchSize() const noexcept {
     // of the partitioned workgroups only
     const uint64_t groups = std::max<uint64_t>(1, groupsOf(n, workload_.epilogue) - config_.wholeGroups);
     // a piece of the dispatch's rows keeps its own, as many as a whole piece takes
-    // (the kernel's row tiles: 1, 2 or 4, which may be more than the rows fill)
+    // (the plan's row tiles: 1, 2 or 4, which may be more than the rows fill and than the kernel's, which may be 3)
     const uint32_t pieces = rowPieces(workload_.rows), pieceTiles = storageRows() / GGUF_ROW_TILE;
     size.partials = uint64_t{pieces} * config_.splits * groups * kWavesAcross * pieceTiles * 256u * sizeof(float);
     size.counters = uint64_t{pieces} * groups * sizeof(uint32_t);
